@@ -22,6 +22,7 @@ _runtime = None
 P = c_void_p
 I = c_int
 F = c_float
+L = c_int64
 
 # name -> argtypes (every kernel launcher returns int: 0 = ok, <0 = bad arguments, >0 = hipError)
 _KERNEL_SIGS = {
@@ -95,13 +96,11 @@ _KERNEL_SIGS = {
     "cfc_prefill_attention_expanded2": [P, c_int64, c_int64, P, P, P, P, P, c_int64, P, P, P, P, I, I, F, I, P, P, c_int64, P,
                                         c_int64, P],
     "cfc_prefill_attention_expanded": [P, P, P, P, c_int64, P, P, P, P, I, I, F, P, c_int64, P],
-    "cfc_knn_scores": [P, P, I, I, I, P, P, P, P],
-    "cfc_topk_pass": [P, P, I, I, I, I, P, P, P],
-    "cfc_knn_topk": [P, P, I, I, I, I, P, P, P, I, P, P, P],
+    "cfc_knn_scan": [P, P, I, I, I, P, P, P, P, L, P, I, I, P],
+    "cfc_topk_block": [I],
+    "cfc_topk_select": [P, P, I, I, L, I, P, I, L, P, P, P],
     "cfc_knn_topk_rows": [],
-    "cfc_knn_flat_rows": [I, I],
     "cfc_ivf_topk": [P, P, I, I, I, P, P, P, P, I, P, I, I, P, P, P],
-    "cfc_topk_chunk_size": [],
     "cfc_l2_normalize": [P, P, P, I, I, P],
     "cfc_pool": [P, P, P, P, I, I, I, I, P],
     "cfc_splitk_reduce": [P, I, I, I, I, P, I, P],

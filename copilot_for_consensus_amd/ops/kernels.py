@@ -1363,16 +1363,38 @@ def decode_advance(next_ids, tokens, step, input_ids, positions, ctx_lens, slots
 
 # ----------------------------------------------------------------------------- vector search
 
+def _knn_scan(X, Q, xnorm2, qnorm2, alive, row_lo: int, N: int, out, bmax) -> None:
+    """Scores of rows [row_lo, N) into ``out`` [nq, >= rows] and their block maxima into ``bmax`` (or None)."""
+    def at(t, step=1):
+        return None if t is None else t.data_ptr() + row_lo * step * t.element_size()
+    lib, n = kernels(), N - row_lo
+    B = lib.cfc_topk_block(n)
+    check(lib.cfc_knn_scan(at(X, X.shape[1]), Q.data_ptr(), n, Q.shape[0], X.shape[1], at(xnorm2), _p(qnorm2), at(alive),
+                           out.data_ptr(), out.stride(0), _p(bmax), -(-n // B), B, _stream(X)), "cfc_knn_scan")
+
+
 def knn_scores(X, Q, xnorm2=None, qnorm2=None, out=None):
     """scores [nq, N] fp32 for nq <= 16 queries (dot, or -squared-L2 when norms are given)."""
     if not X.is_cuda:
         return ref.knn_scores(X, Q, xnorm2, qnorm2)
-    N, dim = X.shape
-    nq = Q.shape[0]
+    N, nq = X.shape[0], Q.shape[0]
     out = torch.empty(nq, N, dtype=torch.float32, device=X.device) if out is None else out
-    check(kernels().cfc_knn_scores(X.data_ptr(), Q.data_ptr(), N, nq, dim, _p(xnorm2), _p(qnorm2), out.data_ptr(),
-                                   _stream(X)), "cfc_knn_scores")
+    _knn_scan(X, Q, xnorm2, qnorm2, None, 0, N, out, None)
     return out
+
+
+def _select(scores, n: int, k: int, ids, bmax, row_lo: int = 0):
+    """(values, ids) [nq, k] descending of the first ``n`` scores of every row of ``scores`` (the lower index first among
+    equals); ``bmax``: their block maxima (None: taken here); ``ids``: the scores' ids (None: row_lo + index)."""
+    lib, nq, dev = kernels(), scores.shape[0], scores.device
+    fill = bmax is None
+    if fill:
+        bmax = torch.empty(nq, -(-n // lib.cfc_topk_block(n)), dtype=torch.int32, device=dev)
+    v = torch.empty(nq, k, dtype=torch.float32, device=dev)
+    i = torch.empty(nq, k, dtype=torch.int64, device=dev)
+    check(lib.cfc_topk_select(scores.data_ptr(), _p(ids), nq, n, scores.stride(0), k, bmax.data_ptr(), int(fill), row_lo, v.data_ptr(),
+                              i.data_ptr(), _stream(scores)), "cfc_topk_select")
+    return v, i
 
 
 def topk(scores: torch.Tensor, k: int, ids: torch.Tensor | None = None):
@@ -1384,30 +1406,15 @@ def topk(scores: torch.Tensor, k: int, ids: torch.Tensor | None = None):
         if ids is not None:
             i = torch.gather(ids, 1, i)
         return v, i
-    lib = kernels()
-    chunk = lib.cfc_topk_chunk_size()
-    cur_v, cur_i, cur_n = scores.contiguous(), ids, n
-    while True:
-        nch = math.ceil(cur_n / chunk)
-        ov = torch.empty(nq, nch * k_eff, dtype=torch.float32, device=scores.device)
-        oi = torch.empty(nq, nch * k_eff, dtype=torch.int64, device=scores.device)
-        check(lib.cfc_topk_pass(cur_v.data_ptr(), _p(cur_i), nq, cur_n, cur_v.shape[1], k_eff, ov.data_ptr(),
-                                oi.data_ptr(), _stream(scores)), "cfc_topk_pass")
-        cur_v, cur_i, cur_n = ov, oi, nch * k_eff
-        if nch == 1:
-            break
-    order = torch.argsort(cur_v, dim=1, descending=True, stable=True)
-    return torch.gather(cur_v, 1, order), torch.gather(cur_i, 1, order)
+    return _select(scores.contiguous(), n, k_eff, None if ids is None else ids.contiguous(), None)
 
 
-def _merge_candidates(cv: torch.Tensor, ci: torch.Tensor, k: int):
-    """Exact top-k of per-chunk candidates [nq, m] (values, row ids) -> sorted [nq, k]."""
-    return topk(cv, k, ci)
+KNN_SCORES = 1 << 26     # scores of one pass over (part of) an index: 256 MB of workspace, what the last-level cache holds
 
 
 def knn_topk(X, Q, k: int, xnorm2=None, qnorm2=None, alive=None, row_lo: int = 0, N: int | None = None):
-    """Fused flat scan + top-k (knn.hip knn_topk_kernel) over rows [row_lo, N) of X for <= 16
-    queries: (scores [nq, k] descending, row indices [nq, k]); the [nq, N] scores never reach HBM."""
+    """Flat scan + top-k over rows [row_lo, N) of X for <= 16 queries and k <= 256: (scores [nq, k] descending, row
+    indices [nq, k]).  The scores of at most KNN_SCORES rows and queries are held at a time."""
     N = X.shape[0] if N is None else N
     nq = Q.shape[0]
     if not X.is_cuda:
@@ -1416,13 +1423,20 @@ def knn_topk(X, Q, k: int, xnorm2=None, qnorm2=None, alive=None, row_lo: int = 0
             sc = sc.masked_fill(~alive[row_lo:N].bool()[None], float("-inf"))
         v, i = torch.topk(sc.float(), min(k, N - row_lo), dim=1)
         return v, i + row_lo
-    R = kernels().cfc_knn_flat_rows(nq, k)
-    nch = -(-(N - row_lo) // R)
-    cv = torch.empty(nq, nch * k, dtype=torch.float32, device=X.device)
-    ci = torch.empty(nq, nch * k, dtype=torch.int64, device=X.device)
-    check(kernels().cfc_knn_topk(X.data_ptr(), Q.data_ptr(), N, row_lo, nq, X.shape[1], _p(xnorm2), _p(qnorm2),
-                                 _p(alive), k, cv.data_ptr(), ci.data_ptr(), _stream(X)), "cfc_knn_topk")
-    return _merge_candidates(cv, ci, min(k, N - row_lo))
+    if not 1 <= k <= 256 or not 1 <= nq <= 16 or N <= row_lo:
+        raise ValueError(f"knn_topk: k {k} (1 to 256), {nq} queries (1 to 16), rows {row_lo} to {N}")
+    step = min(N - row_lo, KNN_SCORES // nq)
+    nb = -(-step // kernels().cfc_topk_block(step))
+    sc = torch.empty(nq, -(-step // 4) * 4, dtype=torch.float32, device=X.device)
+    bmax = torch.empty(nq * nb, dtype=torch.int32, device=X.device)
+    parts = []
+    for lo in range(row_lo, N, step):
+        n = min(step, N - lo)
+        _knn_scan(X, Q, xnorm2, qnorm2, alive, lo, lo + n, sc, bmax)
+        parts.append(_select(sc, n, min(k, n), None, bmax, lo))
+    if len(parts) == 1:
+        return parts[0]
+    return topk(torch.cat([v for v, _ in parts], 1), k, torch.cat([i for _, i in parts], 1))
 
 
 def ivf_topk(X, Q, probe: torch.Tensor, list_off: torch.Tensor, maxc: int, k: int, xnorm2=None, qnorm2=None,

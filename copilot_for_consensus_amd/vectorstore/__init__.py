@@ -363,7 +363,7 @@ class HipFlatIndex(VectorStore):
             Qn = Q.contiguous()
             qn2 = Qn.float().pow(2).sum(1)
         if Q.is_cuda and nq <= 16 and k <= 256:
-            # fused scan + top-k: only k candidates per 1024-row chunk leave the CUs
+            # scores and their block maxima in one pass, then only the blocks that can hold a winner
             return K.knn_topk(self._X, Qn, k, self._norm2 if self.metric == "l2" else None, qn2,
                               self._alive if self._dead else None, row_lo=lo, N=hi)
         xn2 = self._norm2[lo:hi] if self.metric == "l2" else None

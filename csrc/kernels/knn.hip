@@ -5,16 +5,14 @@
 // (adapters/copilot_vectorstore/copilot_vectorstore/inmemory.py:106-119), FAISS IndexFlatL2 /
 // IVFFlat (faiss_store.py:101-111,214) and Qdrant query_points (qdrant_store.py:371).
 //
-//   * cfc_knn_scores: scores[q][n] = <x_n, q>  (or -||x_n - q||^2) for <= 16 queries, one pass
-//     over the bf16 index with MFMA 16x16x32 (queries are the B columns, index rows stream
-//     straight from HBM into the A operand: the GEMV regime of guide §5 table, last row).
-//   * cfc_topk: exact per-query top-k by 4-pass 8-bit radix select in LDS per chunk; applied
-//     recursively on the candidates until one chunk remains.
-//   * cfc_knn_topk / cfc_ivf_topk: the scan and the top-k FUSED: each workgroup scores its
-//     1024-row chunk against its queries into LDS and radix-selects every query's k best there,
-//     so only k candidates per (query, chunk) reach HBM (never the [nq, N] score matrix); the
-//     IVF form takes (query, probed list, chunk) work items from a device list-offset table in
-//     one launch.  The candidates are merged by cfc_topk_pass.
+//   * cfc_knn_scan: scores[q][n] = <x_n, q>  (or -||x_n - q||^2) for <= 16 queries, one pass over
+//     the bf16 index with MFMA 16x16x32 (queries are the B columns, index rows stream straight from
+//     HBM into the A operand), and every block of rows' best score beside them.
+//   * cfc_topk_select: exact sorted top-k of scores with their block maxima: the k-th best block
+//     maximum bounds the k-th best score from below, so only the blocks that reach it are looked at.
+//   * cfc_ivf_topk: scan and top-k of (query, probed list, chunk) work items from a device list-offset
+//     table in one launch: each workgroup scores its chunk into LDS and selects the k best there;
+//     the candidates are merged by cfc_topk_select.
 //   * cfc_l2_normalize: rows -> unit length (+ fp32 norms), used on insert for cosine.
 //   * cfc_pool: masked mean / CLS pooling over varlen sequences (+ optional L2 normalise):
 //     the SentenceTransformer Pooling+Normalize modules.
@@ -24,12 +22,29 @@ namespace {
 
 __device__ __forceinline__ bf16x8_t as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8_t, v); }
 
+__device__ __forceinline__ uint32_t f2key(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float key2f(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
+
+// One wave scores a block of B rows (a multiple of 16) against all queries.  Every lane holds four rows'
+// scores of one query; they are stored as they lie and their largest key goes to bmax [nq][nb].  Nothing
+// is selected here, so the pass is a plain stream over X: 1M x 384 bf16 with one query in 131 us
+// (5.9 TB/s) where scoring 2048-row chunks into LDS and selecting in them took 172 us (4.5 TB/s; 489
+// workgroups, two on most CUs and one on the rest, the selecting wave alone at each one's end).
+// alive: optional row mask; scores of other rows are -inf.
 template <int KC>  // KC = D / 32 MFMA k-steps
-__global__ void __launch_bounds__(256) knn_scores_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q,
-                                                         int N, int nq, const float* __restrict__ xnorm2,
-                                                         const float* __restrict__ qnorm2, float* __restrict__ out) {
+__global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
+                                                       int nq, const float* __restrict__ xnorm2,
+                                                       const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
+                                                       float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
+                                                       int B) {
   constexpr int D = KC * 32;
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, blk = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (blk >= nb) return;
   const int col = lane & 15, g = lane >> 4;
   const bool qv = col < nq;
   bf16x8_t qf[KC];
@@ -40,112 +55,258 @@ __global__ void __launch_bounds__(256) knn_scores_kernel(const uint16_t* __restr
       qf[c] = as_bf16x8(qv ? *reinterpret_cast<const uint4*>(qr + 32 * c + 8 * g) : make_uint4(0, 0, 0, 0));
   }
   const float qn = (qnorm2 && qv) ? qnorm2[col] : 0.f;
-  const int ngroups = (N + 15) / 16;
-  const int wave_global = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int nwaves = (gridDim.x * blockDim.x) >> 6;
-  for (int grp = wave_global; grp < ngroups; grp += nwaves) {
-    const int r0 = grp * 16;
-    const int r = min(r0 + col, N - 1);
-    const uint16_t* xr = X + (size_t)r * D;
-    uint4 a[KC];
+  const int lo = blk * B, hi = min(N, lo + B);
+  uint32_t best = 0u;
+  auto load = [&](uint4* a, int r0) {
+    const uint16_t* xr = X + (size_t)min(r0 + col, N - 1) * D;
 #pragma unroll
     for (int c = 0; c < KC; ++c) a[c] = *reinterpret_cast<const uint4*>(xr + 32 * c + 8 * g);
+  };
+  auto score = [&](const uint4* a, int r0) {
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < KC; ++c) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[c]), qf[c], acc, 0, 0, 0);
-    if (qv) {
-      const int rb = r0 + 4 * g;
-      float v[4];
+    if (!qv) return;
+    const int rb = r0 + 4 * g;
+    float v[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[i] = acc[i];
-        if (xnorm2) v[i] = -(xnorm2[min(rb + i, N - 1)] + qn - 2.f * v[i]);
-      }
-      float* orow = out + (size_t)col * N;
-      if (rb + 3 < N && (N & 3) == 0) {
-        *reinterpret_cast<float4*>(orow + rb) = make_float4(v[0], v[1], v[2], v[3]);
-      } else {
+    for (int i = 0; i < 4; ++i) {
+      const int row = min(rb + i, N - 1);
+      v[i] = acc[i];
+      if (xnorm2) v[i] = -(xnorm2[row] + qn - 2.f * v[i]);
+      if (alive && !alive[row]) v[i] = -INFINITY;
+      if (rb + i < N) best = max(best, f2key(v[i]));
+    }
+    float* o = out + col * ld + rb;
+    if (rb + 3 < N && (ld & 3) == 0) {
+      *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (rb + i < N) orow[rb + i] = v[i];
+      for (int i = 0; i < 4; ++i)
+        if (rb + i < N) o[i] = v[i];
+    }
+  };
+  if constexpr (KC <= 16) {          // the next 16 rows in flight under these (144 -> 131 us); wider rows fill the registers alone
+    uint4 a[2][KC];
+    load(a[0], lo);
+    for (int r0 = lo; r0 < hi; r0 += 32) {
+      if (r0 + 16 < hi) load(a[1], r0 + 16);
+      score(a[0], r0);
+      if (r0 + 32 < hi) load(a[0], r0 + 32);
+      if (r0 + 16 < hi) score(a[1], r0 + 16);
+    }
+  } else {
+    uint4 a[KC];
+    for (int r0 = lo; r0 < hi; r0 += 16) {
+      load(a, r0);
+      score(a, r0);
+    }
+  }
+  if (bmax == nullptr) return;
+  best = max(best, (uint32_t)__shfl_xor((int)best, 16, 64));
+  best = max(best, (uint32_t)__shfl_xor((int)best, 32, 64));
+  if (g == 0 && qv) bmax[(size_t)col * nb + blk] = best;
+}
+
+// ------------------------------------------------------------------ exact top-k
+// Largest key of every B consecutive scores: one wave per block, grid (ceil(nb / 4), nq).
+__global__ void __launch_bounds__(256) block_max_kernel(const float* __restrict__ in, int n, size_t ld, int B, uint32_t* __restrict__ bmax,
+                                                        int nb) {
+  const int lane = threadIdx.x & 63, blk = blockIdx.x * 4 + (threadIdx.x >> 6), qi = blockIdx.y;
+  if (blk >= nb) return;
+  const float* src = in + (size_t)qi * ld;
+  const int hi = (int)min((long)n, (long)(blk + 1) * B);
+  uint32_t best = 0u;
+  for (int i = blk * B + lane; i < hi; i += 64) best = max(best, f2key(src[i]));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) best = max(best, (uint32_t)__shfl_xor((int)best, o, 64));
+  if (lane == 0) bmax[(size_t)qi * nb + blk] = best;
+}
+
+constexpr int SEL_THREADS = 1024, SEL_WAVES = SEL_THREADS / 64;
+constexpr int SEL_BLOCKS = 16384;      // most blocks of a query (16 maxima per thread)
+constexpr int SEL_CAP = 8192;          // candidates held
+constexpr int SEL_STEP = 4096;         // scores looked at between two looks at the candidates' number
+constexpr int SEL_K = 2048;            // most winners: SEL_K + SEL_STEP <= SEL_CAP
+
+// Sum over the workgroup of a wave-uniform count: one barrier a call, the two halves of `red` in turn.
+__device__ __forceinline__ int sel_count(int c, int (*red)[SEL_WAVES], int& turn) {
+  if ((threadIdx.x & 63) == 0) red[turn][threadIdx.x >> 6] = c;
+  __syncthreads();
+  int t = 0;
+#pragma unroll
+  for (int i = 0; i < SEL_WAVES; ++i) t += red[turn][i];
+  turn ^= 1;
+  return t;
+}
+
+// The candidates cut to their kk largest (cnt > kk; all differ, as each holds its row).  Any bound that
+// exactly kk of them reach will do, so the bitwise search ends where the count fits.
+__device__ __forceinline__ void sel_cut(uint64_t* cand, int cnt, int kk, int (*red)[SEL_WAVES], int& turn, int* s_n) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  uint64_t e[SEL_CAP / SEL_THREADS];
+#pragma unroll
+  for (int j = 0; j < SEL_CAP / SEL_THREADS; ++j) e[j] = tid + j * SEL_THREADS < cnt ? cand[tid + j * SEL_THREADS] : 0ull;
+  uint64_t thr = 0;
+  for (int b = 63; b >= 0; --b) {
+    const uint64_t t = thr | (1ull << b);
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < SEL_CAP / SEL_THREADS; ++j) c += __popcll(__ballot(e[j] >= t));
+    c = sel_count(c, red, turn);
+    if (c >= kk) thr = t;
+    if (c == kk) break;
+  }
+  if (tid == 0) *s_n = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < SEL_CAP / SEL_THREADS; ++j) {
+    const bool p = e[j] != 0ull && e[j] >= thr;
+    const uint64_t m = __ballot(p);
+    int at = 0;
+    if (lane == 0 && m) at = atomicAdd(s_n, __popcll(m));
+    at = __shfl(at, 0, 64) + __popcll(m & ((1ull << lane) - 1ull));
+    if (p) cand[at] = e[j];
+  }
+  __syncthreads();
+}
+
+// Sorted top-k of a query's n scores, one workgroup per query.  Largest first, the lower row first among
+// equals.  bmax [nq][nb] holds the largest key of every B rows.  At least k blocks hold a score at or
+// above the k-th best maximum, so no lower score is among the k best: the scores of the blocks that reach
+// this bound (about k of them) are read, those at or above it kept, cut to k and ranked.
+// A chain of short steps: 18 us for 150 of 1M scores, where three rounds of radix histograms in LDS over
+// 2048-row chunks' winners and a library sort took 120.
+// ids (row stride ld, optional): what the rows are called; else row0 + row.
+__global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* __restrict__ in, int n, size_t ld, int B,
+                                                                  const uint32_t* __restrict__ bmax, int nb, int k,
+                                                                  const int64_t* __restrict__ ids, int64_t row0,
+                                                                  float* __restrict__ out_v, int64_t* __restrict__ out_i) {
+  __shared__ uint64_t cand[SEL_CAP];
+  __shared__ uint16_t list[SEL_BLOCKS];
+  __shared__ int red[2][SEL_WAVES], s_n, s_list;
+  __shared__ uint32_t s_lo[SEL_WAVES], s_hi[SEL_WAVES];
+  const int tid = threadIdx.x, lane = tid & 63, qi = blockIdx.x;
+  const uint64_t below = (1ull << lane) - 1ull;
+  int turn = 0;
+  uint32_t key[SEL_BLOCKS / SEL_THREADS];
+#pragma unroll
+  for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
+    const int i = tid + j * SEL_THREADS;
+    key[j] = i < nb ? bmax[(size_t)qi * nb + i] : 0u;
+  }
+  // a bound that k blocks reach, and not many more (none: every block is looked at); the search begins
+  // below the bits that all maxima share
+  uint32_t thr = 0;
+  if (nb > k) {
+    uint32_t lo = ~0u, hi = 0u;
+#pragma unroll
+    for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
+      if (tid + j * SEL_THREADS < nb) lo = min(lo, key[j]);
+      hi = max(hi, key[j]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
+      hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
+    }
+    if (lane == 0) { s_lo[tid >> 6] = lo; s_hi[tid >> 6] = hi; }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < SEL_WAVES; ++i) { lo = min(lo, s_lo[i]); hi = max(hi, s_hi[i]); }
+    if (lo == hi) {
+      thr = hi;
+    } else {
+      const int top = 31 - __clz(lo ^ hi);
+      thr = top == 31 ? 0u : hi >> (top + 1) << (top + 1);
+      for (int b = top; b >= 0; --b) {
+        const uint32_t t = thr | (1u << b);
+        int c = 0;
+#pragma unroll
+        for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) c += __popcll(__ballot(key[j] >= t));
+        c = sel_count(c, red, turn);
+        if (c >= k) thr = t;
+        if (c >= k && c <= k + k / 4) break;
       }
     }
   }
-}
-
-__device__ __forceinline__ uint32_t f2key(float f) {
-  const uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float key2f(uint32_t k) {
-  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
-}
-
-constexpr int TOPK_CHUNK = 8192;
-
-// grid = (nchunks, nq), block = 256.  in: [nq][n] fp32 scores (row stride ld), optional idx_in
-// [nq][n] int64 ids; out: [nq][nchunks][k] (unordered within a chunk).
-__global__ void __launch_bounds__(256) topk_chunk_kernel(const float* __restrict__ in, const int64_t* __restrict__ idx_in,
-                                                         int n, int ld, int k, float* __restrict__ out_v,
-                                                         int64_t* __restrict__ out_i) {
-  __shared__ uint32_t keys[TOPK_CHUNK];
-  __shared__ uint32_t hist[256];
-  __shared__ uint32_t s_prefix, s_need, s_cnt_gt, s_cnt_eq;
-  const int chunk = blockIdx.x, qi = blockIdx.y, tid = threadIdx.x;
-  const int beg = chunk * TOPK_CHUNK;
-  const int len = min(TOPK_CHUNK, n - beg);
-  const float* src = in + (size_t)qi * ld + beg;
-  for (int i = tid; i < len; i += 256) keys[i] = f2key(src[i]);
-  const int kk = min(k, len);
-  if (tid == 0) { s_prefix = 0; s_need = kk; }
+  if (tid == 0) { s_n = 0; s_list = 0; }
   __syncthreads();
-  uint32_t mask = 0;
-  for (int shift = 24; shift >= 0; shift -= 8) {
-    hist[tid] = 0;
-    __syncthreads();
-    const uint32_t prefix = s_prefix;
-    for (int i = tid; i < len; i += 256) {
-      const uint32_t key = keys[i];
-      if ((key & mask) == prefix) atomicAdd(&hist[(key >> shift) & 255u], 1u);
+#pragma unroll
+  for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
+    const int i = tid + j * SEL_THREADS;
+    const bool p = i < nb && key[j] >= thr;
+    const uint64_t m = __ballot(p);
+    int at = 0;
+    if (lane == 0 && m) at = atomicAdd(&s_list, __popcll(m));
+    at = __shfl(at, 0, 64) + __popcll(m & below);
+    if (p) list[at] = (uint16_t)i;
+  }
+  __syncthreads();
+  const int lb = 31 - __clz(B);                      // B is a power of two
+  const long total = (long)s_list << lb;             // scores to look at, four neighbours per thread
+  const float* src = in + (size_t)qi * ld;
+  const bool vec = (ld & 3) == 0 && ((uintptr_t)in & 15) == 0;
+  auto place = [&](long at) { return at < total ? ((int)list[at >> lb] << lb) + (int)(at & (B - 1)) : n; };
+  auto load = [&](int row) {
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (vec && row + 3 < n) {
+      x = *reinterpret_cast<const float4*>(src + row);
+    } else {
+      if (row < n) x.x = src[row];
+      if (row + 1 < n) x.y = src[row + 1];
+      if (row + 2 < n) x.z = src[row + 2];
+      if (row + 3 < n) x.w = src[row + 3];
     }
-    __syncthreads();
-    if (tid == 0) {
-      uint32_t need = s_need, acc = 0;
-      int d = 255;
-      for (; d > 0; --d) {
-        if (acc + hist[d] >= need) break;
-        acc += hist[d];
+    return x;
+  };
+  int row = place(4 * tid);
+  float4 x = load(row);
+  for (long s0 = 0; s0 < total; s0 += SEL_STEP) {
+    const int row1 = place(s0 + SEL_STEP + 4 * tid);
+    const float4 x1 = load(row1);                     // the next step's, under this one's work
+    const float v[4] = {x.x, x.y, x.z, x.w};
+    uint32_t kv[4];
+    uint64_t m[4];
+    int mine = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      kv[u] = f2key(v[u]);
+      m[u] = __ballot(row + u < n && kv[u] >= thr);
+      mine += __popcll(m[u]);
+    }
+    if (mine) {
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&s_n, mine);
+      at = __shfl(at, 0, 64);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (m[u] >> lane & 1) cand[at + __popcll(m[u] & below)] = ((uint64_t)kv[u] << 32) | (0xffffffffu - (uint32_t)(row + u));
+        at += __popcll(m[u]);
       }
-      s_need = need - acc;
-      s_prefix = prefix | ((uint32_t)d << shift);
     }
-    mask |= 255u << shift;
+    row = row1;
+    x = x1;
     __syncthreads();
+    const int cnt = s_n;
+    __syncthreads();
+    if (cnt > SEL_CAP - SEL_STEP) sel_cut(cand, cnt, k, red, turn, &s_n);   // the next step might not fit
   }
-  const uint32_t thr = s_prefix;
-  const uint32_t need_eq = s_need;
-  if (tid == 0) { s_cnt_gt = 0; s_cnt_eq = 0; }
-  __syncthreads();
-  float* ov = out_v + ((size_t)qi * gridDim.x + chunk) * k;
-  int64_t* oi = out_i + ((size_t)qi * gridDim.x + chunk) * k;
-  const uint32_t n_gt = (uint32_t)kk - need_eq;
-  for (int i = tid; i < len; i += 256) {
-    const uint32_t key = keys[i];
-    int slot = -1;
-    if (key > thr) slot = (int)atomicAdd(&s_cnt_gt, 1u);
-    else if (key == thr) {
-      const uint32_t e = atomicAdd(&s_cnt_eq, 1u);
-      if (e < need_eq) slot = (int)(n_gt + e);
-    }
-    if (slot >= 0) {
-      ov[slot] = key2f(key);
-      oi[slot] = idx_in ? idx_in[(size_t)qi * ld + beg + i] : (int64_t)(beg + i);
-    }
+  if (s_n > max(k, SEL_THREADS)) sel_cut(cand, s_n, k, red, turn, &s_n);
+  const int cnt = s_n;                                // at least min(k, n)
+  for (int i = tid; i < cnt; i += SEL_THREADS) {
+    const uint64_t e = cand[i];
+    int rank = 0;
+#pragma unroll 4
+    for (int j = 0; j < cnt; ++j) rank += cand[j] > e;
+    if (rank >= k) continue;
+    const uint32_t r = 0xffffffffu - (uint32_t)e;
+    out_v[(size_t)qi * k + rank] = key2f((uint32_t)(e >> 32));
+    out_i[(size_t)qi * k + rank] = ids ? ids[(size_t)qi * ld + r] : row0 + r;
   }
-  for (int s = kk + tid; s < k; s += 256) { ov[s] = -INFINITY; oi[s] = -1; }
 }
 
-// ------------------------------------------------------------------ fused scan + top-k
+// ------------------------------------------------------------------ IVF: fused scan + top-k
 constexpr int KT_ROWS = 1024;   // rows per workgroup chunk (scores [nqb][KT_ROWS] fp32 in LDS)
 
 // Wave-level exact top-k of sc[0..len) (LDS, len <= KT_ROWS): every lane holds 16 keys in
@@ -155,8 +316,7 @@ constexpr int KT_ROWS = 1024;   // rows per workgroup chunk (scores [nqb][KT_ROW
 // key bytes, and a shuffle-tree sum pays an LDS round trip per level.
 // Writes exactly k slots (ov/oi; -inf / -1 padding when len < k).
 template <int ROWS>
-__device__ __forceinline__ void wave_topk(const float* sc, int len, int k, int64_t row0, const int64_t* ids, float* ov, int64_t* oi,
-                          uint32_t* /*unused*/) {
+__device__ __forceinline__ void wave_topk(const float* sc, int len, int k, int64_t row0, float* ov, int64_t* oi) {
   const int lane = threadIdx.x & 63;
   const int kk = min(k, len);
   uint32_t key[ROWS / 64];
@@ -195,7 +355,7 @@ __device__ __forceinline__ void wave_topk(const float* sc, int len, int k, int64
     }
     if (slot >= 0) {
       ov[slot] = key2f(key[j]);
-      oi[slot] = ids ? ids[row0 + i] : row0 + i;
+      oi[slot] = row0 + i;
     }
     base_gt += __popcll(bg);
     base_eq += __popcll(be);
@@ -203,42 +363,23 @@ __device__ __forceinline__ void wave_topk(const float* sc, int len, int k, int64
   for (int s2 = kk + lane; s2 < k; s2 += 64) { ov[s2] = -INFINITY; oi[s2] = -1; }
 }
 
-// Work item = a chunk of <= ROWS consecutive rows and a set of queries (qsel < 0: all nq, else
-// query qsel only).  Flat: blockIdx.x = chunk, queries all.  IVF (probe != null): blockIdx.x =
+// Work item = a chunk of <= KT_ROWS consecutive rows of a probed list and its query: blockIdx.x =
 // (q * nprobe + j) * maxc + c -> list probe[q][j], its chunk c.  out_v/out_i: [nq][nslots][k].
-// ROWS per workgroup: the scores of all its queries sit in LDS between the scan and the select, so
-// with many queries the chunk is shorter (knn_flat_rows) -- more workgroups resident per CU, one
-// workgroup's select overlapping the others' scans.
-template <int KC, int ROWS>
-__global__ void __launch_bounds__(256) knn_topk_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q,
-                                                       int N, int nq, const float* __restrict__ xnorm2,
+template <int KC>
+__global__ void __launch_bounds__(256) ivf_topk_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q,
+                                                       const float* __restrict__ xnorm2,
                                                        const float* __restrict__ qnorm2,
-                                                       const uint8_t* __restrict__ alive, int k, int row_lo,
+                                                       const uint8_t* __restrict__ alive, int k,
                                                        const int32_t* __restrict__ probe, int nprobe, int maxc,
                                                        const int64_t* __restrict__ list_off, int nslots,
                                                        float* __restrict__ out_v, int64_t* __restrict__ out_i) {
-  constexpr int D = KC * 32;
-  extern __shared__ __attribute__((aligned(16))) float kt_smem[];
+  constexpr int D = KC * 32, ROWS = KT_ROWS, nqb = 1;
+  __shared__ float sc[ROWS];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int lo, hi, q0, nqb, slot;
-  if (probe == nullptr) {
-    lo = row_lo + blockIdx.x * ROWS;
-    hi = min(N, lo + ROWS);
-    q0 = 0;
-    nqb = nq;
-    slot = blockIdx.x;
-  } else {
-    const int c = blockIdx.x % maxc, qj = blockIdx.x / maxc;
-    q0 = qj / nprobe;
-    nqb = 1;
-    slot = (qj % nprobe) * maxc + c;
-    const int l = probe[qj];
-    lo = (int)list_off[l] + c * ROWS;
-    hi = min((int)list_off[l + 1], lo + ROWS);
-  }
+  const int qc = blockIdx.x % maxc, qj = blockIdx.x / maxc;
+  const int q0 = qj / nprobe, slot = (qj % nprobe) * maxc + qc, l = probe[qj];
+  const int lo = (int)list_off[l] + qc * ROWS, hi = min((int)list_off[l + 1], lo + ROWS);
   const int len = max(0, hi - lo);
-  float* sc = kt_smem;                                        // [nqb][ROWS]
-  uint32_t* hist = reinterpret_cast<uint32_t*>(kt_smem + nqb * ROWS) + 256 * w;
   if (len > 0) {
     const int col = lane & 15, g = lane >> 4;
     const bool qv = col < nqb;
@@ -267,173 +408,16 @@ __global__ void __launch_bounds__(256) knn_topk_kernel(const uint16_t* __restric
             float v = acc[i];
             if (xnorm2) v = -(xnorm2[row] + qn - 2.f * v);
             if (alive && !alive[row]) v = -INFINITY;
-            sc[col * ROWS + (row - lo)] = v;
+            sc[row - lo] = v;
           }
         }
       }
     }
   }
   __syncthreads();
-  for (int qi = w; qi < nqb; qi += 4) {
-    const size_t o = ((size_t)(q0 + qi) * nslots + slot) * k;
-    wave_topk<ROWS>(sc + qi * ROWS, len, k, lo, nullptr, out_v + o, out_i + o, hist);
-  }
-}
-
-// ------------------------------------------------------------------ streamed scan + top-k (large k)
-// With a large k the per-chunk candidates of knn_topk_kernel are a big share of the rows (k = 150
-// from 512-row chunks: 29 % of the index written as candidates and read again by the merge).  Here
-// a workgroup (8 waves; two workgroups per CU = 4 waves per SIMD) scans a long span (KS_SPAN rows) in
-// KS_SUB-row sub-chunks and keeps, per query, a
-// candidate buffer in LDS behind a running threshold: only rows scoring above the k-th best key
-// the buffer held at its last cut are appended, and when the next sub-chunk could overflow the
-// buffer it is cut back to its exact top k (the threshold rises).  k candidates per query leave
-// per KS_SPAN rows (0.9 % at k = 150).  Rows equal to the threshold that arrive after a cut are
-// skipped: the buffer already holds k keys >= it, so the result is exact up to tie order.
-constexpr int KS_SUB = 256, KS_CAP = 512, KS_SPAN = 16384;
-
-// keys held KS_CAP / 64 per lane (entry lane + 64 j; 0 = empty): the exact kk-th largest
-__device__ __forceinline__ uint32_t ks_kth(const uint32_t* key, int kk) {
-  uint32_t thr = 0;
-  for (int b = 31; b >= 0; --b) {
-    const uint32_t cand = thr | (1u << b);
-    int c = 0;
-#pragma unroll
-    for (int j = 0; j < KS_CAP / 64; ++j) c += __popcll(__ballot(key[j] >= cand));
-    if (c >= kk) thr = cand;                 // wave-uniform decision
-  }
-  return thr;
-}
-
-// Cut a query's buffer (cnt > kk entries) to its exact top kk, in place (wave-level; every entry is
-// in registers before the first write).  Returns the kk-th largest key (the new threshold).
-__device__ __forceinline__ uint32_t ks_cut(uint32_t* bk, uint32_t* br, int cnt, int kk) {
-  const int lane = threadIdx.x & 63;
-  uint32_t key[KS_CAP / 64], row[KS_CAP / 64];
-#pragma unroll
-  for (int j = 0; j < KS_CAP / 64; ++j) {
-    const int i = lane + 64 * j;
-    key[j] = i < cnt ? bk[i] : 0u;
-    row[j] = i < cnt ? br[i] : 0u;
-  }
-  const uint32_t thr = ks_kth(key, kk);
-  int gt = 0;
-#pragma unroll
-  for (int j = 0; j < KS_CAP / 64; ++j) gt += __popcll(__ballot(key[j] > thr));
-  const uint32_t need = (uint32_t)(kk - gt);
-  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  uint32_t base_gt = 0, base_eq = 0;
-#pragma unroll
-  for (int j = 0; j < KS_CAP / 64; ++j) {
-    const bool g = key[j] > thr, e = key[j] == thr && key[j] != 0u;
-    const uint64_t bg = __ballot(g), be = __ballot(e);
-    int slot = -1;
-    if (g) slot = (int)(base_gt + __popcll(bg & below));
-    else if (e) {
-      const uint32_t q = base_eq + __popcll(be & below);
-      if (q < need) slot = gt + (int)q;
-    }
-    if (slot >= 0) { bk[slot] = key[j]; br[slot] = row[j]; }
-    base_gt += __popcll(bg);
-    base_eq += __popcll(be);
-  }
-  return thr;
-}
-
-template <int KC>
-__global__ void __launch_bounds__(512) knn_topk_stream_kernel(const uint16_t* __restrict__ X,
-                                                              const uint16_t* __restrict__ Q, int N, int nq,
-                                                              const float* __restrict__ xnorm2,
-                                                              const float* __restrict__ qnorm2,
-                                                              const uint8_t* __restrict__ alive, int k, int row_lo,
-                                                              float* __restrict__ out_v, int64_t* __restrict__ out_i) {
-  constexpr int D = KC * 32;
-  __shared__ float sc[16 * KS_SUB];                                        // 16 KB scores
-  __shared__ uint32_t bk[16 * KS_CAP], br[16 * KS_CAP];                     // 64 KB buffers
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int lo = row_lo + blockIdx.x * KS_SPAN, hi = min(N, lo + KS_SPAN);
-  const int col = lane & 15, g = lane >> 4;
-  const bool qv = col < nq;
-  bf16x8_t qf[KC];
-  const uint16_t* qrow = Q + (size_t)(qv ? col : 0) * D;
-#pragma unroll
-  for (int c = 0; c < KC; ++c)
-    qf[c] = as_bf16x8(qv ? *reinterpret_cast<const uint4*>(qrow + 32 * c + 8 * g) : make_uint4(0, 0, 0, 0));
-  const float qn = (qnorm2 && qv) ? qnorm2[col] : 0.f;
-  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  int cnt[2] = {0, 0};                // this wave's queries w, w + 8 (wave-uniform)
-  uint32_t thr[2] = {0u, 0u};
-  for (int s0 = lo; s0 < hi; s0 += KS_SUB) {
-    const int s1 = min(hi, s0 + KS_SUB), len = s1 - s0;
-    const int ngroups = (len + 15) / 16;
-    for (int grp = w; grp < ngroups; grp += 8) {
-      const int r0 = s0 + grp * 16;
-      const int r = min(r0 + col, s1 - 1);
-      const uint16_t* xr = X + (size_t)r * D;
-      uint4 a[KC];
-#pragma unroll
-      for (int c = 0; c < KC; ++c) a[c] = *reinterpret_cast<const uint4*>(xr + 32 * c + 8 * g);
-      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < KC; ++c) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[c]), qf[c], acc, 0, 0, 0);
-      if (qv) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int row = r0 + 4 * g + i;
-          if (row < s1) {
-            float v = acc[i];
-            if (xnorm2) v = -(xnorm2[row] + qn - 2.f * v);
-            if (alive && !alive[row]) v = -INFINITY;
-            sc[col * KS_SUB + (row - s0)] = v;
-          }
-        }
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int qi = w + 8 * t;
-      if (qi < nq) {
-        uint32_t* qk = bk + qi * KS_CAP;
-        uint32_t* qr = br + qi * KS_CAP;
-#pragma unroll
-        for (int j = 0; j < KS_SUB / 64; ++j) {
-          const int i = lane + 64 * j;
-          const uint32_t key = i < len ? f2key(sc[qi * KS_SUB + i]) : 0u;
-          const bool p = i < len && key > thr[t];
-          const uint64_t b = __ballot(p);
-          if (p) {
-            const int slot = cnt[t] + __popcll(b & below);
-            qk[slot] = key;
-            qr[slot] = (uint32_t)(s0 - lo + i);
-          }
-          cnt[t] += __popcll(b);
-        }
-        if (cnt[t] > KS_CAP - KS_SUB) {        // the next sub-chunk might not fit: cut to k (k <= 256)
-          thr[t] = ks_cut(qk, qr, cnt[t], k);
-          cnt[t] = k;
-        }
-      }
-    }
-    __syncthreads();                              // sc is the next sub-chunk's
-  }
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int qi = w + 8 * t;
-    if (qi < nq) {
-      uint32_t* qk = bk + qi * KS_CAP;
-      uint32_t* qr = br + qi * KS_CAP;
-      int n = cnt[t];
-      if (n > k) {
-        ks_cut(qk, qr, n, k);
-        n = k;
-      }
-      const size_t o = ((size_t)qi * gridDim.x + blockIdx.x) * k;
-      for (int s2 = lane; s2 < k; s2 += 64) {
-        out_v[o + s2] = s2 < n ? key2f(qk[s2]) : -INFINITY;
-        out_i[o + s2] = s2 < n ? (int64_t)lo + qr[s2] : -1;
-      }
-    }
+  if (w == 0) {
+    const size_t o = ((size_t)q0 * nslots + slot) * k;
+    wave_topk<ROWS>(sc, len, k, lo, out_v + o, out_i + o);
   }
 }
 
@@ -495,36 +479,45 @@ __global__ void __launch_bounds__(256) pool_kernel(float* __restrict__ out_f32, 
 
 }  // namespace
 
-CFC_API int cfc_knn_scores(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2,
-                           const float* qnorm2, float* out, hipStream_t stream) {
-  if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0) return -1;
-  const int groups = (N + 15) / 16;
-  int blocks = (groups + 3) / 4;
-  if (blocks > 256 * 16) blocks = 256 * 16;
-#define KS(KC) knn_scores_kernel<KC><<<blocks, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, qnorm2, out)
+// Scores of rows [0, N) of X for nq queries into out [nq][ld], and every B rows' largest key into bmax
+// [nq][nb] (null: not wanted).  out 16-byte aligned.
+CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
+                         const uint8_t* alive, float* out, long ld, uint32_t* bmax, int nb, int B, hipStream_t stream) {
+  if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || B < 16 || B % 16 != 0 || (long)nb * B < N || (long)(nb - 1) * B >= N ||
+      ld < N)
+    return -1;
+#define KS(KC) knn_scan_kernel<KC><<<(nb + 3) / 4, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, \
+      qnorm2, alive, out, (size_t)ld, bmax, nb, B); break
   switch (dim / 32) {
-    case 4: KS(4); break;     // 128
-    case 8: KS(8); break;     // 256
-    case 12: KS(12); break;   // 384 (MiniLM, bge-small)
-    case 16: KS(16); break;   // 512
-    case 24: KS(24); break;   // 768 (bge-base, mpnet)
-    case 32: KS(32); break;   // 1024 (bge-large)
+    case 4: KS(4);      // 128
+    case 8: KS(8);      // 256
+    case 12: KS(12);    // 384 (MiniLM, bge-small)
+    case 16: KS(16);    // 512
+    case 24: KS(24);    // 768 (bge-base, mpnet)
+    case 32: KS(32);    // 1024 (bge-large)
     default: return -2;
   }
 #undef KS
   return CFC_CHECK_LAUNCH();
 }
 
-// One radix-select pass: in [nq][n] (row stride ld) -> out [nq][ceil(n/8192)][k].
-CFC_API int cfc_topk_pass(const float* in, const int64_t* idx_in, int nq, int n, int ld, int k, float* out_v,
-                          int64_t* out_i, hipStream_t stream) {
-  if (k <= 0 || k > 2048 || n <= 0) return -1;
-  const int nchunks = (n + TOPK_CHUNK - 1) / TOPK_CHUNK;
-  topk_chunk_kernel<<<dim3(nchunks, nq), 256, 0, stream>>>(in, idx_in, n, ld, k, out_v, out_i);
-  return CFC_CHECK_LAUNCH();
+// Rows per block for the top-k of n scores: as small as the select kernel's number of blocks allows.
+CFC_API int cfc_topk_block(int n) {
+  int b = 16;
+  while ((long)b * SEL_BLOCKS < n) b *= 2;
+  return b;
 }
 
-CFC_API int cfc_topk_chunk_size() { return TOPK_CHUNK; }
+// Sorted top-k of in [nq][n] (row stride ld) -> out [nq][k], k <= n.  bmax [nq][ceil(n / B)], B = cfc_topk_block(n):
+// block maxima from cfc_knn_scan, or (fill) workspace that is filled here.
+CFC_API int cfc_topk_select(const float* in, const int64_t* ids, int nq, int n, long ld, int k, uint32_t* bmax, int fill,
+                            long row0, float* out_v, int64_t* out_i, hipStream_t stream) {
+  if (nq < 1 || k <= 0 || k > SEL_K || k > n || ld < n) return -1;
+  const int B = cfc_topk_block(n), nb = (n + B - 1) / B;
+  if (fill) block_max_kernel<<<dim3((nb + 3) / 4, nq), 256, 0, stream>>>(in, n, (size_t)ld, B, bmax, nb);
+  topk_select_kernel<<<nq, SEL_THREADS, 0, stream>>>(in, n, (size_t)ld, B, bmax, nb, k, ids, row0, out_v, out_i);
+  return CFC_CHECK_LAUNCH();
+}
 
 CFC_API int cfc_l2_normalize(void* out, const void* in, float* norms2, int rows, int dim, hipStream_t stream) {
   if (dim % 8 != 0) return -1;
@@ -541,86 +534,8 @@ CFC_API int cfc_pool(float* out_f32, void* out_bf16, const void* hidden, const i
   return CFC_CHECK_LAUNCH();
 }
 
-namespace {
-// rows per flat-scan workgroup for nq queries and top-k: the [nq][ROWS] fp32 score tile stays at
-// <= 16-32 KB of LDS (several workgroups per CU overlap one chunk's select with the others' scans),
-// and for a large k the chunk grows so the k candidates it emits stay a small share of its rows
-// (the candidate arrays are written and merged: k = 150 from 256-row chunks is 59 % of the index).
-// Measured on 100M x 384: 1 query 2048 rows 12.6 ms (6.1 TB/s) vs 1024 rows 14.1 ms; 16 queries
-// 256 rows 14.1 ms vs 1024 rows 23.6 ms (k = 10), 512 rows 20.7 ms vs 256 rows 22.8 ms (k = 150).
-// k > 32 and more than 4 queries: the streamed kernel, k candidates per KS_SPAN rows (up to 4
-// queries the 2048-row chunks already keep k = 150 at 7 % of the rows, and the streamed kernel's two
-// workgroups per CU scan slower: 1 query, k = 150: 14.8 ms vs 12.6, profiles/r04_bench_knn_*).
-constexpr int knn_flat_rows(int nq, int k) {
-  return nq <= 4 ? 2048 : k > 32 ? KS_SPAN : nq <= 8 ? 512 : 256;
-}
-
-template <int KC>
-int knn_topk_launch(const void* X, const void* Q, int N, int nq, const float* xnorm2, const float* qnorm2,
-                    const uint8_t* alive, int k, int row_lo, const int32_t* probe, int nprobe, int maxc,
-                    const int64_t* list_off, int nslots, float* out_v, int64_t* out_i, int blocks, int nqb,
-                    int rows, hipStream_t stream) {
-  const size_t lds = (size_t)nqb * rows * 4 + 4 * 256 * 4;
-#define KTL(R) knn_topk_kernel<KC, R><<<blocks, 256, lds, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, \
-      xnorm2, qnorm2, alive, k, row_lo, probe, nprobe, maxc, list_off, nslots, out_v, out_i)
-  switch (rows) {
-    case 2048: KTL(2048); break;
-    case 1024: KTL(1024); break;
-    case 512: KTL(512); break;
-    case 256: KTL(256); break;
-    default: return -3;
-  }
-#undef KTL
-  return CFC_CHECK_LAUNCH();
-}
-
-int knn_topk_dispatch(int dim, const void* X, const void* Q, int N, int nq, const float* xnorm2, const float* qnorm2,
-                      const uint8_t* alive, int k, int row_lo, const int32_t* probe, int nprobe, int maxc,
-                      const int64_t* list_off, int nslots, float* out_v, int64_t* out_i, int blocks, int nqb,
-                      int rows, hipStream_t stream) {
-#define KT(KC) return knn_topk_launch<KC>(X, Q, N, nq, xnorm2, qnorm2, alive, k, row_lo, probe, nprobe, maxc, \
-                                          list_off, nslots, out_v, out_i, blocks, nqb, rows, stream)
-  switch (dim / 32) {
-    case 4: KT(4);
-    case 8: KT(8);
-    case 12: KT(12);
-    case 16: KT(16);
-    case 24: KT(24);
-    case 32: KT(32);
-    default: return -2;
-  }
-#undef KT
-}
-}  // namespace
-
-// Flat index, rows [row_lo, N): candidates out [nq][ceil((N - row_lo) / cfc_knn_flat_rows(nq, k))][k]
-// (unsorted within a chunk; merge with cfc_topk_pass).  nq <= 16, k <= 256; alive: optional uint8 row mask.
-CFC_API int cfc_knn_topk(const void* X, const void* Q, int N, int row_lo, int nq, int dim, const float* xnorm2,
-                         const float* qnorm2, const uint8_t* alive, int k, float* out_v, int64_t* out_i,
-                         hipStream_t stream) {
-  if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= row_lo || row_lo < 0 || k < 1 || k > 256) return -1;
-  const int rows = knn_flat_rows(nq, k);
-  const int nch = (N - row_lo + rows - 1) / rows;
-  if (rows == KS_SPAN) {
-#define KS(KC) \
-  case KC: \
-    knn_topk_stream_kernel<KC><<<nch, 512, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, qnorm2, \
-                                                       alive, k, row_lo, out_v, out_i); \
-    return CFC_CHECK_LAUNCH();
-    switch (dim / 32) {
-      KS(4) KS(8) KS(12) KS(16) KS(24) KS(32)
-      default: return -2;
-    }
-#undef KS
-  }
-  return knn_topk_dispatch(dim, X, Q, N, nq, xnorm2, qnorm2, alive, k, row_lo, nullptr, 1, 1, nullptr, nch, out_v,
-                           out_i, nch, nq, rows, stream);
-}
-
 // rows per IVF list chunk (one workgroup each)
 CFC_API int cfc_knn_topk_rows() { return KT_ROWS; }
-// rows per flat-scan workgroup for nq queries and top-k (the candidate count of cfc_knn_topk)
-CFC_API int cfc_knn_flat_rows(int nq, int k) { return knn_flat_rows(nq, k); }
 
 // IVF: probe [nq][nprobe] list ids, list_off [nlist + 1] row offsets (rows grouped by list), maxc =
 // max chunks of any list.  One launch of nq * nprobe * maxc workgroups; candidates out
@@ -631,6 +546,17 @@ CFC_API int cfc_ivf_topk(const void* X, const void* Q, int N, int nq, int dim, c
   if (nq < 1 || nprobe < 1 || maxc < 1 || dim % 32 != 0 || k < 1 || k > 256) return -1;
   const long blocks = (long)nq * nprobe * maxc;
   if (blocks > (1L << 30)) return -1;
-  return knn_topk_dispatch(dim, X, Q, N, nq, xnorm2, qnorm2, alive, k, 0, probe, nprobe, maxc, list_off,
-                           nprobe * maxc, out_v, out_i, (int)blocks, 1, KT_ROWS, stream);
+#define KT(KC) ivf_topk_kernel<KC><<<(int)blocks, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, xnorm2, qnorm2, alive, k, \
+      probe, nprobe, maxc, list_off, nprobe * maxc, out_v, out_i); break
+  switch (dim / 32) {
+    case 4: KT(4);
+    case 8: KT(8);
+    case 12: KT(12);
+    case 16: KT(16);
+    case 24: KT(24);
+    case 32: KT(32);
+    default: return -2;
+  }
+#undef KT
+  return CFC_CHECK_LAUNCH();
 }
