@@ -39,7 +39,7 @@ CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function"]
 # per-source additions.  attention.hip: no NaN ever enters the softmax (masked scores are -inf,
 # which stays honoured), and without NaN semantics fmaxf needs no canonicalising v_max_f32 in front
 # of every MFMA output it reads -- 33 fewer VALU instructions per prefill KV tile
-FILE_FLAGS = {"attention.hip": ["-fno-honor-nans"]}
+FILE_FLAGS = {"attention.hip": ["-fno-honor-nans"], "encoder.hip": ["-fno-honor-nans"]}
 
 KERNELS_LIB = LIB_DIR / "libcfc_kernels.so"
 RUNTIME_LIB = LIB_DIR / "libcfc_runtime.so"

@@ -15,6 +15,7 @@ hundreds of chunks per forward:
 from __future__ import annotations
 
 import dataclasses
+import itertools
 import math
 import os
 from pathlib import Path
@@ -149,6 +150,10 @@ class EncoderModel:
                        tiles=None) -> torch.Tensor:
         """Token states [T, H] for packed varlen input."""
         c = self.cfg
+        if (ids.is_cuda and tiles is not None and os.environ.get("CFC_ENCODER_GEMM", "auto") == "auto"
+                and os.environ.get("CFC_ENCODER_LN_FUSED", "1") != "0"
+                and K.encoder_forward_ok(ids.numel(), self.p, self.layers, c.heads, max_seqlen)):
+            return K.encoder_forward(ids, positions, self.p, self.layers, cu_seqlens, tiles, c.heads, max_seqlen, self.scale, c.ln_eps)
         x = K.embed_layernorm(ids, positions, self.p["word"], self.p["pos"], self.p["type"], self.p["emb_g"],
                               self.p["emb_b"], c.ln_eps)
         lin = self._linear
@@ -190,6 +195,18 @@ class EncoderModel:
             return K.pgemm_ln(x, w, bias, residual, gamma, beta, eps)
         return K.layernorm(self._linear(x, w), gamma, beta, eps, bias=bias, residual=residual)
 
+    def _h2d(self, *arrays) -> list[torch.Tensor]:
+        """The arrays as int32 tensors on the device, by one copy from pinned memory: a copy from pageable memory holds the
+        host until the stream has come to it, so a batch would be prepared after the one before it and not beside it."""
+        import numpy as np
+        at = np.cumsum([0] + [-(-len(a) // 4) * 4 for a in arrays])
+        buf = torch.empty(int(at[-1]), dtype=torch.int32, pin_memory=self.device.type == "cuda")
+        flat = buf.numpy()
+        for o, a in zip(at, arrays):
+            flat[o:o + len(a)] = a
+        d = buf.to(self.device, non_blocking=True)
+        return [d[o:o + len(a)] for o, a in zip(at, arrays)]
+
     @torch.inference_mode()
     def encode_ids(self, batch: list[list[int]], pooling: str | None = None, normalize: bool | None = None,
                    max_tokens_per_forward: int = 65536) -> torch.Tensor:
@@ -198,7 +215,7 @@ class EncoderModel:
         seqs = [s[:self.cfg.max_seq_length] for s in batch]
         cu = np.zeros(len(seqs) + 1, dtype=np.int32)
         np.cumsum([len(s) for s in seqs], out=cu[1:])
-        ids = np.fromiter((t for s in seqs for t in s), dtype=np.int32, count=int(cu[-1]))
+        ids = np.fromiter(itertools.chain.from_iterable(seqs), dtype=np.int32, count=int(cu[-1]))
         return self.encode_packed(ids, cu, pooling, normalize, max_tokens_per_forward)
 
     @torch.inference_mode()
@@ -225,12 +242,11 @@ class EncoderModel:
             j = int(np.searchsorted(cu, cu[i] + max_tokens_per_forward, side="right")) - 1
             j = min(max(j, i + 1), n)
             t0, t1 = int(cu[i]), int(cu[j])
-            cu_part = (cu[i:j + 1] - t0).astype(np.int32)
-            seq_t, q0_t = K.prefill_tiles(cu_part.tolist(), K.ENCODER_TILE_ROWS)
-            tiles = (torch.tensor(seq_t, dtype=torch.int32, device=dev), torch.tensor(q0_t, dtype=torch.int32, device=dev))
-            cu_t = torch.from_numpy(cu_part).to(dev)
-            h = self.forward_packed(torch.from_numpy(ids[t0:t1]).to(dev), torch.from_numpy(pos_all[t0:t1]).to(dev),
-                                    cu_t, int(lens[i:j].max()), tiles=tiles)
+            per = -(-lens[i:j] // K.ENCODER_TILE_ROWS)          # query tiles of each sequence
+            seq_t = np.repeat(np.arange(j - i), per)
+            q0_t = (np.arange(len(seq_t)) - np.repeat(np.cumsum(per) - per, per)) * K.ENCODER_TILE_ROWS
+            ids_t, pos_t, cu_t, *tiles = self._h2d(ids[t0:t1], pos_all[t0:t1], cu[i:j + 1] - t0, seq_t, q0_t)
+            h = self.forward_packed(ids_t, pos_t, cu_t, int(lens[i:j].max()), tiles=tuple(tiles))
             outs.append(K.pool(h, cu_t, pooling, normalize))
             i = j
         return torch.cat(outs, 0)

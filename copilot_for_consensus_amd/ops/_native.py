@@ -96,6 +96,8 @@ _KERNEL_SIGS = {
     "cfc_prefill_attention_expanded2": [P, c_int64, c_int64, P, P, P, P, P, c_int64, P, P, P, P, I, I, F, I, P, P, c_int64, P,
                                         c_int64, P],
     "cfc_prefill_attention_expanded": [P, P, P, P, c_int64, P, P, P, P, I, I, F, P, c_int64, P],
+    "cfc_enc_rows": [I],
+    "cfc_enc_forward": [P] * 10 + [I, I, I, I, P, I, F, F, I] + [P] * 6,
     "cfc_knn_scan": [P, P, I, I, I, P, P, P, P, L, P, I, I, P],
     "cfc_topk_block": [I],
     "cfc_topk_select": [P, P, I, I, L, I, P, I, L, P, P, P],

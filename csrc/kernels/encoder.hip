@@ -1,0 +1,615 @@
+// Sentence-encoder layers for gfx950, post-LN BERT with hidden 384 and inner 1536 (MiniLM-L6, bge-small), bf16 in and out:
+//   x1 = LN(a Wo^T + bo + x), h = GELU(x1 Wu^T + bu), y = LN(h Wd^T + bd + x1), qkv = y Wq^T + bq
+// around the attention (attention.hip).
+//
+// Many rows: one kernel from the attention's output to the layer's.  Product by product these have K = 384 or 1536 and
+// outputs up to four times their inputs: over 65 k rows 311 us (o 45, up 155, down 110), 600 MB of rows written and read
+// again, each tile's epilogue alone on its CU.  Here a row never leaves its lane between them, 226 us:
+//
+//   * a workgroup owns 128 rows, a wave 32.  v_mfma_f32_32x32x16_bf16 with the WEIGHTS as A and the rows as
+//     B: a lane's accumulators are columns of ONE row (lane & 31), half of them its own, half those of
+//     lane ^ 32, so a LayerNorm is a sum over the lane's registers and one lane swap;
+//   * the accumulator layout of one product becomes the B operand of the next by packing to bf16 and one
+//     v_permlane32_swap per two registers (frag_of): rows, hidden rows and residuals stay in registers
+//     (96 for a 384-wide bf16 row block, 192 for its fp32 accumulators: one wave per SIMD);
+//   * only the weights move: steps of two 24-KB stages of 24 fragments (32 columns x 384, or 384 columns x 32),
+//     three in a ring of LDS-DMA behind counted waits, one barrier per step of 48 MFMAs;
+//   * in the feed-forward's step c the up product of columns c and the down product over columns c - 2 take turns,
+//     GELU of columns c - 1 spread between them.
+// What bounds it: a wave alone on its SIMD issues an instruction every six cycles or so, and a step has 575 of them
+// (48 MFMAs, as many LDS reads and waits, 270 of GELU): 85 us for a block of rows on an idle chip, 115 with all CUs at
+// work and the clock down (matrix cores alone 52).  Half-steps of one stage in a ring of six, two elements' GELU at a
+// time, and the projections in the same kernel were each slower: their registers spill, or their order stalls.
+#include "common.h"
+
+namespace {
+
+typedef __attribute__((address_space(3))) void en_lds_t;
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+constexpr int EN_H = 384, EN_F = 1536;           // hidden, inner
+constexpr int EN_T = EN_H / 32;                  // 32-column tiles of a row
+constexpr int EN_S = EN_H / 16;                  // 16-deep k steps of a row
+constexpr int EN_ROWS = 128;                     // rows per workgroup, 32 per wave
+constexpr int EN_STAGE = 24 * 1024, EN_STEP = 2 * EN_STAGE, EN_RING = 3;
+constexpr int EN_PIECES = 12;                    // DMA pieces (1 KB) per wave and step
+constexpr int EN_LDS = EN_RING * EN_STEP + 4 * EN_F;
+
+__device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// One 1-KB LDS-DMA piece: lane l's 16 bytes of sbase + voff land at lds_addr + 16 l (M0 kept).
+__device__ __forceinline__ void en_glds16(uint32_t voff, const void* sbase, uint32_t lds_addr) {
+  unsigned keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(voff), "s"(sbase), "s"(lds_addr)
+      : "memory");
+}
+
+// x Phi(x) = max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, erfc by Abramowitz and Stegun 7.1.26 (as pgemm.hip's), in three
+// parts of about an MFMA's length.
+struct Gelu { float t, m, q; };
+__device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
+template <int PART>
+__device__ __forceinline__ void en_gelu(Gelu& g, float& v) {
+  if constexpr (PART == 0) {
+    pin(v);
+    g.t = __builtin_amdgcn_rcpf(fmaf(fabsf(v), 0.3275911f * 0.70710678f, 1.f));
+    g.m = v * v * (-0.5f * 1.44269504f);
+    pin(g.t);
+    pin(g.m);
+  } else if constexpr (PART == 1) {
+    pin(g.m);
+    const float e = __builtin_amdgcn_exp2f(g.m);
+    float q = fmaf(g.t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
+    q = fmaf(q, g.t, 0.5f * 1.421413741f);
+    q = fmaf(q, g.t, 0.5f * -0.284496736f);
+    q = fmaf(q, g.t, 0.5f * 0.254829592f) * g.t;
+    g.q = q * e;
+    pin(g.q);
+  } else {
+    pin(g.q);
+    v = fmaf(-fabsf(v), g.q, fmaxf(v, 0.f));
+    pin(v);
+  }
+}
+
+// Sixteen columns of a row block between its two layouts, its own inverse.  Accumulators: a lane holds columns
+// 4 hi + 0..3 and 8 + 4 hi + 0..3 (hi = lane >> 5); operands: columns 8 hi + 0..7.
+__device__ __forceinline__ u32x4_t trade(u32x4_t v) {
+  const auto p = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
+  const auto q = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+  return u32x4_t{p[0], q[0], p[1], q[1]};
+}
+
+// accumulators 8 s .. 8 s + 7 of a tile -> operand of k step s
+__device__ __forceinline__ bf16x8_t frag_of(const f32x16_t& a, int s) {
+  const u32x4_t v = {pack2bf(a[8 * s], a[8 * s + 1]), pack2bf(a[8 * s + 2], a[8 * s + 3]), pack2bf(a[8 * s + 4], a[8 * s + 5]),
+                     pack2bf(a[8 * s + 6], a[8 * s + 7])};
+  return __builtin_bit_cast(bf16x8_t, trade(v));
+}
+
+struct EncLayer {
+  const uint16_t *wo, *bo, *g1, *b1, *wu, *bu, *wd, *bd, *g2, *b2;
+};
+
+// out(t, y): tile t of LN over the row of (acc + bias + residual), gamma and beta.  res(k): the residual's operand of
+// k step k.  A tile at a time, the sums kept in accumulation registers between the passes: 192 of them beside the
+// row's operands do not fit the others.
+template <class R, class O>
+__device__ __forceinline__ void en_norm(f32x16_t (&acc)[EN_T], R&& res, const uint16_t* __restrict__ bias,
+                                        const uint16_t* __restrict__ gamma, const uint16_t* __restrict__ beta, float eps, O&& out) {
+  const int hi = (threadIdx.x >> 5) & 1;
+  auto four = [&](const uint16_t* p, int t, int i, float (&v)[4]) {
+    const uint2 b = *reinterpret_cast<const uint2*>(p + 32 * t + 8 * i + 4 * hi);
+    v[0] = __uint_as_float(b.x << 16); v[1] = __uint_as_float(b.x & 0xffff0000u);
+    v[2] = __uint_as_float(b.y << 16); v[3] = __uint_as_float(b.y & 0xffff0000u);
+  };
+  float sum = 0.f;
+#pragma unroll
+  for (int t = 0; t < EN_T; ++t) {
+    f32x16_t y = acc[t];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const u32x4_t r = trade(__builtin_bit_cast(u32x4_t, res(2 * t + s)));
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float b[4];
+        four(bias, t, 2 * s + i, b);
+        const float v[4] = {__uint_as_float(r[2 * i] << 16), __uint_as_float(r[2 * i] & 0xffff0000u),
+                            __uint_as_float(r[2 * i + 1] << 16), __uint_as_float(r[2 * i + 1] & 0xffff0000u)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          y[8 * s + 4 * i + e] += b[e] + v[e];
+          sum += y[8 * s + 4 * i + e];
+        }
+      }
+    }
+    asm volatile("" : "+a"(y));
+    acc[t] = y;
+    if (t % 2) __builtin_amdgcn_sched_barrier(0);
+  }
+  const float mean = xor32_sum(sum) * (1.f / EN_H);
+  float var = 0.f;
+#pragma unroll
+  for (int t = 0; t < EN_T; ++t) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float d = acc[t][r] - mean;
+      var += d * d;
+    }
+    asm volatile("" : "+a"(acc[t]));
+    if (t % 2) __builtin_amdgcn_sched_barrier(0);
+  }
+  const float rstd = rsqrtf(xor32_sum(var) * (1.f / EN_H) + eps);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int t = 0; t < EN_T; ++t) {
+    f32x16_t y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float g[4], b[4];
+      four(gamma, t, i, g);
+      four(beta, t, i, b);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[4 * i + e] = (acc[t][4 * i + e] - mean) * rstd * g[e] + b[e];
+    }
+    out(t, y);
+    if (t % 2) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Steps of the weight stream: 6 of Wo (two 32-deep slices each), 50 of the feed-forward (up columns c, down
+// slice c - 2).
+constexpr int EN_O = EN_T / 2, EN_C = EN_F / 32, EN_STEPS = EN_O + EN_C + 2;
+constexpr int EN_AHEAD = 8;                      // fragments read ahead of their MFMA
+
+__global__ void __launch_bounds__(256, 1)
+    enc_layer_kernel(const uint16_t* __restrict__ att, const uint16_t* x, EncLayer L, uint16_t* xout, int M, float eps) {
+  // xout may be x: a row is read and written by its own lanes alone (lanes past M read row M - 1, to no use)
+  extern __shared__ __attribute__((aligned(16))) char en_smem[];
+  const int lane = threadIdx.x & 63, hi = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = blockIdx.x * EN_ROWS + w * 32 + (lane & 31);
+
+  // ---- weight stream.  Slices (384 rows x 64 B): pieces of 16 rows, 16-byte chunk c of row r at slot
+  // c ^ f((r >> 2) & 3); column groups (32 rows x 768 B): pieces of 8 rows x 128 B, chunk c at slot c ^ (r & 7).
+  // Both are read without bank conflicts, 8 lanes of consecutive rows at a time.  Wave w brings pieces
+  // 6 w .. 6 w + 5 of either stage.
+  const int srow = lane >> 2, sch = (lane & 3) ^ ((4 - ((srow >> 2) & 3)) & 3);
+  const uint32_t v_o = srow * EN_H * 2 + sch * 16, v_d = srow * EN_F * 2 + sch * 16;
+  const uint32_t v_n = (lane >> 3) * EN_H * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(en_lds_t*)en_smem);
+  const uint32_t own = w * (EN_PIECES / 2) * 1024;
+  const char* wo = reinterpret_cast<const char*>(L.wo) + (size_t)w * (EN_PIECES / 2) * 16 * EN_H * 2;
+  const char* wd = reinterpret_cast<const char*>(L.wd) + (size_t)w * (EN_PIECES / 2) * 16 * EN_F * 2;
+  const char* wu = reinterpret_cast<const char*>(L.wu);
+  auto piece = [&](int t, int q) {                // piece q (0 .. 11) of this wave in step t
+    const int i = q % (EN_PIECES / 2), h = q / (EN_PIECES / 2);
+    const uint32_t at = lds0 + (t % EN_RING) * EN_STEP + h * EN_STAGE + own + i * 1024;
+    if (t < EN_O) {
+      en_glds16(v_o, wo + 64 * (2 * t + h) + i * (16 * EN_H * 2), at);
+    } else if (h == 0) {                          // at the ends, columns and slices that are not used
+      const int p = w * (EN_PIECES / 2) + i;
+      en_glds16(v_n, wu + (size_t)min(t - EN_O, EN_C - 1) * (32 * EN_H * 2) + (p & 3) * (8 * EN_H * 2) + (p >> 2) * 128, at);
+    } else {
+      en_glds16(v_d, wd + 64 * max(t - EN_O - 2, 0) + i * (16 * EN_F * 2), at);
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < EN_PIECES; ++q) piece(0, q);
+#pragma unroll
+  for (int q = 0; q < EN_PIECES; ++q) piece(1, q);
+
+  // ---- fragments: of a slice, tile n and k step s at index 12 s + n; of a group, k step s
+  const int r32 = lane & 31, f = (4 - ((r32 >> 2) & 3)) & 3;
+  const int so[2] = {r32 * 64 + ((hi ^ f) << 4), r32 * 64 + (((2 + hi) ^ f) << 4)};
+  int go[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) go[s] = r32 * 128 + (((2 * s + hi) ^ (r32 & 7)) << 4);
+  enum { SS, GS };                                // a step's two stages: slices, a group and a slice
+  // Fragment i (0 .. 47) of a step: two slices one after the other, else the two stages in turn.  One address
+  // per lane offset and step, the rest in the instruction's offset.
+  struct Stage { uint32_t s[2], g[4]; };
+  auto at = [&](int t) {
+    const uint32_t base = lds0 + (t % EN_RING) * EN_STEP;
+    Stage p;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) p.s[s] = base + so[s];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) p.g[s] = base + go[s];
+    return p;
+  };
+  auto frag = [&](const Stage& p, int kind, int i) {
+    const int h = kind == SS ? i / 24 : i & 1, j = kind == SS ? i % 24 : i >> 1;
+    const bool g = kind == GS && h == 0;
+    typedef const __attribute__((address_space(3))) bf16x8_t* lds_frag_t;
+    return *reinterpret_cast<lds_frag_t>((g ? p.g[j & 3] : p.s[j / EN_T]) + (uint32_t)(h * EN_STAGE + (g ? (j >> 2) * 4096 : (j % EN_T) * 2048)));
+  };
+  // One step: its MFMAs in order, each followed by the read of the fragment EN_AHEAD later (from the next step's
+  // stages at the end, behind the barrier that says they are there) and a share of vector work, and every third
+  // by a DMA piece of the step after the next, into the place of the step before.  The order is fixed: left to
+  // itself the compiler reads fragments just ahead of their use and waits for each.
+  bf16x8_t fr[EN_AHEAD];
+  auto run = [&](int t, Stage& st, int kind, int next, auto&& mma, auto&& work) {
+    Stage nst = st;
+#pragma unroll
+    for (int i = 0; i < 48; ++i) {
+      if (i == 48 - EN_AHEAD && t + 1 < EN_STEPS) {
+        // step t + 1's weights are in LDS in every wave, and step t's in registers
+        if (t + 2 < EN_STEPS) asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        nst = at(t + 1);
+      }
+      mma(i, fr[i % EN_AHEAD]);
+      if (i + EN_AHEAD < 48) fr[i % EN_AHEAD] = frag(st, kind, i + EN_AHEAD);
+      else if (t + 1 < EN_STEPS) fr[i % EN_AHEAD] = frag(nst, next, i + EN_AHEAD - 48);
+      if (i % 3 == 2 && i < 3 * EN_PIECES && t + 2 < EN_STEPS) piece(t + 2, i / 3);
+      work(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    st = nst;
+  };
+
+  // ---- biases of the up product, fp32 in LDS behind the ring
+  float* bu = reinterpret_cast<float*>(en_smem + EN_RING * EN_STEP);
+  bf16x8_t xf[EN_S];                              // the row block as operands
+  {
+    const uint16_t* ar = att + (size_t)min(row, M - 1) * EN_H + 8 * hi;
+#pragma unroll
+    for (int s = 0; s < EN_S; ++s) xf[s] = *reinterpret_cast<const bf16x8_t*>(ar + 16 * s);
+  }
+  for (int i = threadIdx.x; i < EN_F; i += 256) bu[i] = bf2f(L.bu[i]);      // read after later barriers
+
+  f32x16_t acc[EN_T];
+  auto clear = [&]() {
+#pragma unroll
+    for (int t = 0; t < EN_T; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+  };
+  clear();
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  Stage st = at(0);
+#pragma unroll
+  for (int i = 0; i < EN_AHEAD; ++i) fr[i] = frag(st, SS, i);
+#pragma unroll
+  for (int t = 0; t < EN_O; ++t)
+    run(t, st, SS, t + 1 < EN_O ? SS : GS, [&](int i, bf16x8_t a) {
+      acc[i % EN_T] = mfma32(a, xf[4 * t + i / EN_T], acc[i % EN_T]);
+    }, [](int) {});
+  {
+    const uint16_t* xr = x + (size_t)min(row, M - 1) * EN_H + 8 * hi;
+    en_norm(acc, [&](int s) { return *reinterpret_cast<const bf16x8_t*>(xr + 16 * s); }, L.bo, L.g1, L.b1, eps, [&](int t, const f32x16_t& y) {
+      xf[2 * t] = frag_of(y, 0);
+      xf[2 * t + 1] = frag_of(y, 1);
+    });
+  }
+  clear();
+
+  // ---- feed-forward: in step c the up product of columns c, GELU of columns c - 1, the down product over c - 2
+  bf16x8_t h[2];
+  f32x16_t up;
+  Gelu ge;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) up[r] = 0.f;
+  h[0] = h[1] = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});       // the first two steps add zeros
+  for (int c = 0; c < EN_C + 2; ++c) {
+    f32x16_t nx;                                  // 32 columns, from their biases
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float4 v = *reinterpret_cast<const float4*>(bu + 32 * min(c, EN_C - 1) + 8 * i + 4 * hi);
+      nx[4 * i] = v.x; nx[4 * i + 1] = v.y; nx[4 * i + 2] = v.z; nx[4 * i + 3] = v.w;
+    }
+    run(EN_O + c, st, GS, GS, [&](int i, bf16x8_t a) {
+      if (i & 1) acc[(i >> 1) % EN_T] = mfma32(a, h[(i >> 1) / EN_T], acc[(i >> 1) % EN_T]);
+      else nx = mfma32(a, xf[i >> 1], nx);
+    }, [&](int i) {
+      // an element's GELU over three MFMAs, pinned there: nothing else spreads it under them
+      float v = up[i / 3];
+      if (i % 3 == 0) en_gelu<0>(ge, v);
+      if (i % 3 == 1) en_gelu<1>(ge, v);
+      if (i % 3 == 2) en_gelu<2>(ge, v);
+      up[i / 3] = v;
+    });
+    h[0] = frag_of(up, 0);
+    h[1] = frag_of(up, 1);
+    up = nx;
+  }
+  uint16_t* o = xout + (size_t)row * EN_H + 8 * hi;
+  en_norm(acc, [&](int s) { return xf[s]; }, L.bd, L.g2, L.b2, eps, [&](int t, const f32x16_t& y) {
+    const bf16x8_t a = frag_of(y, 0), b = frag_of(y, 1);
+    if (row < M) {
+      *reinterpret_cast<bf16x8_t*>(o + 32 * t) = a;
+      *reinterpret_cast<bf16x8_t*>(o + 32 * t + 16) = b;
+    }
+  });
+}
+
+// ---- y = x W^T + b for a 384-wide x and W of 32 N32 rows (the attention's projections), the same way: rows in registers
+// as B operands, W in column groups through a ring of three stages.  No accumulators to hold beside them, so two
+// workgroups share a CU and one's waits are the other's matrix time.  65 k rows x 1152 in 67 us, 256 x 256 tiles of
+// both operands in LDS took 112.
+constexpr int EP_RING = 3;
+
+__global__ void __launch_bounds__(256, 2)
+    enc_proj_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ W, const uint16_t* __restrict__ bias,
+                    uint16_t* __restrict__ out, int M, int groups) {
+  __shared__ __attribute__((aligned(16))) char smem[EP_RING * EN_STAGE];
+  const int lane = threadIdx.x & 63, hi = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = blockIdx.x * EN_ROWS + w * 32 + (lane & 31);
+  const uint32_t v_n = (lane >> 3) * EN_H * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(en_lds_t*)smem);
+  auto issue = [&](int n, uint32_t place) {       // rows 32 n .. of W; past the end, of no use
+    const char* src = reinterpret_cast<const char*>(W) + (size_t)min(n, groups - 1) * (32 * EN_H * 2);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      const int p = 6 * w + i;
+      en_glds16(v_n, src + (p & 3) * (8 * EN_H * 2) + (p >> 2) * 128, place + p * 1024);
+    }
+  };
+  issue(0, lds0);
+  issue(1, lds0 + EN_STAGE);
+  bf16x8_t xf[EN_S];
+  {
+    const uint16_t* xr = x + (size_t)min(row, M - 1) * EN_H + 8 * hi;
+#pragma unroll
+    for (int s = 0; s < EN_S; ++s) xf[s] = *reinterpret_cast<const bf16x8_t*>(xr + 16 * s);
+  }
+  const int r32 = lane & 31;
+  uint32_t go[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) go[s] = r32 * 128 + (((2 * s + hi) ^ (r32 & 7)) << 4);
+  uint16_t* o = out + (size_t)row * 32 * groups + 8 * hi;
+  uint32_t here = lds0, before = lds0 + (EP_RING - 1) * EN_STAGE;
+  auto four = [&](int n, int i, f32x16_t& a) {
+    const uint2 b = *reinterpret_cast<const uint2*>(bias + 32 * n + 8 * i + 4 * hi);
+    a[4 * i] = __uint_as_float(b.x << 16); a[4 * i + 1] = __uint_as_float(b.x & 0xffff0000u);
+    a[4 * i + 2] = __uint_as_float(b.y << 16); a[4 * i + 3] = __uint_as_float(b.y & 0xffff0000u);
+  };
+  for (int n = 0; n < groups; ++n) {
+    // group n is in LDS in every wave, and group n - 1 read: the one after the next takes its place.  Stores of the
+    // group before are younger than its pieces: the count is safe with them.
+    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    issue(n + 2, before);
+    uint32_t a[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) { a[s] = here + go[s]; asm volatile("" : "+v"(a[s])); }
+    auto frag = [&](int i) {
+      typedef const __attribute__((address_space(3))) bf16x8_t* lds_frag_t;
+      return *reinterpret_cast<lds_frag_t>(a[i & 3] + (uint32_t)((i >> 2) * 4096));
+    };
+    f32x16_t acc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) four(n, i, acc);
+    bf16x8_t fr[EN_AHEAD];
+#pragma unroll
+    for (int i = 0; i < EN_AHEAD; ++i) fr[i] = frag(i);
+#pragma unroll
+    for (int i = 0; i < EN_S; ++i) {
+      acc = mfma32(fr[i % EN_AHEAD], xf[i], acc);
+      if (i + EN_AHEAD < EN_S) fr[i % EN_AHEAD] = frag(i + EN_AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const bf16x8_t y0 = frag_of(acc, 0), y1 = frag_of(acc, 1);
+    if (row < M) {
+      *reinterpret_cast<bf16x8_t*>(o + 32 * n) = y0;
+      *reinterpret_cast<bf16x8_t*>(o + 32 * n + 16) = y1;
+    }
+    before = here;
+    here = here == lds0 + (EP_RING - 1) * EN_STAGE ? lds0 : here + EN_STAGE;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // the stream runs past its end
+}
+
+// ================================================================ few rows
+// A query or a few texts would leave most CUs idle above, and one CU brings in no more than some 30 bytes a
+// nanosecond: a layer's 3.5 MB of weights have to be spread over many.  All four products run in tiles of 64 rows and
+// 64 or 16 columns; what a LayerNorm follows leaves unnormed, and every tile of the next product norms its rows itself
+// (a launch less, and rows that few are in every L2).  A query of 12 tokens takes 27 us a layer, attention
+// included, where tiles of 256 and 128 rows took 75.
+
+// What the next product reads: x, or LN(proj + bias + res) rounded to bf16, which the first column's tiles also
+// store to x for the next residual.
+struct EncNorm {
+  const uint16_t *proj, *bias, *res, *gamma, *beta;
+  float eps;
+};
+
+// y = x W^T + b (GELU: x Phi(x) of it) for a 384-wide x and a W of N rows.  A wave owns 16 columns: its fragments of W
+// go straight to registers, all in flight before the tile's rows are staged.
+template <bool GELU, bool LN>
+__global__ void __launch_bounds__(256) enc_tile_kernel(uint16_t* x, EncNorm ln, const uint16_t* __restrict__ W,
+                                                       const uint16_t* __restrict__ bias, uint16_t* __restrict__ out, int M, int N) {
+  constexpr int CH = EN_H / 8, KS = EN_H / 32;    // 16-byte chunks of a row, k steps
+  __shared__ __attribute__((aligned(16))) char smem[64 * EN_H * 2];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 64 + 16 * w, m0 = blockIdx.y * 64, rows = min(64, M - m0);
+  uint4 wf[KS];
+  const uint16_t* wr = W + (size_t)(n0 + r16) * EN_H + 8 * g;
+#pragma unroll
+  for (int k = 0; k < KS; ++k) wf[k] = *reinterpret_cast<const uint4*>(wr + 32 * k);
+  const uint2 bb = *reinterpret_cast<const uint2*>(bias + n0 + 4 * g);
+  // chunk c of row r at slot c ^ (r & 7): 16-row fragment reads without bank conflicts
+  if constexpr (LN) {
+    // a wave per row, chunk `lane` of it in lanes 0 .. 47; four rows' loads at a time
+    const bool on = lane < CH;
+    const int c = on ? lane : 0;
+    float pb[8], ga[8], be[8];
+    unpack8(*reinterpret_cast<const uint4*>(ln.bias + 8 * c), pb);
+    unpack8(*reinterpret_cast<const uint4*>(ln.gamma + 8 * c), ga);
+    unpack8(*reinterpret_cast<const uint4*>(ln.beta + 8 * c), be);
+    for (int r0 = w; r0 < rows; r0 += 16) {
+      uint4 p[4], q[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const size_t at = (size_t)(m0 + min(r0 + 4 * u, rows - 1)) * EN_H + 8 * c;
+        p[u] = *reinterpret_cast<const uint4*>(ln.proj + at);
+        q[u] = *reinterpret_cast<const uint4*>(ln.res + at);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int r = r0 + 4 * u;
+        float v[8], t[8], s = 0.f, d2 = 0.f;
+        unpack8(p[u], v);
+        unpack8(q[u], t);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          v[j] = on ? v[j] + pb[j] + t[j] : 0.f;
+          s += v[j];
+        }
+        const float mean = wave_sum(s) * (1.f / EN_H);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) d2 += on ? (v[j] - mean) * (v[j] - mean) : 0.f;
+        const float rstd = rsqrtf(wave_sum(d2) * (1.f / EN_H) + ln.eps);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = (v[j] - mean) * rstd * ga[j] + be[j];
+        if (on && r < rows) {
+          const uint4 y = pack8(v);
+          *reinterpret_cast<uint4*>(smem + r * (EN_H * 2) + ((c ^ (r & 7)) << 4)) = y;
+          if (blockIdx.x == 0) *reinterpret_cast<uint4*>(x + (size_t)(m0 + r) * EN_H + 8 * c) = y;
+        }
+      }
+    }
+  } else {
+    for (int id = threadIdx.x; id < rows * CH; id += 256) {
+      const int r = id / CH, c = id - r * CH;
+      *reinterpret_cast<uint4*>(smem + r * (EN_H * 2) + ((c ^ (r & 7)) << 4)) =
+          *reinterpret_cast<const uint4*>(x + (size_t)(m0 + r) * EN_H + 8 * c);
+    }
+  }
+  __syncthreads();
+  const float b[4] = {__uint_as_float(bb.x << 16), __uint_as_float(bb.x & 0xffff0000u), __uint_as_float(bb.y << 16),
+                      __uint_as_float(bb.y & 0xffff0000u)};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (16 * i >= rows) break;                    // rows past `rows` of the last group: stale LDS, not stored
+    f32x4_t acc = {b[0], b[1], b[2], b[3]};
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const uint4 xv = *reinterpret_cast<const uint4*>(smem + (16 * i + r16) * (EN_H * 2) + (((4 * k + g) ^ (r16 & 7)) << 4));
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[k]), __builtin_bit_cast(bf16x8_t, xv), acc, 0, 0, 0);
+    }
+    if constexpr (GELU) {
+      Gelu ge;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v = acc[e];
+        en_gelu<0>(ge, v);
+        en_gelu<1>(ge, v);
+        en_gelu<2>(ge, v);
+        acc[e] = v;
+      }
+    }
+    if (16 * i + r16 < rows)
+      *reinterpret_cast<uint2*>(out + (size_t)(m0 + 16 * i + r16) * N + n0 + 4 * g) = make_uint2(pack2bf(acc[0], acc[1]), pack2bf(acc[2], acc[3]));
+  }
+}
+
+// y = x W^T for a K-wide x and a W of 384 rows, rounded to bf16: 64 rows x 16 columns a workgroup, a quarter of K per wave
+// with W's and the rows' fragments straight from memory, the quarters summed through LDS.
+template <int K>
+__global__ void __launch_bounds__(256) enc_ksplit_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ W,
+                                                         uint16_t* __restrict__ out, int M) {
+  constexpr int KS = K / 128;                     // k steps of a wave
+  __shared__ float part[3][4][64][4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 64, rows = min(64, M - m0);
+  const int k0 = w * (K / 4) + 8 * g;
+  uint4 wf[KS];
+  const uint16_t* wr = W + (size_t)(n0 + r16) * K + k0;
+#pragma unroll
+  for (int k = 0; k < KS; ++k) wf[k] = *reinterpret_cast<const uint4*>(wr + 32 * k);
+  f32x4_t acc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (16 * i >= rows) break;
+    const uint16_t* xr = x + (size_t)(m0 + min(16 * i + r16, rows - 1)) * K + k0;
+    uint4 xv[KS];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) xv[k] = *reinterpret_cast<const uint4*>(xr + 32 * k);
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[k]), __builtin_bit_cast(bf16x8_t, xv[k]), acc[i], 0, 0, 0);
+  }
+  // wave q takes the sums of row group q
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i != w && 16 * i < rows) *reinterpret_cast<f32x4_t*>(part[w - (w > i)][i][lane]) = acc[i];
+  __syncthreads();
+  if (16 * w >= rows) return;
+  f32x4_t s = acc[0];
+#pragma unroll
+  for (int i = 1; i < 4; ++i)
+    if (w == i) s = acc[i];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) s += *reinterpret_cast<const f32x4_t*>(part[q][w][lane]);
+  if (16 * w + r16 < rows)
+    *reinterpret_cast<uint2*>(out + (size_t)(m0 + 16 * w + r16) * EN_H + n0 + 4 * g) = make_uint2(pack2bf(s[0], s[1]), pack2bf(s[2], s[3]));
+}
+
+}  // namespace
+
+CFC_API int cfc_layernorm(void* out, const void* x, const void* bias, const void* residual, const void* gamma, const void* beta,
+                          const int32_t* ids, const int32_t* pos, const void* pos_emb, const void* type_emb, int rows, int dim,
+                          float eps, int mode, hipStream_t stream);
+CFC_API int cfc_encoder_attention(const void* qkv, const int32_t* cu_seqlens, const int32_t* tile_seq, const int32_t* tile_q0,
+                                  int n_tiles, int tile_rows, int H, int head_dim, int max_seqlen, float scale, void* out,
+                                  hipStream_t stream);
+
+// Few rows: up to 2560, where a forward of MiniLM takes 696 us here and 789 in pgemm.hip's tiles (2048 rows: 592 and
+// 797, 3072: 803 and 794).  Many: from 13312, 104 of the 256 CUs' row blocks (12288 rows: 1060 us here and 1030 in
+// tiles, 14336: 1070 and 1130, 65536: 2430 and 3100).  Between them neither is faster than the tiles.
+constexpr int EN_FEW_ROWS = 2560, EN_MANY_ROWS = 13312;
+
+// Which rows this file's kernels take: 1 few, 2 many, 0 neither.
+CFC_API int cfc_enc_rows(int T) { return T <= EN_FEW_ROWS ? 1 : T >= EN_MANY_ROWS ? 2 : 0; }
+
+// Token states of a packed batch: embeddings, then every layer, one call for all launches.  W: host array of twelve
+// device pointers per layer (qkv, qkv_b, o, o_b, ln1_g, ln1_b, up, up_b, down, down_b, ln2_g, ln2_b).  x [T][384] the
+// states; att [T][384], qkv [T][1152], and for few rows y [T][384] and h [T][1536]: workspace.  All bf16 and 16-byte
+// aligned.
+CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* word, const void* pos_emb, const void* type_emb,
+                            const void* emb_g, const void* emb_b, const int32_t* cu, const int32_t* tile_seq, const int32_t* tile_q0,
+                            int n_tiles, int tile_rows, int max_seqlen, int layers, const void* const* W, int heads, float scale,
+                            float eps, int T, void* x, void* y, void* att, void* qkv, void* h, hipStream_t stream) {
+  const int kind = cfc_enc_rows(T);
+  if (T < 1 || layers < 1 || heads < 1 || EN_H % heads || kind == 0 || (kind == 1 && (h == nullptr || y == nullptr))) return -1;
+  int rc = cfc_layernorm(x, word, nullptr, nullptr, emb_g, emb_b, ids, pos, pos_emb, type_emb, T, EN_H, eps, 2, stream);
+  uint16_t *xp = (uint16_t*)x, *yp = (uint16_t*)y, *ap = (uint16_t*)att, *qp = (uint16_t*)qkv, *hp = (uint16_t*)h;
+  const int blocks = (T + EN_ROWS - 1) / EN_ROWS, tiles = (T + 63) / 64;
+  const uint16_t* const* P = (const uint16_t* const*)W;
+  for (int l = 0; l < layers && rc == 0; ++l) {
+    const uint16_t* const* p = P + 12 * l;
+    const dim3 gq(3 * EN_H / 64, tiles), gu(EN_F / 64, tiles), gk(EN_H / 16, tiles);
+    // few rows: a sublayer's last product waits in y for the next tiles' norm, which puts the layer's states in x, those
+    // between its sublayers in att (the attention's output is used up by then)
+    if (kind == 2)
+      enc_proj_kernel<<<blocks, 256, 0, stream>>>(xp, p[0], p[1], qp, T, 3 * EN_T);
+    else if (l == 0)
+      enc_tile_kernel<false, false><<<gq, 256, 0, stream>>>(xp, EncNorm{}, p[0], p[1], qp, T, 3 * EN_H);
+    else
+      enc_tile_kernel<false, true><<<gq, 256, 0, stream>>>(xp, EncNorm{yp, p[-3], ap, p[-2], p[-1], eps}, p[0], p[1], qp, T, 3 * EN_H);
+    rc = cfc_encoder_attention(qkv, cu, tile_seq, tile_q0, n_tiles, tile_rows, heads, EN_H / heads, max_seqlen, scale, att, stream);
+    if (rc) break;
+    if (kind == 2) {
+      const EncLayer L = {p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], p[10], p[11]};
+      enc_layer_kernel<<<blocks, 256, EN_LDS, stream>>>(ap, xp, L, xp, T, eps);
+    } else {
+      enc_ksplit_kernel<EN_H><<<gk, 256, 0, stream>>>(ap, p[2], yp, T);
+      enc_tile_kernel<true, true><<<gu, 256, 0, stream>>>(ap, EncNorm{yp, p[3], xp, p[4], p[5], eps}, p[6], p[7], hp, T, EN_F);
+      enc_ksplit_kernel<EN_F><<<gk, 256, 0, stream>>>(hp, p[8], yp, T);
+    }
+  }
+  if (rc) return rc;
+  if (kind == 1) {
+    const uint16_t* const* p = P + 12 * layers;
+    return cfc_layernorm(x, y, p[-3], att, p[-2], p[-1], nullptr, nullptr, nullptr, nullptr, T, EN_H, eps, 1, stream);
+  }
+  return CFC_CHECK_LAUNCH();
+}

@@ -1,0 +1,73 @@
+"""The encoder's kernels for few and for many rows (encoder.hip) at the edges of their tiles, against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _model(cfg, seed):
+    from copilot_for_consensus_amd.models.encoder import EncoderModel
+    m = EncoderModel.random(cfg, DEV, seed=seed)
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    for t in [m.p["emb_g"], m.p["emb_b"]] + [lw[k] for lw in m.layers for k in lw]:
+        if t.dim() == 1:           # no norm's gain or bias is one or zero
+            t.add_(0.1 * torch.randn(t.shape, device=DEV, generator=g).bfloat16())
+    return m
+
+
+def _states(m, ids, lens):
+    """Token states in float64, sequence by sequence."""
+    c, out = m.cfg, []
+    ln = lambda x, g, b: torch.nn.functional.layer_norm(x, (c.hidden,), g.double(), b.double(), c.ln_eps)  # noqa: E731
+    for part in ids.split(lens):
+        x = ln(m.p["word"].double()[part] + m.p["pos"].double()[:len(part)] + m.p["type"].double()[0], m.p["emb_g"], m.p["emb_b"])
+        for lw in m.layers:
+            w = {k: v.double() for k, v in lw.items()}
+            q, k, v = (t.view(len(part), c.heads, -1).transpose(0, 1) for t in (x @ w["qkv"].T + w["qkv_b"]).chunk(3, 1))
+            a = (torch.softmax(q @ k.transpose(1, 2) * m.scale, -1) @ v).transpose(0, 1).reshape(len(part), -1)
+            x = ln(x + a @ w["o"].T + w["o_b"], w["ln1_g"], w["ln1_b"])
+            h = torch.nn.functional.gelu(x @ w["up"].T + w["up_b"])
+            x = ln(x + h @ w["down"].T + w["down_b"], w["ln2_g"], w["ln2_b"])
+        out.append(x)
+    return torch.cat(out)
+
+
+@pytest.mark.parametrize("lens", [[1], [15], [16, 1], [17, 46], [64], [65], [256, 256, 1], [200] * 12 + [160], [200] * 12 + [161],
+                                  [256] * 52 + [1], [256] * 52 + [127, 1], [250] * 60 + [99]], ids=lambda v: str(sum(v)))
+def test_rows_against_float64(lens):
+    import dataclasses
+    from copilot_for_consensus_amd.models.encoder import get_encoder_config
+    from copilot_for_consensus_amd.ops import kernels as K
+    m = _model(dataclasses.replace(get_encoder_config("minilm-l6"), layers=3), seed=len(lens))
+    T = sum(lens)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    ids = torch.randint(0, m.cfg.vocab_size, (T,), device=DEV, dtype=torch.int32, generator=g)
+    pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).to(DEV)
+    cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).to(torch.int32)
+    tiles = tuple(torch.tensor(t, dtype=torch.int32, device=DEV) for t in K.prefill_tiles(cu.tolist(), K.ENCODER_TILE_ROWS))
+    # 2560 rows are few, 13312 many, those between are the tiles'
+    assert K.encoder_forward_ok(T, m.p, m.layers, m.cfg.heads, max(lens)) == (T <= 2560 or T >= 13312)
+    got = m.forward_packed(ids, pos, cu.to(DEV), max(lens), tiles=tiles).double()
+    want = _states(m, ids.long(), lens)
+    # bf16 states: 2^-9 of a value per rounding, some ten of them a layer that add up as a random walk, 3 layers
+    rel = ((got - want).norm(dim=1) / want.norm(dim=1)).max()
+    assert rel < 2.0 ** -9 * (3 * 10) ** 0.5, float(rel)
+
+
+def test_what_the_kernels_are_not_built_for():
+    """Other shapes, types and alignments keep the general path."""
+    from copilot_for_consensus_amd.models.encoder import EncoderModel
+    from copilot_for_consensus_amd.ops import kernels as K
+    m = EncoderModel.random("minilm-l6", DEV, seed=0)
+    ok = lambda **kw: K.encoder_forward_ok(kw.get("T", 12), m.p, kw.get("layers", m.layers), kw.get("heads", 12), kw.get("S", 12))  # noqa: E731
+    assert ok() and ok(heads=6)
+    assert not (ok(T=0) or ok(T=4096) or ok(S=513) or ok(heads=4) or ok(layers=[]))
+    lw = dict(m.layers[0])
+    odd = torch.empty(lw["o"].numel() + 1, dtype=torch.bfloat16, device=DEV)[1:].view_as(lw["o"])
+    for bad in (lw["o"].float(), lw["o"].t(), odd, lw["o"][:, :352]):
+        assert not ok(layers=[dict(lw, o=bad)])
+    texts = [list(range(3, 20)), [7], list(range(100, 350))]
+    want = m.encode_ids(texts)
+    m.layers = [dict(lw, o=odd.copy_(lw["o"])) for lw in m.layers[:1]] + m.layers[1:]
+    assert torch.allclose(m.encode_ids(texts), want, atol=4e-3)
