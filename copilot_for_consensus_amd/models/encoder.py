@@ -151,9 +151,10 @@ class EncoderModel:
         """Token states [T, H] for packed varlen input."""
         c = self.cfg
         if (ids.is_cuda and tiles is not None and os.environ.get("CFC_ENCODER_GEMM", "auto") == "auto"
-                and os.environ.get("CFC_ENCODER_LN_FUSED", "1") != "0"
-                and K.encoder_forward_ok(ids.numel(), self.p, self.layers, c.heads, max_seqlen)):
-            return K.encoder_forward(ids, positions, self.p, self.layers, cu_seqlens, tiles, c.heads, max_seqlen, self.scale, c.ln_eps)
+                and os.environ.get("CFC_ENCODER_LN_FUSED", "1") != "0"):
+            w = K.encoder_weights(ids.numel(), self.p, self.layers, c.heads, max_seqlen)
+            if w is not None:
+                return K.encoder_forward(ids, positions, w, len(self.layers), cu_seqlens, tiles, c.heads, max_seqlen, self.scale, c.ln_eps)
         x = K.embed_layernorm(ids, positions, self.p["word"], self.p["pos"], self.p["type"], self.p["emb_g"],
                               self.p["emb_b"], c.ln_eps)
         lin = self._linear

@@ -378,41 +378,54 @@ ENCODER_LAYER = ("qkv", "qkv_b", "o", "o_b", "ln1_g", "ln1_b", "up", "up_b", "do
 ENCODER_HIDDEN, ENCODER_FFN = 384, 1536      # what encoder.hip is built for
 
 
-def encoder_forward_ok(T: int, p: dict, layers: list[dict], heads: int, max_seqlen: int) -> bool:
-    """Whether encoder.hip takes T rows of this model: few or many, hidden 384, inner 1536, bf16 tensors on one GPU."""
-    H, Fh = ENCODER_HIDDEN, ENCODER_FFN
-    shapes = {"qkv": (3 * H, H), "qkv_b": (3 * H,), "o": (H, H), "up": (Fh, H), "up_b": (Fh,), "down": (H, Fh)}
-    if p["word"].device.type != "cuda" or T < 1 or not kernels().cfc_enc_rows(T) or not layers or not 1 <= max_seqlen <= 512 \
+_ENCODER_SHAPES = [(k, {"qkv": (3 * ENCODER_HIDDEN, ENCODER_HIDDEN), "qkv_b": (3 * ENCODER_HIDDEN,),
+                       "o": (ENCODER_HIDDEN, ENCODER_HIDDEN), "up": (ENCODER_FFN, ENCODER_HIDDEN), "up_b": (ENCODER_FFN,),
+                       "down": (ENCODER_HIDDEN, ENCODER_FFN)}.get(k, (ENCODER_HIDDEN,))) for k in ENCODER_LAYER]
+
+
+def encoder_weights(T: int, p: dict, layers: list[dict], heads: int, max_seqlen: int) -> list[int] | None:
+    """Addresses of what :func:`encoder_forward` reads, embeddings first; None where encoder.hip is not built for T rows
+    (few or many) of this model: hidden 384, inner 1536, contiguous bf16 tensors on one GPU."""
+    H, word = ENCODER_HIDDEN, p["word"]
+    if not word.is_cuda or T < 1 or not kernels().cfc_enc_rows(T) or not layers or not 1 <= max_seqlen <= 512 \
             or heads not in (H // 32, H // 64):
-        return False
-    dev, ts = p["word"].device, [p[k] for k in ("word", "pos", "type")]
-    if any(t.dim() != 2 or t.shape[1] != H for t in ts) or any(p[k].shape != (H,) for k in ("emb_g", "emb_b")):
-        return False
-    ts += [p["emb_g"], p["emb_b"]]
+        return None
+    dev, bf16, out, low = word.get_device(), torch.bfloat16, [], 0
+    def takes(t, shape):
+        return t.shape == shape and t.dtype is bf16 and t.get_device() == dev and t.is_contiguous()
+    for k in ("word", "pos", "type", "emb_g", "emb_b"):
+        t = p[k]
+        if not takes(t, (H,) if k.startswith("emb") else (t.shape[0], H)):
+            return None
+        out.append(t.data_ptr())
     for lw in layers:
-        for k in ENCODER_LAYER:
-            if lw[k].shape != shapes.get(k, (H,)):
-                return False
-            ts.append(lw[k])
-    return all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.device == dev and t.data_ptr() % 16 == 0 for t in ts)
+        for k, shape in _ENCODER_SHAPES:
+            if not takes(lw[k], shape):
+                return None
+            out.append(lw[k].data_ptr())
+    for a in out:
+        low |= a
+    return None if low & 15 else out
 
 
-def encoder_forward(ids, positions, p: dict, layers: list[dict], cu_seqlens, tiles, heads: int, max_seqlen: int, scale: float,
+def encoder_forward(ids, positions, weights: list[int], layers: int, cu_seqlens, tiles, heads: int, max_seqlen: int, scale: float,
                     eps: float) -> torch.Tensor:
-    """Token states [T, 384] of a packed batch, all launches in one call (encoder.hip); see :func:`encoder_forward_ok`."""
+    """Token states [T, 384] of a packed batch, all launches in one call (encoder.hip); ``weights``: :func:`encoder_weights`
+    of the batch's rows."""
     for t in (ids, positions, cu_seqlens, *tiles):
         _req(t, torch.int32, "encoder_forward")
     lib, T, H, dev = kernels(), ids.numel(), ENCODER_HIDDEN, ids.device
-    if positions.numel() != T or tiles[0].numel() != tiles[1].numel():
-        raise ValueError(f"encoder_forward: {T} ids, {positions.numel()} positions, tiles {[t.numel() for t in tiles]}")
+    if positions.numel() != T or tiles[0].numel() != tiles[1].numel() or len(weights) != 5 + len(ENCODER_LAYER) * layers:
+        raise ValueError(f"encoder_forward: {T} ids, {positions.numel()} positions, tiles {[t.numel() for t in tiles]}, "
+                         f"{len(weights)} weights of {layers} layers")
     def rows(n):
         return torch.empty(T, n, dtype=torch.bfloat16, device=dev)
     x, att, qkv = rows(H), rows(H), rows(3 * H)
     y, h = (rows(H), rows(ENCODER_FFN)) if lib.cfc_enc_rows(T) == 1 else (None, None)
-    W = (ctypes.c_void_p * (len(ENCODER_LAYER) * len(layers)))(*(lw[k].data_ptr() for lw in layers for k in ENCODER_LAYER))
-    check(lib.cfc_enc_forward(ids.data_ptr(), positions.data_ptr(), *(p[k].data_ptr() for k in ("word", "pos", "type", "emb_g", "emb_b")),
+    W = (ctypes.c_void_p * (len(weights) - 5))(*weights[5:])
+    check(lib.cfc_enc_forward(ids.data_ptr(), positions.data_ptr(), *weights[:5],
                               cu_seqlens.data_ptr(), tiles[0].data_ptr(), tiles[1].data_ptr(), tiles[0].numel(), ENCODER_TILE_ROWS,
-                              int(max_seqlen), len(layers), W, heads, float(scale), float(eps), T, x.data_ptr(), _p(y), att.data_ptr(),
+                              int(max_seqlen), layers, W, heads, float(scale), float(eps), T, x.data_ptr(), _p(y), att.data_ptr(),
                               qkv.data_ptr(), _p(h), _stream(x)), "cfc_enc_forward")
     return x
 

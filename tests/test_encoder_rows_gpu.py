@@ -47,7 +47,7 @@ def test_rows_against_float64(lens):
     cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).to(torch.int32)
     tiles = tuple(torch.tensor(t, dtype=torch.int32, device=DEV) for t in K.prefill_tiles(cu.tolist(), K.ENCODER_TILE_ROWS))
     # 2560 rows are few, 13312 many, those between are the tiles'
-    assert K.encoder_forward_ok(T, m.p, m.layers, m.cfg.heads, max(lens)) == (T <= 2560 or T >= 13312)
+    assert (K.encoder_weights(T, m.p, m.layers, m.cfg.heads, max(lens)) is not None) == (T <= 2560 or T >= 13312)
     got = m.forward_packed(ids, pos, cu.to(DEV), max(lens), tiles=tiles).double()
     want = _states(m, ids.long(), lens)
     # bf16 states: 2^-9 of a value per rounding, some ten of them a layer that add up as a random walk, 3 layers
@@ -60,7 +60,7 @@ def test_what_the_kernels_are_not_built_for():
     from copilot_for_consensus_amd.models.encoder import EncoderModel
     from copilot_for_consensus_amd.ops import kernels as K
     m = EncoderModel.random("minilm-l6", DEV, seed=0)
-    ok = lambda **kw: K.encoder_forward_ok(kw.get("T", 12), m.p, kw.get("layers", m.layers), kw.get("heads", 12), kw.get("S", 12))  # noqa: E731
+    ok = lambda **kw: K.encoder_weights(kw.get("T", 12), m.p, kw.get("layers", m.layers), kw.get("heads", 12), kw.get("S", 12))  # noqa: E731
     assert ok() and ok(heads=6)
     assert not (ok(T=0) or ok(T=4096) or ok(S=513) or ok(heads=4) or ok(layers=[]))
     lw = dict(m.layers[0])
