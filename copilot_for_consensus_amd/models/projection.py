@@ -1,8 +1,8 @@
 """One weight matrix and the products a model takes with it, on the kernel that fits the row count.
 
-The selection is DecoderModel's: at most K.GEMV_MAX_M rows on the packed GEMV, prompt-sized batches on
-the hand-written prefill GEMM, what lies between on the decode GEMM, all three reading one fragment-
-packed bf16 copy.  Shapes those kernels do not take (N or K not a multiple of 64) and 32-bit weights use
+The selection is DecoderModel's: at most K.GEMV_MAX_M rows on the packed GEMV, up to 128 on the decode GEMM,
+thousands on the prefill GEMM's 256 x 256 tiles, what lies between on the GEMM for a few hundred rows
+(K.mgemm_plan), all four reading one fragment-packed bf16 copy.  Shapes those kernels do not take (N or K not a multiple of 64) and 32-bit weights use
 the library product.  CPU tensors: torch.
 """
 from __future__ import annotations
@@ -55,12 +55,21 @@ class Projection:
     def _prefill(self, M: int) -> bool:
         return M >= 256 and -(-M // 256) * -(-self.N // 256) >= self.min_tiles and M * self.K * 2 < 2 ** 32
 
-    def _kernel(self, x) -> str:
+    def _kernel(self, x, kind: str = "act") -> str:
         if self.packed is None or not x.is_contiguous():
             return "lib"
         if x.shape[0] <= K.GEMV_MAX_M:
             return "gemv"
+        if K.mgemm_plan(x.shape[0], self.N, self.K, kind):
+            return "mgemm"
         return "pgemm" if self._prefill(x.shape[0]) else "dgemm"
+
+    def _mgemm(self, x, epi: str, reduce, **kw):
+        """The product with its epilogue, or with what adds its slabs up."""
+        bm, split = K.mgemm_plan(x.shape[0], self.N, self.K)
+        if split == 1:
+            return K.mgemm(x, self.packed, epi, bm, **kw)
+        return reduce(K.mgemm(x, self.packed, "part", bm, split))
 
     def act(self, x: torch.Tensor) -> torch.Tensor:
         """[M, N] in x's dtype."""
@@ -69,6 +78,8 @@ class Projection:
             return F.linear(x, self.rowmajor())
         if k == "gemv":
             return K.splitk_reduce(K.gemv_part(x, self.packed))
+        if k == "mgemm":
+            return self._mgemm(x, "bf16", K.splitk_reduce)
         if k == "pgemm":
             return K.pgemm(x, self.packed, "bf16", variant="ppp")
         return K.dgemm_linear(x, self.packed)
@@ -77,21 +88,22 @@ class Projection:
         """fp32 k-slice slabs [split, M, N] whose sum is the product (unrounded).  They may live in the
         stream's split-K workspace: consume them before the next product, unless they are to be a tensor of
         their ``own``."""
-        k = self._kernel(x)
-        if own and k in ("gemv", "dgemm"):
-            M = x.shape[0]
+        k = self._kernel(x, "slabs")
+        M, out = x.shape[0], None
+        if k in ("gemv", "dgemm", "mgemm"):
             split = K.gemv_packed_config(self.N, self.K, self.packed.bn // 16, M)[0] if k == "gemv" else \
-                K.dgemm_config(M, self.N, self.K, bn=self.packed.bn)[1]
-            out = torch.empty(split, M, self.N, dtype=torch.float32, device=x.device)
-            return K.gemv_part(x, self.packed, split, out=out) if k == "gemv" else \
-                K.dgemm(x, self.packed, "part", split, part=out)
+                K.dgemm_config(M, self.N, self.K, bn=self.packed.bn)[1] if k == "dgemm" else \
+                K.mgemm_plan(M, self.N, self.K, "slabs")[1]
+            if own:
+                out = torch.empty(split, M, self.N, dtype=torch.float32, device=x.device)
         if k == "gemv":
-            return K.gemv_part(x, self.packed)
+            return K.gemv_part(x, self.packed, split, out=out)
+        if k == "mgemm":
+            return K.mgemm(x, self.packed, "part", K.mgemm_plan(M, self.N, self.K, "slabs")[0], split, out)
         if k == "pgemm":
             return K.pgemm(x, self.packed, "f32", variant="ppp")[None]
         if k == "dgemm":
-            bn, split = K.dgemm_config(x.shape[0], self.N, self.K, bn=self.packed.bn)
-            return K.dgemm(x, self.packed, "part", split, bn=bn)
+            return K.dgemm(x, self.packed, "part", split, part=out)
         w = self.rowmajor()
         if x.is_cuda and x.dtype == torch.bfloat16:
             return torch.mm(x, w.t(), out_dtype=torch.float32)[None]
@@ -101,6 +113,9 @@ class Projection:
         """W = 8-row interleaved gate / up rows: the clamped GLU of the product into ``out`` [M, N / 2]
         (row-strided), in the product's epilogue where one pass over (packed) W fills the chip."""
         k, M = self._kernel(x), x.shape[0]
+        if k == "mgemm" and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0:
+            return self._mgemm(x, "glu", lambda s: clamped_glu(s, out, limit, alpha, beta, interleaved=True, cubic=cubic),
+                               out=out, glu=(limit, alpha, beta, cubic))
         if k == "pgemm" and self.K >= 128 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
             return K.pgemm_glu(x, self.packed, out, limit, alpha, beta, cubic)
         if k in ("pgemm", "dgemm") and self.N // self.packed.bn * -(-M // 256) > K.DGEMM_CUS // 2 \
@@ -111,18 +126,24 @@ class Projection:
     def relu_sq(self, x: torch.Tensor) -> torch.Tensor:
         """relu(product)^2 [M, N] in x's dtype, in the prompt product's epilogue, else with the sum of the slabs."""
         k = self._kernel(x)
+        if k == "mgemm":
+            return self._mgemm(x, "relu2", lambda s: relu_sq(s, x.dtype))
         if k == "pgemm" and self.K >= 128:
             return K.pgemm(x, self.packed, "relu2", variant="ppp")
         return relu_sq(self.slabs(x), x.dtype)
 
     def f32(self, x: torch.Tensor) -> torch.Tensor:
         """[M, N] fp32, a tensor of its own."""
-        k = self._kernel(x)
+        k = self._kernel(x, "whole")
         if k == "gemv":
             return K.gemv(x, self.packed, "f32")
-        if k == "dgemm":
+        if k in ("mgemm", "dgemm"):
             out = torch.empty(1, x.shape[0], self.N, dtype=torch.float32, device=x.device)
+            if k == "mgemm":
+                return K.mgemm(x, self.packed, "part", K.mgemm_plan(x.shape[0], self.N, self.K, "whole")[0], 1, out)[0]
             return K.dgemm(x, self.packed, "part", 1, part=out)[0]
+        if k == "pgemm":
+            return K.pgemm(x, self.packed, "f32", variant="ppp")
         return self.slabs(x)[0]
 
 

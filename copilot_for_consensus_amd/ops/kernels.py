@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes
 import dataclasses
+import functools
 import math
 import os
 
@@ -776,6 +777,85 @@ def dgemm_glu(x: torch.Tensor, w: "PackedWeight", out: torch.Tensor, limit: floa
         raise ValueError(f"dgemm_glu: x {tuple(x.shape)} {x.dtype} w {tuple(w.shape)}")
     check(kernels().cfc_dgemm_glu(x.data_ptr(), w.data.data_ptr(), x.shape[0], w.N, w.K, w.bn, out.data_ptr(),
                                   out.stride(0), float(limit), float(alpha), float(beta), float(cubic), _stream(x)), "cfc_dgemm_glu")
+    return out
+
+
+MGEMM_MIN_ROWS = 129     # up to 128 rows (its tiles of 64 or 128) the decode GEMM streams W as fast or faster
+
+
+def _mgemm_us(M: int, N: int, Kd: int, bm: int, split: int, fp32: bool = False) -> float:
+    """Time of mgemm.hip in bm-row tiles, as measured for N, K of 1024 .. 28672 and 129 .. 5500 rows (mostly within 10 %).
+    A 64-deep stage takes 0.2 + 0.0013 bm us on an idle chip, up to 0.42 more of that on a full one (0.55 in all rounds
+    but the last), and no less than its 16 KB of W and its rows of X at 67 B/ns: a last tile of few rows runs ahead and
+    brings W into the L2 for the others (385 rows 31 us, 384 rows 40), so they count as fewer rows.  One row tile alone
+    waits for W from memory, 0.59 us (64 workgroups) to 0.75.  4 us per round of workgroups, 6 per call; slabs are
+    written and read, one fp32 result is written, at 7 TB/s."""
+    tm = -(-M // bm)
+    last = M - (tm - 1) * bm
+    rows = last + 0.6 * (bm - last) * (1.0 - 1.0 / tm)
+    wgs = tm * -(-N // 128) * split
+    full, fill = (wgs - 1) // DGEMM_CUS, ((wgs - 1) % DGEMM_CUS + 1) / DGEMM_CUS
+    stages, idle = -(-Kd // (64 * split)), 0.2 + 0.0013 * bm
+    least = max((16384 + 128 * rows) / 67e3, 0.51 + 0.24 * min(1.0, wgs / 192) if tm == 1 else 0.0)
+    t = 6.0 + full * (4.0 + stages * max(idle * 1.55, least)) + 4.0 + stages * max(idle * (1.0 + 0.42 * fill ** 3), least)
+    t = max(t, 10.0 + N * Kd * 2 / 5.0e6)
+    return t + (8.0 * split if split > 1 else 4.0 * fp32) * M * N / 7.0e6
+
+
+def _ppp_us(M: int, N: int, Kd: int) -> float:
+    """Time of pgemm's persistent kernel (measured as above): a K-tile takes 1.4 us in a full round of 256 x 256 tiles,
+    0.8 to 1.22 in a partial one."""
+    full, rest = divmod(-(-M // 256) * -(-N // 256), DGEMM_CUS)
+    return 12.0 + Kd / 64 * (1.4 * full + (0.8 + 0.42 * rest / DGEMM_CUS if rest else 0.0))
+
+
+@functools.lru_cache(maxsize=4096)
+def mgemm_plan(M: int, N: int, Kd: int, kind: str = "act") -> tuple[int, int] | None:
+    """(rows per workgroup, split) of the product on mgemm.hip, None where the decode GEMM (up to 128 rows) or pgemm is
+    the faster one.  ``kind``: "act", an epilogue without a split or the sum of the slabs, 2 us for its launch; "slabs",
+    for a consumer that adds them up; "whole", one fp32 result.  pgemm's fp32 results do not come from its persistent
+    kernel and take 1.2 times as long.  Splits are powers of two, so that rows multiplied in batches of different sizes
+    are mostly added up in the same order.  (4096 columns, K = 4096: mgemm up to 1800 rows, 61 us against 74; pgemm at 2100,
+    73 against 81.  28672 columns: mgemm up to 260 rows, 89 us against 95; pgemm at 300, 89 against 91.)"""
+    if M < MGEMM_MIN_ROWS or M * Kd * 2 >= 2 ** 32 or N * Kd * 2 >= 2 ** 32:
+        return None
+    # one row tile of the decode GEMM, or few weights: 129 .. 256 rows, 2^23 of them, 17 us against 18; 2^21: 14 against
+    # 15 at 220 rows, 16 against 17 at 512, but 18.6 against 18.3 at 700
+    if N * Kd <= 2 ** 23 and M <= (256 if N * Kd > 2 ** 22 else 640):
+        return None
+    us, bm, split = min((_mgemm_us(M, N, Kd, bm, s, kind != "act") + (2.0 if s > 1 and kind == "act" else 0.0), bm, s)
+                        for bm in (128, 160, 192, 224, 256)
+                        for s in ((1,) if kind == "whole" else (1, 2, 4, 8)) if s * 64 <= Kd)
+    if -(-M // bm) * -(-N // 128) > 3 * DGEMM_CUS:         # not measured to be faster beyond 3 rounds
+        return None
+    if M >= 256 and _ppp_us(M, N, Kd) * (0.97 if kind == "act" else 1.16) <= us:
+        return None
+    return bm, split
+
+
+def mgemm(x: torch.Tensor, w: "PackedWeight", epi: str, bm: int, split: int = 1, out: torch.Tensor | None = None,
+          glu: tuple = (0.0, 1.0, 0.0, 0.0)) -> torch.Tensor:
+    """One launch of the prompt GEMM for a few hundred rows.  ``epi``: "bf16", "swiglu", "relu2" as :func:`pgemm`'s,
+    "glu" as :func:`pgemm_glu`'s with its constants (out may be row-strided), or "part": fp32 slabs [split, M, N] of
+    ``split`` K slices, in the stream's workspace unless ``out`` is given."""
+    if not (pgemm_ok(x, w) and isinstance(w, PackedWeight)):
+        raise ValueError(f"mgemm: x {tuple(x.shape)} {x.dtype} w {tuple(w.shape)}")
+    M, Kd = x.shape
+    N = w.N
+    mode = {"bf16": 0, "swiglu": 3, "part": 4, "glu": 5, "relu2": 6}[epi]
+    if mode == 4:
+        if out is None:
+            out = _workspace(x.device, split * M * N)[:split * M * N].view(split, M, N)
+        if out.shape != (split, M, N) or out.dtype != torch.float32 or not out.is_contiguous():
+            raise ValueError(f"mgemm: slabs {tuple(out.shape)} {out.dtype}")
+    else:
+        cols = N // 2 if mode in (3, 5) else N
+        if out is None:
+            out = torch.empty(M, cols, dtype=torch.bfloat16, device=x.device)
+        if out.shape != (M, cols) or out.dtype != torch.bfloat16 or out.stride(1) != 1:
+            raise ValueError(f"mgemm: out {tuple(out.shape)} {out.dtype}")
+    check(kernels().cfc_mgemm(x.data_ptr(), w.data.data_ptr(), out.data_ptr(), M, N, Kd, mode, out.stride(-2), bm, split,
+                              w.bn // 16, *map(float, glu), _stream(x)), "cfc_mgemm")
     return out
 
 

@@ -1,0 +1,232 @@
+// Prompt GEMM for gfx950 between the decode GEMM (up to 128 rows) and the 256 x 256 tiles of pgemm.hip
+// (thousands of rows):  Y[M, N] = X[M, K] . W[N, K]^T  (bf16 in, fp32 accumulate, W fragment-packed).
+//
+// A product of a few hundred rows has too few 256 x 256 tiles for 256 CUs (4096 columns of 1536 rows: 96), and the
+// decode GEMM's waves, 16 columns each, read every X fragment from LDS for one MFMA.  Here a workgroup makes a
+// 32 MT x 128 tile, MT = 4 .. 8 (the height that wastes the fewest rows and CUs), of all of K or of one of `split`
+// slices, whose fp32 slabs the consumer adds up.  What bounds it is how fast a CU pulls X and W through its L2:
+// 55 - 66 B/ns with every CU at it (30 for lines that miss), so a 64-deep stage of 32 / 40 / 48 KB (MT = 4 / 6 / 8)
+// takes 0.37 / 0.44 / 0.54 us on a chip that is half idle, 0.53 / 0.62 / 0.75 on a full one; about 10 us of a
+// call are its start, the first stages' way and the stores.
+//
+//   * 8 waves in two groups of 2 x 2; both groups hold the whole tile, a wave 16 MT x 64 of it, and group g
+//     multiplies k = 32 g .. 32 g + 31 of every stage: 4 MT MFMAs per MT + 4 fragment reads, where eight waves side
+//     by side on the tile would read half as much again.  Their sums meet in LDS at the end, each group finishing
+//     half of the columns;
+//   * the groups run one barrier apart (as in pgemm.hip): one's MFMAs cover the other's LDS-DMA issue and fragment
+//     reads;
+//   * a ring of R = 3 .. 5 stages (160 KB): a stage is issued into the slot that both groups read one stage earlier
+//     and has R - 2 stages' time to land;
+//   * X image: row r's chunk c at r * 128 + ((c ^ (r & 7)) << 4), swizzled through the DMA source; W: one 1-KB piece per
+//     16 x 32 fragment.  Reads of both are free of bank conflicts;
+//   * consecutive workgroups of an XCD take the M-tiles of one run of columns, so W comes from memory once.
+//
+// us with the sum of the slabs, N x K 6144 x 4096 / 4096 x 4096 / 4096 x 14336, before (decode GEMM or pgemm) -> here:
+//   160 rows 29 / 23 / 44 -> 25 / 22 / 37;  420 rows 40 / 35 / 69 -> 35 / 28 / 59;
+//   1024 rows 74 / 74 / 129 -> 51 / 41 / 105;  1536 rows (75 in pgemm) / 74 / 227 -> - / 50 / 148.
+#include <type_traits>
+
+#include "pgemm.h"
+
+namespace {
+
+constexpr int MG_BN = 128, MG_BK = 64;
+
+template <int MT>
+struct MgShape {
+  static constexpr int BM = 32 * MT;
+  static constexpr int XB = BM * 128;                  // X image of a stage
+  static constexpr int STAGE = XB + MG_BN * 128;
+  static constexpr int P = (4 * MT + 16 + 7) / 8;      // 1-KB DMA pieces per wave and stage
+  static constexpr int R = 163840 / STAGE < 5 ? 163840 / STAGE : 5;
+};
+
+template <int N>
+__device__ __forceinline__ void mg_wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
+}
+__device__ __forceinline__ void mg_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
+// at most `ahead` stages of P pieces stay in flight
+template <int P, int MAXA>
+__device__ __forceinline__ void mg_wait_ahead(int ahead) {
+  if constexpr (MAXA == 0) {
+    mg_wait_barrier<0>();
+  } else {
+    if (ahead >= MAXA) mg_wait_barrier<MAXA * P>();
+    else mg_wait_ahead<P, MAXA - 1>(ahead);
+  }
+}
+
+template <int MT, int EPI>
+__global__ void __launch_bounds__(512, 1)
+    mgemm_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, float* __restrict__ part,
+                 uint16_t* __restrict__ out, int M, int N, int K, int ldo, int tiles_m, int tiles_n, int split, int wnw,
+                 PgGlu gp) {
+  using S = MgShape<MT>;
+  constexpr int P = S::P, R = S::R;
+  __shared__ __attribute__((aligned(16))) char smem[R * S::STAGE];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = w >> 2, wr = (w >> 1) & 1, wc = w & 1;
+
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = id % (tiles_m * tiles_n), ks = id / (tiles_m * tiles_n);
+  const int m0 = tile % tiles_m * S::BM, n0 = tile / tiles_m * MG_BN;
+  const int nks = K / MG_BK;
+  const int kb = (int)((long)ks * nks / split), nst = (int)((long)(ks + 1) * nks / split) - kb;
+
+  // ---- DMA sources of pieces w, w + 8, ...: 4 MT of X (8 image rows each), 16 of W (fragments)
+  uint32_t voff[P];
+  const char* src[P];
+  uint32_t adv[P];
+  const int kg_all = K / 32;
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const int p = min(w + 8 * i, 4 * MT + 15);
+    if (p < 4 * MT) {
+      const int r = 8 * p + (lane >> 3), c = (lane & 7) ^ (r & 7);
+      voff[i] = ((uint32_t)min(m0 + r, M - 1) * (uint32_t)K + 8u * c) * 2u;
+      adv[i] = MG_BK * 2;
+      src[i] = reinterpret_cast<const char*>(X) + (size_t)kb * adv[i];
+    } else {
+      const int f = p - 4 * MT, g = min(n0 / 16 + (f >> 1), N / 16 - 1);
+      voff[i] = (uint32_t)(((g / wnw) * kg_all + (f & 1)) * wnw + g % wnw) * 1024u + 16u * lane;
+      adv[i] = (uint32_t)wnw * 2048u;
+      src[i] = reinterpret_cast<const char*>(W) + (size_t)kb * adv[i];
+    }
+  }
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(pg_lds_t*)smem);
+  auto issue = [&](int slot) {
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      pg_glds16(voff[i], src[i], lds0 + slot * S::STAGE + min(w + 8 * i, 4 * MT + 15) * 1024);
+      src[i] += adv[i];
+    }
+  };
+
+  f32x4_t acc[MT][4];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int xrd = (16 * MT * wr + (lane & 15)) * 128 + (((4 * grp + (lane >> 4)) ^ (lane & 7)) << 4);
+  const int wrd = S::XB + (8 * wc + grp) * 1024 + 16 * lane;
+
+  // ---- prologue: R - 1 stages under way, the first one landed in every wave
+#pragma unroll
+  for (int s = 0; s < R - 1; ++s)
+    if (s < nst) issue(s);
+  mg_wait_ahead<P, R - 2>(nst - 1);
+  if (grp == 1) mg_barrier();   // the stagger: group 1 runs one barrier behind group 0
+  int slot = 0, fill = R - 1;
+  auto stage = [&](int t, auto last) {
+    constexpr bool LAST = decltype(last)::value;   // nothing left to issue
+    bf16x8_t xf[MT], wf[4];
+    if constexpr (!LAST) issue(fill);
+    const char* img = smem + slot * S::STAGE;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) wf[j] = *reinterpret_cast<const bf16x8_t*>(img + wrd + j * 2048);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) xf[i] = *reinterpret_cast<const bf16x8_t*>(img + xrd + i * 2048);
+    // this wave's pieces of stage t + 1 and its reads of stage t
+    if constexpr (LAST) mg_wait_ahead<P, R - 2>(nst - 2 - t);
+    else mg_wait_barrier<P * (R - 2)>();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[i], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    mg_barrier();
+    slot = slot + 1 == R ? 0 : slot + 1;
+    fill = fill + 1 == R ? 0 : fill + 1;
+  };
+  int t = 0;
+  for (; t + R - 1 < nst; ++t) stage(t, std::false_type{});
+  for (; t < nst; ++t) stage(t, std::true_type{});
+  if (grp == 0) mg_barrier();   // matches the stagger: every read and every DMA is over
+
+  // ---- the two groups' sums: group 0 finishes n-tiles 0, 1 of each wave, group 1 n-tiles 2, 3
+  float4* ex = reinterpret_cast<float4*>(smem) + lane;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float4 give;
+      float* gv = &give.x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float a = acc[i][j][e], b = acc[i][2 + j][e];
+        gv[e] = grp ? a : b;
+        acc[i][j][e] = grp ? b : a;      // what this wave finishes
+      }
+      ex[(((w ^ 4) * MT + i) * 2 + j) * 64] = give;
+    }
+  __syncthreads();
+  const int g = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = m0 + 16 * (MT * wr + i) + (lane & 15);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float4 o = ex[((w * MT + i) * 2 + j) * 64];
+      float v[4] = {acc[i][j][0] + o.x, acc[i][j][1] + o.y, acc[i][j][2] + o.z, acc[i][j][3] + o.w};
+      const int nb = n0 + 64 * wc + 32 * grp + 16 * j, n = nb + 4 * g;
+      if constexpr (pg_gated(EPI)) {
+        const uint32_t y = pg_gate2<EPI>(v, gp);
+        if (m < M && nb < N) *reinterpret_cast<uint32_t*>(out + (size_t)m * ldo + nb / 2 + pg_gate_col(g)) = y;
+      } else if constexpr (EPI == PG_F32) {
+        if (m < M && n < N)
+          *reinterpret_cast<float4*>(part + ((size_t)ks * M + m) * N + n) = make_float4(v[0], v[1], v[2], v[3]);
+      } else if (m < M && n < N) {
+        *reinterpret_cast<uint2*>(out + (size_t)m * ldo + n) =
+            make_uint2(pack2bf(pg_out<EPI>(v[0]), pg_out<EPI>(v[1])), pack2bf(pg_out<EPI>(v[2]), pg_out<EPI>(v[3])));
+      }
+    }
+  }
+}
+
+template <int EPI>
+int mgemm_launch(const void* x, const void* w, void* out, int M, int N, int K, int ldo, int bm, int split, int wnw,
+                 const PgGlu& gp, hipStream_t stream) {
+  const int tm = (M + bm - 1) / bm, tn = (N + MG_BN - 1) / MG_BN;
+#define MG_CASE(MT)                                                                                                 \
+  case 32 * MT:                                                                                                     \
+    mgemm_kernel<MT, EPI><<<tm * tn * split, 512, 0, stream>>>((const uint16_t*)x, (const uint16_t*)w, (float*)out, \
+                                                               (uint16_t*)out, M, N, K, ldo, tm, tn, split, wnw, gp); \
+    break;
+  switch (bm) {
+    MG_CASE(4)
+    MG_CASE(5)
+    MG_CASE(6)
+    MG_CASE(7)
+    MG_CASE(8)
+    default: return (int)hipErrorInvalidValue;
+  }
+#undef MG_CASE
+  return (int)hipGetLastError();
+}
+
+}  // namespace
+
+// epi as cfc_pgemm's (0 bf16, 3 SwiGLU, 4 fp32, 6 squared relu) or 5, the clamped GLU with its constants; out: row stride
+// ldo, or (fp32) slabs [split][M][N].  bm: 128, 160 .. 256 rows per workgroup.  W packed for bn = 16 wnw.
+CFC_API int cfc_mgemm(const void* x, const void* w, void* out, int M, int N, int K, int epi, int ldo, int bm, int split,
+                      int wnw, float limit, float alpha, float beta, float cubic, hipStream_t stream) {
+  if (M < 1 || N < 64 || K < 64 || K % 64 || N % 64 || split < 1 || split > K / 64 || (split > 1 && epi != PG_F32) ||
+      wnw < 1 || N % (16 * wnw) || (uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)N * K * 2 >= (1ull << 32) ||
+      (epi != PG_F32 && (ldo % 4 || ldo < (pg_gated(epi) ? N / 2 : N))) || ((uintptr_t)out & (epi == PG_F32 ? 15 : 7)) ||
+      (int64_t)((M + 127) / 128) * ((N + 127) / 128) * split > (1 << 30))
+    return (int)hipErrorInvalidValue;
+  PgGlu gp;
+  gp.limit = limit; gp.alpha = alpha; gp.beta = beta; gp.cubic = cubic;
+  switch (epi) {
+    case PG_BF16: return mgemm_launch<PG_BF16>(x, w, out, M, N, K, ldo, bm, split, wnw, gp, stream);
+    case PG_SWIGLU: return mgemm_launch<PG_SWIGLU>(x, w, out, M, N, K, ldo, bm, split, wnw, gp, stream);
+    case PG_F32: return mgemm_launch<PG_F32>(x, w, out, M, N, K, ldo, bm, split, wnw, gp, stream);
+    case PG_GLU: return mgemm_launch<PG_GLU>(x, w, out, M, N, K, ldo, bm, split, wnw, gp, stream);
+    case PG_RELU2: return mgemm_launch<PG_RELU2>(x, w, out, M, N, K, ldo, bm, split, wnw, gp, stream);
+    default: return (int)hipErrorInvalidValue;
+  }
+}

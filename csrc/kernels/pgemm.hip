@@ -31,90 +31,13 @@
 #include <atomic>
 #include <type_traits>
 
-#include "common.h"
+#include "pgemm.h"
 
 namespace {
-
-typedef __attribute__((address_space(3))) void pg_lds_t;
-
-// PG_F32: the fp32 accumulators themselves (row stride ldo in floats): a tensor-parallel row-parallel
-// projection's partial, all-reduced in fp32 and rounded to bf16 once, as TP = 1 rounds the full sum
-enum { PG_BF16 = 0, PG_BIAS = 1, PG_BIAS_GELU = 2, PG_SWIGLU = 3, PG_F32 = 4, PG_GLU = 5, PG_RELU2 = 6 };
 
 constexpr int PG_BM = 256, PG_BN = 256, PG_BK = 64;
 constexpr int PG_STAGE = (PG_BM + PG_BN) * PG_BK * 2;   // 64 KB: A image then B image
 constexpr int PG_GROUP_M = 8;
-
-// One 1-KB LDS-DMA piece from sbase + voff (per lane): lane l's 16 bytes land at lds_addr + 16 l.
-// SGPR base + 32-bit VGPR offset (one VGPR per piece instead of a 64-bit pointer).  M0 is saved and
-// restored inside the statement (guide §5.7).
-__device__ __forceinline__ void pg_glds16(uint32_t voff, const void* sbase, uint32_t lds_addr) {
-  unsigned keep;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-      : "=&s"(keep)
-      : "v"(voff), "s"(sbase), "s"(lds_addr)
-      : "memory");
-}
-
-// x Phi(x) = max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, erfc by Hastings' rational approximation (Abramowitz and
-// Stegun 7.1.26: t = 1 / (1 + p y), five terms, times exp(-y^2), within 1.5e-7).  About 15 instructions, two of
-// them transcendental, where erff takes some fifty; as far from x Phi(x) as that is below x = -3, where 1 + erf
-// cancels, within 4e-7 everywhere.  The encoder's up product over 65 k rows with both: 230 -> 155 us.
-__device__ __forceinline__ float pg_gelu(float v) {
-  const float a = fabsf(v);
-  const float t = __builtin_amdgcn_rcpf(fmaf(a, 0.3275911f * 0.70710678f, 1.f));
-  float q = fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
-  q = fmaf(q, t, 0.5f * 1.421413741f);
-  q = fmaf(q, t, 0.5f * -0.284496736f);
-  q = fmaf(q, t, 0.5f * 0.254829592f) * t;
-  return fmaf(-a, q * __builtin_amdgcn_exp2f(a * a * (-0.5f * 1.44269504f)), fmaxf(v, 0.f));
-}
-
-__device__ __forceinline__ float pg_bfr(float v) { return bf2f(f2bf(v)); }
-
-// Gated epilogues over 8-row interleaved gate / up weights: PG_SWIGLU silu(g) * u, and PG_GLU
-// min(g, limit) sigmoid(alpha g (1 + cubic g^2)) (clamp(u, +-limit) + beta) with the constants of PgGlu.
-struct PgGlu { float limit = 0.f, alpha = 1.f, beta = 0.f, cubic = 0.f; };
-constexpr bool pg_gated(int epi) { return epi == PG_SWIGLU || epi == PG_GLU; }
-
-// SwiGLU of one 4-value accumulator group (16-row n-tile = 8 gate rows then 8 up rows: lanes
-// g = 0, 1 hold gate columns, lanes g = 2, 3 -- lane ^ 32 -- the matching up columns).  One VALU lane
-// swap (v_permlane32_swap, common.h) of (v[0], v[2]) gives every lane a (gate, up) pair -- element 0
-// in lanes g < 2, element 2 in lanes g >= 2 -- and one of (v[1], v[3]) elements 1 / 3, so every lane
-// computes two outputs (no idle lane half, no LDS-crossbar shuffles) and returns them packed: output
-// columns pg_gate_col(g) + {0, 1} of the n-tile's 8.  Same values and rounding as the unfused
-// GEMM -> silu_mul path: bf16 of gate and up, silu(g) * u in fp32.
-template <int EPI>
-__device__ __forceinline__ uint32_t pg_gate2(const float (&v)[4], const PgGlu& p) {
-  float g0 = v[0], u0 = v[2], g1 = v[1], u1 = v[3];
-  swap32(g0, u0);
-  swap32(g1, u1);
-  if constexpr (EPI == PG_GLU) {
-    auto glu = [&](float gate, float up) {
-      const float gg = fminf(gate, p.limit), uu = fminf(fmaxf(up, -p.limit), p.limit);
-      return gg * __builtin_amdgcn_rcpf(1.f + __expf(-p.alpha * gg * (1.f + p.cubic * gg * gg))) * (uu + p.beta);
-    };
-    return pack2bf(glu(g0, u0), glu(g1, u1));
-  }
-  auto f = [](float gate, float up) {
-    const float gg = pg_bfr(gate);
-    return gg * __builtin_amdgcn_rcpf(1.f + __expf(-gg)) * pg_bfr(up);
-  };
-  return pack2bf(f(g0, u0), f(g1, u1));
-}
-
-__device__ __forceinline__ int pg_gate_col(int g) { return 4 * (g & 1) + 2 * (g >> 1); }
-
-// what a value leaves as: PG_RELU2 its squared positive part
-template <int EPI>
-__device__ __forceinline__ float pg_out(float v) {
-  if constexpr (EPI == PG_RELU2) {
-    v = fmaxf(v, 0.f);
-    return v * v;
-  }
-  return v;
-}
 
 // Epilogue of every kernel here: lane holds rows m = mw + 16 i + (lane & 15), columns
 // n = nw + 16 j + 4 (lane >> 4) + 0..3 of the wave's 128 x 16 NJ block.
