@@ -658,15 +658,14 @@ __device__ __forceinline__ void ppp_st8(void* p, uint2 v) { *reinterpret_cast<ui
 
 __device__ __forceinline__ void ppp_st16(void* p, uint4 v) { *reinterpret_cast<uint4*>(p) = v; }
 
-template <int EPI, bool STG = false>
-__global__ void __launch_bounds__(512, 1)
-    pgemm_ppp_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, uint16_t* __restrict__ out,
-                     int M, int N, int K, int ldo, int tiles_m, int tiles_n, int wnw, int gm, PgGlu gp) {
-  static_assert(EPI == PG_BF16 || EPI == PG_RELU2 || pg_gated(EPI), "bf16 / gated epilogues");
+template <int EPI, bool STG>
+__device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict__ X, const uint16_t* __restrict__ W,
+                                          uint16_t* __restrict__ out, int M, int N, int K, int ldo, int tiles_m,
+                                          int tiles_n, int wnw, int gm, const PgGlu& gp) {
+  static_assert(EPI == PG_BF16 || EPI == PG_RELU2 || (EPI == PG_F32 && STG) || pg_gated(EPI), "bf16 / gated / staged fp32 epilogues");
   // epilogue store instructions per wave in the interior (counted in the next tile's first waits):
-  // staged bf16 16 x 16 B (128 rows x 128 B), staged SwiGLU 8 x 16 B (128 rows x 64 B), else 32
-  constexpr int PPP_S = STG ? (pg_gated(EPI) ? 8 : 16) : 32;
-  __shared__ __attribute__((aligned(16))) char smem[2 * PP_BUF + (STG ? 8 * PPP_REGION : 0)];
+  // staged bf16 16 x 16 B (128 rows x 128 B), staged SwiGLU 8 x 16 B (128 rows x 64 B), else 32 (staged fp32 of 16 B)
+  constexpr int PPP_S = EPI == PG_F32 ? 32 : STG ? (pg_gated(EPI) ? 8 : 16) : 32;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int grp = w >> 2, wc = w & 3;
@@ -844,7 +843,29 @@ __global__ void __launch_bounds__(512, 1)
           }
         }
       }
-      if constexpr (STG && pg_gated(EPI)) {
+      if constexpr (STG && EPI == PG_F32) {
+        // 8 chunks of 16 rows (one m-tile): 256-byte rows, 16 units of 16 bytes XOR-swizzled by the row
+        char* region = smem + 2 * PP_BUF + w * PPP_REGION;
+        const int rl = lane & 15;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            *reinterpret_cast<f32x4_t*>(region + rl * 256 + (((4 * j + g) ^ rl) << 4)) = acc[q][j];
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+          for (int s4 = 0; s4 < 4; ++s4) {
+            const int r = 4 * s4 + (lane >> 4), unit = lane & 15;
+            const uint4 val = *reinterpret_cast<const uint4*>(region + r * 256 + ((unit ^ r) << 4));
+            ppp_st16(reinterpret_cast<float*>(out) + (size_t)(mw + 16 * q + r) * ldo + nw0 + unit * 4, val);
+          }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+      } else if constexpr (STG && pg_gated(EPI)) {
         // 2 chunks of 64 rows (m-tiles 4q .. 4q+3): 64-byte rows (32 output columns), 16-byte units
         // XOR-swizzled by the row (4 per row); each lane's two outputs (4 bytes) land at column
         // 8 j + pg_gate_col(g) of the chunk row, read back as whole units, stored as 64-byte row
@@ -933,6 +954,24 @@ __global__ void __launch_bounds__(512, 1)
     if (has_next) coords(vb + G, m0n, n0n);
   }
   if (grp == 0) pp_barrier();   // matches group 1's stagger barrier
+}
+
+template <int EPI, bool STG = false>
+__global__ void __launch_bounds__(512, 1)
+    pgemm_ppp_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, uint16_t* __restrict__ out,
+                     int M, int N, int K, int ldo, int tiles_m, int tiles_n, int wnw, int gm, PgGlu gp) {
+  __shared__ __attribute__((aligned(16))) char smem[2 * PP_BUF + (STG ? 8 * PPP_REGION : 0)];
+  ppp_tiles<EPI, STG>(smem, X, W, out, M, N, K, ldo, tiles_m, tiles_n, wnw, gm, gp);
+}
+
+// fp32 results, staged: 32 x 16 B per wave in whole 256-byte rows (straight from the accumulators, 64-byte pieces, 1-4 %
+// slower).  us against pgemm_pp_kernel's, which drains its 256 KB of stores at the end of every tile: 4096 x 4096 of 1537
+// rows 76 -> 69, 16100 rows 405 -> 379 (bf16 359); 4096 x 14336 of 14000 rows 1240 -> 1215.
+__global__ void __launch_bounds__(512, 1)
+    pgemm_ppp32_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, uint16_t* __restrict__ out,
+                       int M, int N, int K, int ldo, int tiles_m, int tiles_n, int wnw, int gm) {
+  __shared__ __attribute__((aligned(16))) char smem[2 * PP_BUF + 8 * PPP_REGION];
+  ppp_tiles<PG_F32, true>(smem, X, W, out, M, N, K, ldo, tiles_m, tiles_n, wnw, gm, PgGlu{});
 }
 
 
@@ -1290,13 +1329,15 @@ int pgemm_launch(const void* x, const void* w, const void* bias, void* out, int 
   return (int)hipGetLastError();
 }
 
-// fp32 output: the ping-pong kernel only (packed or row-major W)
-int pgemm_launch_f32(const void* x, const void* w, void* out, int M, int N, int K, int ldo, int wnw,
+// fp32 output: the persistent kernel for a packed W where it is asked for, else the ping-pong kernel
+int pgemm_launch_f32(const void* x, const void* w, void* out, int M, int N, int K, int ldo, int variant, int wnw,
                      hipStream_t stream) {
   const int tm = (M + PG_BM - 1) / PG_BM, tn = (N + PG_BN - 1) / PG_BN;
   const uint16_t *xp = (const uint16_t*)x, *wp = (const uint16_t*)w;
   uint16_t* op = (uint16_t*)out;
-  if (wnw > 0) pgemm_pp_kernel<PG_F32, true, PP_PF><<<tm * tn, 512, 0, stream>>>(xp, wp, nullptr, op, M, N, K, ldo, tm, tn, wnw);
+  if (wnw > 0 && variant == 6 && K >= 2 * PG_BK)
+    pgemm_ppp32_kernel<<<min(tm * tn, pg_cus()), 512, 0, stream>>>(xp, wp, op, M, N, K, ldo, tm, tn, wnw, ppp_group_m(tn, K));
+  else if (wnw > 0) pgemm_pp_kernel<PG_F32, true, PP_PF><<<tm * tn, 512, 0, stream>>>(xp, wp, nullptr, op, M, N, K, ldo, tm, tn, wnw);
   else pgemm_pp_kernel<PG_F32, false, PP_PF><<<tm * tn, 512, 0, stream>>>(xp, wp, nullptr, op, M, N, K, ldo, tm, tn, 1);
   return (int)hipGetLastError();
 }
@@ -1321,7 +1362,7 @@ CFC_API int cfc_pgemm(const void* x, const void* w, const void* bias, void* out,
     case 1: return pgemm_launch<PG_BIAS>(x, w, bias, out, M, N, K, ldo, variant, wnw, stream);
     case 2: return pgemm_launch<PG_BIAS_GELU>(x, w, bias, out, M, N, K, ldo, variant, wnw, stream);
     case 3: return pgemm_launch<PG_SWIGLU>(x, w, bias, out, M, N, K, ldo, variant, wnw, stream);
-    case 4: return pgemm_launch_f32(x, w, out, M, N, K, ldo, wnw, stream);
+    case 4: return pgemm_launch_f32(x, w, out, M, N, K, ldo, variant, wnw, stream);
     case 6:        // packed W, the persistent kernel
       if (wnw < 1 || K < 2 * PG_BK || ldo % 8 || ((uintptr_t)out & 15)) return (int)hipErrorInvalidValue;
       return ppp_launch<PG_RELU2>((const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, M, N, K, ldo, wnw,
