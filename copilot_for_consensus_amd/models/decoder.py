@@ -603,11 +603,9 @@ class DecoderModel:
         if self.prefill_gemm == "hip" and x.is_cuda and x.is_contiguous() and (
                 epi != "swiglu" or self.w.gate_up_interleaved):
             dg = pw is not None and K.dgemm_ok(x, pw)
-            plan = self._mgemm_plan(x, pw, epi)
-            if plan and plan[1] == 1:
-                return K.mgemm(x, pw, epi, plan[0])
+            plan = self._prompt_plan(x, pw, epi)
             if plan:
-                return K.splitk_reduce(K.mgemm(x, pw, "part", *plan), swiglu=epi == "swiglu")
+                return K.prompt_gemm(x, pw, epi, plan, reduce=lambda part, out: K.splitk_reduce(part, out, epi == "swiglu"))
             if (x.shape[0] >= self.PGEMM_MIN_ROWS and K.pgemm_ok(x, wt)
                     and not (dg and self._dgemm_faster(x.shape[0], wt.shape[0], x.shape[1]))):
                 return K.pgemm(x, wt, epi, variant=self.pgemm_variant_swiglu if epi == "swiglu" else self.pgemm_variant)
@@ -625,9 +623,10 @@ class DecoderModel:
         wt = pw if pw is not None else self.w.layers[i][name]
         if self.prefill_gemm == "hip" and x.is_cuda and x.is_contiguous():
             dg = pw is not None and K.dgemm_ok(x, pw)
-            plan = self._mgemm_plan(x, pw, "f32")
+            plan = self._prompt_plan(x, pw, "f32")
             if plan:
-                return K.mgemm(x, pw, "part", *plan, out=torch.empty(1, x.shape[0], pw.N, dtype=torch.float32, device=x.device))[0]
+                return K.prompt_gemm(x, pw, "f32", plan,
+                                     torch.empty(1, x.shape[0], pw.N, dtype=torch.float32, device=x.device))[0]
             if (x.shape[0] >= self.PGEMM_MIN_ROWS and K.pgemm_ok(x, wt)
                     and not (dg and self._dgemm_faster(x.shape[0], wt.shape[0], x.shape[1]))):
                 return K.pgemm(x, wt, "f32", variant=self.pgemm_variant)
@@ -661,13 +660,13 @@ class DecoderModel:
         (128) 244 vs 298.  A 512-token prompt: 70 -> 40 (qkv), 68 -> 33 (o), 211 -> 83 us (down)."""
         return -(-M // 256) * -(-N // 256) < self.PGEMM_MIN_TILES
 
-    def _mgemm_plan(self, x: torch.Tensor, pw, epi: str) -> tuple[int, int] | None:
-        """(rows per workgroup, split) where the GEMM for a few hundred rows is faster than both.  A K loop asked for by
+    def _prompt_plan(self, x: torch.Tensor, pw, epi: str) -> tuple[int, int, int] | None:
+        """K.prompt_plan, where the GEMM for a few hundred rows is faster than both for some of the rows.  A K loop asked for by
         name, or no lower limit of pgemm's tiles, keeps a product on pgemm."""
         if pw is None or not K.pgemm_ok(x, pw) or not self.PGEMM_MIN_TILES \
                 or (self.pgemm_variant_swiglu if epi == "swiglu" else self.pgemm_variant) != "ppp":
             return None
-        return K.mgemm_plan(x.shape[0], pw.N, pw.K, "whole" if epi == "f32" else "act")
+        return K.prompt_plan(x.shape[0], pw.N, pw.K, "whole" if epi == "f32" else "act")
 
     def _all_reduce(self, x: torch.Tensor) -> torch.Tensor:
         if self.w.tp_size > 1:

@@ -2,7 +2,7 @@
 
 The selection is DecoderModel's: at most K.GEMV_MAX_M rows on the packed GEMV, up to 128 on the decode GEMM,
 thousands on the prefill GEMM's 256 x 256 tiles, what lies between on the GEMM for a few hundred rows
-(K.mgemm_plan), all four reading one fragment-packed bf16 copy.  Shapes those kernels do not take (N or K not a multiple of 64) and 32-bit weights use
+(K.prompt_plan), all four reading one fragment-packed bf16 copy.  Shapes those kernels do not take (N or K not a multiple of 64) and 32-bit weights use
 the library product.  CPU tensors: torch.
 """
 from __future__ import annotations
@@ -60,16 +60,12 @@ class Projection:
             return "lib"
         if x.shape[0] <= K.GEMV_MAX_M:
             return "gemv"
-        if K.mgemm_plan(x.shape[0], self.N, self.K, kind):
+        if K.prompt_plan(x.shape[0], self.N, self.K, kind):
             return "mgemm"
         return "pgemm" if self._prefill(x.shape[0]) else "dgemm"
 
-    def _mgemm(self, x, epi: str, reduce, **kw):
-        """The product with its epilogue, or with what adds its slabs up."""
-        bm, split = K.mgemm_plan(x.shape[0], self.N, self.K)
-        if split == 1:
-            return K.mgemm(x, self.packed, epi, bm, **kw)
-        return reduce(K.mgemm(x, self.packed, "part", bm, split))
+    def _prompt(self, x, epi: str, kind: str = "act", **kw):
+        return K.prompt_gemm(x, self.packed, epi, K.prompt_plan(x.shape[0], self.N, self.K, kind), **kw)
 
     def act(self, x: torch.Tensor) -> torch.Tensor:
         """[M, N] in x's dtype."""
@@ -79,7 +75,7 @@ class Projection:
         if k == "gemv":
             return K.splitk_reduce(K.gemv_part(x, self.packed))
         if k == "mgemm":
-            return self._mgemm(x, "bf16", K.splitk_reduce)
+            return self._prompt(x, "bf16", reduce=K.splitk_reduce)
         if k == "pgemm":
             return K.pgemm(x, self.packed, "bf16", variant="ppp")
         return K.dgemm_linear(x, self.packed)
@@ -93,13 +89,13 @@ class Projection:
         if k in ("gemv", "dgemm", "mgemm"):
             split = K.gemv_packed_config(self.N, self.K, self.packed.bn // 16, M)[0] if k == "gemv" else \
                 K.dgemm_config(M, self.N, self.K, bn=self.packed.bn)[1] if k == "dgemm" else \
-                K.mgemm_plan(M, self.N, self.K, "slabs")[1]
+                K.prompt_plan(M, self.N, self.K, "slabs")[2]
             if own:
                 out = torch.empty(split, M, self.N, dtype=torch.float32, device=x.device)
         if k == "gemv":
             return K.gemv_part(x, self.packed, split, out=out)
         if k == "mgemm":
-            return K.mgemm(x, self.packed, "part", K.mgemm_plan(M, self.N, self.K, "slabs")[0], split, out)
+            return self._prompt(x, "f32", "slabs", out=out)
         if k == "pgemm":
             return K.pgemm(x, self.packed, "f32", variant="ppp")[None]
         if k == "dgemm":
@@ -113,9 +109,9 @@ class Projection:
         """W = 8-row interleaved gate / up rows: the clamped GLU of the product into ``out`` [M, N / 2]
         (row-strided), in the product's epilogue where one pass over (packed) W fills the chip."""
         k, M = self._kernel(x), x.shape[0]
-        if k == "mgemm" and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0:
-            return self._mgemm(x, "glu", lambda s: clamped_glu(s, out, limit, alpha, beta, interleaved=True, cubic=cubic),
-                               out=out, glu=(limit, alpha, beta, cubic))
+        if k == "mgemm" and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
+            return self._prompt(x, "glu", out=out, glu=(limit, alpha, beta, cubic), reduce=lambda slabs, rows: clamped_glu(
+                slabs, rows, limit, alpha, beta, interleaved=True, cubic=cubic))
         if k == "pgemm" and self.K >= 128 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
             return K.pgemm_glu(x, self.packed, out, limit, alpha, beta, cubic)
         if k in ("pgemm", "dgemm") and self.N // self.packed.bn * -(-M // 256) > K.DGEMM_CUS // 2 \
@@ -127,7 +123,7 @@ class Projection:
         """relu(product)^2 [M, N] in x's dtype, in the prompt product's epilogue, else with the sum of the slabs."""
         k = self._kernel(x)
         if k == "mgemm":
-            return self._mgemm(x, "relu2", lambda s: relu_sq(s, x.dtype))
+            return self._prompt(x, "relu2", reduce=lambda slabs, rows: relu_sq(slabs, x.dtype, rows))
         if k == "pgemm" and self.K >= 128:
             return K.pgemm(x, self.packed, "relu2", variant="ppp")
         return relu_sq(self.slabs(x), x.dtype)
@@ -140,7 +136,7 @@ class Projection:
         if k in ("mgemm", "dgemm"):
             out = torch.empty(1, x.shape[0], self.N, dtype=torch.float32, device=x.device)
             if k == "mgemm":
-                return K.mgemm(x, self.packed, "part", K.mgemm_plan(x.shape[0], self.N, self.K, "whole")[0], 1, out)[0]
+                return self._prompt(x, "f32", "whole", out=out)[0]
             return K.dgemm(x, self.packed, "part", 1, part=out)[0]
         if k == "pgemm":
             return K.pgemm(x, self.packed, "f32", variant="ppp")

@@ -780,56 +780,14 @@ def dgemm_glu(x: torch.Tensor, w: "PackedWeight", out: torch.Tensor, limit: floa
     return out
 
 
-MGEMM_MIN_ROWS = 129     # up to 128 rows (its tiles of 64 or 128) the decode GEMM streams W as fast or faster
-
-
-def _mgemm_us(M: int, N: int, Kd: int, bm: int, split: int, fp32: bool = False) -> float:
-    """Time of mgemm.hip in bm-row tiles, as measured for N, K of 1024 .. 28672 and 129 .. 5500 rows (mostly within 10 %).
-    A 64-deep stage takes 0.2 + 0.0013 bm us on an idle chip, up to 0.42 more of that on a full one (0.55 in all rounds
-    but the last), and no less than its 16 KB of W and its rows of X at 67 B/ns: a last tile of few rows runs ahead and
-    brings W into the L2 for the others (385 rows 31 us, 384 rows 40), so they count as fewer rows.  One row tile alone
-    waits for W from memory, 0.59 us (64 workgroups) to 0.75.  4 us per round of workgroups, 6 per call; slabs are
-    written and read, one fp32 result is written, at 7 TB/s."""
-    tm = -(-M // bm)
-    last = M - (tm - 1) * bm
-    rows = last + 0.6 * (bm - last) * (1.0 - 1.0 / tm)
-    wgs = tm * -(-N // 128) * split
-    full, fill = (wgs - 1) // DGEMM_CUS, ((wgs - 1) % DGEMM_CUS + 1) / DGEMM_CUS
-    stages, idle = -(-Kd // (64 * split)), 0.2 + 0.0013 * bm
-    least = max((16384 + 128 * rows) / 67e3, 0.51 + 0.24 * min(1.0, wgs / 192) if tm == 1 else 0.0)
-    t = 6.0 + full * (4.0 + stages * max(idle * 1.55, least)) + 4.0 + stages * max(idle * (1.0 + 0.42 * fill ** 3), least)
-    t = max(t, 10.0 + N * Kd * 2 / 5.0e6)
-    return t + (8.0 * split if split > 1 else 4.0 * fp32) * M * N / 7.0e6
-
-
-def _ppp_us(M: int, N: int, Kd: int) -> float:
-    """Time of pgemm's persistent kernel (measured as above): a K-tile takes 1.4 us in a full round of 256 x 256 tiles,
-    0.8 to 1.22 in a partial one."""
-    full, rest = divmod(-(-M // 256) * -(-N // 256), DGEMM_CUS)
-    return 12.0 + Kd / 64 * (1.4 * full + (0.8 + 0.42 * rest / DGEMM_CUS if rest else 0.0))
-
-
 @functools.lru_cache(maxsize=4096)
-def mgemm_plan(M: int, N: int, Kd: int, kind: str = "act") -> tuple[int, int] | None:
-    """(rows per workgroup, split) of the product on mgemm.hip, None where the decode GEMM (up to 128 rows) or pgemm is
-    the faster one.  ``kind``: "act", an epilogue without a split or the sum of the slabs, 2 us for its launch; "slabs",
-    for a consumer that adds them up; "whole", one fp32 result, which takes pgemm 1.06 times as long.  Splits are powers of two, so that rows multiplied in batches of different sizes
-    are mostly added up in the same order.  (4096 columns, K = 4096: mgemm up to 1800 rows, 61 us against 74; pgemm at 2100,
-    73 against 81.  28672 columns: mgemm up to 260 rows, 89 us against 95; pgemm at 300, 89 against 91.)"""
-    if M < MGEMM_MIN_ROWS or M * Kd * 2 >= 2 ** 32 or N * Kd * 2 >= 2 ** 32:
-        return None
-    # one row tile of the decode GEMM, or few weights: 129 .. 256 rows, 2^23 of them, 17 us against 18; 2^21: 14 against
-    # 15 at 220 rows, 16 against 17 at 512, but 18.6 against 18.3 at 700
-    if N * Kd <= 2 ** 23 and M <= (256 if N * Kd > 2 ** 22 else 640):
-        return None
-    us, bm, split = min((_mgemm_us(M, N, Kd, bm, s, kind != "act") + (2.0 if s > 1 and kind == "act" else 0.0), bm, s)
-                        for bm in (128, 160, 192, 224, 256)
-                        for s in ((1,) if kind == "whole" else (1, 2, 4, 8)) if s * 64 <= Kd)
-    if -(-M // bm) * -(-N // 128) > 3 * DGEMM_CUS:         # not measured to be faster beyond 3 rounds
-        return None
-    if M >= 256 and _ppp_us(M, N, Kd) * (0.97 if kind == "act" else 1.03) <= us:
-        return None
-    return bm, split
+def prompt_plan(M: int, N: int, Kd: int, kind: str = "act") -> tuple[int, int, int] | None:
+    """(head, rows per workgroup, split) of a product whose first ``head`` rows run on pgemm and the others on mgemm; None
+    where all of it is faster on the decode GEMM or on pgemm.  ``kind``: "act", an epilogue without a split or a launch that
+    adds the slabs up; "slabs", for a consumer that does (one slab with a head); "whole", one fp32 result."""
+    plan = (ctypes.c_int * 3)()
+    check(kernels().cfc_prompt_plan(M, N, Kd, ("act", "slabs", "whole").index(kind), ctypes.addressof(plan)), "cfc_prompt_plan")
+    return tuple(plan) if plan[1] else None
 
 
 def mgemm(x: torch.Tensor, w: "PackedWeight", epi: str, bm: int, split: int = 1, out: torch.Tensor | None = None,
@@ -855,6 +813,28 @@ def mgemm(x: torch.Tensor, w: "PackedWeight", epi: str, bm: int, split: int = 1,
             raise ValueError(f"mgemm: out {tuple(out.shape)} {out.dtype}")
     check(kernels().cfc_mgemm(x.data_ptr(), w.data.data_ptr(), out.data_ptr(), M, N, Kd, mode, out.stride(-2), bm, split,
                               w.bn // 16, *map(float, glu), _stream(x)), "cfc_mgemm")
+    return out
+
+
+def prompt_gemm(x: torch.Tensor, w: "PackedWeight", epi: str, plan: tuple[int, int, int], out: torch.Tensor | None = None,
+                reduce=None, glu: tuple = (0.0, 1.0, 0.0, 0.0)) -> torch.Tensor:
+    """A product by :func:`prompt_plan`.  ``epi``: "bf16", "swiglu", "relu2", "glu" as :func:`mgemm`'s, ``reduce(slabs, out)``
+    making a split's result; "f32": fp32 slabs [split, M, N], in the stream's workspace unless a head or ``out`` is given."""
+    (M, _), (head, bm, split) = x.shape, plan
+    if out is None and (epi != "f32" or head):
+        shape = (1, M, w.N) if epi == "f32" else (M, w.N // 2 if epi in ("swiglu", "glu") else w.N)
+        out = torch.empty(shape, dtype=torch.float32 if epi == "f32" else torch.bfloat16, device=x.device)
+    if epi == "f32":
+        if head:
+            pgemm(x[:head], w, "f32", out=out[0, :head], variant="ppp")
+        rest = mgemm(x[head:], w, "part", bm, split, out[:, head:] if out is not None else None)
+        return rest if out is None else out
+    if head:
+        pgemm_glu(x[:head], w, out[:head], *glu) if epi == "glu" else pgemm(x[:head], w, epi, out=out[:head], variant="ppp")
+    if split == 1:
+        mgemm(x[head:], w, epi, bm, 1, out[head:], glu)
+    else:
+        reduce(mgemm(x[head:], w, "part", bm, split), out[head:])
     return out
 
 

@@ -236,11 +236,11 @@ def softcap_(logits: torch.Tensor, cap: float) -> torch.Tensor:
     return logits
 
 
-def relu_sq(x: torch.Tensor, dtype) -> torch.Tensor:
+def relu_sq(x: torch.Tensor, dtype, out: torch.Tensor | None = None) -> torch.Tensor:
     """relu(sum of fp32 slabs [split, T, F])^2 as activations [T, F]."""
     if not x.is_cuda:
         return ref.relu_sq(x.sum(0)).to(dtype)
     _req(x, torch.float32, "x")
-    out = torch.empty(x.shape[1:], dtype=dtype, device=x.device)
+    out = torch.empty(x.shape[1:], dtype=dtype, device=x.device) if out is None else out
     check(kernels().cfc_relu_sq(_act(dtype), out.data_ptr(), x.data_ptr(), x.shape[0], out.numel(), _stream(x)), "cfc_relu_sq")
     return out

@@ -24,6 +24,7 @@
 // us with the sum of the slabs, N x K 6144 x 4096 / 4096 x 4096 / 4096 x 14336, before (decode GEMM or pgemm) -> here:
 //   160 rows 29 / 23 / 44 -> 25 / 22 / 37;  420 rows 40 / 35 / 69 -> 35 / 28 / 59;
 //   1024 rows 74 / 74 / 129 -> 51 / 41 / 105;  1536 rows (75 in pgemm) / 74 / 227 -> - / 50 / 148.
+#include <algorithm>
 #include <type_traits>
 
 #include "pgemm.h"
@@ -208,7 +209,79 @@ int mgemm_launch(const void* x, const void* w, void* out, int M, int N, int K, i
   return (int)hipGetLastError();
 }
 
+// ---- which rows of a product run here.  All times in us, fitted to N, K of 1024 .. 28672 and 129 .. 5500 rows.
+constexpr int MG_CUS = 256;
+
+// mgemm_kernel in bm-row tiles, mostly within 10 %.  A 64-deep stage takes 0.2 + 0.0013 bm on an idle chip, up to 0.42
+// more of that on a full one (0.55 in all rounds but the last), and no less than its 16 KB of W and its rows of X at
+// 67 B/ns: a last tile of few rows runs ahead and brings W into the L2 for the others (385 rows 31 us, 384 rows 40), so
+// they count as fewer rows.  One row tile alone waits for W from memory, 0.59 (64 workgroups) to 0.75.  4 per round of
+// workgroups, 6 per call; slabs are written and read, one fp32 result is written, at 7 TB/s.
+double mgemm_us(int M, int N, int K, int bm, int split, bool fp32) {
+  const int tm = (M + bm - 1) / bm, last = M - (tm - 1) * bm;
+  const double rows = last + 0.6 * (bm - last) * (1.0 - 1.0 / tm);
+  const int64_t wgs = (int64_t)tm * ((N + MG_BN - 1) / MG_BN) * split;
+  const double full = (double)((wgs - 1) / MG_CUS), fill = ((wgs - 1) % MG_CUS + 1) / (double)MG_CUS;
+  const double stages = (K + 64 * split - 1) / (64 * split), idle = 0.2 + 0.0013 * bm;
+  const double least = std::max((16384 + 128 * rows) / 67e3, tm == 1 ? 0.51 + 0.24 * std::min(1.0, wgs / 192.0) : 0.0);
+  double t = 6.0 + full * (4.0 + stages * std::max(idle * 1.55, least)) + 4.0 +
+             stages * std::max(idle * (1.0 + 0.42 * fill * fill * fill), least);
+  t = std::max(t, 10.0 + (double)N * K * 2 / 5.0e6);
+  return t + (split > 1 ? 8.0 * split : 4.0 * fp32) * M * N / 7.0e6;
+}
+
+// pgemm's persistent kernel: a K-tile takes 1.4 in a full round of 256 x 256 tiles, 0.8 to 1.22 in a partial one
+double ppp_us(int M, int N, int K, bool fp32) {
+  const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
+  const int64_t full = tiles / MG_CUS, rest = tiles % MG_CUS;
+  return (12.0 + K / 64 * (1.4 * full + (rest ? 0.8 + 0.42 * rest / MG_CUS : 0.0))) * (fp32 ? 1.06 : 1.0);
+}
+
+enum { MG_ACT = 0, MG_SLABS = 1, MG_WHOLE = 2 };
+
+// the fastest tile and split.  Splits are powers of two, so that rows multiplied in batches of different sizes are
+// mostly added up in the same order; 2 more for the launch that adds an activation's slabs up.  Beyond 3 rounds of
+// workgroups nothing was measured to be faster than pgemm.
+double mgemm_best(int M, int N, int K, int kind, bool split_ok, int& bm, int& split) {
+  double best = 1e30;
+  for (int b = 128; b <= 256; b += 32) {
+    if ((int64_t)((M + b - 1) / b) * ((N + MG_BN - 1) / MG_BN) > 3 * MG_CUS) continue;
+    for (int s = 1; s <= (split_ok ? 8 : 1) && s * 64 <= K; s *= 2) {
+      const double t = mgemm_us(M, N, K, b, s, kind != MG_ACT) + (s > 1 && kind == MG_ACT ? 2.0 : 0.0);
+      if (t < best) best = t, bm = b, split = s;
+    }
+  }
+  return best;
+}
+
 }  // namespace
+
+// A prompt product's plan: plan = {head, bm, split}: `head` rows (whole rounds of pgemm's 256 x 256 tiles) on its
+// persistent kernel and the others here; {0, 0, 0}: all on the decode GEMM or pgemm.  kind 0: an activation (an epilogue,
+// or what adds the slabs up), 1: fp32 slabs for a consumer that adds them up (with a head: one), 2: one fp32 result.
+//   * up to 128 rows, and 256 (640) of 2^23 (2^22) weights or fewer: the decode GEMM (129 .. 256 rows, 2^23 weights: 17
+//     against 18; 2^21: 14 against 15 at 220 rows, 16 against 17 at 512, but 18.6 against 18.3 at 700);
+//   * all here where pgemm's tiles leave the chip idle: 4096 x 4096 up to 1800 rows (61 against 74; 2100: 81 against 73),
+//     28672 x 4096 up to 256 (68 against 87; 300: 91 against 89);
+//   * the rows beyond pgemm's last whole round here: 4096 x 14336 of 4500 rows 512 -> 370, 4096 x 4096 152 -> 124.
+CFC_API int cfc_prompt_plan(int M, int N, int K, int kind, int* plan) {
+  plan[0] = plan[1] = plan[2] = 0;
+  const int64_t weights = (int64_t)N * K;
+  if (M <= 128 || N < 64 || K < 64 || (int64_t)M * K * 2 >= (1ll << 32) || weights * 2 >= (1ll << 32) ||
+      (weights <= 1 << 23 && M <= (weights > 1 << 22 ? 256 : 640)))
+    return 0;
+  int bm = 0, split = 0;
+  double best = M < 256 ? 1e29 : 0.97 * ppp_us(M, N, K, kind != MG_ACT);
+  const double all = mgemm_best(M, N, K, kind, kind != MG_WHOLE, bm, split);
+  if (all < best) best = all, plan[1] = bm, plan[2] = split;
+  const int tn = (N + 255) / 256, tm = (M + 255) / 256;
+  const int rounds = (int)((int64_t)tm * tn / MG_CUS), head = rounds ? (int)((int64_t)MG_CUS * rounds / tn) * 256 : 0;
+  if (head > 0 && head < M && K >= 128) {
+    const double rest = mgemm_best(M - head, N, K, kind, kind == MG_ACT, bm, split);
+    if (ppp_us(head, N, K, kind != MG_ACT) + rest < best) plan[0] = head, plan[1] = bm, plan[2] = split;
+  }
+  return 0;
+}
 
 // epi as cfc_pgemm's (0 bf16, 3 SwiGLU, 4 fp32, 6 squared relu) or 5, the clamped GLU with its constants; out: row stride
 // ldo, or (fp32) slabs [split][M][N].  bm: 128, 160 .. 256 rows per workgroup.  W packed for bn = 16 wnw.

@@ -5,21 +5,24 @@ import torch
 from copilot_for_consensus_amd.models.projection import Projection
 from copilot_for_consensus_amd.ops import kernels as K
 from copilot_for_consensus_amd.ops import reference as ref
+from copilot_for_consensus_amd.ops._native import kernels_available
 
 
+@pytest.mark.skipif(not kernels_available(), reason="the built library is missing")
 def test_plan_takes_what_lies_between_the_decode_gemm_and_pgemm():
     for N, Kd in ((6144, 4096), (4096, 4096), (28672, 4096), (4096, 14336), (1024, 2048), (64, 64)):
         for kind in ("act", "slabs", "whole"):
-            assert all(K.mgemm_plan(M, N, Kd, kind) is None for M in (1, 5, 128))
-            assert K.mgemm_plan(32768, N, Kd, kind) is None or N < 1024
-            for M in range(129, 3000, 97):
-                plan = K.mgemm_plan(M, N, Kd, kind)
+            assert all(K.prompt_plan(M, N, Kd, kind) is None for M in (1, 5, 128))
+            for M in range(129, 20000, 97):
+                plan = K.prompt_plan(M, N, Kd, kind)
                 if plan:
-                    bm, split = plan
+                    head, bm, split = plan
+                    assert 0 <= head < M and head % 256 == 0
                     assert bm in (128, 160, 192, 224, 256) and split in (1, 2, 4, 8) and split * 64 <= Kd
-                    assert kind != "whole" or split == 1
-    assert K.mgemm_plan(700, 4096, 4096) and K.mgemm_plan(1536, 4096, 14336) and not K.mgemm_plan(4096, 28672, 4096)
-    assert K.mgemm_plan(2 ** 19, 64, 4096) is None          # 32-bit DMA offsets
+                    assert split == 1 or kind == "act" or kind == "slabs" and head == 0
+    assert K.prompt_plan(700, 4096, 4096)[0] == 0 and K.prompt_plan(4500, 4096, 14336)[0] == 4096
+    assert K.prompt_plan(4096, 4096, 4096) is None and K.prompt_plan(16384, 28672, 4096) is None
+    assert K.prompt_plan(2 ** 19, 64, 4096) is None         # 32-bit DMA offsets
 
 
 def _data(M, N, Kd, seed, swiglu=False):
@@ -70,7 +73,7 @@ def test_epilogues_round_the_exact_product(bm, M, N, Kd):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M", (129, 256, 300, 700, 1500))
+@pytest.mark.parametrize("M", (129, 256, 300, 700, 1500, 4100, 4500, 8400))
 def test_projection_agrees_with_the_general_path(M, monkeypatch):
     """Every product of a Projection on mgemm and without it: the same sums to fp32, the same rounding."""
     N, Kd = 4096, 2176
@@ -86,9 +89,9 @@ def test_projection_agrees_with_the_general_path(M, monkeypatch):
         p.act(x)                                       # another product: own slabs stay
         assert torch.equal(own.double().sum(0), slabs)
         return slabs, p.f32(x).double(), p.act(x).double(), p.relu_sq(x).double(), p.glu(x, out, 7.0, 1.702, 1.0).double()
-    assert K.mgemm_plan(M, N, Kd)
+    assert K.prompt_plan(M, N, Kd) and K.prompt_plan(M, N, Kd)[0] == M // 4096 * 4096
     new = all_of()
-    monkeypatch.setattr(K, "mgemm_plan", lambda *a: None)
+    monkeypatch.setattr(K, "prompt_plan", lambda *a: None)
     old = all_of()
     for a, b in zip(new[:2], old[:2]):
         assert ((a - b).abs() <= 2 * tol).all()
