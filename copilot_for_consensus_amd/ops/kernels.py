@@ -507,9 +507,6 @@ def lib_splitk_linear_residual_rmsnorm(x: torch.Tensor, w: torch.Tensor, split: 
 
 DGEMM_BNS = (128, 112, 96, 64)   # W rows per workgroup the kernel is built for
 DGEMM_CUS = 256                  # one workgroup per CU
-DGEMM_CU_RATE = 25e9             # W bytes/s one workgroup streams (6.4 TB/s over 256 CUs)
-DGEMM_PART_RATE = 6e12           # fp32 partial slab traffic, bytes/s
-DGEMM_X_RATE = 90e9              # per-CU L2 -> LDS rate of the X re-reads (ablation: X costs ~12 us of gate/up)
 # split-K slabs stored write-through (dgemm.hip DG_PART_WT; CFC_DGEMM_SLAB_WT=0 for plain stores): the
 # kernel boundary no longer writes back 8-17 MB of dirty partials before the reduce / rope_kv may
 # start -- decode 6.48 -> 6.42 s per 128-thread batch, bit-identical (profiles/r05_ab_slab_wt.log)
@@ -566,29 +563,12 @@ def dgemm_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and w.shape[0] % 64 == 0 and x.shape[1] % 64 == 0 and x.shape[0] >= 1)
 
 
+@functools.lru_cache(maxsize=4096)
 def dgemm_config(M: int, N: int, K: int, swiglu: bool = False, bn: int | None = None) -> tuple[int, int]:
-    """(W rows per workgroup, split-K) for one decode projection, from a three-term cost model:
-    each workgroup streams its W slice from HBM at a per-CU rate and re-reads its X slice (every
-    workgroup reads all BM rows of its K range: X traffic / W traffic = BM / BN) from L2 at a
-    per-CU rate, in ceil(blocks / CUs) rounds (a partial second round doubles the time of the CUs
-    that run it), plus the fp32 partial slabs written and read back once.  A fused SwiGLU epilogue
-    needs split 1.  Rates fitted to bench_dgemm.py sweeps on one MI355X (profiles/dgemm_*.txt)."""
-    bm = 64 if M <= 64 else (128 if M <= 128 else 256)
-    mt = (M + bm - 1) // bm
-    best = None
-    for cand in (bn,) if bn else DGEMM_BNS:
-        if N % cand:
-            continue
-        tiles = (N // cand) * mt
-        for split in ([1] if swiglu else range(1, K // 64 + 1)):
-            blocks = tiles * split
-            rounds = -(-blocks // DGEMM_CUS)
-            t = rounds * (cand * K * 2 / split / DGEMM_CU_RATE + bm * K * 2 / split / DGEMM_X_RATE)
-            if split > 1:
-                t += 2 * split * M * N * 4 / DGEMM_PART_RATE
-            if best is None or t < best[0] - 1e-12:
-                best = (t, cand, split)
-    return best[1], best[2]
+    """(W rows per workgroup, split-K) for one decode projection, by the cost model of cfc_dgemm_config (dgemm.hip)."""
+    cfg = (ctypes.c_int * 2)()
+    check(kernels().cfc_dgemm_config(M, N, K, int(swiglu), bn or 0, ctypes.addressof(cfg)), "cfc_dgemm_config")
+    return cfg[0], cfg[1]
 
 
 def dgemm(x: torch.Tensor, w: torch.Tensor, epi: str = "bf16", split: int = 1, bn: int | None = None,

@@ -659,3 +659,33 @@ CFC_API int cfc_dgemm_ablate(const void* x, const void* w, int M, int N, int K, 
   }
   return rc ? rc : CFC_CHECK_LAUNCH();
 }
+
+// (W rows per workgroup, split-K) of one projection: cfg = {bn, split}, from a three-term cost model: each workgroup
+// streams its W slice from HBM at a per-CU rate and re-reads its X slice (all BM rows of its K range: X traffic / W
+// traffic = BM / BN) from L2 at a per-CU rate, in ceil(blocks / CUs) rounds (a partial second round doubles the time of
+// the CUs that run it), plus the fp32 partial slabs written and read back once.  A fused SwiGLU epilogue needs split 1.
+// bn: the width of a packed W, 0 to choose it too.  Rates fitted to sweeps of 64 .. 256 rows; in C because a prompt asks
+// for every product of its row count (K = 14336: 80 us as a Python loop, 1 here).
+CFC_API int cfc_dgemm_config(int M, int N, int K, int swiglu, int bn, int* cfg) {
+  constexpr int CUS = 256;                 // one workgroup per CU
+  constexpr double CU_RATE = 25e9;         // W bytes/s one workgroup streams (6.4 TB/s over 256 CUs)
+  constexpr double PART_RATE = 6e12;       // fp32 partial slab traffic, bytes/s
+  constexpr double X_RATE = 90e9;          // per-CU L2 -> LDS rate of the X re-reads (ablation: X costs ~12 us of gate/up)
+  if (M < 1 || N < 1 || K < 1 || bn < 0) return -1;
+  const int bm = M <= 64 ? 64 : M <= 128 ? 128 : 256;
+  const int64_t mt = (M + bm - 1) / bm;
+  const int widths[4] = {bn ? bn : 128, 112, 96, 64};
+  double best = -1.0;
+  for (int c = 0; c < (bn ? 1 : 4); ++c) {
+    const int w = widths[c];
+    if (N % w) continue;
+    const int64_t tiles = (int64_t)(N / w) * mt;
+    for (int split = 1; split <= (swiglu ? 1 : K / 64); ++split) {
+      const double rounds = (double)((tiles * split + CUS - 1) / CUS);
+      double t = rounds * ((double)w * K * 2 / split / CU_RATE + (double)bm * K * 2 / split / X_RATE);
+      if (split > 1) t += 2.0 * split * M * N * 4 / PART_RATE;
+      if (best < 0 || t < best - 1e-12) best = t, cfg[0] = w, cfg[1] = split;
+    }
+  }
+  return best < 0 ? -1 : 0;
+}
