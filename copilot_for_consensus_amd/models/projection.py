@@ -88,7 +88,7 @@ class Projection:
         M, out = x.shape[0], None
         if k in ("gemv", "dgemm", "mgemm"):
             split = K.gemv_packed_config(self.N, self.K, self.packed.bn // 16, M)[0] if k == "gemv" else \
-                K.dgemm_config(M, self.N, self.K, bn=self.packed.bn)[1] if k == "dgemm" else \
+                K.dgemm_slab_plan(M, self.N, self.K, self.packed.bn)[0] if k == "dgemm" else \
                 K.prompt_plan(M, self.N, self.K, "slabs")[2]
             if own:
                 out = torch.empty(split, M, self.N, dtype=torch.float32, device=x.device)
@@ -99,7 +99,7 @@ class Projection:
         if k == "pgemm":
             return K.pgemm(x, self.packed, "f32", variant="ppp")[None]
         if k == "dgemm":
-            return K.dgemm(x, self.packed, "part", split, part=out)
+            return K.dgemm_slabs(x, self.packed, out)
         w = self.rowmajor()
         if x.is_cuda and x.dtype == torch.bfloat16:
             return torch.mm(x, w.t(), out_dtype=torch.float32)[None]
@@ -198,10 +198,10 @@ class JointProjection:
         else:
             gemv = M <= K.GEMV_MAX_M
             split = K.gemv_packed_config(self.N, self.K, self.packed.bn // 16, M)[0] if gemv else \
-                K.dgemm_config(M, self.N, self.K, bn=self.packed.bn)[1]
+                K.dgemm_slab_plan(M, self.N, self.K, self.packed.bn)[0]
             out = torch.empty(split, M, self.N, dtype=torch.float32, device=acts.device)
             if gemv:
                 K.gemv_part(acts, self.packed, split, out=out, in_of=self.in_of)
             else:
-                K.dgemm_joint(acts, self.packed, self.in_of, out)
+                K.dgemm_slabs(acts, self.packed, out, self.in_of)
         return [Cols(out, o, n) for o, n in zip(self.offsets, self.sizes)]

@@ -113,6 +113,8 @@ _KERNEL_SIGS = {
     "cfc_pgemm_ppp_probe": [P, P, P, I, I, I, I, I, I, I, P],
     "cfc_pgemm_glu": [P, P, P, I, I, I, I, I, F, F, F, F, P],
     "cfc_prompt_plan": [I, I, I, I, P],
+    "cfc_dgemm_stream": [P, P, I, I, I, I, P, P, P],
+    "cfc_dgemm_slab_plan": [I, I, I, I, P],
     "cfc_dgemm_config": [I, I, I, I, I, P],
     "cfc_mgemm": [P, P, P, I, I, I, I, I, I, I, I, F, F, F, F, P],
     "cfc_dgemm_glu": [P, P, I, I, I, I, P, I, F, F, F, F, P],

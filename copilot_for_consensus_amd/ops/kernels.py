@@ -571,6 +571,37 @@ def dgemm_config(M: int, N: int, K: int, swiglu: bool = False, bn: int | None = 
     return cfg[0], cfg[1]
 
 
+@functools.lru_cache(maxsize=4096)
+def dgemm_slab_plan(M: int, N: int, K: int, bn: int) -> tuple[int, bool]:
+    """(slabs, whether they come from one stream over the tiles) of :func:`dgemm_slabs`."""
+    plan = (ctypes.c_int * 2)()
+    check(kernels().cfc_dgemm_slab_plan(M, N, K, bn, ctypes.addressof(plan)), "cfc_dgemm_slab_plan")
+    return plan[0], bool(plan[1])
+
+
+def dgemm_slabs(x: torch.Tensor, w: "PackedWeight", out: torch.Tensor | None = None,
+                in_of: torch.Tensor | None = None) -> torch.Tensor:
+    """fp32 slabs [dgemm_slab_plan's, M, N] whose sum is x @ W^T, in the stream's workspace unless ``out`` is given.
+    ``in_of``: x is [inputs, M, K] and W tile n (bn rows) multiplies input in_of[n]."""
+    M, Kd = x.shape[-2:]
+    slabs, stream = dgemm_slab_plan(M, w.N, Kd, w.bn)
+    if out is None:
+        out = _workspace(x.device, slabs * M * w.N)[:slabs * M * w.N].view(slabs, M, w.N)
+    if not stream:
+        return dgemm(x, w, "part", slabs, part=out) if in_of is None else dgemm_joint(x, w, in_of, out)
+    if not x.is_cuda or x.dtype != torch.bfloat16 or not x.is_contiguous() or Kd != w.K or x.dim() != (2 if in_of is None else 3):
+        raise ValueError(f"dgemm_slabs: x {tuple(x.shape)} {x.dtype} w [{w.N}, {w.K}]")
+    if in_of is not None:
+        _req(in_of, torch.int32, "in_of")
+        if in_of.numel() != w.N // w.bn:
+            raise ValueError(f"dgemm_slabs: {in_of.numel()} tiles of [{w.N}, {w.K}] in {w.bn} rows")
+    if out.shape != (slabs, M, w.N) or out.dtype != torch.float32 or not out.is_contiguous():
+        raise ValueError(f"dgemm_slabs: slabs {tuple(out.shape)} {out.dtype}")
+    check(kernels().cfc_dgemm_stream(x.data_ptr(), w.data.data_ptr(), M, w.N, Kd, w.bn, _p(in_of), out.data_ptr(), _stream(x)),
+          "cfc_dgemm_stream")
+    return out
+
+
 def dgemm(x: torch.Tensor, w: torch.Tensor, epi: str = "bf16", split: int = 1, bn: int | None = None,
           out: torch.Tensor | None = None, part: torch.Tensor | None = None) -> torch.Tensor:
     """One launch of the decode GEMM.  ``epi``: "bf16" -> out [M, N]; "swiglu" -> out [M, N/2]
@@ -624,6 +655,8 @@ def dgemm_linear(x: torch.Tensor, w: torch.Tensor, split: int | None = None, bn:
     bn, split = bn or cbn, split or csplit
     if split == 1:
         return dgemm(x, w, "bf16", bn=bn)
+    if split == csplit and isinstance(w, PackedWeight):
+        return splitk_reduce(dgemm_slabs(x, w))
     return splitk_reduce(dgemm(x, w, "part", split, bn=bn))
 
 
@@ -655,6 +688,8 @@ def dgemm_residual_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Ten
         return _linear_residual_rmsnorm_ref(x, _rowmajor(w), residual, norm_w, eps)
     M, Kd = x.shape
     cbn, csplit = dgemm_config(M, w.shape[0], Kd, bn=getattr(w, "bn", None) or bn)
+    if split is None and isinstance(w, PackedWeight):
+        return splitk_residual_rmsnorm(dgemm_slabs(x, w), residual, norm_w, eps)
     bn, split = bn or cbn, split or csplit
     return splitk_residual_rmsnorm(dgemm(x, w, "part", split, bn=bn), residual, norm_w, eps)
 

@@ -33,6 +33,8 @@
 //
 // MFMA maps (guide §3): A = X rows (m on lane & 15, k = 8 * (lane >> 4) + j), B = W rows (n on
 // lane & 15, same k); C/D: n = lane & 15, m = 4 * (lane >> 4) + i.
+#include <algorithm>
+
 #include "common.h"
 
 namespace {
@@ -417,6 +419,139 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
   }
 }
 
+// The same product with the whole packed matrix as ONE run of 64-deep stages, tile after tile, of which each of gridDim.x
+// workgroups takes an equal share: for tiles x splits that are no whole number of rounds of 256 workgroups (a joint
+// projection of 176 tiles took 10 slices a tile, 7 rounds of short workgroups, to come close).  A workgroup streams W
+// without a stop across tile boundaries -- the packed tiles follow one another -- and stores its sums at each: the parts
+// of a tile go to slabs 0, 1, .. in the order of their workgroups, the last of them filling the slabs that are left with
+// zeros.  One round, `slabs` of 2 or 3.  W tile n multiplies input in_of[n] (null: 0).
+// us, 22528 x 4096 (185 MB, 31 at 5.9 TB/s): 5 rows 44.6 -> 33.8, 12 rows 40.5 -> 35.3; cfc_dgemm_slab_plan has more.
+template <int BM, int BN>
+__global__ void __launch_bounds__((64 * DgShape<BM, BN>::WAVES), 1)
+    dgemm_stream_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, int M, int N, int K, int slabs,
+                        float* __restrict__ part, const int32_t* __restrict__ in_of) {
+  using S = DgShape<BM, BN>;
+  constexpr int NW = S::NW, D = S::D;
+  __shared__ __attribute__((aligned(16))) char smem[S::NSX * S::XSTAGE];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nks = K >> 6, G = gridDim.x, id = xcd_remap(blockIdx.x, G);
+  const int64_t U = (int64_t)(N / BN) * nks;
+  const int64_t u0 = id * U / G;
+  const int nst = (int)((id + 1) * U / G - u0);
+  if (nst == 0) return;
+  const int tile0 = (int)(u0 / nks), k0 = (int)(u0 % nks);
+  const int kq = lane >> 4;
+
+  if (w >= NW) {
+    // ---------------- X loader wave (as dgemm_kernel's)
+    const int l = w - NW;
+    const int prow = lane >> 3, pch = (lane & 7) ^ prow;
+    const uint16_t* xsrc[S::XP];
+#pragma unroll
+    for (int i = 0; i < S::XP; ++i)
+      xsrc[i] = X + (size_t)min(8 * S::XP * l + 8 * i + prow, M - 1) * K + 8 * pch;
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(dg_lds_t*)smem + 8 * S::XP * l * 128);
+    int k = k0, tile = tile0;
+    auto input = [&]() { return in_of ? (size_t)__builtin_amdgcn_readfirstlane(in_of[tile]) * M * K : (size_t)0; };
+    size_t in = input();
+    auto issue = [&](int slot) {
+#pragma unroll
+      for (int i = 0; i < S::XP; ++i) dg_glds16(xsrc[i] + in + (size_t)k * 64, lds0 + slot * S::XSTAGE + i * 1024);
+      if (++k == nks) {
+        k = 0;
+        if (++tile < N / BN) in = input();
+      }
+    };
+#pragma unroll
+    for (int p = 0; p < S::NSX - 1; ++p)
+      if (p < nst) issue(p);
+    int slot = 0;
+    for (int st = 0; st < nst; ++st) {
+      dg_wait_ahead<S::XP, S::NSX - 2>(nst - 1 - st);
+      if (st + S::NSX - 1 < nst) issue(slot == 0 ? S::NSX - 1 : slot - 1);
+      slot = slot + 1 == S::NSX ? 0 : slot + 1;
+    }
+    return;
+  }
+
+  // ---------------- compute wave w: W rows 16 w + (lane & 15) of the current tile
+  uint4 ring[D][2];
+  // a descriptor of this workgroup's run of stages (2 NW KB each)
+  const uint16_t* span = W + (size_t)u0 * BN * 64;
+  const uint32_t span_lo = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)span);
+  const uint32_t span_hi = __builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)span >> 32));
+  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(((uintptr_t)span_hi << 32) | span_lo), (short)0, nst * BN * 128, 0x00020000);
+  const int wvoff = lane * 16, wsoff = w * 1024;
+  // past the run: zeros from an out-of-range offset, no memory access
+  auto load_stage = [&](int s, uint4 (&dst)[2]) {
+    const int so = __builtin_amdgcn_readfirstlane(s < nst ? wsoff + s * 2 * NW * 1024 : 0x40000000);
+    dst[0] = dg_ldw_buf<true>(wrs, wvoff, so);
+    dst[1] = dg_ldw_buf<true>(wrs, wvoff, so + NW * 1024);
+  };
+#pragma unroll
+  for (int p = 0; p < D; ++p) load_stage(p, ring[p]);
+  f32x4_t acc[S::MT];
+#pragma unroll
+  for (int i = 0; i < S::MT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int xoff = (lane & 15) * 128, sw = lane & 7;
+  int xslot = 0, tile = tile0, left = nks - k0;
+
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)part);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)part >> 32));
+  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc((void*)(((uintptr_t)hi << 32) | lo), (short)0, 0x7fffffff, 0x00020000);
+  auto flush = [&](bool whole) {
+    // the workgroup that has the tile's first stage
+    const int first = (int)((((int64_t)tile * nks + 1) * G - 1) / U);
+    const int at = id - first, end = whole ? slabs : at + 1;
+    const int mr = lane & 15, nq = tile * BN + 16 * w + 4 * kq;
+    for (int s = at; s < end; ++s)
+#pragma unroll
+      for (int i = 0; i < S::MT; ++i) {
+        const int m = mr + 16 * i;
+        if (m < M) {
+          const dg_u32x4 v = s == at ? dg_u32x4{__float_as_uint(acc[i][0]), __float_as_uint(acc[i][1]), __float_as_uint(acc[i][2]),
+                                                __float_as_uint(acc[i][3])} : dg_u32x4{0u, 0u, 0u, 0u};
+          __builtin_amdgcn_raw_buffer_store_b128(v, prs, (int)((((size_t)s * M + m) * N + nq) * 4), 0, 16);
+        }
+      }
+#pragma unroll
+    for (int i = 0; i < S::MT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    ++tile;
+    left = nks;
+  };
+  auto compute = [&](const uint4 (&b)[2]) {
+    const char* ximg = smem + xslot * S::XSTAGE + xoff;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int chunk = ((4 * kk + kq) ^ sw) << 4;
+#pragma unroll
+      for (int i = 0; i < S::MT; ++i) acc[i] = dg_mfma(b[kk], *reinterpret_cast<const uint4*>(ximg + i * 16 * 128 + chunk), acc[i]);
+    }
+    xslot = xslot + 1 == S::NSX ? 0 : xslot + 1;
+  };
+  int st = 0;
+  for (; st + D <= nst; st += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      dg_barrier();
+      compute(ring[u]);
+      load_stage(st + u + D, ring[u]);
+      if (--left == 0) flush(true);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < D; ++u) {
+    if (st + u < nst) {
+      dg_barrier();
+      compute(ring[u]);
+      if (--left == 0) flush(true);
+    }
+  }
+  if (left < nks) flush(false);
+}
+
 constexpr bool DG_NT = true;    // nontemporal packed weight stream (bench_dgemm --ablate: ~10 % faster)
 
 template <int BM, int BN, bool NTW, int ABL, bool PK>
@@ -618,6 +753,31 @@ CFC_API int cfc_dgemm_joint(const void* x, const void* w, int M, int N, int K, i
   return rc ? rc : CFC_CHECK_LAUNCH();
 }
 
+// Slabs of cfc_dgemm_stream: the most workgroups that share one tile.
+CFC_API int cfc_dgemm_stream_slabs(int N, int K, int bn) {
+  if (N <= 0 || K < 64 || K % 64 || bn <= 0 || N % bn) return -1;
+  const int64_t nks = K / 64, U = (int64_t)(N / bn) * nks, G = std::min<int64_t>(256, U);
+  int most = 1;
+  for (int64_t t = 0; t < N / bn; ++t)
+    most = std::max(most, (int)((((t + 1) * nks) * G - 1) / U - ((t * nks + 1) * G - 1) / U) + 1);
+  return most;
+}
+
+// dgemm_stream_kernel: x [inputs][M][K], M <= 64, W packed for bn = 64 or 128, part [cfc_dgemm_stream_slabs][M][N]
+CFC_API int cfc_dgemm_stream(const void* x, const void* w, int M, int N, int K, int bn, const int32_t* in_of, float* part,
+                             hipStream_t stream) {
+  if (const int e = dgemm_check(M, N, K, 1, DG_PART_WT, bn, part, nullptr, N)) return e;
+  const int slabs = cfc_dgemm_stream_slabs(N, K, bn);
+  if (M > 64 || (bn != 64 && bn != 128) || (int64_t)slabs * M * N * 4 > 0x7fffffff || (int64_t)N * K * 2 / 256 > 0x3ff00000) return -1;
+#define DG_STREAM(BM, BN)                                                                                       \
+  dgemm_stream_kernel<BM, BN><<<(int)std::min<int64_t>(256, (int64_t)(N / BN) * (K / 64)), 64 * DgShape<BM, BN>::WAVES, 0, stream>>>((const uint16_t*)x, (const uint16_t*)w, M, \
+                                                                              N, K, slabs, part, in_of)
+  if (bn == 64) DG_STREAM(64, 64);
+  else DG_STREAM(64, 128);
+#undef DG_STREAM
+  return CFC_CHECK_LAUNCH();
+}
+
 CFC_API int cfc_dgemm_pack(const void* w, void* wp, int N, int K, int bn, hipStream_t stream) {
   if (N <= 0 || K <= 0 || bn <= 0 || bn % 16 || N % bn || K % 64 || w == wp) return -1;
   const size_t pieces = (size_t)N * K / 8;
@@ -660,32 +820,68 @@ CFC_API int cfc_dgemm_ablate(const void* x, const void* w, int M, int N, int K, 
   return rc ? rc : CFC_CHECK_LAUNCH();
 }
 
-// (W rows per workgroup, split-K) of one projection: cfg = {bn, split}, from a three-term cost model: each workgroup
-// streams its W slice from HBM at a per-CU rate and re-reads its X slice (all BM rows of its K range: X traffic / W
-// traffic = BM / BN) from L2 at a per-CU rate, in ceil(blocks / CUs) rounds (a partial second round doubles the time of
-// the CUs that run it), plus the fp32 partial slabs written and read back once.  A fused SwiGLU epilogue needs split 1.
-// bn: the width of a packed W, 0 to choose it too.  Rates fitted to sweeps of 64 .. 256 rows; in C because a prompt asks
-// for every product of its row count (K = 14336: 80 us as a Python loop, 1 here).
-CFC_API int cfc_dgemm_config(int M, int N, int K, int swiglu, int bn, int* cfg) {
-  constexpr int CUS = 256;                 // one workgroup per CU
-  constexpr double CU_RATE = 25e9;         // W bytes/s one workgroup streams (6.4 TB/s over 256 CUs)
-  constexpr double PART_RATE = 6e12;       // fp32 partial slab traffic, bytes/s
-  constexpr double X_RATE = 90e9;          // per-CU L2 -> LDS rate of the X re-reads (ablation: X costs ~12 us of gate/up)
-  if (M < 1 || N < 1 || K < 1 || bn < 0) return -1;
+namespace {
+constexpr int DG_CUS = 256;                // one workgroup per CU
+
+// us of one launch of dgemm_kernel with its slabs written and read back once: each workgroup streams its W slice from
+// HBM at a per-CU rate and re-reads its X slice (all bm rows of its K range: X traffic / W traffic = bm / bn) from L2 at
+// a per-CU rate, in ceil(blocks / CUs) rounds (a partial second round doubles the time of the CUs that run it).  Rates
+// fitted to sweeps of 64 .. 256 rows; each round after the first costs 1.5 for its start (14336 x 4096, 5 rows: 4 rounds
+// of 9 slices 28.7, one of 2 slices 21.6).
+double dgemm_us(int M, int N, int K, int bn, int split) {
+  constexpr double CU_RATE = 25e3;         // W bytes/us one workgroup streams (6.4 TB/s over 256 CUs)
+  constexpr double PART_RATE = 6e6;        // fp32 partial slab traffic
+  constexpr double X_RATE = 90e3;          // per-CU L2 -> LDS rate of the X re-reads (ablation: X costs ~12 us of gate/up)
   const int bm = M <= 64 ? 64 : M <= 128 ? 128 : 256;
-  const int64_t mt = (M + bm - 1) / bm;
+  const int64_t blocks = (int64_t)(N / bn) * ((M + bm - 1) / bm) * split;
+  const double rounds = (double)((blocks + DG_CUS - 1) / DG_CUS);
+  double t = rounds * ((double)bn * K * 2 / split / CU_RATE + (double)bm * K * 2 / split / X_RATE) + 1.5 * (rounds - 1.0);
+  if (split > 1) t += 2.0 * split * M * N * 4 / PART_RATE;
+  return t;
+}
+
+// us of dgemm_stream_kernel, as measured for 5 .. 64 rows of 9216 .. 22528 columns (within 8 %): 23.5 B/ns of W per CU,
+// a quarter of a percent more per row
+double dgemm_stream_us(int M, int N, int K, int bn, int slabs) {
+  const double stages = (double)(N / bn) * (K / 64) / DG_CUS;
+  return 2.5 + stages * bn * 128 / 23.5e3 * (1.0 + 0.0024 * M) + 2.0 * slabs * M * N * 4 / 6e6;
+}
+
+double dgemm_best(int M, int N, int K, int swiglu, int bn, int* cfg) {
   const int widths[4] = {bn ? bn : 128, 112, 96, 64};
   double best = -1.0;
   for (int c = 0; c < (bn ? 1 : 4); ++c) {
     const int w = widths[c];
     if (N % w) continue;
-    const int64_t tiles = (int64_t)(N / w) * mt;
     for (int split = 1; split <= (swiglu ? 1 : K / 64); ++split) {
-      const double rounds = (double)((tiles * split + CUS - 1) / CUS);
-      double t = rounds * ((double)w * K * 2 / split / CU_RATE + (double)bm * K * 2 / split / X_RATE);
-      if (split > 1) t += 2.0 * split * M * N * 4 / PART_RATE;
-      if (best < 0 || t < best - 1e-12) best = t, cfg[0] = w, cfg[1] = split;
+      const double t = dgemm_us(M, N, K, w, split);
+      if (best < 0 || t < best - 1e-6) best = t, cfg[0] = w, cfg[1] = split;
     }
   }
-  return best < 0 ? -1 : 0;
+  return best;
+}
+}  // namespace
+
+// cfg = {W rows per workgroup, split-K} of one projection.  A fused SwiGLU epilogue needs split 1.  bn: the width of a
+// packed W, 0 to choose it too.  In C because a prompt asks for every product of its row count (K = 14336: 80 us as a
+// Python loop, 1 here).
+CFC_API int cfc_dgemm_config(int M, int N, int K, int swiglu, int bn, int* cfg) {
+  if (M < 1 || N < 1 || K < 1 || bn < 0) return -1;
+  return dgemm_best(M, N, K, swiglu, bn, cfg) < 0 ? -1 : 0;
+}
+
+// plan = {slabs, 1 for dgemm_stream_kernel} of a product that leaves fp32 slabs, W packed for bn.  The stream where it
+// is 7 % faster or more, which it is where no split makes whole rounds (us, 5 / 64 rows, split -> stream: 22528 x 4096
+// 44.6 / 40.2 -> 33.8 / 42.9, 18432 33.4 / 37.2 -> 27.9 / 35.0, 9216 in 64-row tiles 26.5 / 23.3 -> 15.7 / 20.9) and not
+// where one does (4096 x 14336: 21.8 / 23.0 -> 22.6 / 27.7); above 64 rows its workgroups wait for X.
+CFC_API int cfc_dgemm_slab_plan(int M, int N, int K, int bn, int* plan) {
+  int cfg[2];
+  if (M < 1 || N < 1 || K < 1 || bn < 1) return -1;
+  const double t = dgemm_best(M, N, K, 0, bn, cfg);
+  if (t < 0) return -1;
+  plan[0] = cfg[1], plan[1] = 0;
+  if (M > 64 || (bn != 64 && bn != 128) || K % 64) return 0;
+  const int slabs = cfc_dgemm_stream_slabs(N, K, bn);
+  if ((int64_t)slabs * M * N * 4 <= 0x7fffffff && dgemm_stream_us(M, N, K, bn, slabs) < 0.93 * t) plan[0] = slabs, plan[1] = 1;
+  return 0;
 }
