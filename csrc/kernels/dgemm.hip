@@ -157,8 +157,14 @@ struct DgGroup {
   const int32_t* in_of = nullptr;
 };
 
+// Two workgroups per CU: the down products of a batch of experts are several rounds of short workgroups (16 .. 64 stages),
+// whose starts the other one's stream covers; half the ring each, 96 VGPRs, 64 KB of LDS (us of 8 experts of 8192 x 2048:
+// 58.7 -> 55.5, 64 rows 59.7 -> 56.8; gate / up, one round of 128 stages: no difference, one workgroup kept)
+template <int BM, int EPI, int GRP>
+constexpr bool dg_twice() { return BM == 64 && GRP == 1 && EPI == DG_BF16; }
+
 template <int BM, int BN, int EPI, bool NTW, int ABL = 0, bool PACKED = true, int GRP = 0>
-__global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES), 1)
+__global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES), (dg_twice<BM, EPI, GRP>() ? 5 : 1))
     dgemm_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, int M, int N, int K, int ntiles,
                  int split, float* __restrict__ part, uint16_t* __restrict__ out, int ldo, DgGlu gp, DgGroup grp) {
   if constexpr (GRP == 1) {
@@ -168,7 +174,7 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
   }
   using S = DgShape<BM, BN, (ABL & 64) != 0>;
   constexpr int NW = S::NW;
-  constexpr int D = S::D;
+  constexpr int D = dg_twice<BM, EPI, GRP>() ? 4 : S::D;
   __shared__ __attribute__((aligned(16))) char smem[S::NSX * S::XSTAGE];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -873,7 +879,9 @@ CFC_API int cfc_dgemm_config(int M, int N, int K, int swiglu, int bn, int* cfg) 
 // plan = {slabs, 1 for dgemm_stream_kernel} of a product that leaves fp32 slabs, W packed for bn.  The stream where it
 // is 7 % faster or more, which it is where no split makes whole rounds (us, 5 / 64 rows, split -> stream: 22528 x 4096
 // 44.6 / 40.2 -> 33.8 / 42.9, 18432 33.4 / 37.2 -> 27.9 / 35.0, 9216 in 64-row tiles 26.5 / 23.3 -> 15.7 / 20.9) and not
-// where one does (4096 x 14336: 21.8 / 23.0 -> 22.6 / 27.7); above 64 rows its workgroups wait for X.
+// where one does (4096 x 14336: 21.8 / 23.0 -> 22.6 / 27.7; 2048 x 4096 in 64-row tiles is faster in a loop, 7.8 -> 7.3,
+// but slower in a layer, 6.9 -> 7.6: each XCD then needs all of the X that was just written, not one K slice of it);
+// above 64 rows its workgroups wait for X.
 CFC_API int cfc_dgemm_slab_plan(int M, int N, int K, int bn, int* plan) {
   int cfg[2];
   if (M < 1 || N < 1 || K < 1 || bn < 1) return -1;
@@ -882,6 +890,7 @@ CFC_API int cfc_dgemm_slab_plan(int M, int N, int K, int bn, int* plan) {
   plan[0] = cfg[1], plan[1] = 0;
   if (M > 64 || (bn != 64 && bn != 128) || K % 64) return 0;
   const int slabs = cfc_dgemm_stream_slabs(N, K, bn);
-  if ((int64_t)slabs * M * N * 4 <= 0x7fffffff && dgemm_stream_us(M, N, K, bn, slabs) < 0.93 * t) plan[0] = slabs, plan[1] = 1;
+  if ((int64_t)slabs * M * N * 4 > 0x7fffffff) return 0;
+  if (dgemm_stream_us(M, N, K, bn, slabs) < 0.93 * t) plan[0] = slabs, plan[1] = 1;
   return 0;
 }
