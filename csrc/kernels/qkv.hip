@@ -239,7 +239,7 @@ __global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a) {
   }
 }
 
-// Prompt rows from activations: PR_ROWS consecutive rows of one part (0: queries, 1: keys and values) per workgroup, two or four
+// Prompt rows from activations: up to PR_ROWS consecutive rows of one part (0: queries, 1: keys and values) per workgroup, two or four
 // at a time, a vector of V channels per thread.  What the convolution reads back stays in registers, weights are read
 // once, the rows of a time share one reduction.  Heads of a power of two of vectors (per-head norms) and, with a
 // convolution, at most MAX_BACK + 1 taps.
@@ -271,13 +271,13 @@ __device__ __forceinline__ void stw(uint16_t* p, const Vec<8>& r) { *reinterpret
 __device__ __forceinline__ void stw(float* p, const Vec<4>& r) { *reinterpret_cast<float4*>(p) = make_float4(r.v[0], r.v[1], r.v[2], r.v[3]); }
 
 template <typename ACT, int V, int BT, bool CONV>
-__global__ void __launch_bounds__(BT, BT <= 512 ? 4 : 1) qkv_prompt_kernel(QkvArgs a, int T) {
+__global__ void __launch_bounds__(BT, BT <= 512 ? 4 : 1) qkv_prompt_kernel(QkvArgs a, int T, int rows) {
   constexpr int RG = CONV ? 2 : 4, NW = BT / 64;
   __shared__ float red[2][RG][NW];
   __shared__ int4 meta[PR_ROWS];                       // position, rows before it in its portion, cache slot, state slot
   extern __shared__ float2 cs[];                       // [PR_ROWS][rot / 2]
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, part = blockIdx.y;
-  const int t0 = xcd_remap(blockIdx.x, gridDim.x) * PR_ROWS, t1 = min(t0 + PR_ROWS, T);
+  const int t0 = xcd_remap(blockIdx.x, gridDim.x) * rows, t1 = min(t0 + rows, T);
   const int allc = a.H * a.dim + (a.parts > 1 ? a.G * (a.dim + a.vdim) : 0), nk = a.G * a.dim, c = tid * V;
   const int C = part == 0 ? a.H * a.dim : nk, cp = part == 0 ? 0 : a.H * a.dim;
   const bool live = c < (part == 0 ? C : nk + a.G * a.vdim), isv = part == 1 && c >= nk;
@@ -285,7 +285,7 @@ __global__ void __launch_bounds__(BT, BT <= 512 ? 4 : 1) qkv_prompt_kernel(QkvAr
   const float* wn = isv || !live ? nullptr : part == 0 ? a.qn : a.kn;
   const int back = CONV ? a.taps - 1 : 0, half = a.rot / 2;
   const bool turn = !isv && live && cd < a.rot;
-  for (int i = tid; i < PR_ROWS; i += BT) {
+  for (int i = tid; i < rows; i += BT) {
     const int t = min(t0 + i, T - 1);
     meta[i] = make_int4(a.positions[t], a.lead[t], a.cslots ? a.cslots[t] : 0, back ? a.slots[t] : 0);
   }
@@ -314,7 +314,7 @@ __global__ void __launch_bounds__(BT, BT <= 512 ? 4 : 1) qkv_prompt_kernel(QkvAr
 #pragma unroll
   for (int r = 0; r < RG; ++r) win[MAX_BACK + r].get(src + (int64_t)min(t0 + r, T - 1) * a.ld);
   __syncthreads();
-  for (int i = tid; i < PR_ROWS * half; i += BT) {
+  for (int i = tid; i < rows * half; i += BT) {
     float sn, co;
     sincosf((float)meta[i / half].x * a.freq[i % half], &sn, &co);
     cs[i] = make_float2(co, sn);
@@ -431,11 +431,16 @@ int prompt_threads(const QkvArgs& a) {
 
 template <typename ACT, int V>
 int qkv_prompt_go(hipStream_t s, int T, int threads, const QkvArgs& a) {
-  const dim3 grid((T + PR_ROWS - 1) / PR_ROWS, a.parts > 1 ? 2 : 1);
-  const size_t lds = (size_t)PR_ROWS * (a.rot / 2) * sizeof(float2) + 16;
+  // short prompts: fewer rows each, until there is a workgroup per CU (us with 16 rows, here:
+  // 87 rows with a convolution 22.4, 8.9, without 13.0, 5.8; 698 rows 14.7, 8.4)
+  int rows = PR_ROWS;
+  const int parts = a.parts > 1 ? 2 : 1;
+  while (rows > 4 && (T + rows - 1) / rows * parts < 256) rows /= 2;
+  const dim3 grid((T + rows - 1) / rows, parts);
+  const size_t lds = (size_t)rows * (a.rot / 2) * sizeof(float2) + 16;
 #define GO(BT)                                                                             \
-  if (a.conv) qkv_prompt_kernel<ACT, V, BT, true><<<grid, BT, lds, s>>>(a, T);             \
-  else qkv_prompt_kernel<ACT, V, BT, false><<<grid, BT, lds, s>>>(a, T)
+  if (a.conv) qkv_prompt_kernel<ACT, V, BT, true><<<grid, BT, lds, s>>>(a, T, rows);             \
+  else qkv_prompt_kernel<ACT, V, BT, false><<<grid, BT, lds, s>>>(a, T, rows)
   if (threads == 64) { GO(64); }
   else if (threads == 256) { GO(256); }
   else if (threads == 512) { GO(512); }

@@ -124,18 +124,34 @@ __global__ void __launch_bounds__(256) short_conv_kernel(LruArgs a, const int32_
     for (int j = 0; j < TAPS; ++j) w[j] = ldv<V>(a.conv + (size_t)j * W + c);
 #pragma unroll
     for (int j = 0; j + 1 < TAPS; ++j) win[j + 1] = input(j - (TAPS - 1));
-    Vec<V> next = input(0);
-    for (int r = 0; r < n; ++r) {
+    // four rows' loads ahead of their use (698 rows, one ahead: 19.4 us, here 9.3; 14000: 48.6, 49.2)
+    constexpr int AHEAD = 4;
+    Vec<V> nx[AHEAD];
+    auto fetch = [&](int r0) {
 #pragma unroll
-      for (int j = 0; j + 1 < TAPS; ++j) win[j] = win[j + 1];
-      win[TAPS - 1] = next;
-      next = input(min(r + 1, n - 1));
-      Vec<V> y = cb;
+      for (int i = 0; i < AHEAD; ++i) nx[i] = ldv<V>(reinterpret_cast<const ACT*>(a.x.p) + (row0 + min(r0 + i, n - 1)) * a.x.ld + c);
+    };
+    fetch(0);
+    for (int r0 = 0; r0 < n; r0 += AHEAD) {
+      Vec<V> cur[AHEAD];
 #pragma unroll
-      for (int j = 0; j < TAPS; ++j)
+      for (int i = 0; i < AHEAD; ++i)
 #pragma unroll
-        for (int e = 0; e < V; ++e) y.v[e] += w[j].v[e] * win[j].v[e];
-      stv<V>(u + (size_t)(row0 + r) * UW + uc, y);
+        for (int e = 0; e < V; ++e) cur[i].v[e] = nx[i].v[e] + bx.v[e];
+      fetch(r0 + AHEAD);
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) {
+        if (r0 + i >= n) break;
+#pragma unroll
+        for (int j = 0; j + 1 < TAPS; ++j) win[j] = win[j + 1];
+        win[TAPS - 1] = cur[i];
+        Vec<V> y = cb;
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j)
+#pragma unroll
+          for (int e = 0; e < V; ++e) y.v[e] += w[j].v[e] * win[j].v[e];
+        stv<V>(u + (size_t)(row0 + r0 + i) * UW + uc, y);
+      }
     }
   } else {
     for (int r = 0; r < n; ++r) {
