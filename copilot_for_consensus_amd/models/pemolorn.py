@@ -372,7 +372,7 @@ class PemolornModel:
             if isinstance(s.mlp, MoeSpec):
                 src.add("moe")
         if dtype == torch.bfloat16:
-            src |= {"gemm", "dgemm", "pgemm"}
+            src |= {"gemm", "dgemm", "mgemm", "pgemm"}
         return tuple(sorted(src))
 
     def __init__(self, weights: PemolornWeights, tp_group=None, custom_ar=None):

@@ -367,7 +367,7 @@ class TadolixModel:
         for s in cfg.specs:
             src |= {"qkv", "gqa", "gru"} if isinstance(s.mixer, ParallelSpec) else {"rglru"}
         if dtype == torch.bfloat16:
-            src |= {"gemm", "dgemm", "pgemm"}
+            src |= {"gemm", "dgemm", "mgemm", "pgemm"}
         return tuple(sorted(src))
 
     def __init__(self, weights: TadolixWeights, tp_group=None, custom_ar=None):

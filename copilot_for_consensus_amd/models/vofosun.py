@@ -285,7 +285,7 @@ class VofosunModel:
         """csrc/kernels sources a run of this configuration launches kernels from."""
         src = ("elementwise", "stream", "latent")
         if dtype == torch.bfloat16:
-            src += ("gemm", "dgemm", "pgemm")
+            src += ("gemm", "dgemm", "mgemm", "pgemm")
             if any(s.mixer.dim == s.mixer.vdim == L.EXPANDED_DIM for s in cfg.specs):
                 src += ("attention",)
         return src

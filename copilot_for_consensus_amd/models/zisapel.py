@@ -375,7 +375,7 @@ class ZisapelModel:
             if dtype == torch.bfloat16 and isinstance(s.mixer, WindowSpec) and s.mixer.dim == s.mixer.vdim == L.EXPANDED_DIM:
                 src.add("attention")
         if dtype == torch.bfloat16:
-            src |= {"gemm", "dgemm", "pgemm"}
+            src |= {"gemm", "dgemm", "mgemm", "pgemm"}
         return tuple(sorted(src))
 
     def __init__(self, weights: ZisapelWeights, tp_group=None, custom_ar=None):

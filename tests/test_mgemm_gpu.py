@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+from copilot_for_consensus_amd._build import KERNELS_LIB
+from copilot_for_consensus_amd.models import registry
 from copilot_for_consensus_amd.models.projection import Projection
 from copilot_for_consensus_amd.ops import kernels as K
 from copilot_for_consensus_amd.ops import reference as ref
@@ -131,3 +133,14 @@ def test_captured_products_replay():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("preset", ("vofosun-7b", "zisapel-7b", "pemolorn-7b", "tadolix-7b"))
+def test_libraries_of_one_family_hold_every_product(preset):
+    """A library built of the sources that a family names has the entry points of every route of a projection."""
+    cfg = registry.get_config(preset)
+    names = registry.family_of(cfg).model.kernel_sources(cfg, torch.bfloat16)
+    text = "".join((KERNELS_LIB.parents[2] / "csrc" / "kernels" / f"{n}.hip").read_text() for n in names)
+    for entry in ("cfc_prompt_plan", "cfc_mgemm", "cfc_pgemm", "cfc_pgemm_glu", "cfc_dgemm", "cfc_dgemm_config", "cfc_dgemm_slab_plan",
+                  "cfc_dgemm_stream", "cfc_dgemm_joint", "cfc_gemv_packed", "cfc_splitk_reduce", "cfc_clamped_glu"):
+        assert entry + "(" in text, entry
