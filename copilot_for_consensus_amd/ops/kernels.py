@@ -727,7 +727,7 @@ def pgemm(x: torch.Tensor, w, epi: str = "bf16", bias: torch.Tensor | None = Non
     stages of BK=64; "ring5" / "ring4": BK=32 rings of 5 / 4 LDS slots; "pp": two wave groups
     ping-ponging over half-tile stages; "pps": "pp" with the LDS-staged 16-byte-store epilogue;
     "ppp": "pp" made persistent (one workgroup per CU walking the tiles, the DMA stream running on
-    across tile boundaries; packed W, bf16 / SwiGLU epilogues, "pp" otherwise); "w4": four 128x128 waves software-pipelined over a 4-stage ring),
+    across tile boundaries; packed W, bf16 / SwiGLU / squared relu / fp32 epilogues, "pp" otherwise); "w4": four 128x128 waves software-pipelined over a 4-stage ring),
     $CFC_PGEMM_VARIANT when None."""
     mode = PGEMM_EPI[epi]
     packed = isinstance(w, PackedWeight)

@@ -8,7 +8,7 @@ count / get).  Replaces Qdrant / FAISS / Azure AI Search on the hot path (SURVEY
   288 GB MI355X holds 100M x 384 bf16 = 77 GB with room to spare); cosine = dot product of
   L2-normalised rows (normalised on insert by a HIP kernel), or squared-L2 with stored norms
   (FAISS IndexFlatL2 parity, score 1/(1+d), faiss_store.py:224).  Queries: <=16 at a time run the
-  fused MFMA scan kernel, larger batches a hipBLASLt GEMM; exact top-k by the radix-select kernel.
+  fused MFMA scan kernel, larger batches a hipBLASLt GEMM; exact top-k from block maxima in one select kernel.
   Vectors produced on the GPU (the encoder) are inserted without a host round trip.
   Upserts overwrite in place; deletes tombstone + periodic compaction.
 * :class:`HipIVFIndex` -- IVF-flat: k-means coarse quantiser trained on the GPU, rows stored
