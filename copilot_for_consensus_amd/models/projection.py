@@ -109,7 +109,9 @@ class Projection:
         """W = 8-row interleaved gate / up rows: the clamped GLU of the product into ``out`` [M, N / 2]
         (row-strided), in the product's epilogue where one pass over (packed) W fills the chip."""
         k, M = self._kernel(x), x.shape[0]
-        if k == "mgemm" and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
+        # pgemm's part of it stores 16 bytes
+        if k == "mgemm" and (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0 or out.stride(0) % 4 == 0
+                             and out.data_ptr() % 8 == 0 and not K.prompt_plan(M, self.N, self.K)[0]):
             return self._prompt(x, "glu", out=out, glu=(limit, alpha, beta, cubic), reduce=lambda slabs, rows: clamped_glu(
                 slabs, rows, limit, alpha, beta, interleaved=True, cubic=cubic))
         if k == "pgemm" and self.K >= 128 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:

@@ -90,7 +90,11 @@ def test_projection_agrees_with_the_general_path(M, monkeypatch):
         own = p.slabs(x, own=True)
         p.act(x)                                       # another product: own slabs stay
         assert torch.equal(own.double().sum(0), slabs)
-        return slabs, p.f32(x).double(), p.act(x).double(), p.relu_sq(x).double(), p.glu(x, out, 7.0, 1.702, 1.0).double()
+        rows = torch.full((M, N // 2 + 4), 3.0, device="cuda", dtype=torch.bfloat16)          # rows 8 bytes apart from 16
+        glu = p.glu(x, out, 7.0, 1.702, 1.0).double()
+        assert ((p.glu(x, rows[:, 4:], 7.0, 1.702, 1.0).double() - glu).abs() <= 2.0 ** -7 * glu.abs() + 80 * tol.max()).all()
+        assert (rows[:, :4] == 3.0).all()
+        return slabs, p.f32(x).double(), p.act(x).double(), p.relu_sq(x).double(), glu
     assert K.prompt_plan(M, N, Kd) and K.prompt_plan(M, N, Kd)[0] == M // 4096 * 4096
     new = all_of()
     monkeypatch.setattr(K, "prompt_plan", lambda *a: None)
