@@ -906,7 +906,9 @@ struct PfExtra {
   const uint16_t* gate = nullptr;
   int64_t ldg = 0;
 };
-template <int G, bool F8 = false, bool EXP = false, int RD = 0>
+// PARTS: gridDim.z workgroups share a tile, each multiplying 1 / gridDim.z of its row groups (every wave still stages
+// keys and values): short prompts have fewer tiles than CUs, whose SIMDs' two waves then wait for one another.
+template <int G, bool F8 = false, bool EXP = false, int RD = 0, bool PARTS = false>
 __global__ void __launch_bounds__(512, 2) prefill_gqa_kernel(
     const uint16_t* __restrict__ q, const void* __restrict__ kc, const void* __restrict__ vc,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ ctx_lens,
@@ -936,11 +938,15 @@ __global__ void __launch_bounds__(512, 2) prefill_gqa_kernel(
   const int q_begin = cu_q[s], q_len = cu_q[s + 1] - q_begin;
   const int ctx = ctx_lens[s];
   const int pos_base = ctx - q_len;
-  const int row_last = min(qs + QR - 1, q_len - 1);
-  const int kend = pos_base + row_last + 1;         // keys [0, kend) are needed by this tile
+  const int groups = PARTS ? 8 / G / (int)gridDim.z : 8 / G, group0 = PARTS ? (int)blockIdx.z * groups : 0;
+  const bool mine = !PARTS || (rsub >= group0 && rsub < group0 + groups);
+  const int first = qs + 32 * group0;               // the rows this workgroup answers for: first ..
+  if (PARTS && first >= q_len) return;
+  const int row_last = min(first + 32 * groups - 1, q_len - 1);
+  const int kend = pos_base + row_last + 1;         // keys [0, kend) are needed by them
   const int ntiles = (kend + PF_KT - 1) / PF_KT;
-  // sliding window: row at position p sees keys (p - window, p]; the tile's first row bounds it
-  const int kt_begin = window > 0 ? max(0, pos_base + qs - window + 1) / PF_KT : 0;
+  // sliding window: row at position p sees keys (p - window, p]; the first row bounds it
+  const int kt_begin = window > 0 ? max(0, pos_base + first - window + 1) / PF_KT : 0;
   const int32_t* bt = block_tables + (size_t)s * max_blocks;
 
   if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256) __builtin_amdgcn_s_setprio(1);
@@ -1062,7 +1068,7 @@ __global__ void __launch_bounds__(512, 2) prefill_gqa_kernel(
     const char* vb = smem + 32768 + cur * 16384;
     const int key0 = kt * PF_KT;
     const bool below = window > 0 && key0 + PF_KT - 1 <= wave_min_pos - window;  // all keys out of window
-    if (key0 <= wave_min_pos + 31 && !below) {     // else every key of the tile is masked for this wave
+    if (mine && key0 <= wave_min_pos + 31 && !below) {     // else every key of the tile is masked for this wave
       // scores come out of the MFMA already shifted by the running max (the accumulator starts at
       // -m): a tile that needs no rescale goes straight to exp2, without 32 subtractions per lane
       const float mref0 = m == -INFINITY ? 0.f : m;
@@ -1197,7 +1203,7 @@ __global__ void __launch_bounds__(512, 2) prefill_gqa_kernel(
   }
 
   l = pair_sum((lp[0] + lp[1]) + (lp[2] + lp[3]));
-  if (my_row < q_len) {
+  if (mine && my_row < q_len) {
     float inv = l > 0.f ? v_scale / l : 0.f;
     if constexpr (RD != 0) {
       if (ex.sink) {
@@ -1555,7 +1561,19 @@ CFC_API int cfc_prefill_attention(const void* q, const void* k_cache, const void
     tile_seq, tile_q0, scale * LOG2E, Hq, Hkv, max_blocks, window, 1.f, prefill_xcd_local(), (uint16_t*)out
   if (tile_rows != PF_ROWS || (G * tile_rows == 256 && prefill_variant() == 5)) {
     // 5: GQA-packed 8-wave kernel (default)
-    const dim3 grid(n_tiles, Hkv);
+    dim3 grid(n_tiles, Hkv);
+    // parts of tiles while no CU gets two (us whole, in 2 parts: 420 rows, 56 workgroups 20.0, 17.1; 900 rows 33.8, 29.8;
+    // 200 rows behind 1500 keys 52.6, 41.3; four prompts of up to 200 rows 16.0, 13.7)
+    while (n_tiles * Hkv * (int)grid.z * 2 <= 256 && (int)grid.z * 2 <= 8 / G) grid.z *= 2;
+    if (grid.z > 1) {
+      switch (G) {
+        case 1: prefill_gqa_kernel<1, false, false, 0, true><<<grid, 512, lds, stream>>>(PF5_ARGS); break;
+        case 2: prefill_gqa_kernel<2, false, false, 0, true><<<grid, 512, lds, stream>>>(PF5_ARGS); break;
+        case 4: prefill_gqa_kernel<4, false, false, 0, true><<<grid, 512, lds, stream>>>(PF5_ARGS); break;
+        default: return -3;
+      }
+      return CFC_CHECK_LAUNCH();
+    }
     switch (G) {
       case 1: prefill_gqa_kernel<1><<<grid, 512, lds, stream>>>(PF5_ARGS); break;
       case 2: prefill_gqa_kernel<2><<<grid, 512, lds, stream>>>(PF5_ARGS); break;

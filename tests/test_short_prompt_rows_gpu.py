@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from copilot_for_consensus_amd.ops import gqa as A
+from copilot_for_consensus_amd.ops import kernels as K
 from copilot_for_consensus_amd.ops import latent as L
 from copilot_for_consensus_amd.ops.cols import Cols
 from copilot_for_consensus_amd.runtime.kv_cache import PagedHeads
@@ -61,3 +62,30 @@ def test_gathered_latents_are_the_cache_rows(n_tiles):
     part = rows[1].view(n_tiles, RV // 32, 4, 64, 8)
     src = want[:, :RV].view(n_tiles, 64, RV // 32, 4, 8).permute(0, 2, 1, 3, 4)
     assert torch.equal(part.reshape(n_tiles, RV // 32, -1).sort(-1).values, src.reshape(n_tiles, RV // 32, -1).sort(-1).values)
+
+
+@pytest.mark.parametrize("window", (0, 100))
+@pytest.mark.parametrize("H, G", [(4, 4), (4, 2), (8, 2), (16, 8)])
+@pytest.mark.parametrize("lens, past", [((1,), 0), ((33,), 0), ((63, 2), 5), ((300,), 0), ((65, 97, 128), 70), ((420,), 31)])
+def test_attention_of_a_short_prompt_shares_its_tiles(lens, past, H, G, window):
+    """One to eight workgroups per tile against one (the same sequences often enough to fill the chip): bit for bit."""
+    dev, D = "cuda", 128
+    g = torch.Generator(dev).manual_seed(sum(lens) + past)
+    nb = [-(-(n + past) // 32) for n in lens]
+    kc = torch.randn(sum(nb), G, 32, D, device=dev, generator=g).bfloat16()
+    vc = torch.randn(sum(nb), G, 4, D, 8, device=dev, generator=g).bfloat16().view(sum(nb), G, 32, D)
+    q1 = torch.randn(sum(lens), H, D, device=dev, generator=g).bfloat16()
+    table = torch.zeros(len(lens), max(nb), dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(nb):
+        table[i, :n] = torch.arange(at, at + n)
+        at += n
+
+    def run(copies):
+        cu = [0]
+        for n in lens * copies:
+            cu.append(cu[-1] + n)
+        return K.prefill_attention(q1.repeat(copies, 1, 1), kc, vc, table.repeat(copies, 1).to(dev),
+                                   torch.tensor(cu, dtype=torch.int32, device=dev),
+                                   torch.tensor([n + past for n in lens] * copies, dtype=torch.int32, device=dev), D ** -0.5, window=window)
+    assert torch.equal(run(1), run(260)[:sum(lens)])
