@@ -98,9 +98,9 @@ _KERNEL_SIGS = {
     "cfc_prefill_attention_expanded": [P, P, P, P, c_int64, P, P, P, P, I, I, F, P, c_int64, P],
     "cfc_enc_rows": [I],
     "cfc_enc_forward": [P] * 10 + [I, I, I, I, P, I, F, F, I] + [P] * 6,
-    "cfc_knn_scan": [P, P, I, I, I, P, P, P, P, L, P, I, I, P],
+    "cfc_knn_scan": [P, P, I, I, I, P, P, P, P, L, P, L, P],
     "cfc_topk_block": [I],
-    "cfc_topk_select": [P, P, I, I, L, I, P, I, L, P, P, P],
+    "cfc_topk_select": [P, P, I, I, L, I, P, L, I, L, P, P, P],
     "cfc_knn_topk_rows": [],
     "cfc_ivf_topk": [P, P, I, I, I, P, P, P, P, I, P, I, I, P, P, P],
     "cfc_l2_normalize": [P, P, P, I, I, P],

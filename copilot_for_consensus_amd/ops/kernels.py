@@ -1499,9 +1499,13 @@ def _knn_scan(X, Q, xnorm2, qnorm2, alive, row_lo: int, N: int, out, bmax) -> No
     def at(t, step=1):
         return None if t is None else t.data_ptr() + row_lo * step * t.element_size()
     lib, n = kernels(), N - row_lo
-    B = lib.cfc_topk_block(n)
     check(lib.cfc_knn_scan(at(X, X.shape[1]), Q.data_ptr(), n, Q.shape[0], X.shape[1], at(xnorm2), _p(qnorm2), at(alive),
-                           out.data_ptr(), out.stride(0), _p(bmax), -(-n // B), B, _stream(X)), "cfc_knn_scan")
+                           out.data_ptr(), out.stride(0), _p(bmax), 0 if bmax is None else bmax.numel(), _stream(X)), "cfc_knn_scan")
+
+
+def _topk_blocks(n: int) -> int:
+    """Block maxima of n scores.  Not monotonic: 2^k * 16384 scores have 16384 blocks, one more has 8193 of twice the size."""
+    return -(-n // kernels().cfc_topk_block(n))
 
 
 def knn_scores(X, Q, xnorm2=None, qnorm2=None, out=None):
@@ -1520,11 +1524,11 @@ def _select(scores, n: int, k: int, ids, bmax, row_lo: int = 0):
     lib, nq, dev = kernels(), scores.shape[0], scores.device
     fill = bmax is None
     if fill:
-        bmax = torch.empty(nq, -(-n // lib.cfc_topk_block(n)), dtype=torch.int32, device=dev)
+        bmax = torch.empty(nq * _topk_blocks(n), dtype=torch.int32, device=dev)
     v = torch.empty(nq, k, dtype=torch.float32, device=dev)
     i = torch.empty(nq, k, dtype=torch.int64, device=dev)
-    check(lib.cfc_topk_select(scores.data_ptr(), _p(ids), nq, n, scores.stride(0), k, bmax.data_ptr(), int(fill), row_lo, v.data_ptr(),
-                              i.data_ptr(), _stream(scores)), "cfc_topk_select")
+    check(lib.cfc_topk_select(scores.data_ptr(), _p(ids), nq, n, scores.stride(0), k, bmax.data_ptr(), bmax.numel(), int(fill),
+                              row_lo, v.data_ptr(), i.data_ptr(), _stream(scores)), "cfc_topk_select")
     return v, i
 
 
@@ -1557,9 +1561,9 @@ def knn_topk(X, Q, k: int, xnorm2=None, qnorm2=None, alive=None, row_lo: int = 0
     if not 1 <= k <= 256 or not 1 <= nq <= 16 or N <= row_lo:
         raise ValueError(f"knn_topk: k {k} (1 to 256), {nq} queries (1 to 16), rows {row_lo} to {N}")
     step = min(N - row_lo, KNN_SCORES // nq)
-    nb = -(-step // kernels().cfc_topk_block(step))
+    last = (N - row_lo - 1) % step + 1             # rows of the last span, which may have more blocks than a full one
     sc = torch.empty(nq, -(-step // 4) * 4, dtype=torch.float32, device=X.device)
-    bmax = torch.empty(nq * nb, dtype=torch.int32, device=X.device)
+    bmax = torch.empty(nq * max(_topk_blocks(step), _topk_blocks(last)), dtype=torch.int32, device=X.device)
     parts = []
     for lo in range(row_lo, N, step):
         n = min(step, N - lo)

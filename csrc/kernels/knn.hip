@@ -511,13 +511,20 @@ __global__ void __launch_bounds__(256) pool_kernel(float* __restrict__ out_f32, 
 
 }  // namespace
 
-// Scores of rows [0, N) of X for nq queries into out [nq][ld], and every B rows' largest key into bmax
-// [nq][nb] (null: not wanted).  out 16-byte aligned.
+// Rows per block for the top-k of n scores: as small as the select kernel's number of blocks allows.
+CFC_API int cfc_topk_block(int n) {
+  int b = 16;
+  while ((long)b * SEL_BLOCKS < n) b *= 2;
+  return b;
+}
+
+// Scores of rows [0, N) of X for nq queries into out [nq][ld], and the largest key of every cfc_topk_block(N) rows into
+// bmax [nq][blocks] (null: not wanted), which has room for `room` of them.  out 16-byte aligned.
 CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
-                         const uint8_t* alive, float* out, long ld, uint32_t* bmax, int nb, int B, hipStream_t stream) {
-  if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || B < 16 || B % 16 != 0 || (long)nb * B < N || (long)(nb - 1) * B >= N ||
-      ld < N)
-    return -1;
+                         const uint8_t* alive, float* out, long ld, uint32_t* bmax, long room, hipStream_t stream) {
+  if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || ld < N) return -1;
+  const int B = cfc_topk_block(N), nb = (N - 1) / B + 1;
+  if (bmax && (long)nq * nb > room) return -1;
 #define KS(KC) knn_scan_kernel<KC><<<(nb + 3) / 4, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, \
       qnorm2, alive, out, (size_t)ld, bmax, nb, B); break
   switch (dim / 32) {
@@ -533,19 +540,13 @@ CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, c
   return CFC_CHECK_LAUNCH();
 }
 
-// Rows per block for the top-k of n scores: as small as the select kernel's number of blocks allows.
-CFC_API int cfc_topk_block(int n) {
-  int b = 16;
-  while ((long)b * SEL_BLOCKS < n) b *= 2;
-  return b;
-}
-
-// Sorted top-k of in [nq][n] (row stride ld) -> out [nq][k], k <= n.  bmax [nq][ceil(n / B)], B = cfc_topk_block(n):
-// block maxima from cfc_knn_scan, or (fill) workspace that is filled here.
-CFC_API int cfc_topk_select(const float* in, const int64_t* ids, int nq, int n, long ld, int k, uint32_t* bmax, int fill,
-                            long row0, float* out_v, int64_t* out_i, hipStream_t stream) {
+// Sorted top-k of in [nq][n] (row stride ld) -> out [nq][k], k <= n.  bmax [nq][ceil(n / B)], B = cfc_topk_block(n), with
+// room for `room` maxima: those from cfc_knn_scan, or (fill) workspace that is filled here.
+CFC_API int cfc_topk_select(const float* in, const int64_t* ids, int nq, int n, long ld, int k, uint32_t* bmax, long room,
+                            int fill, long row0, float* out_v, int64_t* out_i, hipStream_t stream) {
   if (nq < 1 || k <= 0 || k > SEL_K || k > n || ld < n) return -1;
-  const int B = cfc_topk_block(n), nb = (n + B - 1) / B;
+  const int B = cfc_topk_block(n), nb = (n - 1) / B + 1;
+  if ((long)nq * nb > room) return -1;
   if (fill) block_max_kernel<<<dim3((nb + 3) / 4, nq), 256, 0, stream>>>(in, n, (size_t)ld, B, bmax, nb);
   topk_select_kernel<<<nq, SEL_THREADS, 0, stream>>>(in, n, (size_t)ld, B, bmax, nb, k, ids, row0, out_v, out_i);
   return CFC_CHECK_LAUNCH();

@@ -1,0 +1,52 @@
+"""A flat search in spans of rows: what knn_topk allots and refuses, without a GPU."""
+import types
+
+import pytest
+import torch
+
+from copilot_for_consensus_amd.ops import kernels as K
+from copilot_for_consensus_amd.ops._native import kernels, kernels_available
+
+pytestmark = pytest.mark.skipif(not kernels_available(), reason="the built library is missing")
+
+
+def _fake(*shape):
+    """A tensor on the GPU as far as knn_topk looks at it: its launches are recorded, not made."""
+    return types.SimpleNamespace(shape=shape, is_cuda=True, device="cpu")
+
+
+def _search(monkeypatch, rows, nq, k=10, row_lo=0):
+    spans = []
+
+    def scan(X, Q, xnorm2, qnorm2, alive, lo, hi, out, bmax):
+        spans.append((lo, hi, out, bmax))
+
+    def select(scores, n, k, ids, bmax, row_lo=0):
+        return torch.zeros(nq, k), torch.zeros(nq, k, dtype=torch.long)
+    monkeypatch.setattr(K, "_knn_scan", scan)
+    monkeypatch.setattr(K, "_select", select)
+    K.knn_topk(_fake(row_lo + rows, 128), _fake(nq, 128), k, row_lo=row_lo)
+    return spans
+
+
+@pytest.mark.parametrize("nq", range(1, 17))
+def test_every_span_has_room_for_its_block_maxima(monkeypatch, nq):
+    """A last span of fewer rows may have more blocks than a full one: 15 queries take spans of 4473924 rows, 8739 blocks, and
+    262144 rows are 16384."""
+    step = K.KNN_SCORES // nq
+    rests = {1, 5003, step - 1, step} | {16384 * 2 ** a + d for a in range(4, 13) for d in (-1, 0, 1)}
+    sizes = {1_000_000, 5_500_000, 10_000_000, 35_000_000, 100_000_000} | {step + r for r in rests} | {2 * step + r for r in rests}
+    for rows in sorted(n for n in sizes if 0 < n <= 100_000_000):
+        spans = _search(monkeypatch, rows, nq, row_lo=7)
+        assert spans[0][0] == 7 and spans[-1][1] == 7 + rows and all(a[1] == b[0] for a, b in zip(spans, spans[1:]))
+        for lo, hi, out, bmax in spans:
+            n = hi - lo
+            assert out.shape[0] == nq and n <= out.shape[1]
+            assert bmax.numel() >= nq * -(-n // kernels().cfc_topk_block(n)), (rows, n)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="looks at what is refused before any launch")
+def test_entries_refuse_too_little_room():
+    room = 15 * -(-4_473_924 // kernels().cfc_topk_block(4_473_924))
+    assert kernels().cfc_knn_scan(None, None, 262_144, 15, 128, None, None, None, None, 262_144, 16, room, None) == -1
+    assert kernels().cfc_topk_select(None, None, 15, 262_144, 262_144, 10, 16, room, 0, 0, None, None, None) == -1

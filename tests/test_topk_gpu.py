@@ -51,3 +51,15 @@ def test_knn_topk_in_spans(monkeypatch, dim, nq, N, lo):
     monkeypatch.setattr(K, "KNN_SCORES", nq * max(1, (N - lo) // 5))
     many = K.knn_topk(X, Q, k, alive=alive, row_lo=lo, N=N)
     assert torch.equal(one[0], many[0]) and torch.equal(one[1], many[1])
+
+
+def test_a_last_span_of_more_blocks(monkeypatch):
+    """Spans of 270000 rows, 8438 blocks of 32, and a last one of 262000, 16375 blocks of 16."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    nq, dim, N, k = 3, 128, 532_000, 100
+    g = torch.Generator(device=DEV).manual_seed(N)
+    X, Q = (torch.randn(n, dim, device=DEV, generator=g).bfloat16() for n in (N, nq))
+    rv, ri = K.knn_scores(X, Q).sort(dim=1, descending=True, stable=True)
+    monkeypatch.setattr(K, "KNN_SCORES", nq * 270_000)
+    v, i = K.knn_topk(X, Q, k)
+    assert torch.equal(v, rv[:, :k]) and torch.equal(i, ri[:, :k])
