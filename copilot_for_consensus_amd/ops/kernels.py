@@ -1558,8 +1558,8 @@ def knn_topk(X, Q, k: int, xnorm2=None, qnorm2=None, alive=None, row_lo: int = 0
             sc = sc.masked_fill(~alive[row_lo:N].bool()[None], float("-inf"))
         v, i = torch.topk(sc.float(), min(k, N - row_lo), dim=1)
         return v, i + row_lo
-    if not 1 <= k <= 256 or not 1 <= nq <= 16 or N <= row_lo:
-        raise ValueError(f"knn_topk: k {k} (1 to 256), {nq} queries (1 to 16), rows {row_lo} to {N}")
+    if not 1 <= k <= 256 or not 1 <= nq <= 16 or not 0 <= row_lo < N <= X.shape[0]:
+        raise ValueError(f"knn_topk: k {k} (1 to 256), {nq} queries (1 to 16), rows {row_lo} to {N} of {X.shape[0]}")
     step = min(N - row_lo, KNN_SCORES // nq)
     last = (N - row_lo - 1) % step + 1             # rows of the last span, which may have more blocks than a full one
     sc = torch.empty(nq, -(-step // 4) * 4, dtype=torch.float32, device=X.device)

@@ -50,3 +50,10 @@ def test_entries_refuse_too_little_room():
     room = 15 * -(-4_473_924 // kernels().cfc_topk_block(4_473_924))
     assert kernels().cfc_knn_scan(None, None, 262_144, 15, 128, None, None, None, None, 262_144, 16, room, None) == -1
     assert kernels().cfc_topk_select(None, None, 15, 262_144, 262_144, 10, 16, room, 0, 0, None, None, None) == -1
+
+
+@pytest.mark.parametrize("lo, hi", [(-1, 100), (-5, 0), (0, 101), (50, 50), (60, 50), (100, 101)])
+def test_rows_outside_the_index_are_refused(monkeypatch, lo, hi):
+    monkeypatch.setattr(K, "_knn_scan", lambda *a: pytest.fail("launched"))
+    with pytest.raises(ValueError):
+        K.knn_topk(_fake(100, 128), _fake(1, 128), 10, row_lo=lo, N=hi)
