@@ -1494,13 +1494,18 @@ def decode_advance(next_ids, tokens, step, input_ids, positions, ctx_lens, slots
 
 # ----------------------------------------------------------------------------- vector search
 
+def _row_stride(t: torch.Tensor, n: int) -> int:
+    """Elements between rows of n scores in ``t``.  One row's stride says nothing: a column transposed counts as contiguous."""
+    return t.stride(0) if t.dim() == 2 and t.stride(0) >= n else n
+
+
 def _knn_scan(X, Q, xnorm2, qnorm2, alive, row_lo: int, N: int, out, bmax) -> None:
     """Scores of rows [row_lo, N) into ``out`` [nq, >= rows] and their block maxima into ``bmax`` (or None)."""
     def at(t, step=1):
         return None if t is None else t.data_ptr() + row_lo * step * t.element_size()
     lib, n = kernels(), N - row_lo
     check(lib.cfc_knn_scan(at(X, X.shape[1]), Q.data_ptr(), n, Q.shape[0], X.shape[1], at(xnorm2), _p(qnorm2), at(alive),
-                           out.data_ptr(), out.stride(0), _p(bmax), 0 if bmax is None else bmax.numel(), _stream(X)), "cfc_knn_scan")
+                           out.data_ptr(), _row_stride(out, n), _p(bmax), 0 if bmax is None else bmax.numel(), _stream(X)), "cfc_knn_scan")
 
 
 def _topk_blocks(n: int) -> int:
@@ -1527,7 +1532,7 @@ def _select(scores, n: int, k: int, ids, bmax, row_lo: int = 0):
         bmax = torch.empty(nq * _topk_blocks(n), dtype=torch.int32, device=dev)
     v = torch.empty(nq, k, dtype=torch.float32, device=dev)
     i = torch.empty(nq, k, dtype=torch.int64, device=dev)
-    check(lib.cfc_topk_select(scores.data_ptr(), _p(ids), nq, n, scores.stride(0), k, bmax.data_ptr(), bmax.numel(), int(fill),
+    check(lib.cfc_topk_select(scores.data_ptr(), _p(ids), nq, n, _row_stride(scores, n), k, bmax.data_ptr(), bmax.numel(), int(fill),
                               row_lo, v.data_ptr(), i.data_ptr(), _stream(scores)), "cfc_topk_select")
     return v, i
 

@@ -56,6 +56,7 @@ __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restric
   }
   const float qn = (qnorm2 && qv) ? qnorm2[col] : 0.f;
   const int lo = blk * B, hi = min(N, lo + B);
+  const bool vec = (ld & 3) == 0 && ((uintptr_t)out & 15) == 0;
   uint32_t best = 0u;
   auto load = [&](uint4* a, int r0) {
     const uint16_t* xr = X + (size_t)min(r0 + col, N - 1) * D;
@@ -78,7 +79,7 @@ __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restric
       if (rb + i < N) best = max(best, f2key(v[i]));
     }
     float* o = out + col * ld + rb;
-    if (rb + 3 < N && (ld & 3) == 0) {
+    if (rb + 3 < N && vec) {
       *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
     } else {
 #pragma unroll
@@ -519,7 +520,7 @@ CFC_API int cfc_topk_block(int n) {
 }
 
 // Scores of rows [0, N) of X for nq queries into out [nq][ld], and the largest key of every cfc_topk_block(N) rows into
-// bmax [nq][blocks] (null: not wanted), which has room for `room` of them.  out 16-byte aligned.
+// bmax [nq][blocks] (null: not wanted), which has room for `room` of them.
 CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
                          const uint8_t* alive, float* out, long ld, uint32_t* bmax, long room, hipStream_t stream) {
   if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || ld < N) return -1;

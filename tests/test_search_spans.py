@@ -57,3 +57,27 @@ def test_rows_outside_the_index_are_refused(monkeypatch, lo, hi):
     monkeypatch.setattr(K, "_knn_scan", lambda *a: pytest.fail("launched"))
     with pytest.raises(ValueError):
         K.knn_topk(_fake(100, 128), _fake(1, 128), 10, row_lo=lo, N=hi)
+
+
+def _strides(monkeypatch):
+    """Row strides that the entries are called with."""
+    seen = []
+    lib = types.SimpleNamespace(cfc_topk_block=kernels().cfc_topk_block, cfc_knn_scan=lambda *a: seen.append(a[9]) or 0,
+                                cfc_topk_select=lambda *a: seen.append(a[4]) or 0)
+    monkeypatch.setattr(K, "kernels", lambda: lib)
+    monkeypatch.setattr(K, "_stream", lambda t: None)
+    return seen
+
+
+def test_rows_of_scores_keep_their_distance(monkeypatch):
+    """A column transposed is one contiguous row of stride 1; a flat result is rows one after the other."""
+    seen = _strides(monkeypatch)
+    X, Q, Q1 = (types.SimpleNamespace(shape=(n, 128), is_cuda=True, device="cpu", data_ptr=lambda: 0, element_size=lambda: 2)
+                for n in (40, 3, 1))
+    for q, out, want in ((Q, None, 40), (Q, torch.empty(3, 52)[:, :40], 52), (Q, torch.empty(120), 40), (Q1, torch.empty(40, 1).t(), 40),
+                         (Q1, torch.empty(2, 44)[1:, 4:], 44)):
+        K.knn_scores(X, q, out=out)
+        assert seen.pop() == want
+    for scores, want in ((torch.empty(40, 1).t(), 40), (torch.empty(3, 52)[:, :40].contiguous(), 40), (torch.empty(3, 52), 52)):
+        K._select(scores, 40, 5, None, None)
+        assert seen.pop() == want

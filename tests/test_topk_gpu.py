@@ -63,3 +63,24 @@ def test_a_last_span_of_more_blocks(monkeypatch):
     monkeypatch.setattr(K, "KNN_SCORES", nq * 270_000)
     v, i = K.knn_topk(X, Q, k)
     assert torch.equal(v, rv[:, :k]) and torch.equal(i, ri[:, :k])
+
+
+def test_one_row_and_results_of_other_strides():
+    """A transposed column; results given flat, 4 bytes off 16, in wider rows."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(7)
+    s = torch.randn(5003, 1, device=DEV, generator=g)
+    v, i = K.topk(s.t(), 40)
+    rv, ri = s.t().sort(dim=1, descending=True, stable=True)
+    assert torch.equal(v, rv[:, :40]) and torch.equal(i, ri[:, :40])
+    for nq, N in ((3, 1000), (1, 1001)):
+        X, Q = (torch.randn(n, 128, device=DEV, generator=g).bfloat16() for n in (N, nq))
+        want = K.knn_scores(X, Q)
+        flat = torch.full((nq * N + 2,), 7.0, device=DEV)
+        wide = torch.full((nq, N + 5), 7.0, device=DEV)
+        K.knn_scores(X, Q, out=flat[1:-1])
+        K.knn_scores(X, Q, out=wide[:, 3:N + 3])
+        assert torch.equal(flat[1:-1].view(nq, N), want) and flat[0] == flat[-1] == 7.0
+        assert torch.equal(wide[:, 3:N + 3], want) and (wide[:, :3] == 7.0).all() and (wide[:, N + 3:] == 7.0).all()
+        if nq == 1:
+            assert torch.equal(K.knn_scores(X, Q, out=torch.empty(N, 1, device=DEV).t()), want)
