@@ -141,15 +141,32 @@ __device__ __forceinline__ int sel_count(int c, int (*red)[SEL_WAVES], int& turn
   return t;
 }
 
-// The candidates cut to their kk largest (cnt > kk; all differ, as each holds its row).  Any bound that
-// exactly kk of them reach will do, so the bitwise search ends where the count fits.
-__device__ __forceinline__ void sel_cut(uint64_t* cand, int cnt, int kk, int (*red)[SEL_WAVES], int& turn, int* s_n) {
+// The candidates cut to their kk largest (cnt > kk; all differ, as each holds its row); what all of those reach is returned.
+// Any bound that exactly kk of them reach will do, so the bitwise search begins below the bits that all candidates share
+// (of equal scores, the upper half) and ends where the count fits.
+__device__ __forceinline__ uint64_t sel_cut(uint64_t* cand, int cnt, int kk, int (*red)[SEL_WAVES], int& turn, int* s_n,
+                                            uint64_t (*bits)[SEL_WAVES]) {
   const int tid = threadIdx.x, lane = tid & 63;
-  uint64_t e[SEL_CAP / SEL_THREADS];
+  uint64_t e[SEL_CAP / SEL_THREADS], all = ~0ull, any = 0ull;
 #pragma unroll
-  for (int j = 0; j < SEL_CAP / SEL_THREADS; ++j) e[j] = tid + j * SEL_THREADS < cnt ? cand[tid + j * SEL_THREADS] : 0ull;
-  uint64_t thr = 0;
-  for (int b = 63; b >= 0; --b) {
+  for (int j = 0; j < SEL_CAP / SEL_THREADS; ++j) {
+    const bool in = tid + j * SEL_THREADS < cnt;
+    e[j] = in ? cand[tid + j * SEL_THREADS] : 0ull;
+    any |= e[j];
+    if (in) all &= e[j];
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    all &= (uint64_t)__shfl_xor((unsigned long long)all, o, 64);
+    any |= (uint64_t)__shfl_xor((unsigned long long)any, o, 64);
+  }
+  if (lane == 0) { bits[0][tid >> 6] = all; bits[1][tid >> 6] = any; }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < SEL_WAVES; ++i) { all &= bits[0][i]; any |= bits[1][i]; }
+  const int top = 63 - __clzll((long long)(all ^ any));     // they differ: two candidates or more
+  uint64_t thr = top == 63 ? 0ull : any >> (top + 1) << (top + 1);
+  for (int b = top; b >= 0; --b) {
     const uint64_t t = thr | (1ull << b);
     int c = 0;
 #pragma unroll
@@ -170,12 +187,17 @@ __device__ __forceinline__ void sel_cut(uint64_t* cand, int cnt, int kk, int (*r
     if (p) cand[at] = e[j];
   }
   __syncthreads();
+  return thr;
 }
 
 // Sorted top-k of a query's n scores, one workgroup per query.  Largest first, the lower row first among
 // equals.  bmax [nq][nb] holds the largest key of every B rows.  At least k blocks hold a score at or
 // above the k-th best maximum, so no lower score is among the k best: the scores of the blocks that reach
-// this bound (about k of them) are read, those at or above it kept, cut to k and ranked.
+// this bound (about k of them) are read, those at or above it kept, cut to k and ranked.  Where many blocks' maxima equal
+// the bound (equal scores, or all but a few masked), the first of them do, as many as are missing: each holds a score of
+// that value, at a lower row than any later block's.  Once cut, the k kept bound what may still come.  (300 of 1M: equal
+// scores 48 us where looking at every block that reaches the bound took 5075, all but 100 masked 81 where it took 5586,
+// others as before, 33; the radix passes 258, 189 and 176.)
 // A chain of short steps: 18 us for 150 of 1M scores, where three rounds of radix histograms in LDS over
 // 2048-row chunks' winners and a library sort took 120.
 // ids (row stride ld, optional): what the rows are called; else row0 + row.
@@ -187,6 +209,8 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
   __shared__ uint16_t list[SEL_BLOCKS];
   __shared__ int red[2][SEL_WAVES], s_n, s_list;
   __shared__ uint32_t s_lo[SEL_WAVES], s_hi[SEL_WAVES];
+  __shared__ uint64_t bits[2][SEL_WAVES];
+  __shared__ uint16_t ties[SEL_BLOCKS / SEL_THREADS][SEL_WAVES];
   const int tid = threadIdx.x, lane = tid & 63, qi = blockIdx.x;
   const uint64_t below = (1ull << lane) - 1ull;
   int turn = 0;
@@ -199,6 +223,7 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
   // a bound that k blocks reach, and not many more (none: every block is looked at); the search begins
   // below the bits that all maxima share
   uint32_t thr = 0;
+  int reach = nb;                                    // blocks that do
   if (nb > k) {
     uint32_t lo = ~0u, hi = 0u;
 #pragma unroll
@@ -226,9 +251,32 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
 #pragma unroll
         for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) c += __popcll(__ballot(key[j] >= t));
         c = sel_count(c, red, turn);
-        if (c >= k) thr = t;
+        if (c >= k) thr = t, reach = c;
         if (c >= k && c <= k + k / 4) break;
       }
+    }
+  }
+  uint32_t drop = 0;                                 // bit j: block j of this thread is not looked at
+  if (nb > k && reach > k + k / 4) {                 // thr is the k-th best maximum itself
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
+      const uint64_t m = __ballot(tid + j * SEL_THREADS < nb && key[j] == thr);
+      if (lane == 0) ties[j][tid >> 6] = (uint16_t)__popcll(m);
+      c += __popcll(__ballot(key[j] > thr));
+    }
+    const int missing = k - sel_count(c, red, turn);
+    int before = 0;                                  // ties in lower blocks
+#pragma unroll
+    for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
+      const bool tie = tid + j * SEL_THREADS < nb && key[j] == thr;
+      int mine = before + __popcll(__ballot(tie) & below);
+#pragma unroll 1
+      for (int i = 0; i < SEL_WAVES; ++i) {
+        if (i < tid >> 6) mine += ties[j][i];
+        before += ties[j][i];
+      }
+      if (tie && mine >= missing) drop |= 1u << j;
     }
   }
   if (tid == 0) { s_n = 0; s_list = 0; }
@@ -236,7 +284,7 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
 #pragma unroll
   for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
     const int i = tid + j * SEL_THREADS;
-    const bool p = i < nb && key[j] >= thr;
+    const bool p = i < nb && key[j] >= thr && !(drop >> j & 1);
     const uint64_t m = __ballot(p);
     int at = 0;
     if (lane == 0 && m) at = atomicAdd(&s_list, __popcll(m));
@@ -263,17 +311,17 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
   };
   int row = place(4 * tid);
   float4 x = load(row);
+  uint64_t floor = (uint64_t)thr << 32;               // no lower candidate is among the k best
   for (long s0 = 0; s0 < total; s0 += SEL_STEP) {
     const int row1 = place(s0 + SEL_STEP + 4 * tid);
     const float4 x1 = load(row1);                     // the next step's, under this one's work
     const float v[4] = {x.x, x.y, x.z, x.w};
-    uint32_t kv[4];
-    uint64_t m[4];
+    uint64_t e[4], m[4];
     int mine = 0;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      kv[u] = f2key(v[u]);
-      m[u] = __ballot(row + u < n && kv[u] >= thr);
+      e[u] = ((uint64_t)f2key(v[u]) << 32) | (0xffffffffu - (uint32_t)(row + u));
+      m[u] = __ballot(row + u < n && e[u] >= floor);
       mine += __popcll(m[u]);
     }
     if (mine) {
@@ -282,7 +330,7 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
       at = __shfl(at, 0, 64);
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        if (m[u] >> lane & 1) cand[at + __popcll(m[u] & below)] = ((uint64_t)kv[u] << 32) | (0xffffffffu - (uint32_t)(row + u));
+        if (m[u] >> lane & 1) cand[at + __popcll(m[u] & below)] = e[u];
         at += __popcll(m[u]);
       }
     }
@@ -291,9 +339,9 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
     __syncthreads();
     const int cnt = s_n;
     __syncthreads();
-    if (cnt > SEL_CAP - SEL_STEP) sel_cut(cand, cnt, k, red, turn, &s_n);   // the next step might not fit
+    if (cnt > SEL_CAP - SEL_STEP) floor = sel_cut(cand, cnt, k, red, turn, &s_n, bits);   // the next step might not fit
   }
-  if (s_n > max(k, SEL_THREADS)) sel_cut(cand, s_n, k, red, turn, &s_n);
+  if (s_n > max(k, SEL_THREADS)) sel_cut(cand, s_n, k, red, turn, &s_n, bits);
   const int cnt = s_n;                                // at least min(k, n)
   for (int i = tid; i < cnt; i += SEL_THREADS) {
     const uint64_t e = cand[i];
