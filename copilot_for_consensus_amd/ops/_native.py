@@ -100,6 +100,7 @@ _KERNEL_SIGS = {
     "cfc_enc_forward": [P] * 10 + [I, I, I, I, P, I, F, F, I] + [P] * 6,
     "cfc_knn_scan": [P, P, I, I, I, P, P, P, P, L, P, L, P],
     "cfc_topk_block": [I],
+    "cfc_topk_segment": [I],
     "cfc_topk_select": [P, P, I, I, L, I, P, L, I, L, P, P, P],
     "cfc_knn_topk_rows": [],
     "cfc_ivf_topk": [P, P, I, I, I, P, P, P, P, I, P, I, I, P, P, P],

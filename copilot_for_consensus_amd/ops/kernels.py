@@ -1525,16 +1525,18 @@ def knn_scores(X, Q, xnorm2=None, qnorm2=None, out=None):
 
 def _select(scores, n: int, k: int, ids, bmax, row_lo: int = 0):
     """(values, ids) [nq, k] descending of the first ``n`` scores of every row of ``scores`` (the lower index first among
-    equals); ``bmax``: their block maxima (None: taken here); ``ids``: the scores' ids (None: row_lo + index)."""
+    equals); ``bmax``: their block maxima (None: taken here); ``ids``: the scores' ids (None: row_lo + index).  Many scores
+    are selected from in segments, and then from the segments' winners, whose order is that of their rows among equals."""
     lib, nq, dev = kernels(), scores.shape[0], scores.device
+    parts = -(-n // lib.cfc_topk_segment(n))
     fill = bmax is None
     if fill:
         bmax = torch.empty(nq * _topk_blocks(n), dtype=torch.int32, device=dev)
-    v = torch.empty(nq, k, dtype=torch.float32, device=dev)
-    i = torch.empty(nq, k, dtype=torch.int64, device=dev)
+    v = torch.empty(nq, parts * k, dtype=torch.float32, device=dev)
+    i = torch.empty(nq, parts * k, dtype=torch.int64, device=dev)
     check(lib.cfc_topk_select(scores.data_ptr(), _p(ids), nq, n, _row_stride(scores, n), k, bmax.data_ptr(), bmax.numel(), int(fill),
                               row_lo, v.data_ptr(), i.data_ptr(), _stream(scores)), "cfc_topk_select")
-    return v, i
+    return (v, i) if parts == 1 else _select(v, parts * k, k, i, None)
 
 
 def topk(scores: torch.Tensor, k: int, ids: torch.Tensor | None = None):

@@ -125,7 +125,8 @@ __global__ void __launch_bounds__(256) block_max_kernel(const float* __restrict_
 }
 
 constexpr int SEL_THREADS = 1024, SEL_WAVES = SEL_THREADS / 64;
-constexpr int SEL_BLOCKS = 16384;      // most blocks of a query (16 maxima per thread)
+constexpr int SEL_BLOCKS = 16384;      // most blocks of a workgroup (16 maxima per thread)
+constexpr int SEL_WIDEST = 64;         // most rows of a block: more scores than these hold go in segments
 constexpr int SEL_CAP = 8192;          // candidates held
 constexpr int SEL_STEP = 4096;         // scores looked at between two looks at the candidates' number
 constexpr int SEL_K = 2048;            // most winners: SEL_K + SEL_STEP <= SEL_CAP
@@ -201,7 +202,10 @@ __device__ __forceinline__ uint64_t sel_cut(uint64_t* cand, int cnt, int kk, int
 // A chain of short steps: 18 us for 150 of 1M scores, where three rounds of radix histograms in LDS over
 // 2048-row chunks' winners and a library sort took 120.
 // ids (row stride ld, optional): what the rows are called; else row0 + row.
-__global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* __restrict__ in, int n, size_t ld, int B,
+// grid (queries, segments): workgroup y selects from `seg` of the n scores, a whole number of blocks of B, into
+// out [query][y].  One workgroup brings in 25 B/ns: more than 2^20 scores are shared out, and their winners selected from
+// again (us for 2048 of 20M in one, here: 983, 316; rising scores 4435, 448; the radix passes 634 and 808).
+__global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* __restrict__ in, int n, size_t ld, int B, int seg,
                                                                   const uint32_t* __restrict__ bmax, int nb, int k,
                                                                   const int64_t* __restrict__ ids, int64_t row0,
                                                                   float* __restrict__ out_v, int64_t* __restrict__ out_i) {
@@ -213,12 +217,23 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
   __shared__ uint16_t ties[SEL_BLOCKS / SEL_THREADS][SEL_WAVES];
   const int tid = threadIdx.x, lane = tid & 63, qi = blockIdx.x;
   const uint64_t below = (1ull << lane) - 1ull;
+  {
+    const size_t first = (size_t)blockIdx.y * seg;
+    in += qi * ld + first;
+    if (ids) ids += qi * ld + first;
+    row0 += first;
+    bmax += (size_t)qi * nb + first / B;
+    out_v += ((size_t)qi * gridDim.y + blockIdx.y) * k;
+    out_i += ((size_t)qi * gridDim.y + blockIdx.y) * k;
+    n = (int)min((size_t)seg, n - first);
+    nb = (n - 1) / B + 1;
+  }
   int turn = 0;
   uint32_t key[SEL_BLOCKS / SEL_THREADS];
 #pragma unroll
   for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
     const int i = tid + j * SEL_THREADS;
-    key[j] = i < nb ? bmax[(size_t)qi * nb + i] : 0u;
+    key[j] = i < nb ? bmax[i] : 0u;
   }
   // a bound that k blocks reach, and not many more (none: every block is looked at); the search begins
   // below the bits that all maxima share
@@ -294,8 +309,8 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
   __syncthreads();
   const int lb = 31 - __clz(B);                      // B is a power of two
   const long total = (long)s_list << lb;             // scores to look at, four neighbours per thread
-  const float* src = in + (size_t)qi * ld;
-  const bool vec = (ld & 3) == 0 && ((uintptr_t)in & 15) == 0;
+  const float* src = in;
+  const bool vec = ((uintptr_t)in & 15) == 0;
   auto place = [&](long at) { return at < total ? ((int)list[at >> lb] << lb) + (int)(at & (B - 1)) : n; };
   auto load = [&](int row) {
     float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -350,8 +365,8 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
     for (int j = 0; j < cnt; ++j) rank += cand[j] > e;
     if (rank >= k) continue;
     const uint32_t r = 0xffffffffu - (uint32_t)e;
-    out_v[(size_t)qi * k + rank] = key2f((uint32_t)(e >> 32));
-    out_i[(size_t)qi * k + rank] = ids ? ids[(size_t)qi * ld + r] : row0 + r;
+    out_v[rank] = key2f((uint32_t)(e >> 32));
+    out_i[rank] = ids ? ids[r] : row0 + r;
   }
 }
 
@@ -563,8 +578,16 @@ __global__ void __launch_bounds__(256) pool_kernel(float* __restrict__ out_f32, 
 // Rows per block for the top-k of n scores: as small as the select kernel's number of blocks allows.
 CFC_API int cfc_topk_block(int n) {
   int b = 16;
-  while ((long)b * SEL_BLOCKS < n) b *= 2;
+  while (b < SEL_WIDEST && (long)b * SEL_BLOCKS < n) b *= 2;
   return b;
+}
+
+// Scores per workgroup of the select kernel: all n, or equal shares of whole blocks.
+CFC_API int cfc_topk_segment(int n) {
+  constexpr int most = SEL_BLOCKS * SEL_WIDEST;
+  if (n <= most) return n;
+  const int parts = (n - 1) / most + 1;
+  return ((n - 1) / parts / SEL_WIDEST + 1) * SEL_WIDEST;
 }
 
 // Scores of rows [0, N) of X for nq queries into out [nq][ld], and the largest key of every cfc_topk_block(N) rows into
@@ -589,15 +612,16 @@ CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, c
   return CFC_CHECK_LAUNCH();
 }
 
-// Sorted top-k of in [nq][n] (row stride ld) -> out [nq][k], k <= n.  bmax [nq][ceil(n / B)], B = cfc_topk_block(n), with
-// room for `room` maxima: those from cfc_knn_scan, or (fill) workspace that is filled here.
+// Sorted top-k of every segment of in [nq][n] (row stride ld) -> out [nq][segments][k], k no more than a segment has.
+// bmax [nq][ceil(n / B)], B = cfc_topk_block(n), with room for `room` maxima: those from cfc_knn_scan, or (fill) workspace
+// that is filled here.
 CFC_API int cfc_topk_select(const float* in, const int64_t* ids, int nq, int n, long ld, int k, uint32_t* bmax, long room,
                             int fill, long row0, float* out_v, int64_t* out_i, hipStream_t stream) {
-  if (nq < 1 || k <= 0 || k > SEL_K || k > n || ld < n) return -1;
-  const int B = cfc_topk_block(n), nb = (n - 1) / B + 1;
-  if ((long)nq * nb > room) return -1;
+  if (nq < 1 || n < 1 || k <= 0 || k > SEL_K || ld < n) return -1;
+  const int B = cfc_topk_block(n), nb = (n - 1) / B + 1, seg = cfc_topk_segment(n), parts = (n - 1) / seg + 1;
+  if ((long)nq * nb > room || k > n - (parts - 1) * seg) return -1;
   if (fill) block_max_kernel<<<dim3((nb + 3) / 4, nq), 256, 0, stream>>>(in, n, (size_t)ld, B, bmax, nb);
-  topk_select_kernel<<<nq, SEL_THREADS, 0, stream>>>(in, n, (size_t)ld, B, bmax, nb, k, ids, row0, out_v, out_i);
+  topk_select_kernel<<<dim3(nq, parts), SEL_THREADS, 0, stream>>>(in, n, (size_t)ld, B, seg, bmax, nb, k, ids, row0, out_v, out_i);
   return CFC_CHECK_LAUNCH();
 }
 

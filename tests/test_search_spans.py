@@ -29,14 +29,17 @@ def _search(monkeypatch, rows, nq, k=10, row_lo=0):
     return spans
 
 
+@pytest.mark.parametrize("small", (False, True))
 @pytest.mark.parametrize("nq", range(1, 17))
-def test_every_span_has_room_for_its_block_maxima(monkeypatch, nq):
-    """A last span of fewer rows may have more blocks than a full one: 15 queries take spans of 4473924 rows, 8739 blocks, and
-    262144 rows are 16384."""
+def test_every_span_has_room_for_its_block_maxima(monkeypatch, nq, small):
+    """A last span of fewer rows may have more blocks than a full one: 270000 rows are 8438 blocks of 32, 262144 rows 16384
+    blocks of 16."""
+    if small:
+        monkeypatch.setattr(K, "KNN_SCORES", nq * 270_000)
     step = K.KNN_SCORES // nq
     rests = {1, 5003, step - 1, step} | {16384 * 2 ** a + d for a in range(4, 13) for d in (-1, 0, 1)}
     sizes = {1_000_000, 5_500_000, 10_000_000, 35_000_000, 100_000_000} | {step + r for r in rests} | {2 * step + r for r in rests}
-    for rows in sorted(n for n in sizes if 0 < n <= 100_000_000):
+    for rows in sorted(n for n in sizes if 0 < n <= min(100_000_000, 30 * step)):
         spans = _search(monkeypatch, rows, nq, row_lo=7)
         assert spans[0][0] == 7 and spans[-1][1] == 7 + rows and all(a[1] == b[0] for a, b in zip(spans, spans[1:]))
         for lo, hi, out, bmax in spans:
@@ -47,7 +50,7 @@ def test_every_span_has_room_for_its_block_maxima(monkeypatch, nq):
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="looks at what is refused before any launch")
 def test_entries_refuse_too_little_room():
-    room = 15 * -(-4_473_924 // kernels().cfc_topk_block(4_473_924))
+    room = 15 * -(-270_000 // kernels().cfc_topk_block(270_000))
     assert kernels().cfc_knn_scan(None, None, 262_144, 15, 128, None, None, None, None, 262_144, 16, room, None) == -1
     assert kernels().cfc_topk_select(None, None, 15, 262_144, 262_144, 10, 16, room, 0, 0, None, None, None) == -1
 
@@ -62,8 +65,8 @@ def test_rows_outside_the_index_are_refused(monkeypatch, lo, hi):
 def _strides(monkeypatch):
     """Row strides that the entries are called with."""
     seen = []
-    lib = types.SimpleNamespace(cfc_topk_block=kernels().cfc_topk_block, cfc_knn_scan=lambda *a: seen.append(a[9]) or 0,
-                                cfc_topk_select=lambda *a: seen.append(a[4]) or 0)
+    lib = types.SimpleNamespace(cfc_topk_block=kernels().cfc_topk_block, cfc_topk_segment=kernels().cfc_topk_segment,
+                                cfc_knn_scan=lambda *a: seen.append(a[9]) or 0, cfc_topk_select=lambda *a: seen.append(a[4]) or 0)
     monkeypatch.setattr(K, "kernels", lambda: lib)
     monkeypatch.setattr(K, "_stream", lambda t: None)
     return seen
@@ -81,3 +84,13 @@ def test_rows_of_scores_keep_their_distance(monkeypatch):
     for scores, want in ((torch.empty(40, 1).t(), 40), (torch.empty(3, 52)[:, :40].contiguous(), 40), (torch.empty(3, 52), 52)):
         K._select(scores, 40, 5, None, None)
         assert seen.pop() == want
+
+
+def test_segments_cover_the_scores_in_whole_blocks():
+    """Every workgroup's share fits its registers' block maxima, and the last one holds as many as can be asked for."""
+    lib = kernels()
+    for n in [1, 15, 2048, 262_144, 262_145] + [(1 << 20) * a + d for a in (1, 2, 3, 7, 64, 2000) for d in (-1, 0, 1, 63, 64, 65, 500_000)]:
+        seg, B = lib.cfc_topk_segment(n), lib.cfc_topk_block(n)
+        parts = -(-n // seg)
+        assert -(-seg // B) <= 16384 and B in (16, 32, 64)
+        assert parts == 1 or seg % B == 0 and n - (parts - 1) * seg >= 2048
