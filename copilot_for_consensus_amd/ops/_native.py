@@ -99,6 +99,8 @@ _KERNEL_SIGS = {
     "cfc_enc_rows": [I],
     "cfc_enc_forward": [P] * 10 + [I, I, I, I, P, I, F, F, I] + [P] * 6,
     "cfc_knn_scan": [P, P, I, I, I, P, P, P, P, L, P, L, P],
+    "cfc_knn_maxima": [P, P, I, I, I, P, P, P, P, L, P],
+    "cfc_knn_blocks": [P, P, I, I, I, P, P, P, P, I, L, P, P, P, P],
     "cfc_topk_block": [I],
     "cfc_topk_segment": [I],
     "cfc_topk_select": [P, P, I, I, L, I, P, L, I, L, P, P, P],

@@ -1499,13 +1499,17 @@ def _row_stride(t: torch.Tensor, n: int) -> int:
     return t.stride(0) if t.dim() == 2 and t.stride(0) >= n else n
 
 
-def _knn_scan(X, Q, xnorm2, qnorm2, alive, row_lo: int, N: int, out, bmax) -> None:
-    """Scores of rows [row_lo, N) into ``out`` [nq, >= rows] and their block maxima into ``bmax`` (or None)."""
+def _knn_args(X, Q, xnorm2, qnorm2, alive, row_lo: int, N: int) -> tuple:
+    """The leading arguments of a kernel over rows [row_lo, N)."""
     def at(t, step=1):
         return None if t is None else t.data_ptr() + row_lo * step * t.element_size()
-    lib, n = kernels(), N - row_lo
-    check(lib.cfc_knn_scan(at(X, X.shape[1]), Q.data_ptr(), n, Q.shape[0], X.shape[1], at(xnorm2), _p(qnorm2), at(alive),
-                           out.data_ptr(), _row_stride(out, n), _p(bmax), 0 if bmax is None else bmax.numel(), _stream(X)), "cfc_knn_scan")
+    return at(X, X.shape[1]), Q.data_ptr(), N - row_lo, Q.shape[0], X.shape[1], at(xnorm2), _p(qnorm2), at(alive)
+
+
+def _knn_scan(X, Q, xnorm2, qnorm2, alive, row_lo: int, N: int, out, bmax) -> None:
+    """Scores of rows [row_lo, N) into ``out`` [nq, >= rows] and their block maxima into ``bmax`` (or None)."""
+    check(kernels().cfc_knn_scan(*_knn_args(X, Q, xnorm2, qnorm2, alive, row_lo, N), out.data_ptr(), _row_stride(out, N - row_lo),
+                                 _p(bmax), 0 if bmax is None else bmax.numel(), _stream(X)), "cfc_knn_scan")
 
 
 def _topk_blocks(n: int) -> int:
@@ -1551,12 +1555,16 @@ def topk(scores: torch.Tensor, k: int, ids: torch.Tensor | None = None):
     return _select(scores.contiguous(), n, k_eff, None if ids is None else ids.contiguous(), None)
 
 
-KNN_SCORES = 1 << 26     # scores of one pass over (part of) an index: 256 MB of workspace, what the last-level cache holds
+# Rows whose scores a flat search stores, to select from what one workgroup takes; of more it stores every 16 rows' best
+# score and scores the winning blocks again.  us, stored / scored again, 1 query top-10 and 16 queries top-150: 500 k rows
+# of 384 79 / 93 and 103 / 122, 1 M 146 / 157 and 187 / 194, 1.2 M 180 / 183 and 241 / 224, 4 M 542 / 526 and 692 / 614,
+# 20 M 2606 / 2489 and 3349 / 2791: the stores take four times their share of the bytes.
+KNN_SCORES = 1 << 20
 
 
 def knn_topk(X, Q, k: int, xnorm2=None, qnorm2=None, alive=None, row_lo: int = 0, N: int | None = None):
     """Flat scan + top-k over rows [row_lo, N) of X for <= 16 queries and k <= 256: (scores [nq, k] descending, row
-    indices [nq, k]).  The scores of at most KNN_SCORES rows and queries are held at a time."""
+    indices [nq, k]).  Workspace: a score per query and row up to KNN_SCORES rows, of more one per 16 rows."""
     N = X.shape[0] if N is None else N
     nq = Q.shape[0]
     if not X.is_cuda:
@@ -1567,18 +1575,24 @@ def knn_topk(X, Q, k: int, xnorm2=None, qnorm2=None, alive=None, row_lo: int = 0
         return v, i + row_lo
     if not 1 <= k <= 256 or not 1 <= nq <= 16 or not 0 <= row_lo < N <= X.shape[0]:
         raise ValueError(f"knn_topk: k {k} (1 to 256), {nq} queries (1 to 16), rows {row_lo} to {N} of {X.shape[0]}")
-    step = min(N - row_lo, KNN_SCORES // nq)
-    last = (N - row_lo - 1) % step + 1             # rows of the last span, which may have more blocks than a full one
-    sc = torch.empty(nq, -(-step // 4) * 4, dtype=torch.float32, device=X.device)
-    bmax = torch.empty(nq * max(_topk_blocks(step), _topk_blocks(last)), dtype=torch.int32, device=X.device)
-    parts = []
-    for lo in range(row_lo, N, step):
-        n = min(step, N - lo)
-        _knn_scan(X, Q, xnorm2, qnorm2, alive, lo, lo + n, sc, bmax)
-        parts.append(_select(sc, n, min(k, n), None, bmax, lo))
-    if len(parts) == 1:
-        return parts[0]
-    return topk(torch.cat([v for v, _ in parts], 1), k, torch.cat([i for _, i in parts], 1))
+    n, dev, lib = N - row_lo, X.device, kernels()
+    if n <= KNN_SCORES:
+        sc = torch.empty(nq, -(-n // 4) * 4, dtype=torch.float32, device=dev)
+        bmax = torch.empty(nq * _topk_blocks(n), dtype=torch.int32, device=dev)
+        _knn_scan(X, Q, xnorm2, qnorm2, alive, row_lo, N, sc, bmax)
+        return _select(sc, n, min(k, n), None, bmax, row_lo)
+    args = _knn_args(X, Q, xnorm2, qnorm2, alive, row_lo, N)
+    nb = -(-n // 16)
+    best = torch.empty(nq, -(-nb // 4) * 4, dtype=torch.float32, device=dev)
+    check(lib.cfc_knn_maxima(*args, best.data_ptr(), best.shape[1], _stream(X)), "cfc_knn_maxima")
+    kb = min(k, nb)                     # the blocks of the k best maxima, lowest first among equals, hold the k best rows
+    _, blocks = _select(best, nb, kb, None, None)
+    sc = torch.empty(nq, 16 * kb, dtype=torch.float32, device=dev)
+    ids = torch.empty(nq, 16 * kb, dtype=torch.int64, device=dev)
+    bmax = torch.empty(nq * kb, dtype=torch.int32, device=dev)
+    check(lib.cfc_knn_blocks(*args, blocks.data_ptr(), kb, row_lo, sc.data_ptr(), ids.data_ptr(), bmax.data_ptr(), _stream(X)),
+          "cfc_knn_blocks")
+    return _select(sc, 16 * kb, min(k, n), ids, bmax)
 
 
 def ivf_topk(X, Q, probe: torch.Tensor, list_off: torch.Tensor, maxc: int, k: int, xnorm2=None, qnorm2=None,

@@ -10,6 +10,8 @@
 //     HBM into the A operand), and every block of rows' best score beside them.
 //   * cfc_topk_select: exact sorted top-k of scores with their block maxima: the k-th best block
 //     maximum bounds the k-th best score from below, so only the blocks that reach it are looked at.
+//   * cfc_knn_maxima, cfc_knn_blocks: the scan of many rows, which stores the best score of every 16 rows
+//     alone, and the scores of the k blocks that the k best of these name.
 //   * cfc_ivf_topk: scan and top-k of (query, probed list, chunk) work items from a device list-offset
 //     table in one launch: each workgroup scores its chunk into LDS and selects the k best there;
 //     the candidates are merged by cfc_topk_select.
@@ -30,83 +32,150 @@ __device__ __forceinline__ float key2f(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
 
-// One wave scores a block of B rows (a multiple of 16) against all queries.  Every lane holds four rows'
-// scores of one query; they are stored as they lie and their largest key goes to bmax [nq][nb].  Nothing
+// Sixteen rows' scores against all queries: X streams straight into the A operand, the queries are the B columns; a lane
+// holds four rows' scores (4 (lane >> 4) ..) of query lane & 15.
+template <int KC>  // KC = D / 32 MFMA k-steps
+struct KnnRows {
+  const uint16_t* X;
+  int N;
+  const float* xnorm2;       // optional: scores are -(x^2 + q^2 - 2 x q)
+  const uint8_t* alive;      // optional row mask: scores of other rows are -inf
+  bf16x8_t qf[KC];
+  float qn;
+
+  __device__ __forceinline__ void queries(const uint16_t* Q, const float* qnorm2, int nq) {
+    const int col = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    const bool qv = col < nq;
+    const uint16_t* qr = Q + (size_t)(qv ? col : 0) * (KC * 32);
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+      qf[c] = as_bf16x8(qv ? *reinterpret_cast<const uint4*>(qr + 32 * c + 8 * g) : make_uint4(0, 0, 0, 0));
+    qn = (qnorm2 && qv) ? qnorm2[col] : 0.f;
+  }
+  __device__ __forceinline__ void load(uint4* a, int r0) const {
+    const int col = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    const uint16_t* xr = X + (size_t)min(r0 + col, N - 1) * (KC * 32);
+#pragma unroll
+    for (int c = 0; c < KC; ++c) a[c] = *reinterpret_cast<const uint4*>(xr + 32 * c + 8 * g);
+  }
+  __device__ __forceinline__ f32x4_t score(const uint4* a, int r0) const {
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < KC; ++c) v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[c]), qf[c], v, 0, 0, 0);
+    const int rb = r0 + 4 * ((threadIdx.x & 63) >> 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = min(rb + i, N - 1);
+      if (xnorm2) v[i] = -(xnorm2[row] + qn - 2.f * v[i]);
+      if (alive && !alive[row]) v[i] = -INFINITY;
+    }
+    return v;
+  }
+  // Largest key of the rows that there are, in all lanes of a query.
+  __device__ __forceinline__ uint32_t best(const f32x4_t& v, int r0) const {
+    const int rb = r0 + 4 * ((threadIdx.x & 63) >> 4);
+    uint32_t m = 0u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (rb + i < N) m = max(m, f2key(v[i]));
+    m = max(m, (uint32_t)__shfl_xor((int)m, 16, 64));
+    return max(m, (uint32_t)__shfl_xor((int)m, 32, 64));
+  }
+};
+
+// One wave scores a block of B rows (16, 32 or 64) against all queries.  Every lane holds four rows' scores of one query;
+// they are stored as they lie and their largest key goes to bmax [nq][nb].  Nothing
 // is selected here, so the pass is a plain stream over X: 1M x 384 bf16 with one query in 131 us
 // (5.9 TB/s) where scoring 2048-row chunks into LDS and selecting in them took 172 us (4.5 TB/s; 489
 // workgroups, two on most CUs and one on the rest, the selecting wave alone at each one's end).
-// alive: optional row mask; scores of other rows are -inf.
-template <int KC>  // KC = D / 32 MFMA k-steps
+// MAXIMA: only the best score of every 16 rows is stored, to out [nq][ld] (B = 64).
+template <int KC, bool MAXIMA>
 __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
                                                        int nq, const float* __restrict__ xnorm2,
                                                        const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
                                                        float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
                                                        int B) {
-  constexpr int D = KC * 32;
   const int lane = threadIdx.x & 63, blk = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (blk >= nb) return;
   const int col = lane & 15, g = lane >> 4;
   const bool qv = col < nq;
-  bf16x8_t qf[KC];
-  {
-    const uint16_t* qr = Q + (size_t)(qv ? col : 0) * D;
-#pragma unroll
-    for (int c = 0; c < KC; ++c)
-      qf[c] = as_bf16x8(qv ? *reinterpret_cast<const uint4*>(qr + 32 * c + 8 * g) : make_uint4(0, 0, 0, 0));
-  }
-  const float qn = (qnorm2 && qv) ? qnorm2[col] : 0.f;
+  KnnRows<KC> rows{X, N, xnorm2, alive};
+  rows.queries(Q, qnorm2, nq);
   const int lo = blk * B, hi = min(N, lo + B);
   const bool vec = (ld & 3) == 0 && ((uintptr_t)out & 15) == 0;
   uint32_t best = 0u;
-  auto load = [&](uint4* a, int r0) {
-    const uint16_t* xr = X + (size_t)min(r0 + col, N - 1) * D;
-#pragma unroll
-    for (int c = 0; c < KC; ++c) a[c] = *reinterpret_cast<const uint4*>(xr + 32 * c + 8 * g);
-  };
-  auto score = [&](const uint4* a, int r0) {
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < KC; ++c) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[c]), qf[c], acc, 0, 0, 0);
-    if (!qv) return;
-    const int rb = r0 + 4 * g;
-    float v[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = min(rb + i, N - 1);
-      v[i] = acc[i];
-      if (xnorm2) v[i] = -(xnorm2[row] + qn - 2.f * v[i]);
-      if (alive && !alive[row]) v[i] = -INFINITY;
-      if (rb + i < N) best = max(best, f2key(v[i]));
-    }
-    float* o = out + col * ld + rb;
-    if (rb + 3 < N && vec) {
-      *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+  auto take = [&](const uint4* a, int r0) {
+    const f32x4_t v = rows.score(a, r0);
+    const uint32_t m = rows.best(v, r0);
+    if constexpr (MAXIMA) {
+      if (r0 - lo == 16 * g) best = m;            // group g's
     } else {
+      best = max(best, m);
+      const int rb = r0 + 4 * g;
+      if (!qv) return;
+      float* o = out + col * ld + rb;
+      if (rb + 3 < N && vec) {
+        *reinterpret_cast<f32x4_t*>(o) = v;
+      } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (rb + i < N) o[i] = v[i];
+        for (int i = 0; i < 4; ++i)
+          if (rb + i < N) o[i] = v[i];
+      }
     }
   };
   if constexpr (KC <= 16) {          // the next 16 rows in flight under these (144 -> 131 us); wider rows fill the registers alone
     uint4 a[2][KC];
-    load(a[0], lo);
+    rows.load(a[0], lo);
     for (int r0 = lo; r0 < hi; r0 += 32) {
-      if (r0 + 16 < hi) load(a[1], r0 + 16);
-      score(a[0], r0);
-      if (r0 + 32 < hi) load(a[0], r0 + 32);
-      if (r0 + 16 < hi) score(a[1], r0 + 16);
+      if (r0 + 16 < hi) rows.load(a[1], r0 + 16);
+      take(a[0], r0);
+      if (r0 + 32 < hi) rows.load(a[0], r0 + 32);
+      if (r0 + 16 < hi) take(a[1], r0 + 16);
     }
   } else {
     uint4 a[KC];
     for (int r0 = lo; r0 < hi; r0 += 16) {
-      load(a, r0);
-      score(a, r0);
+      rows.load(a, r0);
+      take(a, r0);
     }
   }
-  if (bmax == nullptr) return;
-  best = max(best, (uint32_t)__shfl_xor((int)best, 16, 64));
-  best = max(best, (uint32_t)__shfl_xor((int)best, 32, 64));
-  if (g == 0 && qv) bmax[(size_t)col * nb + blk] = best;
+  if constexpr (MAXIMA) {
+    if (qv && lo + 16 * g < hi) out[col * ld + 4 * blk + g] = key2f(best);
+  } else if (bmax && g == 0 && qv) {
+    bmax[(size_t)col * nb + blk] = best;
+  }
+}
+
+// The scores of `kb` blocks of 16 rows per query (blocks [nq][kb], in any order) into out [nq][16 kb] and their rows into
+// ids, blocks in rising order, with their largest keys in bmax [nq][kb]; past the last row the lowest NaN.  A wave per block.
+template <int KC>
+__global__ void __launch_bounds__(256) knn_blocks_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
+                                                         int nq, const float* __restrict__ xnorm2,
+                                                         const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
+                                                         const int64_t* __restrict__ blocks, int kb, int64_t row0,
+                                                         float* __restrict__ out, int64_t* __restrict__ ids,
+                                                         uint32_t* __restrict__ bmax) {
+  const int lane = threadIdx.x & 63, j = blockIdx.x * 4 + (threadIdx.x >> 6), q = blockIdx.y;
+  if (j >= kb) return;
+  const int64_t mine = blocks[(size_t)q * kb + j];
+  const int r0 = (int)mine * 16, rb = r0 + 4 * (lane >> 4);
+  KnnRows<KC> rows{X, N, xnorm2, alive};
+  rows.queries(Q, qnorm2, nq);
+  uint4 a[KC];
+  rows.load(a, r0);
+  int rank = 0;
+  for (int i = lane; i < (kb + 63) / 64 * 64; i += 64) rank += __popcll(__ballot(i < kb && blocks[(size_t)q * kb + min(i, kb - 1)] < mine));
+  const f32x4_t v = rows.score(a, r0);
+  const uint32_t m = rows.best(v, r0);
+  if ((lane & 15) != q) return;
+  const size_t to = (size_t)q * kb + rank;
+  if (lane < 16) bmax[to] = m;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int at = 4 * (lane >> 4) + i;
+    out[16 * to + at] = rb + i < N ? v[i] : key2f(0u);
+    ids[16 * to + at] = rb + i < N ? row0 + rb + i : -1;
+  }
 }
 
 // ------------------------------------------------------------------ exact top-k
@@ -575,6 +644,17 @@ __global__ void __launch_bounds__(256) pool_kernel(float* __restrict__ out_f32, 
 
 }  // namespace
 
+#define KNN_DIMS(KS)    \
+  switch (dim / 32) {   \
+    case 4: KS(4);      /* 128 */ \
+    case 8: KS(8);      /* 256 */ \
+    case 12: KS(12);    /* 384 (MiniLM, bge-small) */ \
+    case 16: KS(16);    /* 512 */ \
+    case 24: KS(24);    /* 768 (bge-base, mpnet) */ \
+    case 32: KS(32);    /* 1024 (bge-large) */ \
+    default: return -2; \
+  }
+
 // Rows per block for the top-k of n scores: as small as the select kernel's number of blocks allows.
 CFC_API int cfc_topk_block(int n) {
   int b = 16;
@@ -597,17 +677,34 @@ CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, c
   if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || ld < N) return -1;
   const int B = cfc_topk_block(N), nb = (N - 1) / B + 1;
   if (bmax && (long)nq * nb > room) return -1;
-#define KS(KC) knn_scan_kernel<KC><<<(nb + 3) / 4, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, \
+#define KS(KC) knn_scan_kernel<KC, false><<<(nb + 3) / 4, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, \
       qnorm2, alive, out, (size_t)ld, bmax, nb, B); break
-  switch (dim / 32) {
-    case 4: KS(4);      // 128
-    case 8: KS(8);      // 256
-    case 12: KS(12);    // 384 (MiniLM, bge-small)
-    case 16: KS(16);    // 512
-    case 24: KS(24);    // 768 (bge-base, mpnet)
-    case 32: KS(32);    // 1024 (bge-large)
-    default: return -2;
-  }
+  KNN_DIMS(KS)
+#undef KS
+  return CFC_CHECK_LAUNCH();
+}
+
+// The best score of every 16 rows of [0, N) of X for nq queries, into out [nq][ld].
+CFC_API int cfc_knn_maxima(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
+                           const uint8_t* alive, float* out, long ld, hipStream_t stream) {
+  if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || ld < (N - 1) / 16 + 1) return -1;
+  const int nb = (N - 1) / 64 + 1;
+#define KS(KC) knn_scan_kernel<KC, true><<<(nb + 3) / 4, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, \
+      qnorm2, alive, out, (size_t)ld, nullptr, nb, 64); break
+  KNN_DIMS(KS)
+#undef KS
+  return CFC_CHECK_LAUNCH();
+}
+
+// Scores of kb blocks of 16 rows per query, for a cfc_topk_select over 16 kb: see knn_blocks_kernel.  Every block starts
+// below N.
+CFC_API int cfc_knn_blocks(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
+                           const uint8_t* alive, const int64_t* blocks, int kb, long row0, float* out, int64_t* ids,
+                           uint32_t* bmax, hipStream_t stream) {
+  if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || kb < 1 || kb > (N - 1) / 16 + 1) return -1;
+#define KS(KC) knn_blocks_kernel<KC><<<dim3((kb + 3) / 4, nq), 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, \
+      xnorm2, qnorm2, alive, blocks, kb, row0, out, ids, bmax); break
+  KNN_DIMS(KS)
 #undef KS
   return CFC_CHECK_LAUNCH();
 }

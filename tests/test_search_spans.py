@@ -1,4 +1,4 @@
-"""A flat search in spans of rows: what knn_topk allots and refuses, without a GPU."""
+"""A flat search: what knn_topk and its parts allot, pass on and refuse, without a GPU."""
 import types
 
 import pytest
@@ -12,40 +12,44 @@ pytestmark = pytest.mark.skipif(not kernels_available(), reason="the built libra
 
 def _fake(*shape):
     """A tensor on the GPU as far as knn_topk looks at it: its launches are recorded, not made."""
-    return types.SimpleNamespace(shape=shape, is_cuda=True, device="cpu")
+    return types.SimpleNamespace(shape=shape, is_cuda=True, device="cpu", data_ptr=lambda: 0, element_size=lambda: 2)
 
 
-def _search(monkeypatch, rows, nq, k=10, row_lo=0):
-    spans = []
-
-    def scan(X, Q, xnorm2, qnorm2, alive, lo, hi, out, bmax):
-        spans.append((lo, hi, out, bmax))
-
-    def select(scores, n, k, ids, bmax, row_lo=0):
-        return torch.zeros(nq, k), torch.zeros(nq, k, dtype=torch.long)
-    monkeypatch.setattr(K, "_knn_scan", scan)
-    monkeypatch.setattr(K, "_select", select)
-    K.knn_topk(_fake(row_lo + rows, 128), _fake(nq, 128), k, row_lo=row_lo)
-    return spans
+def _record(monkeypatch):
+    """(entry, its arguments) of every call."""
+    seen = []
+    lib = types.SimpleNamespace(cfc_topk_block=kernels().cfc_topk_block, cfc_topk_segment=kernels().cfc_topk_segment)
+    for name in ("cfc_knn_scan", "cfc_topk_select", "cfc_knn_maxima", "cfc_knn_blocks"):
+        setattr(lib, name, lambda *a, name=name: seen.append((name, a)) or 0)
+    monkeypatch.setattr(K, "kernels", lambda: lib)
+    monkeypatch.setattr(K, "_stream", lambda t: None)
+    return seen
 
 
-@pytest.mark.parametrize("small", (False, True))
-@pytest.mark.parametrize("nq", range(1, 17))
-def test_every_span_has_room_for_its_block_maxima(monkeypatch, nq, small):
-    """A last span of fewer rows may have more blocks than a full one: 270000 rows are 8438 blocks of 32, 262144 rows 16384
-    blocks of 16."""
-    if small:
-        monkeypatch.setattr(K, "KNN_SCORES", nq * 270_000)
-    step = K.KNN_SCORES // nq
-    rests = {1, 5003, step - 1, step} | {16384 * 2 ** a + d for a in range(4, 13) for d in (-1, 0, 1)}
-    sizes = {1_000_000, 5_500_000, 10_000_000, 35_000_000, 100_000_000} | {step + r for r in rests} | {2 * step + r for r in rests}
-    for rows in sorted(n for n in sizes if 0 < n <= min(100_000_000, 30 * step)):
-        spans = _search(monkeypatch, rows, nq, row_lo=7)
-        assert spans[0][0] == 7 and spans[-1][1] == 7 + rows and all(a[1] == b[0] for a, b in zip(spans, spans[1:]))
-        for lo, hi, out, bmax in spans:
-            n = hi - lo
-            assert out.shape[0] == nq and n <= out.shape[1]
-            assert bmax.numel() >= nq * -(-n // kernels().cfc_topk_block(n)), (rows, n)
+@pytest.mark.parametrize("nq", (1, 3, 7, 15, 16))
+def test_block_maxima_have_room(monkeypatch, nq):
+    """The blocks of n scores are not monotonic in n: 270000 are 8438 blocks of 32, 262144 are 16384 of 16."""
+    seen = _record(monkeypatch)
+    sizes = {1, 15, 16, 17, 5003, 5_500_000, 10_000_000, 35_000_000, 100_000_000} | {16384 * 2 ** a + d for a in range(4, 13) for d in (-1, 0, 1)}
+    for rows in sorted(sizes):
+        for k in (10, 256):
+            K.knn_topk(_fake(rows + 7, 128), _fake(nq, 128), k, row_lo=7)
+            for name, a in seen:
+                if name == "cfc_knn_scan":
+                    n, ld, room = a[2], a[9], a[11]
+                    assert n == rows <= ld
+                elif name == "cfc_topk_select":
+                    n, ld, room = a[3], a[4], a[7]
+                    assert n <= ld and a[5] <= n
+                elif name == "cfc_knn_maxima":
+                    assert a[2] == rows and a[9] >= -(-rows // 16)
+                    continue
+                else:
+                    assert a[9] == min(k, -(-rows // 16))
+                    continue
+                assert room >= nq * -(-n // kernels().cfc_topk_block(n)), (name, rows, n)
+            assert (seen[0][0] == "cfc_knn_scan") == (rows <= K.KNN_SCORES)
+            seen.clear()
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="looks at what is refused before any launch")
@@ -57,33 +61,23 @@ def test_entries_refuse_too_little_room():
 
 @pytest.mark.parametrize("lo, hi", [(-1, 100), (-5, 0), (0, 101), (50, 50), (60, 50), (100, 101)])
 def test_rows_outside_the_index_are_refused(monkeypatch, lo, hi):
-    monkeypatch.setattr(K, "_knn_scan", lambda *a: pytest.fail("launched"))
+    seen = _record(monkeypatch)
     with pytest.raises(ValueError):
         K.knn_topk(_fake(100, 128), _fake(1, 128), 10, row_lo=lo, N=hi)
-
-
-def _strides(monkeypatch):
-    """Row strides that the entries are called with."""
-    seen = []
-    lib = types.SimpleNamespace(cfc_topk_block=kernels().cfc_topk_block, cfc_topk_segment=kernels().cfc_topk_segment,
-                                cfc_knn_scan=lambda *a: seen.append(a[9]) or 0, cfc_topk_select=lambda *a: seen.append(a[4]) or 0)
-    monkeypatch.setattr(K, "kernels", lambda: lib)
-    monkeypatch.setattr(K, "_stream", lambda t: None)
-    return seen
+    assert not seen
 
 
 def test_rows_of_scores_keep_their_distance(monkeypatch):
     """A column transposed is one contiguous row of stride 1; a flat result is rows one after the other."""
-    seen = _strides(monkeypatch)
-    X, Q, Q1 = (types.SimpleNamespace(shape=(n, 128), is_cuda=True, device="cpu", data_ptr=lambda: 0, element_size=lambda: 2)
-                for n in (40, 3, 1))
+    seen = _record(monkeypatch)
+    X, Q, Q1 = (_fake(n, 128) for n in (40, 3, 1))
     for q, out, want in ((Q, None, 40), (Q, torch.empty(3, 52)[:, :40], 52), (Q, torch.empty(120), 40), (Q1, torch.empty(40, 1).t(), 40),
                          (Q1, torch.empty(2, 44)[1:, 4:], 44)):
         K.knn_scores(X, q, out=out)
-        assert seen.pop() == want
+        assert seen.pop()[1][9] == want
     for scores, want in ((torch.empty(40, 1).t(), 40), (torch.empty(3, 52)[:, :40].contiguous(), 40), (torch.empty(3, 52), 52)):
         K._select(scores, 40, 5, None, None)
-        assert seen.pop() == want
+        assert seen.pop()[1][4] == want
 
 
 def test_segments_cover_the_scores_in_whole_blocks():

@@ -38,7 +38,8 @@ def test_topk_is_the_stable_sort(kind, nq, n, k):
 
 @pytest.mark.parametrize("dim,nq,N,lo", [(128, 1, 1, 0), (384, 16, 33, 1), (768, 5, 5003, 2), (384, 3, 70_001, 40_000), (1024, 2, 4100, 3)])
 def test_knn_topk_in_spans(monkeypatch, dim, nq, N, lo):
-    """A search in one span and in many gives the same rows, in the order of the scores that knn_scores gives."""
+    """A search that may store all its scores and one that may store a fifth of them give the same rows, in the order of the
+    scores that knn_scores gives."""
     from copilot_for_consensus_amd.ops import kernels as K
     g = torch.Generator(device=DEV).manual_seed(N)
     X, Q = (torch.randn(n, dim, device=DEV, generator=g).bfloat16() for n in (N, nq))
@@ -53,15 +54,49 @@ def test_knn_topk_in_spans(monkeypatch, dim, nq, N, lo):
     assert torch.equal(one[0], many[0]) and torch.equal(one[1], many[1])
 
 
-def test_a_last_span_of_more_blocks(monkeypatch):
-    """Spans of 270000 rows, 8438 blocks of 32, and a last one of 262000, 16375 blocks of 16."""
+@pytest.mark.parametrize("metric", ["dot", "l2"])
+@pytest.mark.parametrize("dim,nq,N,lo", [(128, 1, 1, 0), (384, 16, 33, 1), (768, 5, 5003, 2), (384, 3, 70_001, 40_000), (1024, 2, 4100, 3),
+                                         (256, 1, 300, 17), (512, 7, 16 * 64, 0), (128, 3, 1_100_000, 8)])
+def test_knn_topk_stored_and_by_blocks(monkeypatch, dim, nq, N, lo, metric):
+    """A search that stores all scores and one that stores block maxima give the same rows, in the order of the scores that
+    knn_scores gives; fewer blocks than winners, a last block of one row, maxima in two shares; rows that score alike."""
     from copilot_for_consensus_amd.ops import kernels as K
-    nq, dim, N, k = 3, 128, 532_000, 100
     g = torch.Generator(device=DEV).manual_seed(N)
     X, Q = (torch.randn(n, dim, device=DEV, generator=g).bfloat16() for n in (N, nq))
-    rv, ri = K.knn_scores(X, Q).sort(dim=1, descending=True, stable=True)
-    monkeypatch.setattr(K, "KNN_SCORES", nq * 270_000)
-    v, i = K.knn_topk(X, Q, k)
+    X[N // 2:N // 2 + 9] = X[N // 3]
+    alive = torch.rand(N, device=DEV, generator=g) > 0.2
+    xn, qn = (t.float().pow(2).sum(1) if metric == "l2" else None for t in (X, Q))
+    k = min(100, N - lo)
+    want = K.knn_scores(X, Q, xn, qn)[:, lo:].masked_fill(~alive[lo:][None], float("-inf"))
+    rv, ri = want.sort(dim=1, descending=True, stable=True)
+    for most in (1 << 21, 0):
+        monkeypatch.setattr(K, "KNN_SCORES", most)
+        v, i = K.knn_topk(X, Q, k, xn, qn, alive=alive, row_lo=lo, N=N)
+        assert torch.equal(v, rv[:, :k]) and torch.equal(i, ri[:, :k] + lo), most
+
+
+@pytest.mark.parametrize("kind", ["equal", "few", "rising"])
+def test_search_by_blocks_of_alike_rows(monkeypatch, kind):
+    """Block maxima that are all equal, all but a few masked, and rising with the row."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    N, k = 50_021, 150
+    g = torch.Generator(device=DEV).manual_seed(1)
+    X, Q = (torch.randn(n, 128, device=DEV, generator=g).bfloat16() for n in (N, 2))
+    alive = None
+    if kind == "equal":
+        X[:] = X[:1]
+    elif kind == "few":
+        alive = torch.rand(N, device=DEV, generator=g) < 0.001
+    else:
+        X[:, 1:] = 0.0
+        X[:, 0] = torch.arange(N, device=DEV) / 1000.0
+        Q[:, 0] = 1.0
+    want = K.knn_scores(X, Q)
+    if alive is not None:
+        want = want.masked_fill(~alive[None], float("-inf"))
+    rv, ri = want.sort(dim=1, descending=True, stable=True)
+    monkeypatch.setattr(K, "KNN_SCORES", 0)
+    v, i = K.knn_topk(X, Q, k, alive=alive)
     assert torch.equal(v, rv[:, :k]) and torch.equal(i, ri[:, :k])
 
 
