@@ -49,8 +49,8 @@ __device__ __forceinline__ void en_glds16(uint32_t voff, const void* sbase, uint
       : "memory");
 }
 
-// x Phi(x) = max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, erfc by Abramowitz and Stegun 7.1.26 (as pgemm.hip's), in three
-// parts of about an MFMA's length.
+// x Phi(x) = max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, erfc by Abramowitz and Stegun 7.1.26 (as pgemm.h's, but none of
+// +inf: either way the row's norm makes no number of all its states), in three parts of about an MFMA's length.
 struct Gelu { float t, m, q; };
 __device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
 template <int PART>
