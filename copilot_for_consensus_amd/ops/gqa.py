@@ -259,13 +259,18 @@ def prompt_tiles(cu, ctx, H: int, G: int, rows: int) -> np.ndarray:
 def decode_slices(B: int, H: int, G: int, D: int, visible: int, dtype) -> int:
     """Key slices per row of a decode step, at least eight 32-key tiles each.  MFMA kernel: two of its workgroups share a
     CU, and half a round more than that evens their lengths out (256 items of 1024 keys: 4 slices 34.0 us, 3 31.4, 2
-    32.1; 320 of 1500: 59.2, 56.4, 59.3); from 384 items on one slice, whose merge, 5 us, costs more than the slices gain
-    (448 of 2000: 75.9 against 76.1 and the merge; 384: 65.5 against 60.2; 640 of 1000: 64.0 against 63.4).  Others:
-    about four workgroups per CU."""
+    32.1; 320 of 1500: 59.2, 56.4, 59.3).  From 384 items on one slice where few keys are seen: the merge, 5 us, costs more
+    than slices gain.  What they gain grows with the longest row, whose keys are one workgroup's work, and the rows'
+    differences (us with one slice / with 1024 / items, rows of equal, 0.4 - 1, 0 - 1 times the length: 384 items of 1024 keys
+    48 / 50, 39 / 42, 33 / 36; 896 items 95 / 99, 71 / 76, 57 / 62; 384 of 1536 uneven 54 / 54 and 46 / 46, of 6000 218 / 215,
+    182 / 165, 148 / 129; 448 of 6000 235 / 254, 193 / 187, 160 / 148; one row in 16 eight times the others: 384 of 1024
+    34 / 27, of 6000 153 / 92).  Others: about four workgroups per CU."""
     if dtype != torch.bfloat16 or D not in MFMA_DIMS:
         return max(1, min(math.ceil(1024 / (B * math.ceil(H / ANY_ROWS))), visible // 256, MAX_PARTITIONS))
     items = B * G * math.ceil(H / G / 16)
-    return max(1, min(math.ceil(768 / items), visible // 256, MAX_PARTITIONS)) if items < 384 else 1
+    if items >= 384 and visible <= 1536:
+        return 1
+    return max(1, min(math.ceil((768 if items < 384 else 1024) / items), visible // 256, MAX_PARTITIONS))
 
 
 def attention(a: Heads, q, rows, block_tables, ctx_lens, cu_q=None, tiles=None, P: int = 1, workspace=None, gate: Cols | None = None,

@@ -1,0 +1,19 @@
+"""Key slices of a grouped decode step (ops.gqa.decode_slices): a rule of rows, heads and keys."""
+import math
+
+import pytest
+import torch
+
+from copilot_for_consensus_amd.ops import gqa as A
+
+
+@pytest.mark.parametrize("visible", (255, 512, 1536, 1537, 2048, 6000, 100_000))
+def test_long_rows_of_many_items_are_sliced(visible):
+    """From 384 items on rows of more than 1536 keys get 1024 slices in all: a longest row is never one workgroup's work
+    unless there are a thousand others."""
+    for B in (48, 56, 64, 96, 127, 128, 200):
+        items = 8 * B
+        P = A.decode_slices(B, 32, 8, 128, visible, torch.bfloat16)
+        assert P == (1 if visible <= 1536 else min(math.ceil(1024 / items), visible // 256))
+    assert A.decode_slices(1, 32, 8, 128, visible, torch.bfloat16) == max(1, min(96, visible // 256, A.MAX_PARTITIONS))
+    assert A.decode_slices(48, 32, 8, 128, visible, torch.float32) == max(1, min(math.ceil(1024 / (48 * math.ceil(32 / A.ANY_ROWS))), visible // 256))
