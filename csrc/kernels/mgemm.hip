@@ -211,6 +211,7 @@ int mgemm_launch(const void* x, const void* w, void* out, int M, int N, int K, i
 
 // ---- which rows of a product run here.  All times in us, fitted to N, K of 1024 .. 28672 and 129 .. 5500 rows.
 constexpr int MG_CUS = 256;
+constexpr int MG_PGEMM_TILES = 96;        // fewer tiles than this are not taken to pgemm by its callers
 
 // mgemm_kernel in bm-row tiles, mostly within 10 %.  A 64-deep stage takes 0.2 + 0.0013 bm on an idle chip, up to 0.42
 // more of that on a full one (0.55 in all rounds but the last), and no less than its 16 KB of W and its rows of X at
@@ -230,6 +231,13 @@ double mgemm_us(int M, int N, int K, int bm, int split, bool fp32) {
   return t + (split > 1 ? 8.0 * split : 4.0 * fp32) * M * N / 7.0e6;
 }
 
+// What X alone takes: an XCD's workgroups share columns, not rows, so each of up to 8 runs of columns (and K slices) brings
+// X into its XCD's L2, 7.6 TB/s in all (16041 rows of 512 x 4096 83, in pgemm 67; 8171 of 1024 x 4096 81 and 69).
+double mgemm_x_us(int M, int N, int K, int split) {
+  const int64_t runs = (int64_t)((N + MG_BN - 1) / MG_BN) * split;
+  return 12.0 + (double)M * K * 2 * std::max(1.0, (double)std::min<int64_t>(8, runs) / split) / 7.6e6;
+}
+
 // pgemm's persistent kernel: a K-tile takes 1.4 in a full round of 256 x 256 tiles, 0.8 to 1.22 in a partial one
 double ppp_us(int M, int N, int K, bool fp32) {
   const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
@@ -240,14 +248,16 @@ double ppp_us(int M, int N, int K, bool fp32) {
 enum { MG_ACT = 0, MG_SLABS = 1, MG_WHOLE = 2 };
 
 // the fastest tile and split.  Splits are powers of two, so that rows multiplied in batches of different sizes are
-// mostly added up in the same order; 2 more for the launch that adds an activation's slabs up.  Beyond 3 rounds of
-// workgroups nothing was measured to be faster than pgemm.
-double mgemm_best(int M, int N, int K, int kind, bool split_ok, int& bm, int& split) {
+// mostly added up in the same order; 2 more for the launch that adds an activation's slabs up, 3 more (`alone`) for slices
+// of 8 stages or fewer, over before their ring is full: 1507 rows of 512 x 1024 in 4 slices 17.9, whole 12.3; 339 of
+// 1536 x 4096 in 8 22.2, in 4 19.4.  Beyond 3 rounds of workgroups nothing was measured to be faster than pgemm.
+double mgemm_best(int M, int N, int K, int kind, bool split_ok, bool alone, int& bm, int& split) {
   double best = 1e30;
   for (int b = 128; b <= 256; b += 32) {
     if ((int64_t)((M + b - 1) / b) * ((N + MG_BN - 1) / MG_BN) > 3 * MG_CUS) continue;
     for (int s = 1; s <= (split_ok ? 8 : 1) && s * 64 <= K; s *= 2) {
-      const double t = mgemm_us(M, N, K, b, s, kind != MG_ACT) + (s > 1 && kind == MG_ACT ? 2.0 : 0.0);
+      const double t = mgemm_us(M, N, K, b, s, kind != MG_ACT) + (s > 1 && kind == MG_ACT ? 2.0 : 0.0) +
+                       (s > 1 && alone && K <= 512 * s ? 3.0 : 0.0);
       if (t < best) best = t, bm = b, split = s;
     }
   }
@@ -263,6 +273,7 @@ double mgemm_best(int M, int N, int K, int kind, bool split_ok, int& bm, int& sp
 //     against 18; 2^21: 14 against 15 at 220 rows, 16 against 17 at 512, but 18.6 against 18.3 at 700);
 //   * all here where pgemm's tiles leave the chip idle: 4096 x 4096 up to 1800 rows (61 against 74; 2100: 81 against 73),
 //     28672 x 4096 up to 256 (68 against 87; 300: 91 against 89);
+//     nor where X would be brought into every L2 for a few columns each (mgemm_x_us): 1024 x 4096 up to 7000 rows;
 //   * the rows beyond pgemm's last whole round here: 4096 x 14336 of 4500 rows 512 -> 370, 4096 x 4096 152 -> 124.
 CFC_API int cfc_prompt_plan(int M, int N, int K, int kind, int* plan) {
   plan[0] = plan[1] = plan[2] = 0;
@@ -272,12 +283,13 @@ CFC_API int cfc_prompt_plan(int M, int N, int K, int kind, int* plan) {
     return 0;
   int bm = 0, split = 0;
   double best = M < 256 ? 1e29 : 0.97 * ppp_us(M, N, K, kind != MG_ACT);
-  const double all = mgemm_best(M, N, K, kind, kind != MG_WHOLE, bm, split);
-  if (all < best) best = all, plan[1] = bm, plan[2] = split;
+  double all = mgemm_best(M, N, K, kind, kind != MG_WHOLE, true, bm, split);
   const int tn = (N + 255) / 256, tm = (M + 255) / 256;
+  if (tm * tn >= MG_PGEMM_TILES) all = std::max(all, mgemm_x_us(M, N, K, split));
+  if (all < best) best = all, plan[1] = bm, plan[2] = split;
   const int rounds = (int)((int64_t)tm * tn / MG_CUS), head = rounds ? (int)((int64_t)MG_CUS * rounds / tn) * 256 : 0;
   if (head > 0 && head < M && K >= 128) {
-    const double rest = mgemm_best(M - head, N, K, kind, kind == MG_ACT, bm, split);
+    const double rest = mgemm_best(M - head, N, K, kind, kind == MG_ACT, false, bm, split);
     if (ppp_us(head, N, K, kind != MG_ACT) + rest < best) plan[0] = head, plan[1] = bm, plan[2] = split;
   }
   return 0;
