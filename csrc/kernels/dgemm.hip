@@ -430,7 +430,8 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
 // projection of 176 tiles took 10 slices a tile, 7 rounds of short workgroups, to come close).  A workgroup streams W
 // without a stop across tile boundaries -- the packed tiles follow one another -- and stores its sums at each: the parts
 // of a tile go to slabs 0, 1, .. in the order of their workgroups, the last of them filling the slabs that are left with
-// zeros.  One round, `slabs` of 2 or 3.  W tile n multiplies input in_of[n] (null: 0).
+// zeros.  One round; `slabs`: the most workgroups that share a tile (cfc_dgemm_stream_slabs), 2 to 4 for the products it is
+// planned for, up to K / 64 for few short tiles.  W tile n multiplies input in_of[n] (null: 0).
 // us, 22528 x 4096 (185 MB, 31 at 5.9 TB/s): 5 rows 44.6 -> 33.8, 12 rows 40.5 -> 35.3; cfc_dgemm_slab_plan has more.
 template <int BM, int BN>
 __global__ void __launch_bounds__((64 * DgShape<BM, BN>::WAVES), 1)
@@ -881,14 +882,15 @@ CFC_API int cfc_dgemm_config(int M, int N, int K, int swiglu, int bn, int* cfg) 
 // 44.6 / 40.2 -> 33.8 / 42.9, 18432 33.4 / 37.2 -> 27.9 / 35.0, 9216 in 64-row tiles 26.5 / 23.3 -> 15.7 / 20.9) and not
 // where one does (4096 x 14336: 21.8 / 23.0 -> 22.6 / 27.7; 2048 x 4096 in 64-row tiles is faster in a loop, 7.8 -> 7.3,
 // but slower in a layer, 6.9 -> 7.6: each XCD then needs all of the X that was just written, not one K slice of it);
-// above 64 rows its workgroups wait for X.
+// above 64 rows its workgroups wait for X.  Nor where one slice fills the round: 28672 x 4096, 5 / 16 rows 44.3 / 44.8 ->
+// 44.9 / 47.9, of which dgemm_us thinks 3 more.
 CFC_API int cfc_dgemm_slab_plan(int M, int N, int K, int bn, int* plan) {
   int cfg[2];
   if (M < 1 || N < 1 || K < 1 || bn < 1) return -1;
   const double t = dgemm_best(M, N, K, 0, bn, cfg);
   if (t < 0) return -1;
   plan[0] = cfg[1], plan[1] = 0;
-  if (M > 64 || (bn != 64 && bn != 128) || K % 64) return 0;
+  if (M > 64 || (bn != 64 && bn != 128) || K % 64 || cfg[1] == 1) return 0;
   const int slabs = cfc_dgemm_stream_slabs(N, K, bn);
   if ((int64_t)slabs * M * N * 4 > 0x7fffffff) return 0;
   if (dgemm_stream_us(M, N, K, bn, slabs) < 0.93 * t) plan[0] = slabs, plan[1] = 1;

@@ -13,6 +13,12 @@ def test_plan_streams_where_no_split_makes_whole_rounds():
         assert K.dgemm_slab_plan(M, N, Kd, bn) == (K.dgemm_config(M, N, Kd, bn=bn)[1], False)
 
 
+@pytest.mark.skipif(not kernels_available(), reason="the built library is missing")
+@pytest.mark.parametrize("M", (5, 8, 16, 33, 64))
+def test_one_slice_that_fills_the_round_is_no_stream(M):
+    assert K.dgemm_config(M, 28672, 4096, bn=128)[1] == 1 and K.dgemm_slab_plan(M, 28672, 4096, 128) == (1, False)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", (1, 5, 16, 17, 63, 64))
 @pytest.mark.parametrize("N, Kd, bn", [(64, 64, 64), (128, 192, 128), (640, 320, 128), (16384, 64, 64), (38400, 64, 64),
