@@ -8,7 +8,7 @@ count / get).  Replaces Qdrant / FAISS / Azure AI Search on the hot path (SURVEY
   288 GB MI355X holds 100M x 384 bf16 = 77 GB with room to spare); cosine = dot product of
   L2-normalised rows (normalised on insert by a HIP kernel), or squared-L2 with stored norms
   (FAISS IndexFlatL2 parity, score 1/(1+d), faiss_store.py:224).  Queries: <=16 at a time run the
-  fused MFMA scan kernel, larger batches a hipBLASLt GEMM; exact top-k from block maxima in one select kernel.
+  MFMA scan kernel, larger batches a hipBLASLt GEMM; exact top-k from block maxima.
   Vectors produced on the GPU (the encoder) are inserted without a host round trip.
   Upserts overwrite in place; deletes tombstone + periodic compaction.
 * :class:`HipIVFIndex` -- IVF-flat: k-means coarse quantiser trained on the GPU, rows stored
@@ -363,7 +363,7 @@ class HipFlatIndex(VectorStore):
             Qn = Q.contiguous()
             qn2 = Qn.float().pow(2).sum(1)
         if Q.is_cuda and nq <= 16 and k <= 256:
-            # scores and their block maxima in one pass, then only the blocks that can hold a winner
+            # scores or block maxima in one pass, then only the blocks that can hold a winner
             return K.knn_topk(self._X, Qn, k, self._norm2 if self.metric == "l2" else None, qn2,
                               self._alive if self._dead else None, row_lo=lo, N=hi)
         xn2 = self._norm2[lo:hi] if self.metric == "l2" else None

@@ -84,10 +84,9 @@ struct KnnRows {
 };
 
 // One wave scores a block of B rows (16, 32 or 64) against all queries.  Every lane holds four rows' scores of one query;
-// they are stored as they lie and their largest key goes to bmax [nq][nb].  Nothing
-// is selected here, so the pass is a plain stream over X: 1M x 384 bf16 with one query in 131 us
-// (5.9 TB/s) where scoring 2048-row chunks into LDS and selecting in them took 172 us (4.5 TB/s; 489
-// workgroups, two on most CUs and one on the rest, the selecting wave alone at each one's end).
+// they are stored as they lie and their largest key goes to bmax [nq][nb].  Nothing is selected here, so the pass is a plain
+// stream over X: 1M x 384 bf16 with one query in 131 us (5.9 TB/s) where scoring 2048-row chunks into LDS and selecting in
+// them took 172 us (4.5 TB/s; 489 workgroups, two on most CUs and one on the rest, the selecting wave alone at each one's end).
 // MAXIMA: only the best score of every 16 rows is stored, to out [nq][ld] (B = 64).
 template <int KC, bool MAXIMA>
 __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,

@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """BASELINE config 5 (retrieval half): a 100M x 384 bf16 cosine index resident in one MI355X's HBM
-(77 GB of 288 GB), exact top-k by the fused MFMA scan + radix-select kernel (knn_topk_kernel: the
-[nq, N] scores never reach HBM).  ``--ivf NLIST NPROBE``: the same index as IVF-flat over
+(77 GB of 288 GB), exact top-k by the MFMA scan that stores the best score of every 16 rows and a
+second look at the winning blocks (knn.hip).  ``--ivf NLIST NPROBE``: the same index as IVF-flat over
 clustered data (a Gaussian mixture, so lists mean something), k-means on a bf16 sample, one
 fused launch per query batch; reports build time, ms per batch and recall@10 against the flat
 scan.

@@ -259,8 +259,7 @@ def test_gumbel_sampling_distribution():
                                            (70, 3, 20, "l2"), (40000, 16, 256, "dot"), (100000, 16, 150, "dot"),
                                            (70000, 2, 33, "l2"), (50000, 5, 256, "l2")])
 def test_knn_topk_fused_matches_reference(N, nq, k, metric):
-    """Fused scan + per-chunk radix select (+ candidate merge) vs torch.topk of fp32 scores of the
-    same bf16 rows; dead rows and a row window excluded."""
+    """Scan and select vs torch.topk of fp32 scores of the same bf16 rows; dead rows and a row window excluded."""
     X = torch.nn.functional.normalize(torch.randn(N, 384, device=DEV), dim=1).bfloat16()
     Q = torch.nn.functional.normalize(torch.randn(nq, 384, device=DEV), dim=1).bfloat16()
     alive = torch.rand(N, device=DEV) > 0.1
