@@ -1512,6 +1512,7 @@ def _knn_scan(X, Q, xnorm2, qnorm2, alive, row_lo: int, N: int, out, bmax) -> No
                                  _p(bmax), 0 if bmax is None else bmax.numel(), _stream(X)), "cfc_knn_scan")
 
 
+@functools.lru_cache(maxsize=4096)
 def _topk_blocks(n: int) -> int:
     """Block maxima of n scores.  Not monotonic: 2^k * 16384 scores have 16384 blocks, one more has 8193 of twice the size."""
     return -(-n // kernels().cfc_topk_block(n))
@@ -1527,12 +1528,18 @@ def knn_scores(X, Q, xnorm2=None, qnorm2=None, out=None):
     return out
 
 
+@functools.lru_cache(maxsize=4096)
+def _topk_parts(n: int) -> int:
+    """Shares that n scores are selected from in."""
+    return -(-n // kernels().cfc_topk_segment(n))
+
+
 def _select(scores, n: int, k: int, ids, bmax, row_lo: int = 0):
     """(values, ids) [nq, k] descending of the first ``n`` scores of every row of ``scores`` (the lower index first among
     equals); ``bmax``: their block maxima (None: taken here); ``ids``: the scores' ids (None: row_lo + index).  Many scores
     are selected from in segments, and then from the segments' winners, whose order is that of their rows among equals."""
     lib, nq, dev = kernels(), scores.shape[0], scores.device
-    parts = -(-n // lib.cfc_topk_segment(n))
+    parts = _topk_parts(n)
     fill = bmax is None
     if fill:
         bmax = torch.empty(nq * _topk_blocks(n), dtype=torch.int32, device=dev)

@@ -265,14 +265,14 @@ __device__ __forceinline__ uint64_t sel_cut(uint64_t* cand, int cnt, int kk, int
 // this bound (about k of them) are read, those at or above it kept, cut to k and ranked.  Where many blocks' maxima equal
 // the bound (equal scores, or all but a few masked), the first of them do, as many as are missing: each holds a score of
 // that value, at a lower row than any later block's.  Once cut, the k kept bound what may still come.  (300 of 1M: equal
-// scores 48 us where looking at every block that reaches the bound took 5075, all but 100 masked 81 where it took 5586,
-// others as before, 33; the radix passes 258, 189 and 176.)
+// scores 48 us where looking at every block that reaches the bound took 5075, all but 100 masked 86 where it took 5586,
+// others as before, 32; the radix passes 258, 189 and 176.)
 // A chain of short steps: 18 us for 150 of 1M scores, where three rounds of radix histograms in LDS over
 // 2048-row chunks' winners and a library sort took 120.
 // ids (row stride ld, optional): what the rows are called; else row0 + row.
 // grid (queries, segments): workgroup y selects from `seg` of the n scores, a whole number of blocks of B, into
 // out [query][y].  One workgroup brings in 25 B/ns: more than 2^20 scores are shared out, and their winners selected from
-// again (us for 2048 of 20M in one, here: 983, 316; rising scores 4435, 448; the radix passes 634 and 808).
+// again (us for 2048 of 20M in one, here: 983, 320; rising scores 4435, 510; the radix passes 634 and 808).
 __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* __restrict__ in, int n, size_t ld, int B, int seg,
                                                                   const uint32_t* __restrict__ bmax, int nb, int k,
                                                                   const int64_t* __restrict__ ids, int64_t row0,
@@ -285,16 +285,17 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
   __shared__ uint16_t ties[SEL_BLOCKS / SEL_THREADS][SEL_WAVES];
   const int tid = threadIdx.x, lane = tid & 63, qi = blockIdx.x;
   const uint64_t below = (1ull << lane) - 1ull;
+  const int lb = 31 - __clz(B);                      // B is a power of two
   {
     const size_t first = (size_t)blockIdx.y * seg;
     in += qi * ld + first;
     if (ids) ids += qi * ld + first;
     row0 += first;
-    bmax += (size_t)qi * nb + first / B;
+    bmax += (size_t)qi * nb + (first >> lb);
     out_v += ((size_t)qi * gridDim.y + blockIdx.y) * k;
     out_i += ((size_t)qi * gridDim.y + blockIdx.y) * k;
     n = (int)min((size_t)seg, n - first);
-    nb = (n - 1) / B + 1;
+    nb = ((n - 1) >> lb) + 1;
   }
   int turn = 0;
   uint32_t key[SEL_BLOCKS / SEL_THREADS];
@@ -339,20 +340,23 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
       }
     }
   }
-  uint32_t drop = 0;                                 // bit j: block j of this thread is not looked at
-  if (nb > k && reach > k + k / 4) {                 // thr is the k-th best maximum itself
+  if (nb > k && reach > k + k / 4) {                 // thr is the k-th best maximum itself; seldom so: read again, not unrolled
     int c = 0;
-#pragma unroll
+#pragma unroll 1
     for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
-      const uint64_t m = __ballot(tid + j * SEL_THREADS < nb && key[j] == thr);
+      const int i = tid + j * SEL_THREADS;
+      const uint32_t x = i < nb ? bmax[i] : 0u;
+      const uint64_t m = __ballot(i < nb && x == thr);
       if (lane == 0) ties[j][tid >> 6] = (uint16_t)__popcll(m);
-      c += __popcll(__ballot(key[j] > thr));
+      c += __popcll(__ballot(x > thr));
     }
     const int missing = k - sel_count(c, red, turn);
+    uint32_t drop = 0;                               // bit j: block j of this thread is not looked at
     int before = 0;                                  // ties in lower blocks
-#pragma unroll
+#pragma unroll 1
     for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
-      const bool tie = tid + j * SEL_THREADS < nb && key[j] == thr;
+      const int at = tid + j * SEL_THREADS;
+      const bool tie = at < nb && bmax[at] == thr;
       int mine = before + __popcll(__ballot(tie) & below);
 #pragma unroll 1
       for (int i = 0; i < SEL_WAVES; ++i) {
@@ -361,13 +365,15 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
       }
       if (tie && mine >= missing) drop |= 1u << j;
     }
+#pragma unroll
+    for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) key[j] = drop >> j & 1 ? 0u : key[j];
   }
   if (tid == 0) { s_n = 0; s_list = 0; }
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
     const int i = tid + j * SEL_THREADS;
-    const bool p = i < nb && key[j] >= thr && !(drop >> j & 1);
+    const bool p = i < nb && key[j] >= thr;
     const uint64_t m = __ballot(p);
     int at = 0;
     if (lane == 0 && m) at = atomicAdd(&s_list, __popcll(m));
@@ -375,7 +381,6 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
     if (p) list[at] = (uint16_t)i;
   }
   __syncthreads();
-  const int lb = 31 - __clz(B);                      // B is a power of two
   const long total = (long)s_list << lb;             // scores to look at, four neighbours per thread
   const float* src = in;
   const bool vec = ((uintptr_t)in & 15) == 0;
@@ -422,9 +427,10 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
     __syncthreads();
     const int cnt = s_n;
     __syncthreads();
-    if (cnt > SEL_CAP - SEL_STEP) floor = sel_cut(cand, cnt, k, red, turn, &s_n, bits);   // the next step might not fit
+    // the next step might not fit; at the end, no more than the ranking takes.  One place for both: twice in the way, the cut's
+    // code costs every call 0.6 us
+    if (cnt > (s0 + SEL_STEP < total ? SEL_CAP - SEL_STEP : max(k, SEL_THREADS))) floor = sel_cut(cand, cnt, k, red, turn, &s_n, bits);
   }
-  if (s_n > max(k, SEL_THREADS)) sel_cut(cand, s_n, k, red, turn, &s_n, bits);
   const int cnt = s_n;                                // at least min(k, n)
   for (int i = tid; i < cnt; i += SEL_THREADS) {
     const uint64_t e = cand[i];
