@@ -285,7 +285,7 @@ CFC_API int cfc_prompt_plan(int M, int N, int K, int kind, int* plan) {
   double best = M < 256 ? 1e29 : 0.97 * ppp_us(M, N, K, kind != MG_ACT);
   double all = mgemm_best(M, N, K, kind, kind != MG_WHOLE, true, bm, split);
   const int tn = (N + 255) / 256, tm = (M + 255) / 256;
-  if (tm * tn >= MG_PGEMM_TILES) all = std::max(all, mgemm_x_us(M, N, K, split));
+  if ((int64_t)tm * tn >= MG_PGEMM_TILES) all = std::max(all, mgemm_x_us(M, N, K, split));
   if (all < best) best = all, plan[1] = bm, plan[2] = split;
   const int rounds = (int)((int64_t)tm * tn / MG_CUS), head = rounds ? (int)((int64_t)MG_CUS * rounds / tn) * 256 : 0;
   if (head > 0 && head < M && K >= 128) {

@@ -28,3 +28,8 @@ def test_slices_of_an_activation_fill_their_ring(N, Kd):
 def test_products_with_few_large_tiles_are_planned_as_before():
     """Fewer tiles than pgemm is given: nothing else would take them but the decode GEMM."""
     assert K.prompt_plan(12029, 512, 1024, "whole") == (0, 224, 1) and K.prompt_plan(6000, 1024, 14336) is not None
+
+
+def test_largest_products_are_planned():
+    """More tiles than 32 bits count."""
+    assert K.prompt_plan(2 ** 24, 2 ** 24, 64) is None and K.prompt_plan(2 ** 24, 2 ** 24, 64, "slabs") is None
