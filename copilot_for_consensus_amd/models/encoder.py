@@ -200,6 +200,8 @@ class EncoderModel:
         """The arrays as int32 tensors on the device, by one copy from pinned memory: a copy from pageable memory holds the
         host until the stream has come to it, so a batch would be prepared after the one before it and not beside it."""
         import numpy as np
+        if self.device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("encoding copies its texts from host memory that a graph would not keep: capture forward_packed")
         at = np.cumsum([0] + [-(-len(a) // 4) * 4 for a in arrays])
         buf = torch.empty(int(at[-1]), dtype=torch.int32, pin_memory=self.device.type == "cuda")
         flat = buf.numpy()

@@ -71,3 +71,20 @@ def test_what_the_kernels_are_not_built_for():
     want = m.encode_ids(texts)
     m.layers = [dict(lw, o=odd.copy_(lw["o"])) for lw in m.layers[:1]] + m.layers[1:]
     assert torch.allclose(m.encode_ids(texts), want, atol=4e-3)
+
+
+def test_texts_are_not_captured():
+    """A graph would read the texts from host memory that is another call's by the time it runs."""
+    from copilot_for_consensus_amd.models.encoder import EncoderModel
+    m = EncoderModel.random("minilm-l6", DEV, seed=0)
+    texts = [list(range(3, 20)), [7]]
+    want = m.encode_ids(texts)
+    torch.cuda.synchronize()
+    x = torch.zeros(8, device=DEV)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        with pytest.raises(RuntimeError, match="graph"):
+            m.encode_ids(texts)
+        x += 1
+    g.replay()
+    assert torch.equal(m.encode_ids(texts), want) and bool((x == 1).all())
