@@ -9,8 +9,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("variant", ("pp", "pps", "ring4"))
 def test_gelu_of_every_bf16(variant):
-    """All 65536 arguments, infinities and NaN among them, as a bias over a product of zeros.  A rounding to bf16 apart (8 bits: 2^-8 at most), and the
-    4e-7 that the fp32 value is within: 1.5e-7 |x| / 2 of the approximation up to |x| = 4, and its last places."""
+    """All 65536 arguments, infinities and NaN among them, as a bias over a product of zeros.  A rounding to bf16 apart (8 bits:
+    2^-8 at most), and the 4e-7 that the fp32 value is within: 1.5e-7 |x| / 2 of the approximation up to |x| = 4, and its
+    last places."""
     bias = torch.arange(65536, device="cuda").to(torch.int32).to(torch.int16).view(torch.bfloat16)
     x, w = (torch.zeros(n, 64, device="cuda", dtype=torch.bfloat16) for n in (3, 65536))
     got = K.pgemm(x, w, "bias_gelu", bias=bias, variant=variant)
