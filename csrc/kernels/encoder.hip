@@ -6,20 +6,23 @@
 // outputs up to four times their inputs: over 65 k rows 311 us (o 45, up 155, down 110), 600 MB of rows written and read
 // again, each tile's epilogue alone on its CU.  Here a row never leaves its lane between them, 226 us:
 //
-//   * a workgroup owns 128 rows, a wave 32.  v_mfma_f32_32x32x16_bf16 with the WEIGHTS as A and the rows as
-//     B: a lane's accumulators are columns of ONE row (lane & 31), half of them its own, half those of
+//   * a workgroup owns 128 rows, 32 in each of four pairs of waves.  v_mfma_f32_32x32x16_bf16 with the WEIGHTS as A and
+//     the rows as B: a lane's accumulators are columns of ONE row (lane & 31), half of them its own, half those of
 //     lane ^ 32, so a LayerNorm is a sum over the lane's registers and one lane swap;
+//   * a pair of waves shares a SIMD and its 32 rows, half the registers each.  One holds the rows as operands (96
+//     registers) and takes the up product, 32 hidden columns at a time, with the GELU of the 32 before them between its
+//     MFMAs; the other holds 384 columns of accumulators (192), takes the attention's projection, the down product and
+//     both norms, and issues the weights' loads.  Hidden rows go from one to the other through 2 KB of LDS a pair;
 //   * the accumulator layout of one product becomes the B operand of the next by packing to bf16 and one
-//     v_permlane32_swap per two registers (frag_of): rows, hidden rows and residuals stay in registers
-//     (96 for a 384-wide bf16 row block, 192 for its fp32 accumulators: one wave per SIMD);
-//   * only the weights move: steps of two 24-KB stages of 24 fragments (32 columns x 384, or 384 columns x 32),
-//     three in a ring of LDS-DMA behind counted waits, one barrier per step of 48 MFMAs;
-//   * in the feed-forward's step c the up product of columns c and the down product over columns c - 2 take turns,
-//     GELU of columns c - 1 spread between them.
-// What bounds it: a wave alone on its SIMD issues an instruction every six cycles or so, and a step has 575 of them
-// (48 MFMAs, as many LDS reads and waits, 270 of GELU): 85 us for a block of rows on an idle chip, 115 with all CUs at
-// work and the clock down (matrix cores alone 52).  Half-steps of one stage in a ring of six, two elements' GELU at a
-// time, and the projections in the same kernel were each slower: their registers spill, or their order stalls.
+//     v_permlane32_swap per two registers (trade): rows and residuals stay in registers, and an accumulator starts from
+//     its bias and residual;
+//   * only the weights move: stages of 24 KB (32 columns x 384, or 384 columns x 32), five in a ring of LDS-DMA behind
+//     counted waits, two an interval, one barrier per interval of 24 MFMAs of either wave.
+// What bounds it: with all CUs at work the clock, 1.9 GHz of 2.4 (products alone, without GELU, LDS reads and loads,
+// take 81 us for a block of rows), and on an idle chip the up wave, whose 24 MFMAs, as many LDS reads and waits and 270
+// vector instructions of GELU take 2500 cycles an interval (matrix cores 1536).  A block of rows takes 70 us on an idle
+// chip and 100 with all CUs at work; one wave per SIMD with all 384 registers took 87 and 114 (an instruction every six
+// cycles), two waves with half the columns each and opposite phases 90 and 115 (both wait for the one with the GELU).
 #include "common.h"
 
 namespace {
@@ -30,10 +33,8 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 constexpr int EN_H = 384, EN_F = 1536;           // hidden, inner
 constexpr int EN_T = EN_H / 32;                  // 32-column tiles of a row
 constexpr int EN_S = EN_H / 16;                  // 16-deep k steps of a row
-constexpr int EN_ROWS = 128;                     // rows per workgroup, 32 per wave
-constexpr int EN_STAGE = 24 * 1024, EN_STEP = 2 * EN_STAGE, EN_RING = 3;
-constexpr int EN_PIECES = 12;                    // DMA pieces (1 KB) per wave and step
-constexpr int EN_LDS = EN_RING * EN_STEP + 4 * EN_F;
+constexpr int EN_ROWS = 128;                     // rows per workgroup, 32 per wave or pair of waves
+constexpr int EN_STAGE = 24 * 1024, EN_RING = 5; // a stage of weights, stages
 
 __device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -96,244 +97,320 @@ struct EncLayer {
   const uint16_t *wo, *bo, *g1, *b1, *wu, *bu, *wd, *bd, *g2, *b2;
 };
 
-// out(t, y): tile t of LN over the row of (acc + bias + residual), gamma and beta.  res(k): the residual's operand of
-// k step k.  A tile at a time, the sums kept in accumulation registers between the passes: 192 of them beside the
-// row's operands do not fit the others.
-template <class R, class O>
-__device__ __forceinline__ void en_norm(f32x16_t (&acc)[EN_T], R&& res, const uint16_t* __restrict__ bias,
-                                        const uint16_t* __restrict__ gamma, const uint16_t* __restrict__ beta, float eps, O&& out) {
-  const int hi = (threadIdx.x >> 5) & 1;
-  auto four = [&](const uint16_t* p, int t, int i, float (&v)[4]) {
-    const uint2 b = *reinterpret_cast<const uint2*>(p + 32 * t + 8 * i + 4 * hi);
-    v[0] = __uint_as_float(b.x << 16); v[1] = __uint_as_float(b.x & 0xffff0000u);
-    v[2] = __uint_as_float(b.y << 16); v[3] = __uint_as_float(b.y & 0xffff0000u);
-  };
-  float sum = 0.f;
+// Intervals, each with the stages 2 T and 2 T + 1 of the weight stream: 6 of Wo (two 32-deep slices each), then 50 of the
+// feed-forward (group g's up columns and the down slice g - 2: GELU of g - 1 lies between).
+constexpr int EN_O = EN_T / 2, EN_C = EN_F / 32;
+constexpr int EN_HX = 2 * 4 * 2048;              // hidden rows in LDS: two groups of 128 x 32
+constexpr int EN_VEC = 5;                        // vectors in LDS: g1, b1, bd, g2, b2
+constexpr int EN_LDS = EN_RING * EN_STAGE + EN_HX + 4 * EN_F + EN_VEC * 4 * EN_H;
+constexpr int EN_UA = 6, EN_DA = 4;              // fragments read ahead of their MFMA, by the up and the other waves
+constexpr int EN_MEET = 20;                      // MFMAs of a group ahead of its barrier: all its fragments are read by then
+static_assert(EN_MEET + EN_UA >= 24 && EN_MEET + EN_DA >= 24 && EN_LDS <= 160 * 1024, "");
+
+__device__ __forceinline__ void en_meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// acc: the rows less their means, and 1 / their deviations.  Four chains of sums: one would wait for each addition.
+__device__ __forceinline__ float en_center(f32x16_t (&acc)[EN_T], float eps) {
+  float p[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int t = 0; t < EN_T; ++t) {
-    f32x16_t y = acc[t];
+  for (int t = 0; t < EN_T; ++t)
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const u32x4_t r = trade(__builtin_bit_cast(u32x4_t, res(2 * t + s)));
+    for (int r = 0; r < 16; ++r) p[r & 3] += acc[t][r];
+  const float mean = xor32_sum((p[0] + p[1]) + (p[2] + p[3])) * (1.f / EN_H);
+  float q[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        float b[4];
-        four(bias, t, 2 * s + i, b);
-        const float v[4] = {__uint_as_float(r[2 * i] << 16), __uint_as_float(r[2 * i] & 0xffff0000u),
-                            __uint_as_float(r[2 * i + 1] << 16), __uint_as_float(r[2 * i + 1] & 0xffff0000u)};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          y[8 * s + 4 * i + e] += b[e] + v[e];
-          sum += y[8 * s + 4 * i + e];
-        }
-      }
-    }
-    asm volatile("" : "+a"(y));
-    acc[t] = y;
-    if (t % 2) __builtin_amdgcn_sched_barrier(0);
-  }
-  const float mean = xor32_sum(sum) * (1.f / EN_H);
-  float var = 0.f;
-#pragma unroll
-  for (int t = 0; t < EN_T; ++t) {
+  for (int t = 0; t < EN_T; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const float d = acc[t][r] - mean;
-      var += d * d;
+      acc[t][r] -= mean;
+      q[r & 3] = fmaf(acc[t][r], acc[t][r], q[r & 3]);
     }
-    asm volatile("" : "+a"(acc[t]));
-    if (t % 2) __builtin_amdgcn_sched_barrier(0);
-  }
-  const float rstd = rsqrtf(xor32_sum(var) * (1.f / EN_H) + eps);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int t = 0; t < EN_T; ++t) {
-    f32x16_t y;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float g[4], b[4];
-      four(gamma, t, i, g);
-      four(beta, t, i, b);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) y[4 * i + e] = (acc[t][4 * i + e] - mean) * rstd * g[e] + b[e];
-    }
-    out(t, y);
-    if (t % 2) __builtin_amdgcn_sched_barrier(0);
-  }
+  return rsqrtf(xor32_sum((q[0] + q[1]) + (q[2] + q[3])) * (1.f / EN_H) + eps);
 }
 
-// Steps of the weight stream: 6 of Wo (two 32-deep slices each), 50 of the feed-forward (up columns c, down
-// slice c - 2).
-constexpr int EN_O = EN_T / 2, EN_C = EN_F / 32, EN_STEPS = EN_O + EN_C + 2;
-constexpr int EN_AHEAD = 8;                      // fragments read ahead of their MFMA
-
-__global__ void __launch_bounds__(256, 1)
+__global__ void __launch_bounds__(512, 2)
     enc_layer_kernel(const uint16_t* __restrict__ att, const uint16_t* x, EncLayer L, uint16_t* xout, int M, float eps) {
-  // xout may be x: a row is read and written by its own lanes alone (lanes past M read row M - 1, to no use)
   extern __shared__ __attribute__((aligned(16))) char en_smem[];
-  const int lane = threadIdx.x & 63, hi = lane >> 5;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int row = blockIdx.x * EN_ROWS + w * 32 + (lane & 31);
+  const int lane = threadIdx.x & 63, hi = lane >> 5, r32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wave & 3;
+  const int row = blockIdx.x * EN_ROWS + w * 32 + r32;
+  typedef const __attribute__((address_space(3))) bf16x8_t* lds_frag_t;
+  typedef __attribute__((address_space(3))) bf16x8_t* lds_out_t;
 
-  // ---- weight stream.  Slices (384 rows x 64 B): pieces of 16 rows, 16-byte chunk c of row r at slot
-  // c ^ f((r >> 2) & 3); column groups (32 rows x 768 B): pieces of 8 rows x 128 B, chunk c at slot c ^ (r & 7).
-  // Both are read without bank conflicts, 8 lanes of consecutive rows at a time.  Wave w brings pieces
-  // 6 w .. 6 w + 5 of either stage.
-  const int srow = lane >> 2, sch = (lane & 3) ^ ((4 - ((srow >> 2) & 3)) & 3);
-  const uint32_t v_o = srow * EN_H * 2 + sch * 16, v_d = srow * EN_F * 2 + sch * 16;
-  const uint32_t v_n = (lane >> 3) * EN_H * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(en_lds_t*)en_smem);
-  const uint32_t own = w * (EN_PIECES / 2) * 1024;
-  const char* wo = reinterpret_cast<const char*>(L.wo) + (size_t)w * (EN_PIECES / 2) * 16 * EN_H * 2;
-  const char* wd = reinterpret_cast<const char*>(L.wd) + (size_t)w * (EN_PIECES / 2) * 16 * EN_F * 2;
-  const char* wu = reinterpret_cast<const char*>(L.wu);
-  auto piece = [&](int t, int q) {                // piece q (0 .. 11) of this wave in step t
-    const int i = q % (EN_PIECES / 2), h = q / (EN_PIECES / 2);
-    const uint32_t at = lds0 + (t % EN_RING) * EN_STEP + h * EN_STAGE + own + i * 1024;
-    if (t < EN_O) {
-      en_glds16(v_o, wo + 64 * (2 * t + h) + i * (16 * EN_H * 2), at);
-    } else if (h == 0) {                          // at the ends, columns and slices that are not used
-      const int p = w * (EN_PIECES / 2) + i;
-      en_glds16(v_n, wu + (size_t)min(t - EN_O, EN_C - 1) * (32 * EN_H * 2) + (p & 3) * (8 * EN_H * 2) + (p >> 2) * 128, at);
-    } else {
-      en_glds16(v_d, wd + 64 * max(t - EN_O - 2, 0) + i * (16 * EN_F * 2), at);
-    }
-  };
-#pragma unroll
-  for (int q = 0; q < EN_PIECES; ++q) piece(0, q);
-#pragma unroll
-  for (int q = 0; q < EN_PIECES; ++q) piece(1, q);
+  const uint32_t hx = lds0 + EN_RING * EN_STAGE + w * 2048 + lane * 16;
+  const uint32_t trade_at = lds0 + w * 12288 + lane * 16;
+  float* bu = reinterpret_cast<float*>(en_smem + EN_RING * EN_STAGE + EN_HX);
+  float* vec = bu + EN_F;
 
-  // ---- fragments: of a slice, tile n and k step s at index 12 s + n; of a group, k step s
-  const int r32 = lane & 31, f = (4 - ((r32 >> 2) & 3)) & 3;
-  const int so[2] = {r32 * 64 + ((hi ^ f) << 4), r32 * 64 + (((2 + hi) ^ f) << 4)};
-  int go[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) go[s] = r32 * 128 + (((2 * s + hi) ^ (r32 & 7)) << 4);
-  enum { SS, GS };                                // a step's two stages: slices, a group and a slice
-  // Fragment i (0 .. 47) of a step: two slices one after the other, else the two stages in turn.  One address
-  // per lane offset and step, the rest in the instruction's offset.
-  struct Stage { uint32_t s[2], g[4]; };
-  auto at = [&](int t) {
-    const uint32_t base = lds0 + (t % EN_RING) * EN_STEP;
-    Stage p;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) p.s[s] = base + so[s];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) p.g[s] = base + go[s];
-    return p;
+  // ---- weight stream.  Slices (384 rows x 64 B): pieces of 16 rows, 16-byte chunk c of row r at slot c ^ ((r >> 2) & 3);
+  // column groups (32 rows x 768 B): pieces of 8 rows x 128 B, chunk c at slot c ^ ((r >> 1) & 7).  LDS serves sixteen
+  // lanes' 16 bytes a cycle where they lie in 64 banks: rows of 128 bytes need the swizzle to step every second row (r & 7
+  // there reads 1.6 times as long).
+  const int srow = lane >> 2;
+  const uint32_t sch = ((lane & 3) ^ (srow >> 2)) << 4;
+  const char* wo = reinterpret_cast<const char*>(L.wo) + (size_t)w * 96 * EN_H * 2;
+  const char* wd = reinterpret_cast<const char*>(L.wd) + (size_t)w * 96 * EN_F * 2;
+  const char* wu = reinterpret_cast<const char*>(L.wu) + (size_t)w * 8 * EN_H * 2;
+  const uint32_t v_o = srow * EN_H * 2 + sch, v_d = srow * EN_F * 2 + sch;
+  const uint32_t v_n = (lane >> 3) * EN_H * 2 + (((lane & 7) ^ (((w & 1) << 2) + (lane >> 4))) << 4);
+  auto slot_of = [](int idx) { return (uint32_t)(idx % EN_RING); };
+  auto place = [&](int idx) { return lds0 + slot_of(idx) * EN_STAGE; };
+  // wave w's piece i (0 .. 5) of a stage: number 6 w + i of a slice, w + 4 i of a group; past either end, of no use
+  auto piece_o = [&](int k, int i, uint32_t at) { en_glds16(v_o, wo + i * (16 * EN_H * 2) + 64 * k, at + (6 * w + i) * 1024); };
+  auto piece_d = [&](int g, int i, uint32_t at) {
+    en_glds16(v_d, wd + i * (16 * EN_F * 2) + 64 * min(max(g - 2, 0), EN_C - 1), at + (6 * w + i) * 1024);
   };
-  auto frag = [&](const Stage& p, int kind, int i) {
-    const int h = kind == SS ? i / 24 : i & 1, j = kind == SS ? i % 24 : i >> 1;
-    const bool g = kind == GS && h == 0;
-    typedef const __attribute__((address_space(3))) bf16x8_t* lds_frag_t;
-    return *reinterpret_cast<lds_frag_t>((g ? p.g[j & 3] : p.s[j / EN_T]) + (uint32_t)(h * EN_STAGE + (g ? (j >> 2) * 4096 : (j % EN_T) * 2048)));
+  auto piece_u = [&](int g, int i, uint32_t at) {
+    en_glds16(v_n, wu + (uint32_t)min(g, EN_C - 1) * (32u * EN_H * 2) + 128 * i, at + (w + 4 * i) * 1024);
   };
-  // One step: its MFMAs in order, each followed by the read of the fragment EN_AHEAD later (from the next step's
-  // stages at the end, behind the barrier that says they are there) and a share of vector work, and every third
-  // by a DMA piece of the step after the next, into the place of the step before.  The order is fixed: left to
-  // itself the compiler reads fragments just ahead of their use and waits for each.
-  bf16x8_t fr[EN_AHEAD];
-  auto run = [&](int t, Stage& st, int kind, int next, auto&& mma, auto&& work) {
-    Stage nst = st;
+
+  struct Base { uint32_t s[4]; };
+  uint32_t so[2], go[4];
 #pragma unroll
-    for (int i = 0; i < 48; ++i) {
-      if (i == 48 - EN_AHEAD && t + 1 < EN_STEPS) {
-        // step t + 1's weights are in LDS in every wave, and step t's in registers
-        if (t + 2 < EN_STEPS) asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        nst = at(t + 1);
+  for (int s = 0; s < 2; ++s) so[s] = r32 * 64 + (((2 * s + hi) ^ ((r32 >> 2) & 3)) << 4);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) go[s] = r32 * 128 + (((2 * s + hi) ^ ((r32 >> 1) & 7)) << 4);
+  auto ld = [](uint32_t a) { return *reinterpret_cast<lds_frag_t>(a); };
+
+  if (wave >= 4) {
+    // ================================================= the up product and its GELU; Wo's stream
+    __builtin_amdgcn_s_setprio(2);                // the longer of the two: 102 -> 100 us
+    bf16x8_t fr[EN_UA];
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int i = 0; i < 6; ++i) piece_o(q, i, place(q));
+    for (int i = threadIdx.x - 256; i < EN_F; i += 256) bu[i] = bf2f(L.bu[i]);
+    {
+      const uint16_t* src[EN_VEC] = {L.g1, L.b1, L.bd, L.g2, L.b2};
+#pragma unroll
+      for (int v = 0; v < EN_VEC; ++v)
+        for (int i = threadIdx.x - 256; i < EN_H; i += 256) vec[v * EN_H + i] = bf2f(src[v][i]);
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int T = 0; T < EN_O; ++T) {
+#pragma unroll
+      for (int i = 0; i < 6; ++i) {
+        if (T + 1 < EN_O) piece_o(2 * T + 3, i, place(2 * T + 3));
+        else piece_d(0, i, place(2 * T + 3));
       }
-      mma(i, fr[i % EN_AHEAD]);
-      if (i + EN_AHEAD < 48) fr[i % EN_AHEAD] = frag(st, kind, i + EN_AHEAD);
-      else if (t + 1 < EN_STEPS) fr[i % EN_AHEAD] = frag(nst, next, i + EN_AHEAD - 48);
-      if (i % 3 == 2 && i < 3 * EN_PIECES && t + 2 < EN_STEPS) piece(t + 2, i / 3);
-      work(i);
-      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) {
+        if (T + 2 < EN_O) piece_o(2 * T + 4, i, place(2 * T + 4));
+        else piece_u(T + 2 - EN_O, i, place(2 * T + 4));
+      }
+      if (T + 1 < EN_O) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
-    st = nst;
-  };
-
-  // ---- biases of the up product, fp32 in LDS behind the ring
-  float* bu = reinterpret_cast<float*>(en_smem + EN_RING * EN_STEP);
-  bf16x8_t xf[EN_S];                              // the row block as operands
-  {
-    const uint16_t* ar = att + (size_t)min(row, M - 1) * EN_H + 8 * hi;
+    bf16x8_t xf[EN_S];
 #pragma unroll
-    for (int s = 0; s < EN_S; ++s) xf[s] = *reinterpret_cast<const bf16x8_t*>(ar + 16 * s);
+    for (int p = 0; p < 2; ++p) {
+      en_meet();                                  // half the operands are there
+#pragma unroll
+      for (int i = 0; i < 12; ++i) xf[12 * p + i] = ld(trade_at + i * 1024);
+      en_meet();                                  // and read
+    }
+    f32x16_t a, b;
+    auto biases = [&](f32x16_t& v, int g, int i) {
+      const float4 f = *reinterpret_cast<const float4*>(bu + 32 * min(g, EN_C - 1) + 8 * i + 4 * hi);
+      v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
+    };
+    Base cur;
+    auto base_of = [&](int T) {
+      Base p;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) p.s[s] = place(2 * T) + go[s];
+      return p;
+    };
+    cur = base_of(EN_O);
+#pragma unroll
+    for (int i = 0; i < EN_UA; ++i) fr[i] = ld(cur.s[i & 3] + (i >> 2) * 4096);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) biases(a, 0, i);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) b[r] = 0.f;
+    // group g into `up` while the GELU of the group before, in `old`, runs; `old` then starts from the biases of g + 1
+    auto group = [&](int g, f32x16_t& up, f32x16_t& old) {
+      const uint32_t hout = hx + ((g + 1) & 1) * (4 * 2048);
+      Base nb = cur;
+      Gelu ge[2];
+      u32x4_t hp;
+#pragma unroll
+      for (int i = 0; i < 24; ++i) {
+        if (i == EN_MEET) {
+          en_meet();
+          nb = base_of(EN_O + g + 1);
+        }
+        up = mfma32(fr[i % EN_UA], xf[i], up);
+        if (i + EN_UA < 24) fr[i % EN_UA] = ld(cur.s[(i + EN_UA) & 3] + ((i + EN_UA) >> 2) * 4096);
+        if (i >= EN_MEET) {
+#pragma unroll
+          for (int n = i == EN_MEET ? 0 : i + EN_UA - 24; n <= i + EN_UA - 24; ++n) fr[n] = ld(nb.s[n & 3] + (n >> 2) * 4096);
+        }
+#pragma unroll
+        for (int q = i * 24 / EN_MEET; i < EN_MEET && q < (i + 1) * 24 / EN_MEET; ++q) {     // two elements' GELU, a third at a time
+          const int e = q / 3 * 2;
+          float v0 = old[e], v1 = old[e + 1];
+          if (q % 3 == 0) { en_gelu<0>(ge[0], v0); en_gelu<0>(ge[1], v1); }
+          if (q % 3 == 1) { en_gelu<1>(ge[0], v0); en_gelu<1>(ge[1], v1); }
+          if (q % 3 == 2) {
+            en_gelu<2>(ge[0], v0);
+            en_gelu<2>(ge[1], v1);
+            hp[(e >> 1) & 3] = pack2bf(v0, v1);
+            asm volatile("" : "+v"(hp[(e >> 1) & 3]));
+            if ((e & 7) == 6) *reinterpret_cast<lds_out_t>(hout + (e >> 3) * 1024) = __builtin_bit_cast(bf16x8_t, trade(hp));
+          }
+        }
+        if (i >= EN_MEET) biases(old, g + 1, i - EN_MEET);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      cur = nb;
+    };
+    for (int g = 0; g < EN_C + 2; g += 2) {
+      group(g, a, b);
+      group(g + 1, b, a);
+    }
+    return;
   }
-  for (int i = threadIdx.x; i < EN_F; i += 256) bu[i] = bf2f(L.bu[i]);      // read after later barriers
 
+  // =================================================== the products into 384 columns, the norms; the feed-forward's stream
   f32x16_t acc[EN_T];
-  auto clear = [&]() {
+  bf16x8_t af[4], fr[EN_DA];                      // of the rows, of the weights
+  const uint16_t* ar = att + (size_t)min(row, M - 1) * EN_H + 8 * hi;
+  const uint16_t* xr = x + (size_t)min(row, M - 1) * EN_H + 8 * hi;
 #pragma unroll
-    for (int t = 0; t < EN_T; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+  for (int i = 0; i < 4; ++i) af[i] = *reinterpret_cast<const bf16x8_t*>(ar + 16 * i);
+  // columns 8 i + 4 hi + 0..3 of tile t, of a vector in LDS
+  auto four = [&](const float* p, int t, int i) { return *reinterpret_cast<const float4*>(p + 32 * t + 8 * i + 4 * hi); };
+  // v[4 i ..] += the operand pair's bf16 values
+  auto add2 = [](f32x16_t& v, int i, uint32_t a, uint32_t b) {
+    v[4 * i] += __uint_as_float(a << 16); v[4 * i + 1] += __uint_as_float(a & 0xffff0000u);
+    v[4 * i + 2] += __uint_as_float(b << 16); v[4 * i + 3] += __uint_as_float(b & 0xffff0000u);
   };
-  clear();
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  Stage st = at(0);
 #pragma unroll
-  for (int i = 0; i < EN_AHEAD; ++i) fr[i] = frag(st, SS, i);
-#pragma unroll
-  for (int t = 0; t < EN_O; ++t)
-    run(t, st, SS, t + 1 < EN_O ? SS : GS, [&](int i, bf16x8_t a) {
-      acc[i % EN_T] = mfma32(a, xf[4 * t + i / EN_T], acc[i % EN_T]);
-    }, [](int) {});
-  {
-    const uint16_t* xr = x + (size_t)min(row, M - 1) * EN_H + 8 * hi;
-    en_norm(acc, [&](int s) { return *reinterpret_cast<const bf16x8_t*>(xr + 16 * s); }, L.bo, L.g1, L.b1, eps, [&](int t, const f32x16_t& y) {
-      xf[2 * t] = frag_of(y, 0);
-      xf[2 * t + 1] = frag_of(y, 1);
-    });
-  }
-  clear();
-
-  // ---- feed-forward: in step c the up product of columns c, GELU of columns c - 1, the down product over c - 2
-  bf16x8_t h[2];
-  f32x16_t up;
-  Gelu ge;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) up[r] = 0.f;
-  h[0] = h[1] = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});       // the first two steps add zeros
-  for (int c = 0; c < EN_C + 2; ++c) {
-    f32x16_t nx;                                  // 32 columns, from their biases
+  for (int t = 0; t < EN_T; ++t) {                // the product starts from its bias and the residual
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float4 v = *reinterpret_cast<const float4*>(bu + 32 * min(c, EN_C - 1) + 8 * i + 4 * hi);
-      nx[4 * i] = v.x; nx[4 * i + 1] = v.y; nx[4 * i + 2] = v.z; nx[4 * i + 3] = v.w;
+      const uint2 b = *reinterpret_cast<const uint2*>(L.bo + 32 * t + 8 * i + 4 * hi);
+      acc[t][4 * i] = __uint_as_float(b.x << 16); acc[t][4 * i + 1] = __uint_as_float(b.x & 0xffff0000u);
+      acc[t][4 * i + 2] = __uint_as_float(b.y << 16); acc[t][4 * i + 3] = __uint_as_float(b.y & 0xffff0000u);
     }
-    run(EN_O + c, st, GS, GS, [&](int i, bf16x8_t a) {
-      if (i & 1) acc[(i >> 1) % EN_T] = mfma32(a, h[(i >> 1) / EN_T], acc[(i >> 1) % EN_T]);
-      else nx = mfma32(a, xf[i >> 1], nx);
-    }, [&](int i) {
-      // an element's GELU over three MFMAs, pinned there: nothing else spreads it under them
-      float v = up[i / 3];
-      if (i % 3 == 0) en_gelu<0>(ge, v);
-      if (i % 3 == 1) en_gelu<1>(ge, v);
-      if (i % 3 == 2) en_gelu<2>(ge, v);
-      up[i / 3] = v;
-    });
-    h[0] = frag_of(up, 0);
-    h[1] = frag_of(up, 1);
-    up = nx;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const u32x4_t r = trade(*reinterpret_cast<const u32x4_t*>(xr + 32 * t + 16 * s));
+      add2(acc[t], 2 * s, r[0], r[1]);
+      add2(acc[t], 2 * s + 1, r[2], r[3]);
+    }
   }
-  uint16_t* o = xout + (size_t)row * EN_H + 8 * hi;
-  en_norm(acc, [&](int s) { return xf[s]; }, L.bd, L.g2, L.b2, eps, [&](int t, const f32x16_t& y) {
-    const bf16x8_t a = frag_of(y, 0), b = frag_of(y, 1);
-    if (row < M) {
-      *reinterpret_cast<bf16x8_t*>(o + 32 * t) = a;
-      *reinterpret_cast<bf16x8_t*>(o + 32 * t + 16) = b;
+  Base cur;
+  auto base_of = [&](int idx) {
+    Base p;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) p.s[s] = place(idx) + so[s];
+    return p;
+  };
+  auto frag = [&](const Base& p, int i) { return ld(p.s[i / EN_T] + (i % EN_T) * 2048); };
+  en_meet();
+#pragma unroll 1
+  for (int T = 0; T < EN_O; ++T) {
+    const Base st[2] = {base_of(2 * T), base_of(2 * T + 1)};
+    ar += 64;
+    const uint16_t* nx = T + 1 < EN_O ? ar : xr;   // the next interval's operands, at the end of no use
+#pragma unroll
+    for (int i = 0; i < EN_DA; ++i) fr[i] = frag(st[0], i);
+#pragma unroll
+    for (int i = 0; i < 48; ++i) {
+      const int k = i / EN_T;
+      acc[i % EN_T] = mfma32(fr[i % EN_DA], af[k], acc[i % EN_T]);
+      if (i + EN_DA < 48) fr[i % EN_DA] = frag(st[(i + EN_DA) / 24], (i + EN_DA) % 24);
+      if (i % EN_T == EN_T - 1) af[k] = *reinterpret_cast<const bf16x8_t*>(nx + 16 * k);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  });
+    en_meet();
+  }
+  {
+    const float rstd = en_center(acc, eps);
+#pragma unroll
+    for (int t = 0; t < EN_T; ++t) {
+      // to the other waves through the two stages that are free, half the columns at a time
+      if (t == EN_T / 2) { en_meet(); en_meet(); }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        u32x4_t y;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const float4 g = four(vec, t, 2 * s + i), b = four(vec + EN_H, t, 2 * s + i), d = four(vec + 2 * EN_H, t, 2 * s + i);
+          const int o = 8 * s + 4 * i;
+          y[2 * i] = pack2bf(fmaf(acc[t][o], rstd * g.x, b.x), fmaf(acc[t][o + 1], rstd * g.y, b.y));
+          y[2 * i + 1] = pack2bf(fmaf(acc[t][o + 2], rstd * g.z, b.z), fmaf(acc[t][o + 3], rstd * g.w, b.w));
+          acc[t][o] = d.x; acc[t][o + 1] = d.y; acc[t][o + 2] = d.z; acc[t][o + 3] = d.w;
+          add2(acc[t], 2 * s + i, y[2 * i], y[2 * i + 1]);      // the next product starts from its bias and these rows
+        }
+        *reinterpret_cast<lds_out_t>(trade_at + ((2 * t + s) % 12) * 1024) = __builtin_bit_cast(bf16x8_t, trade(y));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  en_meet();
+  en_meet();
+
+  cur = base_of(2 * EN_O + 1);
+#pragma unroll
+  for (int i = 0; i < EN_DA; ++i) fr[i] = frag(cur, i);
+  bf16x8_t h0, h1;
+  h0 = h1 = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});            // the first two groups add zeros
+  for (int g = 0; g < EN_C + 2; ++g) {
+    const int T = EN_O + g;
+    const uint32_t hin = hx + ((g + 1) & 1) * (4 * 2048), pd = place(2 * T + 3), pu = place(2 * T + 4);
+    Base nb = cur;
+#pragma unroll
+    for (int i = 0; i < 24; ++i) {
+      if (i == EN_MEET) {
+        asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        nb = base_of(2 * T + 3);
+      }
+      acc[i % EN_T] = mfma32(fr[i % EN_DA], i < EN_T ? h0 : h1, acc[i % EN_T]);
+      if (i + EN_DA < 24) fr[i % EN_DA] = frag(cur, i + EN_DA);
+      if (i >= EN_MEET) {
+#pragma unroll
+        for (int n = i == EN_MEET ? 0 : i + EN_DA - 24; n <= i + EN_DA - 24; ++n) fr[n] = frag(nb, n);
+      }
+      if (i < 6) piece_d(g + 1, i, pd);
+      else if (i < 12) piece_u(g + 2, i - 6, pu);
+      if (i == 22 && g > 0) h0 = ld(hin);          // group g - 1, for the next interval
+      if (i == 23 && g > 0) h1 = ld(hin + 1024);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    cur = nb;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // the stream runs past its end
+  uint16_t* o = xout + (size_t)row * EN_H + 8 * hi;
+  const float rstd = en_center(acc, eps);
+#pragma unroll
+  for (int t = 0; t < EN_T; ++t) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      u32x4_t y;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float4 g = four(vec + 3 * EN_H, t, 2 * s + i), b = four(vec + 4 * EN_H, t, 2 * s + i);
+        const int at = 8 * s + 4 * i;
+        y[2 * i] = pack2bf(fmaf(acc[t][at], rstd * g.x, b.x), fmaf(acc[t][at + 1], rstd * g.y, b.y));
+        y[2 * i + 1] = pack2bf(fmaf(acc[t][at + 2], rstd * g.z, b.z), fmaf(acc[t][at + 3], rstd * g.w, b.w));
+      }
+      if (row < M) *reinterpret_cast<u32x4_t*>(o + 32 * t + 16 * s) = trade(y);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
 // ---- y = x W^T + b for a 384-wide x and W of 32 N32 rows (the attention's projections), the same way: rows in registers
 // as B operands, W in column groups through a ring of three stages.  No accumulators to hold beside them, so two
 // workgroups share a CU and one's waits are the other's matrix time.  65 k rows x 1152 in 67 us, 256 x 256 tiles of
 // both operands in LDS took 112.
-constexpr int EP_RING = 3;
+constexpr int EP_RING = 3, EP_AHEAD = 8;
 
 __global__ void __launch_bounds__(256, 2)
     enc_proj_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ W, const uint16_t* __restrict__ bias,
@@ -342,14 +419,14 @@ __global__ void __launch_bounds__(256, 2)
   const int lane = threadIdx.x & 63, hi = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = blockIdx.x * EN_ROWS + w * 32 + (lane & 31);
-  const uint32_t v_n = (lane >> 3) * EN_H * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
+  const uint32_t v_n = (lane >> 3) * EN_H * 2 + (((lane & 7) ^ (lane >> 4)) << 4);     // of even pieces
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(en_lds_t*)smem);
   auto issue = [&](int n, uint32_t place) {       // rows 32 n .. of W; past the end, of no use
     const char* src = reinterpret_cast<const char*>(W) + (size_t)min(n, groups - 1) * (32 * EN_H * 2);
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
       const int p = 6 * w + i;
-      en_glds16(v_n, src + (p & 3) * (8 * EN_H * 2) + (p >> 2) * 128, place + p * 1024);
+      en_glds16(i & 1 ? v_n ^ 64 : v_n, src + (p & 3) * (8 * EN_H * 2) + (p >> 2) * 128, place + p * 1024);
     }
   };
   issue(0, lds0);
@@ -363,7 +440,7 @@ __global__ void __launch_bounds__(256, 2)
   const int r32 = lane & 31;
   uint32_t go[4];
 #pragma unroll
-  for (int s = 0; s < 4; ++s) go[s] = r32 * 128 + (((2 * s + hi) ^ (r32 & 7)) << 4);
+  for (int s = 0; s < 4; ++s) go[s] = r32 * 128 + (((2 * s + hi) ^ ((r32 >> 1) & 7)) << 4);
   uint16_t* o = out + (size_t)row * 32 * groups + 8 * hi;
   uint32_t here = lds0, before = lds0 + (EP_RING - 1) * EN_STAGE;
   auto four = [&](int n, int i, f32x16_t& a) {
@@ -386,13 +463,13 @@ __global__ void __launch_bounds__(256, 2)
     f32x16_t acc;
 #pragma unroll
     for (int i = 0; i < 4; ++i) four(n, i, acc);
-    bf16x8_t fr[EN_AHEAD];
+    bf16x8_t fr[EP_AHEAD];
 #pragma unroll
-    for (int i = 0; i < EN_AHEAD; ++i) fr[i] = frag(i);
+    for (int i = 0; i < EP_AHEAD; ++i) fr[i] = frag(i);
 #pragma unroll
     for (int i = 0; i < EN_S; ++i) {
-      acc = mfma32(fr[i % EN_AHEAD], xf[i], acc);
-      if (i + EN_AHEAD < EN_S) fr[i % EN_AHEAD] = frag(i + EN_AHEAD);
+      acc = mfma32(fr[i % EP_AHEAD], xf[i], acc);
+      if (i + EP_AHEAD < EN_S) fr[i % EP_AHEAD] = frag(i + EP_AHEAD);
       __builtin_amdgcn_sched_barrier(0);
     }
     const bf16x8_t y0 = frag_of(acc, 0), y1 = frag_of(acc, 1);
@@ -599,7 +676,7 @@ CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* 
     if (rc) break;
     if (kind == 2) {
       const EncLayer L = {p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], p[10], p[11]};
-      enc_layer_kernel<<<blocks, 256, EN_LDS, stream>>>(ap, xp, L, xp, T, eps);
+      enc_layer_kernel<<<blocks, 512, EN_LDS, stream>>>(ap, xp, L, xp, T, eps);
     } else {
       enc_ksplit_kernel<EN_H><<<gk, 256, 0, stream>>>(ap, p[2], yp, T);
       enc_tile_kernel<true, true><<<gu, 256, 0, stream>>>(ap, EncNorm{yp, p[3], xp, p[4], p[5], eps}, p[6], p[7], hp, T, EN_F);
