@@ -421,13 +421,18 @@ def encoder_forward(ids, positions, weights: list[int], layers: int, cu_seqlens,
                          f"{len(weights)} weights of {layers} layers")
     def rows(n):
         return torch.empty(T, n, dtype=torch.bfloat16, device=dev)
-    x, att, qkv = rows(H), rows(H), rows(3 * H)
-    y, h = (rows(H), rows(ENCODER_FFN)) if lib.cfc_enc_rows(T) == 1 else (None, None)
+    x, tiny = rows(H), lib.cfc_enc_tiny(T, layers, heads, _stream(ids))
+    if tiny:
+        att = qkv = y = None
+        h = torch.empty(tiny, dtype=torch.bfloat16, device=dev)
+    else:
+        att, qkv = rows(H), rows(3 * H)
+        y, h = (rows(H), rows(ENCODER_FFN)) if lib.cfc_enc_rows(T) == 1 else (None, None)
     W = (ctypes.c_void_p * (len(weights) - 5))(*weights[5:])
     check(lib.cfc_enc_forward(ids.data_ptr(), positions.data_ptr(), *weights[:5],
                               cu_seqlens.data_ptr(), tiles[0].data_ptr(), tiles[1].data_ptr(), tiles[0].numel(), ENCODER_TILE_ROWS,
-                              int(max_seqlen), layers, W, heads, float(scale), float(eps), T, x.data_ptr(), _p(y), att.data_ptr(),
-                              qkv.data_ptr(), _p(h), _stream(x)), "cfc_enc_forward")
+                              int(max_seqlen), layers, W, heads, float(scale), float(eps), T, x.data_ptr(), _p(y), _p(att),
+                              _p(qkv), _p(h), _stream(x)), "cfc_enc_forward")
     return x
 
 

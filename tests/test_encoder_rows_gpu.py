@@ -73,6 +73,55 @@ def test_what_the_kernels_are_not_built_for():
     assert torch.allclose(m.encode_ids(texts), want, atol=4e-3)
 
 
+@pytest.mark.parametrize("lens,layers", [([16], 1), ([17], 2), ([0, 3, 0, 1, 12, 0], 3), ([31, 1], 2), ([33], 2), ([1] * 63, 2), ([40, 0, 24], 3),
+                                         ([1] * 64, 1), ([30, 34], 24), ([30, 34], 25)], ids=lambda v: str(v if isinstance(v, int) else sum(v)))
+def test_a_few_short_texts(lens, layers):
+    """One launch for all layers: edges of its row groups, texts without tokens, the most layers it takes and one more; a
+    captured one again and again, its workspace filled anew each time."""
+    import dataclasses
+    from copilot_for_consensus_amd.models.encoder import get_encoder_config
+    from copilot_for_consensus_amd.ops import kernels as K
+    m = _model(dataclasses.replace(get_encoder_config("minilm-l6"), layers=layers), seed=layers)
+    T = sum(lens)
+    assert (K.kernels().cfc_enc_tiny(T, layers, m.cfg.heads, None) > 0) == (layers <= 24)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    ids = torch.randint(0, m.cfg.vocab_size, (T,), device=DEV, dtype=torch.int32, generator=g)
+    pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).to(DEV)
+    cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).to(torch.int32)
+    tiles = tuple(torch.tensor(t, dtype=torch.int32, device=DEV) for t in K.prefill_tiles(cu.tolist(), K.ENCODER_TILE_ROWS))
+    cu = cu.to(DEV)
+    got = m.forward_packed(ids, pos, cu, max(lens), tiles=tiles)
+    want = _states(m, ids.long(), [n for n in lens if n])
+    rel = ((got.double() - want).norm(dim=1) / want.norm(dim=1)).max()
+    assert rel < 2.0 ** -9 * (layers * 10) ** 0.5, float(rel)       # roundings as above
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        out = m.forward_packed(ids, pos, cu, max(lens), tiles=tiles)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, got)
+        m.forward_packed(ids, pos, cu, max(lens), tiles=tiles)
+
+
+def test_one_launch_needs_most_of_the_chip():
+    """Its workgroups wait for one another: a stream of few CUs keeps a launch per product, and gives the same."""
+    from copilot_for_consensus_amd.models.encoder import EncoderModel
+    from copilot_for_consensus_amd.ops import kernels as K
+    from copilot_for_consensus_amd.runtime.cu_partition import partition_streams
+    half = partition_streams()[0]
+    assert K.kernels().cfc_enc_tiny(12, 6, 12, half.cuda_stream) == 0 < K.kernels().cfc_enc_tiny(12, 6, 12, torch.cuda.Stream().cuda_stream)
+    m = EncoderModel.random("minilm-l6", DEV, seed=0)
+    texts = [list(range(3, 20)), [7]]
+    want = m.encode_ids(texts)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(half):
+        got = m.encode_ids(texts)
+    torch.cuda.synchronize()
+    assert torch.allclose(got, want, atol=4e-3)
+
+
 def test_texts_are_not_captured():
     """A graph would read the texts from host memory that is another call's by the time it runs."""
     from copilot_for_consensus_amd.models.encoder import EncoderModel
