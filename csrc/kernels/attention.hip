@@ -1238,7 +1238,7 @@ __global__ void __launch_bounds__(512, 2) prefill_gqa_kernel(
 // Varlen bidirectional encoder attention (BERT family), D in {32, 64}, S <= 512.
 // Input qkv is the fused projection output [T, 3*H*D] (q | k | v, head-major inside each).
 // 1-D grid over (query tile, head), XCD-remapped; block = 256 = 4 waves, tile = ENC_ROWS = 256
-// query rows (wave w: rows 64w .. 64w+63 as ENC_R = 4 groups of 16).  The WHOLE key/value range
+// query rows (wave w: 16-row groups w, w + 4, .. , ENC_R = 4 of them).  The WHOLE key/value range
 // of the sequence is staged once in LDS per block (K row-major, V transposed with the per-32-key
 // slot permutation) -- with 256-row tiles a MiniLM sequence (S <= 256) stages its K/V once per
 // head instead of once per 64 rows -- then every wave runs the swapped-product online softmax:
@@ -1249,8 +1249,10 @@ __global__ void __launch_bounds__(512, 2) prefill_gqa_kernel(
 constexpr int ENC_R = 4;               // 16-row query groups per wave
 constexpr int ENC_ROWS = 64 * ENC_R;   // query rows per workgroup
 
+// As many workgroups on a CU as their LDS lets there be (heads of 32: 96 registers, 90 -> 74 us for 365 texts of 180 tokens, x 12
+// heads; with V^T by four keys and waves of every fourth row group 68).
 template <int D>
-__global__ void __launch_bounds__(256) encoder_attn_kernel(const uint16_t* __restrict__ qkv,
+__global__ void __launch_bounds__(256, D == 32 ? 5 : 2) encoder_attn_kernel(const uint16_t* __restrict__ qkv,
                                                            const int32_t* __restrict__ cu_seqlens,
                                                            const int32_t* __restrict__ tile_seq,
                                                            const int32_t* __restrict__ tile_q0, float scale_log2,
@@ -1282,12 +1284,12 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const uint16_t* __res
   auto voff_chunk = [&](int d, int c) -> int { return d * Spad * 2 + ((c ^ (d & 15)) << 4); };
 
   // Q fragments first (pre-scaled), so their loads overlap the K/V staging below
-  const int wrow0 = qs + 64 * w;
-  const int ng = min(ENC_R, max(0, (S - wrow0 + 15) >> 4));   // row groups with >= 1 row (wave-uniform)
+  const int wrow0 = qs + 16 * w;       // wave w: every fourth row group, so that short texts keep all waves at work
+  const int ng = min(ENC_R, max(0, (S - wrow0 + 63) >> 6));   // row groups with >= 1 row (wave-uniform)
   bf16x8_t qf[ENC_R][KSTEPS];
 #pragma unroll
   for (int rg = 0; rg < ENC_R; ++rg) {
-    const int r = min(wrow0 + 16 * rg + col, S - 1);
+    const int r = min(wrow0 + 64 * rg + col, S - 1);
     const uint16_t* qr = qkv + (size_t)(beg + r) * row_stride + h * D;
 #pragma unroll
     for (int c = 0; c < KSTEPS; ++c) {
@@ -1302,37 +1304,32 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const uint16_t* __res
     }
   }
 
-  // K / V staging: every thread issues SB chunk loads of K and of V before any LDS write, so one
-  // memory round trip covers SB chunks (a load -> write -> load loop pays the latency per chunk)
-  constexpr int SB = 4;
-  const int nchunks = Spad * NC;
-  for (int id0 = tid; id0 < nchunks; id0 += 256 * SB) {
-    uint4 kv[SB], vv[SB];
+  // K / V staging: a thread takes one chunk of four consecutive rows of K and of V, all loads ahead of the LDS writes, so one
+  // memory round trip covers eight chunks.  Four keys are neighbours in the slot order: V^T takes eight 8-byte writes
+  // of four keys where a row at a time took 32 of two bytes.
+  for (int id = tid; id < Spad / 4 * NC; id += 256) {
+    const int r = id / NC * 4, ch = id % NC;
+    uint4 kv[4], vv[4];
 #pragma unroll
-    for (int b = 0; b < SB; ++b) {
-      const int id = id0 + 256 * b, r = id / NC, ch = id % NC;
+    for (int b = 0; b < 4; ++b) {
       kv[b] = make_uint4(0, 0, 0, 0);
       vv[b] = make_uint4(0, 0, 0, 0);
-      if (id < nchunks && r < S) {
-        const uint16_t* base = qkv + (size_t)(beg + r) * row_stride;
+      if (r + b < S) {
+        const uint16_t* base = qkv + (size_t)(beg + r + b) * row_stride;
         kv[b] = *reinterpret_cast<const uint4*>(base + H * D + h * D + ch * 8);
         vv[b] = *reinterpret_cast<const uint4*>(base + 2 * H * D + h * D + ch * 8);
       }
     }
 #pragma unroll
-    for (int b = 0; b < SB; ++b) {
-      const int id = id0 + 256 * b, r = id / NC, ch = id % NC;
-      if (id >= nchunks) break;
-      *reinterpret_cast<uint4*>(klds + koff(r, ch)) = kv[b];
-      // scatter V row r (d = ch*8 .. +7) into V^T at the permuted slot of key r
-      const int kin = r & 31, hi = kin >> 4, gg = (kin >> 2) & 3, jj = (kin & 3) + 4 * hi;
-      const int slot = (r & ~31) + 8 * gg + jj;
-      const uint16_t* ve = reinterpret_cast<const uint16_t*>(&vv[b]);
+    for (int b = 0; b < 4; ++b) *reinterpret_cast<uint4*>(klds + koff(r + b, ch)) = kv[b];
+    const int kin = r & 31, slot = (r & ~31) + 8 * ((kin >> 2) & 3) + 4 * (kin >> 4);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int d = ch * 8 + e;
-        *reinterpret_cast<uint16_t*>(vlds + voff_chunk(d, slot >> 3) + (slot & 7) * 2) = ve[e];
-      }
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t x[4] = {e < 2 ? vv[0].x : e < 4 ? vv[0].y : e < 6 ? vv[0].z : vv[0].w, e < 2 ? vv[1].x : e < 4 ? vv[1].y : e < 6 ? vv[1].z : vv[1].w,
+                             e < 2 ? vv[2].x : e < 4 ? vv[2].y : e < 6 ? vv[2].z : vv[2].w, e < 2 ? vv[3].x : e < 4 ? vv[3].y : e < 6 ? vv[3].z : vv[3].w};
+      const uint32_t pick = e & 1 ? 0x07060302u : 0x05040100u;     // the upper or the lower halves of two words
+      *reinterpret_cast<uint2*>(vlds + voff_chunk(ch * 8 + e, slot >> 3) + (slot & 7) * 2) =
+          make_uint2(__builtin_amdgcn_perm(x[1], x[0], pick), __builtin_amdgcn_perm(x[3], x[2], pick));
     }
   }
   __syncthreads();
@@ -1412,7 +1409,7 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const uint16_t* __res
 
 #pragma unroll
   for (int rg = 0; rg < ENC_R; ++rg) {
-    const int my_row = wrow0 + 16 * rg + col;
+    const int my_row = wrow0 + 64 * rg + col;
     if (rg < ng && my_row < S) {
       const float inv = l[rg] > 0.f ? 1.f / l[rg] : 0.f;
       uint16_t* orow = out + ((size_t)(beg + my_row) * H + h) * D;
