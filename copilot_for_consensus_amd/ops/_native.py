@@ -97,6 +97,7 @@ _KERNEL_SIGS = {
                                         c_int64, P],
     "cfc_prefill_attention_expanded": [P, P, P, P, c_int64, P, P, P, P, I, I, F, P, c_int64, P],
     "cfc_enc_rows": [I],
+    "cfc_knn_queries": [P, P, P, I, I, I, P],
     "cfc_enc_tiny": [I, I, I, P],
     "cfc_enc_forward": [P] * 10 + [I, I, I, I, P, I, F, F, I] + [P] * 6,
     "cfc_knn_scan": [P, P, I, I, I, P, P, P, P, L, P, L, P],

@@ -1634,6 +1634,17 @@ def l2_normalize(x, out=None, norms2=None):
     return out
 
 
+def knn_queries(q: torch.Tensor, unit: bool):
+    """fp32 queries [nq, dim] on the GPU as the scan takes them, by one launch: (bf16, of unit length if ``unit``, squared
+    norms of the rounded ones)."""
+    rows, dim = q.shape
+    _req(q, torch.float32, "knn_queries")
+    out = torch.empty(rows, dim, dtype=torch.bfloat16, device=q.device)
+    n2 = torch.empty(rows, dtype=torch.float32, device=q.device)
+    check(kernels().cfc_knn_queries(out.data_ptr(), q.data_ptr(), n2.data_ptr(), int(unit), rows, dim, _stream(q)), "cfc_knn_queries")
+    return out, n2
+
+
 def pool(hidden, cu_seqlens, mode="mean", normalize=True):
     """[nseq, dim] fp32 sentence embeddings from packed token states."""
     if not hidden.is_cuda:

@@ -351,12 +351,19 @@ class HipFlatIndex(VectorStore):
         """Device-side exact search: (scores [nq, k], row indices [nq, k]) for queries Q."""
         from ..ops import kernels as K
         lo, hi = rows if rows is not None else (0, self._n)
-        Q = _as_matrix(Q, self.dim, device=self.device, dtype=torch.bfloat16)
+        # floats that lie beside the index need no launch of their own to be rounded
+        beside = (isinstance(Q, torch.Tensor) and Q.is_cuda and Q.device == self._X.device and Q.dtype == torch.float32
+                  and Q.dim() == 2 and Q.shape[1] == self.dim and Q.shape[0] > 0 and self.dim % 8 == 0 and Q.is_contiguous()
+                  and Q.data_ptr() % 16 == 0 and hi > lo and Q.shape[0] <= 16 and k <= 256)
+        if not beside:
+            Q = _as_matrix(Q, self.dim, device=self.device, dtype=torch.bfloat16)
         nq = Q.shape[0]
         if hi <= lo:
             return (torch.empty(nq, 0, device=self.device), torch.empty(nq, 0, dtype=torch.long, device=self.device))
         X = self._X[lo:hi]
-        if self.metric == "cosine":
+        if beside:
+            Qn, qn2 = K.knn_queries(Q, self.metric == "cosine")
+        elif self.metric == "cosine":
             Qn = K.l2_normalize(Q.contiguous())
             qn2 = None
         else:

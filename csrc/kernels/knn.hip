@@ -87,61 +87,61 @@ struct KnnRows {
 // they are stored as they lie and their largest key goes to bmax [nq][nb].  Nothing is selected here, so the pass is a plain
 // stream over X: 1M x 384 bf16 with one query in 131 us (5.9 TB/s) where scoring 2048-row chunks into LDS and selecting in
 // them took 172 us (4.5 TB/s; 489 workgroups, two on most CUs and one on the rest, the selecting wave alone at each one's end).
-// MAXIMA: only the best score of every 16 rows is stored, to out [nq][ld] (B = 64).
+// MAXIMA: only the best score of every 16 rows is stored, to out [nq][ld] (B = 64).  A wave takes every gridDim-th block.
 template <int KC, bool MAXIMA>
 __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
                                                        int nq, const float* __restrict__ xnorm2,
                                                        const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
                                                        float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
                                                        int B) {
-  const int lane = threadIdx.x & 63, blk = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (blk >= nb) return;
-  const int col = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const bool qv = col < nq;
   KnnRows<KC> rows{X, N, xnorm2, alive};
   rows.queries(Q, qnorm2, nq);
-  const int lo = blk * B, hi = min(N, lo + B);
   const bool vec = (ld & 3) == 0 && ((uintptr_t)out & 15) == 0;
-  uint32_t best = 0u;
-  auto take = [&](const uint4* a, int r0) {
-    const f32x4_t v = rows.score(a, r0);
-    const uint32_t m = rows.best(v, r0);
-    if constexpr (MAXIMA) {
-      if (r0 - lo == 16 * g) best = m;            // group g's
-    } else {
-      best = max(best, m);
-      const int rb = r0 + 4 * g;
-      if (!qv) return;
-      float* o = out + col * ld + rb;
-      if (rb + 3 < N && vec) {
-        *reinterpret_cast<f32x4_t*>(o) = v;
+  for (int blk = blockIdx.x * 4 + (threadIdx.x >> 6); blk < nb; blk += gridDim.x * 4) {
+    const int lo = blk * B, hi = min(N, lo + B);
+    uint32_t best = 0u;
+    auto take = [&](const uint4* a, int r0) {
+      const f32x4_t v = rows.score(a, r0);
+      const uint32_t m = rows.best(v, r0);
+      if constexpr (MAXIMA) {
+        if (r0 - lo == 16 * g) best = m;            // group g's
       } else {
+        best = max(best, m);
+        const int rb = r0 + 4 * g;
+        if (!qv) return;
+        float* o = out + col * ld + rb;
+        if (rb + 3 < N && vec) {
+          *reinterpret_cast<f32x4_t*>(o) = v;
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (rb + i < N) o[i] = v[i];
+          for (int i = 0; i < 4; ++i)
+            if (rb + i < N) o[i] = v[i];
+        }
+      }
+    };
+    if constexpr (KC <= 16) {          // the next 16 rows in flight under these (144 -> 131 us); wider rows fill the registers alone
+      uint4 a[2][KC];
+      rows.load(a[0], lo);
+      for (int r0 = lo; r0 < hi; r0 += 32) {
+        if (r0 + 16 < hi) rows.load(a[1], r0 + 16);
+        take(a[0], r0);
+        if (r0 + 32 < hi) rows.load(a[0], r0 + 32);
+        if (r0 + 16 < hi) take(a[1], r0 + 16);
+      }
+    } else {
+      uint4 a[KC];
+      for (int r0 = lo; r0 < hi; r0 += 16) {
+        rows.load(a, r0);
+        take(a, r0);
       }
     }
-  };
-  if constexpr (KC <= 16) {          // the next 16 rows in flight under these (144 -> 131 us); wider rows fill the registers alone
-    uint4 a[2][KC];
-    rows.load(a[0], lo);
-    for (int r0 = lo; r0 < hi; r0 += 32) {
-      if (r0 + 16 < hi) rows.load(a[1], r0 + 16);
-      take(a[0], r0);
-      if (r0 + 32 < hi) rows.load(a[0], r0 + 32);
-      if (r0 + 16 < hi) take(a[1], r0 + 16);
+    if constexpr (MAXIMA) {
+      if (qv && lo + 16 * g < hi) out[col * ld + 4 * blk + g] = key2f(best);
+    } else if (bmax && g == 0 && qv) {
+      bmax[(size_t)col * nb + blk] = best;
     }
-  } else {
-    uint4 a[KC];
-    for (int r0 = lo; r0 < hi; r0 += 16) {
-      rows.load(a, r0);
-      take(a, r0);
-    }
-  }
-  if constexpr (MAXIMA) {
-    if (qv && lo + 16 * g < hi) out[col * ld + 4 * blk + g] = key2f(best);
-  } else if (bmax && g == 0 && qv) {
-    bmax[(size_t)col * nb + blk] = best;
   }
 }
 
@@ -267,7 +267,7 @@ __device__ __forceinline__ uint64_t sel_cut(uint64_t* cand, int cnt, int kk, int
 // that value, at a lower row than any later block's.  Once cut, the k kept bound what may still come.  (300 of 1M: equal
 // scores 48 us where looking at every block that reaches the bound took 5075, all but 100 masked 86 where it took 5586,
 // others as before, 32; the radix passes 258, 189 and 176.)
-// A chain of short steps: 18 us for 150 of 1M scores, where three rounds of radix histograms in LDS over
+// A chain of short steps: 13 us for 150 of 1M scores, where three rounds of radix histograms in LDS over
 // 2048-row chunks' winners and a library sort took 120.
 // ids (row stride ld, optional): what the rows are called; else row0 + row.
 // grid (queries, segments): workgroup y selects from `seg` of the n scores, a whole number of blocks of B, into
@@ -308,7 +308,56 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
   // below the bits that all maxima share
   uint32_t thr = 0;
   int reach = nb;                                    // blocks that do
-  if (nb > k) {
+  const int most = k + k / 4;
+  auto blocks_at = [&](uint32_t t) {
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) c += __popcll(__ballot(key[j] >= t));
+    return c;
+  };
+  if (nb >= SEL_THREADS && k <= SEL_THREADS / 4) {
+    // What k threads' best blocks reach will do if not many more blocks do: few of the k best share one of 1024 threads, of 256
+    // about 40 do, which `most` leaves room for; of more it would not.  One wave looks at the threads' best, without a barrier
+    // a bit (15 625 blocks, k 150: 6.2 -> 3.9 us; 1 250 blocks, k 20: 4.4 -> 2.9).
+    uint32_t best = 0u;
+#pragma unroll
+    for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) best = max(best, key[j]);
+    uint32_t* bests = reinterpret_cast<uint32_t*>(cand);
+    bests[tid] = best;
+    __syncthreads();
+    if (tid < 64) {
+      uint32_t e[SEL_WAVES], lo = ~0u, hi = 0u;
+#pragma unroll
+      for (int j = 0; j < SEL_WAVES; ++j) {
+        e[j] = bests[64 * j + lane];
+        lo = min(lo, e[j]);
+        hi = max(hi, e[j]);
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
+      }
+      uint32_t t = hi;
+      if (lo != hi) {
+        const int top = 31 - __clz(lo ^ hi);
+        t = top == 31 ? 0u : hi >> (top + 1) << (top + 1);
+        for (int b = top; b >= 0; --b) {
+          const uint32_t x = t | (1u << b);
+          int c = 0;
+#pragma unroll
+          for (int j = 0; j < SEL_WAVES; ++j) c += __popcll(__ballot(e[j] >= x));
+          if (c >= k) t = x;
+          if (c >= k && c <= k + k / 16) break;
+        }
+      }
+      if (lane == 0) s_lo[0] = t;
+    }
+    __syncthreads();
+    thr = s_lo[0];
+    reach = sel_count(blocks_at(thr), red, turn);
+  }
+  if (nb > k && reach > most) {
     uint32_t lo = ~0u, hi = 0u;
 #pragma unroll
     for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
@@ -320,10 +369,12 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
       lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
       hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
     }
+    __syncthreads();
     if (lane == 0) { s_lo[tid >> 6] = lo; s_hi[tid >> 6] = hi; }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < SEL_WAVES; ++i) { lo = min(lo, s_lo[i]); hi = max(hi, s_hi[i]); }
+    reach = nb;
     if (lo == hi) {
       thr = hi;
     } else {
@@ -331,16 +382,13 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
       thr = top == 31 ? 0u : hi >> (top + 1) << (top + 1);
       for (int b = top; b >= 0; --b) {
         const uint32_t t = thr | (1u << b);
-        int c = 0;
-#pragma unroll
-        for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) c += __popcll(__ballot(key[j] >= t));
-        c = sel_count(c, red, turn);
+        const int c = sel_count(blocks_at(t), red, turn);
         if (c >= k) thr = t, reach = c;
-        if (c >= k && c <= k + k / 4) break;
+        if (c >= k && c <= most) break;
       }
     }
   }
-  if (nb > k && reach > k + k / 4) {                 // thr is the k-th best maximum itself; seldom so: read again, not unrolled
+  if (nb > k && reach > most) {                      // thr is the k-th best maximum itself; seldom so: read again, not unrolled
     int c = 0;
 #pragma unroll 1
     for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
@@ -370,15 +418,24 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
   }
   if (tid == 0) { s_n = 0; s_list = 0; }
   __syncthreads();
+  {
+    uint64_t m[SEL_BLOCKS / SEL_THREADS];
+    int mine = 0;
 #pragma unroll
-  for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
-    const int i = tid + j * SEL_THREADS;
-    const bool p = i < nb && key[j] >= thr;
-    const uint64_t m = __ballot(p);
-    int at = 0;
-    if (lane == 0 && m) at = atomicAdd(&s_list, __popcll(m));
-    at = __shfl(at, 0, 64) + __popcll(m & below);
-    if (p) list[at] = (uint16_t)i;
+    for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
+      m[j] = __ballot(tid + j * SEL_THREADS < nb && key[j] >= thr);
+      mine += __popcll(m[j]);
+    }
+    if (mine) {
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&s_list, mine);
+      at = __shfl(at, 0, 64);
+#pragma unroll
+      for (int j = 0; j < SEL_BLOCKS / SEL_THREADS; ++j) {
+        if (m[j] >> lane & 1) list[at + __popcll(m[j] & below)] = (uint16_t)(tid + j * SEL_THREADS);
+        at += __popcll(m[j]);
+      }
+    }
   }
   __syncthreads();
   const long total = (long)s_list << lb;             // scores to look at, four neighbours per thread
@@ -432,12 +489,17 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const float* _
     if (cnt > (s0 + SEL_STEP < total ? SEL_CAP - SEL_STEP : max(k, SEL_THREADS))) floor = sel_cut(cand, cnt, k, red, turn, &s_n, bits);
   }
   const int cnt = s_n;                                // at least min(k, n)
-  for (int i = tid; i < cnt; i += SEL_THREADS) {
+  const int share = cnt <= SEL_THREADS / 4 ? 2 : 0;   // few candidates: four threads count for one (173 of them: 3.1 -> 1.6 us)
+  for (int i = tid >> share; i < cnt; i += SEL_THREADS >> share) {
     const uint64_t e = cand[i];
     int rank = 0;
 #pragma unroll 4
-    for (int j = 0; j < cnt; ++j) rank += cand[j] > e;
-    if (rank >= k) continue;
+    for (int j = tid & ((1 << share) - 1); j < cnt; j += 1 << share) rank += cand[j] > e;
+    if (share) {
+      rank += __shfl_xor(rank, 1, 64);
+      rank += __shfl_xor(rank, 2, 64);
+    }
+    if (rank >= k || (tid & ((1 << share) - 1))) continue;
     const uint32_t r = 0xffffffffu - (uint32_t)e;
     out_v[rank] = key2f((uint32_t)(e >> 32));
     out_i[rank] = ids ? ids[r] : row0 + r;
@@ -559,29 +621,43 @@ __global__ void __launch_bounds__(256) ivf_topk_kernel(const uint16_t* __restric
   }
 }
 
-__global__ void __launch_bounds__(256) l2_normalize_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ in,
-                                                           float* __restrict__ norms2, int dim) {
+// Rows of bf16, or of floats that are rounded to bf16 first (queries: a launch that took them there alone was 4 us of a
+// search of a million rows in 154), to unit length; `as_is`: only rounded.
+template <typename T>
+__global__ void __launch_bounds__(256) l2_normalize_kernel(uint16_t* __restrict__ out, const T* __restrict__ in,
+                                                           float* __restrict__ norms2, int dim, bool as_is) {
   __shared__ float red[16];
   const int row = blockIdx.x;
   const int nvec = dim / 8;
   const uint4* src = reinterpret_cast<const uint4*>(in + (size_t)row * dim);
+  auto load = [&](int c) {
+    if constexpr (sizeof(T) == 2) {
+      return src[c];
+    } else {
+      const uint4 a = src[2 * c], b = src[2 * c + 1];
+      return make_uint4(pack2bf(__uint_as_float(a.x), __uint_as_float(a.y)), pack2bf(__uint_as_float(a.z), __uint_as_float(a.w)),
+                        pack2bf(__uint_as_float(b.x), __uint_as_float(b.y)), pack2bf(__uint_as_float(b.z), __uint_as_float(b.w)));
+    }
+  };
   float ss = 0.f;
   for (int c = threadIdx.x; c < nvec; c += blockDim.x) {
     float v[8];
-    unpack8(src[c], v);
+    unpack8(load(c), v);
 #pragma unroll
     for (int j = 0; j < 8; ++j) ss += v[j] * v[j];
   }
   ss = block_sum(ss, red);
   if (norms2 && threadIdx.x == 0) norms2[row] = ss;
-  const float inv = ss > 0.f ? rsqrtf(ss) : 0.f;
+  const float inv = as_is ? 1.f : ss > 0.f ? rsqrtf(ss) : 0.f;
   if (!out) return;
   uint4* dst = reinterpret_cast<uint4*>(out + (size_t)row * dim);
   for (int c = threadIdx.x; c < nvec; c += blockDim.x) {
     float v[8];
-    unpack8(src[c], v);
+    unpack8(load(c), v);
+    if (!as_is) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] *= inv;
+      for (int j = 0; j < 8; ++j) v[j] *= inv;
+    }
     dst[c] = pack8(v);
   }
 }
@@ -675,6 +751,12 @@ CFC_API int cfc_topk_segment(int n) {
   return ((n - 1) / parts / SEL_WIDEST + 1) * SEL_WIDEST;
 }
 
+// Where rows of up to 512 values come from the 256 MB that the chip caches, workgroups of one round (two a CU) take all
+// blocks, and no last round is nearly empty: 50 k rows of 384 9.8 -> 8.6 us, 100 k of 16 queries 21.8 -> 16.5, 200 k 28.4
+// -> 24.7; 300 k 36.2 -> 38.2 (from memory a workgroup per four blocks reads faster), 100 k of 768 28.2 -> 28.5.
+constexpr long KNN_ROUND_BYTES = 160l << 20;
+constexpr int KNN_ROUND = 512;
+
 // Scores of rows [0, N) of X for nq queries into out [nq][ld], and the largest key of every cfc_topk_block(N) rows into
 // bmax [nq][blocks] (null: not wanted), which has room for `room` of them.
 CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
@@ -682,7 +764,8 @@ CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, c
   if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || ld < N) return -1;
   const int B = cfc_topk_block(N), nb = (N - 1) / B + 1;
   if (bmax && (long)nq * nb > room) return -1;
-#define KS(KC) knn_scan_kernel<KC, false><<<(nb + 3) / 4, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, \
+  const int all = (nb + 3) / 4, grid = dim <= 512 && (long)N * dim * 2 <= KNN_ROUND_BYTES ? min(all, KNN_ROUND) : all;
+#define KS(KC) knn_scan_kernel<KC, false><<<grid, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, \
       qnorm2, alive, out, (size_t)ld, bmax, nb, B); break
   KNN_DIMS(KS)
 #undef KS
@@ -730,7 +813,14 @@ CFC_API int cfc_topk_select(const float* in, const int64_t* ids, int nq, int n, 
 CFC_API int cfc_l2_normalize(void* out, const void* in, float* norms2, int rows, int dim, hipStream_t stream) {
   if (dim % 8 != 0) return -1;
   if (rows == 0) return 0;
-  l2_normalize_kernel<<<rows, dim >= 2048 ? 256 : 64, 0, stream>>>((uint16_t*)out, (const uint16_t*)in, norms2, dim);
+  l2_normalize_kernel<<<rows, dim >= 2048 ? 256 : 64, 0, stream>>>((uint16_t*)out, (const uint16_t*)in, norms2, dim, false);
+  return CFC_CHECK_LAUNCH();
+}
+
+// Queries of floats [rows][dim] to bf16, of unit length if `unit`, and the squared norms of the rounded ones (all 16-byte aligned).
+CFC_API int cfc_knn_queries(void* out, const float* in, float* norms2, int unit, int rows, int dim, hipStream_t stream) {
+  if (dim % 8 != 0 || rows < 1) return -1;
+  l2_normalize_kernel<<<rows, dim >= 2048 ? 256 : 64, 0, stream>>>((uint16_t*)out, in, norms2, dim, !unit);
   return CFC_CHECK_LAUNCH();
 }
 

@@ -173,3 +173,65 @@ def test_segments_of_scores(kind, nq, n, k):
     assert torch.equal(v, rv[:, :k]) and torch.equal(i, ri[:, :k])
     ids = torch.randint(0, 1 << 40, (nq, n), device=DEV)
     assert torch.equal(K.topk(s, k, ids)[1], ids.gather(1, ri[:, :k]))
+
+
+@pytest.mark.parametrize("n", [16 * 1023, 16 * 1024, 16 * 1025 + 1, 16 * 16384])
+@pytest.mark.parametrize("k", [1, 150, 255, 256, 257])
+@pytest.mark.parametrize("kind", ["normal", "stacked", "ties"])
+def test_bound_from_the_threads_best(kind, k, n):
+    """Selections that look at 1024 threads' best blocks first, and the next larger k and next fewer blocks, which do not.
+    stacked: the best blocks belong to few threads (block b is thread b % 1024's), so that bound lets too many pass."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    s = _scores("ties" if kind == "ties" else "normal", 2, n)
+    if kind == "stacked":
+        b = torch.arange(n, device=DEV) // 16 % 1024
+        s = s + 100.0 * ((b < 40) | (b == 1023))
+    rv, ri = s.sort(dim=1, descending=True, stable=True)
+    v, i = K.topk(s, k)
+    assert torch.equal(v, rv[:, :k]) and torch.equal(i, ri[:, :k])
+
+
+@pytest.mark.parametrize("dim,nq,N", [(384, 3, 32_767), (384, 16, 32_769), (384, 2, 65_601), (512, 1, 163_840), (512, 1, 163_841),
+                                      (128, 5, 655_347), (768, 2, 70_001)])
+def test_scan_by_workgroups_of_one_round(dim, nq, N):
+    """Sizes about 512 workgroups' first round and about the bytes up to which they take all blocks; rows wider than that."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(N)
+    X, Q = (torch.randn(n, dim, device=DEV, generator=g).bfloat16() for n in (N, nq))
+    want = K.knn_scores(X, Q, None, None)
+    rv, ri = want.sort(dim=1, descending=True, stable=True)
+    v, i = K.knn_topk(X, Q, 100, N=N)
+    assert torch.equal(v, rv[:, :100]) and torch.equal(i, ri[:, :100])
+
+
+@pytest.mark.parametrize("metric", ["cosine", "dot", "l2"])
+@pytest.mark.parametrize("dim,nq", [(128, 1), (384, 16), (768, 2), (1024, 5)])
+def test_float_queries_in_one_launch(metric, dim, nq):
+    """Queries of floats beside the index, rounded and normalized by one launch, against those of other strides and alignments
+    and of 16 bits, which are rounded before: the same bf16 values, so the same cosine and dot scores; of l2 the query's norm
+    is summed in another order, dim products and sums of 2^-24 each."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    from copilot_for_consensus_amd.vectorstore import HipFlatIndex
+    g = torch.Generator().manual_seed(dim)
+    index = HipFlatIndex(dim, distance=metric, device=DEV)
+    index.add_embeddings([str(j) for j in range(700)], torch.randn(700, dim, generator=g))
+    flat = torch.zeros(nq * dim + 1, device=DEV)
+    q = torch.randn(nq, dim, generator=g) * torch.logspace(-20, 15, nq * dim).view(nq, dim)[:, torch.randperm(dim, generator=g)]
+    q[0] = torch.randn(dim, generator=g)
+    if nq > 2:
+        q[1], q[2] = 0.0, torch.linspace(-1, 1, dim) * 2.0 ** -130
+    q = q.to(DEV)
+    flat[1:] = q.flatten()
+    wide = torch.zeros(nq, dim + 8, device=DEV)
+    wide[:, :dim] = q
+    unit = K.l2_normalize(q.bfloat16()) if metric == "cosine" else q.bfloat16()
+    got, n2 = K.knn_queries(q, metric == "cosine")
+    assert torch.equal(got, unit)
+    torch.testing.assert_close(n2, q.bfloat16().double().pow(2).sum(1).float(), rtol=dim * 2.0 ** -24, atol=2.0 ** -126)
+    v, i = index.search(q, 20)
+    for other in (flat[1:].view(nq, dim), wide[:, :dim], q.bfloat16()):
+        ov, oi = index.search(other, 20)
+        if metric == "l2":
+            torch.testing.assert_close(v, ov, rtol=(dim + 4) * 2.0 ** -24, atol=0.0)
+        else:
+            assert torch.equal(v, ov) and torch.equal(i, oi)
