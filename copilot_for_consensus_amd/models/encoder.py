@@ -14,6 +14,7 @@ hundreds of chunks per forward:
 """
 from __future__ import annotations
 
+import ctypes
 import dataclasses
 import itertools
 import math
@@ -24,6 +25,11 @@ import torch
 import torch.nn.functional as F
 
 from ..ops import kernels as K
+from ..ops._native import runtime
+
+
+def _up4(n: int) -> int:
+    return -(-n // 4) * 4
 
 
 @dataclasses.dataclass(frozen=True)
@@ -196,19 +202,27 @@ class EncoderModel:
             return K.pgemm_ln(x, w, bias, residual, gamma, beta, eps)
         return K.layernorm(self._linear(x, w), gamma, beta, eps, bias=bias, residual=residual)
 
-    def _h2d(self, *arrays) -> list[torch.Tensor]:
-        """The arrays as int32 tensors on the device, by one copy from pinned memory: a copy from pageable memory holds the
-        host until the stream has come to it, so a batch would be prepared after the one before it and not beside it."""
-        import numpy as np
-        if self.device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+    def _texts(self, ids, cu) -> tuple[list[torch.Tensor], int]:
+        """([ids, positions, starts, tiles' texts, tiles' first rows] as int32 tensors on the device, longest text) of packed
+        texts.  A short batch goes there with a launch; else by one copy from pinned memory: a copy from pageable memory holds
+        the host until the stream has come to it, so a batch would be prepared after the one before it and not beside it."""
+        cuda = self.device.type == "cuda"
+        if cuda and torch.cuda.is_current_stream_capturing():
             raise RuntimeError("encoding copies its texts from host memory that a graph would not keep: capture forward_packed")
-        at = np.cumsum([0] + [-(-len(a) // 4) * 4 for a in arrays])
-        buf = torch.empty(int(at[-1]), dtype=torch.int32, pin_memory=self.device.type == "cuda")
-        flat = buf.numpy()
-        for o, a in zip(at, arrays):
-            flat[o:o + len(a)] = a
-        d = buf.to(self.device, non_blocking=True)
-        return [d[o:o + len(a)] for o, a in zip(at, arrays)]
+        T, n, tile = int(cu[-1]) - int(cu[0]), len(cu) - 1, K.ENCODER_TILE_ROWS
+        room = 2 * _up4(T) + _up4(n + 1) + 2 * _up4(max(T, 0) // tile + n)
+        small = cuda and room <= K.PUT_INTS
+        buf = torch.empty(max(room, 0), dtype=torch.int32, pin_memory=cuda and not small)
+        sizes = (ctypes.c_int64 * 2)()
+        if runtime().cfc_pack_texts(ids.ctypes.data, ids.size, cu.ctypes.data, n, tile, buf.data_ptr(), buf.numel(), sizes):
+            raise ValueError(f"starts of {n} texts that fall, or lie outside {ids.size} ids")
+        tiles, longest = sizes
+        if longest > self.cfg.max_seq_length:
+            raise ValueError(f"sequence of {longest} tokens > max_seq_length {self.cfg.max_seq_length}")
+        parts = [k for m in (T, T, n + 1, tiles, tiles) for k in (m, -m % 4)]
+        buf = buf[:sum(parts)]
+        d = K.put_ints(buf, self.device) if small else buf.to(self.device, non_blocking=True)
+        return list(d.split_with_sizes(parts)[::2]), longest
 
     @torch.inference_mode()
     def encode_ids(self, batch: list[list[int]], pooling: str | None = None, normalize: bool | None = None,
@@ -216,8 +230,7 @@ class EncoderModel:
         """Sentence embeddings [n, H] fp32 for pre-tokenised sequences (truncated to max_seq_length)."""
         import numpy as np
         seqs = [s[:self.cfg.max_seq_length] for s in batch]
-        cu = np.zeros(len(seqs) + 1, dtype=np.int32)
-        np.cumsum([len(s) for s in seqs], out=cu[1:])
+        cu = np.fromiter(itertools.accumulate(map(len, seqs), initial=0), dtype=np.int64, count=len(seqs) + 1)
         ids = np.fromiter(itertools.chain.from_iterable(seqs), dtype=np.int32, count=int(cu[-1]))
         return self.encode_packed(ids, cu, pooling, normalize, max_tokens_per_forward)
 
@@ -233,23 +246,20 @@ class EncoderModel:
         normalize = c.normalize if normalize is None else normalize
         ids = np.ascontiguousarray(ids, dtype=np.int32)
         cu = np.ascontiguousarray(cu_seqlens, dtype=np.int64)
-        lens = np.diff(cu)
-        if len(lens) and int(lens.max()) > c.max_seq_length:
-            raise ValueError(f"sequence of {int(lens.max())} tokens > max_seq_length {c.max_seq_length}")
-        pos_all = (np.arange(int(cu[-1]), dtype=np.int64) - np.repeat(cu[:-1], lens)).astype(np.int32)
-        dev = self.device
+        if cu.ndim != 1 or int(cu[0]) != 0 or (ids.ndim != 1 and ids.size != 1):
+            raise ValueError(f"ids of shape {ids.shape}, starts of shape {cu.shape} (one dimension each, the first start 0)")
+        n = len(cu) - 1
+        whole = int(cu[-1]) <= max_tokens_per_forward
+        if not whole and int(np.diff(cu).max(initial=0)) > c.max_seq_length:
+            raise ValueError(f"sequence of {int(np.diff(cu).max())} tokens > max_seq_length {c.max_seq_length}")
         outs = []
-        i, n = 0, len(lens)
+        i = 0
         while i < n:
             # as many whole sequences as fit in max_tokens_per_forward (at least one)
-            j = int(np.searchsorted(cu, cu[i] + max_tokens_per_forward, side="right")) - 1
+            j = n if whole else int(np.searchsorted(cu, cu[i] + max_tokens_per_forward, side="right")) - 1
             j = min(max(j, i + 1), n)
-            t0, t1 = int(cu[i]), int(cu[j])
-            per = -(-lens[i:j] // K.ENCODER_TILE_ROWS)          # query tiles of each sequence
-            seq_t = np.repeat(np.arange(j - i), per)
-            q0_t = (np.arange(len(seq_t)) - np.repeat(np.cumsum(per) - per, per)) * K.ENCODER_TILE_ROWS
-            ids_t, pos_t, cu_t, *tiles = self._h2d(ids[t0:t1], pos_all[t0:t1], cu[i:j + 1] - t0, seq_t, q0_t)
-            h = self.forward_packed(ids_t, pos_t, cu_t, int(lens[i:j].max()), tiles=tuple(tiles))
+            (ids_t, pos_t, cu_t, *tiles), longest = self._texts(ids, cu[i:j + 1])
+            h = self.forward_packed(ids_t, pos_t, cu_t, longest, tiles=tuple(tiles))
             outs.append(K.pool(h, cu_t, pooling, normalize))
             i = j
-        return torch.cat(outs, 0)
+        return outs[0] if len(outs) == 1 else torch.cat(outs, 0)

@@ -99,6 +99,7 @@ _KERNEL_SIGS = {
     "cfc_enc_rows": [I],
     "cfc_knn_queries": [P, P, P, I, I, I, P],
     "cfc_enc_tiny": [I, I, I, P],
+    "cfc_put_ints": [P, P, I, P],
     "cfc_enc_forward": [P] * 10 + [I, I, I, I, P, I, F, F, I] + [P] * 6,
     "cfc_knn_scan": [P, P, I, I, I, P, P, P, P, L, P, L, P],
     "cfc_knn_maxima": [P, P, I, I, I, P, P, P, P, L, P],
@@ -171,6 +172,7 @@ _RUNTIME_SIGS = {
     "cfc_blockpool_free": [P, P, I],
     "cfc_blockpool_num_free": [P],
     "cfc_mbox_split": [ctypes.c_char_p, c_int64, P, I],
+    "cfc_pack_texts": [P, c_int64, P, c_int64, I, P, c_int64, P],
 }
 
 _RESTYPES = {

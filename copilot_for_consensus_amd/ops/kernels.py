@@ -16,6 +16,7 @@ import ctypes
 import dataclasses
 import functools
 import math
+import operator
 import os
 
 import torch
@@ -379,9 +380,24 @@ ENCODER_LAYER = ("qkv", "qkv_b", "o", "o_b", "ln1_g", "ln1_b", "up", "up_b", "do
 ENCODER_HIDDEN, ENCODER_FFN = 384, 1536      # what encoder.hip is built for
 
 
-_ENCODER_SHAPES = [(k, {"qkv": (3 * ENCODER_HIDDEN, ENCODER_HIDDEN), "qkv_b": (3 * ENCODER_HIDDEN,),
-                       "o": (ENCODER_HIDDEN, ENCODER_HIDDEN), "up": (ENCODER_FFN, ENCODER_HIDDEN), "up_b": (ENCODER_FFN,),
-                       "down": (ENCODER_HIDDEN, ENCODER_FFN)}.get(k, (ENCODER_HIDDEN,))) for k in ENCODER_LAYER]
+_ENCODER_SHAPES = [{"qkv": (3 * ENCODER_HIDDEN, ENCODER_HIDDEN), "qkv_b": (3 * ENCODER_HIDDEN,),
+                    "o": (ENCODER_HIDDEN, ENCODER_HIDDEN), "up": (ENCODER_FFN, ENCODER_HIDDEN), "up_b": (ENCODER_FFN,),
+                    "down": (ENCODER_HIDDEN, ENCODER_FFN)}.get(k, (ENCODER_HIDDEN,)) for k in ENCODER_LAYER]
+_ENCODER_TENSORS = operator.itemgetter(*ENCODER_LAYER)
+_DTYPE, _SHAPE = operator.attrgetter("dtype"), operator.attrgetter("shape")
+
+
+PUT_INTS = 896          # what a launch carries (elementwise.hip put_ints_kernel)
+
+
+def put_ints(host: torch.Tensor, device) -> torch.Tensor:
+    """At most PUT_INTS int32 values of host memory on the GPU, by a launch that carries them."""
+    _req(host, torch.int32, "put_ints")
+    if host.is_cuda or host.numel() > PUT_INTS:
+        raise ValueError(f"put_ints: {host.numel()} values on {host.device} (up to {PUT_INTS} of host memory)")
+    out = torch.empty(host.shape, dtype=torch.int32, device=device)
+    check(kernels().cfc_put_ints(out.data_ptr(), host.data_ptr(), host.numel(), _stream(out)), "cfc_put_ints")
+    return out
 
 
 def encoder_weights(T: int, p: dict, layers: list[dict], heads: int, max_seqlen: int) -> list[int] | None:
@@ -391,22 +407,15 @@ def encoder_weights(T: int, p: dict, layers: list[dict], heads: int, max_seqlen:
     if not word.is_cuda or T < 1 or not kernels().cfc_enc_rows(T) or not layers or not 1 <= max_seqlen <= 512 \
             or heads not in (H // 32, H // 64):
         return None
-    dev, bf16, out, low = word.get_device(), torch.bfloat16, [], 0
-    def takes(t, shape):
-        return t.shape == shape and t.dtype is bf16 and t.get_device() == dev and t.is_contiguous()
-    for k in ("word", "pos", "type", "emb_g", "emb_b"):
-        t = p[k]
-        if not takes(t, (H,) if k.startswith("emb") else (t.shape[0], H)):
-            return None
-        out.append(t.data_ptr())
-    for lw in layers:
-        for k, shape in _ENCODER_SHAPES:
-            if not takes(lw[k], shape):
-                return None
-            out.append(lw[k].data_ptr())
-    for a in out:
-        low |= a
-    return None if low & 15 else out
+    emb = [p[k] for k in ("word", "pos", "type", "emb_g", "emb_b")]
+    ts = emb + [t for lw in layers for t in _ENCODER_TENSORS(lw)]
+    # all of them by one attribute at a time: half the time of one tensor after the other, which a short text waited for
+    if set(map(torch.Tensor.get_device, ts)) != {word.get_device()} or set(map(_DTYPE, ts)) != {torch.bfloat16} \
+            or not all(map(torch.Tensor.is_contiguous, ts)) \
+            or list(map(_SHAPE, ts)) != [(t.shape[0], H) for t in emb[:3]] + [(H,)] * 2 + _ENCODER_SHAPES * len(layers):
+        return None
+    out = list(map(torch.Tensor.data_ptr, ts))
+    return None if functools.reduce(operator.or_, out) & 15 else out
 
 
 def encoder_forward(ids, positions, weights: list[int], layers: int, cu_seqlens, tiles, heads: int, max_seqlen: int, scale: float,

@@ -137,3 +137,33 @@ def test_texts_are_not_captured():
         x += 1
     g.replay()
     assert torch.equal(m.encode_ids(texts), want) and bool((x == 1).all())
+
+
+@pytest.mark.parametrize("n", [0, 1, 255, 257, 895, 896])
+def test_integers_that_go_with_the_launch(n):
+    from copilot_for_consensus_amd.ops import kernels as K
+    host = torch.arange(n, dtype=torch.int32) * 5 - 7
+    want = host.clone()
+    got = K.put_ints(host, DEV)
+    host.fill_(-1)              # the launch has them already
+    assert torch.equal(got.cpu(), want)
+    with pytest.raises(ValueError):
+        K.put_ints(torch.zeros(897, dtype=torch.int32), DEV)
+
+
+@pytest.mark.parametrize("lens", [[1], [3, 4, 0, 5], [256, 64, 65], [256, 129, 20], [256, 130, 20], [7] * 40, [0, 0, 2], [200] * 9])
+def test_texts_laid_out_for_the_encoder(lens):
+    """What the host lays out for a batch that goes with a launch and one that is copied, against array operations."""
+    import numpy as np
+    from copilot_for_consensus_amd.ops import kernels as K
+    m = _model("minilm-l6", seed=0)
+    cu = np.cumsum([0] + lens).astype(np.int64)
+    ids = np.arange(cu[-1], dtype=np.int32) % 90
+    per = [-(-n // K.ENCODER_TILE_ROWS) for n in lens]
+    want = [ids, np.concatenate([np.arange(n) for n in lens]), cu, np.repeat(np.arange(len(lens)), per),
+            np.concatenate([np.arange(n) * K.ENCODER_TILE_ROWS for n in per])]
+    got, longest = m._texts(ids, cu)
+    assert longest == max(lens) and all(np.array_equal(a.cpu().numpy(), b) for a, b in zip(got, want))
+    for bad in ([0, 5, 3], [0, len(ids) + 1], [1, 2]):
+        with pytest.raises(ValueError):
+            m.encode_packed(ids, bad)
