@@ -51,6 +51,20 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
     const int c = (k * BT + threadIdx.x) * V;
     xv[k] = c < W ? ldv<V>(x + row + c) : zerov<V>();
   }
+  // One vector a thread: the weights are asked for with the row, and not each after the sum before it (32 rows of 4096: 6.7 -> 5.9 us).
+  constexpr bool AHEAD = NV == 1;
+  Vec<V> ahead[AHEAD ? 4 : 1];
+  if constexpr (AHEAD) {
+    const int c = min((int)threadIdx.x * V, W - V);
+    if (branch) {
+      if (b.wy) {
+        ahead[0] = ldv<V>(b.wy + c);
+        ahead[1] = ldv<V>(b.wy2 + c);
+      }
+      ahead[2] = ldgain<V>(b.g, c);
+    }
+    if (h) ahead[3] = ldgain<V>(next, c);
+  }
   if (branch) {
     Vec<V> y[NV];
     float s = 0.f;
@@ -62,22 +76,26 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
         const int c = (k * BT + threadIdx.x) * V;
         y[k] = z[k] = zerov<V>();
         if (c >= W) continue;
-        add_slabs<V>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
-        add_slabs<V>(z[k], b.y2, b.y2split, (int64_t)b.T * W, row + c);
+        Slabs<V> sy, sz;
+        sy.ask(b.y, b.ysplit, (int64_t)b.T * W, row + c);
+        sz.ask(b.y2, b.y2split, (int64_t)b.T * W, row + c);
+        sy.add(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
+        sz.add(z[k], b.y2, b.y2split, (int64_t)b.T * W, row + c);
 #pragma unroll
         for (int e = 0; e < V; ++e) {
           s += y[k].v[e] * y[k].v[e];
           s2 += z[k].v[e] * z[k].v[e];
         }
       }
-      const float r1 = b.factor / sqrtf(block_sum(s, red) * inv_w + b.eps);
-      const float r2 = b.factor / sqrtf(block_sum(s2, red2) * inv_w + b.eps);
+      block_sum2(s, s2, red, red2);
+      const float r1 = b.factor / sqrtf(s * inv_w + b.eps);
+      const float r2 = b.factor / sqrtf(s2 * inv_w + b.eps);
       s = 0.f;
 #pragma unroll
       for (int k = 0; k < NV; ++k) {
         const int c = (k * BT + threadIdx.x) * V;
         if (c >= W) continue;
-        const Vec<V> w1 = ldv<V>(b.wy + c), w2 = ldv<V>(b.wy2 + c);
+        const Vec<V> w1 = AHEAD ? ahead[0] : ldv<V>(b.wy + c), w2 = AHEAD ? ahead[AHEAD] : ldv<V>(b.wy2 + c);
 #pragma unroll
         for (int e = 0; e < V; ++e) {
           y[k].v[e] = y[k].v[e] * r1 * w1.v[e] + z[k].v[e] * r2 * w2.v[e];
@@ -95,13 +113,19 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
           for (int i0 = 0; i0 < b.top; i0 += 4) {         // four choices in flight (past the last: weight 0)
             Vec<V> r[4];
             float wt[4];
+            int id[4], mr[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
               const int64_t i = (int64_t)t * b.top + min(i0 + u, b.top - 1);
-              const bool own = b.ids[i] >= b.experts;
-              const ACT* src = own ? reinterpret_cast<const ACT*>(b.own) + row
-                                   : reinterpret_cast<const ACT*>(b.rows) + (size_t)b.mrow[i] * W;
-              wt[u] = i0 + u < b.top ? b.mwt[i] : 0.f;
+              id[u] = b.ids[i];
+              mr[u] = b.mrow[i];
+              wt[u] = b.mwt[i];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const ACT* src = id[u] >= b.experts ? reinterpret_cast<const ACT*>(b.own) + row
+                                                  : reinterpret_cast<const ACT*>(b.rows) + (size_t)mr[u] * W;
+              if (i0 + u >= b.top) wt[u] = 0.f;
               r[u] = ldv<V>(src + c);
             }
 #pragma unroll
@@ -118,7 +142,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
     for (int k = 0; k < NV; ++k) {
       const int c = (k * BT + threadIdx.x) * V;
       if (c >= W) continue;
-      const Vec<V> g = ldgain<V>(b.g, c);
+      const Vec<V> g = AHEAD ? ahead[2 * AHEAD] : ldgain<V>(b.g, c);
 #pragma unroll
       for (int e = 0; e < V; ++e) xv[k].v[e] += y[k].v[e] * r * g.v[e];
       stv<V>(x + row + c, xv[k]);
@@ -135,7 +159,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
   for (int k = 0; k < NV; ++k) {
     const int c = (k * BT + threadIdx.x) * V;
     if (c >= W) continue;
-    const Vec<V> g = ldgain<V>(next, c);
+    const Vec<V> g = AHEAD ? ahead[3 * AHEAD] : ldgain<V>(next, c);
     Vec<V> o;
 #pragma unroll
     for (int e = 0; e < V; ++e) o.v[e] = xv[k].v[e] * r * g.v[e];

@@ -69,32 +69,77 @@ __device__ __forceinline__ float xor32_max(float x) { float a = x, b = x; swap32
 __device__ __forceinline__ float xor16_sum(float x) { float a = x, b = x; swap16(a, b); return a + b; }
 __device__ __forceinline__ float xor16_max(float x) { float a = x, b = x; swap16(a, b); return fmaxf(a, b); }
 
+// x of the lane N places on in its row of 16.  A butterfly over the lanes i ^ 8, 4, 2, 1 may take its values from here: after
+// the step of 2 N the row repeats itself every 2 N lanes, so lane i + N holds what lane i ^ N does (a shuffle goes by the LDS,
+// 60 ns a step; this is an operand of the add).
+template <int N>
+__device__ __forceinline__ float row_ror(float x) {
+  return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x120 + N, 0xf, 0xf, false));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
   v = xor32_sum(v);
   v = xor16_sum(v);
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v += row_ror<8>(v);
+  v += row_ror<4>(v);
+  v += row_ror<2>(v);
+  return v + row_ror<1>(v);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
   v = xor32_max(v);
   v = xor16_max(v);
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  v = fmaxf(v, row_ror<8>(v));
+  v = fmaxf(v, row_ror<4>(v));
+  v = fmaxf(v, row_ror<2>(v));
+  return fmaxf(v, row_ror<1>(v));
 }
 
-// Block-wide sum for blockDim.x <= 1024 (multiple of 64). `red` must hold >= 16 floats.
+// the least of all lanes' integers (not below zero), in every lane
+__device__ __forceinline__ int wave_min_int(int v) {
+#define CFC_MIN_ROR(N) v = min(v, (int)__builtin_amdgcn_mov_dpp(v, 0x120 + N, 0xf, 0xf, false))
+  CFC_MIN_ROR(8);
+  CFC_MIN_ROR(4);
+  CFC_MIN_ROR(2);
+  CFC_MIN_ROR(1);
+#undef CFC_MIN_ROR
+  return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+             min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+// Block-wide sum for blockDim.x <= 1024 (multiple of 64). `red` must hold >= 16 floats.  All waves' sums are read at once: a
+// loop over them waits for the LDS at each round.
 __device__ __forceinline__ float block_sum(float v, float* red) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
   v = wave_sum(v);
   __syncthreads();
   if (lane == 0) red[wid] = v;
   __syncthreads();
-  float t = 0.f;
-  for (int i = 0; i < nw; ++i) t += red[i];
+  float r[16], t = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r[i] = red[i];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) t = i < nw ? t + r[i] : t;
   return t;
+}
+
+// Two of them between the same barriers.
+__device__ __forceinline__ void block_sum2(float& a, float& b, float* red, float* red2) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  a = wave_sum(a);
+  b = wave_sum(b);
+  __syncthreads();
+  if (lane == 0) { red[wid] = a; red2[wid] = b; }
+  __syncthreads();
+  float r[16], q[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r[i] = red[i], q[i] = red2[i];
+  a = b = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    a = i < nw ? a + r[i] : a;
+    b = i < nw ? b + q[i] : b;
+  }
 }
 
 // Block-wide max, same contract as block_sum.
@@ -104,8 +149,12 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   __syncthreads();
   if (lane == 0) red[wid] = v;
   __syncthreads();
-  float t = red[0];
-  for (int i = 1; i < nw; ++i) t = fmaxf(t, red[i]);
+  float r[16], t;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r[i] = red[i];
+  t = r[0];
+#pragma unroll
+  for (int i = 1; i < 16; ++i) t = i < nw ? fmaxf(t, r[i]) : t;
   return t;
 }
 

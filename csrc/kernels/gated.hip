@@ -135,6 +135,19 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
       if (acts && pos >= 2) xpp[k] = ldv<V>(st + (size_t)(pos & 1) * W + c);
     }
   }
+  // one vector a thread: the weights with the row, and not after the sums before them; so too what the last rows' indexes say
+  int m = 0;
+  if constexpr (MODE == GN_PROMPT) {
+    if (prev) {
+      m = meta[t];
+      pos = positions[t];
+    }
+  }
+  Vec<V> gain, gb1;
+  if (NV == 1 && branch) {
+    gain = ldv<V>(b.norm_w + min((int)threadIdx.x * V, W - V));
+    gb1 = ldv<V>(b.gbias + min((int)threadIdx.x * V, W - V));
+  }
   if (branch) {
     Vec<V> y[NV];
     float s = 0.f;
@@ -143,6 +156,8 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
       const int c = (k * BT + threadIdx.x) * V;
       y[k] = zerov<V>();
       if (c >= W) continue;
+      Vec<V> g = zerov<V>();
+      if (b.gate_act) g = ldv<V>(reinterpret_cast<const ACT*>(b.gate) + (size_t)t * b.gld + c);
       if (b.y) add_slabs<V>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
       if (b.y2) add_slabs<V>(y[k], b.y2, b.y2split, (int64_t)b.T * W, row + c);
       if (b.ym)
@@ -152,10 +167,8 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
 #pragma unroll
           for (int e = 0; e < V; ++e) y[k].v[e] += wt * r.v[e];
         }
-      Vec<V> g = zerov<V>();
-      if (b.gate_act) g = ldv<V>(reinterpret_cast<const ACT*>(b.gate) + (size_t)t * b.gld + c);
-      else add_slabs<V>(g, reinterpret_cast<const float*>(b.gate), b.gsplit, b.gplane, (size_t)t * b.gld + c);
-      const Vec<V> gb = ldv<V>(b.gbias + c);
+      if (!b.gate_act) add_slabs<V>(g, reinterpret_cast<const float*>(b.gate), b.gsplit, b.gplane, (size_t)t * b.gld + c);
+      const Vec<V> gb = NV == 1 ? gb1 : ldv<V>(b.gbias + c);
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         y[k].v[e] *= 1.f / (1.f + expf(-(g.v[e] + gb.v[e])));
@@ -173,13 +186,6 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
           ss += y[k].v[e] * y[k].v[e];
         }
     const float r = 1.f / sqrtf(block_sum(ss, red) / (float)W + b.eps);
-    int m = 0;
-    if constexpr (MODE == GN_PROMPT) {
-      if (prev) {
-        m = meta[t];
-        pos = positions[t];
-      }
-    }
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int c = (k * BT + threadIdx.x) * V;
@@ -187,7 +193,7 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
       if constexpr (MODE == GN_PROMPT) {
         if (prev && (m & META_TAIL)) stv<V>(prev + ((size_t)(m >> META_SLOT) * 2 + (pos & 1)) * W + c, xv[k]);
       }
-      const Vec<V> w = ldv<V>(b.norm_w + c);
+      const Vec<V> w = NV == 1 ? gain : ldv<V>(b.norm_w + c);
 #pragma unroll
       for (int e = 0; e < V; ++e) xv[k].v[e] += y[k].v[e] * r * w.v[e];
       stv<V>(x + row + c, xv[k]);

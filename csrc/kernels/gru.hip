@@ -13,15 +13,6 @@ namespace {
 
 struct GruCols { const void* p; int split; int64_t ld, plane; };      // split 0: activations, else fp32 slabs
 
-template <typename ACT, int V>
-__device__ __forceinline__ Vec<V> gru_ld(const GruCols& a, int64_t t, int c) {
-  const int64_t o = t * a.ld + c;
-  if (a.split == 0) return ldv<V>(reinterpret_cast<const ACT*>(a.p) + o);
-  Vec<V> y = zerov<V>();
-  add_slabs<V>(y, reinterpret_cast<const float*>(a.p), a.split, a.plane, (size_t)o);
-  return y;
-}
-
 // decay 1 - z and contribution z c of one token.  With t = exp(pre_z): 1 - z = 1 / (1 + t) and z = t / (1 + t), neither
 // the other's difference from 1, so that small ones keep their digits; sigmoid(min(u, 0)) is 1/2 where u >= 0
 template <typename ACT>
@@ -62,10 +53,16 @@ __global__ void __launch_bounds__(64) gru_step_kernel(GruCols z, GruCols u, GruC
                                                      ACT* __restrict__ out, int64_t ldo, float oscale) {
   const int b = blockIdx.x, c = (blockIdx.y * 64 + threadIdx.x) * V;
   if (c >= W) return;
+  // all at once; the state last, as it waits for its index (32 rows of 4096: 6.3 -> 4.9 us)
+  ColsIn<ACT, V> zi, ui, gi;
+  zi.ask(z.p, z.split, z.plane, b * z.ld + c);
+  ui.ask(u.p, u.split, u.plane, b * u.ld + c);
+  gi.ask(g.p, g.split, g.plane, b * g.ld + c);
+  const Vec<V> vz = ldv<V>(bz + c), vx = ldv<V>(bx + c);
   float* sp = state + (size_t)slots[b] * W + c;
   Vec<V> S = ctx_lens[b] > 1 ? ldv<V>(sp) : zerov<V>();
-  const Vec<V> zv = gru_ld<ACT, V>(z, b, c), uv = gru_ld<ACT, V>(u, b, c), gv = gru_ld<ACT, V>(g, b, c);
-  const Vec<V> vz = ldv<V>(bz + c), vx = ldv<V>(bx + c);
+  const Vec<V> zv = zi.get(z.p, z.split, z.plane, b * z.ld + c), uv = ui.get(u.p, u.split, u.plane, b * u.ld + c);
+  const Vec<V> gv = gi.get(g.p, g.split, g.plane, b * g.ld + c);
   Vec<V> o;
 #pragma unroll
   for (int e = 0; e < V; ++e) {

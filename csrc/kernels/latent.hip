@@ -16,6 +16,7 @@
 //   * latent_gather   the latents of whole sequences as dense rows, in token order and in the slot order
 //                     of the prefill attention's V^T: two products turn them into per-head keys and
 //                     values for long portions, where that costs fewer flops (attention.hip, EXP)
+#include "rows.h"
 #include "split_merge.h"
 
 namespace {
@@ -44,51 +45,35 @@ __global__ void __launch_bounds__(BT) latent_norm_kernel(const float* __restrict
                                                         const float* __restrict__ wq, const float* __restrict__ wc,
                                                         float eps, const int32_t* __restrict__ slots,
                                                         ACT* __restrict__ q_out, int ldq, ACT* __restrict__ cache, int RS) {
-  __shared__ float red[16];
+  __shared__ float red[16], red2[16];
   const int t = blockIdx.x, N = NQ + NC;
   const size_t plane = (size_t)T * N;
   const float* src = part + (size_t)t * N;
   const int slot = slots[t];
-  float x[NV][V], sq = 0.f, sc = 0.f;
+  float x[NV][V], gain[V], sq = 0.f, sc = 0.f;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int c = (k * BT + threadIdx.x) * V;
 #pragma unroll
     for (int e = 0; e < V; ++e) x[k][e] = 0.f;
     if (c >= N) continue;
-    if (split == 1) {
-      if constexpr (V == 4) {
-        const float4 f = *reinterpret_cast<const float4*>(src + c);
-        x[k][0] = f.x; x[k][1] = f.y; x[k][2] = f.z; x[k][3] = f.w;
-      } else {
-        x[k][0] = src[c];
-      }
-    } else for (int p0 = 0; p0 < split; p0 += 8) {       // eight slabs in flight (past the last: re-read, not added)
-      float y[8][V];
+    Slabs<V, NV == 1 ? 8 : 4> slabs;
+    slabs.ask(src, split, (int64_t)plane, c);
+    if constexpr (NV == 1) {          // asked for with the row
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const float* s = src + (size_t)min(p0 + u, split - 1) * plane + c;
-        if constexpr (V == 4) {
-          const float4 f = *reinterpret_cast<const float4*>(s);
-          y[u][0] = f.x; y[u][1] = f.y; y[u][2] = f.z; y[u][3] = f.w;
-        } else {
-          y[u][0] = *s;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (p0 + u < split)
-#pragma unroll
-          for (int e = 0; e < V; ++e) x[k][e] += y[u][e];
+      for (int e = 0; e < V; ++e) gain[e] = c < NQ ? wq[c + e] : wc[c - NQ + e];
     }
+    Vec<V> y = zerov<V>();
+    slabs.add(y, src, split, (int64_t)plane, c);
+#pragma unroll
+    for (int e = 0; e < V; ++e) x[k][e] = y.v[e];
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < V; ++e) ss += x[k][e] * x[k][e];
     if (c < NQ) sq += ss;
     else sc += ss;
   }
-  sq = block_sum(sq, red);
-  sc = block_sum(sc, red);
+  block_sum2(sq, sc, red, red2);
   const float rq = 1.f / sqrtf(sq / (float)NQ + eps), rc = 1.f / sqrtf(sc / (float)NC + eps);
   ACT* dst = cache + (size_t)slot * RS;
 #pragma unroll
@@ -100,7 +85,7 @@ __global__ void __launch_bounds__(BT) latent_norm_kernel(const float* __restrict
     const float r = isq ? rq : rc;
     float v[V];
 #pragma unroll
-    for (int e = 0; e < V; ++e) v[e] = x[k][e] * r * w[e];
+    for (int e = 0; e < V; ++e) v[e] = x[k][e] * r * (NV == 1 ? gain[e] : w[e]);
     st_vec<ACT, V>(isq ? q_out + (size_t)t * ldq + c : dst + (c - NQ), v);
   }
 }

@@ -25,10 +25,13 @@ __global__ void __launch_bounds__(1024) rmsnorm_kernel(void* __restrict__ out, f
   uint4* rr = reinterpret_cast<uint4*>(residual + (size_t)row * dim);
   float v[VPT][8];
   float ss = 0.f;
+  const uint4* wr = reinterpret_cast<const uint4*>(w);
+  uint4 gain = make_uint4(0, 0, 0, 0);       // one vector a thread: the weights with the row, not after its sum
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
     const int c = threadIdx.x + i * blockDim.x;
     if (c < nvec) {
+      if constexpr (VPT == 1) gain = wr[c];
       unpack8(xr[c], v[i]);
       if (add_residual) {
         float r[8];
@@ -46,7 +49,6 @@ __global__ void __launch_bounds__(1024) rmsnorm_kernel(void* __restrict__ out, f
   }
   ss = block_sum(ss, red);
   const float inv = rsqrtf(ss / (float)dim + eps);
-  const uint4* wr = reinterpret_cast<const uint4*>(w);
   if constexpr (!F8) {
     uint4* orow = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + (size_t)row * dim);
 #pragma unroll
@@ -54,7 +56,7 @@ __global__ void __launch_bounds__(1024) rmsnorm_kernel(void* __restrict__ out, f
       const int c = threadIdx.x + i * blockDim.x;
       if (c < nvec) {
         float g[8], o[8];
-        unpack8(wr[c], g);
+        unpack8(VPT == 1 ? gain : wr[c], g);
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[j] = v[i][j] * inv * g[j];
         orow[c] = pack8(o);
@@ -67,7 +69,7 @@ __global__ void __launch_bounds__(1024) rmsnorm_kernel(void* __restrict__ out, f
       const int c = threadIdx.x + i * blockDim.x;
       if (c < nvec) {
         float g[8];
-        unpack8(wr[c], g);
+        unpack8(VPT == 1 ? gain : wr[c], g);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           v[i][j] = bf2f(f2bf(v[i][j] * inv * g[j]));   // the bf16 value the unfused norm would store

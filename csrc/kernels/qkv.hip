@@ -34,11 +34,9 @@ struct QkvArgs {
 
 template <typename ACT, int V>
 __device__ __forceinline__ Vec<V> qkv_ld(const QkvArgs& a, int64_t t, int c) {
-  const int64_t o = t * a.ld + c;
-  if (a.split == 0) return ldv<V>(reinterpret_cast<const ACT*>(a.p) + o);
-  Vec<V> y = zerov<V>();
-  add_slabs<V>(y, reinterpret_cast<const float*>(a.p), a.split, a.plane, (size_t)o);
-  return y;
+  ColsIn<ACT, V> in;
+  in.ask(a.p, a.split, a.plane, t * a.ld + c);
+  return in.get(a.p, a.split, a.plane, t * a.ld + c);
 }
 
 __device__ __forceinline__ float round_act(float v, const uint16_t*) { return bf2f(f2bf(v)); }
@@ -62,7 +60,11 @@ __global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a) {
   const int nvec = C / V, allc = a.H * a.dim + (a.parts > 1 ? a.G * (a.dim + a.vdim) : 0);
   const float* wn = part == 0 ? a.qn : part == 1 ? a.kn : nullptr;
   const int rot = part == 2 ? 0 : a.rot;
-  Vec<V> x[NV];
+  // asked for with the row, and not where they are needed: the first vectors' weights, the first angles' frequencies, the slot
+  const int cslot = part ? a.cslots[t] : 0;
+  const float freq = tid < rot / 2 ? a.freq[tid] : 0.f;
+  Vec<V> x[NV], gain;
+  if (NV == 1 && wn && tid < nvec) gain = ldv<V>(wn + (a.per_head ? tid * V % hd : tid * V));
   if (!a.conv) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
@@ -80,12 +82,14 @@ __global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a) {
       for (int k = 0; k < NV; ++k) {
         const int c = min((k * BT + tid) * V, C - V);
         Vec<V> o[MAX_BACK], w[MAX_BACK + 1];
+        ColsIn<ACT, V> in;
+        in.ask(a.p, a.split, a.plane, t * a.ld + c0 + c);
 #pragma unroll
         for (int d = 0; d <= MAX_BACK; ++d) w[d] = ldv<V>(a.conv + (size_t)max(back - d, 0) * allc + c0 + c);
 #pragma unroll
         for (int d = 1; d <= MAX_BACK; ++d)
           o[d - 1] = d <= back && d <= pos ? ldv<V>(st + (size_t)((pos - d) % max(back, 1)) * allc + c) : zerov<V>();
-        const Vec<V> u = qkv_ld<ACT, V>(a, t, c0 + c);
+        const Vec<V> u = in.get(a.p, a.split, a.plane, t * a.ld + c0 + c);
 #pragma unroll
         for (int e = 0; e < V; ++e) {
           x[k].v[e] = u.v[e] * w[0].v[e];
@@ -116,7 +120,7 @@ __global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a) {
   }
   for (int i = tid; i < rot / 2; i += BT) {
     float sn, co;
-    sincosf((float)pos * a.freq[i], &sn, &co);
+    sincosf((float)pos * (i == tid ? freq : a.freq[i]), &sn, &co);
     cs[i] = make_float2(co, sn);
   }
   float r[NV];
@@ -161,7 +165,7 @@ __global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a) {
     for (int k = 0; k < NV; ++k) {
       const int c = (k * BT + tid) * V;
       if (c >= C) continue;
-      const Vec<V> w = ldv<V>(wn + (a.per_head ? c % hd : c));
+      const Vec<V> w = NV == 1 ? gain : ldv<V>(wn + (a.per_head ? c % hd : c));
 #pragma unroll
       for (int e = 0; e < V; ++e) x[k].v[e] *= r[k] * w.v[e];
     }
@@ -209,7 +213,7 @@ __global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a) {
     return;
   }
   ACT* cache = reinterpret_cast<ACT*>(part == 1 ? a.kc : a.vc);
-  const int slot = a.cslots[t];
+  const int slot = cslot;
   auto row = [&](int blk, int g, int off) { return (((size_t)blk * a.G + g) * CFC_KV_BS + off) * a.D; };
 #pragma unroll
   for (int k = 0; k < NV; ++k) {

@@ -318,7 +318,8 @@ __device__ __forceinline__ void step_conv(const LruArgs& a, int b0, int nb, int 
   const bool same = blockDim.x % nv == 0;              // a thread's vectors are of the same channels
   for (int i0 = threadIdx.x; i0 < items; i0 += IN * blockDim.x) {
     Vec<V> x[IN], o[IN][3], y[IN], bx[IN], w[IN][4];
-    int64_t at[IN];
+    ColsIn<ACT, V, 4> xin[IN];
+    int64_t at[IN], xo[IN];
     int ps[IN];
 #pragma unroll
     for (int j = 0; j < IN; ++j) {                     // past the last or in the pad: another's, not stored
@@ -326,7 +327,8 @@ __device__ __forceinline__ void step_conv(const LruArgs& a, int b0, int nb, int 
       const int c = blk * a.bs + min(k, a.bs - V);
       ps[j] = positions[b];
       at[j] = (int64_t)a.slots[b] * a.taps * a.W + c;
-      x[j] = lru_ld<ACT, V>(a.x, b, c);
+      xo[j] = b * a.x.ld + c;
+      xin[j].ask(a.x.p, a.x.split, a.x.plane, xo[j]);
       if (j && same) {
         bx[j] = bx[0];
         y[j] = y[0];
@@ -338,11 +340,14 @@ __device__ __forceinline__ void step_conv(const LruArgs& a, int b0, int nb, int 
 #pragma unroll
         for (int d = 0; d < 4; ++d) w[j][d] = ldv<V>(a.conv + (size_t)max(back - d, 0) * a.W + c);
       }
-#pragma unroll
-      for (int d = 1; d <= 3; ++d) o[j][d - 1] = ldv<V>(a.tail + at[j] + (size_t)(max(ps[j] - d, 0) % a.taps) * a.W);
     }
 #pragma unroll
+    for (int j = 0; j < IN; ++j)                       // last, as they wait for their indexes
+#pragma unroll
+      for (int d = 1; d <= 3; ++d) o[j][d - 1] = ldv<V>(a.tail + at[j] + (size_t)(max(ps[j] - d, 0) % a.taps) * a.W);
+#pragma unroll
     for (int j = 0; j < IN; ++j) {
+      x[j] = xin[j].get(a.x.p, a.x.split, a.x.plane, xo[j]);
       const int i = i0 + j * (int)blockDim.x, r = i / nv, k = (i - r * nv) * V, pos = ps[j];
       if (i >= items) break;
       if (k >= a.bs) {
@@ -390,7 +395,9 @@ __global__ void __launch_bounds__(64 * NW) rglru_step_kernel(LruArgs a, const in
   const bool on = col < nb && k0 < a.bs;
   const int c = blk * a.bs + min(k0, a.bs - 1);
   float* sp = a.state + (size_t)a.slots[b] * W + c;
-  Vec<4> S = zerov<4>(), y = zerov<4>(), br, bi, rate;
+  Vec<4> S = zerov<4>(), br, bi, rate, by;
+  constexpr int YN = 4 / V;
+  ColsIn<uint16_t, V, 4> yin[YN];
   auto get = [&](auto ld) {
     Vec<4> r;
     if constexpr (V == 4) {
@@ -401,16 +408,6 @@ __global__ void __launch_bounds__(64 * NW) rglru_step_kernel(LruArgs a, const in
     }
     return r;
   };
-  if (on) {
-    if (ctx_lens[b] > 1) S = get([&](int e, auto n) { return ldv<decltype(n)::value>(sp + e); });
-    y = get([&](int e, auto n) { return lru_ld<uint16_t, decltype(n)::value>(a.y, b, c + e); });
-    const Vec<4> by = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.by + c + e); });
-    br = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.br + c + e); });
-    bi = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.bi + c + e); });
-    rate = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.rate + c + e); });
-#pragma unroll
-    for (int e = 0; e < 4; ++e) y.v[e] += by.v[e];
-  }
   const uint16_t* p = reinterpret_cast<const uint16_t*>(a.wg) + ((size_t)blk * a.NP + min(n0, a.NP - 16) + col) * a.KP + 8 * kq;
   const size_t second = (size_t)a.blocks * a.NP * a.KP;
   const int KS = a.KP / 32;
@@ -424,6 +421,17 @@ __global__ void __launch_bounds__(64 * NW) rglru_step_kernel(LruArgs a, const in
     }
   };
   matrices(0);
+  // behind the matrices, which nothing waits for; the state last, as it waits for its index (5 rows: 9.0 -> 8.6 us)
+  auto y_at = [&](int e) { return (int64_t)b * a.y.ld + c + (V == 4 ? 0 : k0 + e < a.bs ? e : 0); };
+  if (on) {
+#pragma unroll
+    for (int e = 0; e < YN; ++e) yin[e].ask(a.y.p, a.y.split, a.y.plane, y_at(e));
+    by = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.by + c + e); });
+    br = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.br + c + e); });
+    bi = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.bi + c + e); });
+    rate = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.rate + c + e); });
+    if (ctx_lens[b] > 1) S = get([&](int e, auto n) { return ldv<decltype(n)::value>(sp + e); });
+  }
   step_conv<uint16_t, uint16_t, V>(a, b0, nb, blk, g0, g0 + 16 * NW, positions, ul, ldu);
   __syncthreads();
   if (n0 >= a.NP) return;
@@ -440,12 +448,19 @@ __global__ void __launch_bounds__(64 * NW) rglru_step_kernel(LruArgs a, const in
   }
   if (!on) return;
   Vec<4> o;
+  float y[4];
+#pragma unroll
+  for (int e = 0; e < YN; ++e) {
+    const Vec<V> v = yin[e].get(a.y.p, a.y.split, a.y.plane, y_at(e));
+#pragma unroll
+    for (int i = 0; i < V; ++i) y[e * V + i] = v.v[i];
+  }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     float ga, gb;
     lru_gates<uint16_t>(pr[e] + br.v[e], pi[e] + bi.v[e], bf2f(ul[col * ldu + min(k0 + e, a.bs - 1)]), rate.v[e], ga, gb);
     S.v[e] = ga * S.v[e] + gb;
-    o.v[e] = S.v[e] * gelu_tanh<uint16_t>(y.v[e]);
+    o.v[e] = S.v[e] * gelu_tanh<uint16_t>(y[e] + by.v[e]);
   }
   uint16_t* dst = out + (size_t)b * W + c;
   if constexpr (V == 4) {

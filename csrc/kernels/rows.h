@@ -51,26 +51,58 @@ __device__ __forceinline__ Vec<V> zerov() {
   return r;
 }
 
-// y += slabs of row offset `off`, eight in flight (past the last: re-read, not added)
-template <int V>
-__device__ __forceinline__ void add_slabs(Vec<V>& y, const float* p, int split, int64_t plane, size_t off) {
-  if (split == 1) {
-    const Vec<V> a = ldv<V>(p + off);
+// Sums of fp32 k-slice slabs in two steps: the first F slabs are asked for, and added, in their order, where the sum is
+// needed.  No load waits for another: a loop over the slabs made all that was asked for before it arrive first, and a row
+// that one workgroup works on pays a trip to memory, 0.7 us, for each such wait.
+template <int V, int F = 8>
+struct Slabs {
+  Vec<V> a[F];
+  __device__ __forceinline__ void ask(const float* p, int split, int64_t plane, size_t off) {
 #pragma unroll
-    for (int e = 0; e < V; ++e) y.v[e] += a.v[e];
-    return;
+    for (int u = 0; u < F; ++u) a[u] = u == 0 || u < split ? ldv<V>(p + u * plane + off) : zerov<V>();
   }
-  for (int p0 = 0; p0 < split; p0 += 8) {
-    Vec<V> a[8];
+  __device__ __forceinline__ void add(Vec<V>& y, const float* p, int split, int64_t plane, size_t off) const {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) a[u] = ldv<V>(p + (size_t)min(p0 + u, split - 1) * plane + off);
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (p0 + u < split)
+    for (int u = 0; u < F; ++u)
+      if (u < split)
 #pragma unroll
         for (int e = 0; e < V; ++e) y.v[e] += a[u].v[e];
+    for (int p0 = F; p0 < split; p0 += F) {          // past the last: re-read, not added
+      Vec<V> b[F];
+#pragma unroll
+      for (int u = 0; u < F; ++u) b[u] = ldv<V>(p + (size_t)min(p0 + u, split - 1) * plane + off);
+#pragma unroll
+      for (int u = 0; u < F; ++u)
+        if (p0 + u < split)
+#pragma unroll
+          for (int e = 0; e < V; ++e) y.v[e] += b[u].v[e];
+    }
   }
+};
+
+// y += slabs of row offset `off`
+template <int V>
+__device__ __forceinline__ void add_slabs(Vec<V>& y, const float* p, int split, int64_t plane, size_t off) {
+  Slabs<V> s;
+  s.ask(p, split, plane, off);
+  s.add(y, p, split, plane, off);
 }
+
+// V columns of a product that leaves activations (split 0) or fp32 slabs, in the same two steps.
+template <typename ACT, int V, int F = 8>
+struct ColsIn {
+  Slabs<V, F> s;
+  __device__ __forceinline__ void ask(const void* p, int split, int64_t plane, int64_t o) {
+    if (split == 0) s.a[0] = ldv<V>(reinterpret_cast<const ACT*>(p) + o);
+    else s.ask(reinterpret_cast<const float*>(p), split, plane, (size_t)o);
+  }
+  __device__ __forceinline__ Vec<V> get(const void* p, int split, int64_t plane, int64_t o) const {
+    if (split == 0) return s.a[0];
+    Vec<V> y = zerov<V>();
+    s.add(y, reinterpret_cast<const float*>(p), split, plane, (size_t)o);
+    return y;
+  }
+};
 
 }  // namespace
 

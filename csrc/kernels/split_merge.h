@@ -81,14 +81,23 @@ __global__ void __launch_bounds__(128) slice_merge_kernel(const float* __restric
   const float* ml = part_ml + row * P * 2;
   // every wave computes the weights (at most four slices per lane), the first stores them
   const int lane = threadIdx.x & 63;
+  // the first eight slices' columns, asked for before the weights are known (past the last: re-read, weight 0; 160 rows
+  // of a few slices: 5.7 -> 5.0 us)
+  float4 v[8];
+  auto ask = [&](int c, int p0) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(part_o + (row * P + min(p0 + u, P - 1)) * RS + c);
+  };
   float m[MERGE_MAXP / 64], l[MERGE_MAXP / 64], mx = -INFINITY;
 #pragma unroll
   for (int i = 0; i < MERGE_MAXP / 64; ++i) {
     const int p = lane + 64 * i;
     m[i] = p < P ? ml[2 * p] : -INFINITY;
     l[i] = p < P ? ml[2 * p + 1] : 0.f;
-    mx = fmaxf(mx, m[i]);
   }
+  if (threadIdx.x * 4 < RS) ask(threadIdx.x * 4, 0);
+#pragma unroll
+  for (int i = 0; i < MERGE_MAXP / 64; ++i) mx = fmaxf(mx, m[i]);
   mx = wave_max(mx);
   const float sk = sink ? sink[row % H] * 1.4426950408889634f : -INFINITY;
   mx = fmaxf(mx, sk);
@@ -109,10 +118,8 @@ __global__ void __launch_bounds__(128) slice_merge_kernel(const float* __restric
   __syncthreads();
   for (int c = threadIdx.x * 4; c < RS; c += 512) {
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int p0 = 0; p0 < P; p0 += 8) {          // eight slices in flight (past the last: re-read, weight 0)
-      float4 v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(part_o + (row * P + min(p0 + u, P - 1)) * RS + c);
+    for (int p0 = 0; p0 < P; p0 += 8) {          // eight slices in flight
+      if (p0 || c >= 512) ask(c, p0);
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const float e = p0 + u < P ? wt[p0 + u] : 0.f;
