@@ -178,9 +178,9 @@ __global__ void __launch_bounds__(256, F8 ? 2 : 1) paged_decode_kernel(
   // split into P near-equal ranges (balanced per sequence whatever its length -- no nearly empty
   // tail partitions, and P can stay small, so each workgroup streams a long run of KV)
   const int blk0 = part_blocks > 0 ? max(blk_lo, p * part_blocks)
-                                   : blk_lo + (int)(((int64_t)p * (nblk - blk_lo)) / P);
+                                   : blk_lo + share_of(nblk - blk_lo, p, P);
   const int blk1 = part_blocks > 0 ? min(nblk, p * part_blocks + part_blocks)
-                                   : blk_lo + (int)(((int64_t)(p + 1) * (nblk - blk_lo)) / P);
+                                   : blk_lo + share_of(nblk - blk_lo, p + 1, P);
 
   __shared__ float sm_o[4][D][17];
   __shared__ float sm_m[4][16], sm_l[4][16];

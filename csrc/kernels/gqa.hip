@@ -152,15 +152,11 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
   const int hk = item % a.G, s = item / a.G, pos = a.ctx_lens[s] - 1;
   const int32_t* bt = a.block_tables + (size_t)s * a.max_blocks;
   const KeyTiles kt = key_tiles<32>(a, pos, pos);
-  const int t0 = (int)((int64_t)kt.nt * blockIdx.y / a.P), t1 = (int)((int64_t)kt.nt * (blockIdx.y + 1) / a.P);
+  const int t0 = share_of(kt.nt, blockIdx.y, a.P), t1 = share_of(kt.nt, blockIdx.y + 1, a.P);
   const int r0 = 16 * rg, nr = min(16, R - r0);
   const size_t qrow = (size_t)s * a.H + hk * R + r0;
 
   u32x4_t qf[KS];
-#pragma unroll
-  for (int k = 0; k < KS; ++k)
-    qf[k] = *reinterpret_cast<const u32x4_t*>(q + (qrow + min(col, nr - 1)) * D + 32 * k + 8 * kq);
-
   char* vbuf = smem + w * 64 * D;
   const float* bias = SHAPED && a.bias ? a.bias + (size_t)(hk * R + r0 + min(col, nr - 1)) * a.nb : nullptr;
   const float far_bias = bias ? bias[a.nb - 1] : 0.f;
@@ -196,7 +192,10 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
   if (t < t1) {
     int row = rows_of(t);
     load(t, row);
-    row = rows_of(t + 4);
+#pragma unroll
+    for (int k = 0; k < KS; ++k)             // behind the first tile, which waits for indexes
+      qf[k] = *reinterpret_cast<const u32x4_t*>(q + (qrow + min(col, nr - 1)) * D + 32 * k + 8 * kq);
+    if (t + 4 < t1) row = rows_of(t + 4);
     for (; t < t1; t += 4) {
       wave_lds_fence();                      // the last tile's values have been read
 #pragma unroll
@@ -211,8 +210,10 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
 #pragma unroll
         for (int k = 0; k < KS; ++k) sc[g] = mfma16(kf[g][k], qf[k], sc[g]);
       }
-      load(t + 4, row);                      // past the slice: re-read, not used
-      row = rows_of(t + 8);
+      if (t + 4 < t1) {                      // a tile that no one uses was one in three or four of a short slice's loads
+        load(t + 4, row);
+        if (t + 8 < t1) row = rows_of(t + 8);
+      }
       const bool far = t < kt.nat;
       if constexpr (SHAPED) {
         const int k0 = far ? 32 * t : kt.lo + 32 * (t - kt.nat);
@@ -608,7 +609,7 @@ __global__ void __launch_bounds__(256) gqa_any_kernel(const ACT* __restrict__ q,
   int* rw = reinterpret_cast<int*>(sq + 4 * D + 256) + 64 * w;
   for (int c = lane; c < D; c += 64) myq[c] = ldf(q + grow * D + c);
   const KeyTiles kt = key_tiles<64>(a, pos, pos);
-  const int t0 = (int)((int64_t)kt.nt * blockIdx.y / a.P), t1 = (int)((int64_t)kt.nt * (blockIdx.y + 1) / a.P);
+  const int t0 = share_of(kt.nt, blockIdx.y, a.P), t1 = share_of(kt.nt, blockIdx.y + 1, a.P);
   float o[NC], m = -INFINITY, l = 0.f;
 #pragma unroll
   for (int j = 0; j < NC; ++j) o[j] = 0.f;

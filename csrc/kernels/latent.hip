@@ -493,8 +493,8 @@ __device__ __forceinline__ LatTile lat_tile(const LatArgs& a, int tile, int p, i
   r.pos_base = a.ctx_lens[s] - n;
   r.kend = r.pos_base + (min(r.m0 + rows_per_tile, r.rows) - 1) / a.H + 1;
   const int t0 = lat_low(a, r.pos_base + r.m0 / a.H + 1) / 64, nt = (r.kend + 63) / 64 - t0;
-  r.kt0 = t0 + (int)((int64_t)nt * p / a.P);
-  r.kt1 = t0 + (int)((int64_t)nt * (p + 1) / a.P);
+  r.kt0 = t0 + share_of(nt, p, a.P);
+  r.kt1 = t0 + share_of(nt, p + 1, a.P);
   r.bt = a.block_tables + (size_t)s * a.max_blocks;
   return r;
 }
@@ -558,15 +558,6 @@ __global__ void __launch_bounds__(512, 1) latent_attn_kernel(const uint16_t* __r
   const int limit = tl.pos_base + gm / a.H + 1;   // keys this row sees: low .. limit - 1
   const int low = lat_low(a, limit);
   u32x4_t qf[KS];
-  if (scorer) {
-    const uint16_t* qr = q + (size_t)(tl.q_row + gm) * RS + 8 * kq;
-#pragma unroll
-    for (int k = 0; k < KS; ++k)
-      qf[k] = *reinterpret_cast<const u32x4_t*>(qr + min(32 * k, RS - 32));
-#pragma unroll
-    for (int k = 0; k < KS; ++k) qf[k] &= 32 * k < RS ? ~0u : 0u;
-  }
-
   const int nb = (tl.kend + CFC_KV_BS - 1) / CFC_KV_BS;
   u32x4_t st[NL];
   int b0 = 0, b1 = 0;
@@ -710,22 +701,61 @@ __global__ void __launch_bounds__(512, 1) latent_attn_kernel(const uint16_t* __r
     }
   };
 
-  // tile t + 1 into LDS from the registers, the loads of t + 2 (past the last tile: re-read, not used), the
-  // block ids of t + 3
+  // tile t + 1 into LDS from the registers, the loads of t + 2, the block ids of t + 3 (none past the slice: a tile that no
+  // one used was a fifth of the bytes of a slice of four)
   auto advance = [&](int t, int buf) {
     if (t + 1 >= tl.kt1) return;
     lwrite(buf);
+    if (t + 2 >= tl.kt1) return;
     gload();
     ids(t + 3);
   };
 
   if (tl.kt0 < tl.kt1) {
     const int k0 = tl.kt0;
-    ids(k0);
+    // (24 sequences of 2800 keys, 32 heads, 10 slices, with the merge: 32.4 -> 29.6 us; the first tile is there after 6.4 of 18,
+    // was 8.1 of 20)
+    // the first tile's latents ahead of the queries, which come once, by way of the second tile's buffer: a row group's waves
+    // have the same (each its own copy: 128 KB through the CU's one path beside 64 of the first tile)
+    {
+      const int b = tl.bt[min(2 * k0 + (lane & 1), nb - 1)];          // both by one load
+      b0 = __builtin_amdgcn_readlane(b, 0);
+      b1 = __builtin_amdgcn_readlane(b, 1);
+    }
     gload();
+    constexpr bool SHARE = MR < 4;          // more rows: the registers are the output's
+    constexpr int NQ = SHARE ? (16 * MR * CH + 511) / 512 : 0;
+    u32x4_t qs[NQ ? NQ : 1];
+    if (!SHARE && scorer) {
+      const uint16_t* qr = q + (size_t)(tl.q_row + gm) * RS + 8 * kq;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) qf[k] = *reinterpret_cast<const u32x4_t*>(qr + min(32 * k, RS - 32));
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int e = min(tid + 512 * i, 16 * MR * CH - 1), row = e / CH, c = e % CH;
+      qs[i] = *reinterpret_cast<const u32x4_t*>(q + (size_t)(tl.q_row + min(tl.m0 + row, tl.rows - 1)) * RS + min(8 * c, RS - 8));
+    }
     ids(k0 + 1);
     advance(k0 - 1, 0);
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int e = tid + 512 * i, row = e / CH, c = e % CH;
+      qs[i] &= 8 * c < RS ? ~0u : 0u;
+      if (e < 16 * MR * CH)
+        *reinterpret_cast<u32x4_t*>(kbuf + 64 * R64 * 2 + row * (R64 * 2) + ((c ^ swz(row)) << 4)) = qs[i];
+    }
+    lds_barrier();
+    if (!SHARE && scorer) {
+#pragma unroll
+      for (int k = 0; k < KS; ++k) qf[k] &= 32 * k < RS ? ~0u : 0u;
+    }
+    if (SHARE && scorer) {
+      const int row = 16 * rg + col;
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        qf[k] = *reinterpret_cast<const u32x4_t*>(kbuf + 64 * R64 * 2 + row * (R64 * 2) + (((4 * k + kq) ^ swz(row)) << 4));
+    }
     scores(k0, 0);
     lds_barrier();
     softmax();
@@ -743,7 +773,7 @@ __global__ void __launch_bounds__(512, 1) latent_attn_kernel(const uint16_t* __r
     }
   }
   // row sums over the lane groups and the row group's waves
-  __syncthreads();
+  lds_barrier();
   if (scorer) {
     l = xor32_sum(xor16_sum(l));
     if (lane < 16) {
@@ -751,7 +781,7 @@ __global__ void __launch_bounds__(512, 1) latent_attn_kernel(const uint16_t* __r
       if (slot == 0) salpha[16 * rg + lane] = m;
     }
   }
-  __syncthreads();
+  lds_barrier();
 #pragma unroll
   for (int r = 0; r < MR; ++r) {
     const int mrow = tl.m0 + 16 * r + col;

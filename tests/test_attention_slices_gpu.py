@@ -1,0 +1,56 @@
+"""Decode attention in slices of no, one and few key tiles: a slice's start asks for its first tiles at once and reads none
+past its end.  Against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _tables(B, longest, g):
+    n = -(-longest // 32)
+    return torch.randperm(B * n, device=DEV, generator=g).int().view(B, n).contiguous(), B * n
+
+
+def _close(got, want, scale):
+    # bf16 weights and results (2^-9 each, of values that add up to `scale` at most); scores are fp32 sums
+    assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -9 * scale).all()), float((got.double() - want).abs().max())
+
+
+@pytest.mark.parametrize("H,RS,RV", [(3, 64, None), (16, 512, None), (32, 512, None), (64, 256, None), (20, 96, None), (32, 576, 512), (40, 192, 128)])
+@pytest.mark.parametrize("P", [1, 2, 3, 5, 16])
+@pytest.mark.parametrize("window", [0, 100])
+def test_latent_slices(H, RS, RV, P, window):
+    from copilot_for_consensus_amd.ops import latent
+    ctx = [1, 63, 64, 65, 127, 128, 129, 191, 193, 320, 385]
+    g = torch.Generator(device=DEV).manual_seed(H * P + RS)
+    bt, blocks = _tables(len(ctx), max(ctx), g)
+    cache = torch.randn(blocks, 32, RS, device=DEV, generator=g).bfloat16()
+    q = torch.randn(len(ctx), H, RS, device=DEV, generator=g).bfloat16()
+    out = latent.latent_attention(q, cache, bt, None, torch.tensor(ctx, dtype=torch.int32, device=DEV), RS ** -0.5, P=P, window=window, RV=RV)
+    for s, n in enumerate(ctx):
+        c = cache[bt[s].long()].reshape(-1, RS)[max(0, n - window) if window else 0:n].double()
+        p = torch.softmax(q[s].double() @ c.T * RS ** -0.5, -1)
+        v = c[:, :RV]
+        _close(out[s], p @ v, (p @ v.abs()).max())
+
+
+@pytest.mark.parametrize("H,G,D", [(8, 2, 128), (16, 1, 64), (40, 2, 128), (4, 4, 256)])
+@pytest.mark.parametrize("P", [1, 2, 3, 7])
+def test_grouped_slices(H, G, D, P):
+    """Waves of no, one, two and three 32-key tiles."""
+    from copilot_for_consensus_amd.ops import gqa
+    from copilot_for_consensus_amd.runtime.kv_cache import PagedHeads
+    ctx = [1, 31, 33, 64, 128, 129, 160, 257, 300, 390, 500]
+    g = torch.Generator(device=DEV).manual_seed(H * P + D)
+    bt, blocks = _tables(len(ctx), max(ctx), g)
+    rows = PagedHeads(blocks, G, D, 0, 0, DEV, torch.bfloat16)
+    for t in (rows.k, rows.v):
+        t.copy_(torch.randn(t.shape, device=DEV, generator=g))
+    a = gqa.Heads(H, G, D, D, D ** -0.5, gqa.Mask(0), 1e-6, None, None, False, None)
+    q = (torch.randn(len(ctx), H, D, device=DEV, generator=g) * a.q_scale).bfloat16()
+    out = gqa.attention(a, q, rows, bt, torch.tensor(ctx, dtype=torch.int32, device=DEV), P=P)
+    for s, n in enumerate(ctx):
+        kk, vv = (t[bt[s].long()].transpose(1, 2).reshape(-1, G, D)[:n].double().transpose(0, 1).contiguous() for t in (rows.k, rows.v))
+        p = torch.softmax((q[s].double().view(G, H // G, 1, D) * kk[:, None]).sum(-1) / gqa.LOG2E, -1)
+        _close(out[s].view(G, H // G, D), torch.matmul(p, vv), torch.matmul(p, vv.abs()).max())
