@@ -9,8 +9,11 @@
 //   * an LDS-DMA W ring (4-6 stages in flight per CU) stayed at ~4.1-4.5 TB/s however deep.
 // So here W never touches LDS:
 //
-//   * workgroup = BN/16 compute waves + 2 X-loader waves, tile = ALL M rows (BM = 64/128/256) x BN
-//     W rows (BN = 64..128, chosen per shape so ~256 workgroups run: one per CU);
+//   * workgroup = BN/16 compute waves + 2 X-loader waves, tile = ALL M rows (BM = 16/32/64/128/256) x BN
+//     W rows (BN = 64..128, chosen per shape so ~256 workgroups run: one per CU).  A batch of at most 16 or 32 rows
+//     takes a tile of no more: in 64 rows X was half of W's bytes again through the CU, its LDS writes and reads four
+//     times W's (us, 64-row tiles -> 16, of 5 rows: 4096 x 4096 9.4 -> 8.0, 6144 x 4096 11.7 -> 10.8, 28672 x 4096
+//     38.7 -> 36.8, 4096 x 14336 21.6 -> 20.9; -> 32, of 24 rows: 9.4 -> 8.2, 12.0 -> 11.2, 40.2 -> 38.6, 22.0 -> 21.5);
 //   * compute wave w owns 16 W rows and loads its B fragments straight from HBM into a D-stage
 //     register ring (D = 8 x 64-deep K stages = 16 KB per wave in flight, the GEMV's depth).  Its
 //     only vector-memory instructions are those loads, so hipcc's own counted vmcnt waits are
@@ -69,7 +72,7 @@ struct DgShape {
   static constexpr int XP = BM / 8 / LOADERS;         // 1-KB DMA pieces per loader wave per stage
   // X ring slots (64-128 KB); a loader keeps NSX - 2 stages in flight at its wait, and vmcnt
   // counts at most 63 of its pieces
-  static constexpr int NSX_BASE = MX ? 8 : (BM == 256 ? 4 : (BM == 128 ? 6 : 8));
+  static constexpr int NSX_BASE = MX ? 8 : (BM == 256 ? 4 : (BM == 128 ? 6 : 8));    // BM 16, 32: a ring of 16 is no faster
   static constexpr int NSX = (NSX_BASE - 2 <= 63 / XP ? NSX_BASE : 2 + 63 / XP);
 };
 
@@ -161,7 +164,7 @@ struct DgGroup {
 // whose starts the other one's stream covers; half the ring each, 96 VGPRs, 64 KB of LDS (us of 8 experts of 8192 x 2048:
 // 58.7 -> 55.5, 64 rows 59.7 -> 56.8; gate / up, one round of 128 stages: no difference, one workgroup kept)
 template <int BM, int EPI, int GRP>
-constexpr bool dg_twice() { return BM == 64 && GRP == 1 && EPI == DG_BF16; }
+constexpr bool dg_twice() { return BM <= 64 && GRP == 1 && EPI == DG_BF16; }
 
 template <int BM, int BN, int EPI, bool NTW, int ABL = 0, bool PACKED = true, int GRP = 0>
 __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES), (dg_twice<BM, EPI, GRP>() ? 5 : 1))
@@ -630,8 +633,8 @@ int dgemm_check(int M, int N, int K, int split, int epi, int bn, const float* pa
 
 }  // namespace
 
-// Which row tile (64 / 128 / 256) a batch of M rows runs with (M > 256 loops 256-row tiles over grid.y).
-CFC_API int cfc_dgemm_bm(int M) { return M <= 64 ? 64 : (M <= 128 ? 128 : 256); }
+// Which row tile (16 / 32 / 64 / 128 / 256; at least 64 of a row-major W) a batch of M rows runs with (M > 256 loops 256-row tiles over grid.y).
+CFC_API int cfc_dgemm_bm(int M) { return M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : M <= 128 ? 128 : 256; }
 
 // epi 0: fp32 split-K partials into part[split][M][N]; 1: bf16 into out (row stride ldo, split 1);
 // 2: SwiGLU over 8-row interleaved gate/up W -> bf16 [M, N/2] into out (split 1); 3: as 0 with
@@ -642,7 +645,9 @@ CFC_API int cfc_dgemm(const void* x, const void* w, int M, int N, int K, int spl
                       float* part, void* out, int ldo, hipStream_t stream) {
   if (const int e = dgemm_check(M, N, K, split, epi, bn, part, out, ldo)) return e;
   int rc;
-  switch (cfc_dgemm_bm(M)) {
+  switch (packed ? cfc_dgemm_bm(M) : std::max(64, cfc_dgemm_bm(M))) {
+    case 16: rc = dgemm_launch_pk<16, DG_NT, 0, true>(x, w, M, N, K, split, epi, bn, part, out, ldo, stream); break;
+    case 32: rc = dgemm_launch_pk<32, DG_NT, 0, true>(x, w, M, N, K, split, epi, bn, part, out, ldo, stream); break;
     case 64: rc = dgemm_launch<64>(x, w, M, N, K, split, epi, bn, packed, part, out, ldo, stream); break;
     case 128: rc = dgemm_launch<128>(x, w, M, N, K, split, epi, bn, packed, part, out, ldo, stream); break;
     default: rc = dgemm_launch<256>(x, w, M, N, K, split, epi, bn, packed, part, out, ldo, stream); break;
@@ -679,6 +684,8 @@ CFC_API int cfc_dgemm_glu(const void* x, const void* w, int M, int N, int K, int
   gp.limit = limit; gp.alpha = alpha; gp.beta = beta; gp.cubic = cubic;
   int rc;
   switch (cfc_dgemm_bm(M)) {
+    case 16: rc = dgemm_glu_bn<16>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
+    case 32: rc = dgemm_glu_bn<32>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
     case 64: rc = dgemm_glu_bn<64>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
     case 128: rc = dgemm_glu_bn<128>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
     default: rc = dgemm_glu_bn<256>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
@@ -710,7 +717,7 @@ int dgemm_group_bn(int glu, const void* x, const void* w, int M, int N, int K, i
 }
 }  // namespace
 
-// Products of rows sorted by expert with W[experts][N][K] (each packed for bn): M sorted rows in tiles of bm = 64 or
+// Products of rows sorted by expert with W[experts][N][K] (each packed for bn): M sorted rows in tiles of bm = 16, 32, 64 or
 // 128, rows / tile_expert as in DgGroup.  bf16 out of row stride ldo: [M][N], or (glu) the clamped GLU of 8-row
 // interleaved gate / up rows [M][N / 2]
 CFC_API int cfc_dgemm_group(int glu, const void* x, const void* w, int M, int N, int K, int bn, int bm, const int32_t* rows,
@@ -718,13 +725,18 @@ CFC_API int cfc_dgemm_group(int glu, const void* x, const void* w, int M, int N,
                             hipStream_t stream) {
   if (M == 0) return 0;
   if (const int e = dgemm_check(M, N, K, 1, glu ? DG_GLU : DG_BF16, bn, nullptr, out, ldo)) return e;
-  if (!tile_expert || (bm != 64 && bm != 128) || M % bm) return -1;
+  if (!tile_expert || (bm != 16 && bm != 32 && bm != 64 && bm != 128) || M % bm) return -1;
   DgGlu gp;
   gp.limit = limit; gp.alpha = alpha; gp.beta = beta;
   DgGroup g;
   g.rows = rows; g.tile_expert = tile_expert;
-  const int rc = bm == 64 ? dgemm_group_bn<64>(glu, x, w, M, N, K, bn, out, ldo, gp, g, stream)
-                          : dgemm_group_bn<128>(glu, x, w, M, N, K, bn, out, ldo, gp, g, stream);
+  int rc;
+  switch (bm) {
+    case 16: rc = dgemm_group_bn<16>(glu, x, w, M, N, K, bn, out, ldo, gp, g, stream); break;
+    case 32: rc = dgemm_group_bn<32>(glu, x, w, M, N, K, bn, out, ldo, gp, g, stream); break;
+    case 64: rc = dgemm_group_bn<64>(glu, x, w, M, N, K, bn, out, ldo, gp, g, stream); break;
+    default: rc = dgemm_group_bn<128>(glu, x, w, M, N, K, bn, out, ldo, gp, g, stream); break;
+  }
   return rc ? rc : CFC_CHECK_LAUNCH();
 }
 
@@ -753,6 +765,8 @@ CFC_API int cfc_dgemm_joint(const void* x, const void* w, int M, int N, int K, i
   g.in_of = in_of;
   int rc;
   switch (cfc_dgemm_bm(M)) {
+    case 16: rc = dgemm_joint_bn<16>(x, w, M, N, K, split, bn, part, g, stream); break;
+    case 32: rc = dgemm_joint_bn<32>(x, w, M, N, K, split, bn, part, g, stream); break;
     case 64: rc = dgemm_joint_bn<64>(x, w, M, N, K, split, bn, part, g, stream); break;
     case 128: rc = dgemm_joint_bn<128>(x, w, M, N, K, split, bn, part, g, stream); break;
     default: rc = dgemm_joint_bn<256>(x, w, M, N, K, split, bn, part, g, stream); break;
@@ -779,8 +793,14 @@ CFC_API int cfc_dgemm_stream(const void* x, const void* w, int M, int N, int K, 
 #define DG_STREAM(BM, BN)                                                                                       \
   dgemm_stream_kernel<BM, BN><<<(int)std::min<int64_t>(256, (int64_t)(N / BN) * (K / 64)), 64 * DgShape<BM, BN>::WAVES, 0, stream>>>((const uint16_t*)x, (const uint16_t*)w, M, \
                                                                               N, K, slabs, part, in_of)
-  if (bn == 64) DG_STREAM(64, 64);
-  else DG_STREAM(64, 128);
+  switch (cfc_dgemm_bm(M) * 1000 + bn) {
+    case 16064: DG_STREAM(16, 64); break;
+    case 16128: DG_STREAM(16, 128); break;
+    case 32064: DG_STREAM(32, 64); break;
+    case 32128: DG_STREAM(32, 128); break;
+    case 64064: DG_STREAM(64, 64); break;
+    default: DG_STREAM(64, 128); break;
+  }
 #undef DG_STREAM
   return CFC_CHECK_LAUNCH();
 }
@@ -839,7 +859,7 @@ double dgemm_us(int M, int N, int K, int bn, int split) {
   constexpr double CU_RATE = 25e3;         // W bytes/us one workgroup streams (6.4 TB/s over 256 CUs)
   constexpr double PART_RATE = 6e6;        // fp32 partial slab traffic
   constexpr double X_RATE = 90e3;          // per-CU L2 -> LDS rate of the X re-reads (ablation: X costs ~12 us of gate/up)
-  const int bm = M <= 64 ? 64 : M <= 128 ? 128 : 256;
+  const int bm = M <= 64 ? 64 : M <= 128 ? 128 : 256;   // the tiles of 16 and 32 rows keep the splits of 64: no other was faster
   const int64_t blocks = (int64_t)(N / bn) * ((M + bm - 1) / bm) * split;
   const double rounds = (double)((blocks + DG_CUS - 1) / DG_CUS);
   double t = rounds * ((double)bn * K * 2 / split / CU_RATE + (double)bm * K * 2 / split / X_RATE) + 1.5 * (rounds - 1.0);

@@ -1,0 +1,58 @@
+"""The decode GEMM's row tiles of 16 and 32 (dgemm.hip): the rows of a small batch are, bit for bit, those of a batch of 64
+whose first rows they are (the same products in the same order), and those are what 64-bit sums say."""
+import pytest
+import torch
+
+from copilot_for_consensus_amd.ops import kernels as K
+from copilot_for_consensus_amd.ops import moe
+
+ROWS = (1, 5, 15, 16, 17, 31, 32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N, Kd, bn, split", [(64, 64, 64, 1), (448, 192, 64, 3), (192, 1088, 96, 2), (448, 640, 112, 1), (384, 2176, 128, 4)])
+def test_rows_are_those_of_a_larger_batch(N, Kd, bn, split):
+    g = torch.Generator("cuda").manual_seed(N)
+    x = torch.randn(2, 64, Kd, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, Kd, device="cuda", generator=g) * 0.1).bfloat16()
+    pk = K.pack_dgemm_weight(w, bn=bn)
+    in_of = torch.randint(0, 2, (N // bn,), device="cuda", dtype=torch.int32, generator=g)
+
+    def products(M):
+        xs = x[:, :M].contiguous()
+        out = {"part": K.dgemm(xs[0], pk, "part", split, part=torch.full((split, M, N), float("nan"), device="cuda"))}
+        for epi, cols in (("bf16", N), ("swiglu", N // 2)):
+            out[epi] = K.dgemm(xs[0], pk, epi, out=torch.full((M, cols), float("nan"), device="cuda", dtype=torch.bfloat16))
+        out["glu"] = torch.full((M, N // 2), float("nan"), device="cuda", dtype=torch.bfloat16)
+        K.dgemm_glu(xs[0], pk, out["glu"], 7.0, 1.7, 1.0, 0.0)
+        if bn in (64, 128):
+            out["joint"] = K.dgemm_joint(xs, pk, in_of, torch.full((split, M, N), float("nan"), device="cuda"))
+        return out
+
+    want = products(64)
+    exact = x[0].double() @ w.double().t()
+    # sums of K products in fp32, in any order
+    assert ((want["part"].double().sum(0) - exact).abs() <= Kd * 2.0 ** -24 * (x[0].double().abs() @ w.double().abs().t())).all()
+    for M in ROWS:
+        for name, got in products(M).items():
+            assert torch.equal(got, want[name][..., :M, :]), (M, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T, E, tile", [(9, 8, 16), (12, 8, 16), (20, 8, 16), (24, 8, 32), (40, 8, 32), (17, 32, 16)])
+def test_experts_rows_do_not_depend_on_the_tile(monkeypatch, T, E, tile):
+    """Evenly spread choices, and all of them on one expert: several tiles of it."""
+    g = torch.Generator("cuda").manual_seed(T)
+    F, W, top = 128, 256, 2
+    gate, up, down = ((torch.randn(*s, device="cuda", generator=g) * 0.1).bfloat16() for s in ((E, F, W), (E, F, W), (E, W, F)))
+    weights = moe.ExpertWeights(gate, up, down)
+    x = torch.randn(T, W, device="cuda", generator=g).bfloat16()
+    ids = torch.stack([torch.randperm(E, device="cuda", generator=g)[:top] for _ in range(T)]).int()
+    assert weights.tile(ids.numel()) == tile and ids.numel() > moe.GEMV_PAIRS
+    for choice in (ids, torch.full_like(ids, 3)):
+        y, pos = moe.experts(x, weights, choice)
+        got = y[pos.long()].clone()
+        monkeypatch.setattr(moe.ExpertWeights, "tile", lambda self, pairs: 64)
+        y, pos = moe.experts(x, weights, choice)
+        assert torch.equal(got, y[pos.long()])
+        monkeypatch.undo()
