@@ -20,6 +20,7 @@ MI355X layout choices:
 from __future__ import annotations
 
 import dataclasses
+import functools
 import json
 import math
 import os
@@ -30,7 +31,7 @@ import torch
 import torch.nn.functional as F
 
 from ..ops import kernels as K
-from ..ops.reference import interleave_gate_up, rope_cos_sin
+from ..ops.reference import KV_BLOCK, interleave_gate_up, rope_cos_sin
 
 
 @dataclasses.dataclass(frozen=True)
@@ -411,6 +412,24 @@ def argmax_keys(local: torch.Tensor, offset: int) -> torch.Tensor:
     return ((ku - 2 ** 31) << 32) | (0xFFFFFFFF - (i.to(torch.int64) + offset))
 
 
+@functools.lru_cache(maxsize=4096)
+def kv_partitions(B: int, heads: int, kv_heads: int, blocks: int) -> int:
+    """Partitions of each of B sequences of up to ``blocks`` cache blocks in the paged decode attention, by what a launch
+    takes in us, fitted to 620 measured (B of 1 .. 128, 2 .. 172 blocks, 1 .. 64 partitions of 8 KV heads): 3.3, 4.2 and
+    0.045 per 32 rows and partition more for the merge, and what the busiest of 256 CUs, two workgroups each, reads: one
+    block per wave takes 3.1 to 3.8 where a CU has one workgroup, 4.5 to 5.5 where some have two, 5 per full round of 512.
+    A workgroup for every slot and a few more is a round more, and few keys are not worth a merge.  us of attention and
+    merge, 512 workgroups or more -> this: 24 of 5500 106 -> 92, 24 of 200 12.0 -> 8.9, 5 of 2600 19.7 -> 16.6, 3 of 1500
+    17.4 -> 13.7, 48 of 400 24.1 -> 20.7; on average over all measured sizes 10 % less, and 0.4 % more than the best P."""
+    def us(P):
+        full, rest = divmod(B * kv_heads * P, 512)
+        x = rest / 256
+        part = 0.0 if rest == 0 else 3.1 + 0.63 * x * x if rest <= 256 else 3.5 + x
+        return (3.3 + (4.2 + 0.045 * B * P * heads / 32 if P > 1 else 0.0)
+                + max(1.0, (blocks / P + 0.94) / 4) * (5.0 * full + part))
+    return min(range(1, max(1, min(64, blocks // 2)) + 1), key=us)
+
+
 class DecoderModel:
     """Stateless forward functions over :class:`DecoderWeights` + a paged KV cache."""
 
@@ -511,13 +530,13 @@ class DecoderModel:
                             dtype=dtype or torch.bfloat16)
 
     def decode_partitions(self, B: int, max_blocks: int) -> int:
-        """KV partitions per sequence of a B-row decode step: the smallest P giving >= CFC_DECODE_WGS
-        workgroups (default 512, two per CU).  Long KV runs per workgroup win: at B=128 P=1 streams
-        6.5 TB/s vs 5.0-5.4 for fixed 26-block partitions (scripts/bench_decode_attn.py,
-        profiles/decode_attn_partitions_r01.log)."""
-        target = int(os.environ.get("CFC_DECODE_WGS", "512"))
-        P = max(1, math.ceil(target / max(1, B * self.w.kv_heads)))
-        return min(P, max(1, max_blocks // 2))
+        """KV partitions per sequence of a B-row decode step over tables of ``max_blocks`` blocks
+        (:func:`kv_partitions`).  CFC_DECODE_WGS: the smallest P that gives so many workgroups instead."""
+        target = os.environ.get("CFC_DECODE_WGS")
+        if target:
+            return min(max(1, math.ceil(int(target) / max(1, B * self.w.kv_heads))), max(1, max_blocks // 2))
+        seen = min(max_blocks, self.window // KV_BLOCK + 2) if self.window else max_blocks
+        return kv_partitions(B, self.w.heads, self.w.kv_heads, seen)
 
     def decode_workspace(self, B: int, P: int) -> int:
         """fp32 elements of the split-KV partials of a B-row decode step over P partitions."""

@@ -54,3 +54,25 @@ def test_grouped_slices(H, G, D, P):
         kk, vv = (t[bt[s].long()].transpose(1, 2).reshape(-1, G, D)[:n].double().transpose(0, 1).contiguous() for t in (rows.k, rows.v))
         p = torch.softmax((q[s].double().view(G, H // G, 1, D) * kk[:, None]).sum(-1) / gqa.LOG2E, -1)
         _close(out[s].view(G, H // G, D), torch.matmul(p, vv), torch.matmul(p, vv.abs()).max())
+
+
+@pytest.mark.parametrize("P", [2, 7, 15, 16, 17, 33, 63, 64, 65, 128, 131])
+def test_merge_of_partitions(P):
+    """Whole and broken runs of sixteen and sixty-four partitions, most of them empty for the short sequences; rows that are
+    no whole workgroups of four, and a workspace and an output no more aligned than their elements."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    ctx = [1, 32, 33, 500, 65 * 32, 131 * 32]
+    heads, kv, D = 3, 3, 128
+    g = torch.Generator(device=DEV).manual_seed(P)
+    bt, blocks = _tables(len(ctx), max(ctx), g)
+    kc = torch.randn(blocks, kv, 32, D, device=DEV, generator=g).bfloat16()
+    vc = torch.randn(blocks, kv, D, 32, device=DEV, generator=g).bfloat16()
+    q = torch.randn(len(ctx), heads, D, device=DEV, generator=g).bfloat16()
+    lens = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    want = K.paged_decode_attention(q, kc, vc, bt, lens, D ** -0.5, part_blocks=-1)
+    n = len(ctx) * heads * P * (D + 2)
+    ws = torch.full((n + 1,), float("nan"), device=DEV)[1:]
+    out = torch.full((q.numel() + 1,), float("nan"), device=DEV, dtype=torch.bfloat16)[1:].view_as(q)
+    got = K.paged_decode_attention(q, kc, vc, bt, lens, D ** -0.5, part_blocks=-P, workspace=ws, out=out)
+    # weights of a partition are rounded to bf16 from another maximum (2^-9 each, of values up to 4.5), results once more
+    assert bool(((got.double() - want.double()).abs() <= 2.0 ** -8 * want.double().abs() + 2.0 ** -8).all())
