@@ -101,8 +101,9 @@ struct DepthArgs {
 };
 
 // one workgroup of BT threads per row; a thread holds NV vectors of V channels, NV * V * BT >= W
+// (DN_RSTD, a prompt's rows: two workgroups of 1024 a CU)
 template <typename ACT, int V, int NV, int MODE, int BT>
-__global__ void __launch_bounds__(BT) depth_norm_kernel(DepthArgs a, ACT* __restrict__ h1, ACT* __restrict__ h2) {
+__global__ void __launch_bounds__(BT, MODE == DN_RSTD ? 8 : 1) depth_norm_kernel(DepthArgs a, ACT* __restrict__ h1, ACT* __restrict__ h2) {
   __shared__ float red[16];
   const int b = blockIdx.x, t = a.rows ? a.rows[b] : b;
   const size_t row = (size_t)t * a.W, plane = (size_t)a.T * a.W;
@@ -150,7 +151,7 @@ __global__ void __launch_bounds__(BT) depth_norm_kernel(DepthArgs a, ACT* __rest
       Vec<V> pre, bias, hist[4];
       float wj[4];
       const float an = a.dwa[a.n];
-      Slabs<V> slabs;
+      Slabs<V, ONE ? 8 : 4> slabs;       // many rows: fewer registers, more rows a CU
       slabs.ask(a.part, a.split, (int64_t)plane, row + c);
       if (a.pre) pre = ldv<V>(a.pre + row + c);
       if (a.bias) bias = ldv<V>(a.bias + c);
