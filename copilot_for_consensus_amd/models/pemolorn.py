@@ -451,7 +451,7 @@ class PemolornModel:
     def _mixer(self, i, h, io: _Pass) -> N.Branch:
         lw = self.w.layers[i]
         decode, hs = io.plan is None, h[None]
-        c = lw["in"].joint(hs) if decode else [lw["in"].act(j, hs) for j in range(len(lw["in"].sizes))]
+        c = lw["in"].joint(hs) if decode else lw["in"].prompt(hs)
         b = N.Branch(lw["norm1b"], self.cfg.norm_eps)
         s = None
         if "gru" in lw:

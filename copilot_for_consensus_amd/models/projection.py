@@ -147,8 +147,8 @@ class Projection:
 
 class JointProjection:
     """Several matrices of one width read by one layer, each multiplying one of a few inputs [inputs, T, K]: one
-    packed matrix (every part padded with zero rows to whole tiles).  A decode step runs them all in one launch; a
-    prompt's rows take each part on its own."""
+    packed matrix (every part padded with zero rows to whole tiles).  A decode step runs them all in one launch, and so
+    does a prompt of up to 128 rows; more rows take runs of parts in one launch where that is faster."""
 
     def __init__(self, parts: list[tuple[torch.Tensor, int]]):
         """parts: (W [N, K], index of its input)."""
@@ -156,7 +156,7 @@ class JointProjection:
         self.inputs = [i for _, i in parts]
         self.K = parts[0][0].shape[1]
         w0 = parts[0][0]
-        self.packed = None
+        self.packed, self.runs = None, {}
         pad, bn = (lambda n: n), 64
         if Projection.packs(w0, 64, self.K):
             total = {b: sum(-(-n // b) * b for n in self.sizes) for b in (64, 128)}
@@ -190,6 +190,48 @@ class JointProjection:
     def slabs(self, j: int, acts: torch.Tensor) -> Cols:
         """Part j's columns in fp32 (a tensor of its own)."""
         return Cols(self.parts[j].slabs(acts[self.inputs[j]], own=True), 0, self.sizes[j])
+
+    def prompt(self, acts: torch.Tensor, slabs: tuple[int, ...] = ()) -> list[Cols]:
+        """Every part's columns of a prompt's rows, as activations, or (the parts named in ``slabs``) in fp32.
+
+        Up to 128 rows, where a product is a stream of W: one product and one sum of its slabs, in place of a product and
+        a sum for every part.  More rows: runs of parts side by side as one product, whose tiles fill rounds of the chip that
+        each part's alone leave part empty (joint_plan).  us, apart -> in one: five inputs' products of 4096 x 4096 134 ->
+        40 (130 rows), 158 -> 133 (862); 22528 columns in three parts of one input 106 -> 73 (420), 365 -> 334 (2569)."""
+        M, n = acts.shape[1], len(self.sizes)
+        if self.packed is None or not acts.is_contiguous() or n == 1:
+            return [self.slabs(j, acts) if j in slabs else self.act(j, acts) for j in range(n)]
+        if M <= 128:
+            c = self.joint(acts)
+            y = K.splitk_reduce(c[0].t)
+            return [c[j] if j in slabs else Cols(y, self.offsets[j], self.sizes[j]) for j in range(n)]
+        out: list = [None] * n
+        for first, last, run, in_of in self._runs(slabs):
+            at = self.offsets[first]
+            widths = tuple(self.parts[j].N for j in range(first, last))
+            plan = K.joint_plan(M, widths, self.K, in_of is None) if last - first > 1 else 0
+            if plan:
+                y = run.act(acts[self.inputs[first]]) if in_of is None else K.mgemm_joint(acts, run.packed, in_of, plan)
+                out[first:last] = [Cols(y, self.offsets[j] - at, self.sizes[j]) for j in range(first, last)]
+        return [c if c is not None else self.slabs(j, acts) if j in slabs else self.act(j, acts) for j, c in enumerate(out)]
+
+    def _runs(self, slabs: tuple[int, ...]) -> list[tuple]:
+        """(first part, one past the last, their columns as one projection, input per 128 of them or None: all the same) of
+        the runs of neighbours that leave activations."""
+        if slabs not in self.runs:
+            ends, runs, j = self.offsets[1:] + [self.N], [], 0
+            while j < len(self.sizes):
+                first = j
+                while j < len(self.sizes) and j not in slabs:
+                    j += 1
+                one = len(set(self.inputs[first:j])) == 1
+                if j - first > 1 and (one or self.packed.bn == 128):
+                    o, e, bn = self.offsets[first], ends[j - 1], self.packed.bn
+                    run = Projection.of_packed(K.PackedWeight(self.packed.data[o * self.K:e * self.K], e - o, self.K, bn))
+                    runs.append((first, j, run, None if one else self.in_of[o // bn:e // bn].contiguous()))
+                j = max(j, first + 1)
+            self.runs[slabs] = runs
+        return self.runs[slabs]
 
     def joint(self, acts: torch.Tensor) -> list[Cols]:
         """Every part's columns in fp32, of one product (a tensor of its own)."""

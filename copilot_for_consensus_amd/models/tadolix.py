@@ -464,7 +464,7 @@ class TadolixModel:
         """fp32 slabs [split, T, W] of layer i's mixer."""
         lw, m = self.w.layers[i], self.cfg.specs[i].mixer
         hs = h[None]
-        c = lw["in"].joint(hs) if io.plan is None else [lw["in"].act(j, hs) for j in range(len(lw["in"].sizes))]
+        c = lw["in"].joint(hs) if io.plan is None else lw["in"].prompt(hs)
         if "lru" in lw:
             return self._sum(lw["o"].slabs(self._lru(lw["lru"], run, c[0], io)))
         a, n = lw["heads"], lw["gru"].width

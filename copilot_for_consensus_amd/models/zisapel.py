@@ -479,23 +479,21 @@ class ZisapelModel:
             sh, part = self._shift(i, kv), lw["in"]
             acts = self._acts(sh, T, bufs)
             G.shift_mix(x, sh, plan["meta"], positions, acts)
-            gate = part.act(0, acts)
+            gate, *c = part.prompt(acts, (5,) if isinstance(s.mixer, WkvSpec) else (2,))
             if isinstance(s.mixer, WkvSpec):
                 o = torch.empty(T, lw["H"] * s.mixer.dim, dtype=dt, device=dev)
-                R.prefill(lw["wkv"], *(part.act(j, acts) for j in (1, 2, 3, 4)), part.slabs(5, acts), plan["states"], cu_q,
-                          ctx_lens, plan["chunks"], plan["chunk_cu"], kv.recur[i], o)
+                R.prefill(lw["wkv"], *c, plan["states"], cu_q, ctx_lens, plan["chunks"], plan["chunk_cu"], kv.recur[i], o)
             else:
                 rows = self._rows(i)
                 tiles = plan[f"attn_{lw['H']}_{rows}_{s.mixer.window}"]
                 keys = self._visible(s.mixer, plan["max_ctx"])
-                o = self._attend(i, part.act(1, acts), part.slabs(2, acts), part.act(3, acts), positions, slots, ctx_lens,
-                                 block_tables, kv, dict(cu_q=cu_q, tiles=(tiles[0], tiles[1]), rows=rows,
+                o = self._attend(i, *c, positions, slots, ctx_lens, block_tables, kv, dict(cu_q=cu_q, tiles=(tiles[0], tiles[1]), rows=rows,
                                                         P=L.partitions(tiles.shape[1], keys)), plan)
             b = G.Branch(gate, lw["rg1_b"], lw["norm1"], self.cfg.norm_eps, y=self._sum(lw["o"].slabs(o)))
             G.gated_norm(x, b, dt, h if s.mlp is not None else None, kv.prev[i], plan["meta"], positions)
             if s.mlp is not None:
                 ff, hs = lw["ff_in"], h[None]
-                G.gated_norm(x, self._feed(i, h, ff.act(0, hs), ff.slabs(1, hs) if len(ff.sizes) > 1 else None), dt)
+                G.gated_norm(x, self._feed(i, h, *ff.prompt(hs, (1,))), dt)
         return G.final_norm(x, self.w.final_norm, self.cfg.norm_eps, dt, None if last_idx is None else last_idx.to(torch.int32))
 
     def forward_decode(self, ids, positions, slots, ctx_lens, block_tables, kv, attn_workspace=None, part_blocks=-1,

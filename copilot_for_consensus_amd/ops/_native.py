@@ -11,7 +11,7 @@ import ctypes
 from pathlib import Path
 import os
 import threading
-from ctypes import c_float, c_int, c_int64, c_uint32, c_void_p
+from ctypes import c_double, c_float, c_int, c_int64, c_uint32, c_void_p
 
 from .._build import KERNELS_LIB, RUNTIME_LIB
 
@@ -119,6 +119,9 @@ _KERNEL_SIGS = {
     "cfc_pgemm_ppp_probe": [P, P, P, I, I, I, I, I, I, I, P],
     "cfc_pgemm_glu": [P, P, P, I, I, I, I, I, F, F, F, F, P],
     "cfc_prompt_plan": [I, I, I, I, P],
+    "cfc_prompt_us": [I, I, I, I],
+    "cfc_joint_plan": [I, I, I, P, P],
+    "cfc_mgemm_joint": [P, P, P, I, I, I, I, I, P, P],
     "cfc_dgemm_stream": [P, P, I, I, I, I, P, P, P],
     "cfc_dgemm_slab_plan": [I, I, I, I, P],
     "cfc_dgemm_config": [I, I, I, I, I, P],
@@ -177,7 +180,7 @@ _RUNTIME_SIGS = {
 
 _RESTYPES = {
     "cfc_bpe_create": c_void_p, "cfc_wp_create": c_void_p, "cfc_blockpool_create": c_void_p,
-    "cfc_mbox_split": c_int64,
+    "cfc_mbox_split": c_int64, "cfc_prompt_us": c_double,
 }
 
 

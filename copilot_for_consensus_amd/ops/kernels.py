@@ -845,6 +845,33 @@ def mgemm(x: torch.Tensor, w: "PackedWeight", epi: str, bm: int, split: int = 1,
     return out
 
 
+@functools.lru_cache(maxsize=4096)
+def joint_plan(M: int, sizes: tuple[int, ...], Kd: int, one_input: bool) -> int:
+    """How M prompt rows take products of ``sizes`` columns that lie side by side in one packed matrix: 0, each on its own;
+    -1, as one product (of one input); else the rows per workgroup of :func:`mgemm_joint`.  By the kernels' fitted times."""
+    lib, N = kernels(), sum(sizes)
+    apart = sum(lib.cfc_prompt_us(M, n, Kd, 0) for n in sizes)
+    if M * N * 2 >= 2 ** 31:           # columns of it are read with 32-bit offsets
+        return 0
+    if one_input:
+        return -1 if lib.cfc_prompt_us(M, N, Kd, 0) < 0.985 * apart else 0
+    bm, us = ctypes.c_int(), ctypes.c_double()
+    check(lib.cfc_joint_plan(M, N, Kd, ctypes.addressof(bm), ctypes.addressof(us)), "cfc_joint_plan")
+    return bm.value if bm.value and us.value < apart else 0
+
+
+def mgemm_joint(x: torch.Tensor, w: "PackedWeight", in_of: torch.Tensor, bm: int) -> torch.Tensor:
+    """bf16 [M, N] of x [inputs, M, K], W columns 128 t .. 128 t + 127 multiplying input in_of[t] (W packed for 128)."""
+    M, Kd = x.shape[1:]
+    if x.dtype != torch.bfloat16 or not x.is_contiguous() or Kd != w.K or w.bn != 128 or in_of.numel() != w.N // 128:
+        raise ValueError(f"mgemm_joint: x {tuple(x.shape)} {x.dtype} w [{w.N}, {w.K}] in {w.bn}, {in_of.numel()} tiles")
+    _req(in_of, torch.int32, "in_of")
+    out = torch.empty(M, w.N, dtype=torch.bfloat16, device=x.device)
+    check(kernels().cfc_mgemm_joint(x.data_ptr(), w.data.data_ptr(), out.data_ptr(), M, w.N, Kd, w.N, bm, in_of.data_ptr(),
+                                    _stream(x)), "cfc_mgemm_joint")
+    return out
+
+
 def prompt_gemm(x: torch.Tensor, w: "PackedWeight", epi: str, plan: tuple[int, int, int], out: torch.Tensor | None = None,
                 reduce=None, glu: tuple = (0.0, 1.0, 0.0, 0.0)) -> torch.Tensor:
     """A product by :func:`prompt_plan`.  ``epi``: "bf16", "swiglu", "relu2", "glu" as :func:`mgemm`'s, ``reduce(slabs, out)``

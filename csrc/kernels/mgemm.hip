@@ -63,7 +63,7 @@ template <int MT, int EPI>
 __global__ void __launch_bounds__(512, 1)
     mgemm_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, float* __restrict__ part,
                  uint16_t* __restrict__ out, int M, int N, int K, int ldo, int tiles_m, int tiles_n, int split, int wnw,
-                 PgGlu gp) {
+                 PgGlu gp, const int32_t* __restrict__ in_of) {
   using S = MgShape<MT>;
   constexpr int P = S::P, R = S::R;
   __shared__ __attribute__((aligned(16))) char smem[R * S::STAGE];
@@ -74,6 +74,8 @@ __global__ void __launch_bounds__(512, 1)
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   const int tile = id % (tiles_m * tiles_n), ks = id / (tiles_m * tiles_n);
   const int m0 = tile % tiles_m * S::BM, n0 = tile / tiles_m * MG_BN;
+  // several inputs [inputs][M][K]: columns n0 .. n0 + 127 multiply input in_of[n0 / 128]
+  if (in_of) X += (size_t)__builtin_amdgcn_readfirstlane(in_of[tile / tiles_m]) * M * K;
   const int nks = K / MG_BK;
   const int kb = (int)((long)ks * nks / split), nst = (int)((long)(ks + 1) * nks / split) - kb;
 
@@ -190,12 +192,12 @@ __global__ void __launch_bounds__(512, 1)
 
 template <int EPI>
 int mgemm_launch(const void* x, const void* w, void* out, int M, int N, int K, int ldo, int bm, int split, int wnw,
-                 const PgGlu& gp, hipStream_t stream) {
+                 const PgGlu& gp, hipStream_t stream, const int32_t* in_of = nullptr) {
   const int tm = (M + bm - 1) / bm, tn = (N + MG_BN - 1) / MG_BN;
 #define MG_CASE(MT)                                                                                                 \
   case 32 * MT:                                                                                                     \
     mgemm_kernel<MT, EPI><<<tm * tn * split, 512, 0, stream>>>((const uint16_t*)x, (const uint16_t*)w, (float*)out, \
-                                                               (uint16_t*)out, M, N, K, ldo, tm, tn, split, wnw, gp); \
+                                                               (uint16_t*)out, M, N, K, ldo, tm, tn, split, wnw, gp, in_of); \
     break;
   switch (bm) {
     MG_CASE(4)
@@ -251,15 +253,37 @@ enum { MG_ACT = 0, MG_SLABS = 1, MG_WHOLE = 2 };
 // mostly added up in the same order; 2 more for the launch that adds an activation's slabs up, 3 more (`alone`) for slices
 // of 8 stages or fewer, over before their ring is full: 1507 rows of 512 x 1024 in 4 slices 17.9, whole 12.3; 339 of
 // 1536 x 4096 in 8 22.2, in 4 19.4.  Beyond 3 rounds of workgroups nothing was measured to be faster than pgemm.
-double mgemm_best(int M, int N, int K, int kind, bool split_ok, bool alone, int& bm, int& split) {
+double mgemm_best(int M, int N, int K, int kind, bool split_ok, bool alone, int& bm, int& split, int rounds = 3) {
   double best = 1e30;
   for (int b = 128; b <= 256; b += 32) {
-    if ((int64_t)((M + b - 1) / b) * ((N + MG_BN - 1) / MG_BN) > 3 * MG_CUS) continue;
+    if ((int64_t)((M + b - 1) / b) * ((N + MG_BN - 1) / MG_BN) > rounds * MG_CUS) continue;
     for (int s = 1; s <= (split_ok ? 8 : 1) && s * 64 <= K; s *= 2) {
       const double t = mgemm_us(M, N, K, b, s, kind != MG_ACT) + (s > 1 && kind == MG_ACT ? 2.0 : 0.0) +
                        (s > 1 && alone && K <= 512 * s ? 3.0 : 0.0);
       if (t < best) best = t, bm = b, split = s;
     }
+  }
+  return best;
+}
+
+// cfc_prompt_plan's choice and its us
+double prompt_best(int M, int N, int K, int kind, int* plan) {
+  plan[0] = plan[1] = plan[2] = 0;
+  const int64_t weights = (int64_t)N * K;
+  int bm = 0, split = 0;
+  if (M <= 128 || N < 64 || K < 64 || (int64_t)M * K * 2 >= (1ll << 32) || weights * 2 >= (1ll << 32))
+    return ppp_us(M, N, K, kind != MG_ACT);
+  double all = mgemm_best(M, N, K, kind, kind != MG_WHOLE, true, bm, split);
+  if (weights <= 1 << 23 && M <= (weights > 1 << 22 ? 256 : 640)) return all;       // the decode GEMM, within 10 %
+  double best = M < 256 ? 1e29 : 0.97 * ppp_us(M, N, K, kind != MG_ACT);
+  const int tn = (N + 255) / 256, tm = (M + 255) / 256;
+  if ((int64_t)tm * tn >= MG_PGEMM_TILES) all = std::max(all, mgemm_x_us(M, N, K, split));
+  if (all < best) best = all, plan[1] = bm, plan[2] = split;
+  const int rounds = (int)((int64_t)tm * tn / MG_CUS), head = rounds ? (int)((int64_t)MG_CUS * rounds / tn) * 256 : 0;
+  if (head > 0 && head < M && K >= 128) {
+    const double rest = mgemm_best(M - head, N, K, kind, kind == MG_ACT, false, bm, split);
+    const double both = ppp_us(head, N, K, kind != MG_ACT) + rest;
+    if (both < best) best = both, plan[0] = head, plan[1] = bm, plan[2] = split;
   }
   return best;
 }
@@ -276,22 +300,24 @@ double mgemm_best(int M, int N, int K, int kind, bool split_ok, bool alone, int&
 //     nor where X would be brought into every L2 for a few columns each (mgemm_x_us): 1024 x 4096 up to 7000 rows;
 //   * the rows beyond pgemm's last whole round here: 4096 x 14336 of 4500 rows 512 -> 370, 4096 x 4096 152 -> 124.
 CFC_API int cfc_prompt_plan(int M, int N, int K, int kind, int* plan) {
-  plan[0] = plan[1] = plan[2] = 0;
-  const int64_t weights = (int64_t)N * K;
-  if (M <= 128 || N < 64 || K < 64 || (int64_t)M * K * 2 >= (1ll << 32) || weights * 2 >= (1ll << 32) ||
-      (weights <= 1 << 23 && M <= (weights > 1 << 22 ? 256 : 640)))
-    return 0;
-  int bm = 0, split = 0;
-  double best = M < 256 ? 1e29 : 0.97 * ppp_us(M, N, K, kind != MG_ACT);
-  double all = mgemm_best(M, N, K, kind, kind != MG_WHOLE, true, bm, split);
-  const int tn = (N + 255) / 256, tm = (M + 255) / 256;
-  if ((int64_t)tm * tn >= MG_PGEMM_TILES) all = std::max(all, mgemm_x_us(M, N, K, split));
-  if (all < best) best = all, plan[1] = bm, plan[2] = split;
-  const int rounds = (int)((int64_t)tm * tn / MG_CUS), head = rounds ? (int)((int64_t)MG_CUS * rounds / tn) * 256 : 0;
-  if (head > 0 && head < M && K >= 128) {
-    const double rest = mgemm_best(M - head, N, K, kind, kind == MG_ACT, false, bm, split);
-    if (ppp_us(head, N, K, kind != MG_ACT) + rest < best) plan[0] = head, plan[1] = bm, plan[2] = split;
-  }
+  prompt_best(M, N, K, kind, plan);
+  return 0;
+}
+
+// us of a product by its plan
+CFC_API double cfc_prompt_us(int M, int N, int K, int kind) {
+  int plan[3];
+  return M < 1 || N < 1 || K < 1 ? 0.0 : prompt_best(M, N, K, kind, plan);
+}
+
+// Rows per workgroup of cfc_mgemm_joint and its us; 0 where it does not fit or takes more than six rounds of workgroups
+// (five products of 4096 x 4096: 2300 rows 400 -> 360, 2569 rows 404 -> 427).
+CFC_API int cfc_joint_plan(int M, int N, int K, int* bm, double* us) {
+  int split = 0;
+  *bm = 0;
+  *us = 1e30;
+  if (M > 128 && N >= 128 && K >= 64 && (int64_t)M * K * 2 < (1ll << 32) && (int64_t)N * K * 2 < (1ll << 32))
+    *us = mgemm_best(M, N, K, MG_ACT, false, false, *bm, split, 6);
   return 0;
 }
 
@@ -314,4 +340,15 @@ CFC_API int cfc_mgemm(const void* x, const void* w, void* out, int M, int N, int
     case PG_RELU2: return mgemm_launch<PG_RELU2>(x, w, out, M, N, K, ldo, bm, split, wnw, gp, stream);
     default: return (int)hipErrorInvalidValue;
   }
+}
+
+// Activations [M][N] (row stride ldo) of x [inputs][M][K], columns 128 t .. of W (packed for bn = 128) multiplying input
+// in_of[t]: several products of a layer in one launch.
+CFC_API int cfc_mgemm_joint(const void* x, const void* w, void* out, int M, int N, int K, int ldo, int bm, const int32_t* in_of,
+                            hipStream_t stream) {
+  if (M < 1 || N < MG_BN || N % MG_BN || K < 64 || K % 64 || !in_of || (uint64_t)M * K * 2 >= (1ull << 32) ||
+      (uint64_t)N * K * 2 >= (1ull << 32) || ldo % 4 || ldo < N || ((uintptr_t)out & 7) ||
+      (int64_t)((M + 127) / 128) * (N / MG_BN) > (1 << 30))
+    return (int)hipErrorInvalidValue;
+  return mgemm_launch<PG_BF16>(x, w, out, M, N, K, ldo, bm, 1, MG_BN / 16, PgGlu{}, stream, in_of);
 }
