@@ -862,7 +862,7 @@ class DecoderModel:
         x = K.embedding(w.embed, ids)
         B = ids.shape[0]
         if (self.fused_decode and x.is_cuda and (B <= DGEMM_MAX_ROWS or self.w.packed_only)
-                and not (B <= K.GEMV_MAX_M and (self.decode_gemv or self.decode_qgemv))):
+                and not (B <= K.GEMV_MAX_M and (self.decode_gemv and not self._small_dgemm(B) or self.decode_qgemv))):
             return self._forward_decode_fused(x, positions, slots, ctx_lens, block_tables, kv, attn_workspace,
                                               part_blocks)
         if self.decode_gemm in ("splitk", "dgemm") and x.is_cuda and self.w.tp_size == 1:
@@ -889,6 +889,15 @@ class DecoderModel:
         if x32 is not None:
             return self._tp_norm(x32, residual, w.final_norm)
         return K.rmsnorm(x, w.final_norm, cfg.rms_eps, residual=residual)
+
+    def _small_dgemm(self, B: int) -> bool:
+        """Whether 2 .. GEMV_MAX_M rows run on the decode GEMM, which reads the packed copies faster than the GEMV in its
+        tile of 16 rows (us of 2 / 4 rows: 28672 x 4096 39.1 / 40.7 -> 37.3, 4096 x 14336 22.4 / 22.1 -> 20.8 / 19.7,
+        6144 x 4096 11.7 / 12.2 -> 10.5, 4096 x 4096 8.8 / 9.2 -> 8.0; one row: 37.4 / 21.8 / 10.8 / 7.9 against 37.4 /
+        20.7 / 10.5 / 8.0).  Matrices of 2^24 weights and more: smaller ones stay in the caches and were not measured."""
+        w = self.w
+        return (1 < B <= K.GEMV_MAX_M and self.decode_gemv and w.packed_only and self.fused_decode and not self.gemv_norm_fused and not self.decode_qgemv
+                and "CFC_DECODE_GEMV" not in os.environ and w.packed[0]["gate_up"].N * w.packed[0]["gate_up"].K >= 1 << 24)
 
     def _rope_attention(self, i, qkv, positions, slots, ctx_lens, block_tables, kv, attn_workspace, part_blocks):
         """RoPE + K/V cache write + paged decode attention of layer ``i`` from the qkv projection output
@@ -1141,11 +1150,12 @@ class DecoderModel:
                 and K.qgemv_fits(hidden.shape[0], hidden.shape[1])):
             local = K.qgemv(hidden, self.w.q_lm_head)
         elif (self.decode_gemv and hidden.is_cuda and hidden.shape[0] <= K.GEMV_MAX_M
+                and not (self.w.packed_lm_head is not None and self._small_dgemm(hidden.shape[0]))
                 and hidden.is_contiguous() and head.shape[0] % 2 == 0 and head.shape[1] % 8 == 0):
             # (the GEMV takes row pairs and 16-byte K slices: odd vocabularies, e.g. 32001-token
             # fine-tunes, stay on the library GEMM)
             local = K.gemv(hidden, self.w.lm_head)   # 262 MB weight stream: 4.6 -> ~6 TB/s at B=1
-        elif (self.fused_decode and hidden.is_cuda and hidden.shape[0] > K.GEMV_MAX_M
+        elif (self.fused_decode and hidden.is_cuda and (hidden.shape[0] > K.GEMV_MAX_M or self._small_dgemm(hidden.shape[0]))
                 and hidden.shape[0] <= DGEMM_MAX_ROWS and K.dgemm_ok(hidden, head)):
             # the 262 MB (Mistral) / 1 GB (Llama-3) vocab stream
             ph = self.w.packed_lm_head

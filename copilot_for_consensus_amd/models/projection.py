@@ -1,8 +1,9 @@
 """One weight matrix and the products a model takes with it, on the kernel that fits the row count.
 
-The selection is DecoderModel's: at most K.GEMV_MAX_M rows on the packed GEMV, up to 128 on the decode GEMM,
-thousands on the prefill GEMM's 256 x 256 tiles, what lies between on the GEMM for a few hundred rows
-(K.prompt_plan), all four reading one fragment-packed bf16 copy.  Shapes those kernels do not take (N or K not a multiple of 64) and 32-bit weights use
+Up to 128 rows run on the decode GEMM, thousands on the prefill GEMM's 256 x 256 tiles, what lies between on the GEMM
+for a few hundred rows (K.prompt_plan), all three reading one fragment-packed bf16 copy.  (One to four rows, too: with its
+tile of 16 rows the decode GEMM takes 29 us where the packed GEMV takes 32 to 38, 20608 x 4096, 4.8 where it takes 5.2 to
+8.2, 4096 x 1536, and the same at worst; and it gates and clamps in its epilogue.)  Shapes those kernels do not take (N or K not a multiple of 64) and 32-bit weights use
 the library product.  CPU tensors: torch.
 """
 from __future__ import annotations
@@ -58,8 +59,6 @@ class Projection:
     def _kernel(self, x, kind: str = "act") -> str:
         if self.packed is None or not x.is_contiguous():
             return "lib"
-        if x.shape[0] <= K.GEMV_MAX_M:
-            return "gemv"
         if K.prompt_plan(x.shape[0], self.N, self.K, kind):
             return "mgemm"
         return "pgemm" if self._prefill(x.shape[0]) else "dgemm"
@@ -72,8 +71,6 @@ class Projection:
         k = self._kernel(x)
         if k == "lib":
             return F.linear(x, self.rowmajor())
-        if k == "gemv":
-            return K.splitk_reduce(K.gemv_part(x, self.packed))
         if k == "mgemm":
             return self._prompt(x, "bf16", reduce=K.splitk_reduce)
         if k == "pgemm":
@@ -86,14 +83,11 @@ class Projection:
         their ``own``."""
         k = self._kernel(x, "slabs")
         M, out = x.shape[0], None
-        if k in ("gemv", "dgemm", "mgemm"):
-            split = K.gemv_packed_config(self.N, self.K, self.packed.bn // 16, M)[0] if k == "gemv" else \
-                K.dgemm_slab_plan(M, self.N, self.K, self.packed.bn)[0] if k == "dgemm" else \
+        if k in ("dgemm", "mgemm"):
+            split = K.dgemm_slab_plan(M, self.N, self.K, self.packed.bn)[0] if k == "dgemm" else \
                 K.prompt_plan(M, self.N, self.K, "slabs")[2]
             if own:
                 out = torch.empty(split, M, self.N, dtype=torch.float32, device=x.device)
-        if k == "gemv":
-            return K.gemv_part(x, self.packed, split, out=out)
         if k == "mgemm":
             return self._prompt(x, "f32", "slabs", out=out)
         if k == "pgemm":
@@ -133,8 +127,6 @@ class Projection:
     def f32(self, x: torch.Tensor) -> torch.Tensor:
         """[M, N] fp32, a tensor of its own."""
         k = self._kernel(x, "whole")
-        if k == "gemv":
-            return K.gemv(x, self.packed, "f32")
         if k in ("mgemm", "dgemm"):
             out = torch.empty(1, x.shape[0], self.N, dtype=torch.float32, device=x.device)
             if k == "mgemm":
@@ -240,12 +232,7 @@ class JointProjection:
             x = [F.linear(acts[i].float(), p.rowmajor().float()) for p, i in zip(self.parts, self.inputs)]
             out = torch.cat(x, 1)[None]            # no padding: the parts lie side by side
         else:
-            gemv = M <= K.GEMV_MAX_M
-            split = K.gemv_packed_config(self.N, self.K, self.packed.bn // 16, M)[0] if gemv else \
-                K.dgemm_slab_plan(M, self.N, self.K, self.packed.bn)[0]
+            split = K.dgemm_slab_plan(M, self.N, self.K, self.packed.bn)[0]
             out = torch.empty(split, M, self.N, dtype=torch.float32, device=acts.device)
-            if gemv:
-                K.gemv_part(acts, self.packed, split, out=out, in_of=self.in_of)
-            else:
-                K.dgemm_slabs(acts, self.packed, out, self.in_of)
+            K.dgemm_slabs(acts, self.packed, out, self.in_of)
         return [Cols(out, o, n) for o, n in zip(self.offsets, self.sizes)]
