@@ -410,8 +410,8 @@ __global__ void __launch_bounds__(512, 2)
 
 // ---- y = x W^T + b for a 384-wide x and W of 32 N32 rows (the attention's projections), the same way: rows in registers
 // as B operands, W in column groups through a ring of three stages.  No accumulators to hold beside them, so two
-// workgroups share a CU and one's waits are the other's matrix time.  65 k rows x 1152 in 67 us, 256 x 256 tiles of
-// both operands in LDS took 112.
+// workgroups share a CU and one's waits are the other's matrix time.  65 k rows x 1152 in 78 us, 256 x 256 tiles of
+// both operands in LDS took 112; more than 32 k rows now take the kernel after this one.
 constexpr int EP_RING = 3, EP_AHEAD = 8;
 
 __global__ void __launch_bounds__(256, 2)
@@ -482,6 +482,132 @@ __global__ void __launch_bounds__(256, 2)
     before = here;
     here = here == lds0 + (EP_RING - 1) * EN_STAGE ? lds0 : here + EN_STAGE;
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // the stream runs past its end
+}
+
+// The same for more rows than one workgroup of 128 a CU: above, every fragment of W that a wave reads from LDS feeds one
+// MFMA, and with two waves a SIMD those reads take all of the LDS's 128 bytes a cycle.  Here a wave holds 64 rows, two MFMAs a
+// fragment, one wave a SIMD (260 registers); what it has to wait for is asked for a group ahead: fragments and bias of the
+// next group in the last third of this one, after a barrier in its middle that says that the next group is there and the last
+// one read; the last group's rows leave while this one is multiplied, two groups at a time by way of the LDS, so that eight
+// lanes store a whole line of a row.  The same sums.  us in a forward of 49266 / 65484 rows: workgroups of 128 rows 73 / 78,
+// this with 32-byte pieces of rows stored 63 / 69, with whole lines 62.5 / 62.8; without any stores 45 / 55.
+constexpr int EW_ROWS = 256, EW_AHEAD = 4, EW_RING = EW_AHEAD + 1, EW_FR = 8, EW_MEET = 12, EW_GROUPS = 3 * EN_T;
+
+__global__ void __launch_bounds__(256, 1)
+    enc_proj_wide_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ W, const uint16_t* __restrict__ bias,
+                         uint16_t* __restrict__ out, int M) {
+  constexpr int groups = EW_GROUPS;
+  __shared__ __attribute__((aligned(16))) char smem[EW_RING * EN_STAGE];
+  __shared__ __attribute__((aligned(16))) float bias_s[32 * groups];
+  __shared__ __attribute__((aligned(16))) char turn[4][64 * 128];      // two groups of a wave's rows, on their way out
+  const int lane = threadIdx.x & 63, hi = lane >> 5, r32 = lane & 31;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row0 = blockIdx.x * EW_ROWS + w * 64 + r32;
+  const uint32_t v_n = (lane >> 3) * EN_H * 2 + (((lane & 7) ^ (lane >> 4)) << 4);     // of even pieces
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(en_lds_t*)smem);
+  auto issue = [&](int n, int slot) {       // rows 32 n .. of W; past the end, of no use
+    const char* src = reinterpret_cast<const char*>(W) + (size_t)min(n, groups - 1) * (32 * EN_H * 2);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      const int p = 6 * w + i;
+      en_glds16(i & 1 ? v_n ^ 64 : v_n, src + (p & 3) * (8 * EN_H * 2) + (p >> 2) * 128, lds0 + slot * EN_STAGE + p * 1024);
+    }
+  };
+#pragma unroll
+  for (int n = 0; n < EW_AHEAD; ++n) issue(n, n);
+  for (int i = threadIdx.x; i < 32 * groups; i += 256) bias_s[i] = bf2f(bias[i]);
+  bf16x8_t xf[2][EN_S];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const uint16_t* xr = x + (size_t)min(row0 + 32 * t, M - 1) * EN_H + 8 * hi;
+#pragma unroll
+    for (int s = 0; s < EN_S; ++s) xf[t][s] = *reinterpret_cast<const bf16x8_t*>(xr + 16 * s);
+  }
+  uint32_t go[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) go[s] = r32 * 128 + (((2 * s + hi) ^ ((r32 >> 1) & 7)) << 4);
+  // stores to rows past the last are issued and dropped: the waits below count them
+  const int first = blockIdx.x * EW_ROWS;
+  const uintptr_t ob = (uintptr_t)(out + (size_t)first * 32 * groups);
+  const __amdgpu_buffer_rsrc_t os = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(((uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(ob >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)ob)),
+      (short)0, min(EW_ROWS, M - first) * 64 * groups, 0x00020000);
+  // eight lanes a row: whole lines, in place of 32-byte pieces of them
+  const int o = (w * 64 + (lane >> 3)) * 64 * groups + 16 * (lane & 7);
+  char* const turn_in = turn[w] + r32 * 128;
+  const char* const turn_out = turn[w] + (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) << 4);
+  struct At { uint32_t a[4]; };
+  auto at_slot = [&](int slot) {
+    At r;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) { r.a[s] = lds0 + slot * EN_STAGE + go[s]; asm volatile("" : "+v"(r.a[s])); }
+    return r;
+  };
+  auto frag = [&](const At& b, int i) {
+    typedef const __attribute__((address_space(3))) bf16x8_t* lds_frag_t;
+    return *reinterpret_cast<lds_frag_t>(b.a[i & 3] + (uint32_t)((i >> 2) * 4096));
+  };
+  // the first groups, the rows and the bias are there, in every wave
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  At cur = at_slot(0);
+  bf16x8_t fr[EW_FR];
+#pragma unroll
+  for (int i = 0; i < EW_FR; ++i) fr[i] = frag(cur, i);
+  f32x16_t start;                          // a group's bias, what both row tiles' sums start from
+  auto biases = [&](int n) {
+    const float* b = bias_s + 32 * n + 4 * hi;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float4 v = *reinterpret_cast<const float4*>(b + 8 * i);
+      start[4 * i] = v.x; start[4 * i + 1] = v.y; start[4 * i + 2] = v.z; start[4 * i + 3] = v.w;
+    }
+  };
+  biases(0);
+  int slot = 0;
+  // chunk 4 (n & 1) + 2 s + hi of rows 32 t + r32; chunk c of row r at c ^ (r & 7)
+  auto turn_chunk = [&](const f32x16_t& a, int t, int s, int n) {
+    *reinterpret_cast<u32x4_t*>(turn_in + t * 32 * 128 + (((4 * (n & 1) + 2 * s + hi) ^ (r32 & 7)) << 4)) = __builtin_bit_cast(u32x4_t, frag_of(a, s));
+  };
+  auto leave = [&](int k, int n) {          // rows 8 k .. 8 k + 7 of groups n - 1 and n
+    __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4_t*>(turn_out + k * 1024), os, o + k * 8 * 64 * groups, 64 * (n - 1), 0);
+  };
+  auto group = [&](int n, f32x16_t (&acc)[2], f32x16_t (&last)[2]) {
+    At next = cur;
+    const int fill = slot == 0 ? EW_RING - 1 : slot - 1;
+    slot = slot + 1 == EW_RING ? 0 : slot + 1;
+#pragma unroll
+    for (int i = 0; i < EN_S; ++i) {
+      if (i == EW_MEET) {
+        // group n + 1, asked for three groups ago, is there; every wave is past group n - 1, whose place takes n + 4
+        // (younger than its pieces: two groups', and the eight stores of every second group; the first four groups came
+        // before the loop)
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(6 * (EW_AHEAD - 2) + 8) : "memory");
+        issue(n + EW_AHEAD, fill);
+        next = at_slot(slot);
+      }
+      acc[0] = mfma32(fr[i % EW_FR], xf[0][i], i ? acc[0] : start);
+      acc[1] = mfma32(fr[i % EW_FR], xf[1][i], i ? acc[1] : start);
+      fr[i % EW_FR] = i + EW_FR < EN_S ? frag(cur, i + EW_FR) : frag(next, i + EW_FR - EN_S);
+      if (n > 0 && i >= 2 && i < 10 && i % 2 == 0) turn_chunk(last[(i - 2) / 4], (i - 2) / 4, (i - 2) / 2 % 2, n - 1);
+      if (n > 0 && n % 2 == 0 && i >= 14 && i < 22) leave(i - 14, n - 1);
+      if (i == EN_S - 4) biases(min(n + 1, groups - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    cur = next;
+  };
+  static_assert(EN_S % EW_FR == 0 && EN_S - EW_FR >= EW_MEET && groups % 2 == 0 && groups > EW_AHEAD);
+  f32x16_t a[2], b[2];
+  for (int n = 0; n < groups; n += 2) {
+    group(n, a, b);
+    group(n + 1, b, a);
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) turn_chunk(b[t], t, s, groups - 1);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) leave(k, groups - 1);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // the stream runs past its end
 }
 
@@ -1093,7 +1219,10 @@ CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* 
     // few rows: a sublayer's last product waits in y for the next tiles' norm, which puts the layer's states in x, those
     // between its sublayers in att (the attention's output is used up by then)
     if (kind == 2)
-      enc_proj_kernel<<<blocks, 256, 0, stream>>>(xp, p[0], p[1], qp, T, 3 * EN_T);
+      if (T > 256 * EN_ROWS)          // more than a workgroup of 128 rows a CU
+        enc_proj_wide_kernel<<<(T + EW_ROWS - 1) / EW_ROWS, 256, 0, stream>>>(xp, p[0], p[1], qp, T);
+      else
+        enc_proj_kernel<<<blocks, 256, 0, stream>>>(xp, p[0], p[1], qp, T, 3 * EN_T);
     else if (l == 0)
       enc_tile_kernel<false, false><<<gq, 256, 0, stream>>>(xp, EncNorm{}, p[0], p[1], qp, T, 3 * EN_H);
     else

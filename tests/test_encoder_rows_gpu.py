@@ -167,3 +167,27 @@ def test_texts_laid_out_for_the_encoder(lens):
     for bad in ([0, 5, 3], [0, len(ids) + 1], [1, 2]):
         with pytest.raises(ValueError):
             m.encode_packed(ids, bad)
+
+
+@pytest.mark.parametrize("rows", [32769, 32768 + 65, 33024 + 33, 65536])
+def test_projections_of_more_rows_than_a_workgroup_a_cu(rows):
+    """Workgroups of 256 rows: a last one of one row, of one wave, of a wave and one row, none.  The same sums as those of
+    128 rows: the same texts in two batches of fewer rows, bit for bit."""
+    import dataclasses
+    from copilot_for_consensus_amd.models.encoder import get_encoder_config
+    from copilot_for_consensus_amd.ops import kernels as K
+    m = _model(dataclasses.replace(get_encoder_config("minilm-l6"), layers=2), seed=rows)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    lens = [256] * (rows // 256) + ([rows % 256] if rows % 256 else [])
+
+    def states(lens, ids):
+        pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).to(DEV)
+        cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).to(torch.int32)
+        tiles = tuple(torch.tensor(t, dtype=torch.int32, device=DEV) for t in K.prefill_tiles(cu.tolist(), K.ENCODER_TILE_ROWS))
+        return m.forward_packed(ids, pos, cu.to(DEV), max(lens), tiles=tiles)
+
+    ids = torch.randint(0, m.cfg.vocab_size, (rows,), device=DEV, dtype=torch.int32, generator=g)
+    half = len(lens) // 2
+    cut = sum(lens[:half])
+    assert 10753 <= cut <= 32768 and 10753 <= rows - cut <= 32768
+    assert torch.equal(states(lens, ids), torch.cat([states(lens[:half], ids[:cut]), states(lens[half:], ids[cut:])]))
