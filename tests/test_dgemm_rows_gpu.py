@@ -56,3 +56,15 @@ def test_experts_rows_do_not_depend_on_the_tile(monkeypatch, T, E, tile):
         y, pos = moe.experts(x, weights, choice)
         assert torch.equal(got, y[pos.long()])
         monkeypatch.undo()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T, top, E", [(256, 4, 5), (1023, 1, 3), (1025, 1, 3), (1024, 4, 7), (1025, 4, 32), (2731, 3, 1), (5000, 2, 1024)])
+def test_rows_of_pairs_about_a_step(T, top, E):
+    """One step of 1024 pairs, a few more, whole and broken steps of 4096; choices without an expert among them."""
+    import numpy as np
+
+    from copilot_for_consensus_amd.ops.reference import moe_rows
+    ids = torch.randint(0, E + 2, (T, top), generator=torch.Generator().manual_seed(T), dtype=torch.int32)
+    for got, want in zip(moe.sort_rows(ids.cuda(), E, 32), moe_rows(ids, E, 32)):
+        assert np.array_equal(got.cpu().numpy(), want)
