@@ -9,11 +9,12 @@
 //   * an LDS-DMA W ring (4-6 stages in flight per CU) stayed at ~4.1-4.5 TB/s however deep.
 // So here W never touches LDS:
 //
-//   * workgroup = BN/16 compute waves + 2 X-loader waves, tile = ALL M rows (BM = 16/32/64/128/256) x BN
+//   * workgroup = BN/16 compute waves + 2 X-loader waves, tile = ALL M rows (BM = 16/32/64/96/128/256) x BN
 //     W rows (BN = 64..128, chosen per shape so ~256 workgroups run: one per CU).  A batch of at most 16 or 32 rows
 //     takes a tile of no more: in 64 rows X was half of W's bytes again through the CU, its LDS writes and reads four
 //     times W's (us, 64-row tiles -> 16, of 5 rows: 4096 x 4096 9.4 -> 8.0, 6144 x 4096 11.7 -> 10.8, 28672 x 4096
-//     38.7 -> 36.8, 4096 x 14336 21.6 -> 20.9; -> 32, of 24 rows: 9.4 -> 8.2, 12.0 -> 11.2, 40.2 -> 38.6, 22.0 -> 21.5);
+//     38.7 -> 36.8, 4096 x 14336 21.6 -> 20.9; -> 32, of 24 rows: 9.4 -> 8.2, 12.0 -> 11.2, 40.2 -> 38.6, 22.0 -> 21.5).  65 .. 96 rows in 128 paid a third more of
+//     X's traffic (two steps of four 7B layers, 81 rows 1093 -> 1040 us, 71 rows 1165 -> 1112);
 //   * compute wave w owns 16 W rows and loads its B fragments straight from HBM into a D-stage
 //     register ring (D = 8 x 64-deep K stages = 16 KB per wave in flight, the GEMV's depth).  Its
 //     only vector-memory instructions are those loads, so hipcc's own counted vmcnt waits are
@@ -633,8 +634,8 @@ int dgemm_check(int M, int N, int K, int split, int epi, int bn, const float* pa
 
 }  // namespace
 
-// Which row tile (16 / 32 / 64 / 128 / 256; at least 64 of a row-major W) a batch of M rows runs with (M > 256 loops 256-row tiles over grid.y).
-CFC_API int cfc_dgemm_bm(int M) { return M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : M <= 128 ? 128 : 256; }
+// Which row tile (16 / 32 / 64 / 96 / 128 / 256; 64, 128 or 256 of a row-major W) a batch of M rows runs with (M > 256 loops 256-row tiles over grid.y).
+CFC_API int cfc_dgemm_bm(int M) { return M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : M <= 96 ? 96 : M <= 128 ? 128 : 256; }
 
 // epi 0: fp32 split-K partials into part[split][M][N]; 1: bf16 into out (row stride ldo, split 1);
 // 2: SwiGLU over 8-row interleaved gate/up W -> bf16 [M, N/2] into out (split 1); 3: as 0 with
@@ -645,9 +646,11 @@ CFC_API int cfc_dgemm(const void* x, const void* w, int M, int N, int K, int spl
                       float* part, void* out, int ldo, hipStream_t stream) {
   if (const int e = dgemm_check(M, N, K, split, epi, bn, part, out, ldo)) return e;
   int rc;
-  switch (packed ? cfc_dgemm_bm(M) : std::max(64, cfc_dgemm_bm(M))) {
+  const int bm = cfc_dgemm_bm(M);
+  switch (packed ? bm : bm == 96 ? 128 : std::max(64, bm)) {
     case 16: rc = dgemm_launch_pk<16, DG_NT, 0, true>(x, w, M, N, K, split, epi, bn, part, out, ldo, stream); break;
     case 32: rc = dgemm_launch_pk<32, DG_NT, 0, true>(x, w, M, N, K, split, epi, bn, part, out, ldo, stream); break;
+    case 96: rc = dgemm_launch_pk<96, DG_NT, 0, true>(x, w, M, N, K, split, epi, bn, part, out, ldo, stream); break;
     case 64: rc = dgemm_launch<64>(x, w, M, N, K, split, epi, bn, packed, part, out, ldo, stream); break;
     case 128: rc = dgemm_launch<128>(x, w, M, N, K, split, epi, bn, packed, part, out, ldo, stream); break;
     default: rc = dgemm_launch<256>(x, w, M, N, K, split, epi, bn, packed, part, out, ldo, stream); break;
@@ -686,6 +689,7 @@ CFC_API int cfc_dgemm_glu(const void* x, const void* w, int M, int N, int K, int
   switch (cfc_dgemm_bm(M)) {
     case 16: rc = dgemm_glu_bn<16>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
     case 32: rc = dgemm_glu_bn<32>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
+    case 96: rc = dgemm_glu_bn<96>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
     case 64: rc = dgemm_glu_bn<64>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
     case 128: rc = dgemm_glu_bn<128>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
     default: rc = dgemm_glu_bn<256>(x, w, M, N, K, bn, out, ldo, gp, stream); break;
@@ -767,6 +771,7 @@ CFC_API int cfc_dgemm_joint(const void* x, const void* w, int M, int N, int K, i
   switch (cfc_dgemm_bm(M)) {
     case 16: rc = dgemm_joint_bn<16>(x, w, M, N, K, split, bn, part, g, stream); break;
     case 32: rc = dgemm_joint_bn<32>(x, w, M, N, K, split, bn, part, g, stream); break;
+    case 96: rc = dgemm_joint_bn<96>(x, w, M, N, K, split, bn, part, g, stream); break;
     case 64: rc = dgemm_joint_bn<64>(x, w, M, N, K, split, bn, part, g, stream); break;
     case 128: rc = dgemm_joint_bn<128>(x, w, M, N, K, split, bn, part, g, stream); break;
     default: rc = dgemm_joint_bn<256>(x, w, M, N, K, split, bn, part, g, stream); break;
@@ -859,7 +864,7 @@ double dgemm_us(int M, int N, int K, int bn, int split) {
   constexpr double CU_RATE = 25e3;         // W bytes/us one workgroup streams (6.4 TB/s over 256 CUs)
   constexpr double PART_RATE = 6e6;        // fp32 partial slab traffic
   constexpr double X_RATE = 90e3;          // per-CU L2 -> LDS rate of the X re-reads (ablation: X costs ~12 us of gate/up)
-  const int bm = M <= 64 ? 64 : M <= 128 ? 128 : 256;   // the tiles of 16 and 32 rows keep the splits of 64: no other was faster
+  const int bm = M <= 64 ? 64 : M <= 128 ? 128 : 256;   // the tiles of 16 and 32 rows keep the splits of 64 (no other was faster), 96 those of 128
   const int64_t blocks = (int64_t)(N / bn) * ((M + bm - 1) / bm) * split;
   const double rounds = (double)((blocks + DG_CUS - 1) / DG_CUS);
   double t = rounds * ((double)bn * K * 2 / split / CU_RATE + (double)bm * K * 2 / split / X_RATE) + 1.5 * (rounds - 1.0);

@@ -1,4 +1,4 @@
-"""The decode GEMM's row tiles of 16 and 32 (dgemm.hip): the rows of a small batch are, bit for bit, those of a batch of 64
+"""The decode GEMM's row tiles of 16, 32 and 96 (dgemm.hip): the rows of a batch are, bit for bit, those of a batch of 128
 whose first rows they are (the same products in the same order), and those are what 64-bit sums say."""
 import pytest
 import torch
@@ -6,14 +6,14 @@ import torch
 from copilot_for_consensus_amd.ops import kernels as K
 from copilot_for_consensus_amd.ops import moe
 
-ROWS = (1, 5, 15, 16, 17, 31, 32)
+ROWS = (1, 5, 15, 16, 17, 31, 32, 33, 65, 81, 96, 97)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("N, Kd, bn, split", [(64, 64, 64, 1), (448, 192, 64, 3), (192, 1088, 96, 2), (448, 640, 112, 1), (384, 2176, 128, 4)])
 def test_rows_are_those_of_a_larger_batch(N, Kd, bn, split):
     g = torch.Generator("cuda").manual_seed(N)
-    x = torch.randn(2, 64, Kd, device="cuda", generator=g).bfloat16()
+    x = torch.randn(2, 128, Kd, device="cuda", generator=g).bfloat16()
     w = (torch.randn(N, Kd, device="cuda", generator=g) * 0.1).bfloat16()
     pk = K.pack_dgemm_weight(w, bn=bn)
     in_of = torch.randint(0, 2, (N // bn,), device="cuda", dtype=torch.int32, generator=g)
@@ -29,7 +29,7 @@ def test_rows_are_those_of_a_larger_batch(N, Kd, bn, split):
             out["joint"] = K.dgemm_joint(xs, pk, in_of, torch.full((split, M, N), float("nan"), device="cuda"))
         return out
 
-    want = products(64)
+    want = products(128)
     exact = x[0].double() @ w.double().t()
     # sums of K products in fp32, in any order
     assert ((want["part"].double().sum(0) - exact).abs() <= Kd * 2.0 ** -24 * (x[0].double().abs() @ w.double().abs().t())).all()
