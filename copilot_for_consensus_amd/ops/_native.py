@@ -100,7 +100,7 @@ _KERNEL_SIGS = {
     "cfc_knn_queries": [P, P, P, I, I, I, P],
     "cfc_enc_tiny": [I, I, I, P],
     "cfc_put_ints": [P, P, I, P],
-    "cfc_enc_forward": [P] * 10 + [I, I, I, I, P, I, F, F, I] + [P] * 6,
+    "cfc_enc_forward": [P] * 10 + [I, I, I, I, P, I, F, F, I] + [P] * 5 + [I, P],
     "cfc_knn_scan": [P, P, I, I, I, P, P, P, P, L, P, L, P],
     "cfc_knn_maxima": [P, P, I, I, I, P, P, P, P, L, P],
     "cfc_knn_blocks": [P, P, I, I, I, P, P, P, P, I, L, P, P, P, P],

@@ -419,9 +419,10 @@ def encoder_weights(T: int, p: dict, layers: list[dict], heads: int, max_seqlen:
 
 
 def encoder_forward(ids, positions, weights: list[int], layers: int, cu_seqlens, tiles, heads: int, max_seqlen: int, scale: float,
-                    eps: float) -> torch.Tensor:
+                    eps: float, polls: int = -1) -> torch.Tensor:
     """Token states [T, 384] of a packed batch, all launches in one call (encoder.hip); ``weights``: :func:`encoder_weights`
-    of the batch's rows."""
+    of the batch's rows.  ``polls``: loads after which workgroups of one launch give up on one another and another launch takes
+    the batch, to the same bits (below 0: some 20 ms of them)."""
     for t in (ids, positions, cu_seqlens, *tiles):
         _req(t, torch.int32, "encoder_forward")
     lib, T, H, dev = kernels(), ids.numel(), ENCODER_HIDDEN, ids.device
@@ -441,7 +442,7 @@ def encoder_forward(ids, positions, weights: list[int], layers: int, cu_seqlens,
     check(lib.cfc_enc_forward(ids.data_ptr(), positions.data_ptr(), *weights[:5],
                               cu_seqlens.data_ptr(), tiles[0].data_ptr(), tiles[1].data_ptr(), tiles[0].numel(), ENCODER_TILE_ROWS,
                               int(max_seqlen), layers, W, heads, float(scale), float(eps), T, x.data_ptr(), _p(y), _p(att),
-                              _p(qkv), _p(h), _stream(x)), "cfc_enc_forward")
+                              _p(qkv), _p(h), int(polls), _stream(x)), "cfc_enc_forward")
     return x
 
 

@@ -772,11 +772,13 @@ __global__ void __launch_bounds__(256) enc_ksplit_kernel(const uint16_t* __restr
 // 12 tokens through MiniLM's six layers 136 -> 80 us, 32 tokens 188 -> 119, 64 tokens 295 -> 178.  A layer's 12 us are
 // its four hand-overs of 2 to 2.5 us (a store and a poll of about 1 us each), two norms and the products between.
 //
-// The workgroups wait for one another, so all have to be resident.  One fits a CU: four such launches side by side, as
-// many as a process has hardware queues, fill 240 CUs, and with fewer than that the kernels for few rows are taken.  A
-// wait is bounded all the same: a wave that has polled EN_SPINS times takes what is there, and ~0 words are NaN in
-// every result.
-constexpr int EN_TINY_ROWS = 64, EN_TINY_LAYERS = 24, EN_SPINS = 1 << 20;
+// The workgroups wait for one another, so all have to be resident, and nothing can promise that: launches of other streams
+// and processes may hold the CUs that some of them need, and wait for others of their own.  So a wait is bounded: a wave that
+// has polled `polls` times takes what is there and says so in the workspace's last word, which ends all waits for it, and
+// a launch of one workgroup behind this one, which waits for nothing, looks at that word and takes all layers by itself,
+// the same products in the same order: the same bits, in 1.5 ms of 12 tokens and 2.5 of 64 (6 layers).  Where no wait was
+// given up it is over in 2 us, so a call of 12 tokens takes 85.6 us, 83.7 without it.
+constexpr int EN_TINY_ROWS = 64, EN_TINY_LAYERS = 24, EN_POLLS = 1 << 14;
 constexpr uint32_t EN_EMPTY = ~0u;
 constexpr int EN_HEADS = EN_H / 32, EN_BLOCKS = EN_H / 16, EN_INNER = EN_F / 64;      // workgroups of each kind
 
@@ -792,8 +794,12 @@ __global__ void __launch_bounds__(256) enc_empty_kernel(uint4* __restrict__ p, i
 // Sixteen bytes at every off + 64 s, once none of their words is empty (the words are looked at one by one: a load need be
 // no more than them in one piece).  With pauses and at low priority: loads go out oldest wave first, and waves that poll
 // without a pause keep a younger one of their CU from ever storing what they wait for.
+struct EncWait {
+  int polls;              // left
+  uint32_t* late;         // empty, until a wave gave up
+};
 template <int N, int S>
-__device__ __forceinline__ void en_take(const uint16_t* base, int bytes, const uint32_t (&off)[N], uint4 (&v)[N][S], int& spins) {
+__device__ __forceinline__ void en_take(const uint16_t* base, int bytes, const uint32_t (&off)[N], uint4 (&v)[N][S], EncWait& wait) {
   const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, bytes, 0x00020000);
   __builtin_amdgcn_s_setprio(0);
   for (;;) {
@@ -807,8 +813,12 @@ __device__ __forceinline__ void en_take(const uint16_t* base, int bytes, const u
     for (int i = 0; i < N; ++i)
 #pragma unroll
       for (int s = 0; s < S; ++s) all &= v[i][s].x != EN_EMPTY && v[i][s].y != EN_EMPTY && v[i][s].z != EN_EMPTY && v[i][s].w != EN_EMPTY;
-    if (__all(all) || spins >= EN_SPINS) break;
-    ++spins;
+    if (__all(all)) break;
+    if (wait.polls <= 0) {
+      __hip_atomic_store(wait.late, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      break;
+    }
+    --wait.polls;
     __builtin_amdgcn_s_sleep(1);
     asm volatile("" ::: "memory");                // loaded again
   }
@@ -829,12 +839,13 @@ __device__ __forceinline__ f32x4_t four_bf(uint2 b) {
   return f32x4_t{__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u), __uint_as_float(b.y << 16), __uint_as_float(b.y & 0xffff0000u)};
 }
 
-// G groups of 16 rows, T of them rows; grid EN_HEADS + EN_BLOCKS + EN_INNER.
-template <int G>
+// G groups of 16 rows, T of them rows; grid EN_HEADS + EN_BLOCKS + EN_INNER.  ALONE: one workgroup, which does all in turn
+// if a wait of the launch before it was given up.
+template <int G, bool ALONE>
 __global__ void __launch_bounds__(512, 2)
     enc_tiny_kernel(const int32_t* __restrict__ ids, const int32_t* __restrict__ pos, EncTiny W, const int32_t* __restrict__ cu,
                     const int32_t* __restrict__ tile_seq, int n_tiles, int layers, uint16_t* buf, uint16_t* __restrict__ out, int T,
-                    float scale_log2, float eps) {
+                    float scale_log2, float eps, int polls) {
   constexpr int U = 2 * G, V = U < 4 ? U : 4, ROW = EN_H * 2;     // rows of a wave (w, w + 8, ..), at a time; bytes of a row
   extern __shared__ __attribute__((aligned(16))) char en_smem[];
   char* rows = en_smem;                           // [16 G][384], chunk c of row r at slot c ^ (r & 15)
@@ -842,9 +853,10 @@ __global__ void __launch_bounds__(512, 2)
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
   const bool on = lane < EN_H / 8;                // a row's chunks
   const int c = on ? lane : 0;
-  int spins = 0;
-  __builtin_amdgcn_s_setprio(1);
   const size_t place = (size_t)T * (3 * EN_H + EN_F);
+  EncWait wait = {polls, reinterpret_cast<uint32_t*>(buf + layers * place)};
+  if (ALONE && *wait.late == EN_EMPTY) return;
+  __builtin_amdgcn_s_setprio(1);
   uint4 x[U];                                     // this wave's rows of the layer's input, then of what lies between its sublayers
 
   auto put = [&]() {                              // to where the products read them
@@ -897,7 +909,7 @@ __global__ void __launch_bounds__(512, 2)
     uint4 t[U][1];
 #pragma unroll
     for (int u = 0; u < U; ++u) at[u] = min(w + 8 * u, T - 1) * ROW + 16 * c;
-    en_take(y, T * ROW, at, t, spins);
+    en_take(y, T * ROW, at, t, wait);
     float b[8];
     unpack8(pb, b);
 #pragma unroll
@@ -938,13 +950,12 @@ __global__ void __launch_bounds__(512, 2)
     __syncthreads();
   }
 
-  if (blockIdx.x < EN_HEADS) {
-    // ---- a head: waves 0 .. 5 take 16 of q's, k's and v's 32 columns each, waves 0 .. G - 1 a group of queries
-    constexpr int QS = 80, VS = 32 * ((G + 1) / 2) + 8;      // row strides: bytes of q and k, values of V^T
-    const int head = blockIdx.x, n0 = (w >> 1) * EN_H + head * 32 + (w & 1) * 16;
-    char *q = rest, *k = q + 16 * G * QS;
-    uint16_t* vt = reinterpret_cast<uint16_t*>(k + 16 * G * QS);
-    int *from = reinterpret_cast<int*>(vt + 32 * VS), *to = from + 16 * G;
+  // ---- a head: waves 0 .. 5 take 16 of q's, k's and v's 32 columns each, waves 0 .. G - 1 a group of queries
+  constexpr int QS = 80, VS = 32 * ((G + 1) / 2) + 8;      // row strides: bytes of q and k, values of V^T
+  char *q = rest, *k = q + 16 * G * QS;
+  uint16_t* vt = reinterpret_cast<uint16_t*>(k + 16 * G * QS);
+  int *from = reinterpret_cast<int*>(vt + 32 * VS), *to = from + 16 * G;
+  auto texts = [&]() {                            // which keys a row sees; V^T past the rows: zeros
     for (int i = threadIdx.x; i < 32 * VS; i += 512) vt[i] = 0;
     for (int i = threadIdx.x; i < 16 * G; i += 512) from[i] = i, to[i] = i + 1;
     __syncthreads();
@@ -952,162 +963,132 @@ __global__ void __launch_bounds__(512, 2)
       const int a = cu[tile_seq[i]], b = min(cu[tile_seq[i] + 1], T);
       for (int t = max(a, 0); t < b; ++t) from[t] = a, to[t] = b;
     }
-    uint4 wf[12];
-    uint2 bb;
-    auto load = [&](int l) {
-      if (w >= 6) return;
-      const uint16_t* p = W.layer[l][0] + (size_t)(n0 + r16) * EN_H + 8 * g;
+  };
+  uint4 wf[12];
+  uint2 bb;
+  auto load_head = [&](int l, int head) {
+    if (w >= 6) return;
+    const int n0 = (w >> 1) * EN_H + head * 32 + (w & 1) * 16;
+    const uint16_t* p = W.layer[l][0] + (size_t)(n0 + r16) * EN_H + 8 * g;
 #pragma unroll
-      for (int s = 0; s < 12; ++s) wf[s] = *reinterpret_cast<const uint4*>(p + 32 * s);
-      bb = *reinterpret_cast<const uint2*>(W.layer[l][1] + n0 + 4 * g);
-    };
-    load(0);
-    put();
-    for (int l = 0; l < layers; ++l) {
-      uint16_t *att = buf + l * place, *y1 = att + (size_t)T * EN_H, *y2 = y1 + (size_t)T * (EN_H + EN_F);
-      __syncthreads();                            // the rows are there
-      if (w < 6) {
-        f32x4_t a[G];
+    for (int s = 0; s < 12; ++s) wf[s] = *reinterpret_cast<const uint4*>(p + 32 * s);
+    bb = *reinterpret_cast<const uint2*>(W.layer[l][1] + n0 + 4 * g);
+  };
+  auto attend = [&](int head, uint16_t* att) {
+    if (w < 6) {
+      f32x4_t a[G];
 #pragma unroll
-        for (int i = 0; i < G; ++i) a[i] = four_bf(bb);
+      for (int i = 0; i < G; ++i) a[i] = four_bf(bb);
 #pragma unroll
-        for (int s = 0; s < 12; ++s)
+      for (int s = 0; s < 12; ++s)
 #pragma unroll
-          for (int i = 0; i < G; ++i) a[i] = mfma16(wf[s], frag(i, s), a[i]);
-#pragma unroll
-        for (int i = 0; i < G; ++i) {
-          const int t = 16 * i + r16;
-          const uint2 y = make_uint2(pack2bf(a[i][0], a[i][1]), pack2bf(a[i][2], a[i][3]));
-          if (w < 4) {
-            *reinterpret_cast<uint2*>((w < 2 ? q : k) + t * QS + 32 * (w & 1) + 8 * g) = y;
-          } else {
-            uint16_t* v = vt + (16 * (w & 1) + 4 * g) * VS + t;
-            v[0] = (uint16_t)y.x; v[VS] = (uint16_t)(y.x >> 16); v[2 * VS] = (uint16_t)y.y; v[3 * VS] = (uint16_t)(y.y >> 16);
-          }
-        }
-      }
-      __syncthreads();
-      if (w < G) {
-        // scores with the keys along a lane's registers: key 16 i + 4 g + e of query 16 w + r16
-        const uint4 qf = *reinterpret_cast<const uint4*>(q + (16 * w + r16) * QS + 16 * g);
-        const int t = 16 * w + r16, a = from[t], b = to[t];
-        f32x4_t s[2 * ((G + 1) / 2)];
-        float m = -INFINITY, sum = 0.f;
-#pragma unroll
-        for (int i = 0; i < 2 * ((G + 1) / 2); ++i) {
-          s[i] = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-          if (i >= G) continue;
-          const f32x4_t z = mfma16(*reinterpret_cast<const uint4*>(k + (16 * i + r16) * QS + 16 * g), qf, f32x4_t{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int j = 16 * i + 4 * g + e;
-            s[i][e] = j >= a && j < b ? z[e] * scale_log2 : -INFINITY;
-            m = fmaxf(m, s[i][e]);
-          }
-        }
-        m = xor32_max(xor16_max(m));
-        const float ref = m == -INFINITY ? 0.f : m;
-#pragma unroll
-        for (int i = 0; i < 2 * ((G + 1) / 2); ++i)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            s[i][e] = __builtin_amdgcn_exp2f(s[i][e] - ref);
-            sum += s[i][e];
-          }
-        sum = xor32_sum(xor16_sum(sum));
-        f32x4_t o[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-        for (int i = 0; i < (G + 1) / 2; ++i) {   // 32 keys, in the order that the scores have them
-          const uint4 p = make_uint4(pack2bf(s[2 * i][0], s[2 * i][1]), pack2bf(s[2 * i][2], s[2 * i][3]), pack2bf(s[2 * i + 1][0], s[2 * i + 1][1]),
-                                     pack2bf(s[2 * i + 1][2], s[2 * i + 1][3]));
-#pragma unroll
-          for (int d = 0; d < 2; ++d) {
-            const uint16_t* v = vt + (16 * d + r16) * VS + 32 * i + 4 * g;
-            const uint2 lo = *reinterpret_cast<const uint2*>(v), hi = *reinterpret_cast<const uint2*>(v + 16);
-            o[d] = mfma16(make_uint4(lo.x, lo.y, hi.x, hi.y), p, o[d]);
-          }
-        }
-        const float inv = 1.f / sum;
-#pragma unroll
-        for (int d = 0; d < 2; ++d)
-          if (t < T) en_give(att + (size_t)t * EN_H + head * 32 + 16 * d + 4 * g, o[d] * inv);
-      }
-      if (l + 1 < layers) load(l + 1);            // loads return in order: ahead of nothing that is waited for
-      next(y1, W.layer[l][3], W.layer[l][4], W.layer[l][5]);
-      next(y2, W.layer[l][9], W.layer[l][10], W.layer[l][11]);
-      put();
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int r = w + 8 * u;
-      if (on && r < T && r % EN_HEADS == head) *reinterpret_cast<uint4*>(out + (size_t)r * EN_H + 8 * c) = x[u];
-    }
-    return;
-  }
-
-  if (blockIdx.x >= EN_HEADS + EN_BLOCKS) {
-    // ---- 64 inner columns: 16 per wave of a group of rows
-    const int n0 = (blockIdx.x - EN_HEADS - EN_BLOCKS) * 64 + 16 * (w & 3);
-    uint4 wf[12];
-    uint2 bb;
-    auto load = [&](int l) {
-      const uint16_t* p = W.layer[l][6] + (size_t)(n0 + r16) * EN_H + 8 * g;
-#pragma unroll
-      for (int s = 0; s < 12; ++s) wf[s] = *reinterpret_cast<const uint4*>(p + 32 * s);
-      bb = *reinterpret_cast<const uint2*>(W.layer[l][7] + n0 + 4 * g);
-    };
-    load(0);
-    for (int l = 0; l < layers; ++l) {
-      const uint16_t* y1 = buf + l * place + (size_t)T * EN_H;
-      uint16_t* h = buf + l * place + (size_t)T * 2 * EN_H;
-      next(y1, W.layer[l][3], W.layer[l][4], W.layer[l][5]);
-      put();                                      // the rows before were read: these came of what was made of them
-      __syncthreads();
+        for (int i = 0; i < G; ++i) a[i] = mfma16(wf[s], frag(i, s), a[i]);
 #pragma unroll
       for (int i = 0; i < G; ++i) {
-        if ((i & 1) != w >> 2) continue;
-        f32x4_t a = four_bf(bb);
-#pragma unroll
-        for (int s = 0; s < 12; ++s) a = mfma16(wf[s], frag(i, s), a);
-        Gelu ge;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float v = a[e];
-          en_gelu<0>(ge, v);
-          en_gelu<1>(ge, v);
-          en_gelu<2>(ge, v);
-          a[e] = v;
+        const int t = 16 * i + r16;
+        const uint2 y = make_uint2(pack2bf(a[i][0], a[i][1]), pack2bf(a[i][2], a[i][3]));
+        if (w < 4) {
+          *reinterpret_cast<uint2*>((w < 2 ? q : k) + t * QS + 32 * (w & 1) + 8 * g) = y;
+        } else {
+          uint16_t* v = vt + (16 * (w & 1) + 4 * g) * VS + t;
+          v[0] = (uint16_t)y.x; v[VS] = (uint16_t)(y.x >> 16); v[2 * VS] = (uint16_t)y.y; v[3 * VS] = (uint16_t)(y.y >> 16);
         }
-        if (16 * i + r16 < T) en_give(h + (size_t)(16 * i + r16) * EN_F + n0 + 4 * g, a);
-      }
-      if (l + 1 < layers) {
-        load(l + 1);                              // loads return in order: ahead of nothing that is waited for
-        next(h + (size_t)T * EN_F, W.layer[l][9], W.layer[l][10], W.layer[l][11]);
       }
     }
-    return;
-  }
+    __syncthreads();
+    if (w >= G) return;
+    // scores with the keys along a lane's registers: key 16 i + 4 g + e of query 16 w + r16
+    const uint4 qf = *reinterpret_cast<const uint4*>(q + (16 * w + r16) * QS + 16 * g);
+    const int t = 16 * w + r16, a = from[t], b = to[t];
+    f32x4_t s[2 * ((G + 1) / 2)];
+    float m = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2 * ((G + 1) / 2); ++i) {
+      s[i] = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (i >= G) continue;
+      const f32x4_t z = mfma16(*reinterpret_cast<const uint4*>(k + (16 * i + r16) * QS + 16 * g), qf, f32x4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = 16 * i + 4 * g + e;
+        s[i][e] = j >= a && j < b ? z[e] * scale_log2 : -INFINITY;
+        m = fmaxf(m, s[i][e]);
+      }
+    }
+    m = xor32_max(xor16_max(m));
+    const float ref = m == -INFINITY ? 0.f : m;
+#pragma unroll
+    for (int i = 0; i < 2 * ((G + 1) / 2); ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[i][e] = __builtin_amdgcn_exp2f(s[i][e] - ref);
+        sum += s[i][e];
+      }
+    sum = xor32_sum(xor16_sum(sum));
+    f32x4_t o[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int i = 0; i < (G + 1) / 2; ++i) {       // 32 keys, in the order that the scores have them
+      const uint4 p = make_uint4(pack2bf(s[2 * i][0], s[2 * i][1]), pack2bf(s[2 * i][2], s[2 * i][3]), pack2bf(s[2 * i + 1][0], s[2 * i + 1][1]),
+                                 pack2bf(s[2 * i + 1][2], s[2 * i + 1][3]));
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        const uint16_t* v = vt + (16 * d + r16) * VS + 32 * i + 4 * g;
+        const uint2 lo = *reinterpret_cast<const uint2*>(v), hi = *reinterpret_cast<const uint2*>(v + 16);
+        o[d] = mfma16(make_uint4(lo.x, lo.y, hi.x, hi.y), p, o[d]);
+      }
+    }
+    const float inv = 1.f / sum;
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+      if (t < T) en_give(att + (size_t)t * EN_H + head * 32 + 16 * d + 4 * g, o[d] * inv);
+  };
+
+  // ---- 64 inner columns: 16 per wave of a group of rows
+  auto load_up = [&](int l, int block) {
+    const int n0 = block * 64 + 16 * (w & 3);
+    const uint16_t* p = W.layer[l][6] + (size_t)(n0 + r16) * EN_H + 8 * g;
+#pragma unroll
+    for (int s = 0; s < 12; ++s) wf[s] = *reinterpret_cast<const uint4*>(p + 32 * s);
+    bb = *reinterpret_cast<const uint2*>(W.layer[l][7] + n0 + 4 * g);
+  };
+  auto up = [&](int block, uint16_t* h) {
+    const int n0 = block * 64 + 16 * (w & 3);
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      if ((i & 1) != w >> 2) continue;
+      f32x4_t a = four_bf(bb);
+#pragma unroll
+      for (int s = 0; s < 12; ++s) a = mfma16(wf[s], frag(i, s), a);
+      Gelu ge;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v = a[e];
+        en_gelu<0>(ge, v);
+        en_gelu<1>(ge, v);
+        en_gelu<2>(ge, v);
+        a[e] = v;
+      }
+      if (16 * i + r16 < T) en_give(h + (size_t)(16 * i + r16) * EN_F + n0 + 4 * g, a);
+    }
+  };
 
   // ---- 16 columns of o (waves 4 .. 7, a quarter of K each) and of down (an eighth of K per wave)
-  const int n0 = (blockIdx.x - EN_HEADS) * 16;
   f32x4_t *po = reinterpret_cast<f32x4_t*>(rest), *pd = po + 4 * G * 64;        // parts of sums [4][G][64], [8][G][64]
   uint4 wo[3], wd[6];
-  auto load = [&](int l) {
+  auto load_block = [&](int l, int block) {
+    const int n0 = block * 16;
     const uint16_t *p = W.layer[l][2] + (size_t)(n0 + r16) * EN_H + 96 * (w & 3) + 8 * g, *q = W.layer[l][8] + (size_t)(n0 + r16) * EN_F + 192 * w + 8 * g;
 #pragma unroll
     for (int s = 0; s < 3; ++s) wo[s] = *reinterpret_cast<const uint4*>(p + 32 * s);
 #pragma unroll
     for (int s = 0; s < 6; ++s) wd[s] = *reinterpret_cast<const uint4*>(q + 32 * s);
   };
-  load(0);
-  for (int l = 0; l < layers; ++l) {
-    uint16_t *att = buf + l * place, *y1 = att + (size_t)T * EN_H, *h = y1 + (size_t)T * EN_H, *y2 = h + (size_t)T * EN_F;
+  auto project = [&](int block, const uint16_t* att, uint16_t* y1) {
     if (w >= 4) {
       uint32_t at[G];
       uint4 v[G][3];
 #pragma unroll
       for (int i = 0; i < G; ++i) at[i] = min(16 * i + r16, T - 1) * ROW + 192 * (w & 3) + 16 * g;
-      en_take(att, T * ROW, at, v, spins);
+      en_take(att, T * ROW, at, v, wait);
 #pragma unroll
       for (int i = 0; i < G; ++i) {
         f32x4_t a = {0.f, 0.f, 0.f, 0.f};
@@ -1122,8 +1103,10 @@ __global__ void __launch_bounds__(512, 2)
       f32x4_t a = po[i * 64 + lane];
 #pragma unroll
       for (int s = 1; s < 4; ++s) a += po[(s * G + i) * 64 + lane];
-      if (t < T) en_give(y1 + (size_t)t * EN_H + n0 + 4 * g, a);
+      if (t < T) en_give(y1 + (size_t)t * EN_H + block * 16 + 4 * g, a);
     }
+  };
+  auto down = [&](int block, const uint16_t* h, uint16_t* y2) {
 #pragma unroll
     for (int i0 = 0; i0 < G; i0 += 2) {
       constexpr int N = G < 2 ? G : 2;            // at a time: registers
@@ -1131,7 +1114,7 @@ __global__ void __launch_bounds__(512, 2)
       uint4 v[N][6];
 #pragma unroll
       for (int i = 0; i < N; ++i) at[i] = min(16 * (i0 + i) + r16, T - 1) * (2 * EN_F) + 384 * w + 16 * g;
-      en_take(h, T * 2 * EN_F, at, v, spins);
+      en_take(h, T * 2 * EN_F, at, v, wait);
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         f32x4_t a = {0.f, 0.f, 0.f, 0.f};
@@ -1146,9 +1129,101 @@ __global__ void __launch_bounds__(512, 2)
       f32x4_t a = pd[w * 64 + lane];
 #pragma unroll
       for (int s = 1; s < 8; ++s) a += pd[(s * G + w) * 64 + lane];
-      if (t < T) en_give(y2 + (size_t)t * EN_H + n0 + 4 * g, a);
+      if (t < T) en_give(y2 + (size_t)t * EN_H + block * 16 + 4 * g, a);
     }
-    if (l + 1 < layers) load(l + 1);
+  };
+
+  if constexpr (ALONE) {
+    // what one product left is there for the next one: stored, and all waves past it
+    auto settle = [&]() {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    };
+    put();
+    for (int l = 0; l < layers; ++l) {
+      uint16_t *att = buf + l * place, *y1 = att + (size_t)T * EN_H, *h = y1 + (size_t)T * EN_H, *y2 = h + (size_t)T * EN_F;
+      texts();                                    // again: the parts of sums lay there
+      for (int head = 0; head < EN_HEADS; ++head) {
+        load_head(l, head);
+        settle();
+        attend(head, att);
+      }
+      settle();
+      for (int block = 0; block < EN_BLOCKS; ++block) {
+        load_block(l, block);
+        project(block, att, y1);
+        settle();
+      }
+      next(y1, W.layer[l][3], W.layer[l][4], W.layer[l][5]);
+      put();
+      settle();
+      for (int block = 0; block < EN_INNER; ++block) {
+        load_up(l, block);
+        up(block, h);
+      }
+      settle();
+      for (int block = 0; block < EN_BLOCKS; ++block) {
+        load_block(l, block);
+        down(block, h, y2);
+        settle();
+      }
+      next(y2, W.layer[l][9], W.layer[l][10], W.layer[l][11]);
+      put();
+      settle();
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (on && w + 8 * u < T) *reinterpret_cast<uint4*>(out + (size_t)(w + 8 * u) * EN_H + 8 * c) = x[u];
+    return;
+  }
+
+  if (blockIdx.x < EN_HEADS) {
+    const int head = blockIdx.x;
+    texts();
+    load_head(0, head);
+    put();
+    for (int l = 0; l < layers; ++l) {
+      uint16_t *att = buf + l * place, *y1 = att + (size_t)T * EN_H, *y2 = y1 + (size_t)T * (EN_H + EN_F);
+      __syncthreads();                            // the rows are there
+      attend(head, att);
+      if (l + 1 < layers) load_head(l + 1, head); // loads return in order: ahead of nothing that is waited for
+      next(y1, W.layer[l][3], W.layer[l][4], W.layer[l][5]);
+      next(y2, W.layer[l][9], W.layer[l][10], W.layer[l][11]);
+      put();
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int r = w + 8 * u;
+      if (on && r < T && r % EN_HEADS == head) *reinterpret_cast<uint4*>(out + (size_t)r * EN_H + 8 * c) = x[u];
+    }
+    return;
+  }
+
+  if (blockIdx.x >= EN_HEADS + EN_BLOCKS) {
+    const int block = blockIdx.x - EN_HEADS - EN_BLOCKS;
+    load_up(0, block);
+    for (int l = 0; l < layers; ++l) {
+      const uint16_t* y1 = buf + l * place + (size_t)T * EN_H;
+      uint16_t* h = buf + l * place + (size_t)T * 2 * EN_H;
+      next(y1, W.layer[l][3], W.layer[l][4], W.layer[l][5]);
+      put();                                      // the rows before were read: these came of what was made of them
+      __syncthreads();
+      up(block, h);
+      if (l + 1 < layers) {
+        load_up(l + 1, block);                    // loads return in order: ahead of nothing that is waited for
+        next(h + (size_t)T * EN_F, W.layer[l][9], W.layer[l][10], W.layer[l][11]);
+      }
+    }
+    return;
+  }
+
+  const int block = blockIdx.x - EN_HEADS;
+  load_block(0, block);
+  for (int l = 0; l < layers; ++l) {
+    uint16_t *att = buf + l * place, *y1 = att + (size_t)T * EN_H, *h = y1 + (size_t)T * EN_H, *y2 = h + (size_t)T * EN_F;
+    project(block, att, y1);
+    down(block, h, y2);
+    if (l + 1 < layers) load_block(l + 1, block);
   }
 }
 
@@ -1174,25 +1249,26 @@ constexpr int EN_FEW_ROWS = 2560, EN_MANY_ROWS = 10753;
 // Which rows this file's kernels take: 1 few, 2 many, 0 neither.
 CFC_API int cfc_enc_rows(int T) { return T <= EN_FEW_ROWS ? 1 : T >= EN_MANY_ROWS ? 2 : 0; }
 
-// Values of workspace (bf16) that the one launch for T rows of a model takes on a stream; 0: it does not take them, or too few
-// CUs are the stream's.
+// Values of workspace (bf16) that the one launch for T rows of a model takes on a stream; 0: it does not take them, or so few
+// CUs are the stream's that its workgroups would be long in coming.
 CFC_API int cfc_enc_tiny(int T, int layers, int heads, hipStream_t stream) {
   if (T < 1 || T > EN_TINY_ROWS || layers < 1 || layers > EN_TINY_LAYERS || heads != EN_HEADS) return 0;
   uint32_t mask[8];                               // 256 CUs
   int cus = 0;
   if (hipExtStreamGetCUMask(stream, 8, mask) != hipSuccess) return 0;
   for (const uint32_t m : mask) cus += __builtin_popcount(m);
-  return cus >= 4 * (EN_HEADS + EN_BLOCKS + EN_INNER) ? layers * T * (3 * EN_H + EN_F) : 0;
+  return cus >= 4 * (EN_HEADS + EN_BLOCKS + EN_INNER) ? layers * T * (3 * EN_H + EN_F) + 8 : 0;
 }
 
 // Token states of a packed batch: embeddings, then every layer, one call for all launches.  W: host array of twelve
 // device pointers per layer (qkv, qkv_b, o, o_b, ln1_g, ln1_b, up, up_b, down, down_b, ln2_g, ln2_b).  x [T][384] the
 // states; att [T][384], qkv [T][1152], and for few rows y [T][384] and h [T][1536]: workspace.  All bf16 and 16-byte
-// aligned.  With att null, h is the workspace of cfc_enc_tiny and no other is read.
+// aligned.  With att null, h is the workspace of cfc_enc_tiny and no other is read; a wait in that launch is given up after
+// `polls` loads (below 0: EN_POLLS).
 CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* word, const void* pos_emb, const void* type_emb,
                             const void* emb_g, const void* emb_b, const int32_t* cu, const int32_t* tile_seq, const int32_t* tile_q0,
                             int n_tiles, int tile_rows, int max_seqlen, int layers, const void* const* W, int heads, float scale,
-                            float eps, int T, void* x, void* y, void* att, void* qkv, void* h, hipStream_t stream) {
+                            float eps, int T, void* x, void* y, void* att, void* qkv, void* h, int polls, hipStream_t stream) {
   const int kind = cfc_enc_rows(T);
   if (att == nullptr) {
     const int n = cfc_enc_tiny(T, layers, heads, stream);
@@ -1200,11 +1276,17 @@ CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* 
     EncTiny w = {(const uint16_t*)word, (const uint16_t*)pos_emb, (const uint16_t*)type_emb, (const uint16_t*)emb_g, (const uint16_t*)emb_b};
     memcpy(w.layer, W, sizeof(void*) * 12 * layers);
     enc_empty_kernel<<<min(256, (n / 8 + 255) / 256), 256, 0, stream>>>((uint4*)h, n / 8);
-#define TINY(G) enc_tiny_kernel<G><<<EN_HEADS + EN_BLOCKS + EN_INNER, 512, en_tiny_lds(G), stream>>>(ids, pos, w, cu, tile_seq, n_tiles, layers, \
-                                                                                         (uint16_t*)h, (uint16_t*)x, T, scale * 1.44269504f, eps)
-    if (T <= 16) TINY(1);
-    else if (T <= 32) TINY(2);
-    else TINY(4);
+#define TINY(G, ALONE, GRID, POLLS) enc_tiny_kernel<G, ALONE><<<GRID, 512, en_tiny_lds(G), stream>>>(ids, pos, w, cu, tile_seq, n_tiles, layers, \
+                                                                                         (uint16_t*)h, (uint16_t*)x, T, scale * 1.44269504f, eps, POLLS)
+#define TINY_GO(G)                                                                                         \
+  do {                                                                                                     \
+    TINY(G, false, EN_HEADS + EN_BLOCKS + EN_INNER, polls < 0 ? EN_POLLS : polls);                          \
+    TINY(G, true, 1, 0);                                                                                    \
+  } while (0)
+    if (T <= 16) TINY_GO(1);
+    else if (T <= 32) TINY_GO(2);
+    else TINY_GO(4);
+#undef TINY_GO
 #undef TINY
     return CFC_CHECK_LAUNCH();
   }

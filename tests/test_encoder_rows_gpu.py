@@ -105,8 +105,47 @@ def test_a_few_short_texts(lens, layers):
         m.forward_packed(ids, pos, cu, max(lens), tiles=tiles)
 
 
+@pytest.mark.parametrize("lens,layers", [([1], 1), ([12], 6), ([16], 24), ([9, 0, 8], 2), ([20, 12], 3), ([33], 2), ([1] * 40 + [24], 3)],
+                         ids=lambda v: str(v if isinstance(v, int) else sum(v)))
+def test_a_wait_that_is_given_up(lens, layers):
+    """Workgroups of the one launch that give up on one another, at once or after a few loads, say so, and the launch behind
+    it leaves the same bits; captured, again in each replay.  Where no wait is given up, it leaves what there is."""
+    import ctypes
+    import dataclasses
+    from copilot_for_consensus_amd.models.encoder import get_encoder_config
+    from copilot_for_consensus_amd.ops import kernels as K
+    m = _model(dataclasses.replace(get_encoder_config("minilm-l6"), layers=layers), seed=layers)
+    T, lib, c = sum(lens), K.kernels(), m.cfg
+    g = torch.Generator(device=DEV).manual_seed(T)
+    ids = torch.randint(0, c.vocab_size, (T,), device=DEV, dtype=torch.int32, generator=g)
+    pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).to(DEV)
+    cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).to(torch.int32)
+    tiles = tuple(torch.tensor(t, dtype=torch.int32, device=DEV) for t in K.prefill_tiles(cu.tolist(), K.ENCODER_TILE_ROWS))
+    cu, w = cu.to(DEV), K.encoder_weights(T, m.p, m.layers, c.heads, max(lens))
+    want = m.forward_packed(ids, pos, cu, max(lens), tiles=tiles)
+    call = lambda polls: K.encoder_forward(ids, pos, w, layers, cu, tiles, c.heads, max(lens), m.scale, c.ln_eps, polls)  # noqa: E731
+    for polls in (0, 2, -1):
+        assert torch.equal(call(polls), want)
+    h = torch.empty(lib.cfc_enc_tiny(T, layers, c.heads, None), dtype=torch.bfloat16, device=DEV)
+    ptrs, x = (ctypes.c_void_p * (12 * layers))(*w[5:]), torch.empty_like(want)
+    for polls, late in ((0, 0), (-1, -1)):
+        K.check(lib.cfc_enc_forward(ids.data_ptr(), pos.data_ptr(), *w[:5], cu.data_ptr(), tiles[0].data_ptr(), tiles[1].data_ptr(),
+                                    tiles[0].numel(), K.ENCODER_TILE_ROWS, max(lens), layers, ptrs, c.heads, m.scale, c.ln_eps, T,
+                                    x.data_ptr(), None, None, None, h.data_ptr(), polls, torch.cuda.current_stream().cuda_stream), "enc")
+        assert int(h.view(torch.int32)[-4]) == late and torch.equal(x, want)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        out = call(0)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
 def test_one_launch_needs_most_of_the_chip():
-    """Its workgroups wait for one another: a stream of few CUs keeps a launch per product, and gives the same."""
+    """A stream of few CUs, where its workgroups would be long in coming, keeps a launch per product, and gives the same."""
     from copilot_for_consensus_amd.models.encoder import EncoderModel
     from copilot_for_consensus_amd.ops import kernels as K
     from copilot_for_consensus_amd.runtime.cu_partition import partition_streams
