@@ -839,6 +839,9 @@ __device__ __forceinline__ f32x4_t four_bf(uint2 b) {
   return f32x4_t{__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u), __uint_as_float(b.y << 16), __uint_as_float(b.y & 0xffff0000u)};
 }
 
+// Whether either bf16 of the word is no finite number.
+__device__ __forceinline__ bool infinite(uint32_t v) { return (v & 0x7f80u) == 0x7f80u || (v & 0x7f800000u) == 0x7f800000u; }
+
 // G groups of 16 rows, T of them rows; grid EN_HEADS + EN_BLOCKS + EN_INNER.  ALONE: one workgroup, which does all in turn
 // if a wait of the launch before it was given up.
 template <int G, bool ALONE>
@@ -954,8 +957,9 @@ __global__ void __launch_bounds__(512, 2)
   constexpr int QS = 80, VS = 32 * ((G + 1) / 2) + 8;      // row strides: bytes of q and k, values of V^T
   char *q = rest, *k = q + 16 * G * QS;
   uint16_t* vt = reinterpret_cast<uint16_t*>(k + 16 * G * QS);
-  int *from = reinterpret_cast<int*>(vt + 32 * VS), *to = from + 16 * G;
+  int *from = reinterpret_cast<int*>(vt + 32 * VS), *to = from + 16 * G, *odd = to + 16 * G;
   auto texts = [&]() {                            // which keys a row sees; V^T past the rows: zeros
+    if (threadIdx.x == 0) *odd = 0;
     for (int i = threadIdx.x; i < 32 * VS; i += 512) vt[i] = 0;
     for (int i = threadIdx.x; i < 16 * G; i += 512) from[i] = i, to[i] = i + 1;
     __syncthreads();
@@ -992,6 +996,7 @@ __global__ void __launch_bounds__(512, 2)
         } else {
           uint16_t* v = vt + (16 * (w & 1) + 4 * g) * VS + t;
           v[0] = (uint16_t)y.x; v[VS] = (uint16_t)(y.x >> 16); v[2 * VS] = (uint16_t)y.y; v[3 * VS] = (uint16_t)(y.y >> 16);
+          if (infinite(y.x) || infinite(y.y)) *odd = 1;
         }
       }
     }
@@ -1025,15 +1030,42 @@ __global__ void __launch_bounds__(512, 2)
       }
     sum = xor32_sum(xor16_sum(sum));
     f32x4_t o[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+    uint4 p[(G + 1) / 2];                         // 32 keys each, in the order that the scores have them
 #pragma unroll
-    for (int i = 0; i < (G + 1) / 2; ++i) {       // 32 keys, in the order that the scores have them
-      const uint4 p = make_uint4(pack2bf(s[2 * i][0], s[2 * i][1]), pack2bf(s[2 * i][2], s[2 * i][3]), pack2bf(s[2 * i + 1][0], s[2 * i + 1][1]),
-                                 pack2bf(s[2 * i + 1][2], s[2 * i + 1][3]));
+    for (int i = 0; i < (G + 1) / 2; ++i)
+      p[i] = make_uint4(pack2bf(s[2 * i][0], s[2 * i][1]), pack2bf(s[2 * i][2], s[2 * i][3]), pack2bf(s[2 * i + 1][0], s[2 * i + 1][1]),
+                        pack2bf(s[2 * i + 1][2], s[2 * i + 1][3]));
+    auto values = [&](int i, int d) {
+      const uint16_t* v = vt + (16 * d + r16) * VS + 32 * i + 4 * g;
+      const uint2 lo = *reinterpret_cast<const uint2*>(v), hi = *reinterpret_cast<const uint2*>(v + 16);
+      return make_uint4(lo.x, lo.y, hi.x, hi.y);
+    };
+    if (__builtin_amdgcn_readfirstlane(*odd) == 0) {
 #pragma unroll
-      for (int d = 0; d < 2; ++d) {
-        const uint16_t* v = vt + (16 * d + r16) * VS + 32 * i + 4 * g;
-        const uint2 lo = *reinterpret_cast<const uint2*>(v), hi = *reinterpret_cast<const uint2*>(v + 16);
-        o[d] = mfma16(make_uint4(lo.x, lo.y, hi.x, hi.y), p, o[d]);
+      for (int i = 0; i < (G + 1) / 2; ++i)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) o[d] = mfma16(values(i, d), p[i], o[d]);
+    } else {
+      // Zero weights of other texts' keys do not take their infinite values out: text after text, its keys' values alone.
+      for (int j = 0; j < T;) {
+        const int a0 = from[j], b0 = to[j];
+        j = max(b0, j + 1);
+        if (!__any(a == a0)) continue;
+        f32x4_t z[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int i = 0; i < (G + 1) / 2; ++i) {
+          auto keep = [&](int at) {               // of keys at and at + 1
+            const int key = 32 * i + 4 * g + at;
+            return (key >= a0 && key < b0 ? 0xffffu : 0u) | (key + 1 >= a0 && key + 1 < b0 ? 0xffff0000u : 0u);
+          };
+          const uint4 m = make_uint4(keep(0), keep(2), keep(16), keep(18));
+#pragma unroll
+          for (int d = 0; d < 2; ++d) {
+            const uint4 v = values(i, d);
+            z[d] = mfma16(make_uint4(v.x & m.x, v.y & m.y, v.z & m.z, v.w & m.w), p[i], z[d]);
+          }
+        }
+        if (a == a0) o[0] = z[0], o[1] = z[1];
       }
     }
     const float inv = 1.f / sum;
@@ -1229,7 +1261,7 @@ __global__ void __launch_bounds__(512, 2)
 
 // Bytes of LDS: the rows, and the larger of what either kind keeps beside them.
 constexpr int en_tiny_lds(int G) { return 16 * G * EN_H * 2 + 12 * G * 1024; }
-static_assert(2 * 16 * 1 * 80 + 32 * 40 * 2 + 2 * 16 * 4 <= 12 * 1024 && 2 * 64 * 80 + 32 * 72 * 2 + 2 * 64 * 4 <= 48 * 1024, "");
+static_assert(2 * 16 * 1 * 80 + 32 * 40 * 2 + 2 * 16 * 4 + 4 <= 12 * 1024 && 2 * 64 * 80 + 32 * 72 * 2 + 2 * 64 * 4 + 4 <= 48 * 1024, "");
 
 }  // namespace
 

@@ -144,6 +144,25 @@ def test_a_wait_that_is_given_up(lens, layers):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("lens", [[3, 4, 5], [1] * 16, [15, 2, 15], [16, 16], [31, 2, 31], [7, 30, 27], [1] * 64, [300, 40, 9], [200] * 60],
+                         ids=lambda v: "-".join(map(str, v[:3])))
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_a_text_without_finite_states_spoils_no_other(lens, bad):
+    """Where one text's embedding is infinite or not a number, its neighbours' rows are the same bits as without."""
+    import dataclasses
+    from copilot_for_consensus_amd.models.encoder import get_encoder_config
+    m = _model(dataclasses.replace(get_encoder_config("minilm-l6"), layers=2), seed=1)
+    texts = [[100 * i + j for j in range(n)] for i, n in enumerate(lens)]
+    hit = len(lens) // 2
+    texts[hit][lens[hit] // 2] = 29_000
+    want = m.encode_ids(texts)
+    assert bool(want.isfinite().all())
+    m.p["word"][29_000] = bad
+    got = m.encode_ids(texts)
+    others = [i for i in range(len(lens)) if i != hit]
+    assert torch.equal(got[others], want[others]) and not bool(got[hit].isfinite().all())
+
+
 def test_one_launch_needs_most_of_the_chip():
     """A stream of few CUs, where its workgroups would be long in coming, keeps a launch per product, and gives the same."""
     from copilot_for_consensus_amd.models.encoder import EncoderModel
