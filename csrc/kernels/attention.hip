@@ -408,8 +408,9 @@ __global__ void __launch_bounds__(256, F8 ? 2 : 1) paged_decode_kernel(
 }
 
 // Merge of the P partition results of each (sequence, head) row, one wave a row: no barrier and no LDS.  The first sixteen
-// partitions (eight a half wave, four columns a lane) are asked for before their weights are known, and what is past the
-// last one is read again with weight zero: a loop of single loads for the remainder paid a trip to memory for each.
+// partitions (eight a half wave, four columns a lane) are asked for before their weights are known; past the last one that
+// one is read again and left out (as zeros: a weight of zero leaves an infinite sum in).  A loop of single loads for the
+// remainder paid a trip to memory for each.
 // us with the attention before it, one wave's barriers and single loads -> this: 24 sequences of 3 partitions 57.6 -> 54.8,
 // 12 of 6 23.3 -> 21.5, 5 of 4 8.5 -> 7.8, one of 44 14.1 -> 12.5 (of 8, whose loads were together before, 0.1).
 __global__ void __launch_bounds__(256) decode_combine_kernel(const float* __restrict__ part_o,
@@ -446,11 +447,12 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(const float* __rest
     for (int p0 = 0; p0 < np; p0 += 16) {
       if (p0) ask(p0);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {          // lanes past the last partition hold weight 0
+      for (int u = 0; u < 8; ++u) {
         const float w0 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), p0 + 2 * u));
         const float w1 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), p0 + 2 * u + 1));
         const float w = half ? w1 : w0;
-        O.x += w * v[u].x; O.y += w * v[u].y; O.z += w * v[u].z; O.w += w * v[u].w;
+        const f32x4_el o = p0 + 2 * u + half < np ? v[u] : f32x4_el{0.f, 0.f, 0.f, 0.f};
+        O.x += w * o.x; O.y += w * o.y; O.z += w * o.z; O.w += w * o.w;
       }
     }
   }

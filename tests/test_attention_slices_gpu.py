@@ -76,3 +76,24 @@ def test_merge_of_partitions(P):
     got = K.paged_decode_attention(q, kc, vc, bt, lens, D ** -0.5, part_blocks=-P, workspace=ws, out=out)
     # weights of a partition are rounded to bf16 from another maximum (2^-9 each, of values up to 4.5), results once more
     assert bool(((got.double() - want.double()).abs() <= 2.0 ** -8 * want.double().abs() + 2.0 ** -8).all())
+
+
+@pytest.mark.parametrize("P", [1, 2, 3, 5, 8, 15, 16, 17, 33])
+def test_merge_of_an_infinite_sum(P):
+    """An infinite value, in the last partition or in all, is infinite in the result, and alone there."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(P)
+    bt, blocks = _tables(2, 20 * 32, g)
+    kc = torch.randn(blocks, 1, 32, 128, device=DEV, generator=g).bfloat16()
+    vc = torch.randn(blocks, 1, 128, 32, device=DEV, generator=g).bfloat16()
+    q = torch.randn(2, 1, 128, device=DEV, generator=g).bfloat16()
+    lens = torch.tensor([640, 640], dtype=torch.int32, device=DEV)
+
+    def run(P):
+        return K.paged_decode_attention(q, kc, vc, bt, lens, 128 ** -0.5, part_blocks=-P).float()
+
+    vc[bt[0, -1].long(), 0, 3, 31] = float("inf")
+    vc[bt[1].long(), 0, 5] = float("-inf")
+    one, many = run(1), run(P)
+    assert one.isinf().sum() >= 2 and not bool(many.isnan().any())
+    assert torch.equal(many[one.isinf()], one[one.isinf()]) and torch.equal(many.isinf(), one.isinf())
