@@ -414,8 +414,8 @@ def argmax_keys(local: torch.Tensor, offset: int) -> torch.Tensor:
 
 @functools.lru_cache(maxsize=4096)
 def kv_partitions(B: int, heads: int, kv_heads: int, blocks: int) -> int:
-    """Partitions of each of B sequences of up to ``blocks`` cache blocks in the paged decode attention, by what a launch
-    takes in us, fitted to 620 measured (B of 1 .. 128, 2 .. 172 blocks, 1 .. 64 partitions of 8 KV heads): 3.3, 4.2 and
+    """Partitions of each of B sequences of ``blocks`` cache blocks in the paged decode attention, by what a launch
+    takes in us, fitted to 1048 measured (B of 1 .. 128, 2 .. 172 blocks, 1 .. 64 partitions of 8 KV heads): 3.3, 4.2 and
     0.045 per 32 rows and partition more for the merge, and what the busiest of 256 CUs, two workgroups each, reads: one
     block per wave takes 3.1 to 3.8 where a CU has one workgroup, 4.5 to 5.5 where some have two, 5 per full round of 512.
     A workgroup for every slot and a few more is a round more, and few keys are not worth a merge.  us of attention and
@@ -529,14 +529,21 @@ class DecoderModel:
         return PagedKVCache(self.cfg.layers, num_blocks, self.w.kv_heads, self.cfg.head_dim, device or self.w.device,
                             dtype=dtype or torch.bfloat16)
 
-    def decode_partitions(self, B: int, max_blocks: int) -> int:
-        """KV partitions per sequence of a B-row decode step over tables of ``max_blocks`` blocks
-        (:func:`kv_partitions`).  CFC_DECODE_WGS: the smallest P that gives so many workgroups instead."""
-        target = os.environ.get("CFC_DECODE_WGS")
-        if target:
-            return min(max(1, math.ceil(int(target) / max(1, B * self.w.kv_heads))), max(1, max_blocks // 2))
+    def decode_partitions(self, B: int, max_blocks: int, full: bool = True, fp8: bool = False) -> int:
+        """KV partitions per sequence of a B-row decode step over tables of ``max_blocks`` blocks: what fills the tables by
+        :func:`kv_partitions`, or the fewest that give 512 workgroups (CFC_DECODE_WGS: so many, and always these).
+
+        More than those pay where the contexts do fill the tables (``full``; 24 of 5500 keys 106 -> 92 us, 24 of 400 in tables
+        for 5500 15.1 -> 19.2), and were measured for 32 query and 8 key heads; fewer are right for any context up to the
+        table's, and for 1 to 10 key heads (0.53 to 1.05 of the time, 48 of 200 keys with one key head 1.10).  The 8-bit cache
+        has a kernel of its own, which the model does not fit (48 of 1500 35 -> 40 us)."""
+        fewest = min(max(1, math.ceil(int(os.environ.get("CFC_DECODE_WGS") or 512) / max(1, B * self.w.kv_heads))),
+                     max(1, max_blocks // 2))
+        if fp8 or os.environ.get("CFC_DECODE_WGS"):
+            return fewest
         seen = min(max_blocks, self.window // KV_BLOCK + 2) if self.window else max_blocks
-        return kv_partitions(B, self.w.heads, self.w.kv_heads, seen)
+        P = kv_partitions(B, self.w.heads, self.w.kv_heads, seen)
+        return P if full and (self.w.heads, self.w.kv_heads) == (32, 8) else min(P, fewest)
 
     def decode_workspace(self, B: int, P: int) -> int:
         """fp32 elements of the split-KV partials of a B-row decode step over P partitions."""

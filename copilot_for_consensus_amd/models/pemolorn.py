@@ -394,7 +394,7 @@ class PemolornModel:
                            "recur": lw["gru"].width if "gru" in lw else None})
         return GroupedCache(layers, num_blocks, sequences or min(num_blocks, DEFAULT_SEQUENCES), device or self.w.device, self.w.dtype)
 
-    def decode_partitions(self, B: int, max_blocks: int) -> int:
+    def decode_partitions(self, B: int, max_blocks: int, full: bool = True, fp8: bool = False) -> int:
         """Key slices per sequence of a B-row decode step over block tables ``max_blocks`` wide."""
         ctx = max_blocks * KV_BLOCK
         return max(A.decode_slices(B, a.H, a.G, a.D, a.mask.visible(ctx), self.w.dtype) for a in (lw["heads"] for lw in self.w.layers))

@@ -393,7 +393,7 @@ class TadolixModel:
     def _heads(self):
         return [lw["heads"] for lw in self.w.layers if "heads" in lw]
 
-    def decode_partitions(self, B: int, max_blocks: int) -> int:
+    def decode_partitions(self, B: int, max_blocks: int, full: bool = True, fp8: bool = False) -> int:
         """Key slices per sequence of a B-row decode step over block tables ``max_blocks`` wide."""
         ctx = max_blocks * KV_BLOCK
         return max([1] + [A.decode_slices(B, a.H, a.G, a.D, a.mask.visible(ctx), self.w.dtype) for a in self._heads()])

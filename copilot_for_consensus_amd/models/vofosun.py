@@ -303,7 +303,7 @@ class VofosunModel:
         return LatentKVCache([s.mixer.kv_rank for s in self.cfg.specs], num_blocks, self.cfg.hidden, tail_slots(self.cfg.taps),
                              device or self.w.device, self.w.dtype)
 
-    def decode_partitions(self, B: int, max_blocks: int) -> int:
+    def decode_partitions(self, B: int, max_blocks: int, full: bool = True, fp8: bool = False) -> int:
         """Key slices per sequence of a B-row decode step over block tables ``max_blocks`` wide."""
         if self.w.dtype != torch.bfloat16:
             return max(1, min(math.ceil(512 / B), max_blocks // 8))

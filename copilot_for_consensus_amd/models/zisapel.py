@@ -410,7 +410,7 @@ class ZisapelModel:
         """Keys a decoded token's 64-key tiles cover."""
         return min(ctx, m.window + 63) if m.window else ctx
 
-    def decode_partitions(self, B: int, max_blocks: int) -> int:
+    def decode_partitions(self, B: int, max_blocks: int, full: bool = True, fp8: bool = False) -> int:
         """Key slices per sequence of a B-row decode step over block tables ``max_blocks`` wide."""
         best = 1
         for _, m, H, rs, _ in self._windows():

@@ -154,8 +154,9 @@ class LLMEngine:
     # ------------------------------------------------------------------ helpers
     def _part_blocks(self, B, max_blocks):
         """Split-KV partitioning of the decode attention, as ``-P``: each sequence's own blocks in
-        P balanced ranges, P the model's pick (DecoderModel.decode_partitions)."""
-        return -self.model.decode_partitions(B, max_blocks)
+        P balanced ranges, P the model's pick for contexts that may be anything up to the tables
+        (DecoderModel.decode_partitions)."""
+        return -self.model.decode_partitions(B, max_blocks, full=False, fp8=getattr(self.kv, "dtype", None) == torch.float8_e4m3fn)
 
     def _i32(self, x):
         return torch.tensor(x, dtype=torch.int32, device=self.device)

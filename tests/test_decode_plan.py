@@ -1,4 +1,10 @@
 """How decode attention shares its work out (host rules)."""
+import math
+import types
+
+import pytest
+import torch
+
 
 def test_kv_partitions_fill_rounds_and_leave_short_contexts_whole():
     from copilot_for_consensus_amd.models.decoder import kv_partitions
@@ -11,3 +17,35 @@ def test_kv_partitions_fill_rounds_and_leave_short_contexts_whole():
     for B in (3, 5, 24, 48):
         P = kv_partitions(B, 32, 8, 176)
         assert B * 8 * P % 512 == 0 or B * 8 * P % 512 > 128     # not a round for a few workgroups
+
+
+def _model(heads, kv_heads, window=0):
+    import functools
+    from copilot_for_consensus_amd.models.decoder import DecoderModel
+    w = types.SimpleNamespace(heads=heads, kv_heads=kv_heads)
+    m = types.SimpleNamespace(w=w, window=window)
+    m.decode_partitions = functools.partial(DecoderModel.decode_partitions, m)
+    return m
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(32, 8), (4, 1), (8, 2), (64, 8), (40, 10)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_engines_partitions_are_no_slower_for_short_contexts(heads, kv_heads, dtype, monkeypatch):
+    """An engine's tables are as wide as its contexts may become: no more partitions than give 512 workgroups, whose launch
+    short contexts would pay for, and those of the 8-bit cache as they were."""
+    from copilot_for_consensus_amd.models.decoder import kv_partitions
+    from copilot_for_consensus_amd.runtime.engine import LLMEngine
+    monkeypatch.delenv("CFC_DECODE_WGS", raising=False)
+    m = _model(heads, kv_heads)
+    engine = types.SimpleNamespace(model=m, kv=types.SimpleNamespace(dtype=dtype))
+    for B in (1, 2, 3, 5, 12, 24, 48, 91, 128):
+        for blocks in (8, 24, 48, 128, 256, 344):
+            fewest = min(max(1, math.ceil(512 / (B * kv_heads))), max(1, blocks // 2))
+            P = -LLMEngine._part_blocks(engine, B, blocks)
+            assert 1 <= P <= fewest and (P == fewest or dtype == torch.bfloat16)
+            if dtype == torch.bfloat16:
+                assert P == min(fewest, kv_partitions(B, heads, kv_heads, blocks))
+                full = m.decode_partitions(B, blocks)
+                assert full == (kv_partitions(B, heads, kv_heads, blocks) if (heads, kv_heads) == (32, 8) else P)
+    monkeypatch.setenv("CFC_DECODE_WGS", "2048")
+    assert -LLMEngine._part_blocks(engine, 128, 88) == m.decode_partitions(128, 88) == math.ceil(2048 / (128 * kv_heads))
