@@ -78,14 +78,22 @@ class ExpertWeights:
         return (self.gu.numel() + self.down.numel()) * self.gu.element_size()
 
     def tile(self, pairs: int) -> int:
-        """Rows per tile for this many (token, choice) pairs: whole 256-row tiles once the experts fill them."""
+        """Rows per tile for this many (token, choice) pairs, evenly spread: whole 256-row tiles once the experts fill them."""
         if not self.packed:
             return ANY_TILE
         per = pairs / self.E
-        # Few rows of each expert: tiles of 16 or 32, lighter to stage and multiply than 64 mostly empty ones, while about
-        # three times an even share fits (an expert with more reads its matrices once per tile).  Two steps of 32 tokens,
-        # four each of 32 experts of 1024 x 4096: 64-row tiles 1643 us, 32 rows 1556
+        # Few rows of each expert: tiles of 16 or 32, lighter to stage and multiply than 64 mostly empty ones.  Two steps of 32
+        # tokens, four each of 32 experts of 1024 x 4096: 64-row tiles 1643 us, 32 rows 1556
         return 16 if per <= 5 else 32 if per <= 10 else 64 if per <= 96 else 128 if per <= 160 else 256
+
+
+def _least_tile(tokens: int) -> int:
+    """Rows per tile that few tokens may have at least.  An expert reads its matrices once per tile and has up to a row of every
+    token, however even the average: tiles of 16 and 32 rows are for so many tokens that the most chosen expert takes two.
+    us of a layer in tiles of 16 / 32 / 64, of 128 experts of 768 x 2048, eight a token: even choices of 32 tokens 186 / 194 /
+    216, all of them on the same experts 35 / 33 / 38; of 64 tokens 200 / 209 / 230 and 49 / 38 / 39; of 96 202 / 211 / 232 and 64 /
+    52 / 43.  Half the tokens of 64 on the same four of 32 experts of 1024 x 4096: 142 / 150 / 146, even ones 131 / 135 / 147."""
+    return 16 if tokens <= 32 else 32 if tokens <= 64 else 64
 
 
 def route(logits: Cols, r: Router) -> tuple[torch.Tensor, torch.Tensor]:
@@ -157,6 +165,8 @@ def experts(x, w: ExpertWeights, ids, glu: Glu = Glu()) -> tuple[torch.Tensor, t
         _req(ids, torch.int32, "ids")
         return _experts_gemv(x, w, ids, glu)
     tile = w.tile(ids.numel())
+    if w.packed:
+        tile = max(tile, _least_tile(ids.shape[0]))
     rows, pos, te = sort_rows(ids, w.E, tile)
     M = te.numel() * tile
     y = torch.empty(M, w.W, dtype=x.dtype, device=x.device)

@@ -59,6 +59,20 @@ def test_experts_rows_do_not_depend_on_the_tile(monkeypatch, T, E, tile):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T, top, E, tile", [(9, 1, 8, 16), (32, 4, 32, 16), (33, 2, 64, 32), (40, 4, 32, 32), (64, 1, 64, 32), (65, 2, 64, 64),
+                                             (128, 4, 128, 64), (64, 2, 4, 64)])
+def test_no_expert_takes_more_than_two_small_tiles(monkeypatch, T, top, E, tile):
+    """All tokens on the same experts: however few rows an expert has on average, its matrices are read twice at most."""
+    g = torch.Generator("cuda").manual_seed(T)
+    weights = moe.ExpertWeights(*((torch.randn(*s, device="cuda", generator=g) * 0.1).bfloat16() for s in ((E, 64, 64),) * 3))
+    seen, sort = [], moe.sort_rows
+    monkeypatch.setattr(moe, "sort_rows", lambda ids, experts, tile: seen.append(tile) or sort(ids, experts, tile))
+    ids = torch.arange(top, device="cuda").int().expand(T, top).contiguous()
+    y, pos = moe.experts(torch.randn(T, 64, device="cuda", generator=g).bfloat16(), weights, ids)
+    assert seen == [tile] and (tile == 64 or T <= 2 * tile) and bool(y[pos.long()].isfinite().all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T, top, E", [(256, 4, 5), (1023, 1, 3), (1025, 1, 3), (1024, 4, 7), (1025, 4, 32), (2731, 3, 1), (5000, 2, 1024)])
 def test_rows_of_pairs_about_a_step(T, top, E):
     """One step of 1024 pairs, a few more, whole and broken steps of 4096; choices without an expert among them."""
