@@ -38,7 +38,7 @@ __device__ __forceinline__ Vec<V> ldgain(const Gain& g, int c) {
   return r;
 }
 
-// FEW: no more rows than CUs, whose time is trips to memory; more rows keep to 64 VGPRs, two workgroups of 1024 a CU
+// FEW: FEW_ROWS at most, of one vector a thread; more rows keep to 64 VGPRs, two workgroups of 1024 a CU
 // (3222 rows of 4096: 58 us in 95 VGPRs, 42 in 64)
 template <typename ACT, int V, int NV, int BT, bool FEW>
 __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch, float* __restrict__ x, Gain next,
@@ -54,8 +54,8 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
     xv[k] = c < W ? ldv<V>(x + row + c) : zerov<V>();
   }
   // One vector a thread: the weights are asked for with the row, and not each after the sum before it (32 rows of 4096: 6.7 -> 5.9 us).
-  constexpr bool AHEAD = NV == 1 && FEW;
-  constexpr int F = FEW ? 8 : 4;
+  constexpr bool AHEAD = FEW;
+  constexpr int F = FEW || NV > 1 ? 8 : 4;
   Vec<V> ahead[AHEAD ? 4 : 1];
   if constexpr (AHEAD) {
     const int c = min((int)threadIdx.x * V, W - V);
@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
         const int c = (k * BT + threadIdx.x) * V;
         y[k] = z[k] = zerov<V>();
         if (c >= W) continue;
-        Slabs<V, F> sy, sz;
+        Slabs<V, F, NV == 1> sy, sz;
         sy.ask(b.y, b.ysplit, (int64_t)b.T * W, row + c);
         sz.ask(b.y2, b.y2split, (int64_t)b.T * W, row + c);
         sy.add(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
           s2 += z[k].v[e] * z[k].v[e];
         }
       }
-      block_sum2(s, s2, red, red2);
+      block_sum2<NV == 1 ? 16 : 1>(s, s2, red, red2);
       const float r1 = b.factor / sqrtf(s * inv_w + b.eps);
       const float r2 = b.factor / sqrtf(s2 * inv_w + b.eps);
       s = 0.f;
@@ -111,25 +111,31 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
         const int c = (k * BT + threadIdx.x) * V;
         y[k] = zerov<V>();
         if (c >= W) continue;
-        if (b.y) add_slabs<V>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
+        if (b.y) sum_slabs<V, 8, FEW>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
         if (b.mrow)
           for (int i0 = 0; i0 < b.top; i0 += 4) {         // four choices in flight (past the last: weight 0)
             Vec<V> r[4];
             float wt[4];
             int id[4], mr[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            auto index = [&](int u) {
               const int64_t i = (int64_t)t * b.top + min(i0 + u, b.top - 1);
               id[u] = b.ids[i];
               mr[u] = b.mrow[i];
-              wt[u] = b.mwt[i];
+              wt[u] = i0 + u < b.top ? b.mwt[i] : 0.f;
+            };
+            auto load = [&](int u) {
+              const ACT* src = id[u] >= b.experts ? reinterpret_cast<const ACT*>(b.own) + row
+                                                  : reinterpret_cast<const ACT*>(b.rows) + (size_t)mr[u] * W;
+              r[u] = ldv<V>(src + c);
+            };
+            if constexpr (NV == 1) {               // all indexes, then all rows
+#pragma unroll
+              for (int u = 0; u < 4; ++u) index(u);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-              const ACT* src = id[u] >= b.experts ? reinterpret_cast<const ACT*>(b.own) + row
-                                                  : reinterpret_cast<const ACT*>(b.rows) + (size_t)mr[u] * W;
-              if (i0 + u >= b.top) wt[u] = 0.f;
-              r[u] = ldv<V>(src + c);
+              if constexpr (NV != 1) index(u);
+              load(u);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
@@ -140,7 +146,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
         for (int e = 0; e < V; ++e) s += y[k].v[e] * y[k].v[e];
       }
     }
-    const float r = 1.f / sqrtf(block_sum(s, red) * inv_w + b.eps);
+    const float r = 1.f / sqrtf(block_sum<NV == 1 ? 16 : 1>(s, red) * inv_w + b.eps);
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int c = (k * BT + threadIdx.x) * V;
@@ -157,7 +163,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
   for (int k = 0; k < NV; ++k)
 #pragma unroll
     for (int e = 0; e < V; ++e) s += xv[k].v[e] * xv[k].v[e];
-  const float r = 1.f / sqrtf(block_sum(s, red2) * inv_w + b.eps);
+  const float r = 1.f / sqrtf(block_sum<NV == 1 ? 16 : 1>(s, red2) * inv_w + b.eps);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int c = (k * BT + threadIdx.x) * V;
@@ -175,7 +181,7 @@ int branch_go(hipStream_t s, const BranchIn& b, int branch, float* x, Gain next,
   const int vecs = (b.W + V - 1) / V;
 #define GO(NV, BT)                                                                                            \
   do {                                                                                                        \
-    if (b.T <= 256) branch_norm_kernel<ACT, V, NV, BT, true><<<b.T, BT, 0, s>>>(b, branch, x, next, (ACT*)h); \
+    if (NV == 1 && b.T <= FEW_ROWS) branch_norm_kernel<ACT, V, NV, BT, NV == 1><<<b.T, BT, 0, s>>>(b, branch, x, next, (ACT*)h); \
     else branch_norm_kernel<ACT, V, NV, BT, false><<<b.T, BT, 0, s>>>(b, branch, x, next, (ACT*)h);           \
   } while (0)
   ROW_SHAPES(GO, vecs);

@@ -106,7 +106,8 @@ struct BranchArgs {
 // MODE 0: prompt rows; 1: decoded rows (shift_mix of the next layer follows); 2: decoded rows, shift only
 // (b.y == null, b.y2 == null, b.ym == null: no branch, the first layer's).  x is updated in place.
 enum { GN_PROMPT = 0, GN_SHIFT = 1 };
-template <typename ACT, int V, int NV, int BT, int MODE>
+// FEW: FEW_ROWS at most, of one vector a thread.
+template <typename ACT, int V, int NV, int BT, int MODE, bool FEW>
 __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __restrict__ x, ACT* __restrict__ h,
                                                        float* __restrict__ prev, const int32_t* __restrict__ meta,
                                                        const int32_t* __restrict__ positions, ShiftArgs a,
@@ -135,7 +136,7 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
       if (acts && pos >= 2) xpp[k] = ldv<V>(st + (size_t)(pos & 1) * W + c);
     }
   }
-  // one vector a thread: the weights with the row, and not after the sums before them; so too what the last rows' indexes say
+  // few rows: the weights with the row, and not after the sums before them; so too what the last rows' indexes say
   int m = 0;
   if constexpr (MODE == GN_PROMPT) {
     if (prev) {
@@ -144,7 +145,7 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
     }
   }
   Vec<V> gain, gb1;
-  if (NV == 1 && branch) {
+  if (FEW && branch) {
     gain = ldv<V>(b.norm_w + min((int)threadIdx.x * V, W - V));
     gb1 = ldv<V>(b.gbias + min((int)threadIdx.x * V, W - V));
   }
@@ -157,9 +158,10 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
       y[k] = zerov<V>();
       if (c >= W) continue;
       Vec<V> g = zerov<V>();
-      if (b.gate_act) g = ldv<V>(reinterpret_cast<const ACT*>(b.gate) + (size_t)t * b.gld + c);
-      if (b.y) add_slabs<V>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
-      if (b.y2) add_slabs<V>(y[k], b.y2, b.y2split, (int64_t)b.T * W, row + c);
+      auto gate = [&] { g = ldv<V>(reinterpret_cast<const ACT*>(b.gate) + (size_t)t * b.gld + c); };
+      if (NV <= 4 && b.gate_act) gate();          // ahead of the sums, where there are registers for it
+      if (b.y) sum_slabs<V, 8, FEW>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
+      if (b.y2) sum_slabs<V, 8, FEW>(y[k], b.y2, b.y2split, (int64_t)b.T * W, row + c);
       if (b.ym)
         for (int i = 0; i < b.top; ++i) {
           const float wt = b.mwt[(size_t)t * b.top + i];
@@ -167,15 +169,16 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
 #pragma unroll
           for (int e = 0; e < V; ++e) y[k].v[e] += wt * r.v[e];
         }
-      if (!b.gate_act) add_slabs<V>(g, reinterpret_cast<const float*>(b.gate), b.gsplit, b.gplane, (size_t)t * b.gld + c);
-      const Vec<V> gb = NV == 1 ? gb1 : ldv<V>(b.gbias + c);
+      if (NV > 4 && b.gate_act) gate();
+      if (!b.gate_act) sum_slabs<V, 8, FEW>(g, reinterpret_cast<const float*>(b.gate), b.gsplit, b.gplane, (size_t)t * b.gld + c);
+      const Vec<V> gb = FEW ? gb1 : ldv<V>(b.gbias + c);
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         y[k].v[e] *= 1.f / (1.f + expf(-(g.v[e] + gb.v[e])));
         s += y[k].v[e];
       }
     }
-    const float mean = block_sum(s, red) / (float)W;
+    const float mean = block_sum<NV == 1 ? 16 : 1>(s, red) / (float)W;
     float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < NV; ++k)
@@ -185,7 +188,7 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
           y[k].v[e] -= mean;
           ss += y[k].v[e] * y[k].v[e];
         }
-    const float r = 1.f / sqrtf(block_sum(ss, red) / (float)W + b.eps);
+    const float r = 1.f / sqrtf(block_sum<NV == 1 ? 16 : 1>(ss, red) / (float)W + b.eps);
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int c = (k * BT + threadIdx.x) * V;
@@ -193,7 +196,7 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
       if constexpr (MODE == GN_PROMPT) {
         if (prev && (m & META_TAIL)) stv<V>(prev + ((size_t)(m >> META_SLOT) * 2 + (pos & 1)) * W + c, xv[k]);
       }
-      const Vec<V> w = NV == 1 ? gain : ldv<V>(b.norm_w + c);
+      const Vec<V> w = FEW ? gain : ldv<V>(b.norm_w + c);
 #pragma unroll
       for (int e = 0; e < V; ++e) xv[k].v[e] += y[k].v[e] * r * w.v[e];
       stv<V>(x + row + c, xv[k]);
@@ -227,7 +230,7 @@ __global__ void __launch_bounds__(BT) final_norm_kernel(const float* __restrict_
 #pragma unroll
     for (int e = 0; e < V; ++e) s += y[k].v[e];
   }
-  const float mean = block_sum(s, red) / (float)W;
+  const float mean = block_sum<NV == 1 ? 16 : 1>(s, red) / (float)W;
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < NV; ++k)
@@ -237,7 +240,7 @@ __global__ void __launch_bounds__(BT) final_norm_kernel(const float* __restrict_
         y[k].v[e] -= mean;
         ss += y[k].v[e] * y[k].v[e];
       }
-  const float r = 1.f / sqrtf(block_sum(ss, red) / (float)W + eps);
+  const float r = 1.f / sqrtf(block_sum<NV == 1 ? 16 : 1>(ss, red) / (float)W + eps);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int c = (k * BT + threadIdx.x) * V;
@@ -253,10 +256,16 @@ template <typename ACT, int V, int MODE>
 int gated_go(hipStream_t s, int n, const BranchArgs& b, float* x, void* h, float* prev, const int32_t* meta,
              const int32_t* positions, const ShiftArgs& a, const int32_t* slots, void* acts) {
   const int vecs = (b.W + V - 1) / V;
-#define GO(NV, BT) \
-  gated_norm_kernel<ACT, V, NV, BT, MODE><<<n, BT, 0, s>>>(b, x, (ACT*)h, prev, meta, positions, a, slots, (ACT*)acts)
+#define GN_GO(NV, BT, FEW) \
+  gated_norm_kernel<ACT, V, NV, BT, MODE, FEW><<<n, BT, 0, s>>>(b, x, (ACT*)h, prev, meta, positions, a, slots, (ACT*)acts)
+#define GO(NV, BT)                                               \
+  do {                                                           \
+    if (NV == 1 && n <= FEW_ROWS) GN_GO(NV, BT, NV == 1);        \
+    else GN_GO(NV, BT, false);                                   \
+  } while (0)
   ROW_SHAPES(GO, vecs);
 #undef GO
+#undef GN_GO
   return CFC_CHECK_LAUNCH();
 }
 

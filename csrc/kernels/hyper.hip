@@ -39,35 +39,40 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
   const float* xr = a.x + t * a.ldx;
   // All that a row's first vectors need is asked for before anything is waited for, what waits for an index last (5 rows of
   // 4096 in 4 streams: 6.9 -> 6.2 us, of which 300 KB a row through one CU take most).
-  constexpr int MX = SM * SM + 2 * SM, MI = (MX + BT - 1) / BT;
-  float mv[MI];
-#pragma unroll
-  for (int j = 0; j < MI; ++j) {
-    const int i = threadIdx.x + j * BT, s = i / SM, k = i % SM;
-    const float* p = xr;                       // some address that there is
-    if (k < S) {
-      if (s < S && a.y) p = a.mix + s * S + k;
-      else if (s == SM && a.y) p = a.out + k;
-      else if (s == SM + 1 && a.in) p = a.in + k;
-    }
-    mv[j] = *p;
+  constexpr bool ONE = NV == 1 && SM <= 4;     // else the registers are wanted for more vectors or streams
+  constexpr int MX = SM * SM + 2 * SM;
+  static_assert(!ONE || MX <= BT, "");
+  float mv = 0.f;
+  auto weight = [&](int i) {                   // past S: 0
+    const int s = i / SM, k = i % SM;
+    if (k >= S) return 0.f;
+    if (s < SM) return s >= S ? 0.f : a.y ? a.mix[s * S + k] : s == k ? 1.f : 0.f;
+    if (s == SM) return a.y ? a.out[k] : 0.f;
+    return a.in ? a.in[k] : 1.f;
+  };
+  if constexpr (ONE) {
+    if (threadIdx.x < MX) mv = weight(threadIdx.x);
+  } else {
+    for (int i = threadIdx.x; i < MX; i += BT) mx[i] = weight(i);
   }
   constexpr int PRE = NV == 1 && V == 4 ? 3 : 0;
   const int back = a.taps - 1;
   const bool ahead = PRE > 0 && back <= PRE;
   const int c0 = min((int)threadIdx.x * V, W - V);
   Vec<V> u[NV], x[SM], y = zerov<V>(), past[PRE ? PRE : 1], cw[PRE ? PRE + 1 : 1], gain;
-  constexpr bool ONE = NV == 1 && SM <= 4;     // else the registers are wanted for more vectors or streams
-  Slabs<V, ONE ? 8 : 4> slabs;
+  Slabs<V, 8, ONE> slabs;
   float ss = 0.f;
   auto ask = [&](int c) {
 #pragma unroll
     for (int s = 0; s < SM; ++s) x[s] = ldv<V>(xr + min(s, S - 1) * a.lds + c);
-    if (ONE && a.y) slabs.ask(a.y, a.split, (int64_t)a.T * W, (size_t)t * W + c);
+    if (!a.y) return;
+    y = zerov<V>();
+    slabs.ask(a.y, a.split, (int64_t)a.T * W, (size_t)t * W + c);
+    if constexpr (!ONE) slabs.add(y, a.y, a.split, (int64_t)a.T * W, (size_t)t * W + c);
   };
-  ask(c0);
+  if constexpr (ONE) ask(c0);
   if constexpr (PRE > 0) {
-    if (mode != HN_RSTD) gain = ldv<V>(a.w + c0);
+    if (ONE && mode != HN_RSTD) gain = ldv<V>(a.w + c0);
     if (mode == HN_CONV && ahead)
 #pragma unroll
       for (int d = 0; d <= PRE; ++d) cw[d] = ldv<V>(a.cw + (size_t)max(back - d, 0) * W + c0);
@@ -78,17 +83,8 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
     if (mode == HN_CONV && ahead)
 #pragma unroll
       for (int d = 1; d <= PRE; ++d) past[d - 1] = d <= back && d <= pos ? ldv<V>(tail + (size_t)((pos - d) % a.ring) * W + c0) : zerov<V>();
-#pragma unroll
-  for (int j = 0; j < MI; ++j) {
-    const int i = threadIdx.x + j * BT, s = i / SM, k = i % SM;          // past S: weight 0
-    float v = 0.f;
-    if (k < S) {
-      if (s < SM) v = s >= S ? 0.f : a.y ? mv[j] : s == k ? 1.f : 0.f;
-      else if (s == SM) v = a.y ? mv[j] : 0.f;
-      else v = a.in ? mv[j] : 1.f;
-    }
-    if (i < MX) mx[i] = v;
-  }
+  if constexpr (!ONE) ask(c0);
+  if (ONE && threadIdx.x < MX) mx[threadIdx.x] = mv;
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
@@ -97,9 +93,7 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
     if (c >= W) continue;
     if (k) ask(c);
     if (a.y) {
-      y = zerov<V>();
-      if constexpr (!ONE) slabs.ask(a.y, a.split, (int64_t)a.T * W, (size_t)t * W + c);
-      slabs.add(y, a.y, a.split, (int64_t)a.T * W, (size_t)t * W + c);
+      if constexpr (ONE) slabs.add(y, a.y, a.split, (int64_t)a.T * W, (size_t)t * W + c);
 #pragma unroll
       for (int q = 0; q < SM; ++q) {
         if (q >= S) break;
@@ -123,7 +117,7 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
 #pragma unroll
     for (int e = 0; e < V; ++e) ss += u[k].v[e] * u[k].v[e];
   }
-  const float r = 1.f / sqrtf(block_sum(ss, red) / (float)W + a.eps);
+  const float r = 1.f / sqrtf(block_sum<NV == 1 ? 16 : 1>(ss, red) / (float)W + a.eps);
   if (mode == HN_RSTD) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
@@ -138,7 +132,7 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
     const int c = (k * BT + threadIdx.x) * V;
     if (c >= W) continue;
     Vec<V> g, n;
-    if constexpr (PRE > 0) g = gain;
+    if constexpr (PRE > 0 && ONE) g = gain;
     else g = ldv<V>(a.w + c);
 #pragma unroll
     for (int e = 0; e < V; ++e) n.v[e] = u[k].v[e] * r * g.v[e];

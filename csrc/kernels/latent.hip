@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(BT) latent_norm_kernel(const float* __restrict
 #pragma unroll
     for (int e = 0; e < V; ++e) x[k][e] = 0.f;
     if (c >= N) continue;
-    Slabs<V, NV == 1 ? 8 : 4> slabs;
+    Slabs<V, 8, NV == 1> slabs;
     slabs.ask(src, split, (int64_t)plane, c);
     if constexpr (NV == 1) {          // asked for with the row
 #pragma unroll
@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(BT) latent_norm_kernel(const float* __restrict
     if (c < NQ) sq += ss;
     else sc += ss;
   }
-  block_sum2(sq, sc, red, red2);
+  block_sum2<NV == 1 ? 16 : 1>(sq, sc, red, red2);
   const float rq = 1.f / sqrtf(sq / (float)NQ + eps), rc = 1.f / sqrtf(sc / (float)NC + eps);
   ACT* dst = cache + (size_t)slot * RS;
 #pragma unroll

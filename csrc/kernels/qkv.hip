@@ -34,8 +34,7 @@ struct QkvArgs {
 
 template <typename ACT, int V>
 __device__ __forceinline__ Vec<V> qkv_ld(const QkvArgs& a, int64_t t, int c) {
-  ColsIn<ACT, V> in;
-  in.ask(a.p, a.split, a.plane, t * a.ld + c);
+  ColsIn<ACT, V, 8, false> in;
   return in.get(a.p, a.split, a.plane, t * a.ld + c);
 }
 
@@ -82,7 +81,7 @@ __global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a) {
       for (int k = 0; k < NV; ++k) {
         const int c = min((k * BT + tid) * V, C - V);
         Vec<V> o[MAX_BACK], w[MAX_BACK + 1];
-        ColsIn<ACT, V> in;
+        ColsIn<ACT, V, 8, NV == 1> in;
         in.ask(a.p, a.split, a.plane, t * a.ld + c0 + c);
 #pragma unroll
         for (int d = 0; d <= MAX_BACK; ++d) w[d] = ldv<V>(a.conv + (size_t)max(back - d, 0) * allc + c0 + c);
@@ -137,7 +136,7 @@ __global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a) {
     }
     const int hv = hd / V;
     if (!a.per_head) {
-      const float v = 1.f / sqrtf(block_sum(all, red) / (float)C + a.eps);
+      const float v = 1.f / sqrtf(block_sum<NV == 1 ? 16 : 1>(all, red) / (float)C + a.eps);
 #pragma unroll
       for (int k = 0; k < NV; ++k) r[k] = v;
     } else if (hv <= 64 && (hv & (hv - 1)) == 0) {     // a head is a run of lanes

@@ -51,53 +51,82 @@ __device__ __forceinline__ Vec<V> zerov() {
   return r;
 }
 
-// Sums of fp32 k-slice slabs in two steps: the first F slabs are asked for, and added, in their order, where the sum is
-// needed.  No load waits for another: a loop over the slabs made all that was asked for before it arrive first, and a row
-// that one workgroup works on pays a trip to memory, 0.7 us, for each such wait.
+// y += slabs of row offset `off`, F in flight (past the last: re-read, not added)
 template <int V, int F = 8>
-struct Slabs {
-  Vec<V> a[F];
-  __device__ __forceinline__ void ask(const float* p, int split, int64_t plane, size_t off) {
+__device__ __forceinline__ void add_slabs(Vec<V>& y, const float* p, int split, int64_t plane, size_t off, int first = 0) {
+  if (split == 1) {
+    const Vec<V> a = ldv<V>(p + off);
 #pragma unroll
-    for (int u = 0; u < F; ++u) a[u] = u == 0 || u < split ? ldv<V>(p + u * plane + off) : zerov<V>();
+    for (int e = 0; e < V; ++e) y.v[e] += a.v[e];
+    return;
   }
-  __device__ __forceinline__ void add(Vec<V>& y, const float* p, int split, int64_t plane, size_t off) const {
+  for (int p0 = first; p0 < split; p0 += F) {
+    Vec<V> a[F];
+#pragma unroll
+    for (int u = 0; u < F; ++u) a[u] = ldv<V>(p + (size_t)min(p0 + u, split - 1) * plane + off);
 #pragma unroll
     for (int u = 0; u < F; ++u)
-      if (u < split)
+      if (p0 + u < split)
 #pragma unroll
         for (int e = 0; e < V; ++e) y.v[e] += a[u].v[e];
-    for (int p0 = F; p0 < split; p0 += F) {          // past the last: re-read, not added
-      Vec<V> b[F];
+  }
+}
+
+// The same sum in two steps, in its order: the first F slabs are asked for, and added where the sum is needed.  No load waits
+// for another: a loop over the slabs made all that was asked for before it arrive first, and a row that one workgroup works
+// on pays a trip to memory, 0.7 us, for each such wait.  Only where a thread has one vector (AHEAD): rows of more want their
+// registers for these, and asking ahead was slower (5 rows of 8192 gated 6.5 -> 8.5 us, of 20480 34 -> 43).
+template <int V, int F = 8, bool AHEAD = true>
+struct Slabs {
+  Vec<V> a[AHEAD ? F : 1];
+  __device__ __forceinline__ void ask(const float* p, int split, int64_t plane, size_t off) {
+    if constexpr (AHEAD) {
+      a[0] = ldv<V>(p + off);
+      if (split == 1) return;
 #pragma unroll
-      for (int u = 0; u < F; ++u) b[u] = ldv<V>(p + (size_t)min(p0 + u, split - 1) * plane + off);
+      for (int u = 1; u < F; ++u) a[u] = u < split ? ldv<V>(p + u * plane + off) : zerov<V>();
+    }
+  }
+  __device__ __forceinline__ void add(Vec<V>& y, const float* p, int split, int64_t plane, size_t off) const {
+    if constexpr (AHEAD) {
 #pragma unroll
-      for (int u = 0; u < F; ++u)
-        if (p0 + u < split)
+      for (int e = 0; e < V; ++e) y.v[e] += a[0].v[e];
+      if (split == 1) return;
 #pragma unroll
-          for (int e = 0; e < V; ++e) y.v[e] += b[u].v[e];
+      for (int u = 1; u < F; ++u)
+        if (u < split)
+#pragma unroll
+          for (int e = 0; e < V; ++e) y.v[e] += a[u].v[e];
+      add_slabs<V, F>(y, p, split, plane, off, F);
+    } else {
+      add_slabs<V, F>(y, p, split, plane, off);
     }
   }
 };
 
-// y += slabs of row offset `off`
-template <int V>
-__device__ __forceinline__ void add_slabs(Vec<V>& y, const float* p, int split, int64_t plane, size_t off) {
-  Slabs<V> s;
+// both steps at once
+template <int V, int F, bool AHEAD>
+__device__ __forceinline__ void sum_slabs(Vec<V>& y, const float* p, int split, int64_t plane, size_t off) {
+  Slabs<V, F, AHEAD> s;
   s.ask(p, split, plane, off);
   s.add(y, p, split, plane, off);
 }
 
 // V columns of a product that leaves activations (split 0) or fp32 slabs, in the same two steps.
-template <typename ACT, int V, int F = 8>
+template <typename ACT, int V, int F = 8, bool AHEAD = true>
 struct ColsIn {
-  Slabs<V, F> s;
+  Slabs<V, F, AHEAD> s;
   __device__ __forceinline__ void ask(const void* p, int split, int64_t plane, int64_t o) {
-    if (split == 0) s.a[0] = ldv<V>(reinterpret_cast<const ACT*>(p) + o);
-    else s.ask(reinterpret_cast<const float*>(p), split, plane, (size_t)o);
+    if constexpr (AHEAD) {
+      if (split == 0) s.a[0] = ldv<V>(reinterpret_cast<const ACT*>(p) + o);
+      else s.ask(reinterpret_cast<const float*>(p), split, plane, (size_t)o);
+    }
   }
   __device__ __forceinline__ Vec<V> get(const void* p, int split, int64_t plane, int64_t o) const {
-    if (split == 0) return s.a[0];
+    if (split == 0) {
+      if constexpr (AHEAD) return s.a[0];
+      else return ldv<V>(reinterpret_cast<const ACT*>(p) + o);
+    }
     Vec<V> y = zerov<V>();
     s.add(y, reinterpret_cast<const float*>(p), split, plane, (size_t)o);
     return y;
@@ -105,6 +134,9 @@ struct ColsIn {
 };
 
 }  // namespace
+
+// Up to so many rows, no more than there are CUs, a row's time is its trips to memory; of more, what the registers let a CU hold.
+constexpr int FEW_ROWS = 256;
 
 // NV, BT for rows of W channels in vectors of V
 #define ROW_SHAPES(GO, vecs)           \

@@ -101,18 +101,17 @@ struct DepthArgs {
 };
 
 // one workgroup of BT threads per row; a thread holds NV vectors of V channels, NV * V * BT >= W
-// (DN_RSTD, a prompt's rows: two workgroups of 1024 a CU)
-template <typename ACT, int V, int NV, int MODE, int BT>
-__global__ void __launch_bounds__(BT, MODE == DN_RSTD ? 8 : 1) depth_norm_kernel(DepthArgs a, ACT* __restrict__ h1, ACT* __restrict__ h2) {
+// (FEW: FEW_ROWS at most, of one vector a thread)
+template <typename ACT, int V, int NV, int MODE, int BT, bool FEW>
+__global__ void __launch_bounds__(BT) depth_norm_kernel(DepthArgs a, ACT* __restrict__ h1, ACT* __restrict__ h2) {
   __shared__ float red[16];
   const int b = blockIdx.x, t = a.rows ? a.rows[b] : b;
   const size_t row = (size_t)t * a.W, plane = (size_t)a.T * a.W;
   Vec<V> x[NV];
   float ss = 0.f;
-  // One vector a thread: all is asked for before anything is waited for (24 rows of 4096: 9.6 -> 9.4
-  // us, 370 KB a row through one CU).
+  // ONE: all is asked for before anything is waited for (24 rows of 4096: 9.6 -> 9.4 us, 370 KB a row through one CU).
   constexpr int PRE = MODE == DN_CONV && NV == 1 ? 4 : 0;
-  constexpr bool ONE = NV == 1;
+  constexpr bool ONE = FEW || (NV == 1 && MODE == DN_CONV);
   Vec<V> past[PRE ? PRE : 1], k1[PRE ? PRE : 1], k2[PRE ? PRE : 1], gw;
   const bool pre_ok = PRE > 0 && a.taps <= PRE;
   int pos = 0;
@@ -149,12 +148,12 @@ __global__ void __launch_bounds__(BT, MODE == DN_RSTD ? 8 : 1) depth_norm_kernel
     Vec<V> cur = ldv<V>(a.x_in + row + c);
     if (a.part) {
       Vec<V> pre, bias, hist[4];
-      float wj[4];
-      const float an = a.dwa[a.n];
-      Slabs<V, ONE ? 8 : 4> slabs;       // many rows: fewer registers, more rows a CU
+      float wj[4], an;
+      if constexpr (ONE) an = a.dwa[a.n];
+      Slabs<V, ONE ? 8 : 4, ONE> slabs;
       slabs.ask(a.part, a.split, (int64_t)plane, row + c);
       if (a.pre) pre = ldv<V>(a.pre + row + c);
-      if (a.bias) bias = ldv<V>(a.bias + c);
+      if (ONE && a.bias) bias = ldv<V>(a.bias + c);
       auto ask_hist = [&](int j) {               // four rows of the history in flight (past the last: again, weight 0)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -162,24 +161,42 @@ __global__ void __launch_bounds__(BT, MODE == DN_RSTD ? 8 : 1) depth_norm_kernel
           wj[u] = j + u < a.n ? a.dwa[j + u] : 0.f;
         }
       };
-      if (a.j0 < a.n) ask_hist(a.j0);
+      if (ONE && a.j0 < a.n) ask_hist(a.j0);
       if constexpr (ONE) ask_rest();
       slabs.add(cur, a.part, a.split, (int64_t)plane, row + c);
       ask_second();
       if (a.bias) {
+        if constexpr (!ONE) bias = ldv<V>(a.bias + c);
 #pragma unroll
         for (int e = 0; e < V; ++e) cur.v[e] += bias.v[e];
       }
       if (MODE != DN_NORM) stv<V>(a.hist + (size_t)a.n * plane + row + c, cur);   // DN_NORM: nothing reads it again
       Vec<V> acc;
+      if constexpr (ONE) {
 #pragma unroll
-      for (int e = 0; e < V; ++e) acc.v[e] = an * cur.v[e];
-      for (int j = a.j0; j < a.n; j += 4) {
-        if (j != a.j0) ask_hist(j);
+        for (int e = 0; e < V; ++e) acc.v[e] = an * cur.v[e];
+        for (int j = a.j0; j < a.n; j += 4) {
+          if (j != a.j0) ask_hist(j);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+          for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int e = 0; e < V; ++e) acc.v[e] += wj[u] * hist[u].v[e];
+            for (int e = 0; e < V; ++e) acc.v[e] += wj[u] * hist[u].v[e];
+        }
+      } else {                                   // its own loop: through the other's registers 2000 rows of 8192 took 72 us, so 66
+        an = a.dwa[a.n];
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc.v[e] = an * cur.v[e];
+        for (int j = a.j0; j < a.n; j += 4) {
+          Vec<V> y[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) y[u] = ldv<V>(a.hist + (size_t)min(j + u, a.n - 1) * plane + row + c);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const float w = j + u < a.n ? a.dwa[j + u] : 0.f;
+#pragma unroll
+            for (int e = 0; e < V; ++e) acc.v[e] += w * y[u].v[e];
+          }
+        }
       }
       if (a.pre) {
 #pragma unroll
@@ -195,7 +212,7 @@ __global__ void __launch_bounds__(BT, MODE == DN_RSTD ? 8 : 1) depth_norm_kernel
 #pragma unroll
     for (int e = 0; e < V; ++e) ss += cur.v[e] * cur.v[e];
   }
-  ss = block_sum(ss, red);
+  ss = block_sum<NV == 1 ? 16 : 1>(ss, red);
   const float rstd = 1.f / sqrtf(ss / (float)a.W + a.eps);
   if constexpr (MODE == DN_RSTD) {
     if (threadIdx.x == 0) a.rstd[t] = rstd;
@@ -452,7 +469,11 @@ __global__ void __launch_bounds__(256) softcap_kernel(float* __restrict__ x, siz
 // few rows (a decode step): the widest workgroup the row fills, one vector per thread
 template <typename ACT, int V, int MODE>
 int depth_nv(int W, dim3 grid, hipStream_t s, const DepthArgs& a, void* h1, void* h2) {
-#define DN_GO(NV, BT) depth_norm_kernel<ACT, V, NV, MODE, BT><<<grid, BT, 0, s>>>(a, (ACT*)h1, (ACT*)h2)
+#define DN_GO(NV, BT)                                                                                                       \
+  do {                                                                                                                      \
+    if (NV == 1 && grid.x <= FEW_ROWS) depth_norm_kernel<ACT, V, NV, MODE, BT, NV == 1><<<grid, BT, 0, s>>>(a, (ACT*)h1, (ACT*)h2); \
+    else depth_norm_kernel<ACT, V, NV, MODE, BT, false><<<grid, BT, 0, s>>>(a, (ACT*)h1, (ACT*)h2);                          \
+  } while (0)
   const int vecs = (W + V - 1) / V;
   const bool few = grid.x <= 512 && vecs > 256;
   if (vecs <= 256) DN_GO(1, 256);

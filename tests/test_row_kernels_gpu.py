@@ -66,3 +66,43 @@ def test_experts_chosen_among_equals(E, top, kind):
     torch.testing.assert_close(w[:, :n].double(), s.gather(1, order)[:, :n], rtol=2.0 ** -21, atol=0)      # an exponential of 2 ulp
     if kind == "few":            # nothing is left to choose
         assert bool((ids[:, n:] == E - 1).all()) and bool((w[:, n:] == 0).all())
+
+
+@pytest.mark.parametrize("split", [1, 3, 9])
+@pytest.mark.parametrize("W", [1, 1020, 4096, 4100, 16384, 16400])
+def test_rows_of_few_and_of_many_are_the_same(W, split):
+    """256 rows ask for all they need at once, 257 do not, nor do rows wider than one vector a thread: the same sums."""
+    from copilot_for_consensus_amd.ops import branch, gated, stream
+    from copilot_for_consensus_amd.ops.cols import Cols
+    g = torch.Generator(device=DEV).manual_seed(W + split)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    T, bf = 257, torch.bfloat16
+    x, y, y2, gate, hist = rnd(T, W), rnd(split, T, W), rnd(split, T, W), rnd(split, T, W), rnd(5, T, W)
+    gain, w1, w2, bias, dwa = rnd(W), rnd(W), rnd(W), rnd(W), torch.rand(6, device=DEV, generator=g)
+    rows, own = rnd(4 * T, W).to(bf), rnd(T, W).to(bf)
+    pos = torch.randint(0, 4 * T, (T, 5), device=DEV, generator=g).int()
+    ids, wt = torch.randint(0, 5, (T, 5), device=DEV, generator=g).int(), torch.rand(T, 5, device=DEV, generator=g)
+
+    def results(n):
+        c = lambda t: t[..., :n, :].contiguous()  # noqa: E731
+        out = []
+
+        def norm(fn, *a, **kw):
+            s, h = c(x).clone(), torch.empty(n, W, device=DEV, dtype=bf)
+            fn(s, h, *a, **kw)
+            out.extend([s, h])
+
+        norm(lambda s, h: branch.branch_norm(s, branch.Branch(gain, 1e-6, y=c(y)), w1, 1e-6, h))
+        norm(lambda s, h: branch.branch_norm(s, branch.Branch(gain, 1e-6, y=c(y), w=w1, y2=c(y2), w2=w2), w2, 1e-6, h))
+        norm(lambda s, h: branch.branch_norm(s, branch.Branch(gain, 1e-6, y=c(y), routed=(rows, c(pos), c(wt), c(ids), 4, c(own))), w1, 1e-6, h))
+        for z in (Cols(c(gate)), Cols(c(gate)[0].to(bf))):
+            norm(lambda s, h: gated.gated_norm(s, gated.Branch(z, bias, w1, 1e-6, y=c(y), y2=c(y2)), bf, h))
+            norm(lambda s, h: gated.gated_shift(s, gated.Branch(z, bias, w1, 1e-6, y=c(y)), bf, h))
+        up = stream.Update(c(y), bias, dwa, 5)
+        a, r = torch.empty(n, W, device=DEV), torch.empty(n, device=DEV)
+        stream.depth_stats(c(x), c(hist).clone(), stream.Update(c(y), bias, dwa[:5], 4), 1e-6, a, r)
+        out.extend([a, r[:, None], stream.depth_norm(c(x), torch.cat([c(hist), c(x)[None]]), up, w1, 1e-6, bf)])
+        return out
+
+    for few, many in zip(results(T - 1), results(T)):
+        assert torch.equal(few, many[:T - 1])
