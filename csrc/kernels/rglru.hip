@@ -310,7 +310,7 @@ __global__ void __launch_bounds__(256, KS <= 4 ? 4 : KS <= 8 ? 3 : 2) rglru_scan
 // ------------------------------------------------------------------------------------------ one token per sequence
 // u of up to 16 rows x a block's columns into LDS (row stride ldu), the block's raw inputs into the state by the workgroup
 // whose channels n0 .. n1 they are
-template <typename ACT, typename LT, int V>
+template <typename ACT, typename LT, int V, bool AHEAD>
 __device__ __forceinline__ void step_conv(const LruArgs& a, int b0, int nb, int blk, int n0, int n1, const int32_t* positions, LT* ul,
                                           int ldu) {
   constexpr int IN = 2;                                // vectors a thread asks for together
@@ -318,9 +318,13 @@ __device__ __forceinline__ void step_conv(const LruArgs& a, int b0, int nb, int 
   const bool same = blockDim.x % nv == 0;              // a thread's vectors are of the same channels
   for (int i0 = threadIdx.x; i0 < items; i0 += IN * blockDim.x) {
     Vec<V> x[IN], o[IN][3], y[IN], bx[IN], w[IN][4];
-    ColsIn<ACT, V, 4> xin[IN];
+    ColsIn<ACT, V, AHEAD ? 4 : 8, AHEAD> xin[IN];
     int64_t at[IN], xo[IN];
     int ps[IN];
+    auto past = [&](int j) {
+#pragma unroll
+      for (int d = 1; d <= 3; ++d) o[j][d - 1] = ldv<V>(a.tail + at[j] + (size_t)(max(ps[j] - d, 0) % a.taps) * a.W);
+    };
 #pragma unroll
     for (int j = 0; j < IN; ++j) {                     // past the last or in the pad: another's, not stored
       const int i = min(i0 + j * (int)blockDim.x, items - 1), r = i / nv, k = (i - r * nv) * V, b = b0 + r;
@@ -328,7 +332,8 @@ __device__ __forceinline__ void step_conv(const LruArgs& a, int b0, int nb, int 
       ps[j] = positions[b];
       at[j] = (int64_t)a.slots[b] * a.taps * a.W + c;
       xo[j] = b * a.x.ld + c;
-      xin[j].ask(a.x.p, a.x.split, a.x.plane, xo[j]);
+      if constexpr (AHEAD) xin[j].ask(a.x.p, a.x.split, a.x.plane, xo[j]);
+      else x[j] = xin[j].get(a.x.p, a.x.split, a.x.plane, xo[j]);
       if (j && same) {
         bx[j] = bx[0];
         y[j] = y[0];
@@ -340,14 +345,15 @@ __device__ __forceinline__ void step_conv(const LruArgs& a, int b0, int nb, int 
 #pragma unroll
         for (int d = 0; d < 4; ++d) w[j][d] = ldv<V>(a.conv + (size_t)max(back - d, 0) * a.W + c);
       }
+      if constexpr (!AHEAD) past(j);
+    }
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int j = 0; j < IN; ++j) past(j);            // last, as they wait for their indexes
     }
 #pragma unroll
-    for (int j = 0; j < IN; ++j)                       // last, as they wait for their indexes
-#pragma unroll
-      for (int d = 1; d <= 3; ++d) o[j][d - 1] = ldv<V>(a.tail + at[j] + (size_t)(max(ps[j] - d, 0) % a.taps) * a.W);
-#pragma unroll
     for (int j = 0; j < IN; ++j) {
-      x[j] = xin[j].get(a.x.p, a.x.split, a.x.plane, xo[j]);
+      if constexpr (AHEAD) x[j] = xin[j].get(a.x.p, a.x.split, a.x.plane, xo[j]);
       const int i = i0 + j * (int)blockDim.x, r = i / nv, k = (i - r * nv) * V, pos = ps[j];
       if (i >= items) break;
       if (k >= a.bs) {
@@ -373,8 +379,11 @@ __device__ __forceinline__ void step_conv(const LruArgs& a, int b0, int nb, int 
 }
 
 // 1-D grid of rows / 16 x blocks x NP / 16 NW, rounded up each; where eight divides the blocks, an XCD takes all of a block's,
-// so that its matrices and inputs come into one L2.  NW waves of 16 channels.  V: vectors of channels (4 or 1)
-template <int V, int NW>
+// so that its matrices and inputs come into one L2.  NW waves of 16 channels.  V: vectors of channels (4 or 1).
+// AHEAD: x and y are four slabs or fewer, asked for behind the matrices and added where they are needed; of more, what that
+// leaves for later would be waited for at the end (16 rows of 8 x 512, cold: of 1 / 4 slabs 21.5 / 21.6 -> 19.7 / 21.0 us, of 8
+// 25.2 -> 27.4)
+template <int V, int NW, bool AHEAD>
 __global__ void __launch_bounds__(64 * NW) rglru_step_kernel(LruArgs a, const int32_t* __restrict__ positions,
                                                         const int32_t* __restrict__ ctx_lens, int B, uint16_t* __restrict__ out) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -397,7 +406,7 @@ __global__ void __launch_bounds__(64 * NW) rglru_step_kernel(LruArgs a, const in
   float* sp = a.state + (size_t)a.slots[b] * W + c;
   Vec<4> S = zerov<4>(), br, bi, rate, by;
   constexpr int YN = 4 / V;
-  ColsIn<uint16_t, V, 4> yin[YN];
+  ColsIn<uint16_t, V, AHEAD ? 4 : 8, AHEAD> yin[YN];
   auto get = [&](auto ld) {
     Vec<4> r;
     if constexpr (V == 4) {
@@ -420,19 +429,33 @@ __global__ void __launch_bounds__(64 * NW) rglru_step_kernel(LruArgs a, const in
       wi[j] = *reinterpret_cast<const u32x4_t*>(p + second + o);
     }
   };
-  matrices(0);
-  // behind the matrices, which nothing waits for; the state last, as it waits for its index (5 rows: 9.0 -> 8.6 us)
+  if constexpr (AHEAD) matrices(0);              // nothing waits for them
   auto y_at = [&](int e) { return (int64_t)b * a.y.ld + c + (V == 4 ? 0 : k0 + e < a.bs ? e : 0); };
-  if (on) {
+  float y[4];
+  auto sum_y = [&] {
 #pragma unroll
-    for (int e = 0; e < YN; ++e) yin[e].ask(a.y.p, a.y.split, a.y.plane, y_at(e));
+    for (int e = 0; e < YN; ++e) {
+      const Vec<V> v = yin[e].get(a.y.p, a.y.split, a.y.plane, y_at(e));
+#pragma unroll
+      for (int i = 0; i < V; ++i) y[e * V + i] = v.v[i];
+    }
+  };
+  if (on) {
+    if constexpr (!AHEAD) {
+      if (ctx_lens[b] > 1) S = get([&](int e, auto n) { return ldv<decltype(n)::value>(sp + e); });
+      sum_y();
+    } else {
+#pragma unroll
+      for (int e = 0; e < YN; ++e) yin[e].ask(a.y.p, a.y.split, a.y.plane, y_at(e));
+    }
     by = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.by + c + e); });
     br = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.br + c + e); });
     bi = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.bi + c + e); });
     rate = get([&](int e, auto n) { return ldv<decltype(n)::value>(a.rate + c + e); });
-    if (ctx_lens[b] > 1) S = get([&](int e, auto n) { return ldv<decltype(n)::value>(sp + e); });
+    if (AHEAD && ctx_lens[b] > 1) S = get([&](int e, auto n) { return ldv<decltype(n)::value>(sp + e); });      // last: it waits for its index
   }
-  step_conv<uint16_t, uint16_t, V>(a, b0, nb, blk, g0, g0 + 16 * NW, positions, ul, ldu);
+  if constexpr (!AHEAD) matrices(0);
+  step_conv<uint16_t, uint16_t, V, AHEAD>(a, b0, nb, blk, g0, g0 + 16 * NW, positions, ul, ldu);
   __syncthreads();
   if (n0 >= a.NP) return;
   f32x4_t pr{0.f, 0.f, 0.f, 0.f}, pi{0.f, 0.f, 0.f, 0.f};
@@ -448,13 +471,7 @@ __global__ void __launch_bounds__(64 * NW) rglru_step_kernel(LruArgs a, const in
   }
   if (!on) return;
   Vec<4> o;
-  float y[4];
-#pragma unroll
-  for (int e = 0; e < YN; ++e) {
-    const Vec<V> v = yin[e].get(a.y.p, a.y.split, a.y.plane, y_at(e));
-#pragma unroll
-    for (int i = 0; i < V; ++i) y[e * V + i] = v.v[i];
-  }
+  if constexpr (AHEAD) sum_y();
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     float ga, gb;
@@ -497,7 +514,7 @@ __global__ void __launch_bounds__(256) rglru_any_kernel(LruArgs a, const ACT* __
   if (u) {
     for (int k = threadIdx.x; k < a.bs; k += 256) ul[k] = ld1(u + (size_t)t * a.blocks * a.KP + blk * a.KP + k);
   } else {
-    step_conv<ACT, float, 1>(a, t, 1, blk, 0, a.bs, positions, ul, a.KP);
+    step_conv<ACT, float, 1, true>(a, t, 1, blk, 0, a.bs, positions, ul, a.KP);
     __syncthreads();
     for (int k = threadIdx.x; k < a.bs; k += 256) ul[k] = round_act(ul[k], (const ACT*)nullptr);
   }
@@ -598,7 +615,12 @@ CFC_API int cfc_rglru_step(int f32, const void* x, int x_split, int64_t x_ld, in
     const int nw = B >= 32 && NP > 64 ? 8 : 4, grid = (B + 15) / 16 * blocks * ((NP + 16 * nw - 1) / (16 * nw));
     const size_t lds = (size_t)16 * (KP + 8) * 2;
     const bool v4 = bs % 4 == 0 && lru_cols_vec(a.x, 0) && lru_cols_vec(a.y, 0) && ((uintptr_t)out & 7) == 0;
-#define ST(V, NW) rglru_step_kernel<V, NW><<<grid, 64 * NW, lds, stream>>>(a, positions, ctx_lens, B, (uint16_t*)out)
+    const bool few = x_split <= 4 && y_split <= 4;
+#define ST(V, NW)                                                                                                                   \
+  do {                                                                                                                              \
+    if (few) rglru_step_kernel<V, NW, true><<<grid, 64 * NW, lds, stream>>>(a, positions, ctx_lens, B, (uint16_t*)out);               \
+    else rglru_step_kernel<V, NW, false><<<grid, 64 * NW, lds, stream>>>(a, positions, ctx_lens, B, (uint16_t*)out);                  \
+  } while (0)
     if (nw == 8) { if (v4) ST(4, 8); else ST(1, 8); }
     else if (v4) ST(4, 4);
     else ST(1, 4);
