@@ -161,15 +161,25 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
   const float* bias = SHAPED && a.bias ? a.bias + (size_t)(hk * R + r0 + min(col, nr - 1)) * a.nb : nullptr;
   const float far_bias = bias ? bias[a.nb - 1] : 0.f;
   u32x4_t kf[2][KS], vf[NV];
-  // row of this lane's key (lane & 31) in a tile; tiles past the slice: its last
-  auto rows_of = [&](int t) {
+  const int first = a.size ? window_first(a, pos) : 0;
+  // This lane's key (lane & 31) in a tile (past the slice: its last), the cache block that it is in, and its row.  The block goes
+  // from one step to the next, and not the row: that would be waited for as soon as it is asked for, and with it all that was
+  // asked for before it, the next tile (one slice of 2800 keys, heads of 128: 38 us with rows, 30).  Heads of more than 160
+  // columns have no registers left for it (of 256: 62 with rows, 80).
+  constexpr bool ROWS = D > 160;
+  auto key_of = [&](int t) {
     t = min(t, t1 - 1);
-    const bool far = t < kt.nat, pooled = far && a.pool;
-    const int e = far ? min(32 * t + (lane & 31), kt.na - 1) : kt.lo + 32 * (t - kt.nat) + (lane & 31);
-    return key_row(a, pooled, bt[key_page(a, pooled, e)], hk, e);
+    return t < kt.nat ? min(32 * t + (lane & 31), kt.na - 1) : kt.lo + 32 * (t - kt.nat) + (lane & 31);
   };
-  auto load = [&](int t, int row) {
-    const bool pooled = a.pool && min(t, t1 - 1) < kt.nat;
+  auto pooled_at = [&](int t) { return a.pool && min(t, t1 - 1) < kt.nat; };
+  auto row_in = [&](int t, int block) { return key_row(a, pooled_at(t), block, hk, key_of(t)); };
+  auto find = [&](int t) {
+    const int block = bt[key_page(a, pooled_at(t), key_of(t))];
+    return ROWS ? row_in(t, block) : block;
+  };
+  auto load = [&](int t, int found) {
+    const bool pooled = pooled_at(t);
+    const int row = ROWS ? found : row_in(t, found);
     const uint16_t *kb = pooled ? pk : kc, *vb = pooled ? pv : vc;
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
@@ -190,13 +200,13 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
   float m = -INFINITY, l = 0.f;
   int t = t0 + w;
   if (t < t1) {
-    int row = rows_of(t);
-    load(t, row);
+    int found = find(t);
+    load(t, found);
 #pragma unroll
     for (int k = 0; k < KS; ++k)             // behind the first tile, which waits for indexes
       qf[k] = *reinterpret_cast<const u32x4_t*>(q + (qrow + min(col, nr - 1)) * D + 32 * k + 8 * kq);
-    if (t + 4 < t1) row = rows_of(t + 4);
-    for (; t < t1; t += 4) {
+    found = find(t + 4);
+    auto step = [&](auto more) {
       wave_lds_fence();                      // the last tile's values have been read
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
@@ -210,13 +220,14 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
 #pragma unroll
         for (int k = 0; k < KS; ++k) sc[g] = mfma16(kf[g][k], qf[k], sc[g]);
       }
-      if (t + 4 < t1) {                      // a tile that no one uses was one in three or four of a short slice's loads
-        load(t + 4, row);
-        if (t + 8 < t1) row = rows_of(t + 8);
+      if constexpr (decltype(more)::value) {
+        load(t + 4, found);
+        found = find(t + 8);
       }
       const bool far = t < kt.nat;
+      // (key <= last ..: what sees() says of the tile's keys, without its branches at each of them)
+      const int k0 = far ? 32 * t : kt.lo + 32 * (t - kt.nat), last = far ? kt.na - 1 : pos, lo = far ? 0 : first;
       if constexpr (SHAPED) {
-        const int k0 = far ? 32 * t : kt.lo + 32 * (t - kt.nat);
         float bt8[2][4];
         if (bias && pos - k0 - 31 < a.nb - 1) {
 #pragma unroll
@@ -239,8 +250,8 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
       for (int g = 0; g < 2; ++g)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int key = 16 * g + 4 * kq + i;
-          const bool see = far ? 32 * t + key < kt.na : sees(a, pos, kt.lo + 32 * (t - kt.nat) + key);
+          const int key = k0 + 16 * g + 4 * kq + i;
+          const bool see = ROWS ? (far ? key < kt.na : sees(a, pos, key)) : (key <= last) & ((key >= lo) | (key < a.keep));
           if (!see) sc[g][i] = -INFINITY;
           mx = fmaxf(mx, sc[g][i]);
         }
@@ -278,7 +289,11 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
         }
         o[d] = mfma16(vt, pf, o[d]);
       }
-    }
+    };
+    // The last step asks for nothing: a tile that no one uses was one in three or four of a short slice's loads.  In a step of its
+    // own: behind a condition in the loop the loads stay where they are (2800 keys in one slice 38 -> 50 us)
+    for (; t + 4 < t1; t += 4) step(std::true_type{});
+    step(std::false_type{});
   }
   l = xor32_sum(xor16_sum(l));
   wave_lds_fence();
