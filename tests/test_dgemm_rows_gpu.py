@@ -82,3 +82,23 @@ def test_rows_of_pairs_about_a_step(T, top, E):
     ids = torch.randint(0, E + 2, (T, top), generator=torch.Generator().manual_seed(T), dtype=torch.int32)
     for got, want in zip(moe.sort_rows(ids.cuda(), E, 32), moe_rows(ids, E, 32)):
         assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("split", [1, 2, 7, 8, 9, 16, 17, 112])
+def test_slabs_are_added_in_their_order(split):
+    """One slab, less and more than are in flight, one of them without bounds."""
+    g = torch.Generator("cuda").manual_seed(split)
+    part = torch.randn(split, 3, 1104, device="cuda", generator=g)
+    part[-1, 1, 5], part[0, 2, 1000] = float("inf"), float("nan")
+    want = torch.zeros(3, 1104, device="cuda")
+    for p in part:
+        want += p
+    same = lambda a, b: torch.equal(a.nan_to_num(7.0, 8.0, 9.0), b.nan_to_num(7.0, 8.0, 9.0))
+    assert same(K.splitk_reduce(part), want.bfloat16())
+    rows = want.bfloat16().float().view(3, 69, 2, 8)
+    gate, up = rows[:, :, 0].reshape(3, -1), rows[:, :, 1].reshape(3, -1)
+    got, want = K.splitk_reduce(part, swiglu=True).float(), (torch.nn.functional.silu(gate).bfloat16().float() * up)
+    # silu before its rounding is within a few parts in 2^22 (the exponential's), so its rounding within one step: 2^-8, the product's 2^-9
+    ok = torch.isfinite(want)
+    assert torch.equal(ok, torch.isfinite(got)) and ((got - want).abs()[ok] <= 2.0 ** -7 * want.abs()[ok]).all()
