@@ -3,8 +3,9 @@
 Up to 128 rows run on the decode GEMM, thousands on the prefill GEMM's 256 x 256 tiles, what lies between on the GEMM
 for a few hundred rows (K.prompt_plan), all three reading one fragment-packed bf16 copy.  (One to four rows, too: with its
 tile of 16 rows the decode GEMM takes 29 us where the packed GEMV takes 32 to 38, 20608 x 4096, 4.8 where it takes 5.2 to
-8.2, 4096 x 1536, and the same at worst; and it gates and clamps in its epilogue.)  Shapes those kernels do not take (N or K not a multiple of 64) and 32-bit weights use
-the library product.  CPU tensors: torch.
+8.2, 4096 x 1536; and it gates and clamps in its epilogue.  A narrow matrix of long rows only fills the chip in so many
+slabs that their sum takes longer than the product: NARROW_SLABS.)  Shapes those kernels do not take (N or K not a multiple
+of 64) and 32-bit weights use the library product.  CPU tensors: torch.
 """
 from __future__ import annotations
 
@@ -16,6 +17,13 @@ import torch.nn.functional as F
 from ..ops import kernels as K
 from ..ops.cols import Cols
 from ..ops.stream import clamped_glu, relu_sq
+
+
+# One to four rows whose product the decode GEMM would cut into more slabs than this run on the packed GEMV, whose workgroup
+# reads longer rows: us of product and sum, one and four rows, GEMM -> GEMV, 64 x 4096 in 64 slabs 10.1 -> 7.1 and 10.3 -> 7.0,
+# 256 x 7168 in 64 10.5 -> 7.3 and 11.6 -> 8.3, 576 x 4096 in 28 8.2 -> 7.5 and 8.8 -> 7.5; with 16 the GEMM is ahead, 1024 x 4096 7.1
+# and 7.4 where the GEMV takes 7.7 and 7.6.
+NARROW_SLABS = 16
 
 
 class Projection:
@@ -61,6 +69,9 @@ class Projection:
             return "lib"
         if K.prompt_plan(x.shape[0], self.N, self.K, kind):
             return "mgemm"
+        if kind != "whole" and 1 <= x.shape[0] <= K.GEMV_MAX_M \
+                and K.dgemm_slab_plan(x.shape[0], self.N, self.K, self.packed.bn)[0] > NARROW_SLABS:
+            return "gemv"
         return "pgemm" if self._prefill(x.shape[0]) else "dgemm"
 
     def _prompt(self, x, epi: str, kind: str = "act", **kw):
@@ -75,6 +86,8 @@ class Projection:
             return self._prompt(x, "bf16", reduce=K.splitk_reduce)
         if k == "pgemm":
             return K.pgemm(x, self.packed, "bf16", variant="ppp")
+        if k == "gemv":
+            return K.splitk_reduce(K.gemv_part(x, self.packed))
         return K.dgemm_linear(x, self.packed)
 
     def slabs(self, x: torch.Tensor, own: bool = False) -> torch.Tensor:
@@ -83,8 +96,9 @@ class Projection:
         their ``own``."""
         k = self._kernel(x, "slabs")
         M, out = x.shape[0], None
-        if k in ("dgemm", "mgemm"):
-            split = K.dgemm_slab_plan(M, self.N, self.K, self.packed.bn)[0] if k == "dgemm" else \
+        if k in ("gemv", "dgemm", "mgemm"):
+            split = K.gemv_packed_config(self.N, self.K, self.packed.bn // 16, M)[0] if k == "gemv" else \
+                K.dgemm_slab_plan(M, self.N, self.K, self.packed.bn)[0] if k == "dgemm" else \
                 K.prompt_plan(M, self.N, self.K, "slabs")[2]
             if own:
                 out = torch.empty(split, M, self.N, dtype=torch.float32, device=x.device)
@@ -92,6 +106,8 @@ class Projection:
             return self._prompt(x, "f32", "slabs", out=out)
         if k == "pgemm":
             return K.pgemm(x, self.packed, "f32", variant="ppp")[None]
+        if k == "gemv":
+            return K.gemv_part(x, self.packed, out=out)
         if k == "dgemm":
             return K.dgemm_slabs(x, self.packed, out)
         w = self.rowmajor()

@@ -3,6 +3,7 @@ whose first rows they are (the same products in the same order), and those are w
 import pytest
 import torch
 
+from copilot_for_consensus_amd.models.projection import Projection
 from copilot_for_consensus_amd.ops import kernels as K
 from copilot_for_consensus_amd.ops import moe
 
@@ -102,3 +103,22 @@ def test_slabs_are_added_in_their_order(split):
     # silu before its rounding is within a few parts in 2^22 (the exponential's), so its rounding within one step: 2^-8, the product's 2^-9
     ok = torch.isfinite(want)
     assert torch.equal(ok, torch.isfinite(got)) and ((got - want).abs()[ok] <= 2.0 ** -7 * want.abs()[ok]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N, Kd, narrow", [(64, 1024, False), (64, 2048, True), (256, 7168, True), (576, 4096, True), (1024, 4096, False)])
+def test_few_rows_of_a_narrow_matrix(N, Kd, narrow):
+    """Both sides of the rule: the product of 64-bit sums, as activations (rounded to bf16) and in slabs."""
+    g = torch.Generator("cuda").manual_seed(N)
+    w = (torch.randn(N, Kd, device="cuda", generator=g) * Kd ** -0.5).bfloat16()
+    p = Projection(w)
+    for M in (1, 2, 4, 5):
+        assert (p._kernel(w[:M]) == "gemv") == (narrow and M <= K.GEMV_MAX_M) and p._kernel(w[:M], "whole") == "dgemm"
+        x = torch.randn(M, Kd, device="cuda", generator=g).bfloat16()
+        exact = x.double() @ w.double().t()
+        bound = Kd * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())     # sums of Kd products in fp32, in any order
+        for own in (False, True):
+            slabs = p.slabs(x, own=own)
+            assert ((slabs.double().sum(0) - exact).abs() <= bound).all()
+        assert ((p.act(x).double() - exact).abs() <= bound + 2.0 ** -8 * (exact.abs() + bound)).all()
+        assert ((p.f32(x).double() - exact).abs() <= bound).all()
