@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Headline benchmark: end-to-end threads summarized / s (+ p50 summary latency), Mistral-7B.
 
-BASELINE.json metric: "end-to-end threads summarized/sec + p50 summary latency, Mistral-7B TP=1/8".
+The metric: "end-to-end threads summarized/sec + p50 summary latency, Mistral-7B TP=1/8".
 One step = one batch of mailing-list threads per GPU taken through the whole pipeline of the
 reference (ingest bytes -> parse mbox -> thread -> chunk -> embed (HIP encoder) -> index (HIP kNN)
 -> orchestrator top-k context selection -> prompt -> Mistral-7B prefill + 512-token greedy decode
@@ -26,14 +26,14 @@ import time
 # threads (--pipeline node) as a warning
 os.environ.setdefault("TORCH_CPP_LOG_LEVEL", "ERROR")
 
-# Reference operating point derived in BASELINE.md: best published number (RTX 4090, 150-200
+# Reference operating point: best published number (RTX 4090, 150-200
 # tok/s Ollama decode) => ~3-4 s per thread => 0.25-0.33 threads/s.  We divide by the MOST
 # favourable-to-the-reference value (1/3 thread/s); the AMD RX 6700 XT point is 0.07-0.09.
 BASELINE_THREADS_PER_S = 1.0 / 3.0
 
 
 def metric_name(model: str) -> str:
-    """BASELINE.json's metric string, with the decoder actually run (``--model``) in it."""
+    """The metric string, with the decoder actually run (``--model``) in it."""
     words = model.split("-")
     pretty = "-".join(w.capitalize() if not w[:1].isdigit() else w.upper() for w in words)
     return f"end-to-end threads summarized/sec + p50 summary latency, {pretty} TP=1/8"

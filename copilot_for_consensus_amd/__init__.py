@@ -2,6 +2,6 @@
 
 Control plane (Python): contracts, config, bus, storage, archive, parsing, chunking,
 orchestration, reporting, services.  Data plane (HIP/CDNA4 + hipBLASLt + RCCL): models/, ops/,
-runtime/, parallel/, vectorstore/ (see SURVEY.md §7 for the blueprint).
+runtime/, parallel/, vectorstore/.
 """
 __version__ = "0.1.0"

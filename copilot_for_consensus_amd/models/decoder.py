@@ -493,7 +493,7 @@ class DecoderModel:
         self.gemv_norm_fused = os.environ.get("CFC_DECODE_GEMV_NORM", "0") == "1"
         # TP > 1: the row-parallel (o / down) partials are all-reduced in fp32 and rounded to bf16
         # ONCE, as TP = 1 rounds the full sum (CFC_TP_AR_DTYPE=fp32, default); "bf16" rounds each
-        # rank's partial first and halves the prefill all-reduce bytes (round 5's behaviour).  The
+        # rank's partial first and halves the prefill all-reduce bytes.  The
         # batched decode always sums fp32 (one-shot kernel: latency-bound, bytes do not matter)
         ard = os.environ.get("CFC_TP_AR_DTYPE", "fp32")
         if ard not in ("fp32", "bf16"):
@@ -562,7 +562,7 @@ class DecoderModel:
     # "ppp": the persistent ping-pong kernel (one workgroup per CU walking the tiles, the DMA
     # stream running on across tile boundaries, LDS-staged 16-byte stores for bf16) --
     # bit-identical to "pp" / "pps"; against "pps" (the ping-pong K loop with the LDS-staged
-    # epilogue, round 4's default) on the 16k-row chunk: qkv -3.3 %, o -2.3 %, gate_up + SwiGLU
+    # epilogue, the former default) on the 16k-row chunk: qkv -3.3 %, o -2.3 %, gate_up + SwiGLU
     # -3.9 %, down -1.0 % (profiles/r06_pgemm_ppp_v2.jsonl, r06_pgemm_k3.jsonl)
     PGEMM_VARIANT_DEFAULT = "ppp"
     PGEMM_VARIANT_SWIGLU_DEFAULT = "ppp"

@@ -905,7 +905,7 @@ def pgemm_ln_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 def pgemm_ln(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, residual: torch.Tensor, gamma: torch.Tensor,
              beta: torch.Tensor, eps: float, out: torch.Tensor | None = None) -> torch.Tensor:
     """LayerNorm(x @ w^T + bias + residual) * gamma + beta in one kernel (the post-LN encoder
-    sub-layer: attention o-proj and FFN down with their residual and LayerNorm, SURVEY K5 / K6).
+    sub-layer: attention o-proj and FFN down with their residual and LayerNorm).
     Numerics as the unfused path: projection rounded to bf16, the rest in fp32."""
     if not x.is_cuda:
         y = torch.nn.functional.linear(x.float(), w.float()).to(x.dtype)

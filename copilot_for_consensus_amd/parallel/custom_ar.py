@@ -4,8 +4,8 @@ Why: TP decode issues two all-reduces per layer (after o_proj and down_proj) of 
 64 collectives per token for a 32-layer model, each 8 KiB-1 MiB.  At these sizes RCCL's ring
 pays per-hop latency on every one of them; the xGMI mesh of an MI355X node is point-to-point
 (every GPU pair one hop, 7 links per GPU), so each rank can simply READ all peers' contributions
-directly: one barrier + one pass, every link used in parallel.  ("custom one-shot
-all-reduce via IPC peer pointers, captured in the hipGraph with the decode step".)
+directly: one barrier + one pass, every link used in parallel.
+It is captured in the hipGraph with the decode step.
 
 Setup (collective over the TP group, once): every rank allocates an uncached region
 (signals + 2 staging buffers), exports its IPC handle, all-gathers the handles (over a CPU/gloo

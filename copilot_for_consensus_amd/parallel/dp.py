@@ -1,7 +1,7 @@
 """Data parallelism for the summarization pipeline.
 
 The reference scales horizontally by running more service replicas behind RabbitMQ competing
-consumers (SURVEY §3.2; orchestrator and summarization are stateless per thread).  On a node of
+consumers (orchestrator and summarization are stateless per thread).  On a node of
 8 MI355X the equivalent is one engine per GPU (or per TP group) and a deterministic split of the
 threads across them:
 

@@ -79,7 +79,7 @@ def _waiter(store):
     except ImportError:  # pragma: no cover
         return None
     if not isinstance(store, TCPStore) or os.environ.get("CFC_DP_WAIT", "block") == "poll":
-        return None                   # CFC_DP_WAIT=poll: round 5's check polling (A/B)
+        return None                   # CFC_DP_WAIT=poll: check polling, to compare
     cache = getattr(_waiters, "clients", None)
     if cache is None:
         cache = _waiters.clients = {}

@@ -1,7 +1,6 @@
 """Fault-tolerant data-parallel work loop: one worker per GPU (or TP group) pulls thread batches
 from a shared ledger, heartbeats while it works, and the survivors take over a dead worker's
-unfinished threads ("GPU worker watchdog, requeue of in-flight thread batches if a GPU
-worker dies").
+unfinished threads.
 
 Coordination goes only through the job's key-value store (torchrun's TCPStore), never through a
 collective, so a rank that dies -- process gone, node lost, or stuck in a kernel (its progress

@@ -1,6 +1,6 @@
-"""Failure detection and forward progress for multi-GPU summarization workers (SURVEY §5.3 rebuild:
-per-GPU heartbeat watchdog, requeue of a dead worker's in-flight threads, RCCL timeouts that raise
-instead of hanging).
+"""Failure detection and forward progress for multi-GPU summarization workers:
+a per-GPU heartbeat watchdog, requeue of a dead worker's in-flight threads, RCCL timeouts that raise
+instead of hanging.
 
 All state lives in a ``torch.distributed`` key-value Store (the job's TCPStore under torchrun, a
 FileStore / HashStore otherwise), so any surviving rank -- or an external supervisor -- can see it:

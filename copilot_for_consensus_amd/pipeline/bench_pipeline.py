@@ -105,7 +105,7 @@ class BenchPipeline:
             self.rag.prepare_sources(self.threads_per_step, steps)
 
     def _synthetic_prompts(self, n):
-        # ~2.5-3k prompt tokens: BASELINE.md "prefill of about 2.5k-3k tokens"
+        # ~2.5-3k prompt tokens: the reference operating point's "prefill of about 2.5k-3k tokens"
         out = []
         for _ in range(n):
             L = self.rng.randint(2560, 3072)

@@ -17,7 +17,7 @@ batch's chunks in a few packed forwards, the vectors go from the encoder to the 
 leaving the GPU, and the orchestrator scores all threads' candidates in one index pass
 (centroid_scores_many).
 
-Reference: the six-service event flow (SURVEY §3.3); orchestrator context selection
+Reference: the six-service event flow; orchestrator context selection
 (orchestrator/app/context_selectors.py:17,95-107; context_sources.py:21,57-64) and the
 summarization request path (summarization/app/service.py:289).
 """

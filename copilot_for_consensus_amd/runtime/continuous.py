@@ -1,5 +1,4 @@
-"""Continuous batching over the paged KV cache ("continuous batching of
-threads"; the reference's llama.cpp / Ollama servers interleave concurrent requests the same way,
+"""Continuous batching over the paged KV cache (the reference's llama.cpp / Ollama servers interleave concurrent requests the same way,
 llamacpp_summarizer.py:108 -> llama-server slots, docker-compose.infra.yml:296-298).
 
 :class:`LLMEngine.generate` runs a batch to completion; a thread that finishes early leaves its row

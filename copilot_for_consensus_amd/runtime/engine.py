@@ -140,7 +140,7 @@ class LLMEngine:
         # and the one-shot all-reduce's epoch bookkeeping checked on the CPU
         # (tests/test_parallel_cpu.py); the TP=2 rehearsal on one GPU (gloo) runs it to completion
         # with the one-shot all-reduce's error counter at 0 and identical per-block epochs on both
-        # ranks after every batch (profiles/r06_tp2_overlap_gloo_1gpu.log).  The round-5 rehearsal
+        # ranks after every batch (profiles/r06_tp2_overlap_gloo_1gpu.log).  The former rehearsal
         # that stopped at its 150 s limit inside the second batch's decode graph was rerun this way
         # and completed: no all-reduce timed out and no epoch desync -- not reproduced.
         # Not measured on a multi-GPU node (RCCL), so it stays opt-in.

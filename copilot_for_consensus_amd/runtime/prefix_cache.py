@@ -1,7 +1,7 @@
 """Prefix cache over the paged KV cache: full 32-token blocks shared across sequences.
 
-Every summarization prompt starts with the same system prompt and template head (SURVEY §3.3,
-orchestrator prompts), so the KV of those leading blocks is identical for every thread.  The
+Every summarization prompt starts with the same system prompt and template head (the
+orchestrator's prompts), so the KV of those leading blocks is identical for every thread.  The
 engine looks each prompt's leading full blocks up by a hash chain (block j's key covers tokens
 [0, 32(j+1))), points the sequence's block table at the cached physical blocks and starts its
 prefill after them -- the prefill kernel already reads keys [0, ctx) from the cache, so no kernel

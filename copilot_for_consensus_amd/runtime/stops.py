@@ -1,4 +1,4 @@
-"""Stop strings evaluated on the device, inside the captured decode step (SURVEY K17).
+"""Stop strings evaluated on the device, inside the captured decode step.
 
 llama.cpp stops generating as soon as the detokenized text contains one of the request's stop
 strings (the reference passes ``["</s>", "\\n\\n\\n"]``, llamacpp_summarizer.py:111-113).  A stop

@@ -1,6 +1,6 @@
 """Shared service scaffolding.
 
-Every bus-driven service of the reference has the same process model (SURVEY §1): build adapters
+Every bus-driven service of the reference has the same process model: build adapters
 from typed config, start a non-daemon consumer thread (``service.start()`` + blocking
 ``subscriber.start_consuming()``), run uvicorn on the main thread with ``/health``, ``/readyz``,
 ``/stats`` and ``/.well-known/configuration-schema`` (e.g. parsing/main.py:101-145,303-318).

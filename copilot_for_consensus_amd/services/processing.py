@@ -1,7 +1,7 @@
 """The five bus-driven processing services: parsing, chunking, embedding, orchestrator, summarization.
 
-Each mirrors its reference service's event contract and forward-progress behaviour (SURVEY §3.3,
-§3.5): consume the upstream event with the retry policy, read documents (eventual-consistency
+Each mirrors its reference service's event contract and forward-progress behaviour:
+consume the upstream event with the retry policy, read documents (eventual-consistency
 misses raise DocumentNotFoundError -> jittered retry), write documents idempotently (deterministic
 ids, duplicate inserts tolerated), publish the downstream event or the stage's *Failed event,
 requeue incomplete work at startup, and delete a source's documents on SourceDeletionRequested

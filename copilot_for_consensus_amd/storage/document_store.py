@@ -4,7 +4,7 @@ decorator, MongoDB driver (optional, needs pymongo) and factory.
 Interface = adapters/copilot_storage/copilot_storage/document_store.py:40-138 of the reference
 (insert_document / get_document / query_documents(filter, limit, sort_by, sort_order) /
 update_document / delete_document / aggregate_documents) plus batched ``insert_many`` /
-``update_many`` so the pipeline's per-document hot loops (SURVEY §3.3) become one call.
+``update_many`` so the pipeline's per-document hot loops become one call.
 """
 from __future__ import annotations
 

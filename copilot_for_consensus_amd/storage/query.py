@@ -2,7 +2,7 @@
 
 The reference's InMemoryDocumentStore supports only equality filters
 (adapters/copilot_storage/copilot_storage/inmemory_document_store.py:132), so its services ship
-shims for ``$in`` in tests (SURVEY §4).  This matcher implements the operators the pipeline and
+shims for ``$in`` in tests.  This matcher implements the operators the pipeline and
 the REST queries use: $eq $ne $gt $gte $lt $lte $in $nin $exists $regex $size $all $elemMatch
 $not $and $or $nor, dotted paths, and Mongo's array semantics (a scalar condition on an array
 field matches if ANY element matches).

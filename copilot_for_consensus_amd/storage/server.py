@@ -9,7 +9,7 @@ over TCP, and :class:`RemoteDocumentStore` (``DOCUMENT_STORE_TYPE=cfcstore``) is
 Durability: every mutating call is appended to a write-ahead log (JSON lines, optional fsync)
 after it is applied and before it is acknowledged; a snapshot of all collections replaces the log
 every ``snapshot_every`` writes and at shutdown.  Start-up = snapshot + log replay, so the
-pipeline's status fields and deterministic ids (SURVEY §5.4) survive a restart of the store.
+pipeline's status fields and deterministic ids survive a restart of the store.
 
 Wire format: u32 big-endian length + UTF-8 JSON, request ``{"id", "op", "args", "kwargs"}``,
 reply ``{"id", "ok", "result"}`` or ``{"id", "ok": false, "error": <class>, "message"}``.

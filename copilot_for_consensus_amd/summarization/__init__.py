@@ -143,7 +143,7 @@ class HipLLMSummarizer(Summarizer):
         self.last_stats: dict = {}
 
     def gpu_stats(self, res) -> dict:
-        """Engine/GPU figures of the last batch (SURVEY §5.5: tokens/s, TTFT, HBM use)."""
+        """Engine/GPU figures of the last batch (tokens/s, TTFT, HBM use)."""
         gen = sum(len(t) for t in res.tokens)
         st = {"ttft_seconds": res.ttft_s, "prefill_seconds": res.prefill_s, "decode_seconds": res.decode_s,
               "decode_tokens_per_second": gen / res.decode_s if res.decode_s > 0 else 0.0,
@@ -235,7 +235,7 @@ class HipLLMSummarizer(Summarizer):
         """Serve :meth:`submit` ted threads through a ContinuousEngine on a background thread: a
         thread joins the running decode batch at the next burst boundary and leaves it at its stop
         (EOS, a stop string on the device, or max_new_tokens), its slot refilled from the queue --
-        no batch-of-N latency for a bursty bus load (SURVEY §7.2 step 5).  Under tensor
+        no batch-of-N latency for a bursty bus load.  Under tensor
         parallelism the followers build the same engine and replay every step (``tp_hook``)."""
         import collections
         import threading

@@ -1,3 +1,3 @@
-"""Operational tools (the reference's scripts/ directory, SURVEY §2.7): stuck-document retry job,
+"""Operational tools (the reference's scripts/ directory): stuck-document retry job,
 failed-queue CLI, Prometheus exporters, Drain log mining, schema export / validation, gateway
 (OpenAPI + nginx) generation.  Each module has a ``main`` and runs with ``python -m``."""

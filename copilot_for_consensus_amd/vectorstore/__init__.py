@@ -2,7 +2,7 @@
 
 Interface = adapters/copilot_vectorstore/copilot_vectorstore/interface.py:12-114 of the reference
 (add_embedding / add_embeddings [upsert] / query(vector, top_k) -> [SearchResult] / delete / clear /
-count / get).  Replaces Qdrant / FAISS / Azure AI Search on the hot path (SURVEY §2.4 K8/K9):
+count / get).  Replaces Qdrant / FAISS / Azure AI Search on the hot path:
 
 * :class:`HipFlatIndex` -- the whole index lives in one bf16 [capacity, dim] HBM tensor (a
   288 GB MI355X holds 100M x 384 bf16 = 77 GB with room to spare); cosine = dot product of
@@ -456,7 +456,7 @@ class HipFlatIndex(VectorStore):
         idx._alive[:n] = True
         if meta.get("format") == "rowtable-1":
             idx._tab = RowTable.load(p)
-        else:                                  # round-3 JSON sidecar (ids / metadata lists)
+        else:                                  # former JSON sidecar (ids / metadata lists)
             idx._tab = RowTable(n + 1024)
             idx._tab.append_bulk(meta["ids"], meta["metadata"])
         idx._n = n

@@ -7,13 +7,13 @@
 // They replace the attention inside the engines the reference drives over HTTP
 // (Ollama /api/generate: local_llm_summarizer.py:107; llama.cpp /completion:
 // llamacpp_summarizer.py:108) and inside SentenceTransformer.encode
-// (sentence_transformer_provider.py:93).  The reference itself has no kernels (SURVEY §2.4).
+// (sentence_transformer_provider.py:93).  The reference itself has no kernels.
 //
 // Layout decisions (MI355X-first, not a CUDA translation):
 //   * "Swapped" products: S^T = K . Q^T and O^T = V^T . P^T.  With the 16x16x32 C/D map
 //     (col = lane&15, row = 4*(lane>>4)+i) every lane then owns ONE query column, so the
 //     online-softmax max/sum are lane-local plus two xor-shuffles, and the S^T accumulator is
-//     already the P^T B-operand of the next MFMA (guide §3 "accumulator as the next operand").
+//     already the P^T B-operand of the next MFMA ("accumulator as the next operand").
 //   * KV cache block = 32 tokens = one MFMA k-step.  K is stored [blk][kvh][32][D] (row = key),
 //     V is stored TRANSPOSED in slot groups, [blk][kvh][4 groups g][D][8] (common.h kv_v_off), with
 //     the keys of each block permuted so that slot 8g+j holds key perm(g,j) = (j<4 ? 4g+j : 16+4g+j-4).
@@ -21,7 +21,7 @@
 //     contiguous 16-byte load per lane (no LDS transpose, no ds_read_tr needed) in both decode
 //     (straight from HBM) and prefill; and one decode token's V column dirties 16 cache lines
 //     ([D][32] rows: 64), which is what its write costs the step.
-//   * LDS tiles are XOR-swizzled for conflict-free ds_read_b128 (guide §5.5 T2); the swizzles
+//   * LDS tiles are XOR-swizzled for conflict-free ds_read_b128; the swizzles
 //     were derived against the gfx950 ds_read_b128 lane groups {0-3,12-15,20-27}, ...
 #include "common.h"
 #include <stdlib.h>
@@ -48,8 +48,8 @@ __device__ __forceinline__ bf16x8_t pack_p(const f32x4_t& a, const f32x4_t& b) {
 // ------------------------------------------------------------------------------------------
 // Paged decode attention.
 // grid = (P partitions, Hkv, B); block = 256 (4 waves).  Each wave walks the partition's KV
-// blocks with stride 4, K/V fragments straight from HBM into VGPRs (guide: "GEMV / M<=16 decode:
-// load straight to VGPRs"), next block prefetched while the current one is in the MFMAs.
+// blocks with stride 4, K/V fragments straight from HBM into VGPRs
+// (no reuse for the LDS to serve), next block prefetched while the current one is in the MFMAs.
 // The G = Hq/Hkv query heads of the kv-head share every K/V byte (GQA packing: the G heads are
 // the MFMA's B columns).
 // ------------------------------------------------------------------------------------------
@@ -469,12 +469,12 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(const float* __rest
 // positions ctx - q_len + row (chunked prefill / prefix reuse: keys come from the cache).
 //   * K tile (64 keys x 128) and V^T tile (2 blocks x 128 x 32) double-buffered in LDS and shared
 //     by all 8 waves; register-staged (next tile's loads issue before this tile's MFMAs, LDS
-//     writes after -- guide §5.5 T14); one barrier per tile.
+//     writes after); one barrier per tile.
 //   * <= 128 VGPRs so two workgroups (16 waves, 4 per SIMD) share a CU: one wave's softmax VALU
 //     overlaps another's MFMAs (a 1-wave-per-SIMD build of this loop was VALU-serialised).
 //   * VALU trimmed: Q is pre-scaled by softmax_scale*log2(e) once (scores come out of the MFMA
 //     in the exp2 domain), the causal mask is applied only on tiles that cross the diagonal, and
-//     the O rescale is deferred until the running max grows by > RESCALE_THR (guide T13; P is
+//     the O rescale is deferred until the running max grows by > RESCALE_THR (P is
 //     then bounded by 2^THR, exact after the final 1/l).
 //   * The host orders tiles heaviest-first (most keys) so the causal triangle drains evenly.
 // ------------------------------------------------------------------------------------------
@@ -661,7 +661,7 @@ __global__ void __launch_bounds__(512, MINW) prefill_paged_kernel(
 //     over D = 128).  C/D of 32x32: col = lane & 31 (query), row = 8(i>>2) + 4(lane>>5) + (i&3)
 //     (key), so each lane owns one query row's scores for 16 of every 32 keys (the other 16 in
 //     lane ^ 32): row max / sum = 31 local ops + one xor-32 shuffle.
-//   * O^T = V^T . P^T: the S^T accumulator IS the P^T B-operand (guide §3: k-step s of a 32-key
+//   * O^T = V^T . P^T: the S^T accumulator IS the P^T B-operand (k-step s of a 32-key
 //     tile = registers 8s..8s+7, key order 16s + 8(j>>2) + 4h + (j&3)); the V^T LDS image stores
 //     each d row's 64 keys in exactly that slot order, so the A fragment is one ds_read_b128.
 //     The cache's V^T blocks are in the decode (16x16) slot order; the permutation to the 32x32
@@ -1383,7 +1383,7 @@ __global__ void __launch_bounds__(256, D == 32 ? 5 : 2) encoder_attn_kernel(cons
       float tmax = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])),
                          fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
       tmax = quad_max(tmax);
-      // deferred rescale (guide T13, as in the prefill kernel): O and l are rescaled only when the
+      // deferred rescale (as in the prefill kernel): O and l are rescaled only when the
       // running max grows by more than RESCALE_THR, not on every 32-key step -- the per-step
       // multiply of O (held in AGPRs) cost a read / multiply / write per register
       if (!__all(tmax - m[rg] <= RESCALE_THR)) {

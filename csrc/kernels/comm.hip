@@ -1,5 +1,5 @@
 // One-shot all-reduce over IPC-mapped peer buffers (xGMI point-to-point), for the latency-bound
-// tensor-parallel decode collectives (SURVEY §5.8 / §7.4: 64 per token, each B x hidden bf16).
+// tensor-parallel decode collectives (64 per token, each B x hidden bf16).
 //
 // Every rank owns ONE shared region, allocated uncached (fine-grained: stores write through and
 // remote loads are never served from a stale L2 line) and exported with hipIpcGetMemHandle:

@@ -3,7 +3,7 @@
 // Conventions used by every kernel in this directory:
 //   * bf16 tensors are passed as `const uint16_t*` / `uint16_t*` (raw bits) and converted with
 //     the helpers below; vector loads go through 16-byte `uint4` (8 bf16) whenever the row
-//     length allows it (guide §6 Guideline 13: scalar bf16 loads cost 2-2.5x).
+//     length allows it (scalar bf16 loads cost 2-2.5x).
 //   * Wavefront = 64 lanes; block sizes are multiples of 64.
 //   * Every launcher is `extern "C"` and takes an explicit hipStream_t so PyTorch's current
 //     stream (and therefore hipGraph capture) is honoured.
@@ -169,7 +169,7 @@ __device__ __forceinline__ int share_of(int n, int p, int P) {
   return (int)(q * (uint32_t)p + r * (uint32_t)p / (uint32_t)P);
 }
 
-// XCD-aware bijective remap of a 1-D block id (guide §5 "XCD swizzle must be bijective"):
+// XCD-aware bijective remap of a 1-D block id:
 // consecutive logical tiles land on the same XCD so neighbouring tiles share that XCD's L2.
 __device__ __forceinline__ int xcd_remap(int orig, int nwg) {
   const int q = nwg / 8, r = nwg % 8, xcd = orig % 8;
@@ -218,7 +218,7 @@ __device__ __forceinline__ int kv_v_slot(int key_in_block) {
 // [4 slot groups][D][8 slots]: the 8 positions 8g..8g+7 of one d (one P.V MFMA fragment) are 16
 // contiguous bytes, and one token's column touches D * 2 B / 128 B = 16 cache lines (bf16, D = 128)
 // instead of 64 in a [D][32] tile -- the decode step's V write costs by lines dirtied
-// (profiles/ROOFLINE.md, round 6).
+// (profiles/ROOFLINE.md).
 __device__ __forceinline__ int kv_v_off(int d, int p, int D) { return (p >> 3) * (D * 8) + d * 8 + (p & 7); }
 
 // 8 consecutive qkv values of token row element offset `off`: from the bf16 qkv, or summed from

@@ -19,7 +19,7 @@
 //     register ring (D = 8 x 64-deep K stages = 16 KB per wave in flight, the GEMV's depth).  Its
 //     only vector-memory instructions are those loads, so hipcc's own counted vmcnt waits are
 //     exact and never drain the ring; every load is unconditional (the tail re-reads the last
-//     stage) so no branch joins force a vmcnt(0) (round-2 finding);
+//     stage) so no branch joins force a vmcnt(0);
 //   * X (an L2 hit, shared by all compute waves) is staged by the 2 loader waves with LDS-DMA
 //     (`global_load_lds_dwordx4`, written in asm so hipcc orders nothing behind it) into an
 //     NSX-slot LDS ring; only the loaders wait on vmcnt for it (counted, in one asm statement with
@@ -27,15 +27,15 @@
 //     vmcnt counter;
 //   * the X image is lane-linear per DMA piece and XOR-swizzled through the SOURCE address: chunk
 //     c of row r at r*128 + ((c ^ (r & 7)) << 4), so the 16-row ds_read_b128 A-fragment reads are
-//     bank-conflict free (guide rule 21 / T2);
+//     bank-conflict free;
 //   * split-K over the grid for the small-N projections; blocks are remapped XCD-locally so the
-//     blocks of one XCD share a K slice and therefore the same X slice in that XCD's L2 (guide T1);
+//     blocks of one XCD share a K slice and therefore the same X slice in that XCD's L2;
 //   * epilogues: fp32 split-K partials (reduced by the residual + RMSNorm / SwiGLU reduce), bf16,
 //     or SwiGLU over gate/up weights interleaved in 8-row groups (each 16-row n-tile = 8 gate +
 //     8 up rows, so silu(g) * u is one lane swap away; same bf16 rounding points as
 //     GEMM -> silu_mul).
 //
-// MFMA maps (guide §3): A = X rows (m on lane & 15, k = 8 * (lane >> 4) + j), B = W rows (n on
+// MFMA maps: A = X rows (m on lane & 15, k = 8 * (lane >> 4) + j), B = W rows (n on
 // lane & 15, same k); C/D: n = lane & 15, m = 4 * (lane >> 4) + i.
 #include <algorithm>
 
@@ -84,7 +84,7 @@ __device__ __forceinline__ f32x4_t dg_mfma(uint4 a, uint4 b, f32x4_t c) {
 
 // One 1-KB LDS-DMA piece: lane l's 16 source bytes land at lds_addr + 16 l.  Inline asm, so hipcc
 // sees no LDS write to order the compute waves' ds_reads behind; M0 (compiler-reserved) is saved
-// and restored inside the statement (guide §5.7).
+// and restored inside the statement.
 __device__ __forceinline__ void dg_glds16(const void* gsrc, uint32_t lds_addr) {
   unsigned keep;
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
@@ -139,7 +139,7 @@ __device__ __forceinline__ uint4 dg_ldw(const uint16_t* p) {
 //   32 = contiguous W pieces: wave w loads fragments 2w, 2w+1 of the stage's 2 NW KB region (one
 //   2-KB run per wave) instead of its own group's two 1-KB fragments NW KB apart (wrong sums);
 //   64 = two X-loader waves + an 8-slot X ring (DgShape MX);
-//   256 = the round-5 tail (re-reads the last stage instead of issuing no loads);
+//   256 = the former tail (re-reads the last stage instead of issuing no loads);
 //   128 = no workgroup barrier in the compute waves' stage loop (with 1 only: the loader waves
 //   return at once) -- is the per-stage lockstep of the compute waves what slows the W stream?
 // PACKED: W in the fragment-packed layout of cfc_dgemm_pack for this BN: tile-major, then 32-deep
@@ -150,7 +150,7 @@ __device__ __forceinline__ uint4 dg_ldw(const uint16_t* p) {
 // 8 KB row stride) stream at 3.8-4.2 TB/s however deep the ring; contiguous 1-KB pieces at
 // 6.0 TB/s from the same 224-256 workgroups.  Packed loads are buffer loads (32-bit offsets into
 // the workgroup's span) so the cache policy can be set: NTW = nontemporal for these once-read
-// bytes (guide "nt-weights").
+// bytes.
 // GRP 1: one matrix per expert, W[experts][N][K] packed one after the other.  grid.y walks the row tiles of a
 // batch sorted by expert: tile y multiplies rows y BM .. by matrix tile_expert[y] (negative: no such tile, the
 // workgroup leaves), row m of it being row rows[m] of X (rows null: m itself); M counts the sorted rows.
@@ -199,7 +199,7 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
   auto phys = [&](int s) { s += rot; return s >= nst ? s - nst : s; };
 
   constexpr bool NOBAR = (ABL & 128) != 0;
-  // XT: the MFMA's A operand is the W fragment, B the X fragment (probe 512: the round-5
+  // XT: the MFMA's A operand is the W fragment, B the X fragment (probe 512: the former
   // orientation, X as A, one output element per lane per row -> 4-byte epilogue stores)
   constexpr bool XT = (ABL & 512) == 0;
   static_assert(!NOBAR || (ABL & 1), "no-barrier probe only without the X stream");
@@ -241,7 +241,7 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
   // ---------------- compute wave w: W rows n0 + 16 w + (lane & 15)
   uint4 ring[D][2];
   // packed: the workgroup's span, tile n0 / BN over all of K (split slices are sub-ranges of it),
-  // as a buffer descriptor built from wave-uniform values (guide T20: no waterfall loops)
+  // as a buffer descriptor built from wave-uniform values (no waterfall loops)
   const uint16_t* span = W + (size_t)(n0 / BN) * ((size_t)BN * K);
   const uint32_t span_lo = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)span);
   const uint32_t span_hi = __builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)span >> 32));
@@ -306,10 +306,10 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
   // s + D.  Every load is unconditional (a branch around a load makes hipcc drain the ring at the
   // join), so the last D refills of a slice name stages past its end: on the packed path they are
   // buffer loads at an offset past the descriptor's range, which return zeros without touching
-  // memory (round 5 and before re-read the last stage D times instead: up to half of a small
+  // memory (it re-read the last stage D times instead: up to half of a small
   // slice's loads, e.g. 8 redundant 2-KB stages per wave of qkv's 16 at split 4).  The ring is never
   // read past the slice (the tail computes only real stages).
-  constexpr bool TAIL_RELOAD = (ABL & 256) != 0;    // probe: the round-5 re-reading tail
+  constexpr bool TAIL_RELOAD = (ABL & 256) != 0;    // probe: the former tail, which reads again
   int st = 0;
   for (; st + D <= nst; st += D) {
 #pragma unroll
@@ -331,7 +331,7 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
   if constexpr (XT) {
     // ---- epilogue: lane holds X row m0 + 16 i + (lane & 15) at the four consecutive W rows (output
     // columns) n0 + 16 w + 4 (lane >> 4) + r, r = 0..3 -- one 16-byte (fp32) / 8-byte (bf16) store per
-    // lane and m-tile, 16 rows x 64 B per wave instruction (the round-5 orientation stored 4 bytes
+    // lane and m-tile, 16 rows x 64 B per wave instruction (the former orientation stored 4 bytes
     // per lane: 4x the store instructions, the epilogue's store-issue tail of a small-N projection)
     const int mr = m0 + (lane & 15);
     const int nq = n0 + 16 * w + 4 * kq;
@@ -360,7 +360,7 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
       }
     } else if constexpr (EPI == DG_PART_WT) {
       // write-through (sc1) 16-byte stores through a buffer descriptor of the slab array (the
-      // guide's R1 form: the consumer kernel reads them from memory, no dirty lines at the boundary)
+      // consumer kernel reads them from memory, no dirty lines at the boundary)
       const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)part);
       const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)part >> 32));
       const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
@@ -390,7 +390,7 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
     }
     return;
   }
-  // ---- epilogue (round-5 orientation): lane holds rows m0 + 16 i + 4 (lane >> 4) + r of W row n
+  // ---- epilogue (the former orientation): lane holds rows m0 + 16 i + 4 (lane >> 4) + r of W row n
   const int n = n0 + 16 * w + (lane & 15);
   const int mb = m0 + 4 * kq;
   if constexpr (EPI == DG_SILU) {

@@ -4,9 +4,9 @@
 //   * bias + GELU (erf) for the BERT FFN
 //   * token-embedding gather
 //   * greedy argmax / Gumbel-max temperature sampling + on-device decode-state advance, so a
-//     whole decode step (and the EOS/stop check, SURVEY K17) replays from a hipGraph with no
+//     whole decode step (and the EOS/stop check) replays from a hipGraph with no
 //     host synchronisation.
-// All loads/stores are 16-byte vectors (guide §6 Guideline 13).
+// All loads/stores are 16-byte vectors.
 #include "common.h"
 
 namespace {

@@ -17,7 +17,7 @@
 //     the candidates are merged by cfc_topk_select.
 //   * cfc_l2_normalize: rows -> unit length (+ fp32 norms), used on insert for cosine.
 //   * cfc_pool: masked mean / CLS pooling over varlen sequences (+ optional L2 normalise):
-//     the SentenceTransformer Pooling+Normalize modules (SURVEY §2.5 K7).
+//     the SentenceTransformer Pooling+Normalize modules.
 #include "common.h"
 
 namespace {

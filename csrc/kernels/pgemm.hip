@@ -15,11 +15,11 @@
 //     tile (its counted wait retires tile t's DMA and the previous tile's ds_reads together);
 //   * each LDS image is 256 rows x 128 B, XOR-swizzled through the SOURCE address (chunk c of row r
 //     at r * 128 + ((c ^ (r & 7)) << 4)), so the 16-row ds_read_b128 fragment reads are
-//     bank-conflict free (guide rule 21 / T2) -- the same image as the decode GEMM's X stage;
+//     bank-conflict free -- the same image as the decode GEMM's X stage;
 //   * operands swapped in the MFMA (W fragment as A, X fragment as B) so each lane's accumulator
 //     holds 4 CONSECUTIVE output columns of one row: the epilogue stores 8 bytes per lane straight
 //     from registers, and SwiGLU's gate/up pairs are one lane swap (v_permlane32_swap) away;
-//   * blockIdx -> tile: bijective XCD remap (guide T1), then groups of 8 M-tiles sweep the N-tiles,
+//   * blockIdx -> tile: bijective XCD remap, then groups of 8 M-tiles sweep the N-tiles,
 //     so the ~32 workgroups resident on one XCD share X rows and W rows in that XCD's L2.
 //
 // Epilogues: bf16; + bias (encoder qkv); + bias -> GELU(erf) (encoder FFN up); SwiGLU over 8-row
@@ -215,13 +215,13 @@ __global__ void __launch_bounds__(512, 1)
 // then one raw barrier: step t + 1 is readable everywhere and step t's slot (in registers in every
 // wave) is free, so the DMA of step t + R goes into it right away.  A slot's DMA thus has R - 1
 // steps of MFMA work (~1k cycles per step per SIMD pair) to land, against one 64-deep tile in the
-// 2-stage kernel: what that kernel waits for at its vmcnt(0) (guide "Pipelining across barriers").
+// 2-stage kernel: what that kernel waits for at its vmcnt(0).
 //
 // 64-B image rows: 4 rows share a 256-B bank row, so the 16-row fragment read (lane: row
 // lane & 15, chunk lane >> 4) is swizzled as chunk' = chunk ^ f((row >> 2) & 3), f = 0,3,2,1: every
 // ds_read_b128 lane group then covers the 16 bank slots of one bank row exactly once.  The DMA
 // writes lane-linear (16-row x 64-B piece per wave instruction), so the swizzle goes on its source
-// chunk (guide rule 21).
+// chunk.
 constexpr int PR_BK = 32;
 constexpr int PR_SLOT = (PG_BM + PG_BN) * PR_BK * 2;   // 32 KB
 
@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(512, 1)
 // covers either.  Here the 8 waves are two groups of 4 (waves 0-3, 4-7: one of each on every SIMD),
 // run one barrier apart, so on each SIMD one wave's MFMA segment covers its partner's load segment
 // (LDS-DMA issue, fragment ds_reads, counted vmcnt) and the matrix pipe never waits for either
-// (guide §5 "The 256² 8-phase template", MI355X_MICROARCH "Two waves per SIMD").
+// (a 256 x 256 tile in eight phases, two waves per SIMD).
 //
 //   * tile 256 x 256, BK = 64; wave (grp, wc) owns output rows 128 grp .. +128, cols 64 wc .. +64;
 //   * a K-tile is 4 half-tiles of 16 KB: X0 = X tile rows {0-63, 128-191}, X1 = {64-127, 192-255},
@@ -366,7 +366,7 @@ __global__ void __launch_bounds__(512, 1)
 //     2-3 half-tiles of DMA in flight per wave (48-64 KB per CU) and retire exactly what the next
 //     segment reads, one barrier (two for the lagging group) ahead of the read;
 //   * X image: 128 rows x 128 B per half, chunk c of image row r at r*128 + ((c ^ (r & 7)) << 4)
-//     (swizzled through the DMA SOURCE address, guide rule 21), 8-row x 128-B pieces;
+//     (swizzled through the DMA SOURCE address), 8-row x 128-B pieces;
 //   * W: row-major as X, or fragment-packed (the decode GEMM's cfc_dgemm_pack layout, wnw = its
 //     bn / 16): every 16-row x 32-k MFMA fragment is 1 KB contiguous in lane order, so each DMA piece
 //     is one whole fragment and its ds_read_b128 at lane * 16 is conflict free -- one weight copy
@@ -980,7 +980,7 @@ __global__ void __launch_bounds__(512, 1)
 // K = 4 x hidden) for hidden NC16 x 16 (384: MiniLM / bge-small).  A workgroup owns WHOLE rows: a
 // 128-row x N tile, so the row statistics of the LayerNorm are reduced inside it (waves' partial
 // sums through LDS) and the normalised row is written once -- no bf16 round trip of the projection
-// output and no separate residual + LayerNorm pass (SURVEY K5 / K6).
+// output and no separate residual + LayerNorm pass.
 //   * 8 waves = 2 (M) x 4 (N), wave tile 64 rows x N/4 columns: acc[4][NC16/4] tiles of 16 x 16;
 //   * K in 64-deep tiles, A (128 rows) and B (N rows) images staged by LDS-DMA in 8-row x 128-B
 //     pieces, XOR-swizzled through the source address as the 2-stage kernel, two LDS stages;
@@ -1123,7 +1123,7 @@ __global__ void __launch_bounds__(512, 1)
 // r03s2_pmc_pgemm_vs_hipblaslt.txt): a wave owns a 128 x 128 output block (64 accumulator tiles,
 // 256 registers -- the AGPR half of the file), so each MFMA costs half the LDS fragment bytes of the
 // 8-wave kernels' 128 x 64 blocks (16 ds_read_b128 per 64 MFMAs) -- less LDS traffic and less
-// energy per flop, which is what the clock under DVFS rewards (guide §5.4 rule 28).  With one wave
+// energy per flop, which is what the clock under DVFS rewards.  With one wave
 // per SIMD nothing else covers its waits, so the wave pipelines itself:
 //   * K in 32-deep steps through a ring of 4 LDS stages (X image 256 rows x 64 B + W image 16
 //     fragments, 32 KB per stage); the DMA of step t + 4 is issued at the top of step t into the
@@ -1281,7 +1281,7 @@ constexpr bool PPP_STG = true;
 
 // M-tiles per N sweep of the persistent kernel's tile order.  Measured (scripts/probe_ppp_gm.py,
 // profiles/r06_ppp_gm.jsonl, gm 2 / 4 / 8 / 16): 8 is best on qkv, o and gate_up; the long-K,
-// narrow-N down projection (K = 14336, 16 N-tiles) runs 2.3 % faster at 4 (round 4 saw the same
+// narrow-N down projection (K = 14336, 16 N-tiles) runs 2.3 % faster at 4 (the same was seen
 // on the one-tile kernel: r04_pgemm_pp_probes.jsonl)
 int ppp_group_m(int tiles_n, int K) { return (K >= 8192 && tiles_n <= 16) ? 4 : PG_GROUP_M; }
 

@@ -2,7 +2,7 @@
 //   * ASan + UBSan: BPE build/encode/decode/train, WordPiece, mbox splitting, block pool;
 //   * TSan: the block pool under concurrent alloc/free from several threads (the engine, the
 //     bench's prepare worker and the prefix cache can touch it from different threads).
-// (GPU sanitizers / XNACK are not available on the GPU pool; the kernels are covered by the
+// (GPU sanitizers / XNACK are not available; the kernels are covered by the
 // fp32-reference numerics tests instead.)
 #include <cstdint>
 #include <cstdio>

@@ -12,7 +12,7 @@
 //    max-heap), so 32k merges over a multi-MB corpus take seconds, not hours.
 //
 // The reference tokenises inside HF `tokenizers` (Rust) / sentence-transformers and inside
-// llama.cpp (SURVEY §2.5 K1); these are the native replacements.  All entry points are extern "C".
+// llama.cpp; these are the native replacements.  All entry points are extern "C".
 #include <algorithm>
 #include <cstdint>
 #include <cstring>
