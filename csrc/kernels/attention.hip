@@ -26,6 +26,8 @@
 #include "common.h"
 #include <stdlib.h>
 
+#include <type_traits>
+
 namespace {
 
 constexpr int KV_BS = 32;          // tokens per KV-cache block
@@ -1251,13 +1253,16 @@ __global__ void __launch_bounds__(512, 2) prefill_gqa_kernel(
 // Softmax: Q is pre-scaled by scale*log2(e) at load, the key mask runs only on the sequence's
 // last (partial) 32-key tile, exponentials are v_exp_f32 (inputs <= 0).
 // ------------------------------------------------------------------------------------------
-constexpr int ENC_R = 4;               // 16-row query groups per wave
-constexpr int ENC_ROWS = 64 * ENC_R;   // query rows per workgroup
+constexpr int ENC_ROWS = 256;          // query rows per workgroup, 16 ENC_R of a wave
+constexpr float ENC_NONE = 3e38f;      // less a maximum that no score is below; finite, so that a score of -inf keeps its weight of 0
 
-// As many workgroups on a CU as their LDS lets there be (heads of 32: 96 registers, 90 -> 74 us for 365 texts of 180 tokens, x 12
-// heads; with V^T by four keys and waves of every fourth row group 68).
-template <int D>
-__global__ void __launch_bounds__(256, D == 32 ? 5 : 2) encoder_attn_kernel(const uint16_t* __restrict__ qkv,
+// Vector instructions bound it: 32 keys of 16 rows are 8 exponentials a lane, a quarter of the rate of others, and were some 40
+// others, 14 of them for a maximum and a sum across lanes in every step.  Now scores start from the maximum (an MFMA's
+// addend), a lane compares and sums its own keys only and the end masks in a copy of the step: some 22 others, 16 VGPRs more,
+// so four workgroups a CU where there were five.  Texts of up to 128 tokens have two row groups a wave, and six workgroups.
+// us a layer: 365 texts of 180 tokens, 12 heads of 32, 72 -> 61; forwards of 800 texts of 30 in all 953 -> 923, of 100 2868 -> 2784.
+template <int D, int ENC_R>
+__global__ void __launch_bounds__(256, D == 32 ? (ENC_R == 4 ? 4 : 6) : 2) encoder_attn_kernel(const uint16_t* __restrict__ qkv,
                                                            const int32_t* __restrict__ cu_seqlens,
                                                            const int32_t* __restrict__ tile_seq,
                                                            const int32_t* __restrict__ tile_q0, float scale_log2,
@@ -1271,7 +1276,7 @@ __global__ void __launch_bounds__(256, D == 32 ? 5 : 2) encoder_attn_kernel(cons
   // fetched from HBM once into that XCD's L2 instead of once per XCD.
   const int lb = xcd_remap(blockIdx.x, gridDim.x);
   const int t = lb / H, h = lb - t * H;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, tid = threadIdx.x;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tid = threadIdx.x;
   const int col = lane & 15, g = lane >> 4;
   const int s = tile_seq[t], qs = tile_q0[t];
   const int beg = cu_seqlens[s], S = cu_seqlens[s + 1] - beg;
@@ -1341,16 +1346,18 @@ __global__ void __launch_bounds__(256, D == 32 ? 5 : 2) encoder_attn_kernel(cons
   if (ng == 0) return;   // no barrier follows
 
   f32x4_t o[ENC_R][DT];
-  float m[ENC_R], l[ENC_R];
+  float l[ENC_R];                 // a lane's own keys' share of the sums until the end
+  f32x4_t ref[ENC_R];             // less the running maxima, what the scores start from: no subtraction is left for later
 #pragma unroll
   for (int rg = 0; rg < ENC_R; ++rg) {
-    m[rg] = -INFINITY;
+    ref[rg] = f32x4_t{ENC_NONE, ENC_NONE, ENC_NONE, ENC_NONE};
     l[rg] = 0.f;
 #pragma unroll
     for (int i = 0; i < DT; ++i) o[rg][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  for (int k0 = 0; k0 < S; k0 += 32) {
+  auto keys = [&](int k0, auto last) {
+    constexpr bool TAIL = decltype(last)::value;      // fewer than 32 keys
     bf16x8_t kf[2][KSTEPS];
 #pragma unroll
     for (int st = 0; st < 2; ++st)
@@ -1361,56 +1368,65 @@ __global__ void __launch_bounds__(256, D == 32 ? 5 : 2) encoder_attn_kernel(cons
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
       vf[dt] = as_bf16x8(*reinterpret_cast<const uint4*>(vlds + voff_chunk(16 * dt + col, (k0 >> 3) + g)));
-    const bool tail = k0 + 32 > S;
 
 #pragma unroll
     for (int rg = 0; rg < ENC_R; ++rg) {
       if (rg >= ng) break;
       f32x4_t sc[2];
+      auto scores = [&](const f32x4_t& from) {
 #pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        sc[st] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int st = 0; st < 2; ++st) {
+          sc[st] = from;
 #pragma unroll
-        for (int c = 0; c < KSTEPS; ++c) sc[st] = mfma16(kf[st][c], qf[rg][c], sc[st]);
-      }
-      if (tail) {
+          for (int c = 0; c < KSTEPS; ++c) sc[st] = mfma16(kf[st][c], qf[rg][c], sc[st]);
+        }
+        if constexpr (TAIL) {
 #pragma unroll
-        for (int st = 0; st < 2; ++st)
+          for (int st = 0; st < 2; ++st)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (k0 + 16 * st + 4 * g + i >= S) sc[st][i] = -INFINITY;
-      }
-      float tmax = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])),
-                         fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
-      tmax = quad_max(tmax);
-      // deferred rescale (as in the prefill kernel): O and l are rescaled only when the
-      // running max grows by more than RESCALE_THR, not on every 32-key step -- the per-step
-      // multiply of O (held in AGPRs) cost a read / multiply / write per register
-      if (!__all(tmax - m[rg] <= RESCALE_THR)) {
-        const float mn = fmaxf(m[rg], tmax);
-        const float alpha = __builtin_amdgcn_exp2f(m[rg] - (mn == -INFINITY ? 0.f : mn));
+            for (int i = 0; i < 4; ++i)
+              if (k0 + 16 * st + 4 * g + i >= S) sc[st][i] = -INFINITY;
+        }
+      };
+      // three values an instruction
+      auto largest = [&]() {
+        const float a = fmaxf(fmaxf(sc[0][0], sc[0][1]), sc[0][2]), b = fmaxf(fmaxf(sc[1][0], sc[1][1]), sc[1][2]);
+        return fmaxf(fmaxf(fmaxf(a, sc[0][3]), b), sc[1][3]);
+      };
+      scores(ref[rg]);
+      // The running maximum moves, and O and l with it, only where a score exceeds it by more than RESCALE_THR (as in the
+      // prefill kernel); each lane looks at its own keys, so nothing crosses lanes where none does.  Before the first
+      // keys it lies below all scores.
+      if (!__all(largest() <= RESCALE_THR)) {
+        scores(f32x4_t{0.f, 0.f, 0.f, 0.f});
+        const float m = -ref[rg][0], mn = fmaxf(m, quad_max(largest()));
+        const float alpha = __builtin_amdgcn_exp2f(m - mn);
         l[rg] *= alpha;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[rg][dt] *= alpha;
-        m[rg] = mn;
+        ref[rg] = f32x4_t{-mn, -mn, -mn, -mn};
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sc[st][i] -= mn;
       }
-      const float mref = m[rg] == -INFINITY ? 0.f : m[rg];
-      float rs = 0.f;
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float e = __builtin_amdgcn_exp2f(sc[st][i] - mref);
-          sc[st][i] = e;
-          rs += e;
+          sc[st][i] = __builtin_amdgcn_exp2f(sc[st][i]);
+          l[rg] += sc[st][i];
         }
-      rs = quad_sum(rs);
-      l[rg] += rs;
       const bf16x8_t pf = pack_p(sc[0], sc[1]);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) o[rg][dt] = mfma16(vf[dt], pf, o[rg][dt]);
     }
-  }
+  };
+  int k0 = 0;
+  for (; k0 + 32 <= S; k0 += 32) keys(k0, std::false_type{});
+  if (k0 < S) keys(k0, std::true_type{});
+#pragma unroll
+  for (int rg = 0; rg < ENC_R; ++rg) l[rg] = quad_sum(l[rg]);
 
 #pragma unroll
   for (int rg = 0; rg < ENC_R; ++rg) {
@@ -1673,12 +1689,15 @@ CFC_API int cfc_encoder_attention(const void* qkv, const int32_t* cu_seqlens, co
   if (max_seqlen > 512) return -2;
   const int spad = (max_seqlen + 127) & ~127;
   const size_t lds = (size_t)spad * head_dim * 2 * 2;
+#define ENC_GO(D, R)                                                                                                   \
+  encoder_attn_kernel<D, R><<<dim3(n_tiles * H), 256, lds, stream>>>((const uint16_t*)qkv, cu_seqlens, tile_seq, tile_q0, \
+                                                                     scale * LOG2E, H, (uint16_t*)out)
   if (head_dim == 32) {
-    encoder_attn_kernel<32><<<dim3(n_tiles * H), 256, lds, stream>>>((const uint16_t*)qkv, cu_seqlens, tile_seq, tile_q0,
-                                                                    scale * LOG2E, H, (uint16_t*)out);
+    if (max_seqlen <= 128) ENC_GO(32, 2);
+    else ENC_GO(32, 4);
   } else if (head_dim == 64) {
-    encoder_attn_kernel<64><<<dim3(n_tiles * H), 256, lds, stream>>>((const uint16_t*)qkv, cu_seqlens, tile_seq, tile_q0,
-                                                                    scale * LOG2E, H, (uint16_t*)out);
+    if (max_seqlen <= 128) ENC_GO(64, 2);
+    else ENC_GO(64, 4);
   } else {
     return -1;
   }

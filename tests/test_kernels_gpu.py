@@ -226,6 +226,31 @@ def test_encoder_attention(D):
     _close(out, ref, 2e-2)
 
 
+@pytest.mark.parametrize("D,longest", [(32, 1), (32, 32), (32, 127), (32, 128), (32, 129), (64, 33), (64, 128), (64, 512)])
+def test_encoder_attention_steps(D, longest):
+    """Maxima that grow from one step of 32 keys to the next by less and by more than what moves them, keys without weight
+    (-inf scores) first, texts at the edges of steps, row groups and of the texts that take two groups a wave."""
+    H, dt = 3, torch.bfloat16
+    lens = [n for n in (1, 31, 32, 33, 63, 65, 96, 128, 257) if n < longest] + [longest]
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    T = int(cu[-1])
+    g = torch.Generator().manual_seed(longest)
+    qkv = torch.randn(T, 3, H, D, generator=g)
+    at = torch.cat([torch.arange(n) for n in lens])
+    qkv[:, 1, 0] *= 0.5 * (at[:, None] // 32).clamp(max=4) + 0.5     # the first head's scores grow with the keys, to about 10
+    qkv[:, :2, 1] = qkv[:, :2, 1].abs()
+    qkv[:, 1, 1] = torch.where((at[:, None] // 32) % 2 == 1, qkv[:, 1, 1], -3e38)    # the second's: none in every other step
+    qkv = qkv.to(dt).view(T, -1)
+    out = K.encoder_attention(qkv.to(DEV), cu.to(DEV), H, D, 1 / math.sqrt(D), max(lens)).float().cpu().view(T, H, D)
+    ref = R.encoder_attention(qkv, cu, H, D, 1 / math.sqrt(D)).float().view(T, H, D)
+    some = torch.cat([torch.full((n,), n > 32) for n in lens])       # texts with a finite score of the second head
+    # queries are rounded to bf16 after their scale, 2^-9 of scores of 10: weights off by 2 %, by 2^-9 more as operands, of
+    # values of about 1, up to 4
+    _close(out[:, 0::2], ref[:, 0::2], 4e-2)
+    if bool(some.any()):
+        _close(out[some, 1], ref[some, 1], 4e-2)
+
+
 def test_silu_mul_and_gelu():
     gu = torch.randn(33, 2 * 1536, device=DEV).bfloat16()
     _close(K.silu_mul(gu), R.silu_mul(gu.cpu()), 2e-2)
