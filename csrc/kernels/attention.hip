@@ -32,6 +32,8 @@ namespace {
 
 constexpr int KV_BS = 32;          // tokens per KV-cache block
 constexpr float LOG2E = 1.4426950408889634f;
+constexpr int DEC_ORDER_ROWS = 128;   // sequences that longest_first orders at most: two threads of 256 each
+constexpr int DEC_ORDER_FROM = 1024;  // the longest context from which it does
 
 __device__ __forceinline__ bf16x8_t as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8_t, v); }
 
@@ -113,6 +115,42 @@ __device__ __forceinline__ uint4 set_bf16(uint4 v, int e, uint32_t h) {
   return make_uint4(put(v.x, 0), put(v.y, 1), put(v.z, 2), put(v.w, 3));
 }
 
+// {sequence, its context} of the one that has `rank` others before it, longest contexts first (of equal ones the first
+// first): more workgroups than the chip holds at once start as others end, and a long one that starts last is waited for
+// alone.  In the order that they have where the contexts are short or differ by no more than `least` sixteenths of the
+// longest: the ranking, 0.5 us a workgroup, would be more than it saves.
+__device__ __forceinline__ int2 longest_first(const int32_t* __restrict__ ctx_lens, int B, int rank, int least) {
+  __shared__ __attribute__((aligned(16))) int key[DEC_ORDER_ROWS], before[DEC_ORDER_ROWS], ends[4];
+  __shared__ int found;
+  const int t = threadIdx.x, s = t & (DEC_ORDER_ROWS - 1), n = ctx_lens[min(s, B - 1)];     // two threads a sequence
+  const int lo = wave_min_int(n), hi = -wave_min_int(-n);
+  if (t < DEC_ORDER_ROWS) {
+    key[t] = t < B ? (n << 8) + (255 - t) : -1;
+    before[t] = 0;
+    if ((t & 63) == 0) ends[t >> 5] = lo, ends[(t >> 5) + 1] = hi;
+  }
+  __syncthreads();
+  const int4 e = *reinterpret_cast<const int4*>(ends);
+  const int longest = max(e.y, e.w);
+  int b = rank;
+  if (__builtin_amdgcn_readfirstlane(longest >= DEC_ORDER_FROM && (longest - min(e.x, e.z)) * 16 > least * longest)) {
+    const int own = key[s];
+    int c = 0;
+#pragma unroll 8
+    for (int j = 0; j < DEC_ORDER_ROWS / 2; j += 4) {              // each with half of the others
+      const int4 k = *reinterpret_cast<const int4*>(key + (t & DEC_ORDER_ROWS) / 2 + j);
+      c += (k.x > own) + (k.y > own) + (k.z > own) + (k.w > own);
+    }
+    atomicAdd(before + s, c);
+    __syncthreads();
+    if (t < B && before[t] == rank) found = t;
+    __syncthreads();
+    b = found;
+  }
+  b = __builtin_amdgcn_readfirstlane(b);
+  return make_int2(b, __builtin_amdgcn_readfirstlane(key[b] >> 8));
+}
+
 struct DecRope {
   const uint16_t* qkv;     // [B, (Hq + 2 Hkv) D] bf16, or nullptr with part
   const float* part;       // [split, B, (Hq + 2 Hkv) D] fp32 split-K slabs
@@ -162,16 +200,24 @@ __global__ void __launch_bounds__(256, F8 ? 2 : 1) paged_decode_kernel(
     const uint16_t* __restrict__ q, const void* __restrict__ kc, const void* __restrict__ vc,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ ctx_lens, float scale_log2, int Hkv,
     int max_blocks, int part_blocks, int P, int window, float v_scale, float* __restrict__ part_o,
-    float* __restrict__ part_ml, uint16_t* __restrict__ out, DecRope rp, const int32_t* __restrict__ shared_blocks) {
+    float* __restrict__ part_ml, uint16_t* __restrict__ out, DecRope rp, const int32_t* __restrict__ shared_blocks,
+    int ordered) {
   // F8: kc / vc hold e4m3 of K / k_scale and V / v_scale; k_scale is folded into scale_log2 by the
   // host, v_scale multiplies the output here
   typedef typename KvFrag<F8>::raw Raw;
   constexpr int D = 128;
-  const int p = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const int p = blockIdx.x, h = blockIdx.y;
+  int b = blockIdx.z, ctx;
+  if (ordered) {
+    const int2 s = longest_first(ctx_lens, gridDim.z, blockIdx.z, ordered);
+    b = s.x;
+    ctx = s.y;
+  } else {
+    ctx = ctx_lens[b];
+  }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
   const int Hq = Hkv * G;
-  const int ctx = ctx_lens[b];
   const int nblk = (ctx + KV_BS - 1) / KV_BS;
   // sliding window (window > 0): the query at position ctx-1 sees keys [ctx - window, ctx)
   const int key_lo = window > 0 ? max(0, ctx - window) : 0;
@@ -1463,8 +1509,15 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
   const int G = Hq / Hkv;
   dim3 grid(P, Hkv, B);
   const float sl2 = scale * LOG2E;
+  // Longest first where more workgroups than two a CU wait for a place.  Just above 512 only for contexts that differ by more than
+  // seven sixteenths: the few that are left over start when the first end, and those are longer in this order.  us of 8 key heads,
+  // one partition, contexts from 0.4 / 0.7 of 2600: 66 sequences 103 -> 92 / 132 -> 127, 72 114 -> 105 / 137 -> (144), 80 130 -> 116 /
+  // 143 -> (150), 104 157 -> 138 / 176 -> 165, 128 181 -> 159 / 197 -> 186; of 1100, 128 81 -> 73 / 88 -> 85.  136 and more: 0.95 to 1.08.
+  // Tables for less than the shortest that is ordered do not ask (the contexts' extremes take 0.5).
+  const int64_t wgs = (int64_t)P * Hkv * B;
+  const int ordered = wgs <= 512 || B > DEC_ORDER_ROWS || max_blocks * KV_BS < DEC_ORDER_FROM || max_blocks >= 1 << 17 ? 0 : wgs < 704 ? 7 : 2;
 #define DEC_ARGS (const uint16_t*)q, k_cache, v_cache, block_tables, ctx_lens, sl2, Hkv, max_blocks, part_blocks, P, \
-    window, v_scale, part_o, part_ml, (uint16_t*)out, rp, shared_blocks
+    window, v_scale, part_o, part_ml, (uint16_t*)out, rp, shared_blocks, ordered
   // nontemporal KV loads for large batches (B=128: 6.5 vs 5.9 TB/s; B=8: 3.8 vs 4.2 -- there the
   // plain loads win), profiles/decode_attn_partitions_r01.log; CFC_DECODE_NT=0/1 forces either
   static const int nt_env = [] { const char* e = getenv("CFC_DECODE_NT"); return e ? atoi(e) : -1; }();
