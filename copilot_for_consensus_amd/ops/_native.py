@@ -117,6 +117,7 @@ _KERNEL_SIGS = {
     "cfc_pgemm_ln": [P, P, P, P, P, P, P, I, I, I, F, P],
     "cfc_pgemm_probe": [P, P, P, I, I, I, I, I, I, P],
     "cfc_pgemm_ppp_probe": [P, P, P, I, I, I, I, I, I, I, P],
+    "cfc_ppp_height": [I, I, I],
     "cfc_pgemm_glu": [P, P, P, I, I, I, I, I, F, F, F, F, P],
     "cfc_prompt_plan": [I, I, I, I, P],
     "cfc_prompt_us": [I, I, I, I],

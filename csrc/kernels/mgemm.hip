@@ -240,11 +240,9 @@ double mgemm_x_us(int M, int N, int K, int split) {
   return 12.0 + (double)M * K * 2 * std::max(1.0, (double)std::min<int64_t>(8, runs) / split) / 7.6e6;
 }
 
-// pgemm's persistent kernel: a K-tile takes 1.4 in a full round of 256 x 256 tiles, 0.8 to 1.22 in a partial one
+// pgemm's persistent kernel, in tiles of the height it takes
 double ppp_us(int M, int N, int K, bool fp32) {
-  const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-  const int64_t full = tiles / MG_CUS, rest = tiles % MG_CUS;
-  return (12.0 + K / 64 * (1.4 * full + (rest ? 0.8 + 0.42 * rest / MG_CUS : 0.0))) * (fp32 ? 1.06 : 1.0);
+  return ppp_us_at(M, N, K, ppp_height(M, N, K)) * (fp32 ? 1.06 : 1.0);
 }
 
 enum { MG_ACT = 0, MG_SLABS = 1, MG_WHOLE = 2 };
@@ -275,7 +273,10 @@ double prompt_best(int M, int N, int K, int kind, int* plan) {
     return ppp_us(M, N, K, kind != MG_ACT);
   double all = mgemm_best(M, N, K, kind, kind != MG_WHOLE, true, bm, split);
   if (weights <= 1 << 23 && M <= (weights > 1 << 22 ? 256 : 640)) return all;       // the decode GEMM, within 10 %
-  double best = M < 256 ? 1e29 : 0.97 * ppp_us(M, N, K, kind != MG_ACT);
+  // a few rows beyond a whole round are faster here than its model says beside tiles of other heights than 256: 560 and 640
+  // rows of 28672 x 4096
+  const double bias = ppp_height(M, N, K) < 8 && M > 512 ? 1.04 : 0.97;
+  double best = M < 256 ? 1e29 : bias * ppp_us(M, N, K, kind != MG_ACT);
   const int tn = (N + 255) / 256, tm = (M + 255) / 256;
   if ((int64_t)tm * tn >= MG_PGEMM_TILES) all = std::max(all, mgemm_x_us(M, N, K, split));
   if (all < best) best = all, plan[1] = bm, plan[2] = split;

@@ -1,5 +1,7 @@
-// What the prompt GEMMs share: the LDS-DMA piece and the epilogues' arithmetic.
+// What the prompt GEMMs share: the LDS-DMA piece, the epilogues' arithmetic, and what the persistent kernel takes.
 #pragma once
+
+#include <algorithm>
 
 #include "common.h"
 
@@ -84,6 +86,33 @@ __device__ __forceinline__ float pg_out(float v) {
     return v * v;
   }
   return v;
+}
+
+// us of pgemm's persistent kernel in tiles of 32 mt x 256 (mt = 6, 7, 8): a K-tile of 256 rows takes 1.4 in a full round of
+// workgroups, 0.8 to 1.22 in a partial one; of 224 rows 0.91 of that, of 192 0.83, on an idle chip 0.95 and 0.88 to 0.97 (what
+// the waves read from LDS, not the MFMAs, takes the time there).
+inline double ppp_us_at(int M, int N, int K, int mt) {
+  constexpr int CUS = 256;
+  const int64_t tiles = (int64_t)((M + 32 * mt - 1) / (32 * mt)) * ((N + 255) / 256);
+  const double full = (double)(tiles / CUS), fill = (double)(tiles % CUS) / CUS;
+  const double part = fill > 0 ? 0.8 + 0.42 * fill : 0.0;
+  const double all = mt == 6 ? 0.83 : mt == 7 ? 0.91 : 1.0;
+  const double idle = mt == 6 ? (full > 0 ? 0.14 : 0.05) : mt == 7 && full > 0 ? 0.04 : 0.0;
+  return 12.0 + K / 64 * (1.4 * full * all + part * (all + idle * (1.0 - fill)));
+}
+
+// The height that takes the least: fewer rows than 256 where they leave fewer rows of the last tile unused or fill the last
+// round (us of 28672 x 4096 + SwiGLU, 256 rows -> this: 300 / 384 rows 96 -> 85 / 97 -> 83 in 192, 420 95 -> 90 and 896
+// 185 -> 168 in 224, 1100 250 -> 225 in 192, 1344 264 -> 245 in 224; 12288 x 4096 1700 163 -> 150; 4096 x 14336 3500 296 -> 286).
+// The sums are the same in every height, so it changes no bit.
+inline int ppp_height(int M, int N, int K) {
+  int best = 8;
+  double least = 0.985 * ppp_us_at(M, N, K, 8);
+  for (int mt = 7; mt >= 6; --mt) {
+    const double t = ppp_us_at(M, N, K, mt);
+    if (t < least) least = t, best = mt;
+  }
+  return best;
 }
 
 }  // namespace

@@ -41,14 +41,14 @@ constexpr int PG_GROUP_M = 8;
 
 // Epilogue of every kernel here: lane holds rows m = mw + 16 i + (lane & 15), columns
 // n = nw + 16 j + 4 (lane >> 4) + 0..3 of the wave's 128 x 16 NJ block.
-template <int EPI, int NJ>
-__device__ __forceinline__ void pg_epilogue(const f32x4_t (&acc)[8][NJ], const uint16_t* __restrict__ bias,
+template <int EPI, int NJ, int MT = 8>
+__device__ __forceinline__ void pg_epilogue(const f32x4_t (&acc)[MT][NJ], const uint16_t* __restrict__ bias,
                                             uint16_t* __restrict__ out, int M, int N, int ldo, int mw, int nw,
                                             const PgGlu& gp = PgGlu{}) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < MT; ++i) {
     const int m = mw + i * 16 + (lane & 15);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
@@ -658,14 +658,18 @@ __device__ __forceinline__ void ppp_st8(void* p, uint2 v) { *reinterpret_cast<ui
 
 __device__ __forceinline__ void ppp_st16(void* p, uint4 v) { *reinterpret_cast<uint4*>(p) = v; }
 
-template <int EPI, bool STG>
+// MT: 16-row MFMA tiles of a wave, BM = 32 MT rows of a workgroup (see pgemm_pph_kernel).
+template <int EPI, bool STG, int MT = 8>
 __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict__ X, const uint16_t* __restrict__ W,
                                           uint16_t* __restrict__ out, int M, int N, int K, int ldo, int tiles_m,
                                           int tiles_n, int wnw, int gm, const PgGlu& gp) {
   static_assert(EPI == PG_BF16 || EPI == PG_RELU2 || (EPI == PG_F32 && STG) || pg_gated(EPI), "bf16 / gated / staged fp32 epilogues");
   // epilogue store instructions per wave in the interior (counted in the next tile's first waits):
   // staged bf16 16 x 16 B (128 rows x 128 B), staged SwiGLU 8 x 16 B (128 rows x 64 B), else 32 (staged fp32 of 16 B)
-  constexpr int PPP_S = EPI == PG_F32 ? 32 : STG ? (pg_gated(EPI) ? 8 : 16) : 32;
+  constexpr int PPP_S = MT * (EPI == PG_F32 ? 4 : STG ? (pg_gated(EPI) ? 1 : 2) : 4);
+  // segment B: MB m-tiles a wave, an X1 image of 32 MB rows, P1 pieces of it a wave (beyond the last: that one again)
+  constexpr int BM = 32 * MT, MB = MT - 4, P1 = MB > 2 ? 2 : 1;
+  static_assert(MT >= 6 && MT <= 8 && (MT == 8 || STG), "");
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int grp = w >> 2, wc = w & 3;
@@ -678,7 +682,7 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
     const int first_m = (id / per_group) * gm;
     const int gsz = min(tiles_m - first_m, gm);
     const int in_group = id % per_group;
-    m0 = (first_m + in_group % gsz) * PG_BM;
+    m0 = (first_m + in_group % gsz) * BM;
     n0 = (in_group / gsz) * PG_BN;
   };
   // DMA source offsets of one tile (as pgemm_pp_kernel, packed W)
@@ -687,8 +691,8 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const int r = 8 * (w + 8 * i) + (lane >> 3);
-        const int trow = (r >> 6) * 128 + 64 * h + (r & 63);
+        const int r = 8 * (h == 1 && MT < 8 ? min(w + 8 * i, 4 * MB - 1) : w + 8 * i) + (lane >> 3);
+        const int trow = h == 0 || MT == 8 ? (r >> 6) * (16 * MT) + 64 * h + (r & 63) : r / (16 * MB) * (16 * MT) + 64 + r % (16 * MB);
         const int c = (lane & 7) ^ (r & 7);
         vx[h][i] = ((uint32_t)min(m0 + trow, M - 1) * (uint32_t)K + 8u * c) * 2u;
         const int f = w + 8 * i;
@@ -703,12 +707,13 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
   bool has_next = vb + G < nwg;
   if (has_next) coords(vb + G, m0n, n0n);   // its DMA offsets: computed where first needed (MODE 1)
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(pg_lds_t*)smem + w * 1024);
+  const uint32_t last1 = (uint32_t)(min(w + 8, 4 * MB - 1) - w) * 1024u;
   const size_t wstep = (size_t)2 * wnw * 512;
   auto issue_x = [&](int kt, int slot, const uint32_t (&o)[2][2], int h) {
     const uint16_t* src = X + (size_t)kt * PG_BK;
     const uint32_t la = lds0 + slot * PP_BUF + h * PP_HALF;
     pg_glds16(o[h][0], src, la);
-    pg_glds16(o[h][1], src, la + 8192);
+    if (h == 0 || P1 == 2) pg_glds16(o[h][1], src, la + (h == 1 && MT < 8 ? last1 : 8192u));
   };
   auto issue_w = [&](int kt, int slot, const uint32_t (&o)[2][2], int h) {
     const uint16_t* src = W + (size_t)kt * wstep;
@@ -716,10 +721,10 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
     pg_glds16(o[h][0], src, la);
     pg_glds16(o[h][1], src, la + 8192);
   };
-  const int xrd = (64 * grp + (lane & 15)) * 128;
+  const int xrd = (64 * grp + (lane & 15)) * 128, xrd1 = (16 * MB * grp + (lane & 15)) * 128;
   const int sw = lane & 7;
   auto rd_x = [&](int buf, int h, int i, int kk) {
-    return *reinterpret_cast<const bf16x8_t*>(smem + buf + h * PP_HALF + xrd + i * 16 * 128 +
+    return *reinterpret_cast<const bf16x8_t*>(smem + buf + h * PP_HALF + (h ? xrd1 : xrd) + i * 16 * 128 +
                                               (((4 * kk + (lane >> 4)) ^ sw) << 4));
   };
   auto rd_w = [&](int buf, int j, int kk) {
@@ -736,16 +741,16 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
   issue_x(1, 1, vx, 0);
   issue_w(1, 1, vw, 0);
   issue_w(1, 1, vw, 1);
-  pp_wait_barrier<8>();
+  pp_wait_barrier<6 + P1>();
   if (grp == 1) pp_barrier();   // the stagger: group 1 runs one barrier behind group 0
 
-  f32x4_t acc[8][4];
+  f32x4_t acc[MT][4];
   bf16x8_t wf[4][2], xf[4][2];
   int par = 0;          // LDS slot of K-tile 0 of the current tile (stream position parity)
   bool st = false;      // S epilogue stores of the previous tile still counted in vmcnt
   for (;;) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     // K-tile kt of this tile.  TAIL false: kt + 2 < nk (this tile's DMA only, no branches); TAIL
@@ -770,8 +775,8 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) xf[i][kk] = rd_x(buf, 0, i, kk);
-      if (held) pp_wait_barrier<8 + PPP_S>();   // (held: kt = 0, so kt + 1 exists)
-      else if (e1) pp_wait_barrier<8>();
+      if (held) pp_wait_barrier<6 + P1 + PPP_S>();   // (held: kt = 0, so kt + 1 exists)
+      else if (e1) pp_wait_barrier<6 + P1>();
       else pp_wait_barrier<0>();
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -796,17 +801,17 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
         issue_w(kt + 2 - nk, s0, nwv, 1);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) xf[i][kk] = rd_x(buf, 1, i, kk);
       const bool e2 = !TAIL || has_next;   // position kt + 2 exists
       if (held) {
-        if (e2) pp_wait_barrier<8 + PPP_S>();
-        else pp_wait_barrier<2 + PPP_S>();
+        if (e2) pp_wait_barrier<6 + P1 + PPP_S>();
+        else pp_wait_barrier<P1 + PPP_S>();
       } else if (e2) {
-        pp_wait_barrier<8>();
+        pp_wait_barrier<6 + P1>();
       } else if (e1) {
-        pp_wait_barrier<2>();
+        pp_wait_barrier<P1>();
       } else {
         pp_wait_barrier<0>();
       }
@@ -814,7 +819,7 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MB; ++i)
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             acc[4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][kk], xf[i][kk], acc[4 + i][j], 0, 0, 0);
@@ -825,11 +830,11 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
     for (; kt < nk - 2; ++kt) step(kt, std::false_type{}, st && kt == 0);
     for (; kt < nk; ++kt) step(kt, std::true_type{}, st && kt == 0);
     // ---- epilogue of this tile (no LDS: the next tile's DMA is already landing there)
-    const int mw = m0 + grp * 128, nw0 = n0 + wc * 64;
-    if (mw + 128 <= M && nw0 + 64 <= N) {
+    const int mw = m0 + grp * (16 * MT), nw0 = n0 + wc * 64;
+    if (mw + 16 * MT <= M && nw0 + 64 <= N) {
       const int g = lane >> 4;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < MT; ++i) {
         const int m = mw + i * 16 + (lane & 15);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -848,7 +853,7 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
         char* region = smem + 2 * PP_BUF + w * PPP_REGION;
         const int rl = lane & 15;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < MT; ++q) {
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             *reinterpret_cast<f32x4_t*>(region + rl * 256 + (((4 * j + g) ^ rl) << 4)) = acc[q][j];
@@ -875,7 +880,7 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
 #pragma unroll
-          for (int ii = 0; ii < 4; ++ii) {
+          for (int ii = 0; ii < (q ? MB : 4); ++ii) {
             const int r = 16 * ii + rl;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -889,7 +894,7 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-          for (int s4 = 0; s4 < 4; ++s4) {
+          for (int s4 = 0; s4 < (q ? MB : 4); ++s4) {
             const int r = 16 * s4 + (lane >> 2), unit = lane & 3;
             const uint4 val = *reinterpret_cast<const uint4*>(region + r * 64 + ((unit ^ (r & 3)) << 4));
             ppp_st16(out + (size_t)(mw + 64 * q + r) * ldo + nw0 / 2 + unit * 8, val);
@@ -904,9 +909,9 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
         char* region = smem + 2 * PP_BUF + w * PPP_REGION;
         const int rl = lane & 15;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < (MT + 1) / 2; ++q) {
 #pragma unroll
-          for (int ii = 0; ii < 2; ++ii) {
+          for (int ii = 0; ii < min(2, MT - 2 * q); ++ii) {
             const int r = 16 * ii + rl;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -920,7 +925,7 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-          for (int s4 = 0; s4 < 4; ++s4) {
+          for (int s4 = 0; s4 < 2 * min(2, MT - 2 * q); ++s4) {
             const int r = 8 * s4 + (lane >> 3), unit = lane & 7;
             const uint4 val = *reinterpret_cast<const uint4*>(region + r * 128 + ((unit ^ (r & 7)) << 4));
             ppp_st16(out + (size_t)(mw + 32 * q + r) * ldo + nw0 + unit * 8, val);
@@ -974,6 +979,18 @@ __global__ void __launch_bounds__(512, 1)
   ppp_tiles<PG_F32, true>(smem, X, W, out, M, N, K, ldo, tiles_m, tiles_n, wnw, gm, PgGlu{});
 }
 
+
+// Tiles of 32 MT = 192 or 224 rows (ppp_height): where 256 leave rows of the last tile unused or the last round of
+// workgroups short.  Segment A keeps its 64 rows of either group, segment B has 32 or 48, and the stream's waits count one
+// or two pieces of X1.  Two segments of equal length, each a half of K, read less at once but wait for X three segments, not
+// four, after asking for it: 4 % faster in 192 rows, no faster in 224.
+template <int EPI, int MT>
+__global__ void __launch_bounds__(512, 1)
+    pgemm_pph_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, uint16_t* __restrict__ out,
+                     int M, int N, int K, int ldo, int tiles_m, int tiles_n, int wnw, int gm, PgGlu gp) {
+  __shared__ __attribute__((aligned(16))) char smem[2 * PP_BUF + 8 * PPP_REGION];
+  ppp_tiles<EPI, true, MT>(smem, X, W, out, M, N, K, ldo, tiles_m, tiles_n, wnw, gm, gp);
+}
 
 // ---- encoder sub-layer epilogue: Y = LayerNorm(X . W^T + bias + residual) --------------------------
 // The post-LN BERT projections whose output width is the hidden size (o-proj K = hidden, FFN down
@@ -1285,14 +1302,19 @@ constexpr bool PPP_STG = true;
 // on the one-tile kernel: r04_pgemm_pp_probes.jsonl)
 int ppp_group_m(int tiles_n, int K) { return (K >= 8192 && tiles_n <= 16) ? 4 : PG_GROUP_M; }
 
+// mt: 6 or 7, tiles of 192 or 224 rows; 8, 256
 template <int EPI>
 int ppp_launch(const uint16_t* xp, const uint16_t* wp, uint16_t* op, int M, int N, int K, int ldo, int wnw, int gm,
-               bool stg, hipStream_t stream, const PgGlu& gp = PgGlu{}) {
-  const int tm = (M + PG_BM - 1) / PG_BM, tn = (N + PG_BN - 1) / PG_BN;
-  if (stg)
-    pgemm_ppp_kernel<EPI, true><<<min(tm * tn, pg_cus()), 512, 0, stream>>>(xp, wp, op, M, N, K, ldo, tm, tn, wnw, gm, gp);
-  else
-    pgemm_ppp_kernel<EPI, false><<<min(tm * tn, pg_cus()), 512, 0, stream>>>(xp, wp, op, M, N, K, ldo, tm, tn, wnw, gm, gp);
+               bool stg, int mt, hipStream_t stream, const PgGlu& gp = PgGlu{}) {
+  const int tm = (M + 32 * mt - 1) / (32 * mt), tn = (N + PG_BN - 1) / PG_BN, grid = min(tm * tn, pg_cus());
+#define PPP_ARGS xp, wp, op, M, N, K, ldo, tm, tn, wnw, gm
+  if (mt == 7) pgemm_pph_kernel<EPI, 7><<<grid, 512, 0, stream>>>(PPP_ARGS, gp);
+  else if (mt == 6) pgemm_pph_kernel<EPI, 6><<<grid, 512, 0, stream>>>(PPP_ARGS, gp);
+  else if constexpr (EPI == PG_F32) pgemm_ppp32_kernel<<<grid, 512, 0, stream>>>(PPP_ARGS);
+  else if constexpr (EPI == PG_GLU) pgemm_ppp_kernel<EPI, true><<<grid, 512, 0, stream>>>(PPP_ARGS, gp);
+  else if (stg) pgemm_ppp_kernel<EPI, true><<<grid, 512, 0, stream>>>(PPP_ARGS, gp);
+  else pgemm_ppp_kernel<EPI, false><<<grid, 512, 0, stream>>>(PPP_ARGS, gp);
+#undef PPP_ARGS
   return (int)hipGetLastError();
 }
 
@@ -1309,7 +1331,8 @@ int pgemm_launch(const void* x, const void* w, const void* bias, void* out, int 
     else if (variant == 6) {   // persistent: one workgroup per CU walking the tiles
       // (bias epilogues and K < 128 take the non-persistent kernel)
       if constexpr (EPI == PG_BF16 || EPI == PG_SWIGLU) {
-        if (K >= 2 * PG_BK) return ppp_launch<EPI>(xp, wp, op, M, N, K, ldo, wnw, ppp_group_m(tn, K), PPP_STG, stream);
+        if (K >= 2 * PG_BK)
+          return ppp_launch<EPI>(xp, wp, op, M, N, K, ldo, wnw, ppp_group_m(tn, K), PPP_STG, ppp_height(M, N, K), stream);
       }
       pgemm_pp_kernel<EPI, true, PP_PF><<<tm * tn, 512, 0, stream>>>(xp, wp, bp, op, M, N, K, ldo, tm, tn, wnw);
     }
@@ -1336,7 +1359,7 @@ int pgemm_launch_f32(const void* x, const void* w, void* out, int M, int N, int 
   const uint16_t *xp = (const uint16_t*)x, *wp = (const uint16_t*)w;
   uint16_t* op = (uint16_t*)out;
   if (wnw > 0 && variant == 6 && K >= 2 * PG_BK)
-    pgemm_ppp32_kernel<<<min(tm * tn, pg_cus()), 512, 0, stream>>>(xp, wp, op, M, N, K, ldo, tm, tn, wnw, ppp_group_m(tn, K));
+    return ppp_launch<PG_F32>(xp, wp, op, M, N, K, ldo, wnw, ppp_group_m(tn, K), true, ppp_height(M, N, K), stream);
   else if (wnw > 0) pgemm_pp_kernel<PG_F32, true, PP_PF><<<tm * tn, 512, 0, stream>>>(xp, wp, nullptr, op, M, N, K, ldo, tm, tn, wnw);
   else pgemm_pp_kernel<PG_F32, false, PP_PF><<<tm * tn, 512, 0, stream>>>(xp, wp, nullptr, op, M, N, K, ldo, tm, tn, 1);
   return (int)hipGetLastError();
@@ -1366,10 +1389,13 @@ CFC_API int cfc_pgemm(const void* x, const void* w, const void* bias, void* out,
     case 6:        // packed W, the persistent kernel
       if (wnw < 1 || K < 2 * PG_BK || ldo % 8 || ((uintptr_t)out & 15)) return (int)hipErrorInvalidValue;
       return ppp_launch<PG_RELU2>((const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, M, N, K, ldo, wnw,
-                                  ppp_group_m((N + PG_BN - 1) / PG_BN, K), PPP_STG, stream);
+                                  ppp_group_m((N + PG_BN - 1) / PG_BN, K), PPP_STG, ppp_height(M, N, K), stream);
     default: return (int)hipErrorInvalidValue;
   }
 }
+
+// 16-row MFMA tiles of a wave that the persistent kernel takes M rows with: 6, 7 or 8, tiles of 192, 224 or 256 rows
+CFC_API int cfc_ppp_height(int M, int N, int K) { return M < 1 || N < 1 || K < 1 ? 0 : ppp_height(M, N, K); }
 
 // Clamped GLU epilogue over packed, 8-row interleaved gate / up weights on the persistent kernel:
 // out [M, N / 2] (row stride ldo) = min(g, limit) sigmoid(alpha g (1 + cubic g^2)) (clamp(u, +-limit) + beta).
@@ -1378,12 +1404,10 @@ CFC_API int cfc_pgemm_glu(const void* x, const void* w, void* out, int M, int N,
   if (M < 1 || N < 64 || K < 2 * PG_BK || K % 64 || N % 64 || ldo % 8 || ldo < N / 2 || ((uintptr_t)out & 15) || wnw < 1 ||
       N % (16 * wnw) || (uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)N * K * 2 >= (1ull << 32))
     return (int)hipErrorInvalidValue;
-  const int tm = (M + PG_BM - 1) / PG_BM, tn = (N + PG_BN - 1) / PG_BN;
   PgGlu gp;
   gp.limit = limit; gp.alpha = alpha; gp.beta = beta; gp.cubic = cubic;
-  pgemm_ppp_kernel<PG_GLU, true><<<min(tm * tn, pg_cus()), 512, 0, stream>>>(
-      (const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, M, N, K, ldo, tm, tn, wnw, ppp_group_m(tn, K), gp);
-  return (int)hipGetLastError();
+  return ppp_launch<PG_GLU>((const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, M, N, K, ldo, wnw,
+                            ppp_group_m((N + PG_BN - 1) / PG_BN, K), true, ppp_height(M, N, K), stream, gp);
 }
 
 // Products of rows sorted by expert with W[experts][N][K] (each packed for bn = 16 wnw): M sorted rows in tiles of
@@ -1439,18 +1463,19 @@ CFC_API int cfc_pgemm_probe(const void* x, const void* w, void* out, int M, int 
 
 // Timing probe only (scripts/probe_ppp_gm.py): the persistent kernel (packed W, bf16 or SwiGLU
 // epilogue: epi 0 / 3, +16 for register-direct instead of LDS-staged stores) with an explicit
-// tile-order group gm (M-tiles per N sweep).
+// tile-order group gm (M-tiles per N sweep); epi_s >> 5: 6 or 7 for tiles of 192 or 224 rows.
 CFC_API int cfc_pgemm_ppp_probe(const void* x, const void* w, void* out, int M, int N, int K, int epi_s, int ldo,
                                 int wnw, int gm, hipStream_t stream) {
   const int epi = epi_s & 15;
   const bool stg = (epi_s & 16) == 0;   // +16: register-direct epilogue stores
+  const int mt = epi_s >> 5 ? epi_s >> 5 : 8;
   if (M < 1 || K < 2 * PG_BK || K % 64 || N % 64 || wnw < 1 || N % (16 * wnw) || gm < 1 || (epi != 0 && epi != 3) ||
-      ldo < (epi == 3 ? N / 2 : N) || ldo % 4 || (uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)N * K * 2 >= (1ull << 32))
+      mt < 6 || mt > 8 || ldo < (epi == 3 ? N / 2 : N) || ldo % 4 || (uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)N * K * 2 >= (1ull << 32))
     return (int)hipErrorInvalidValue;
   const uint16_t *xp = (const uint16_t*)x, *wp = (const uint16_t*)w;
   uint16_t* op = (uint16_t*)out;
-  return epi == 0 ? ppp_launch<PG_BF16>(xp, wp, op, M, N, K, ldo, wnw, gm, stg, stream)
-                  : ppp_launch<PG_SWIGLU>(xp, wp, op, M, N, K, ldo, wnw, gm, stg, stream);
+  return epi == 0 ? ppp_launch<PG_BF16>(xp, wp, op, M, N, K, ldo, wnw, gm, stg, mt, stream)
+                  : ppp_launch<PG_SWIGLU>(xp, wp, op, M, N, K, ldo, wnw, gm, stg, mt, stream);
 }
 
 // Y[M, N] = LayerNorm(X[M, K] . W[N, K]^T + bias + residual) * gamma + beta, N = 384 (the encoder
