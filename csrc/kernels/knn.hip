@@ -62,6 +62,10 @@ struct KnnRows {
     f32x4_t v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < KC; ++c) v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[c]), qf[c], v, 0, 0, 0);
+    return finish(v, r0);
+  }
+  // scores of the products
+  __device__ __forceinline__ f32x4_t finish(f32x4_t v, int r0) const {
     const int rb = r0 + 4 * ((threadIdx.x & 63) >> 4);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -121,20 +125,139 @@ __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restric
         }
       }
     };
-    if constexpr (KC <= 16) {          // the next 16 rows in flight under these (144 -> 131 us); wider rows fill the registers alone
-      uint4 a[2][KC];
-      rows.load(a[0], lo);
-      for (int r0 = lo; r0 < hi; r0 += 32) {
-        if (r0 + 16 < hi) rows.load(a[1], r0 + 16);
-        take(a[0], r0);
-        if (r0 + 32 < hi) rows.load(a[0], r0 + 32);
-        if (r0 + 16 < hi) take(a[1], r0 + 16);
+    uint4 a[2][KC];                  // the next 16 rows in flight under these (144 -> 131 us)
+    rows.load(a[0], lo);
+    for (int r0 = lo; r0 < hi; r0 += 32) {
+      if (r0 + 16 < hi) rows.load(a[1], r0 + 16);
+      take(a[0], r0);
+      if (r0 + 32 < hi) rows.load(a[0], r0 + 32);
+      if (r0 + 16 < hi) take(a[1], r0 + 16);
+    }
+    if constexpr (MAXIMA) {
+      if (qv && lo + 16 * g < hi) out[col * ld + 4 * blk + g] = key2f(best);
+    } else if (bmax && g == 0 && qv) {
+      bmax[(size_t)col * nb + blk] = best;
+    }
+  }
+}
+
+// The same scan for rows that come from memory.  A fragment's sixteen rows give 64 bytes each to a load, and memory serves
+// that at 6.2 TB/s; whole runs, marked as read once, at 6.8 (768 MB of 16 x 768 bytes: 122 us, 129 marked; in runs 124, 112
+// marked).  So rows go to LDS first, by LDS-DMA in pieces of 1 KB, a ring of R units per wave: 16 rows of KU k-steps.  Chunk c
+// of row r lies at c ^ (r & 15) of its row's sixteen (through the pieces' source addresses), and sixteen rows' reads
+// touch all banks.  No barrier: each wave waits for its own pieces alone.  Workgroups of one round, whose waves' streams
+// run on from block to block.
+// us with the selection, fragments from memory -> this: 1M rows of 384 148 -> 132 (of 16 queries 181 -> 166), 3M 413 -> 374;
+// of 768 values, whose fragments fill the registers alone, 500 k 165 -> 131, 100 k 38 -> 33, 5000 16.9 -> 15.7, of 1024 141 k 64 -> 56.
+template <int KC>
+struct KnnUnit {
+  static constexpr int KU = KC <= 16 ? KC : KC % 12 == 0 ? 12 : KC % 16 == 0 ? 16 : KC % 8 == 0 ? 8 : 4;      // k-steps of a unit, and KB
+  static constexpr int R = KU > 12 ? 2 : KU > 8 ? 3 : 4, NU = KC / KU;
+  static_assert(KC % KU == 0 && KU % 4 == 0 && 4 * R * KU <= 160, "");
+};
+
+typedef __attribute__((address_space(3))) void kn_lds_t;
+
+// One 1-KB LDS-DMA piece of sbase + voff (per lane), read once (M0 kept).
+__device__ __forceinline__ void kn_piece(uint32_t voff, const void* sbase, uint32_t lds_addr) {
+  unsigned keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(voff), "s"(sbase), "s"(lds_addr)
+      : "memory");
+}
+
+template <int KC, bool MAXIMA>
+__global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
+                                                            int nq, const float* __restrict__ xnorm2,
+                                                            const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
+                                                            float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
+                                                            int B) {
+  constexpr int KU = KnnUnit<KC>::KU, R = KnnUnit<KC>::R, NU = KnnUnit<KC>::NU, UB = KU * 1024;
+  __shared__ __attribute__((aligned(16))) char kn_smem[4 * R * UB];
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), stride = gridDim.x * 4;
+  const bool qv = col < nq;
+  KnnRows<KC> rows{X, N, xnorm2, alive};
+  rows.queries(Q, qnorm2, nq);
+  const bool vec = (ld & 3) == 0 && ((uintptr_t)out & 15) == 0;
+  int blk = blockIdx.x * 4 + w;
+  if (blk >= nb) return;
+  const char* ring = kn_smem + w * (R * UB);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(kn_lds_t*)kn_smem) + w * (R * UB);
+  uint32_t voff[KU];
+#pragma unroll
+  for (int i = 0; i < KU; ++i) {
+    const int p = 64 * i + lane, r = p / (4 * KU), c = p % (4 * KU);
+    voff[i] = (uint32_t)(r * (KC * 64) + ((c & ~15) | ((c ^ r) & 15)) * 16);
+  }
+  // ---- what is asked for: unit iu of the 16 rows from ir0 of block iblk
+  int iblk = blk, ir0 = blk * B, iu = 0, fill = 0;
+  auto issue = [&]() {
+    if (iblk >= nb) return;
+    const char* src = reinterpret_cast<const char*>(X) + (size_t)ir0 * (KC * 64) + iu * (KU * 64);
+    if (ir0 + 16 <= N) {
+#pragma unroll
+      for (int i = 0; i < KU; ++i) kn_piece(voff[i], src, lds0 + fill * UB + i * 1024);
+    } else {                                          // past the last row: that one again
+#pragma unroll
+      for (int i = 0; i < KU; ++i) {
+        const int r = (64 * i + lane) / (4 * KU);
+        kn_piece(voff[i] - (uint32_t)(max(0, ir0 + r - (N - 1)) * (KC * 64)), src, lds0 + fill * UB + i * 1024);
       }
-    } else {
-      uint4 a[KC];
-      for (int r0 = lo; r0 < hi; r0 += 16) {
-        rows.load(a, r0);
-        take(a, r0);
+    }
+    fill = fill + 1 == R ? 0 : fill + 1;
+    if (++iu == NU) {
+      iu = 0;
+      ir0 += 16;
+      if (ir0 >= min(N, iblk * B + B)) {
+        iblk += stride;
+        ir0 = iblk * B;
+      }
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < R - 1; ++i) issue();
+  int slot = 0;
+  for (; blk < nb; blk += stride) {
+    const int lo = blk * B, hi = min(N, lo + B);
+    uint32_t best = 0u;
+    for (int r0 = lo; r0 < hi; r0 += 16) {
+      f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        // this unit's pieces (scores stored since count too: it waits for no less), and the reads of the one before, whose
+        // place the next one takes
+        if (iblk < nb) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(KU * (R - 2)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        issue();
+        const char* img = ring + slot * UB + col * (KU * 64);
+#pragma unroll
+        for (int c = 0; c < KU; ++c) {
+          const int ch = 4 * c + g;
+          const uint4 a = *reinterpret_cast<const uint4*>(img + ((ch & ~15) | ((ch ^ col) & 15)) * 16);
+          v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), rows.qf[u * KU + c], v, 0, 0, 0);
+        }
+        slot = slot + 1 == R ? 0 : slot + 1;
+      }
+      v = rows.finish(v, r0);
+      const uint32_t m = rows.best(v, r0);
+      if constexpr (MAXIMA) {
+        if (r0 - lo == 16 * g) best = m;            // group g's
+      } else {
+        best = max(best, m);
+        const int rb = r0 + 4 * g;
+        if (qv) {
+          float* o = out + col * ld + rb;
+          if (rb + 3 < N && vec) {
+            *reinterpret_cast<f32x4_t*>(o) = v;
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (rb + i < N) o[i] = v[i];
+          }
+        }
       }
     }
     if constexpr (MAXIMA) {
@@ -759,6 +882,13 @@ CFC_API int cfc_topk_segment(int n) {
 // -> 24.7; 300 k 36.2 -> 38.2 (from memory a workgroup per four blocks reads faster), 100 k of 768 28.2 -> 28.5.
 constexpr long KNN_ROUND_BYTES = 160l << 20;
 constexpr int KNN_ROUND = 512;
+// More than the cache holds goes by knn_stream_kernel, which marks rows as read once (MB of 384 values, us: 230 46 -> 48, 260
+// 50 -> 52, 290 58.5 -> 56.5, 330 69 -> 63; of 256 270 56.5 -> 55, 300 58 -> 58.6, 400 84 -> 74), and all rows of more than 512
+// values; rows of 128, a quarter of a unit each, do not (200 MB 44 -> 65, 400 97 -> 127).
+constexpr long KNN_STREAM_BYTES = 288l << 20;
+constexpr int KNN_CUS = 256;
+
+#define KNN_ARGS(OUT, B) (const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, qnorm2, alive, OUT, (size_t)ld, B
 
 // Scores of rows [0, N) of X for nq queries into out [nq][ld], and the largest key of every cfc_topk_block(N) rows into
 // bmax [nq][blocks] (null: not wanted), which has room for `room` of them.
@@ -767,9 +897,17 @@ CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, c
   if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || ld < N) return -1;
   const int B = cfc_topk_block(N), nb = (N - 1) / B + 1;
   if (bmax && (long)nq * nb > room) return -1;
-  const int all = (nb + 3) / 4, grid = dim <= 512 && (long)N * dim * 2 <= KNN_ROUND_BYTES ? min(all, KNN_ROUND) : all;
-#define KS(KC) knn_scan_kernel<KC, false><<<grid, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, \
-      qnorm2, alive, out, (size_t)ld, bmax, nb, B); break
+  const int all = (nb + 3) / 4;
+  const long bytes = (long)N * dim * 2;
+#define KS(KC)                                                                                                             \
+  if constexpr (KC > 4)                                                                                                    \
+    if (KC > 16 || bytes > KNN_STREAM_BYTES) {                                                                             \
+      knn_stream_kernel<KC, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B);                     \
+      break;                                                                                                               \
+    }                                                                                                                      \
+  if constexpr (KC <= 16)                                                                                                  \
+    knn_scan_kernel<KC, false><<<bytes <= KNN_ROUND_BYTES ? min(all, KNN_ROUND) : all, 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B); \
+  break
   KNN_DIMS(KS)
 #undef KS
   return CFC_CHECK_LAUNCH();
@@ -779,11 +917,14 @@ CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, c
 CFC_API int cfc_knn_maxima(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
                            const uint8_t* alive, float* out, long ld, hipStream_t stream) {
   if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || ld < (N - 1) / 16 + 1) return -1;
-  const int nb = (N - 1) / 64 + 1;
-#define KS(KC) knn_scan_kernel<KC, true><<<(nb + 3) / 4, 256, 0, stream>>>((const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, \
-      qnorm2, alive, out, (size_t)ld, nullptr, nb, 64); break
+  const int nb = (N - 1) / 64 + 1, all = (nb + 3) / 4;
+#define KS(KC)                                                                                                  \
+  if constexpr (KC > 4) knn_stream_kernel<KC, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64); \
+  else knn_scan_kernel<KC, true><<<all, 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);                       \
+  break
   KNN_DIMS(KS)
 #undef KS
+#undef KNN_ARGS
   return CFC_CHECK_LAUNCH();
 }
 

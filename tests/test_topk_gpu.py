@@ -235,3 +235,34 @@ def test_float_queries_in_one_launch(metric, dim, nq):
             torch.testing.assert_close(v, ov, rtol=(dim + 4) * 2.0 ** -24, atol=0.0)
         else:
             assert torch.equal(v, ov) and torch.equal(i, oi)
+
+
+@pytest.mark.parametrize("metric", ["dot", "l2"])
+@pytest.mark.parametrize("dim,nq,N", [(768, 1, 1), (768, 3, 15), (1024, 16, 17), (768, 2, 63), (1024, 1, 65), (768, 5, 16 * 4 * 256 + 1), (1024, 2, 40_003),
+                                      (384, 2, 393_300), (512, 1, 295_001), (256, 3, 600_007)])
+def test_knn_scores_by_the_stream(dim, nq, N, metric):
+    """Rows that come through LDS: fewer than a unit's sixteen, one more than whole blocks, rows of one and two units, more
+    rows than the chip caches; infinite and masked rows spoil no other, and nothing is written past the last row."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(N + dim)
+    X, Q = (torch.randn(n, dim, device=DEV, generator=g).bfloat16() for n in (N, nq))
+    bad = torch.arange(0, N, 1001, device=DEV)[1:]
+    X[bad] = float("inf")
+    alive = torch.rand(N, device=DEV, generator=g) > 0.1
+    xn, qn = (t.float().pow(2).sum(1) if metric == "l2" else None for t in (X, Q))
+    out = torch.full((nq, N + 3), 7.0, device=DEV)
+    got = K.knn_scores(X, Q, xn, qn, out=out[:, :N])
+    assert bool((out[:, N:] == 7.0).all())
+    fine = torch.ones(N, dtype=torch.bool, device=DEV).index_fill_(0, bad, False)
+    for at in range(0, N, 100_000):
+        x = X[at:at + 100_000].double()
+        want = Q.double() @ x.T
+        if metric == "l2":
+            want = 2 * want - qn.double()[:, None] - xn.double()[None, at:at + 100_000]
+        ok = fine[at:at + 100_000]
+        # fp32 sums of `dim` products (and three terms) of about 1 each, the largest sum some dim
+        assert float((got[:, at:at + 100_000].double() - want)[:, ok].abs().max()) < 2.0 ** -22 * dim * 4
+    assert not bool(got[:, bad].isfinite().any())
+    v, i = K.knn_topk(X, Q, min(50, N), xn, qn, alive=alive & fine)
+    rv, ri = got.masked_fill(~(alive & fine)[None], float("-inf")).sort(dim=1, descending=True, stable=True)
+    assert torch.equal(v, rv[:, :min(50, N)]) and torch.equal(i, ri[:, :min(50, N)])
