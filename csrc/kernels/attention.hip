@@ -32,7 +32,7 @@ namespace {
 
 constexpr int KV_BS = 32;          // tokens per KV-cache block
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr int DEC_ORDER_ROWS = 128;   // sequences that longest_first orders at most: two threads of 256 each
+constexpr int DEC_ORDER_ROWS = 128;   // sequences that longest_first orders at most
 constexpr int DEC_ORDER_FROM = 1024;  // the longest context from which it does
 
 __device__ __forceinline__ bf16x8_t as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8_t, v); }
@@ -119,10 +119,13 @@ __device__ __forceinline__ uint4 set_bf16(uint4 v, int e, uint32_t h) {
 // first): more workgroups than the chip holds at once start as others end, and a long one that starts last is waited for
 // alone.  In the order that they have where the contexts are short or differ by no more than `least` sixteenths of the
 // longest: the ranking, 0.5 us a workgroup, would be more than it saves.
+template <int THREADS>
 __device__ __forceinline__ int2 longest_first(const int32_t* __restrict__ ctx_lens, int B, int rank, int least) {
+  constexpr int SHARES = THREADS / DEC_ORDER_ROWS;    // threads of a sequence, each with a share of the others
+  static_assert(SHARES == 1 || SHARES == 2, "");
   __shared__ __attribute__((aligned(16))) int key[DEC_ORDER_ROWS], before[DEC_ORDER_ROWS], ends[4];
   __shared__ int found;
-  const int t = threadIdx.x, s = t & (DEC_ORDER_ROWS - 1), n = ctx_lens[min(s, B - 1)];     // two threads a sequence
+  const int t = threadIdx.x, s = t & (DEC_ORDER_ROWS - 1), n = ctx_lens[min(s, B - 1)];
   const int lo = wave_min_int(n), hi = -wave_min_int(-n);
   if (t < DEC_ORDER_ROWS) {
     key[t] = t < B ? (n << 8) + (255 - t) : -1;
@@ -137,11 +140,12 @@ __device__ __forceinline__ int2 longest_first(const int32_t* __restrict__ ctx_le
     const int own = key[s];
     int c = 0;
 #pragma unroll 8
-    for (int j = 0; j < DEC_ORDER_ROWS / 2; j += 4) {              // each with half of the others
+    for (int j = 0; j < DEC_ORDER_ROWS / SHARES; j += 4) {
       const int4 k = *reinterpret_cast<const int4*>(key + (t & DEC_ORDER_ROWS) / 2 + j);
       c += (k.x > own) + (k.y > own) + (k.z > own) + (k.w > own);
     }
-    atomicAdd(before + s, c);
+    if constexpr (SHARES == 1) before[s] = c;
+    else atomicAdd(before + s, c);
     __syncthreads();
     if (t < B && before[t] == rank) found = t;
     __syncthreads();
@@ -209,7 +213,7 @@ __global__ void __launch_bounds__(256, F8 ? 2 : 1) paged_decode_kernel(
   const int p = blockIdx.x, h = blockIdx.y;
   int b = blockIdx.z, ctx;
   if (ordered) {
-    const int2 s = longest_first(ctx_lens, gridDim.z, blockIdx.z, ordered);
+    const int2 s = longest_first<256>(ctx_lens, gridDim.z, blockIdx.z, ordered);
     b = s.x;
     ctx = s.y;
   } else {
@@ -451,6 +455,234 @@ __global__ void __launch_bounds__(256, F8 ? 2 : 1) paged_decode_kernel(
       const size_t pi = ((size_t)b * Hq + head) * P + p;
       part_o[pi * D + d] = O;
       if (d == 0) { part_ml[pi * 2] = M; part_ml[pi * 2 + 1] = L; }
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// The same attention where keys and values come from memory at its full rate: fragments of K take 64 bytes of a row each,
+// which memory serves at 5.8 to 6.3 TB/s, whole runs that are marked as read once at 6.8.  So a wave brings each (block, kv
+// head) tile of K and of V, 8 KB each, to LDS by LDS-DMA in pieces of 1 KB, through a ring of T tiles of its own (no barrier:
+// it waits for its own pieces).  A tile is read to registers as soon as it is there, and the one T tiles on takes its place.
+// Chunk c of K's row r lies at c ^ (r & 15) (through the pieces' source addresses), so that sixteen rows' reads touch all
+// banks; V's slot groups lie as in the cache.
+// A workgroup of NWV waves has one (partition of a) sequence and kv head, wave w its blocks w, w + NWV, ...
+// bf16 cache, queries roped.
+// ------------------------------------------------------------------------------------------
+typedef __attribute__((address_space(3))) void pd_lds_t;
+
+template <bool NT>
+__device__ __forceinline__ void pd_piece(uint32_t voff, const void* sbase, uint32_t lds_addr) {
+  unsigned keep;
+  if constexpr (NT)
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
+        : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+        : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+}
+
+template <int N>
+__device__ __forceinline__ void pd_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(N) : "memory");
+}
+
+// behind tile j of `tiles`: those that are asked for
+template <int T>
+__device__ __forceinline__ void pd_landed(int j, int tiles) {
+  const int left = tiles - 1 - j;
+  if (left >= T - 1) pd_wait<8 * (T - 1)>();
+  else if (T > 3 && left == 2) pd_wait<16>();
+  else if (T > 2 && left == 1) pd_wait<8>();
+  else pd_wait<0>();
+}
+
+template <int G, int NWV, int T>
+__global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+    const int32_t* __restrict__ block_tables, const int32_t* __restrict__ ctx_lens, float scale_log2, int Hkv, int max_blocks,
+    int P, int window, float v_scale, float* __restrict__ part_o, float* __restrict__ part_ml, uint16_t* __restrict__ out,
+    const int32_t* __restrict__ shared_blocks, int ordered) {
+  constexpr int D = 128, TILE = KV_BS * D * 2, QB = (G + 3) / 4 * 1024, RING = T * TILE;
+  __shared__ __attribute__((aligned(16))) char smem[NWV * (RING + QB)];
+  const int p = blockIdx.x, h = blockIdx.y;
+  int b = blockIdx.z, ctx;
+  if (T == 2 && ordered) {
+    const int2 s = longest_first<64 * (T == 2 ? NWV : 4)>(ctx_lens, gridDim.z, blockIdx.z, ordered);
+    b = s.x;
+    ctx = s.y;
+  } else {
+    ctx = ctx_lens[b];
+  }
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int Hq = Hkv * G;
+  const int nblk = (ctx + KV_BS - 1) / KV_BS;
+  const int key_lo = window > 0 ? max(0, ctx - window) : 0, blk_lo = key_lo / KV_BS;
+  const int blk0 = blk_lo + share_of(nblk - blk_lo, p, P), blk1 = blk_lo + share_of(nblk - blk_lo, p + 1, P);
+  const int32_t* bt = block_tables + (size_t)b * max_blocks;
+  const int first = blk0 + w, n = first < blk1 ? (blk1 - 1 - first) / NWV + 1 : 0;        // this wave's blocks
+  const int temporal = shared_blocks != nullptr ? shared_blocks[0] : 0;                   // blocks read through the caches
+  char* mine = smem + w * (RING + QB);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(pd_lds_t*)mine);
+  const uint32_t kvoff = (lane >> 4) * 256u, vvoff = lane * 16u;     // K: a piece has four rows, chunk (lane & 15) ^ row of each
+  auto id = [&](int i) { return i < n ? bt[first + i * NWV] : 0; };
+  // tile 2 i + v: keys (v 0) or values of this wave's block i
+  auto issue = [&](int j, int block) {
+    const bool key = (j & 1) == 0;
+    const char* src = reinterpret_cast<const char*>(key ? kc : vc) + ((size_t)block * Hkv + h) * TILE;
+    const uint32_t at = lds0 + (j & (T - 1)) * TILE;
+    const bool nt = first + (j >> 1) * NWV >= temporal;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t vo = key ? kvoff + (((lane & 15) ^ ((4 * e + (lane >> 4)) & 15)) << 4) : vvoff;
+      if (nt) pd_piece<true>(vo, src + e * 1024, at + e * 1024);
+      else pd_piece<false>(vo, src + e * 1024, at + e * 1024);
+    }
+  };
+  f32x4_t o[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  bf16x8_t qf[4];
+  if (n > 0) {
+    // the queries' rows first: they are there when the first keys are (past the G heads: the last one's, not used)
+    const char* qs = reinterpret_cast<const char*>(q + ((size_t)b * Hq + h * G) * D);
+#pragma unroll
+    for (int e = 0; e < QB / 1024; ++e)
+      pd_piece<false>((uint32_t)min(4 * e + (lane >> 4), G - 1) * 256u + (lane & 15) * 16u, qs, lds0 + RING + e * 1024);
+#pragma unroll
+    for (int j = 0; j < T; j += 2)
+      if (j < 2 * n) {
+        const int block = id(j / 2);
+        issue(j, block);
+        issue(j + 1, block);
+      }
+    int ahead = id(T / 2);                         // the block of the tiles T on
+    for (int i = 0; i < n; ++i) {
+      const int bi = first + i * NWV, next = id(i + 1 + T / 2);
+      pd_landed<T>(2 * i, 2 * n);
+      if (i == 0) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          qf[c] = col < G ? as_bf16x8(*reinterpret_cast<const uint4*>(mine + RING + min(col, G - 1) * 256 + c * 64 + g * 16))
+                          : as_bf16x8(make_uint4(0, 0, 0, 0));
+      }
+      uint4 kf[2][4];
+      const char* ki = mine + (2 * i & (T - 1)) * TILE;
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) kf[st][c] = *reinterpret_cast<const uint4*>(ki + (16 * st + col) * 256 + (((4 * c + g) ^ col) << 4));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // read: the place is free
+      if (i + T / 2 < n) issue(2 * i + T, ahead);
+      f32x4_t s[2];
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        s[st] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[st] = mfma16(as_bf16x8(kf[st][c]), qf[c], s[st]);
+      }
+      const int key0 = bi * KV_BS;
+      float tmax = -INFINITY;
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = key0 + 16 * st + 4 * g + e;
+          float v = s[st][e] * scale_log2;
+          v = key < ctx && key >= key_lo ? v : -INFINITY;
+          s[st][e] = v;
+          tmax = fmaxf(tmax, v);
+        }
+      tmax = xor16_max(tmax);
+      tmax = xor32_max(tmax);
+      const float mn = fmaxf(m, tmax);
+      const float alpha = exp2f(m - mn);
+      float rs = 0.f;
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = exp2f(s[st][e] - mn);
+          s[st][e] = x;
+          rs += x;
+        }
+      rs = xor16_sum(rs);
+      rs = xor32_sum(rs);
+      l = l * alpha + rs;
+      m = mn;
+      const bf16x8_t pf = pack_p(s[0], s[1]);
+      pd_landed<T>(2 * i + 1, 2 * n);
+      uint4 vf[8];
+      const char* vi = mine + ((2 * i + 1) & (T - 1)) * TILE + g * 2048 + col * 16;
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) vf[dt] = *reinterpret_cast<const uint4*>(vi + dt * 256);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (i + T / 2 < n) issue(2 * i + 1 + T, ahead);
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) {
+        o[dt] *= alpha;
+        o[dt] = mfma16(as_bf16x8(vf[dt]), pf, o[dt]);
+      }
+      ahead = next;
+    }
+  }
+
+  // lane (col, g) holds O^T[d = 16 dt + 4 g + i][col]
+  if constexpr (NWV == 1) {
+    if (col >= G) return;
+    const size_t row = (size_t)b * Hq + h * G + col;
+    const float inv = P == 1 ? (l > 0.f ? v_scale / l : 0.f) : v_scale;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) {
+      const int d = 16 * dt + 4 * g;
+      if (P == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[row * D + d + i] = f2bf(o[dt][i] * inv);         // out is aligned to its elements only
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part_o[(row * P + p) * D + d + i] = o[dt][i] * inv;
+      }
+    }
+    if (P > 1 && g == 0) {
+      part_ml[(row * P + p) * 2] = m;
+      part_ml[(row * P + p) * 2 + 1] = l;
+    }
+    return;
+  }
+  __syncthreads();                                 // every wave's tiles are used up
+  float(*sm_o)[D][17] = reinterpret_cast<float(*)[D][17]>(smem);
+  float(*sm_ml)[16][2] = reinterpret_cast<float(*)[16][2]>(smem + NWV * D * 17 * 4);
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sm_o[w][16 * dt + 4 * g + i][col] = o[dt][i];
+  if (g == 0) sm_ml[w][col][0] = m, sm_ml[w][col][1] = l;
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < G * D; idx += 64 * NWV) {
+    const int qh = idx / D, d = idx % D;
+    float M = -INFINITY;
+#pragma unroll
+    for (int ww = 0; ww < NWV; ++ww) M = fmaxf(M, sm_ml[ww][qh][0]);
+    float L = 0.f, O = 0.f;
+    if (M != -INFINITY) {
+#pragma unroll
+      for (int ww = 0; ww < NWV; ++ww) {
+        const float f = exp2f(sm_ml[ww][qh][0] - M);
+        L += sm_ml[ww][qh][1] * f;
+        O += sm_o[ww][d][qh] * f;
+      }
+    }
+    const size_t row = (size_t)b * Hq + h * G + qh;
+    O *= v_scale;
+    if (P == 1) {
+      out[row * D + d] = f2bf(L > 0.f ? O / L : 0.f);
+    } else {
+      part_o[(row * P + p) * D + d] = O;
+      if (d == 0) { part_ml[(row * P + p) * 2] = M; part_ml[(row * P + p) * 2 + 1] = L; }
     }
   }
 }
@@ -1522,6 +1754,37 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
   // plain loads win), profiles/decode_attn_partitions_r01.log; CFC_DECODE_NT=0/1 forces either
   static const int nt_env = [] { const char* e = getenv("CFC_DECODE_NT"); return e ? atoi(e) : -1; }();
   const bool nt = nt_env >= 0 ? nt_env != 0 : B >= 32;
+  // Through LDS in whole runs, unless the table holds 256 keys at most and the workgroups are few, or more sequences than are
+  // ordered wait: those have 2 GB of cache and more to read from, and what waits in registers is deeper.
+  // us of 8 key heads, one partition, fragments from memory -> this: 8 of 2617 keys 50.3 -> 35.7, 24 59.9 -> 44.3, 32 66.2 -> 58, 48 97 ->
+  // 88, 64 111 -> 108, 72 158 -> 131, 90 170 -> 157, 128 219 -> 212, from 0.8 of it 198 -> 191; 24 of 700 19.1 -> 16.3, 8 of 300 9.1 -> 8.5; 12 of
+  // 64 4.5 -> 5.1, 192 of 2617 315 -> 330.
+  if constexpr (!F8) {
+    if (!rope && part_blocks <= 0 && (wgs > 256 || max_blocks > 8) && B <= DEC_ORDER_ROWS) {
+#define PDS_GO(NWV, T)                                                                                                      \
+  paged_stream_kernel<GG, NWV, T><<<grid, 64 * NWV, 0, stream>>>((const uint16_t*)q, (const uint16_t*)k_cache,               \
+      (const uint16_t*)v_cache, block_tables, ctx_lens, sl2, Hkv, max_blocks, P, window, v_scale, part_o, part_ml,           \
+      (uint16_t*)out, shared_blocks, ordered)
+      // 96 to 128 KB under way in a CU: four waves of one workgroup, of two, or eight waves of two that the next ones follow
+      // one by one; few keys in one wave each, which have nothing to merge (128 of 60 11.7 -> 9.5 us, 11.5 in four)
+#define PDS_CASE(G_)                        \
+  case G_: {                                \
+    constexpr int GG = G_;                  \
+    if (wgs <= 256) PDS_GO(4, 4);           \
+    else if (wgs <= 512) PDS_GO(2, 4);      \
+    else if (max_blocks <= 8) PDS_GO(1, 4); \
+    else PDS_GO(4, 2);                      \
+  } break;
+      switch (G) {
+        PDS_CASE(1) PDS_CASE(2) PDS_CASE(4) PDS_CASE(8) PDS_CASE(16)
+        default: return -3;
+      }
+#undef PDS_CASE
+#undef PDS_GO
+      if (P > 1) decode_combine_kernel<<<(Hq * B + 3) / 4, 256, 0, stream>>>(part_o, part_ml, P, Hq * B, (uint16_t*)out);
+      return CFC_CHECK_LAUNCH();
+    }
+  }
 #define DEC_CASE(GG) \
   case GG: \
     if (rope) { \

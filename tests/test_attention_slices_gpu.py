@@ -99,22 +99,62 @@ def test_merge_of_an_infinite_sum(P):
     assert torch.equal(many[one.isinf()], one[one.isinf()]) and torch.equal(many.isinf(), one.isinf())
 
 
-@pytest.mark.parametrize("B,kv,P", [(65, 8, 1), (120, 8, 1), (66, 8, 2), (128, 6, 1), (129, 6, 1), (1, 9, 57)])
-def test_longest_first(B, kv, P):
-    """More workgroups than are held at once start with the longest sequences: every sequence's result is what it is in a
-    batch of its own, whatever the order, with equal lengths among them."""
+@pytest.mark.parametrize("B,kv,P,longest", [(65, 8, 1, 1030), (120, 8, 1, 1030), (66, 8, 2, 1030), (128, 6, 1, 2000), (129, 6, 1, 1030), (1, 9, 57, 2000),
+                                            (128, 8, 1, 900)])
+def test_longest_first(B, kv, P, longest):
+    """More workgroups than are held at once start with the longest sequences: every sequence's result is what it is when the
+    batch comes the other way round, whatever the order, with equal lengths among them."""
     from copilot_for_consensus_amd.ops import kernels as K
     heads, D = kv, 128
     g = torch.Generator(device=DEV).manual_seed(B)
     ctx = torch.randint(1, 8, (B,), generator=g, device=DEV) * 37 + torch.arange(B, device=DEV) % 2
-    ctx[B // 2:B // 2 + 2] = 1024
-    ctx[-1:] = 1030
+    ctx[B // 2:B // 2 + 2] = longest - 6
+    ctx[-1:] = longest
     lens = ctx.to(torch.int32)
-    bt, blocks = _tables(B, 1056, g)
+    bt, blocks = _tables(B, longest + 20, g)
     kc = torch.randn(blocks, kv, 32, D, device=DEV, generator=g).bfloat16()
     vc = torch.randn(blocks, kv, D, 32, device=DEV, generator=g).bfloat16()
     q = torch.randn(B, heads, D, device=DEV, generator=g).bfloat16()
-    run = lambda s: K.paged_decode_attention(q[s].contiguous(), kc, vc, bt[s].contiguous(), lens[s].contiguous(), D ** -0.5, part_blocks=-P)  # noqa: E731
-    step = max(1, 512 // (kv * P))
-    want = torch.cat([run(slice(i, i + step)) for i in range(0, B, step)])
-    assert torch.equal(run(slice(0, B)), want)
+    run = lambda t, *a: K.paged_decode_attention(t, kc, vc, *a, D ** -0.5, part_blocks=-P)  # noqa: E731
+    got = run(q, bt, lens)
+    assert torch.equal(got.flip(0), run(q.flip(0).contiguous(), bt.flip(0).contiguous(), lens.flip(0).contiguous()))
+    part = slice(0, B, max(1, B // 4))                  # another number of sequences, another share of waves
+    some = run(q[part].contiguous(), bt[part].contiguous(), lens[part].contiguous())
+    # weights rounded to bf16 from another maximum (2^-9 each, of values up to 4.5), results once more
+    assert bool(((got[part].double() - some.double()).abs() <= 2.0 ** -8 * some.double().abs() + 2.0 ** -8).all())
+
+
+def _keys_values(kc, vc, table, n):
+    """Keys and values [kv, n, D] in float64 of a sequence, from the cache's layouts."""
+    kv, D = kc.shape[1], kc.shape[3]
+    slot = torch.tensor([4 * s + j if j < 4 else 16 + 4 * s + j - 4 for s in range(4) for j in range(8)], device=DEV)
+    k = kc[table.long()].transpose(0, 1).reshape(kv, -1, D)[:, :n].double()
+    t = vc[table.long()].view(-1, kv, 4, D, 8).permute(0, 1, 2, 4, 3).reshape(-1, kv, 32, D)
+    v = torch.empty_like(t).index_copy_(2, slot, t).transpose(0, 1).reshape(kv, -1, D)[:, :n].double()
+    return k, v
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("B,kv,P", [(24, 8, 1), (40, 8, 1), (40, 8, 3), (70, 8, 1), (9, 1, 5)])
+@pytest.mark.parametrize("width", [300, 1100])
+def test_keys_and_values_by_the_stream(G, B, kv, P, width):
+    """Workgroups of four, two and one wave; waves of no, one, two and three blocks, last blocks of one key; slices and whole
+    sequences; a window; shared leading blocks.  Against float64."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    D, heads = 128, kv * G
+    edge = [1, 31, 32, 33, 64, 65, 96, 127, 129, 160, 193, 257, 288, 300]
+    ctx = [edge[i % len(edge)] for i in range(B)]
+    g = torch.Generator(device=DEV).manual_seed(G * B + P)
+    bt, blocks = _tables(B, width, g)
+    kc = torch.randn(blocks, kv, 32, D, device=DEV, generator=g).bfloat16()
+    vc = torch.randn(blocks, kv, D, 32, device=DEV, generator=g).bfloat16()
+    bt[1::2, :2] = bt[:1, :2]                           # what odd sequences share with the first
+    q = torch.randn(B, heads, D, device=DEV, generator=g).bfloat16()
+    lens = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    for window, shared in ((0, None), (70, None), (0, torch.tensor([2], dtype=torch.int32, device=DEV))):
+        got = K.paged_decode_attention(q, kc, vc, bt, lens, D ** -0.5, part_blocks=-P, window=window, shared_blocks=shared)
+        for s in range(0, B, 3):
+            k, v = _keys_values(kc, vc, bt[s], ctx[s])
+            lo = max(0, ctx[s] - window) if window else 0
+            p = torch.softmax(q[s].double().view(kv, G, D) @ k[:, lo:].transpose(1, 2).contiguous() * D ** -0.5, -1)
+            _close(got[s].view(kv, G, D), p @ v[:, lo:], (p @ v[:, lo:].abs()).max())
