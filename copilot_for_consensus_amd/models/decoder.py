@@ -415,19 +415,15 @@ def argmax_keys(local: torch.Tensor, offset: int) -> torch.Tensor:
 @functools.lru_cache(maxsize=4096)
 def kv_partitions(B: int, heads: int, kv_heads: int, blocks: int) -> int:
     """Partitions of each of B sequences of ``blocks`` cache blocks in the paged decode attention, by what a launch takes in
-    us.  5 to 128 sequences, whose keys and values come through LDS, fitted to 848 measured (32 query and 8 key heads, 4 to 173
-    blocks, 1 to 12 partitions): 3.6, 2.2 and 0.03 per 32 rows and partition more for the merge, and what the chip reads, 6.5
-    TB/s, or the busiest of 256 CUs, four blocks in 1.54, whichever is longer.  Before, a workgroup for every place, and now: 20
-    of 700 16.2 -> 14.0, 24 of 1500 31.1 -> 26.7, 24 of 2617 47.4 -> 43.1, 32 of 2617 61.0 -> 57.8, 5 of 2617 16.2 -> 15.7, 8 of 300
-    8.0 -> (8.4); on average 0.9 % more than the best P.
+    us.  5 to 128 sequences, whose keys and values come through LDS: :func:`ops.kernels.streamed_us`.  As many as give a
+    workgroup for every place, and this many: 20 of 700 15.9 -> 13.9, 24 of 1500 32.6 -> 26.5, 24 of 2617 48.3 -> 42.6, 12 of 2617
+    27.4 -> 26.6, 32 of 2617 61.1 -> 57.5.
     Fewer or more sequences fitted to 1048 measured (B of 1 .. 128, 2 .. 172 blocks, 1 .. 64 partitions of 8 KV heads, fragments
     from memory): 3.3, 4.2 and 0.045 for the merge, and what the busiest of 256 CUs, two workgroups each, reads: one block
     per wave takes 3.1 to 3.8 where a CU has one workgroup, 4.5 to 5.5 where some have two, 5 per full round of 512.  A
     workgroup for every slot and a few more is a round more, and few keys are not worth a merge."""
     def streamed(P):
-        chip = B * kv_heads * blocks * 16384 / 6.5e6
-        cu = math.ceil(B * kv_heads * P / 256) * math.ceil(blocks / P / 4) * 1.54
-        return 3.6 + (2.2 + 0.03 * B * P * heads / 32 if P > 1 else 0.0) + (chip ** 4 + cu ** 4) ** 0.25
+        return K.streamed_us(blocks, B * kv_heads, 16384, B * heads, P)
 
     def us(P):
         full, rest = divmod(B * kv_heads * P, 512)

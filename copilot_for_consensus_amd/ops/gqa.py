@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import bisect
 import dataclasses
+import functools
 import math
 from fractions import Fraction
 
@@ -17,7 +18,7 @@ import torch
 from . import reference as ref
 from ._native import check, kernels
 from .cols import Cols
-from .kernels import _p, _req, _stream, _workspace
+from .kernels import _p, _req, _stream, _workspace, streamed_us
 from .stream import _act
 
 KV_BLOCK = ref.KV_BLOCK
@@ -256,21 +257,23 @@ def prompt_tiles(cu, ctx, H: int, G: int, rows: int) -> np.ndarray:
     return np.stack([np.concatenate(seq)[order], np.concatenate(m0)[order]]).astype(np.int32)
 
 
+@functools.lru_cache(maxsize=4096)
 def decode_slices(B: int, H: int, G: int, D: int, visible: int, dtype) -> int:
-    """Key slices per row of a decode step, at least eight 32-key tiles each.  MFMA kernel: two of its workgroups share a
-    CU, and half a round more than that evens their lengths out (256 items of 1024 keys: 4 slices 34.0 us, 3 31.4, 2
-    32.1; 320 of 1500: 59.2, 56.4, 59.3).  From 384 items on one slice where few keys are seen: the merge, 5 us, costs more
-    than slices gain.  What they gain grows with the longest row, whose keys are one workgroup's work, and the rows'
-    differences (us with one slice / with 1024 / items, rows of equal, 0.4 - 1, 0 - 1 times the length: 384 items of 1024 keys
-    48 / 50, 39 / 42, 33 / 36; 896 items 95 / 99, 71 / 76, 57 / 62; 384 of 1536 uneven 54 / 54 and 46 / 46, of 6000 218 / 215,
-    182 / 165, 148 / 129; 448 of 6000 235 / 254, 193 / 187, 160 / 148; one row in 16 eight times the others: 384 of 1024
-    34 / 27, of 6000 153 / 92).  Others: about four workgroups per CU."""
+    """Key slices per row of a decode step, at least eight 32-key tiles each.  MFMA kernel: from 384 items on one slice where few
+    keys are seen, else 1024 in all: what more gain grows with the longest row, whose keys are one workgroup's work, and the rows'
+    differences.  Fewer: at most 768 in all, and as many as :func:`streamed_us` finds fastest.  us of 8 key heads with 768 and with
+    this many: 24 of 512 keys 16.0 -> 12.5, 24 of 2000 41.3 -> 35.3, 32 of 1024 31.2 -> 25.1, 8 of 4000 31.4 -> 27.3, 12 of 1024 16.0 ->
+    15.3.  One row: as many as there are.  Others: about four workgroups per CU."""
     if dtype != torch.bfloat16 or D not in MFMA_DIMS:
         return max(1, min(math.ceil(1024 / (B * math.ceil(H / ANY_ROWS))), visible // 256, MAX_PARTITIONS))
     items = B * G * math.ceil(H / G / 16)
     if items >= 384 and visible <= 1536:
         return 1
-    return max(1, min(math.ceil((768 if items < 384 else 1024) / items), visible // 256, MAX_PARTITIONS))
+    most = max(1, min(math.ceil((768 if items < 384 else 1024) / items), visible // 256, MAX_PARTITIONS))
+    if items >= 384 or B == 1:
+        return most
+    most = max(1, min(math.ceil(768 / items), math.ceil(visible / 256)))      # (the last slice may have fewer tiles)
+    return min(range(1, most + 1), key=lambda P: streamed_us(math.ceil(visible / 32), items, 128 * D, B * H, P))
 
 
 def attention(a: Heads, q, rows, block_tables, ctx_lens, cu_q=None, tiles=None, P: int = 1, workspace=None, gate: Cols | None = None,

@@ -194,6 +194,18 @@ def rope_kv_write(qkv, positions, slots, cos_sin, k_cache, v_cache, Hq, Hkv, D, 
     return q_out
 
 
+def streamed_us(tiles: int, items: int, tile_bytes: int, rows: int, P: int) -> float:
+    """What a decode step's attention and merge take in us, less its start: ``items`` workgroups by ``P`` slices of ``tiles`` tiles
+    of 32 keys (``tile_bytes`` of keys and values each) that come through LDS (csrc/kernels/lds_ring.h), ``rows`` query rows.  The
+    chip's 6.5 TB/s, or the busiest of 256 CUs, 3.4 us for its eight waves' tiles of 16 KB, whichever is longer; eight waves of one
+    workgroup, or four of each of two.  Its best P takes 0.8 % more than the best of 1400 measured (2 to 128 sequences, 32 query and
+    8 key heads of 128 columns, 100 to 5500 keys, 1 to 24 slices)."""
+    w = items * P
+    cu = math.ceil(tiles / P / 8) if w <= 256 else math.ceil(w / 256) * math.ceil(tiles / P / 4) / 2
+    merge = 3.4 + 0.06 * rows * P / 32 if P > 1 else 0.0
+    return merge + ((items * tiles * tile_bytes / 6.5e6) ** 4 + (cu * tile_bytes / 16384 * 3.4) ** 4) ** 0.25
+
+
 def decode_partitions(max_ctx: int, part_blocks: int) -> int:
     return max(1, math.ceil(math.ceil(max_ctx / KV_BLOCK) / part_blocks))
 

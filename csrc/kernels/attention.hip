@@ -23,7 +23,7 @@
 //     ([D][32] rows: 64), which is what its write costs the step.
 //   * LDS tiles are XOR-swizzled for conflict-free ds_read_b128; the swizzles
 //     were derived against the gfx950 ds_read_b128 lane groups {0-3,12-15,20-27}, ...
-#include "common.h"
+#include "lds_ring.h"
 #include <stdlib.h>
 
 #include <type_traits>
@@ -469,36 +469,6 @@ __global__ void __launch_bounds__(256, F8 ? 2 : 1) paged_decode_kernel(
 // A workgroup of NWV waves has one (partition of a) sequence and kv head, wave w its blocks w, w + NWV, ...
 // bf16 cache, queries roped.
 // ------------------------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void pd_lds_t;
-
-template <bool NT>
-__device__ __forceinline__ void pd_piece(uint32_t voff, const void* sbase, uint32_t lds_addr) {
-  unsigned keep;
-  if constexpr (NT)
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
-        : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
-  else
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-        : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void pd_wait() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(N) : "memory");
-}
-
-// behind tile j of `tiles`: those that are asked for
-template <int T>
-__device__ __forceinline__ void pd_landed(int j, int tiles) {
-  const int left = tiles - 1 - j;
-  if (left >= T - 1) pd_wait<8 * (T - 1)>();
-  else if (T > 3 && left == 2) pd_wait<16>();
-  else if (T > 2 && left == 1) pd_wait<8>();
-  else pd_wait<0>();
-}
-
 template <int G, int NWV, int T>
 __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
@@ -506,17 +476,20 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
     int P, int window, float v_scale, float* __restrict__ part_o, float* __restrict__ part_ml, uint16_t* __restrict__ out,
     const int32_t* __restrict__ shared_blocks, int ordered) {
   constexpr int D = 128, TILE = KV_BS * D * 2, QB = (G + 3) / 4 * 1024, RING = T * TILE;
+  constexpr bool ORD = NWV == 4 && T == 2;
   __shared__ __attribute__((aligned(16))) char smem[NWV * (RING + QB)];
   const int p = blockIdx.x, h = blockIdx.y;
   int b = blockIdx.z, ctx;
-  if (T == 2 && ordered) {
-    const int2 s = longest_first<64 * (T == 2 ? NWV : 4)>(ctx_lens, gridDim.z, blockIdx.z, ordered);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool whole = !(ORD && ordered) && P == 1 && window == 0;       // the table's blocks: asked for beside the length
+  const int spec = whole ? block_tables[(size_t)b * max_blocks + min(w + NWV * lane, max_blocks - 1)] : 0;
+  if (ORD && ordered) {
+    const int2 s = longest_first<256>(ctx_lens, gridDim.z, blockIdx.z, ordered);
     b = s.x;
     ctx = s.y;
   } else {
     ctx = ctx_lens[b];
   }
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
   const int Hq = Hkv * G;
   const int nblk = (ctx + KV_BS - 1) / KV_BS;
@@ -526,9 +499,15 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
   const int first = blk0 + w, n = first < blk1 ? (blk1 - 1 - first) / NWV + 1 : 0;        // this wave's blocks
   const int temporal = shared_blocks != nullptr ? shared_blocks[0] : 0;                   // blocks read through the caches
   char* mine = smem + w * (RING + QB);
-  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(pd_lds_t*)mine);
+  const uint32_t lds0 = lds_at(mine);
   const uint32_t kvoff = (lane >> 4) * 256u, vvoff = lane * 16u;     // K: a piece has four rows, chunk (lane & 15) ^ row of each
-  auto id = [&](int i) { return i < n ? bt[first + i * NWV] : 0; };
+  int ids = whole ? spec : n > 0 ? bt[first + min(lane, n - 1) * NWV] : 0;
+  // the block of tile i, asked for in turn, from the lane that has it: a scalar load of its own would be waited for with every
+  // read of LDS
+  auto id = [&](int i) {
+    if (i > 0 && (i & 63) == 0 && i < n) ids = bt[first + min(i + lane, n - 1) * NWV];
+    return __builtin_amdgcn_readlane(ids, i & 63);
+  };
   // tile 2 i + v: keys (v 0) or values of this wave's block i
   auto issue = [&](int j, int block) {
     const bool key = (j & 1) == 0;
@@ -538,8 +517,8 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const uint32_t vo = key ? kvoff + (((lane & 15) ^ ((4 * e + (lane >> 4)) & 15)) << 4) : vvoff;
-      if (nt) pd_piece<true>(vo, src + e * 1024, at + e * 1024);
-      else pd_piece<false>(vo, src + e * 1024, at + e * 1024);
+      if (nt) ring_piece<true>(vo, src + e * 1024, at + e * 1024);
+      else ring_piece<false>(vo, src + e * 1024, at + e * 1024);
     }
   };
   f32x4_t o[8];
@@ -552,7 +531,7 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
     const char* qs = reinterpret_cast<const char*>(q + ((size_t)b * Hq + h * G) * D);
 #pragma unroll
     for (int e = 0; e < QB / 1024; ++e)
-      pd_piece<false>((uint32_t)min(4 * e + (lane >> 4), G - 1) * 256u + (lane & 15) * 16u, qs, lds0 + RING + e * 1024);
+      ring_piece<false>((uint32_t)min(4 * e + (lane >> 4), G - 1) * 256u + (lane & 15) * 16u, qs, lds0 + RING + e * 1024);
 #pragma unroll
     for (int j = 0; j < T; j += 2)
       if (j < 2 * n) {
@@ -563,7 +542,7 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
     int ahead = id(T / 2);                         // the block of the tiles T on
     for (int i = 0; i < n; ++i) {
       const int bi = first + i * NWV, next = id(i + 1 + T / 2);
-      pd_landed<T>(2 * i, 2 * n);
+      ring_landed<T, 8>(2 * i, 2 * n);
       if (i == 0) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
@@ -615,7 +594,7 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
       l = l * alpha + rs;
       m = mn;
       const bf16x8_t pf = pack_p(s[0], s[1]);
-      pd_landed<T>(2 * i + 1, 2 * n);
+      ring_landed<T, 8>(2 * i + 1, 2 * n);
       uint4 vf[8];
       const char* vi = mine + ((2 * i + 1) & (T - 1)) * TILE + g * 2048 + col * 16;
 #pragma unroll
@@ -1756,8 +1735,8 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
   const bool nt = nt_env >= 0 ? nt_env != 0 : B >= 32;
   // Through LDS in whole runs, unless the table holds 256 keys at most and the workgroups are few, or more sequences than are
   // ordered wait: those have 2 GB of cache and more to read from, and what waits in registers is deeper.
-  // us of 8 key heads, one partition, fragments from memory -> this: 8 of 2617 keys 50.3 -> 35.7, 24 59.9 -> 44.3, 32 66.2 -> 58, 48 97 ->
-  // 88, 64 111 -> 108, 72 158 -> 131, 90 170 -> 157, 128 219 -> 212, from 0.8 of it 198 -> 191; 24 of 700 19.1 -> 16.3, 8 of 300 9.1 -> 8.5; 12 of
+  // us of 8 key heads, one partition, fragments from memory -> this: 8 of 2617 keys 50.3 -> 31.4, 24 59.9 -> 42.6, 32 66.2 -> 57.5, 48
+  // 97 -> 88, 72 158 -> 131, 90 170 -> 157, 128 219 -> 212, from 0.8 of it 198 -> 191; 24 of 700 19.1 -> 14.9, 8 of 300 9.1 -> 7.7; 12 of
   // 64 4.5 -> 5.1, 192 of 2617 315 -> 330.
   if constexpr (!F8) {
     if (!rope && part_blocks <= 0 && (wgs > 256 || max_blocks > 8) && B <= DEC_ORDER_ROWS) {
@@ -1765,15 +1744,17 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
   paged_stream_kernel<GG, NWV, T><<<grid, 64 * NWV, 0, stream>>>((const uint16_t*)q, (const uint16_t*)k_cache,               \
       (const uint16_t*)v_cache, block_tables, ctx_lens, sl2, Hkv, max_blocks, P, window, v_scale, part_o, part_ml,           \
       (uint16_t*)out, shared_blocks, ordered)
-      // 96 to 128 KB under way in a CU: four waves of one workgroup, of two, or eight waves of two that the next ones follow
-      // one by one; few keys in one wave each, which have nothing to merge (128 of 60 11.7 -> 9.5 us, 11.5 in four)
+      // 128 KB under way in a CU, in the eight waves of one workgroup (four with rings of twice the depth: 24 of 1500 28.1 against
+      // 25.7, 16 of 700 14.5 against 13.8) or the four of each of two (two waves with twice the depth: 40 of 1500 52.7 against 49.1,
+      // 48 of 300 15.4 against 14.3); two blocks in one wave, which has nothing to merge (128 of 60 11.4 -> 9.1 us).  Up to
+      // 64 workgroups in four waves all the same: those of the fused step, whose small batches get the same bits either way
 #define PDS_CASE(G_)                        \
   case G_: {                                \
     constexpr int GG = G_;                  \
-    if (wgs <= 256) PDS_GO(4, 4);           \
-    else if (wgs <= 512) PDS_GO(2, 4);      \
-    else if (max_blocks <= 8) PDS_GO(1, 4); \
-    else PDS_GO(4, 2);                      \
+    if (wgs <= 64) PDS_GO(4, 4);            \
+    else if (wgs <= 256) PDS_GO(8, 2);      \
+    else if (max_blocks > 2) PDS_GO(4, 2);  \
+    else PDS_GO(1, 4);                      \
   } break;
       switch (G) {
         PDS_CASE(1) PDS_CASE(2) PDS_CASE(4) PDS_CASE(8) PDS_CASE(16)

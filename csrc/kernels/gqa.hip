@@ -9,14 +9,15 @@
 // with a cap so that exp2 of the score is e^(2 score / cap).
 // Heads h of G groups: R = H / G consecutive heads share a key / value head.
 //
-//   * gqa_decode   one token per sequence: a workgroup per (sequence, key head, slice of its keys), its four waves on
-//                  32-key tiles of their own.  Keys go straight from memory into the score product's operand, values
-//                  through a wave's own LDS tile, read back transposed (ds_read_b64_tr_b16); the score product's
-//                  result is the output product's operand as it lies.  No barrier until the waves merge
+//   * gqa_decode   one token per sequence: a workgroup per (sequence, key head, slice of its keys), its waves on 32-key
+//                  tiles of their own, which come to LDS in whole runs; values are read back transposed
+//                  (ds_read_b64_tr_b16); the score product's result is the output product's operand as it lies.  No
+//                  barrier until the waves merge
 //   * gqa_prompt   portions of prompts: 32 rows of the flattened (token, head of the group) rows per wave, 64-key tiles
 //                  of both ranges double-buffered in LDS
 //   * gqa_any      any head size and the 32-bit path: a wave per (token, head) row
 //   * slices of a row's keys are merged by slice_merge (split_merge.h)
+#include "lds_ring.h"
 #include "split_merge.h"
 
 namespace {
@@ -36,6 +37,7 @@ struct GqaArgs {
   const int32_t* tile_m0;
   int n_tiles;
   int H, G, D, DV, max_blocks, P;      // DV: value columns that leave
+  int R, RG;                           // query rows of a key head, sixteens of them
   int size, keep, pool, le;            // window; first tokens; tokens per pooled block, log2 of entries per page
   int chunk;                           // size counts from multiples of it
   int capped; float cap2;              // 0: no cap, 1: any score, 2, 3: |score| <= 0.35, 0.25 cap; cap log2(e)
@@ -133,64 +135,81 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 
 // ------------------------------------------------------------------------------------------ decoded tokens
-// grid (B * G * ceil(R / 16), P)
-template <int D, bool SHAPED>
-__global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const uint16_t* __restrict__ q,
-                                                                          const uint16_t* __restrict__ kc,
-                                                                          const uint16_t* __restrict__ vc,
-                                                                          const uint16_t* __restrict__ pk,
-                                                                          const uint16_t* __restrict__ pv, GqaArgs a,
-                                                                          uint16_t* __restrict__ out) {
-  constexpr int KS = D / 32, NV = D / 16, CH = D / 8, DT = D / 16;
-  __shared__ __attribute__((aligned(16))) char smem[4 * 64 * D];     // a wave's 32 x D values; then its 16 x D outputs
-  __shared__ float ml[4][16][2];
+// grid (B * G * ceil(R / 16), P).  A workgroup of NWV waves, wave w on its slice's tiles w, w + NWV, ..; keys and values come
+// through a ring of T tiles of the wave's own (lds_ring.h), chunks swizzled through the pieces' source addresses.  A tile that is
+// one cache block's is one run; those of pooled pages of fewer entries and the last of the far range, past whose keys nothing
+// is read, come by rows.  What bounds it is memory: loads straight to registers (keys 64 bytes of 16 rows each) kept one tile of
+// each wave under way, 3.6 to 5.4 TB/s; us of heads of 128, 8 key heads, 0.7 to 1 times the keys, with the slices of either: 12
+// of 4000 39.8 -> 36, 32 of 1024 31.7 -> 23, 48 of 1024 39.7 -> 34.3, 105 of 852 65.9 -> 57.3, 128 of 2600 212 -> 191; heads of 256, 64
+// of 1024 39.6 -> 29; of 64, 64 of 3000 69.7 -> 62.9.  Of 30 keys, one tile, 4.9 -> 5.1, and heads of 32 to 96 of up to 100 keys
+// 0.2 to 0.4 more than before.
+template <int D, bool SHAPED, int NWV, int T>
+__global__ void __launch_bounds__(64 * NWV, D <= 64 || (D <= 128 && NWV < 8 && T == 2) ? 2 : 1) gqa_decode_kernel(const uint16_t* __restrict__ q,
+                                                                                       const uint16_t* __restrict__ kc,
+                                                                                       const uint16_t* __restrict__ vc,
+                                                                                       const uint16_t* __restrict__ pk,
+                                                                                       const uint16_t* __restrict__ pv, GqaArgs a,
+                                                                                       uint16_t* __restrict__ out) {
+  constexpr int KS = D / 32, CH = D / 8, DT = D / 16, NP = D / 16, TILE = 64 * D, RING = T * TILE;
+  __shared__ __attribute__((aligned(16))) char smem[NWV * RING + 32 * D + 256];     // rings (then 16 x D outputs each), queries, far biases
+  __shared__ float ml[NWV][16][2];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, kq = lane >> 4;
-  const int R = a.H / a.G, RG = (R + 15) / 16;
-  int item = blockIdx.x;
-  const int rg = item % RG;
-  item /= RG;
-  const int hk = item % a.G, s = item / a.G, pos = a.ctx_lens[s] - 1;
+  const int R = a.R, RG = a.RG;
+  const int rg = RG == 1 ? 0 : blockIdx.x % RG, item = RG == 1 ? blockIdx.x : blockIdx.x / RG;
+  const int s = item / a.G, hk = item - s * a.G, pos = a.ctx_lens[s] - 1;
   const int32_t* bt = a.block_tables + (size_t)s * a.max_blocks;
+  const bool whole = a.size == 0 && a.P == 1;       // the tiles are the table's: asked for beside the length
+  int pages = whole ? bt[min(w + NWV * lane, a.max_blocks - 1)] : 0;
   const KeyTiles kt = key_tiles<32>(a, pos, pos);
-  const int t0 = share_of(kt.nt, blockIdx.y, a.P), t1 = share_of(kt.nt, blockIdx.y + 1, a.P);
+  const int t0 = share_of(kt.nt, blockIdx.y, a.P) + w, t1 = share_of(kt.nt, blockIdx.y + 1, a.P);
+  const int n = t0 < t1 ? (t1 - 1 - t0) / NWV + 1 : 0;                              // this wave's tiles
   const int r0 = 16 * rg, nr = min(16, R - r0);
   const size_t qrow = (size_t)s * a.H + hk * R + r0;
-
-  u32x4_t qf[KS];
-  char* vbuf = smem + w * 64 * D;
+  char* mine = smem + w * RING;
+  char* qbuf = smem + NWV * RING;
+  const uint32_t lds0 = lds_at(mine);
   const float* bias = SHAPED && a.bias ? a.bias + (size_t)(hk * R + r0 + min(col, nr - 1)) * a.nb : nullptr;
-  const float far_bias = bias ? bias[a.nb - 1] : 0.f;
-  u32x4_t kf[2][KS], vf[NV];
+  float far_bias = 0.f;
   const int first = a.size ? window_first(a, pos) : 0;
-  // This lane's key (lane & 31) in a tile (past the slice: its last), the cache block that it is in, and its row.  The block goes
-  // from one step to the next, and not the row: that would be waited for as soon as it is asked for, and with it all that was
-  // asked for before it, the next tile (one slice of 2800 keys, heads of 128: 38 us with rows, 30).  Heads of more than 160
-  // columns have no registers left for it (of 256: 62 with rows, 80).
-  constexpr bool ROWS = D > 160;
-  auto key_of = [&](int t) {
-    t = min(t, t1 - 1);
-    return t < kt.nat ? min(32 * t + (lane & 31), kt.na - 1) : kt.lo + 32 * (t - kt.nat) + (lane & 31);
+  // the pages of the first keys of this wave's tiles i, i + 1, .. in its lanes
+  auto find = [&](int i) {
+    const int t = t0 + min(i + lane, n - 1) * NWV;
+    return bt[t >= kt.nat ? (kt.lo >> 5) + t - kt.nat : a.pool ? (32 * t) >> a.le : t];
   };
-  auto pooled_at = [&](int t) { return a.pool && min(t, t1 - 1) < kt.nat; };
-  auto row_in = [&](int t, int block) { return key_row(a, pooled_at(t), block, hk, key_of(t)); };
-  auto find = [&](int t) {
-    const int block = bt[key_page(a, pooled_at(t), key_of(t))];
-    return ROWS ? row_in(t, block) : block;
+  // that of tile i, asked for in turn: a scalar load of its own would be waited for with every read of LDS
+  auto page_of = [&](int i) {
+    if (i > 0 && (i & 63) == 0 && i < n) pages = find(i);
+    return __builtin_amdgcn_readlane(pages, i & 63);
   };
-  auto load = [&](int t, int found) {
-    const bool pooled = pooled_at(t);
-    const int row = ROWS ? found : row_in(t, found);
-    const uint16_t *kb = pooled ? pk : kc, *vb = pooled ? pv : vc;
+  int erow = 0;                                    // the row of this lane's key (lane & 31) of a tile that comes by rows
+  // tile 2 i + v: keys (v 0) or values of this wave's tile i
+  auto issue = [&](int j, int page) {
+    const bool key = (j & 1) == 0;
+    const int t = t0 + (j >> 1) * NWV;
+    const uint32_t at = __builtin_amdgcn_readfirstlane(lds0 + (j & (T - 1)) * TILE);
+    const bool pooled = a.pool && t < kt.nat;
+    const uint16_t* c = pooled ? (key ? pk : pv) : (key ? kc : vc);
+    if (t < kt.nat && (32 * t + 32 > kt.na || (pooled && a.le < 5))) {
+      if (key) {
+        const int l = pooled ? a.le : 5, e = min(32 * t + (lane & 31), kt.na - 1), last = (kt.na - 1) >> l;
+        int pg = page;
+        for (int p = ((32 * t) >> l) + 1; p <= last && p < (32 * t + 32) >> l; ++p) pg = e >> l == p ? bt[p] : pg;
+        erow = key_row(a, pooled, pg, hk, e);
+      }
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const uint16_t* p = kb + (size_t)__shfl(row, 16 * g + col, 64) * D + 8 * kq;
+      for (int i = 0; i < NP; ++i) {
+        const int e = lane + 64 * i, r = e / CH, ch = (e % CH) ^ (key ? kswz<D>(r) : vswz<D>(r));
+        ring_piece_at(c + (size_t)__shfl(erow, r, 64) * D + 8 * ch, at + 1024 * i);
+      }
+    } else {
+      const uint16_t* src = c + (size_t)key_row(a, false, page, hk, 0) * D;
 #pragma unroll
-      for (int k = 0; k < KS; ++k) kf[g][k] = *reinterpret_cast<const u32x4_t*>(p + 32 * k);
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int e = lane + 64 * i;
-      vf[i] = *reinterpret_cast<const u32x4_t*>(vb + (size_t)__shfl(row, e / CH, 64) * D + 8 * (e % CH));
+      for (int i = 0; i < NP; ++i) {
+        const int e = lane + 64 * i, r = e / CH, ch = (e % CH) ^ (key ? kswz<D>(r) : vswz<D>(r));
+        const uint32_t vo = r * (2 * D) + 16 * ch;
+        if (RG == 1) ring_piece<true>(vo, src, at + 1024 * i);       // more than 16 rows a key head: others read the tile, too
+        else ring_piece<false>(vo, src, at + 1024 * i);
+      }
     }
   };
 
@@ -198,31 +217,47 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
 #pragma unroll
   for (int d = 0; d < DT; ++d) o[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
-  int t = t0 + w;
-  if (t < t1) {
-    int found = find(t);
-    load(t, found);
+  if (n > 0) {
+    // the queries first (each wave brings the same bytes): they are there when the first keys are
 #pragma unroll
-    for (int k = 0; k < KS; ++k)             // behind the first tile, which waits for indexes
-      qf[k] = *reinterpret_cast<const u32x4_t*>(q + (qrow + min(col, nr - 1)) * D + 32 * k + 8 * kq);
-    found = find(t + 4);
-    auto step = [&](auto more) {
-      wave_lds_fence();                      // the last tile's values have been read
+    for (int i = 0; i < KS; ++i) {
+      const int e = lane + 64 * i;
+      ring_piece<false>(min(e / CH, nr - 1) * (2 * D) + 16 * (e % CH), q + qrow * D, lds_at(qbuf) + 1024 * i);
+    }
+    if (!whole) pages = find(0);
+    if (SHAPED && a.bias) ring_word_at(bias + a.nb - 1, lds_at(qbuf) + 32 * D);
 #pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int e = lane + 64 * i, key = e / CH, c = e % CH;
-        *reinterpret_cast<u32x4_t*>(vbuf + key * (2 * D) + ((c ^ vswz<D>(key)) << 4)) = vf[i];
+    for (int i = 0; i < T / 2; ++i)
+      if (i < n) {
+        const int page = page_of(i);
+        issue(2 * i, page);
+        issue(2 * i + 1, page);
       }
+    int ahead = page_of(T / 2);
+    u32x4_t qf[KS];
+    for (int i = 0; i < n; ++i) {
+      const int t = t0 + i * NWV, next = page_of(i + 1 + T / 2);
+      ring_landed<T, NP>(2 * i, 2 * n);
+      if (i == 0) {
+#pragma unroll
+        for (int k = 0; k < KS; ++k) qf[k] = *reinterpret_cast<const u32x4_t*>(qbuf + col * (2 * D) + 64 * k + 16 * kq);
+        if (SHAPED && a.bias) far_bias = *reinterpret_cast<const float*>(qbuf + 32 * D + 4 * lane);
+      }
+      u32x4_t kf[2][KS];
+      const char* ki = mine + (2 * i & (T - 1)) * TILE;
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+          kf[g][k] = *reinterpret_cast<const u32x4_t*>(ki + (16 * g + col) * (2 * D) + (((4 * k + kq) ^ kswz<D>(16 * g + col)) << 4));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // read: the place is free
+      if (i + T / 2 < n) issue(2 * i + T, ahead);
       f32x4_t sc[2];
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
         sc[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < KS; ++k) sc[g] = mfma16(kf[g][k], qf[k], sc[g]);
-      }
-      if constexpr (decltype(more)::value) {
-        load(t + 4, found);
-        found = find(t + 8);
       }
       const bool far = t < kt.nat;
       // (key <= last ..: what sees() says of the tile's keys, without its branches at each of them)
@@ -233,27 +268,26 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
 #pragma unroll
           for (int g = 0; g < 2; ++g)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) bt8[g][i] = bias[min(max(pos - k0 - (16 * g + 4 * kq + i), 0), a.nb - 1)];
+            for (int e = 0; e < 4; ++e) bt8[g][e] = bias[min(max(pos - k0 - (16 * g + 4 * kq + e), 0), a.nb - 1)];
         } else {
 #pragma unroll
           for (int g = 0; g < 2; ++g)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) bt8[g][i] = far_bias;
+            for (int e = 0; e < 4; ++e) bt8[g][e] = far_bias;
         }
 #pragma unroll
         for (int g = 0; g < 2; ++g)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) sc[g][i] = a.capped ? cap_score<uint16_t>(a, sc[g][i], bt8[g][i]) : sc[g][i] + bt8[g][i];
+          for (int e = 0; e < 4; ++e) sc[g][e] = a.capped ? cap_score<uint16_t>(a, sc[g][e], bt8[g][e]) : sc[g][e] + bt8[g][e];
       }
       float mx = -INFINITY;
 #pragma unroll
       for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = k0 + 16 * g + 4 * kq + i;
-          const bool see = ROWS ? (far ? key < kt.na : sees(a, pos, key)) : (key <= last) & ((key >= lo) | (key < a.keep));
-          if (!see) sc[g][i] = -INFINITY;
-          mx = fmaxf(mx, sc[g][i]);
+        for (int e = 0; e < 4; ++e) {
+          const int key = k0 + 16 * g + 4 * kq + e;
+          if (!((key <= last) & ((key >= lo) | (key < a.keep)))) sc[g][e] = -INFINITY;
+          mx = fmaxf(mx, sc[g][e]);
         }
       mx = xor32_max(xor16_max(mx));
       const float mn = fmaxf(m, mx), ref = mn == -INFINITY ? 0.f : mn, alpha = __builtin_amdgcn_exp2f(m - ref);
@@ -266,9 +300,9 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
 #pragma unroll
       for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          sc[g][i] = __builtin_amdgcn_exp2f(sc[g][i] - ref);
-          l += sc[g][i];
+        for (int e = 0; e < 4; ++e) {
+          sc[g][e] = __builtin_amdgcn_exp2f(sc[g][e] - ref);
+          l += sc[g][e];
         }
       // operand slots 8 kq + j: keys 4 kq + j of the first 16, then of the second
       u32x4_t pf;
@@ -276,47 +310,46 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_decode_kernel(const
       pf[1] = cvt_pk_bf16_f32(sc[0][2], sc[0][3]);
       pf[2] = cvt_pk_bf16_f32(sc[1][0], sc[1][1]);
       pf[3] = cvt_pk_bf16_f32(sc[1][2], sc[1][3]);
-      wave_lds_fence();
+      ring_landed<T, NP>(2 * i + 1, 2 * n);
+      const char* vi = mine + ((2 * i + 1) & (T - 1)) * TILE;
+      u32x4_t vt[DT];
 #pragma unroll
-      for (int d = 0; d < DT; ++d) {
-        u32x4_t vt;
+      for (int d = 0; d < DT; ++d)
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const int key = 16 * u + 4 * kq + (col >> 2), c = 2 * d + ((col & 3) >> 1);
-          const uint2 v = tr_read(vbuf + key * (2 * D) + ((c ^ vswz<D>(key)) << 4) + 8 * (col & 1));
-          vt[2 * u] = v.x;
-          vt[2 * u + 1] = v.y;
+          const uint2 v = tr_read(vi + key * (2 * D) + ((c ^ vswz<D>(key)) << 4) + 8 * (col & 1));
+          vt[d][2 * u] = v.x;
+          vt[d][2 * u + 1] = v.y;
         }
-        o[d] = mfma16(vt, pf, o[d]);
-      }
-    };
-    // The last step asks for nothing: a tile that no one uses was one in three or four of a short slice's loads.  In a step of its
-    // own: behind a condition in the loop the loads stay where they are (2800 keys in one slice 38 -> 50 us)
-    for (; t + 4 < t1; t += 4) step(std::true_type{});
-    step(std::false_type{});
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (i + T / 2 < n) issue(2 * i + 1 + T, ahead);
+#pragma unroll
+      for (int d = 0; d < DT; ++d) o[d] = mfma16(vt[d], pf, o[d]);
+      ahead = next;
+    }
   }
   l = xor32_sum(xor16_sum(l));
-  wave_lds_fence();
-  float* ob = reinterpret_cast<float*>(vbuf);            // [16][D]
+  float* ob = reinterpret_cast<float*>(mine);            // [16][D + 4]: the wave's tiles are used up
 #pragma unroll
-  for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(ob + col * D + 16 * d + 4 * kq) = o[d];
+  for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(ob + col * (D + 4) + 16 * d + 4 * kq) = o[d];
   if (lane < 16) {
     ml[w][lane][0] = m;
     ml[w][lane][1] = l;
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < nr * (D / 4); e += 256) {
+  for (int e = threadIdx.x; e < nr * (D / 4); e += 64 * NWV) {
     const int r = e / (D / 4), c = 4 * (e % (D / 4));
     float M = -INFINITY, L = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) M = fmaxf(M, ml[i][r][0]);
+    for (int i = 0; i < NWV; ++i) M = fmaxf(M, ml[i][r][0]);
     const float ref = M == -INFINITY ? 0.f : M;
     f32x4_t y{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NWV; ++i) {
       const float f = exp2f(ml[i][r][0] - ref);
       L += f * ml[i][r][1];
-      y += f * *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(smem + i * 64 * D) + r * D + c);
+      y += f * *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(smem + i * RING) + r * (D + 4) + c);
     }
     const size_t grow = qrow + r;
     if (a.P > 1) {
@@ -698,6 +731,29 @@ int prompt_go(int grid, hipStream_t s, const void* q, const void* kc, const void
   return CFC_CHECK_LAUNCH();
 }
 
+template <int D, bool SHAPED>
+int decode_go(dim3 grid, hipStream_t s, const void* q, const void* kc, const void* vc, const void* pk, const void* pv, const GqaArgs& a,
+              void* out) {
+#define GDK(NWV, T)                                                                                                                 \
+  gqa_decode_kernel<D, SHAPED, NWV, T><<<grid, 64 * NWV, 0, s>>>((const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc,        \
+                                                                 (const uint16_t*)pk, (const uint16_t*)pv, a, (uint16_t*)out)
+  // 64 to 128 KB under way in a CU, as in attention.hip: eight waves of one workgroup, or of each of two where the rings are small
+  // enough (heads of 128, four waves with rings of twice the depth -> eight: 5 of 700 15.4 -> 11.7 us, 24 of 1500 30.9 -> 27.6), four of
+  // two (two of twice the depth: 48 of 1024 38.4 -> 34.3); one for two blocks (128 of 60 12.4 -> 11.4); heads of more than 128
+  // columns four of one, two of each of two (heads of 160, 300 to 512 workgroups: 22.5 -> 19.4; more in fours: 158 -> 142)
+  const int64_t wgs = (int64_t)grid.x * grid.y;
+  if constexpr (D > 128) {
+    if (wgs > 256 && wgs <= 512) GDK(2, 2);
+    else GDK(4, 2);
+  } else {
+    if (a.max_blocks <= 2 && wgs > 512) GDK(1, 4);
+    else if (a.max_blocks > 4 && wgs <= (D <= 64 ? 512 : 256)) GDK(8, 2);
+    else GDK(4, 2);
+  }
+#undef GDK
+  return CFC_CHECK_LAUNCH();
+}
+
 constexpr int prompt_waves(int D) { return D == 64 || D == 128 ? 8 : 4; }
 
 }  // namespace
@@ -733,7 +789,7 @@ CFC_API int cfc_gqa_attention(int kind, int f32, const void* q, const void* kc, 
   og.vec = DV % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out & (4 * esz - 1)) == 0 &&
            (!gate || (gate_ld % 4 == 0 && gate_plane % 4 == 0 && ((uintptr_t)gate & (4 * gsz - 1)) == 0));
   const float h = 0.5f * LN2, h2 = h * h, h3 = h2 * h;
-  const GqaArgs a{block_tables, cu_q, ctx_lens, tile_seq, tile_m0, n_tiles, H, G, D, DV, max_blocks, P, size, keep, pool, le,
+  const GqaArgs a{block_tables, cu_q, ctx_lens, tile_seq, tile_m0, n_tiles, H, G, D, DV, max_blocks, P, H / G, (H / G + 15) / 16, size, keep, pool, le,
                   chunk, capped, cap2, h * cap2, -h3 / 3.f * cap2, 2.f * h3 * h2 / 15.f * cap2, -17.f * h3 * h2 * h2 / 315.f * cap2,
                   bias, nb, og, sink, part_o, part_ml};
   const bool shaped = capped || bias;
@@ -750,15 +806,10 @@ CFC_API int cfc_gqa_attention(int kind, int f32, const void* q, const void* kc, 
   }
   if (kind == 1) {
     const dim3 grid(B * G * ((H / G + 15) / 16), P);
-#define GD(DD)                                                                                                            \
-  case DD:                                                                                                                \
-    if (shaped)                                                                                                           \
-      gqa_decode_kernel<DD, true><<<grid, 256, 0, stream>>>((const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, \
-                                                            (const uint16_t*)pk, (const uint16_t*)pv, a, (uint16_t*)out); \
-    else                                                                                                                  \
-      gqa_decode_kernel<DD, false><<<grid, 256, 0, stream>>>((const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, \
-                                                             (const uint16_t*)pk, (const uint16_t*)pv, a, (uint16_t*)out); \
-    rc = CFC_CHECK_LAUNCH();                                                                                              \
+#define GD(DD)                                                                          \
+  case DD:                                                                              \
+    rc = shaped ? decode_go<DD, true>(grid, stream, q, kc, vc, pk, pv, a, out)          \
+                : decode_go<DD, false>(grid, stream, q, kc, vc, pk, pv, a, out);        \
     break
     switch (D) { GD(32); GD(64); GD(96); GD(128); GD(160); GD(192); GD(256); }
 #undef GD

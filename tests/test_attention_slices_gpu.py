@@ -138,7 +138,7 @@ def _keys_values(kc, vc, table, n):
 @pytest.mark.parametrize("B,kv,P", [(24, 8, 1), (40, 8, 1), (40, 8, 3), (70, 8, 1), (9, 1, 5)])
 @pytest.mark.parametrize("width", [300, 1100])
 def test_keys_and_values_by_the_stream(G, B, kv, P, width):
-    """Workgroups of four, two and one wave; waves of no, one, two and three blocks, last blocks of one key; slices and whole
+    """Workgroups of eight and of four waves; waves of no, one, two and three blocks, last blocks of one key; slices and whole
     sequences; a window; shared leading blocks.  Against float64."""
     from copilot_for_consensus_amd.ops import kernels as K
     D, heads = 128, kv * G
@@ -155,6 +155,32 @@ def test_keys_and_values_by_the_stream(G, B, kv, P, width):
         got = K.paged_decode_attention(q, kc, vc, bt, lens, D ** -0.5, part_blocks=-P, window=window, shared_blocks=shared)
         for s in range(0, B, 3):
             k, v = _keys_values(kc, vc, bt[s], ctx[s])
+            lo = max(0, ctx[s] - window) if window else 0
+            p = torch.softmax(q[s].double().view(kv, G, D) @ k[:, lo:].transpose(1, 2).contiguous() * D ** -0.5, -1)
+            _close(got[s].view(kv, G, D), p @ v[:, lo:], (p @ v[:, lo:].abs()).max())
+
+
+@pytest.mark.parametrize("G", [1, 4, 16])
+@pytest.mark.parametrize("B,kv,first,others", [(40, 8, 64, 33), (70, 8, 33, 64), (2, 2, 16900, 70), (40, 8, 8500, 60)])
+def test_stream_of_two_blocks_and_of_many(G, B, kv, first, others):
+    """A wave for tables of two blocks; more blocks a wave than its lanes hold, of eight waves and of four.  Against float64."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    D, ctx = 128, [first] + [others] * (B - 1)
+    g = torch.Generator(device=DEV).manual_seed(G + first)
+    width = -(-max(ctx) // 32)
+    need = [-(-n // 32) for n in ctx]
+    order = torch.randperm(sum(need) + 1, device=DEV, generator=g).int()
+    bt = order[-1].repeat(B, width)                     # past a sequence: a block of no one's
+    for s, m in enumerate(need):
+        bt[s, :m] = order[sum(need[:s]):sum(need[:s]) + m]
+    kc = torch.randn(len(order), kv, 32, D, device=DEV, generator=g).bfloat16()
+    vc = torch.randn(len(order), kv, D, 32, device=DEV, generator=g).bfloat16()
+    q = torch.randn(B, kv * G, D, device=DEV, generator=g).bfloat16()
+    lens = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    for P, window in ((1, 0), (1, 50), (2, 0)):
+        got = K.paged_decode_attention(q, kc, vc, bt, lens, D ** -0.5, part_blocks=-P, window=window)
+        for s in (0, 1, B - 1):
+            k, v = _keys_values(kc, vc, bt[s, :need[s]], ctx[s])
             lo = max(0, ctx[s] - window) if window else 0
             p = torch.softmax(q[s].double().view(kv, G, D) @ k[:, lo:].transpose(1, 2).contiguous() * D ** -0.5, -1)
             _close(got[s].view(kv, G, D), p @ v[:, lo:], (p @ v[:, lo:].abs()).max())
