@@ -38,11 +38,12 @@ __device__ __forceinline__ Vec<V> ldgain(const Gain& g, int c) {
   return r;
 }
 
-// FEW: FEW_ROWS at most, of one vector a thread; more rows keep to 64 VGPRs, two workgroups of 1024 a CU
+// ROWS: FEW_ROWS at most, of one vector a thread, or past the caches; more rows than few keep to 64 VGPRs, two workgroups of 1024 a CU
 // (3222 rows of 4096: 58 us in 95 VGPRs, 42 in 64)
-template <typename ACT, int V, int NV, int BT, bool FEW>
+template <typename ACT, int V, int NV, int BT, int ROWS>
 __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch, float* __restrict__ x, Gain next,
                                                         ACT* __restrict__ h) {
+  constexpr bool FEW = ROWS == ROWS_FEW, NT = ROWS == ROWS_PAST;
   __shared__ float red[16], red2[16];
   const int t = blockIdx.x, W = b.W;
   const size_t row = (size_t)t * W;
@@ -51,7 +52,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int c = (k * BT + threadIdx.x) * V;
-    xv[k] = c < W ? ldv<V>(x + row + c) : zerov<V>();
+    xv[k] = c < W ? ldv<V, NT>(x + row + c) : zerov<V>();
   }
   // One vector a thread: the weights are asked for with the row, and not each after the sum before it (32 rows of 4096: 6.7 -> 5.9 us).
   constexpr bool AHEAD = FEW;
@@ -79,7 +80,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
         const int c = (k * BT + threadIdx.x) * V;
         y[k] = z[k] = zerov<V>();
         if (c >= W) continue;
-        Slabs<V, F, NV == 1> sy, sz;
+        Slabs<V, F, NV == 1, NT> sy, sz;
         sy.ask(b.y, b.ysplit, (int64_t)b.T * W, row + c);
         sz.ask(b.y2, b.y2split, (int64_t)b.T * W, row + c);
         sy.add(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
@@ -111,7 +112,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
         const int c = (k * BT + threadIdx.x) * V;
         y[k] = zerov<V>();
         if (c >= W) continue;
-        if (b.y) sum_slabs<V, 8, FEW>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
+        if (b.y) sum_slabs<V, 8, FEW, NT>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
         if (b.mrow)
           for (int i0 = 0; i0 < b.top; i0 += 4) {         // four choices in flight (past the last: weight 0)
             Vec<V> r[4];
@@ -154,7 +155,7 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
       const Vec<V> g = AHEAD ? ahead[2 * AHEAD] : ldgain<V>(b.g, c);
 #pragma unroll
       for (int e = 0; e < V; ++e) xv[k].v[e] += y[k].v[e] * r * g.v[e];
-      stv<V>(x + row + c, xv[k]);
+      stv<V, NT>(x + row + c, xv[k]);
     }
   }
   if (!h) return;
@@ -179,13 +180,17 @@ __global__ void __launch_bounds__(BT) branch_norm_kernel(BranchIn b, int branch,
 template <typename ACT, int V>
 int branch_go(hipStream_t s, const BranchIn& b, int branch, float* x, Gain next, void* h) {
   const int vecs = (b.W + V - 1) / V;
-#define GO(NV, BT)                                                                                            \
-  do {                                                                                                        \
-    if (NV == 1 && b.T <= FEW_ROWS) branch_norm_kernel<ACT, V, NV, BT, NV == 1><<<b.T, BT, 0, s>>>(b, branch, x, next, (ACT*)h); \
-    else branch_norm_kernel<ACT, V, NV, BT, false><<<b.T, BT, 0, s>>>(b, branch, x, next, (ACT*)h);           \
+  constexpr bool PAST = V == 4;       // 14 000 rows of 4096 160 -> 154 us, 4800 55.4 -> 54.5, 2400 the same
+#define BN_GO(NV, BT, ROWS) branch_norm_kernel<ACT, V, NV, BT, ROWS><<<b.T, BT, 0, s>>>(b, branch, x, next, (ACT*)h)
+#define GO(NV, BT)                                                                                                   \
+  do {                                                                                                               \
+    if (NV == 1 && b.T <= FEW_ROWS) BN_GO(NV, BT, (NV == 1 ? ROWS_FEW : ROWS_SOME));                                 \
+    else if (PAST && 4ll * b.T * b.W > PAST_BYTES) BN_GO(NV, BT, (PAST ? ROWS_PAST : ROWS_SOME));                    \
+    else BN_GO(NV, BT, ROWS_SOME);                                                                                   \
   } while (0)
   ROW_SHAPES(GO, vecs);
 #undef GO
+#undef BN_GO
   return CFC_CHECK_LAUNCH();
 }
 

@@ -106,12 +106,13 @@ struct BranchArgs {
 // MODE 0: prompt rows; 1: decoded rows (shift_mix of the next layer follows); 2: decoded rows, shift only
 // (b.y == null, b.y2 == null, b.ym == null: no branch, the first layer's).  x is updated in place.
 enum { GN_PROMPT = 0, GN_SHIFT = 1 };
-// FEW: FEW_ROWS at most, of one vector a thread.
-template <typename ACT, int V, int NV, int BT, int MODE, bool FEW>
+// ROWS: FEW_ROWS at most, of one vector a thread; prompt rows past the caches.
+template <typename ACT, int V, int NV, int BT, int MODE, int ROWS>
 __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __restrict__ x, ACT* __restrict__ h,
                                                        float* __restrict__ prev, const int32_t* __restrict__ meta,
                                                        const int32_t* __restrict__ positions, ShiftArgs a,
                                                        const int32_t* __restrict__ slots, ACT* __restrict__ acts) {
+  constexpr bool FEW = ROWS == ROWS_FEW, NT = ROWS == ROWS_PAST;
   __shared__ float red[16];
   const int t = blockIdx.x, W = b.W;
   const size_t row = (size_t)t * W;
@@ -129,7 +130,7 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
   for (int k = 0; k < NV; ++k) {          // asked for ahead of the branch they wait for
     const int c = (k * BT + threadIdx.x) * V;
     if (c >= W) continue;
-    xv[k] = ldv<V>(x + row + c);
+    xv[k] = ldv<V, NT>(x + row + c);
     if constexpr (MODE == GN_SHIFT) {
       xp[k] = xpp[k] = zerov<V>();
       if (acts && pos >= 1) xp[k] = ldv<V>(st + (size_t)((pos - 1) & 1) * W + c);
@@ -158,10 +159,10 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
       y[k] = zerov<V>();
       if (c >= W) continue;
       Vec<V> g = zerov<V>();
-      auto gate = [&] { g = ldv<V>(reinterpret_cast<const ACT*>(b.gate) + (size_t)t * b.gld + c); };
+      auto gate = [&] { g = ldv<V, NT>(reinterpret_cast<const ACT*>(b.gate) + (size_t)t * b.gld + c); };
       if (NV <= 4 && b.gate_act) gate();          // ahead of the sums, where there are registers for it
-      if (b.y) sum_slabs<V, 8, FEW>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
-      if (b.y2) sum_slabs<V, 8, FEW>(y[k], b.y2, b.y2split, (int64_t)b.T * W, row + c);
+      if (b.y) sum_slabs<V, 8, FEW, NT>(y[k], b.y, b.ysplit, (int64_t)b.T * W, row + c);
+      if (b.y2) sum_slabs<V, 8, FEW, NT>(y[k], b.y2, b.y2split, (int64_t)b.T * W, row + c);
       if (b.ym)
         for (int i = 0; i < b.top; ++i) {
           const float wt = b.mwt[(size_t)t * b.top + i];
@@ -170,7 +171,7 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
           for (int e = 0; e < V; ++e) y[k].v[e] += wt * r.v[e];
         }
       if (NV > 4 && b.gate_act) gate();
-      if (!b.gate_act) sum_slabs<V, 8, FEW>(g, reinterpret_cast<const float*>(b.gate), b.gsplit, b.gplane, (size_t)t * b.gld + c);
+      if (!b.gate_act) sum_slabs<V, 8, FEW, NT>(g, reinterpret_cast<const float*>(b.gate), b.gsplit, b.gplane, (size_t)t * b.gld + c);
       const Vec<V> gb = FEW ? gb1 : ldv<V>(b.gbias + c);
 #pragma unroll
       for (int e = 0; e < V; ++e) {
@@ -199,7 +200,7 @@ __global__ void __launch_bounds__(BT) gated_norm_kernel(BranchArgs b, float* __r
       const Vec<V> w = FEW ? gain : ldv<V>(b.norm_w + c);
 #pragma unroll
       for (int e = 0; e < V; ++e) xv[k].v[e] += y[k].v[e] * r * w.v[e];
-      stv<V>(x + row + c, xv[k]);
+      stv<V, NT>(x + row + c, xv[k]);
       if (h) stv<V>(h + row + c, xv[k]);
     }
   }
@@ -256,12 +257,14 @@ template <typename ACT, int V, int MODE>
 int gated_go(hipStream_t s, int n, const BranchArgs& b, float* x, void* h, float* prev, const int32_t* meta,
              const int32_t* positions, const ShiftArgs& a, const int32_t* slots, void* acts) {
   const int vecs = (b.W + V - 1) / V;
-#define GN_GO(NV, BT, FEW) \
-  gated_norm_kernel<ACT, V, NV, BT, MODE, FEW><<<n, BT, 0, s>>>(b, x, (ACT*)h, prev, meta, positions, a, slots, (ACT*)acts)
-#define GO(NV, BT)                                               \
-  do {                                                           \
-    if (NV == 1 && n <= FEW_ROWS) GN_GO(NV, BT, NV == 1);        \
-    else GN_GO(NV, BT, false);                                   \
+  constexpr bool PAST = MODE == GN_PROMPT && V == 4;       // 16 100 rows of 4096 220 -> 213 us, 9600 133 -> 125, 4800 65.6 -> 64.0, 1200 the same
+#define GN_GO(NV, BT, ROWS) \
+  gated_norm_kernel<ACT, V, NV, BT, MODE, ROWS><<<n, BT, 0, s>>>(b, x, (ACT*)h, prev, meta, positions, a, slots, (ACT*)acts)
+#define GO(NV, BT)                                                                                                   \
+  do {                                                                                                               \
+    if (NV == 1 && n <= FEW_ROWS) GN_GO(NV, BT, (NV == 1 ? ROWS_FEW : ROWS_SOME));                                  \
+    else if (PAST && 4ll * n * b.W > PAST_BYTES) GN_GO(NV, BT, (PAST ? ROWS_PAST : ROWS_SOME));                      \
+    else GN_GO(NV, BT, ROWS_SOME);                                                                                 \
   } while (0)
   ROW_SHAPES(GO, vecs);
 #undef GO

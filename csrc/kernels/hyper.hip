@@ -30,16 +30,18 @@ struct HyperArgs {
   float* tail; int ring;       // [slots][ring][W], position p at p % ring
 };
 
-// SM >= S copies in registers; a thread holds NV vectors of V channels
-template <typename ACT, int V, int SM, int NV, int BT>
+// SM >= S copies in registers; a thread holds NV vectors of V channels.  ROWS: FEW_ROWS at most, all that a row needs asked for
+// ahead (90 VGPRs), or more: two workgroups of 1024 a CU (46; 2400 rows of 4096 in 4 streams 63.9 -> 58.5 us), or past the caches
+template <typename ACT, int V, int SM, int NV, int BT, int ROWS>
 __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, ACT* __restrict__ h) {
+  constexpr bool NT = ROWS == ROWS_PAST;
   __shared__ float red[16];
   __shared__ float mx[SM * SM + 2 * SM];       // mix [from][to], out, in
   const int b = blockIdx.x, t = a.rows ? a.rows[b] : b, W = a.W, S = a.S;
   const float* xr = a.x + t * a.ldx;
   // All that a row's first vectors need is asked for before anything is waited for, what waits for an index last (5 rows of
   // 4096 in 4 streams: 6.9 -> 6.2 us, of which 300 KB a row through one CU take most).
-  constexpr bool ONE = NV == 1 && SM <= 4;     // else the registers are wanted for more vectors or streams
+  constexpr bool ONE = NV == 1 && SM <= 4 && ROWS == ROWS_FEW;     // else the registers are wanted for more vectors or streams
   constexpr int MX = SM * SM + 2 * SM;
   static_assert(!ONE || MX <= BT, "");
   float mv = 0.f;
@@ -55,24 +57,24 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
   } else {
     for (int i = threadIdx.x; i < MX; i += BT) mx[i] = weight(i);
   }
-  constexpr int PRE = NV == 1 && V == 4 ? 3 : 0;
+  constexpr int PRE = NV == 1 && V == 4 && ROWS == ROWS_FEW ? 3 : 0;
   const int back = a.taps - 1;
   const bool ahead = PRE > 0 && back <= PRE;
   const int c0 = min((int)threadIdx.x * V, W - V);
   Vec<V> u[NV], x[SM], y = zerov<V>(), past[PRE ? PRE : 1], cw[PRE ? PRE + 1 : 1], gain;
-  Slabs<V, 8, ONE> slabs;
+  Slabs<V, (ROWS == ROWS_FEW || NV > 1 || SM > 4 ? 8 : 4), ONE, NT> slabs;
   float ss = 0.f;
   auto ask = [&](int c) {
 #pragma unroll
-    for (int s = 0; s < SM; ++s) x[s] = ldv<V>(xr + min(s, S - 1) * a.lds + c);
+    for (int s = 0; s < SM; ++s) x[s] = ldv<V, NT>(xr + min(s, S - 1) * a.lds + c);
     if (!a.y) return;
     y = zerov<V>();
     slabs.ask(a.y, a.split, (int64_t)a.T * W, (size_t)t * W + c);
     if constexpr (!ONE) slabs.add(y, a.y, a.split, (int64_t)a.T * W, (size_t)t * W + c);
   };
   if constexpr (ONE) ask(c0);
+  if (NV == 1 && V == 4 && SM <= 4 && mode != HN_RSTD) gain = ldv<V>(a.w + c0);
   if constexpr (PRE > 0) {
-    if (ONE && mode != HN_RSTD) gain = ldv<V>(a.w + c0);
     if (mode == HN_CONV && ahead)
 #pragma unroll
       for (int d = 0; d <= PRE; ++d) cw[d] = ldv<V>(a.cw + (size_t)max(back - d, 0) * W + c0);
@@ -104,7 +106,7 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
         for (int s = 0; s < SM; ++s)
 #pragma unroll
           for (int e = 0; e < V; ++e) n.v[e] += mx[s * SM + q] * x[s].v[e];
-        if (a.x_out) stv<V>(a.x_out + ((size_t)t * S + q) * W + c, n);
+        if (a.x_out) stv<V, NT>(a.x_out + ((size_t)t * S + q) * W + c, n);
 #pragma unroll
         for (int e = 0; e < V; ++e) u[k].v[e] += mx[SM * SM + SM + q] * n.v[e];
       }
@@ -132,7 +134,7 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
     const int c = (k * BT + threadIdx.x) * V;
     if (c >= W) continue;
     Vec<V> g, n;
-    if constexpr (PRE > 0 && ONE) g = gain;
+    if constexpr (NV == 1 && V == 4 && SM <= 4) g = gain;
     else g = ldv<V>(a.w + c);
 #pragma unroll
     for (int e = 0; e < V; ++e) n.v[e] = u[k].v[e] * r * g.v[e];
@@ -165,7 +167,16 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
 template <typename ACT, int V, int SM>
 int hyper_go(hipStream_t s, int n, const HyperArgs& a, int mode, void* h) {
   const int vecs = (a.W + V - 1) / V;
-#define GO(NV, BT) hyper_norm_kernel<ACT, V, SM, NV, BT><<<n, BT, 0, s>>>(a, mode, (ACT*)h)
+  // past the caches: several streams stay there longer.  us of 4 x 4096 to fp32 and to bf16 rows, before, two workgroups a CU, and past the
+  // caches: 14 000 rows 342, 336, 307 and 352, 347, 333; 4800 rows 105, 103, 104 and 115, 109, 118
+#define HN_GO(NV, BT, ROWS) hyper_norm_kernel<ACT, V, SM, NV, BT, ROWS><<<n, BT, 0, s>>>(a, mode, (ACT*)h)
+#define GO(NV, BT)                                                                                                   \
+  do {                                                                                                               \
+    constexpr bool one = V == 4 && NV == 1, past = V == 4 && SM <= 4 && NV <= 4;                                     \
+    if (one && (SM > 4 || n <= FEW_ROWS)) HN_GO(NV, BT, (one ? ROWS_FEW : ROWS_SOME));                               \
+    else if (past && 4ll * n * a.S * a.W > 8 * PAST_BYTES) HN_GO(NV, BT, (past ? ROWS_PAST : ROWS_SOME));            \
+    else HN_GO(NV, BT, ROWS_SOME);                                                                                   \
+  } while (0)
   if (vecs <= 64) GO(1, 64);
   else if (vecs <= 256) GO(1, 256);
   else if (vecs <= 512) GO(1, 512);
@@ -174,6 +185,7 @@ int hyper_go(hipStream_t s, int n, const HyperArgs& a, int mode, void* h) {
   else if (vecs <= 16384) GO(16, 1024);
   else return -4;
 #undef GO
+#undef HN_GO
   return CFC_CHECK_LAUNCH();
 }
 

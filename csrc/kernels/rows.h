@@ -10,22 +10,35 @@ __device__ __forceinline__ float ld1(const float* p) { return *p; }
 
 template <int V> struct Vec { float v[V]; };
 
-template <int V>
+// NT: past the caches (nontemporal), as far as vectors of four go
+typedef float row_f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t row_u2 __attribute__((ext_vector_type(2)));
+template <bool NT, typename T>
+__device__ __forceinline__ T row_ld(const void* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const T*>(p));
+  else return *reinterpret_cast<const T*>(p);
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void row_st(void* p, T v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<T*>(p));
+  else *reinterpret_cast<T*>(p) = v;
+}
+template <int V, bool NT = false>
 __device__ __forceinline__ Vec<V> ldv(const float* p) {
   Vec<V> r;
   if constexpr (V == 4) {
-    const float4 f = *reinterpret_cast<const float4*>(p);
+    const row_f4 f = row_ld<NT, row_f4>(p);
     r.v[0] = f.x; r.v[1] = f.y; r.v[2] = f.z; r.v[3] = f.w;
   } else {
     r.v[0] = *p;
   }
   return r;
 }
-template <int V>
+template <int V, bool NT = false>
 __device__ __forceinline__ Vec<V> ldv(const uint16_t* p) {
   Vec<V> r;
   if constexpr (V == 4) {
-    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    const row_u2 u = row_ld<NT, row_u2>(p);
     r.v[0] = __uint_as_float(u.x << 16); r.v[1] = __uint_as_float(u.x & 0xffff0000u);
     r.v[2] = __uint_as_float(u.y << 16); r.v[3] = __uint_as_float(u.y & 0xffff0000u);
   } else {
@@ -33,14 +46,14 @@ __device__ __forceinline__ Vec<V> ldv(const uint16_t* p) {
   }
   return r;
 }
-template <int V>
+template <int V, bool NT = false>
 __device__ __forceinline__ void stv(float* p, const Vec<V>& r) {
-  if constexpr (V == 4) *reinterpret_cast<float4*>(p) = make_float4(r.v[0], r.v[1], r.v[2], r.v[3]);
+  if constexpr (V == 4) row_st<NT>(p, row_f4{r.v[0], r.v[1], r.v[2], r.v[3]});
   else *p = r.v[0];
 }
-template <int V>
+template <int V, bool NT = false>
 __device__ __forceinline__ void stv(uint16_t* p, const Vec<V>& r) {
-  if constexpr (V == 4) *reinterpret_cast<uint2*>(p) = make_uint2(pack2bf(r.v[0], r.v[1]), pack2bf(r.v[2], r.v[3]));
+  if constexpr (V == 4) row_st<NT>(p, row_u2{pack2bf(r.v[0], r.v[1]), pack2bf(r.v[2], r.v[3])});
   else *p = f2bf(r.v[0]);
 }
 template <int V>
@@ -52,10 +65,10 @@ __device__ __forceinline__ Vec<V> zerov() {
 }
 
 // y += slabs of row offset `off`, F in flight (past the last: re-read, not added)
-template <int V, int F = 8>
+template <int V, int F = 8, bool NT = false>
 __device__ __forceinline__ void add_slabs(Vec<V>& y, const float* p, int split, int64_t plane, size_t off, int first = 0) {
   if (split == 1) {
-    const Vec<V> a = ldv<V>(p + off);
+    const Vec<V> a = ldv<V, NT>(p + off);
 #pragma unroll
     for (int e = 0; e < V; ++e) y.v[e] += a.v[e];
     return;
@@ -63,7 +76,7 @@ __device__ __forceinline__ void add_slabs(Vec<V>& y, const float* p, int split, 
   for (int p0 = first; p0 < split; p0 += F) {
     Vec<V> a[F];
 #pragma unroll
-    for (int u = 0; u < F; ++u) a[u] = ldv<V>(p + (size_t)min(p0 + u, split - 1) * plane + off);
+    for (int u = 0; u < F; ++u) a[u] = ldv<V, NT>(p + (size_t)min(p0 + u, split - 1) * plane + off);
 #pragma unroll
     for (int u = 0; u < F; ++u)
       if (p0 + u < split)
@@ -76,15 +89,15 @@ __device__ __forceinline__ void add_slabs(Vec<V>& y, const float* p, int split, 
 // for another: a loop over the slabs made all that was asked for before it arrive first, and a row that one workgroup works
 // on pays a trip to memory, 0.7 us, for each such wait.  Only where a thread has one vector (AHEAD): rows of more want their
 // registers for these, and asking ahead was slower (5 rows of 8192 gated 6.5 -> 8.5 us, of 20480 34 -> 43).
-template <int V, int F = 8, bool AHEAD = true>
+template <int V, int F = 8, bool AHEAD = true, bool NT = false>
 struct Slabs {
   Vec<V> a[AHEAD ? F : 1];
   __device__ __forceinline__ void ask(const float* p, int split, int64_t plane, size_t off) {
     if constexpr (AHEAD) {
-      a[0] = ldv<V>(p + off);
+      a[0] = ldv<V, NT>(p + off);
       if (split == 1) return;
 #pragma unroll
-      for (int u = 1; u < F; ++u) a[u] = u < split ? ldv<V>(p + u * plane + off) : zerov<V>();
+      for (int u = 1; u < F; ++u) a[u] = u < split ? ldv<V, NT>(p + u * plane + off) : zerov<V>();
     }
   }
   __device__ __forceinline__ void add(Vec<V>& y, const float* p, int split, int64_t plane, size_t off) const {
@@ -97,17 +110,17 @@ struct Slabs {
         if (u < split)
 #pragma unroll
           for (int e = 0; e < V; ++e) y.v[e] += a[u].v[e];
-      add_slabs<V, F>(y, p, split, plane, off, F);
+      add_slabs<V, F, NT>(y, p, split, plane, off, F);
     } else {
-      add_slabs<V, F>(y, p, split, plane, off);
+      add_slabs<V, F, NT>(y, p, split, plane, off);
     }
   }
 };
 
 // both steps at once
-template <int V, int F, bool AHEAD>
+template <int V, int F, bool AHEAD, bool NT = false>
 __device__ __forceinline__ void sum_slabs(Vec<V>& y, const float* p, int split, int64_t plane, size_t off) {
-  Slabs<V, F, AHEAD> s;
+  Slabs<V, F, AHEAD, NT> s;
   s.ask(p, split, plane, off);
   s.add(y, p, split, plane, off);
 }
@@ -137,6 +150,11 @@ struct ColsIn {
 
 // Up to so many rows, no more than there are CUs, a row's time is its trips to memory; of more, what the registers let a CU hold.
 constexpr int FEW_ROWS = 256;
+
+// What a kernel keeps in mind of its number of rows: ROWS_FEW, and ROWS_PAST of so many that their stream no longer waits in the
+// caches (256 MB) for its next use: it is read and written past them, and what others read next is not pushed out.
+enum { ROWS_SOME = 0, ROWS_FEW = 1, ROWS_PAST = 2 };
+constexpr int64_t PAST_BYTES = 64ll << 20;      // of one stream
 
 // NV, BT for rows of W channels in vectors of V
 #define ROW_SHAPES(GO, vecs)           \
