@@ -90,6 +90,15 @@ class Projection:
             return K.splitk_reduce(K.gemv_part(x, self.packed))
         return K.dgemm_linear(x, self.packed)
 
+    def few_slabs(self, x: torch.Tensor) -> torch.Tensor | None:
+        """The slabs that :meth:`act` would sum for a decode step's rows (None: it sums none), to be consumed before the next product."""
+        k = self._kernel(x)
+        if k == "gemv":
+            return K.gemv_part(x, self.packed)
+        if k == "dgemm" and x.is_cuda and K.dgemm_config(x.shape[0], self.N, self.K, bn=self.packed.bn)[1] > 1:
+            return K.dgemm_slabs(x, self.packed)
+        return None
+
     def slabs(self, x: torch.Tensor, own: bool = False) -> torch.Tensor:
         """fp32 k-slice slabs [split, M, N] whose sum is the product (unrounded).  They may live in the
         stream's split-K workspace: consume them before the next product, unless they are to be a tensor of

@@ -435,7 +435,9 @@ class VofosunModel:
         T, dt, dev = hs[0].shape[0], self.w.dtype, hs[0].device
         cq = L.latent_norm(lw["down_in"].slabs(hs[0]), m.q_rank, lw["dq_norm"], lw["dkv_norm"], self.cfg.norm_eps, slots,
                            kv.latents[i], dt)
-        q = lw["uq"].act(cq).view(T, H, m.dim)
+        # a decode step's queries: what their product leaves is summed by the per-head product after it
+        part = lw["uq"].few_slabs(cq) if dense is None and cq.is_cuda and L.slabs_fit(T, lw["uk"]) else None
+        q = lw["uq"].act(cq).view(T, H, m.dim) if part is None else None
         F = spec.mlp.ff // self.w.tp_size if spec.mlp is not None else 0
         cat = torch.empty(T, H * m.vdim + F, dtype=dt, device=dev)
         o = cat[:, :H * m.vdim].unflatten(1, (H, m.vdim))
@@ -443,7 +445,8 @@ class VofosunModel:
             k, vt = L.expand(kv.latents[i], block_tables, ctx_lens, dense["gather"], lw["uk_full"], lw["uv_full"])
             L.expanded_attention(q, k, vt, dense["tok_base"], attn["cu_q"], ctx_lens, m.scale, dense["pf_tiles"], o)
         else:
-            ql = L.head_linear(q, lw["uk"], torch.empty(T, H, self._rs(i), dtype=dt, device=dev))
+            ql = torch.empty(T, H, self._rs(i), dtype=dt, device=dev)
+            ql = L.head_linear(q, lw["uk"], ql) if part is None else L.head_linear_slabs(part, lw["uk"], ql)
             ol = L.latent_attention(ql, kv.latents[i], block_tables, ctx_lens=ctx_lens, scale=m.scale, **attn)
             L.head_linear(ol, lw["uv"], o)
         if F:

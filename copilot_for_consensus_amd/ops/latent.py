@@ -20,6 +20,7 @@ from .stream import _act
 MFMA_MAX_RANK = 512       # latent ranks the MFMA attention kernel is built for
 MFMA_MAX_KEY = 576        # and key columns (the latent and what follows it in the row)
 ANY_ROWS = 4              # rows per tile of the general kernel
+SLAB_ROWS, SLAB_COLS = 64, 256      # of head_linear_slabs
 
 
 def padded_rank(rank: int) -> int:
@@ -64,6 +65,24 @@ def head_linear(x: torch.Tensor, w: HeadWeight, out: torch.Tensor, gate: torch.T
                                     out.stride(1), _p(gate), gate.stride(0) if gate is not None else 0, _stream(x)),
           "cfc_head_linear")
     return out
+
+
+def head_linear_slabs(part: torch.Tensor, w: HeadWeight, out: torch.Tensor) -> torch.Tensor:
+    """:func:`head_linear` of the bf16 sum of ``part``, fp32 slabs [split, T, H K], of SLAB_ROWS tokens at most; bf16 out [T, H,
+    >= N]."""
+    split, T, cols = part.shape
+    if not (part.is_cuda and slabs_fit(T, w) and cols == w.H * w.K and part.is_contiguous() and out.stride(2) == 1
+            and out.shape[:2] == (T, w.H) and out.shape[2] >= w.N and out.dtype == w.data.dtype):
+        raise ValueError(f"head_linear_slabs: {tuple(part.shape)} w {w.H} x {w.N} x {w.K} out {tuple(out.shape)} {out.dtype}")
+    _req(part, torch.float32, "part")
+    check(kernels().cfc_head_linear_slabs(part.data_ptr(), split, T * cols, cols, w.data.data_ptr(), w.data.shape[1], w.data.shape[2], T,
+                                          w.H, w.N, w.K, out.data_ptr(), out.stride(0), out.stride(1), _stream(part)),
+          "cfc_head_linear_slabs")
+    return out
+
+
+def slabs_fit(T: int, w: HeadWeight) -> bool:
+    return 1 <= T <= SLAB_ROWS and w.data.dtype == torch.bfloat16 and w.data.shape[2] <= SLAB_COLS and w.K % 4 == 0 and w.N % 4 == 0
 
 
 def latent_norm(part, nq: int, wq, wc, eps: float, slots, cache, dtype) -> torch.Tensor:

@@ -8,7 +8,8 @@
 //                     joint down projection; the latter goes straight into the cache slot
 //   * latent_rope     the same for designs with rotary positions: the normed latent and, behind it in the
 //                     row, the rotated key part all heads share; the heads' rotated query parts
-//   * head_linear     out[t][h] = W[h] in[t][h], the per-head products on both sides of the attention
+//   * head_linear     out[t][h] = W[h] in[t][h], the per-head products on both sides of the attention; of few tokens
+//                     from the fp32 slabs of the product before
 //   * latent_attn     flash-style attention over the paged latents.  A work item is 16 MR rows of the
 //                     flattened (token, head) rows of one sequence -- one decoded token's heads and a
 //                     prompt portion's rows are the same thing to it -- and a slice of its keys
@@ -438,6 +439,68 @@ __global__ void __launch_bounds__(256) head_linear_ks_kernel(const uint16_t* __r
       if (gate) gate4(v, gate + (int64_t)t * ldg + (size_t)h * N + n);
       *reinterpret_cast<uint2*>(out + (int64_t)t * ldo + h * hso + n) = make_uint2(pack2bf(v[0], v[1]), pack2bf(v[2], v[3]));
     }
+  }
+}
+
+// Few tokens, x the sum of a product's slabs [split][T][ldx], head h's K columns at h K: a workgroup sums its head's rows to bf16 in
+// LDS (as splitk_reduce, in its order) beside its weights' loads, and the four waves take 16 outputs each.  In place of a launch
+// for the sum and one for the product: 24 tokens of 32 heads, 128 -> 512, 4.8 and 4.9 us -> 6.0.
+constexpr int HS_K = 256;      // columns at most
+template <int TT>
+__global__ void __launch_bounds__(256) head_linear_slabs_kernel(const float* __restrict__ part, int split, int64_t plane, int64_t ldx,
+                                                               const uint16_t* __restrict__ w, int NP, int KP, int T, int N, int K,
+                                                               uint16_t* __restrict__ out, int64_t ldo, int64_t hso) {
+  constexpr int ROWS = 16 * TT, LD = HS_K + 8, AHEAD = 4;
+  __shared__ __attribute__((aligned(16))) uint16_t xs[ROWS][LD];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, col = lane & 15, kq = lane >> 4;
+  const int h = blockIdx.z, t0 = blockIdx.x * ROWS, n0 = (blockIdx.y * 4 + wv) * 16;
+  const uint16_t* wp = w + ((size_t)h * NP + n0 + col) * KP + 8 * kq;
+  const int ks = KP / 32;
+  uint4 a[HS_K / 32];
+#pragma unroll
+  for (int k = 0; k < HS_K / 32; ++k) a[k] = *reinterpret_cast<const uint4*>(wp + 32 * min(k, ks - 1));
+  const int q4 = KP / 4, total = min(ROWS, T - t0) * q4;
+  for (int e0 = tid; e0 < total; e0 += 256 * AHEAD) {      // AHEAD fours of columns at once, four slabs of each
+    Vec<4> s[AHEAD];
+    size_t at[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int e = min(e0 + 256 * u, total - 1);
+      s[u] = zerov<4>();
+      at[u] = (size_t)(t0 + e / q4) * ldx + (size_t)h * K + min(4 * (e % q4), K - 4);
+    }
+    for (int p0 = 0; p0 < split; p0 += 4) {
+      Vec<4> v[AHEAD][4];
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) v[u][p] = ldv<4>(part + (size_t)min(p0 + p, split - 1) * plane + at[u]);
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          if (p0 + p < split)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[u].v[i] += v[u][p].v[i];
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int e = e0 + 256 * u, c = 4 * (e % q4);
+      if (e < total) stv<4>(&xs[e / q4][c], c < K ? s[u] : zerov<4>());
+    }
+  }
+  __syncthreads();
+  if (n0 >= NP) return;
+#pragma unroll
+  for (int i = 0; i < TT; ++i) {
+    const int t = t0 + 16 * i + col;
+    f32x4_t acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < HS_K / 32; ++k)
+      if (k < ks) acc = mfma16(a[k], *reinterpret_cast<const uint4*>(&xs[min(16 * i + col, T - 1 - t0)][32 * k + 8 * kq]), acc);
+    const int n = n0 + 4 * kq;
+    if (t < T && n < N)
+      *reinterpret_cast<uint2*>(out + (int64_t)t * ldo + h * hso + n) = make_uint2(pack2bf(acc[0], acc[1]), pack2bf(acc[2], acc[3]));
   }
 }
 
@@ -1020,6 +1083,21 @@ CFC_API int cfc_head_linear(int f32, const void* x, int64_t ldx, int64_t hsx, co
   else HL(4, 2, true);
 #undef HL
 #undef HK
+  return CFC_CHECK_LAUNCH();
+}
+
+// bf16 outputs of the product's slabs [split][T][ldx], head h's K columns at h K (see head_linear_slabs_kernel)
+CFC_API int cfc_head_linear_slabs(const float* part, int split, int64_t plane, int64_t ldx, const void* w, int NP, int KP, int T, int H,
+                                  int N, int K, void* out, int64_t ldo, int64_t hso, hipStream_t stream) {
+  if (T <= 0) return 0;
+  if (H < 1 || H > 65535 || N < 1 || K < 4 || N > NP || K > KP || NP % 64 || KP % 32 || KP > HS_K || split < 1) return -1;
+  if (ldx < (int64_t)H * K || ldx % 4 || plane % 4 || K % 4 || ((uintptr_t)part & 15) || N % 4 || ldo % 4 || hso % 4 || ((uintptr_t)out & 7)) return -2;
+#define HS(TT)                                                                                                              \
+  head_linear_slabs_kernel<TT><<<dim3((T + 16 * TT - 1) / (16 * TT), NP / 64, H), 256, 0, stream>>>(part, split, plane, ldx, \
+      (const uint16_t*)w, NP, KP, T, N, K, (uint16_t*)out, ldo, hso)
+  if (T <= 16) HS(1);
+  else HS(2);
+#undef HS
   return CFC_CHECK_LAUNCH();
 }
 

@@ -346,3 +346,19 @@ def test_decode_plan_covers_every_head_and_key():
                 for ctx in (1, 64, 2848, 100000):
                     rows, P = L.decode_plan(B, H, RS, ctx)
                     assert rows in (16, 32, 64) and 1 <= P <= L.MAX_PARTITIONS and P <= max(1, -(-ctx // 64))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,N,Kd,split", [(1, 2, 64, 64, 1), (5, 3, 40, 72, 3), (16, 4, 100, 128, 4), (17, 2, 512, 128, 5), (32, 32, 512, 128, 8),
+                                            (33, 1, 192, 96, 9), (64, 2, 128, 256, 2), (24, 1, 64, 4, 16)])
+def test_head_linear_of_slabs(T, H, N, Kd, split):
+    """The same bits as the sum of the slabs and the product of it."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    part, w = rnd(split, T, H * Kd).cuda(), L.HeadWeight(rnd(H, N, Kd, seed=1).bfloat16().cuda())
+    x = K.splitk_reduce(part).view(T, H, Kd)
+    a, b = (torch.zeros(T, H * N + 16, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    L.head_linear(x, w, a[:, 16:].unflatten(1, (H, N)))
+    L.head_linear_slabs(part, w, b[:, 16:].unflatten(1, (H, N)))
+    # one difference is left: a sum of products of K in other groups, where the general product takes a part of K a wave
+    assert float((a.float() - b.float()).abs().max()) <= (0.0 if w.data.shape[2] < 256 else 2.0 ** -8 * float(a.float().abs().max()))
+    assert not b[:, :16].any()
