@@ -559,12 +559,15 @@ __global__ void __launch_bounds__(512, 1)
     if constexpr (FLIP) __builtin_amdgcn_s_setprio(1);
     if constexpr (MM) {
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int n = 0; n < 4; ++n)
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+          for (int kk = 0; kk < 2; ++kk) {
+            const int j = i & 1 ? 3 - n : n;
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][kk], xf[i][kk], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
     } else {
       keep();
     }
@@ -593,12 +596,15 @@ __global__ void __launch_bounds__(512, 1)
     if constexpr (FLIP) __builtin_amdgcn_s_setprio(1);
     if constexpr (MM) {
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int n = 0; n < 4; ++n)
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+          for (int kk = 0; kk < 2; ++kk) {
+            const int j = i & 1 ? 3 - n : n;
             acc[4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][kk], xf[i][kk], acc[4 + i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
     } else {
       keep();
     }
@@ -641,6 +647,12 @@ __global__ void __launch_bounds__(512, 1)
 //     segment B of a two-K-tile last tile); the next waits see them older than the DMA they retire,
 //     so the stores have one MFMA segment to drain;
 //   * an edge block (rows past M / columns past N) stores through pg_epilogue and drains (vmcnt(0));
+//   * an accumulator's two K steps are multiplied back to back (kept so by a sched_barrier behind each product; left alone the
+//     compiler takes them apart).  Large products are bound by energy: at 84 % of the matrix cores' cycles the clock is 1.6 GHz.
+//     A loop of nothing but these MFMAs runs at 2.02 PFLOP/s with one operand kept from product to product, at 1.97 with none,
+//     2.06 with rows walked to and fro, 2.16 with an accumulator used twice in turn (four times: the same); 32x32x16, with half
+//     the K for its accumulators' traffic, 1.67 to 1.82.  us: 15 760 x 4096 x 14336 1373 -> 1332, SwiGLU 28672 x 4096 2531 -> 2473, 4096 x
+//     4096 362 -> 349, 14 000 to fp32 358 -> 338; the same bits (four waves of 128 x 128 each, a third fewer LDS reads: no faster);
 //   * the steady K-tiles (kt + 2 < nk) run a branch-free copy of the K step; only the last two run
 //     the copy whose DMA continues into the next tile (its offsets computed there), so the loop
 //     the MFMAs wait on carries no tile-boundary logic (71 scalar instructions per K-tile, "pp" 102);
@@ -780,12 +792,15 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
       else pp_wait_barrier<0>();
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int n = 0; n < 4; ++n)
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+          for (int kk = 0; kk < 2; ++kk) {
+            const int j = i & 1 ? 3 - n : n;
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][kk], xf[i][kk], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
       __builtin_amdgcn_sched_barrier(0);
       pp_barrier();
       // ======== segment B: position kt+2's X0 / W0 / W1 (slot s0); K-tile kt's X1 fragments
@@ -817,12 +832,15 @@ __device__ __forceinline__ void ppp_tiles(char* smem, const uint16_t* __restrict
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
+      for (int i = 0; i < MB; ++i)
 #pragma unroll
-        for (int i = 0; i < MB; ++i)
+        for (int n = 0; n < 4; ++n)
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+          for (int kk = 0; kk < 2; ++kk) {
+            const int j = i & 1 ? 3 - n : n;
             acc[4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][kk], xf[i][kk], acc[4 + i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
       __builtin_amdgcn_sched_barrier(0);
       pp_barrier();
     };
