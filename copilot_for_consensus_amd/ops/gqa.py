@@ -272,7 +272,7 @@ def decode_slices(B: int, H: int, G: int, D: int, visible: int, dtype) -> int:
     most = max(1, min(math.ceil((768 if items < 384 else 1024) / items), visible // 256, MAX_PARTITIONS))
     if items >= 384 or B == 1:
         return most
-    most = max(1, min(math.ceil(768 / items), math.ceil(visible / 256)))      # (the last slice may have fewer tiles)
+    most = max(1, min(math.ceil(768 / items), math.ceil(visible / 256), MAX_PARTITIONS))      # (the last slice may have fewer tiles)
     return min(range(1, most + 1), key=lambda P: streamed_us(math.ceil(visible / 32), items, 128 * D, B * H, P))
 
 

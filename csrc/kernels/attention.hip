@@ -481,7 +481,7 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
   const int p = blockIdx.x, h = blockIdx.y;
   int b = blockIdx.z, ctx;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool whole = !(ORD && ordered) && P == 1 && window == 0;       // the table's blocks: asked for beside the length
+  const bool whole = !(ORD && ordered) && P == 1 && window == 0 && max_blocks > 0;       // the table's blocks: asked for beside the length
   const int spec = whole ? block_tables[(size_t)b * max_blocks + min(w + NWV * lane, max_blocks - 1)] : 0;
   if (ORD && ordered) {
     const int2 s = longest_first<256>(ctx_lens, gridDim.z, blockIdx.z, ordered);

@@ -17,3 +17,9 @@ def test_long_rows_of_many_items_are_sliced(visible):
         assert P == (1 if visible <= 1536 else min(math.ceil(1024 / items), visible // 256))
     assert A.decode_slices(1, 32, 8, 128, visible, torch.bfloat16) == max(1, min(96, visible // 256, A.MAX_PARTITIONS))
     assert A.decode_slices(48, 32, 8, 128, visible, torch.float32) == max(1, min(math.ceil(1024 / (48 * math.ceil(32 / A.ANY_ROWS))), visible // 256))
+
+
+@pytest.mark.parametrize("B,H,G,visible", [(2, 4, 1, 1_000_000), (2, 32, 8, 100_000), (3, 8, 1, 40_000), (47, 32, 8, 4000), (5, 32, 8, 1)])
+def test_slices_are_no_more_than_the_merge_takes(B, H, G, visible):
+    for D in (32, 128, 256):
+        assert 1 <= A.decode_slices(B, H, G, D, visible, torch.bfloat16) <= min(A.MAX_PARTITIONS, max(1, math.ceil(visible / 256)))
