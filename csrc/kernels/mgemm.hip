@@ -275,9 +275,9 @@ double prompt_best(int M, int N, int K, int kind, int* plan) {
   if (weights <= 1 << 23 && M <= (weights > 1 << 22 ? 256 : 640)) return all;       // the decode GEMM, within 10 %
   // a few rows beyond a whole round are faster here than its model says beside tiles of other heights than 256: 560 and 640
   // rows of 28672 x 4096
-  const double bias = ppp_height(M, N, K) < 8 && M > 512 ? 1.04 : 0.97;
-  double best = M < 256 ? 1e29 : bias * ppp_us(M, N, K, kind != MG_ACT);
   const int tn = (N + 255) / 256, tm = (M + 255) / 256;
+  const double bias = ppp_height(M, N, K) < 8 && M > 512 && (int64_t)tm * tn > MG_CUS ? 1.04 : 0.97;
+  double best = M < 256 ? 1e29 : bias * ppp_us(M, N, K, kind != MG_ACT);
   if ((int64_t)tm * tn >= MG_PGEMM_TILES) all = std::max(all, mgemm_x_us(M, N, K, split));
   if (all < best) best = all, plan[1] = bm, plan[2] = split;
   const int rounds = (int)((int64_t)tm * tn / MG_CUS), head = rounds ? (int)((int64_t)MG_CUS * rounds / tn) * 256 : 0;
