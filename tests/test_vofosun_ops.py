@@ -339,6 +339,29 @@ def test_expanded_keys_and_values_equal_the_latent_space():
     assert not out[:, H * 128:].any()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("RS,H,rows,P", [(64, 20, 16, 1), (192, 20, 32, 3), (512, 20, 16, 1), (512, 32, 32, 2), (512, 40, 64, 1), (512, 32, 32, 5), (576, 9, 16, 4)])
+def test_latent_slices_of_one_two_and_more_tiles(RS, H, rows, P):
+    """Contexts at the edges of 32-key blocks and 64-key tiles; blocks that no context reaches hold NaN.  A weight and a result are
+    rounded to bf16 (2^-9 each), twice that is allowed."""
+    ctx, RV, width = [1, 31, 32, 33, 64, 65, 96, 128, 129, 191, 193, 257, 320, 321], min(RS, 512), 11
+    B = len(ctx)
+    cache = torch.full((B * width, 32, RS), math.nan)
+    bt = torch.randperm(B * width, generator=torch.Generator().manual_seed(1)).view(B, width).int()
+    q, lat = rnd(B, H, RS, seed=2, scale=0.2).bfloat16(), [rnd(n, RS, seed=3 + n).bfloat16() for n in ctx]
+    for b, n in enumerate(ctx):
+        used = bt[b, :-(-n // 32)].long()
+        rows_of = torch.zeros(len(used) * 32, RS)
+        rows_of[:n] = lat[b].float()
+        cache[used] = rows_of.view(-1, 32, RS)
+    got = L.latent_attention(q.cuda(), cache.bfloat16().cuda(), bt.cuda(), None, torch.tensor(ctx, dtype=torch.int32).cuda(), 0.5,
+                             rows=rows, P=P, RV=RV).double().cpu().view(B, H, RV)
+    for b in range(B):
+        p = torch.softmax(q[b].double() @ lat[b].double().t() * 0.5, -1)
+        v = lat[b][:, :RV].double()
+        assert ((got[b] - p @ v).abs() <= 2 ** -8 * (p @ v.abs()) + 2 ** -8 * (p @ v).abs()).all(), ctx[b]
+
+
 def test_decode_plan_covers_every_head_and_key():
     for B in (1, 3, 24, 128, 400):
         for H in (1, 8, 20, 32, 128):
