@@ -6,8 +6,9 @@
 // IVFFlat (faiss_store.py:101-111,214) and Qdrant query_points (qdrant_store.py:371).
 //
 //   * cfc_knn_scan: scores[q][n] = <x_n, q>  (or -||x_n - q||^2) for <= 16 queries, one pass over
-//     the bf16 index with MFMA 16x16x32 (queries are the B columns, index rows stream straight from
-//     HBM into the A operand), and every block of rows' best score beside them.
+//     the bf16 index with MFMA 16x16x32 (queries are the B columns, index rows the A operand: from
+//     the caches straight to registers, from memory in whole runs by way of LDS), and every block of
+//     rows' best score beside them.
 //   * cfc_topk_select: exact sorted top-k of scores with their block maxima: the k-th best block
 //     maximum bounds the k-th best score from below, so only the blocks that reach it are looked at.
 //   * cfc_knn_maxima, cfc_knn_blocks: the scan of many rows, which stores the best score of every 16 rows
@@ -18,7 +19,7 @@
 //   * cfc_l2_normalize: rows -> unit length (+ fp32 norms), used on insert for cosine.
 //   * cfc_pool: masked mean / CLS pooling over varlen sequences (+ optional L2 normalise):
 //     the SentenceTransformer Pooling+Normalize modules.
-#include "common.h"
+#include "lds_ring.h"
 
 namespace {
 
@@ -74,6 +75,30 @@ struct KnnRows {
       if (alive && !alive[row]) v[i] = -INFINITY;
     }
     return v;
+  }
+  // The same from LDS: what word() brought there for the rows r0 ..
+  __device__ __forceinline__ f32x4_t finish(f32x4_t v, int r0, const char* at) const {
+    const int g = (threadIdx.x & 63) >> 4, rb = r0 + 4 * g;
+    if (xnorm2) {
+      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(at + 16 * g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = -(x[i] + qn - 2.f * v[i]);
+    }
+    if (alive) {
+      const uint4 a = *reinterpret_cast<const uint4*>(at + 64 + 16 * g);
+      const uint32_t m[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (!((m[i] >> (8 * ((uintptr_t)(alive + min(rb + i, N - 1)) & 3))) & 255)) v[i] = -INFINITY;
+    }
+    return v;
+  }
+  // lanes 0 .. 15: the norms of rows r0 .., 16 .. 31: the words that hold their bytes of the mask (of one that is not there, the
+  // other's; the lanes after them alike)
+  __device__ __forceinline__ const void* word(int r0) const {
+    const int lane = threadIdx.x & 63, row = min(r0 + (lane & 15), N - 1);
+    const bool mask = alive && (!xnorm2 || (lane & 16));
+    return mask ? (const void*)((uintptr_t)(alive + row) & ~(uintptr_t)3) : (const void*)(xnorm2 + row);
   }
   // Largest key of the rows that there are, in all lanes of a query.
   __device__ __forceinline__ uint32_t best(const f32x4_t& v, int r0) const {
@@ -146,7 +171,10 @@ __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restric
 // marked).  So rows go to LDS first, by LDS-DMA in pieces of 1 KB, a ring of R units per wave: 16 rows of KU k-steps.  Chunk c
 // of row r lies at c ^ (r & 15) of its row's sixteen (through the pieces' source addresses), and sixteen rows' reads
 // touch all banks.  No barrier: each wave waits for its own pieces alone.  Workgroups of one round, whose waves' streams
-// run on from block to block.
+// run on from block to block.  Norms and the mask come with the rows, a word a lane: loads to registers, which hipcc knows nothing else to be
+// in flight beside, waited for all units that had been asked for (us of squared distances / masked / both, fragments from memory, such
+// loads, this: 1M rows of 512, 4 queries 219 / 217 / 229, 232 / 227 / 254, 182 / 181 / 181; 2M of 256 217 / 215 / 239, 235 / 240 / 271, 184 /
+// 187 / 189; 1M of 384 164 / 162 / 178, this 134 / 134 / 135).
 // us with the selection, fragments from memory -> this: 1M rows of 384 148 -> 132 (of 16 queries 181 -> 166), 3M 413 -> 374;
 // of 768 values, whose fragments fill the registers alone, 500 k 165 -> 131, 100 k 38 -> 33, 5000 16.9 -> 15.7, of 1024 141 k 64 -> 56.
 template <int KC>
@@ -156,18 +184,6 @@ struct KnnUnit {
   static_assert(KC % KU == 0 && KU % 4 == 0 && 4 * R * KU <= 160, "");
 };
 
-typedef __attribute__((address_space(3))) void kn_lds_t;
-
-// One 1-KB LDS-DMA piece of sbase + voff (per lane), read once (M0 kept).
-__device__ __forceinline__ void kn_piece(uint32_t voff, const void* sbase, uint32_t lds_addr) {
-  unsigned keep;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
-      : "=&s"(keep)
-      : "v"(voff), "s"(sbase), "s"(lds_addr)
-      : "memory");
-}
-
 template <int KC, bool MAXIMA>
 __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
                                                             int nq, const float* __restrict__ xnorm2,
@@ -175,7 +191,7 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
                                                             float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
                                                             int B) {
   constexpr int KU = KnnUnit<KC>::KU, R = KnnUnit<KC>::R, NU = KnnUnit<KC>::NU, UB = KU * 1024;
-  __shared__ __attribute__((aligned(16))) char kn_smem[4 * R * UB];
+  __shared__ __attribute__((aligned(16))) char kn_smem[4 * R * (UB + 256)];      // rings, then those of norms and masks
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), stride = gridDim.x * 4;
   const bool qv = col < nq;
@@ -185,7 +201,10 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
   int blk = blockIdx.x * 4 + w;
   if (blk >= nb) return;
   const char* ring = kn_smem + w * (R * UB);
-  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(kn_lds_t*)kn_smem) + w * (R * UB);
+  const uint32_t lds0 = lds_at(ring);
+  const bool extra = xnorm2 || alive;
+  const char* words = kn_smem + 4 * R * UB + w * (R * 256);
+  const uint32_t words0 = lds_at(words);
   uint32_t voff[KU];
 #pragma unroll
   for (int i = 0; i < KU; ++i) {
@@ -193,18 +212,22 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
     voff[i] = (uint32_t)(r * (KC * 64) + ((c & ~15) | ((c ^ r) & 15)) * 16);
   }
   // ---- what is asked for: unit iu of the 16 rows from ir0 of block iblk
-  int iblk = blk, ir0 = blk * B, iu = 0, fill = 0;
+  int iblk = blk, ir0 = blk * B, iu = 0, fill = 0, wfill = 0;
   auto issue = [&]() {
     if (iblk >= nb) return;
+    if (extra && iu == 0) {
+      ring_word_at(rows.word(ir0), words0 + wfill * 256);
+      wfill = wfill + 1 == R ? 0 : wfill + 1;
+    }
     const char* src = reinterpret_cast<const char*>(X) + (size_t)ir0 * (KC * 64) + iu * (KU * 64);
     if (ir0 + 16 <= N) {
 #pragma unroll
-      for (int i = 0; i < KU; ++i) kn_piece(voff[i], src, lds0 + fill * UB + i * 1024);
+      for (int i = 0; i < KU; ++i) ring_piece<true>(voff[i], src, lds0 + fill * UB + i * 1024);
     } else {                                          // past the last row: that one again
 #pragma unroll
       for (int i = 0; i < KU; ++i) {
         const int r = (64 * i + lane) / (4 * KU);
-        kn_piece(voff[i] - (uint32_t)(max(0, ir0 + r - (N - 1)) * (KC * 64)), src, lds0 + fill * UB + i * 1024);
+        ring_piece<true>(voff[i] - (uint32_t)(max(0, ir0 + r - (N - 1)) * (KC * 64)), src, lds0 + fill * UB + i * 1024);
       }
     }
     fill = fill + 1 == R ? 0 : fill + 1;
@@ -219,7 +242,7 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
   };
 #pragma unroll
   for (int i = 0; i < R - 1; ++i) issue();
-  int slot = 0;
+  int slot = 0, wslot = 0;
   for (; blk < nb; blk += stride) {
     const int lo = blk * B, hi = min(N, lo + B);
     uint32_t best = 0u;
@@ -229,8 +252,10 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
       for (int u = 0; u < NU; ++u) {
         // this unit's pieces (scores stored since count too: it waits for no less), and the reads of the one before, whose
         // place the next one takes
-        if (iblk < nb) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(KU * (R - 2)) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        constexpr int LATER = KU * (R - 2);
+        if (iblk >= nb) ring_wait<0>();
+        else if (NU == 1 && extra) ring_wait<LATER + R - 2>();       // (more units a row: a word of the next rows, too, now and then)
+        else ring_wait<LATER>();
         issue();
         const char* img = ring + slot * UB + col * (KU * 64);
 #pragma unroll
@@ -241,7 +266,10 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
         }
         slot = slot + 1 == R ? 0 : slot + 1;
       }
-      v = rows.finish(v, r0);
+      if (extra) {
+        v = rows.finish(v, r0, words + wslot * 256);
+        wslot = wslot + 1 == R ? 0 : wslot + 1;
+      }
       const uint32_t m = rows.best(v, r0);
       if constexpr (MAXIMA) {
         if (r0 - lo == 16 * g) best = m;            // group g's
@@ -879,7 +907,7 @@ CFC_API int cfc_topk_segment(int n) {
 
 // Where rows of up to 512 values come from the 256 MB that the chip caches, workgroups of one round (two a CU) take all
 // blocks, and no last round is nearly empty: 50 k rows of 384 9.8 -> 8.6 us, 100 k of 16 queries 21.8 -> 16.5, 200 k 28.4
-// -> 24.7; 300 k 36.2 -> 38.2 (from memory a workgroup per four blocks reads faster), 100 k of 768 28.2 -> 28.5.
+// -> 24.7; 300 k 36.2 -> 38.2 (from memory a workgroup per four blocks reads faster).
 constexpr long KNN_ROUND_BYTES = 160l << 20;
 constexpr int KNN_ROUND = 512;
 // More than the cache holds goes by knn_stream_kernel, which marks rows as read once (MB of 384 values, us: 230 46 -> 48, 260
