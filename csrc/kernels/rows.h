@@ -13,21 +13,14 @@ template <int V> struct Vec { float v[V]; };
 // NT: past the caches (nontemporal), as far as vectors of four go
 typedef float row_f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t row_u2 __attribute__((ext_vector_type(2)));
-template <bool NT, typename T>
-__device__ __forceinline__ T row_ld(const void* p) {
-  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const T*>(p));
-  else return *reinterpret_cast<const T*>(p);
-}
-template <bool NT, typename T>
-__device__ __forceinline__ void row_st(void* p, T v) {
-  if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<T*>(p));
-  else *reinterpret_cast<T*>(p) = v;
-}
 template <int V, bool NT = false>
 __device__ __forceinline__ Vec<V> ldv(const float* p) {
   Vec<V> r;
-  if constexpr (V == 4) {
-    const row_f4 f = row_ld<NT, row_f4>(p);
+  if constexpr (V == 4 && NT) {
+    const row_f4 f = __builtin_nontemporal_load(reinterpret_cast<const row_f4*>(p));
+    r.v[0] = f.x; r.v[1] = f.y; r.v[2] = f.z; r.v[3] = f.w;
+  } else if constexpr (V == 4) {
+    const float4 f = *reinterpret_cast<const float4*>(p);
     r.v[0] = f.x; r.v[1] = f.y; r.v[2] = f.z; r.v[3] = f.w;
   } else {
     r.v[0] = *p;
@@ -38,7 +31,13 @@ template <int V, bool NT = false>
 __device__ __forceinline__ Vec<V> ldv(const uint16_t* p) {
   Vec<V> r;
   if constexpr (V == 4) {
-    const row_u2 u = row_ld<NT, row_u2>(p);
+    uint2 u;
+    if constexpr (NT) {
+      const row_u2 n = __builtin_nontemporal_load(reinterpret_cast<const row_u2*>(p));
+      u = make_uint2(n.x, n.y);
+    } else {
+      u = *reinterpret_cast<const uint2*>(p);
+    }
     r.v[0] = __uint_as_float(u.x << 16); r.v[1] = __uint_as_float(u.x & 0xffff0000u);
     r.v[2] = __uint_as_float(u.y << 16); r.v[3] = __uint_as_float(u.y & 0xffff0000u);
   } else {
@@ -48,12 +47,14 @@ __device__ __forceinline__ Vec<V> ldv(const uint16_t* p) {
 }
 template <int V, bool NT = false>
 __device__ __forceinline__ void stv(float* p, const Vec<V>& r) {
-  if constexpr (V == 4) row_st<NT>(p, row_f4{r.v[0], r.v[1], r.v[2], r.v[3]});
+  if constexpr (V == 4 && NT) __builtin_nontemporal_store(row_f4{r.v[0], r.v[1], r.v[2], r.v[3]}, reinterpret_cast<row_f4*>(p));
+  else if constexpr (V == 4) *reinterpret_cast<float4*>(p) = make_float4(r.v[0], r.v[1], r.v[2], r.v[3]);
   else *p = r.v[0];
 }
 template <int V, bool NT = false>
 __device__ __forceinline__ void stv(uint16_t* p, const Vec<V>& r) {
-  if constexpr (V == 4) row_st<NT>(p, row_u2{pack2bf(r.v[0], r.v[1]), pack2bf(r.v[2], r.v[3])});
+  if constexpr (V == 4 && NT) __builtin_nontemporal_store(row_u2{pack2bf(r.v[0], r.v[1]), pack2bf(r.v[2], r.v[3])}, reinterpret_cast<row_u2*>(p));
+  else if constexpr (V == 4) *reinterpret_cast<uint2*>(p) = make_uint2(pack2bf(r.v[0], r.v[1]), pack2bf(r.v[2], r.v[3]));
   else *p = f2bf(r.v[0]);
 }
 template <int V>
