@@ -164,6 +164,8 @@ __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, A
   }
 }
 
+constexpr int64_t HYPER_PAST_BYTES = 512ll << 20;      // of all streams
+
 template <typename ACT, int V, int SM>
 int hyper_go(hipStream_t s, int n, const HyperArgs& a, int mode, void* h) {
   const int vecs = (a.W + V - 1) / V;
@@ -174,7 +176,7 @@ int hyper_go(hipStream_t s, int n, const HyperArgs& a, int mode, void* h) {
   do {                                                                                                               \
     constexpr bool one = V == 4 && NV == 1, past = V == 4 && SM <= 4 && NV <= 4;                                     \
     if (one && (SM > 4 || n <= FEW_ROWS)) HN_GO(NV, BT, (one ? ROWS_FEW : ROWS_SOME));                               \
-    else if (past && 4ll * n * a.S * a.W > 8 * PAST_BYTES) HN_GO(NV, BT, (past ? ROWS_PAST : ROWS_SOME));            \
+    else if (past && 4ll * n * a.S * a.W > HYPER_PAST_BYTES) HN_GO(NV, BT, (past ? ROWS_PAST : ROWS_SOME));            \
     else HN_GO(NV, BT, ROWS_SOME);                                                                                   \
   } while (0)
   if (vecs <= 64) GO(1, 64);

@@ -153,9 +153,12 @@ struct ColsIn {
 constexpr int FEW_ROWS = 256;
 
 // What a kernel keeps in mind of its number of rows: ROWS_FEW, and ROWS_PAST of so many that their stream no longer waits in the
-// caches (256 MB) for its next use: it is read and written past them, and what others read next is not pushed out.
+// caches (256 MB) for its next use: it is read and written past them, and what others read next is not pushed out.  A row kernel
+// has 10 to 12 bytes a value, x's 4, 4 of a product's and 2 for each of its 16-bit rows: from 88 MB of x they do not all stay (us of
+// branch_norm / gated_norm on the same rows again and again, through the caches and past them: 4800 rows of 4096, 75 MB, 47 and 55 / 50
+// and 60; 9600, 150 MB, 104 and 103 / 117 and 110).
 enum { ROWS_SOME = 0, ROWS_FEW = 1, ROWS_PAST = 2 };
-constexpr int64_t PAST_BYTES = 64ll << 20;      // of one stream
+constexpr int64_t PAST_BYTES = 88ll << 20;      // of one stream
 
 // NV, BT for rows of W channels in vectors of V
 #define ROW_SHAPES(GO, vecs)           \

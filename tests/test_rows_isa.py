@@ -14,3 +14,9 @@ def test_plain_vectors_are_not_built_for_the_nontemporal_ones():
             if name in line and not line.startswith("typedef"):
                 assert "__builtin_nontemporal" in line, line
     assert len(re.findall("__builtin_nontemporal", src)) == 4
+
+
+def test_streams_past_the_caches_do_not_fit_them():
+    """x (4 bytes a value), a product's 4 and two 16-bit rows' of a gated norm are 256 MB together where x goes past them."""
+    past = int(re.search(r"PAST_BYTES = (\d+)ll << 20", (CSRC / "rows.h").read_text()).group(1))
+    assert past * (4 + 4 + 2 + 2) / 4 >= 256

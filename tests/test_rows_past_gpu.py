@@ -22,8 +22,8 @@ def same(a, b):
     assert float((d / b.float().abs().clamp_min(1.0)).max()) <= (2.0 ** -7 if a.dtype == torch.bfloat16 else 2.0 ** -18)
 
 
-# a stream of 64 MB and a row less, and more; channels of one and of several vectors a thread
-@pytest.mark.parametrize("T,W", [(4096, 4096), (4097, 4096), (2800, 6000), (16400, 1028)])
+# a stream of 88 MB and a row more, and less; channels of one and of several vectors a thread
+@pytest.mark.parametrize("T,W", [(4096, 4096), (4097, 4096), (2800, 6000), (16400, 1028), (5632, 4096), (5633, 4096), (3900, 6000), (1500, 16384), (22500, 1028)])
 @pytest.mark.parametrize("split", [1, 3])
 def test_branches(T, W, split):
     few = slice(T - 200, T)
