@@ -31,7 +31,8 @@ struct HyperArgs {
 };
 
 // SM >= S copies in registers; a thread holds NV vectors of V channels.  ROWS: FEW_ROWS at most, all that a row needs asked for
-// ahead (90 VGPRs), or more: two workgroups of 1024 a CU (46; 2400 rows of 4096 in 4 streams 63.9 -> 58.5 us), or past the caches
+// ahead (90 VGPRs), or more: two workgroups of 1024 a CU (46; 2400 rows of 4096 in 4 streams 63.9 -> 58.5 us; smaller workgroups are
+// enough to a CU either way, 700 rows of 1024 in 4 streams 6.1 ahead, 6.6 without), or past the caches
 template <typename ACT, int V, int SM, int NV, int BT, int ROWS>
 __global__ void __launch_bounds__(BT) hyper_norm_kernel(HyperArgs a, int mode, ACT* __restrict__ h) {
   constexpr bool NT = ROWS == ROWS_PAST;
@@ -175,7 +176,7 @@ int hyper_go(hipStream_t s, int n, const HyperArgs& a, int mode, void* h) {
 #define GO(NV, BT)                                                                                                   \
   do {                                                                                                               \
     constexpr bool one = V == 4 && NV == 1, past = V == 4 && SM <= 4 && NV <= 4;                                     \
-    if (one && (SM > 4 || n <= FEW_ROWS)) HN_GO(NV, BT, (one ? ROWS_FEW : ROWS_SOME));                               \
+    if (one && (SM > 4 || n <= FEW_ROWS || BT < 1024)) HN_GO(NV, BT, (one ? ROWS_FEW : ROWS_SOME));                  \
     else if (past && 4ll * n * a.S * a.W > HYPER_PAST_BYTES) HN_GO(NV, BT, (past ? ROWS_PAST : ROWS_SOME));            \
     else HN_GO(NV, BT, ROWS_SOME);                                                                                   \
   } while (0)

@@ -42,8 +42,8 @@ def test_branches(T, W, split):
         same(out[0][1], out[1][1])
 
 
-# four streams: of 512 MB and less, of more rows than a launch of few; two and five
-@pytest.mark.parametrize("T,W,S", [(8200, 4096, 4), (300, 4096, 4), (16500, 4096, 2), (700, 5000, 3), (300, 4096, 5), (600, 1024, 4)])
+# four streams: of 512 MB and less, of more rows than a launch of few; two and five; past the caches with two and four vectors a thread
+@pytest.mark.parametrize("T,W,S", [(8200, 4096, 4), (300, 4096, 4), (16500, 4096, 2), (700, 5000, 3), (300, 4096, 5), (600, 1024, 4), (8200, 8192, 2), (9000, 5000, 3), (4100, 16384, 2)])
 def test_streams(T, W, S):
     e, y, y2 = rnd(T, W), rnd(1, T, W, seed=1), rnd(2, T, W, seed=2)
     c = H.Connection(rnd(S, seed=3), rnd(S, S, seed=4), rnd(S, seed=5))
