@@ -631,21 +631,21 @@ __global__ void __launch_bounds__(512, 1) latent_attn_kernel(const uint16_t* __r
   };
   // unconditional (a branch per load would wait at every join): columns past the stride re-read the last
   // chunk -- q' is zero there and such outputs are not stored
-  auto gload = [&](u32x4_t (&d)[NL], int b0, int b1, int row) {
+  auto gload = [&]() {
     const uint16_t* p0 = cache + (size_t)b0 * 32 * RS;
     const uint16_t* p1 = cache + (size_t)b1 * 32 * RS;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = tid + 512 * i, key = e / CH, c = e % CH;
-      const int off = (key & 31) * row + min(8 * c, row - 8);
-      d[i] = *reinterpret_cast<const u32x4_t*>((key < 32 ? p0 : p1) + off);
+      const int off = (key & 31) * RS + min(8 * c, RS - 8);
+      st[i] = *reinterpret_cast<const u32x4_t*>((key < 32 ? p0 : p1) + off);
     }
   };
-  auto lwrite = [&](int buf, const u32x4_t (&d)[NL]) {
+  auto lwrite = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = tid + 512 * i, key = e / CH, c = e % CH;
-      *reinterpret_cast<u32x4_t*>(kbuf + buf * (64 * R64 * 2) + key * (R64 * 2) + ((c ^ swz(key)) << 4)) = d[i];
+      *reinterpret_cast<u32x4_t*>(kbuf + buf * (64 * R64 * 2) + key * (R64 * 2) + ((c ^ swz(key)) << 4)) = st[i];
     }
   };
 
@@ -768,41 +768,46 @@ __global__ void __launch_bounds__(512, 1) latent_attn_kernel(const uint16_t* __r
   // one used was a fifth of the bytes of a slice of four)
   auto advance = [&](int t, int buf) {
     if (t + 1 >= tl.kt1) return;
-    lwrite(buf, st);
+    lwrite(buf);
     if (t + 2 >= tl.kt1) return;
-    gload(st, b0, b1, RS);
+    gload();
     ids(t + 3);
   };
 
   if (tl.kt0 < tl.kt1) {
     const int k0 = tl.kt0;
-    // the queries come while the block ids do, once, by way of the second tile's buffer (a row group's waves have the same: each
-    // its own copy is 128 KB through the CU's one path), and the first two tiles together, 128 KB under way
+    // (24 sequences of 2800 keys, 32 heads, 10 slices, with the merge: 32.4 -> 29.6 us; the first tile is there after 6.4 of 18,
+    // was 8.1 of 20)
+    // the first tile's latents ahead of the queries, which come once, by way of the second tile's buffer: a row group's waves
+    // have the same (each its own copy: 128 KB through the CU's one path beside 64 of the first tile)
+    {
+      const int b = tl.bt[min(2 * k0 + (lane & 1), nb - 1)];          // both by one load
+      b0 = __builtin_amdgcn_readlane(b, 0);
+      b1 = __builtin_amdgcn_readlane(b, 1);
+    }
+    gload();
     constexpr bool SHARE = MR < 4;          // more rows: the registers are the output's
     constexpr int NQ = SHARE ? (16 * MR * CH + 511) / 512 : 0;
-    u32x4_t qs[NQ ? NQ : 1], first[NL];
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const int e = min(tid + 512 * i, 16 * MR * CH - 1), row = e / CH, c = e % CH;
-      qs[i] = *reinterpret_cast<const u32x4_t*>(q + (size_t)(tl.q_row + min(tl.m0 + row, tl.rows - 1)) * RS + min(8 * c, RS - 8));
-    }
-    const int b = tl.bt[min(min(2 * k0 + (lane & 3), 2 * tl.kt1 - 1), nb - 1)];      // both tiles' by one load
-    gload(first, __builtin_amdgcn_readlane(b, 0), __builtin_amdgcn_readlane(b, 1), RS);
-    // (a slice of one tile: 1 KB that no one uses, as a branch would have the first tile wait for these loads too)
-    gload(st, __builtin_amdgcn_readlane(b, 2), __builtin_amdgcn_readlane(b, 3), k0 + 1 < tl.kt1 ? RS : 8);
+    u32x4_t qs[NQ ? NQ : 1];
     if (!SHARE && scorer) {
       const uint16_t* qr = q + (size_t)(tl.q_row + gm) * RS + 8 * kq;
 #pragma unroll
       for (int k = 0; k < KS; ++k) qf[k] = *reinterpret_cast<const u32x4_t*>(qr + min(32 * k, RS - 32));
     }
-    ids(k0 + 2);
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
-      const int e = min(tid + 512 * i, 16 * MR * CH - 1), row = e / CH, c = e % CH;      // (no branch: hipcc moves the load into it)
-      qs[i] &= 8 * c < RS ? ~0u : 0u;
-      *reinterpret_cast<u32x4_t*>(kbuf + 64 * R64 * 2 + row * (R64 * 2) + ((c ^ swz(row)) << 4)) = qs[i];
+      const int e = min(tid + 512 * i, 16 * MR * CH - 1), row = e / CH, c = e % CH;
+      qs[i] = *reinterpret_cast<const u32x4_t*>(q + (size_t)(tl.q_row + min(tl.m0 + row, tl.rows - 1)) * RS + min(8 * c, RS - 8));
     }
-    lwrite(0, first);
+    ids(k0 + 1);
+    advance(k0 - 1, 0);
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int e = tid + 512 * i, row = e / CH, c = e % CH;
+      qs[i] &= 8 * c < RS ? ~0u : 0u;
+      if (e < 16 * MR * CH)
+        *reinterpret_cast<u32x4_t*>(kbuf + 64 * R64 * 2 + row * (R64 * 2) + ((c ^ swz(row)) << 4)) = qs[i];
+    }
     lds_barrier();
     if (!SHARE && scorer) {
 #pragma unroll
