@@ -182,15 +182,16 @@ def most_rows(RS: int) -> int:
 
 
 MAX_PARTITIONS = 256
-_TILE_US = {16: 1.4, 32: 1.8, 64: 3.4}     # one 64-key tile at rank 512, by rows per work item (one workgroup alone)
+_TILE_US = {16: 1.37, 32: 1.76, 64: 3.0}     # one 64-key tile at rank 512, by rows per work item (one workgroup alone)
+_SPILLED = 1.9                               # of 64 rows at ranks above 384, whose outputs and queries spill
 
 
 def decode_plan(B: int, heads: int, RS: int, max_ctx: int, P: int | None = None) -> tuple[int, int]:
     """(rows per work item, key slices) of a decode step, from the time of its longest workgroup, the latents' way to all that
     read them and the slices' partials (written and merged in fp32), but no less than the latents' way from memory: fitted
-    to 678 measured (2 to 128 sequences of 300 to 5500 keys, 32 heads, rank 512, 16 and 32 rows, 1 to 32 slices), whose best it
-    misses by 0.4 %.  A merge was taken to cost 8 us before: 4 of 300 keys 12.1 -> 10.0 us, 8 of 1000 15.5 -> 13.7, 24 of 1000
-    20.2 -> 18.7, 96 of 1000 36.8 -> 34.5; 8 to 128 heads of rank 64 to 576 1.0 to 1.39 times as fast where the plan changed."""
+    to 17 269 measured (1 to 128 sequences of 64 to 4000 keys, 8 to 128 heads, rank 64 to 576, 16 to 64 rows, 1 to 32 slices), whose best
+    it misses by 0.8 % on average, 0.3 % at 32 heads of rank 512.  us where a merge was taken to cost 8 and now: 4 of 200 keys 11.0
+    -> 10.0, 8 of 1000 16.0 -> 14.6, 24 of 1000 20.5 -> 19.4; 24 of 1000 with 128 heads 30.3 -> 32.5, all others within 4 %."""
     scale = max(0.35, RS / 512)
     per_cu = max(1, min(4, (160 * 1024) // (2 * 64 * 64 * math.ceil(RS / 64) * 2 + 12 * 1024)))
     nt, best = max(1, math.ceil(max_ctx / 64)), None
@@ -201,11 +202,11 @@ def decode_plan(B: int, heads: int, RS: int, max_ctx: int, P: int | None = None)
         g = math.ceil(heads / rows)
         for p in cand:
             rounds = math.ceil(B * g * p / (256 * per_cu))
-            us = _TILE_US[rows] * scale * (1.15 if rows > 16 and RS > MFMA_MAX_RANK else 1.0)
-            t = max(rounds * (0.7 + math.ceil(nt / p) * us * min(per_cu, math.ceil(B * g * p / 256))) + B * max_ctx * RS * 2 * g / 24e6,
+            us = _TILE_US[rows] * scale * (1.17 if rows > 16 and RS > MFMA_MAX_RANK else 1.0) * (_SPILLED if rows == 64 and RS > 384 else 1.0)
+            t = max(rounds * (1.2 + math.ceil(nt / p) * us * min(per_cu, math.ceil(B * g * p / 256))) + B * max_ctx * RS * 2 * g / 29e6,
                     B * max_ctx * RS * 2 / 7e6)
             if p > 1:
-                t += 4.1 + 2 * B * heads * p * RS * 4 / 4e6
+                t += 2.8 + 2 * B * heads * p * RS * 4 / 4e6
             if best is None or t < best[0]:
                 best = (t, rows, p)
     return best[1], best[2]

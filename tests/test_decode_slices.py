@@ -23,3 +23,11 @@ def test_long_rows_of_many_items_are_sliced(visible):
 def test_slices_are_no_more_than_the_merge_takes(B, H, G, visible):
     for D in (32, 128, 256):
         assert 1 <= A.decode_slices(B, H, G, D, visible, torch.bfloat16) <= min(A.MAX_PARTITIONS, max(1, math.ceil(visible / 256)))
+
+
+@pytest.mark.parametrize("B,heads,RS,keys,plan", [(64, 128, 512, 4000, (32, 1)), (24, 128, 512, 4000, (32, 2)), (4, 32, 512, 200, (16, 4)), (8, 32, 512, 1000, (16, 8))])
+def test_latent_plans_follow_the_measured_best(B, heads, RS, keys, plan):
+    """us of these plans and of others: 133 and, in two slices of 64 rows, which spill at this rank, 202; 79 and 93 in five; 10.0 and in one
+    slice 11.0; 14.6 and in sixteen 16.0."""
+    from copilot_for_consensus_amd.ops import latent as L
+    assert L.decode_plan(B, heads, RS, keys) == plan
