@@ -242,7 +242,7 @@ double mgemm_x_us(int M, int N, int K, int split) {
 
 // pgemm's persistent kernel, in tiles of the height it takes
 double ppp_us(int M, int N, int K, bool fp32) {
-  return ppp_us_at(M, N, K, ppp_height(M, N, K)) * (fp32 ? 1.06 : 1.0);
+  return ppp_us_at(M, N, K, ppp_height(M, N, K)) * (fp32 ? 1.04 : 1.0);
 }
 
 enum { MG_ACT = 0, MG_SLABS = 1, MG_WHOLE = 2 };
@@ -273,16 +273,16 @@ double prompt_best(int M, int N, int K, int kind, int* plan) {
     return ppp_us(M, N, K, kind != MG_ACT);
   double all = mgemm_best(M, N, K, kind, kind != MG_WHOLE, true, bm, split);
   if (weights <= 1 << 23 && M <= (weights > 1 << 22 ? 256 : 640)) return all;       // the decode GEMM, within 10 %
-  // a few rows beyond a whole round are faster here than its model says beside tiles of other heights than 256: 560 and 640
-  // rows of 28672 x 4096
   const int tn = (N + 255) / 256, tm = (M + 255) / 256;
-  const double bias = ppp_height(M, N, K) < 8 && M > 512 && (int64_t)tm * tn > MG_CUS ? 1.04 : 0.97;
-  double best = M < 256 ? 1e29 : bias * ppp_us(M, N, K, kind != MG_ACT);
+  double best = M < 256 ? 1e29 : ppp_us(M, N, K, kind != MG_ACT);
   if ((int64_t)tm * tn >= MG_PGEMM_TILES) all = std::max(all, mgemm_x_us(M, N, K, split));
   if (all < best) best = all, plan[1] = bm, plan[2] = split;
   const int rounds = (int)((int64_t)tm * tn / MG_CUS), head = rounds ? (int)((int64_t)MG_CUS * rounds / tn) * 256 : 0;
   if (head > 0 && head < M && K >= 128) {
-    const double rest = mgemm_best(M - head, N, K, kind, kind == MG_ACT, false, bm, split);
+    // behind another launch its own start is hidden, and W waits in the 256 MB cache for a row tile or two (tails of 1 to 128 rows of
+    // 28672 x 4096 40 to 49 us, alone 58; of 679 of 4096 x 2048 19, alone 24)
+    double rest = mgemm_best(M - head, N, K, kind, kind == MG_ACT, false, bm, split) - 3.0;
+    if (M - head <= 256 && weights <= 1 << 27) rest *= 0.8;
     const double both = ppp_us(head, N, K, kind != MG_ACT) + rest;
     if (both < best) best = both, plan[0] = head, plan[1] = bm, plan[2] = split;
   }
@@ -291,15 +291,18 @@ double prompt_best(int M, int N, int K, int kind, int* plan) {
 
 }  // namespace
 
-// A prompt product's plan: plan = {head, bm, split}: `head` rows (whole rounds of pgemm's 256 x 256 tiles) on its
-// persistent kernel and the others here; {0, 0, 0}: all on the decode GEMM or pgemm.  kind 0: an activation (an epilogue,
+// The model misses the fastest of the heights, this kernel alone and a head with its rest by 0.2 % on average of 550 sizes measured (257 to
+// 15 049 rows of 1024 .. 28672 x 2048 .. 14336), and by 9 % at most.
+// A prompt product's plan: plan = {head, bm, split}: `head` rows (as many as whole rounds of 256 x 256 tiles have) on pgemm's
+// persistent kernel, in tiles of the height it takes, and the others here; {0, 0, 0}: all on the decode GEMM or pgemm.  kind 0: an activation (an epilogue,
 // or what adds the slabs up), 1: fp32 slabs for a consumer that adds them up (with a head: one), 2: one fp32 result.
 //   * up to 128 rows, and 256 (640) of 2^23 (2^22) weights or fewer: the decode GEMM (129 .. 256 rows, 2^23 weights: 17
 //     against 18; 2^21: 14 against 15 at 220 rows, 16 against 17 at 512, but 18.6 against 18.3 at 700);
-//   * all here where pgemm's tiles leave the chip idle: 4096 x 4096 up to 1800 rows (61 against 74; 2100: 81 against 73),
-//     28672 x 4096 up to 256 (68 against 87; 300: 91 against 89);
+//   * all here where pgemm's tiles leave the chip idle: 4096 x 4096 up to 1866 rows (62 against 65; 2072: 78 against 65),
+//     28672 x 4096 up to 256 (68 against 87; 285: 82 against 76 in tiles of 192 rows);
 //     nor where X would be brought into every L2 for a few columns each (mgemm_x_us): 1024 x 4096 up to 7000 rows;
-//   * the rows beyond pgemm's last whole round here: 4096 x 14336 of 4500 rows 512 -> 370, 4096 x 4096 152 -> 124.
+//   * the rows beyond pgemm's last whole round here: 4096 x 14336 of 4500 rows 438 -> 367, 4096 x 4096 136 -> 124, 28672 x
+//     4096 of 560 138 -> 125 (of 1344 not: 242 and 264).
 CFC_API int cfc_prompt_plan(int M, int N, int K, int kind, int* plan) {
   prompt_best(M, N, K, kind, plan);
   return 0;

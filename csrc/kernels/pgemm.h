@@ -90,7 +90,8 @@ __device__ __forceinline__ float pg_out(float v) {
 
 // us of pgemm's persistent kernel in tiles of 32 mt x 256 (mt = 6, 7, 8): a K-tile of 256 rows takes 1.4 in a full round of
 // workgroups, 0.8 to 1.22 in a partial one; of 224 rows 0.91 of that, of 192 0.83, on an idle chip 0.95 and 0.88 to 0.97 (what
-// the waves read from LDS, not the MFMAs, takes the time there).
+// the waves read from LDS, not the MFMAs, takes the time there); all of it 0.945, and 7 % more in a run of 1.2 ms or longer, whose clock
+// is lower, 1 or 2 % more again in the lower tiles.  Within 3 to 4 % of 1650 measured: 257 to 15 049 rows of 1024 .. 28672 x 2048 .. 14336.
 inline double ppp_us_at(int M, int N, int K, int mt) {
   constexpr int CUS = 256;
   const int64_t tiles = (int64_t)((M + 32 * mt - 1) / (32 * mt)) * ((N + 255) / 256);
@@ -98,12 +99,15 @@ inline double ppp_us_at(int M, int N, int K, int mt) {
   const double part = fill > 0 ? 0.8 + 0.42 * fill : 0.0;
   const double all = mt == 6 ? 0.83 : mt == 7 ? 0.91 : 1.0;
   const double idle = mt == 6 ? (full > 0 ? 0.14 : 0.05) : mt == 7 && full > 0 ? 0.04 : 0.0;
-  return 12.0 + K / 64 * (1.4 * full * all + part * (all + idle * (1.0 - fill)));
+  const double us = 12.0 + K / 64 * (1.4 * full * all + part * (all + idle * (1.0 - fill)));
+  const double slow = us < 1200.0 ? us / 1200.0 : 1.0;
+  return us * (0.945 + 0.07 * slow) * (1.0 + 0.01 * (8 - mt) * slow);
 }
 
 // The height that takes the least: fewer rows than 256 where they leave fewer rows of the last tile unused or fill the last
-// round (us of 28672 x 4096 + SwiGLU, 256 rows -> this: 300 / 384 rows 96 -> 85 / 97 -> 83 in 192, 420 95 -> 90 and 896
-// 185 -> 168 in 224, 1100 250 -> 225 in 192, 1344 264 -> 245 in 224; 12288 x 4096 1700 163 -> 150; 4096 x 14336 3500 296 -> 286).
+// round (us of 28672 x 4096, 256 rows -> this: 285 / 351 rows 85 -> 76 / 87 -> 74 and
+// 1107 243 -> 226 in 192; 433 88 -> 82, 896 175 -> 163 and 1344 256 -> 242 in 224; 4096 x 14336 3491 282 -> 276): 0.3 % more than the fastest of the three
+// on average of the sizes above.
 // The sums are the same in every height, so it changes no bit.
 inline int ppp_height(int M, int N, int K) {
   int best = 8;

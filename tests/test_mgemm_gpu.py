@@ -148,3 +148,12 @@ def test_libraries_of_one_family_hold_every_product(preset):
     for entry in ("cfc_prompt_plan", "cfc_mgemm", "cfc_pgemm", "cfc_pgemm_glu", "cfc_dgemm", "cfc_dgemm_config", "cfc_dgemm_slab_plan",
                   "cfc_dgemm_stream", "cfc_dgemm_joint", "cfc_gemv_packed", "cfc_splitk_reduce", "cfc_clamped_glu"):
         assert entry + "(" in text, entry
+
+
+@pytest.mark.skipif(not kernels_available(), reason="the built library is missing")
+def test_plan_goes_by_one_model():
+    """A rule for one size made others worse: 14 000 rows of 4096 x 4096 in two launches (326 us, one 321); a few
+    rows beyond a whole round of 28672 x 4096 are a launch of their own (513 rows 123 us against 133 of all on mgemm)."""
+    assert K.prompt_plan(14_000, 4096, 4096, "whole") is None and K.prompt_plan(14_000, 4096, 4096) is None
+    assert all(K.prompt_plan(M, 28672, 4096)[0] == 512 for M in (513, 533, 560, 640))
+    assert K.prompt_plan(1344, 28672, 4096) is None           # (one launch of 224 rows a tile 242, with a tail 264)
