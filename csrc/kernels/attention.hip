@@ -204,24 +204,16 @@ __global__ void __launch_bounds__(256, F8 ? 2 : 1) paged_decode_kernel(
     const uint16_t* __restrict__ q, const void* __restrict__ kc, const void* __restrict__ vc,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ ctx_lens, float scale_log2, int Hkv,
     int max_blocks, int part_blocks, int P, int window, float v_scale, float* __restrict__ part_o,
-    float* __restrict__ part_ml, uint16_t* __restrict__ out, DecRope rp, const int32_t* __restrict__ shared_blocks,
-    int ordered) {
+    float* __restrict__ part_ml, uint16_t* __restrict__ out, DecRope rp, const int32_t* __restrict__ shared_blocks) {
   // F8: kc / vc hold e4m3 of K / k_scale and V / v_scale; k_scale is folded into scale_log2 by the
   // host, v_scale multiplies the output here
   typedef typename KvFrag<F8>::raw Raw;
   constexpr int D = 128;
-  const int p = blockIdx.x, h = blockIdx.y;
-  int b = blockIdx.z, ctx;
-  if (ordered) {
-    const int2 s = longest_first<256>(ctx_lens, gridDim.z, blockIdx.z, ordered);
-    b = s.x;
-    ctx = s.y;
-  } else {
-    ctx = ctx_lens[b];
-  }
+  const int p = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
   const int Hq = Hkv * G;
+  const int ctx = ctx_lens[b];
   const int nblk = (ctx + KV_BS - 1) / KV_BS;
   // sliding window (window > 0): the query at position ctx-1 sees keys [ctx - window, ctx)
   const int key_lo = window > 0 ? max(0, ctx - window) : 0;
@@ -1728,7 +1720,7 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
   const int64_t wgs = (int64_t)P * Hkv * B;
   const int ordered = wgs <= 512 || B > DEC_ORDER_ROWS || max_blocks * KV_BS < DEC_ORDER_FROM || max_blocks >= 1 << 17 ? 0 : wgs < 704 ? 7 : 2;
 #define DEC_ARGS (const uint16_t*)q, k_cache, v_cache, block_tables, ctx_lens, sl2, Hkv, max_blocks, part_blocks, P, \
-    window, v_scale, part_o, part_ml, (uint16_t*)out, rp, shared_blocks, ordered
+    window, v_scale, part_o, part_ml, (uint16_t*)out, rp, shared_blocks
   // nontemporal KV loads for large batches (B=128: 6.5 vs 5.9 TB/s; B=8: 3.8 vs 4.2 -- there the
   // plain loads win), profiles/decode_attn_partitions_r01.log; CFC_DECODE_NT=0/1 forces either
   static const int nt_env = [] { const char* e = getenv("CFC_DECODE_NT"); return e ? atoi(e) : -1; }();
