@@ -1503,7 +1503,7 @@ __global__ void __launch_bounds__(512, 2) prefill_gqa_kernel(
 // last (partial) 32-key tile, exponentials are v_exp_f32 (inputs <= 0).
 // ------------------------------------------------------------------------------------------
 constexpr int ENC_ROWS = 256;          // query rows per workgroup, 16 ENC_R of a wave
-constexpr float ENC_NONE = 3e38f;      // less a maximum that no score is below; finite, so that a score of -inf keeps its weight of 0
+constexpr float ENC_NONE = 3.4028235e38f;      // less a maximum that no finite score is below, but finite: a score of -inf keeps its weight of 0
 
 // Vector instructions bound it: 32 keys of 16 rows are 8 exponentials a lane, a quarter of the rate of others, and were some 40
 // others, 14 of them for a maximum and a sum across lanes in every step.  Now scores start from the maximum (an MFMA's
