@@ -119,12 +119,14 @@ __device__ __forceinline__ uint4 set_bf16(uint4 v, int e, uint32_t h) {
 // first): more workgroups than the chip holds at once start as others end, and a long one that starts last is waited for
 // alone.  In the order that they have where the contexts are short or differ by no more than `least` sixteenths of the
 // longest: the ranking, 0.5 us a workgroup, would be more than it saves.
+// `lds`: ORDER_LDS bytes, free again when it returns.
+constexpr int ORDER_LDS = (2 * DEC_ORDER_ROWS + 5) * 4;
 template <int THREADS>
-__device__ __forceinline__ int2 longest_first(const int32_t* __restrict__ ctx_lens, int B, int rank, int least) {
+__device__ __forceinline__ int2 longest_first(const int32_t* __restrict__ ctx_lens, int B, int rank, int least, char* lds) {
   constexpr int SHARES = THREADS / DEC_ORDER_ROWS;    // threads of a sequence, each with a share of the others
   static_assert(SHARES == 1 || SHARES == 2, "");
-  __shared__ __attribute__((aligned(16))) int key[DEC_ORDER_ROWS], before[DEC_ORDER_ROWS], ends[4];
-  __shared__ int found;
+  int* key = reinterpret_cast<int*>(lds);
+  int *before = key + DEC_ORDER_ROWS, *ends = before + DEC_ORDER_ROWS, *found = ends + 4;
   const int t = threadIdx.x, s = t & (DEC_ORDER_ROWS - 1), n = ctx_lens[min(s, B - 1)];
   const int lo = wave_min_int(n), hi = -wave_min_int(-n);
   if (t < DEC_ORDER_ROWS) {
@@ -147,12 +149,14 @@ __device__ __forceinline__ int2 longest_first(const int32_t* __restrict__ ctx_le
     if constexpr (SHARES == 1) before[s] = c;
     else atomicAdd(before + s, c);
     __syncthreads();
-    if (t < B && before[t] == rank) found = t;
+    if (t < B && before[t] == rank) *found = t;
     __syncthreads();
-    b = found;
+    b = *found;
   }
   b = __builtin_amdgcn_readfirstlane(b);
-  return make_int2(b, __builtin_amdgcn_readfirstlane(key[b] >> 8));
+  const int ctx = __builtin_amdgcn_readfirstlane(key[b] >> 8);
+  __syncthreads();
+  return make_int2(b, ctx);
 }
 
 struct DecRope {
@@ -470,13 +474,14 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
   constexpr int D = 128, TILE = KV_BS * D * 2, QB = (G + 3) / 4 * 1024, RING = T * TILE;
   constexpr bool ORD = NWV == 4 && T == 2;
   __shared__ __attribute__((aligned(16))) char smem[NWV * (RING + QB)];
+  static_assert(sizeof(smem) <= (T == 2 && NWV == 4 ? 80 : 160) * 1024 && sizeof(smem) >= ORDER_LDS, "four waves: two workgroups a CU");
   const int p = blockIdx.x, h = blockIdx.y;
   int b = blockIdx.z, ctx;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool whole = !(ORD && ordered) && P == 1 && window == 0 && max_blocks > 0;       // the table's blocks: asked for beside the length
   const int spec = whole ? block_tables[(size_t)b * max_blocks + min(w + NWV * lane, max_blocks - 1)] : 0;
   if (ORD && ordered) {
-    const int2 s = longest_first<256>(ctx_lens, gridDim.z, blockIdx.z, ordered);
+    const int2 s = longest_first<256>(ctx_lens, gridDim.z, blockIdx.z, ordered, smem);
     b = s.x;
     ctx = s.y;
   } else {

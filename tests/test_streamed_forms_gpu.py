@@ -1,4 +1,4 @@
-"""What comes by LDS-DMA, in forms beside the usual; encoder scores at the end of the range.  Against float64."""
+"""What comes by LDS-DMA, in forms beside the usual, sixteen query heads a key head among them; encoder scores at the end of the range.  Against float64."""
 import pytest
 import torch
 
@@ -31,6 +31,41 @@ def test_search(dim, N, lo, form):
     tol = 2.0 ** -22 * dim * 4
     assert float((v.double() - want.gather(1, i - lo)).abs().max()) < tol
     assert float((v.double() - want.topk(40).values).abs().max()) < tol
+
+
+def _paged(heads, kv, ctx, blocks, g):
+    n = -(-max(ctx) // 32)
+    bt = torch.randperm(len(ctx) * n, device=DEV, generator=g).int().view(len(ctx), n).contiguous()
+    kc = torch.randn(len(ctx) * n, kv, 32, 128, device=DEV, generator=g).bfloat16()
+    vc = torch.randn(len(ctx) * n, kv, 128, 32, device=DEV, generator=g).bfloat16()
+    q = torch.randn(len(ctx), heads, 128, device=DEV, generator=g).bfloat16()
+    return bt, kc, vc, q, torch.tensor(ctx, dtype=torch.int32, device=DEV)
+
+
+def _paged_want(q, kc, vc, bt, n):
+    kv = kc.shape[1]
+    slots = torch.tensor([4 * g + j if j < 4 else 16 + 4 * g + j - 4 for g in range(4) for j in range(8)], device=DEV)
+    k = kc[bt.long()].transpose(0, 1).reshape(kv, -1, 128)[:, :n].double()
+    v = torch.empty(len(bt), kv, 32, 128, dtype=torch.float64, device=DEV)
+    v[:, :, slots] = vc[bt.long()].view(-1, kv, 4, 128, 8).permute(0, 1, 2, 4, 3).reshape(-1, kv, 32, 128).double()
+    v = v.transpose(0, 1).reshape(kv, -1, 128)[:, :n]
+    p = torch.softmax((q.double().view(kv, -1, 1, 128) * k[:, None]).sum(-1) * 128 ** -0.5, -1)
+    return torch.matmul(p, v).view(-1, 128), torch.matmul(p, v.abs()).max()
+
+
+# more than 512 workgroups of uneven contexts, in their order and longest first; few of them
+@pytest.mark.parametrize("heads,kv,ctx", [(32, 2, [1500 - 23 * (i % 61) for i in range(128)] ), (16, 1, [900, 33, 1400, 256, 1]), (32, 2, [1300] * 40),
+                                          (32, 8, [2100 - 170 * (i % 12) for i in range(90)])])
+@pytest.mark.parametrize("P", [1, 3])
+def test_many_heads_a_key_head(heads, kv, ctx, P):
+    from copilot_for_consensus_amd.ops import kernels as K
+    ctx = ctx[:128]
+    g = torch.Generator(device=DEV).manual_seed(heads + len(ctx))
+    bt, kc, vc, q, lens = _paged(heads, kv, ctx, 0, g)
+    got = K.paged_decode_attention(q, kc, vc, bt, lens, 128 ** -0.5, part_blocks=-P)
+    for s in {0, 1, len(ctx) // 2, len(ctx) - 1}:
+        n = ctx[s]
+        _close(got[s], *_paged_want(q[s], kc, vc, bt[s, :-(-n // 32)], n))
 
 
 @pytest.mark.parametrize("D", [32, 64])
