@@ -24,6 +24,7 @@
 //   * LDS tiles are XOR-swizzled for conflict-free ds_read_b128; the swizzles
 //     were derived against the gfx950 ds_read_b128 lane groups {0-3,12-15,20-27}, ...
 #include "lds_ring.h"
+#include <limits.h>
 #include <stdlib.h>
 
 #include <type_traits>
@@ -470,7 +471,7 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ ctx_lens, float scale_log2, int Hkv, int max_blocks,
     int P, int window, float v_scale, float* __restrict__ part_o, float* __restrict__ part_ml, uint16_t* __restrict__ out,
-    const int32_t* __restrict__ shared_blocks, int ordered) {
+    const int32_t* __restrict__ shared_blocks, int cached, int ordered) {
   constexpr int D = 128, TILE = KV_BS * D * 2, QB = (G + 3) / 4 * 1024, RING = T * TILE;
   constexpr bool ORD = NWV == 4 && T == 2;
   __shared__ __attribute__((aligned(16))) char smem[NWV * (RING + QB)];
@@ -494,7 +495,7 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
   const int blk0 = blk_lo + share_of(nblk - blk_lo, p, P), blk1 = blk_lo + share_of(nblk - blk_lo, p + 1, P);
   const int32_t* bt = block_tables + (size_t)b * max_blocks;
   const int first = blk0 + w, n = first < blk1 ? (blk1 - 1 - first) / NWV + 1 : 0;        // this wave's blocks
-  const int temporal = shared_blocks != nullptr ? shared_blocks[0] : 0;                   // blocks read through the caches
+  const int temporal = shared_blocks != nullptr ? max(cached, shared_blocks[0]) : cached;  // blocks read through the caches
   char* mine = smem + w * (RING + QB);
   const uint32_t lds0 = lds_at(mine);
   const uint32_t kvoff = (lane >> 4) * 256u, vvoff = lane * 16u;     // K: a piece has four rows, chunk (lane & 15) ^ row of each
@@ -1726,8 +1727,8 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
   const int ordered = wgs <= 512 || B > DEC_ORDER_ROWS || max_blocks * KV_BS < DEC_ORDER_FROM || max_blocks >= 1 << 17 ? 0 : wgs < 704 ? 7 : 2;
 #define DEC_ARGS (const uint16_t*)q, k_cache, v_cache, block_tables, ctx_lens, sl2, Hkv, max_blocks, part_blocks, P, \
     window, v_scale, part_o, part_ml, (uint16_t*)out, rp, shared_blocks
-  // nontemporal KV loads for large batches (B=128: 6.5 vs 5.9 TB/s; B=8: 3.8 vs 4.2 -- there the
-  // plain loads win), profiles/decode_attn_partitions_r01.log; CFC_DECODE_NT=0/1 forces either
+  // Read once, or through the caches.  CFC_DECODE_NT=0/1 forces either; of keys and values that come to registers B=128: 6.5 TB/s
+  // read once, 5.9 through the caches, B=8: 3.8, 4.2; runs through LDS are read once
   static const int nt_env = [] { const char* e = getenv("CFC_DECODE_NT"); return e ? atoi(e) : -1; }();
   const bool nt = nt_env >= 0 ? nt_env != 0 : B >= 32;
   // Through LDS in whole runs, unless the table holds 256 keys at most and the workgroups are few, or more sequences than are
@@ -1740,7 +1741,7 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
 #define PDS_GO(NWV, T)                                                                                                      \
   paged_stream_kernel<GG, NWV, T><<<grid, 64 * NWV, 0, stream>>>((const uint16_t*)q, (const uint16_t*)k_cache,               \
       (const uint16_t*)v_cache, block_tables, ctx_lens, sl2, Hkv, max_blocks, P, window, v_scale, part_o, part_ml,           \
-      (uint16_t*)out, shared_blocks, ordered)
+      (uint16_t*)out, shared_blocks, nt_env == 0 ? INT_MAX : 0, ordered)
       // 128 KB under way in a CU, in the eight waves of one workgroup (four with rings of twice the depth: 24 of 1500 28.1 against
       // 25.7, 16 of 700 14.5 against 13.8) or the four of each of two (two waves with twice the depth: 40 of 1500 52.7 against 49.1,
       // 48 of 300 15.4 against 14.3); two blocks in one wave, which has nothing to merge (128 of 60 11.4 -> 9.1 us).  Up to

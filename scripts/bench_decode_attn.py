@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Paged decode attention bandwidth study (Mistral-7B shapes, B=128): random vs sequential block
-tables, part_blocks sweep.  Run twice (CFC_DECODE_NT=0/1) to compare plain and nontemporal loads."""
+tables, part_blocks sweep.  Run twice (CFC_DECODE_NT=0/1) to compare loads through the caches and past them."""
 import math
 import os
 import sys
