@@ -415,15 +415,14 @@ def argmax_keys(local: torch.Tensor, offset: int) -> torch.Tensor:
 @functools.lru_cache(maxsize=4096)
 def kv_partitions(B: int, heads: int, kv_heads: int, blocks: int) -> int:
     """Partitions of each of B sequences of ``blocks`` cache blocks in the paged decode attention, by what a launch takes in
-    us.  5 to 128 sequences, whose keys and values come through LDS: :func:`ops.kernels.streamed_us`.  As many as give a
-    workgroup for every place, and this many: 20 of 700 15.9 -> 13.9, 24 of 1500 32.6 -> 26.5, 24 of 2617 48.3 -> 42.6, 12 of 2617
-    27.4 -> 26.6, 32 of 2617 61.1 -> 57.5.
+    us.  5 to 128 sequences: :func:`ops.kernels.streamed_us`.  As many as give a workgroup for every place, and this many, from 0.8 of
+    the keys: 24 of 700 18.8 -> 14.5, 24 of 1500 32.0 -> 24.8, 24 of 2617 48.1 -> 39.3, 32 of 2617 54.2 -> 51.1, 8 of 400 9.2 -> 8.8.
     Fewer or more sequences fitted to 1048 measured (B of 1 .. 128, 2 .. 172 blocks, 1 .. 64 partitions of 8 KV heads, fragments
     from memory): 3.3, 4.2 and 0.045 for the merge, and what the busiest of 256 CUs, two workgroups each, reads: one block
     per wave takes 3.1 to 3.8 where a CU has one workgroup, 4.5 to 5.5 where some have two, 5 per full round of 512.  A
     workgroup for every slot and a few more is a round more, and few keys are not worth a merge."""
     def streamed(P):
-        return K.streamed_us(blocks, B * kv_heads, 16384, B * heads, P)
+        return K.streamed_us(blocks, B * kv_heads, 16384, B * heads, P, *K.paged_waves(B * kv_heads * P, blocks, P))
 
     def us(P):
         full, rest = divmod(B * kv_heads * P, 512)
@@ -537,10 +536,9 @@ class DecoderModel:
         """KV partitions per sequence of a B-row decode step over tables of ``max_blocks`` blocks: what fills the tables by
         :func:`kv_partitions`, or the fewest that give 512 workgroups (CFC_DECODE_WGS: so many, and always these).
 
-        More than those pay where the contexts do fill the tables (``full``; 24 of 5500 keys 106 -> 92 us, 24 of 400 in tables
-        for 5500 15.1 -> 19.2), and were measured for 32 query and 8 key heads; fewer are right for any context up to the
-        table's, and for 1 to 10 key heads (0.53 to 1.05 of the time, 48 of 200 keys with one key head 1.10).  The 8-bit cache
-        has a kernel of its own, which the model does not fit (48 of 1500 35 -> 40 us)."""
+        More than those pay where the contexts do fill the tables (``full``), and only for 32 query and 8 key heads are they taken;
+        fewer are right for any context up to the table's.  The 8-bit cache has a kernel of its own, which the model does not fit
+        (48 of 1500 35 -> 40 us)."""
         fewest = min(max(1, math.ceil(int(os.environ.get("CFC_DECODE_WGS") or 512) / max(1, B * self.w.kv_heads))),
                      max(1, max_blocks // 2))
         if fp8 or os.environ.get("CFC_DECODE_WGS"):

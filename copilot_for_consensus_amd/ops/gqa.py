@@ -273,7 +273,10 @@ def decode_slices(B: int, H: int, G: int, D: int, visible: int, dtype) -> int:
     if items >= 384 or B == 1:
         return most
     most = max(1, min(math.ceil(768 / items), math.ceil(visible / 256), MAX_PARTITIONS))      # (the last slice may have fewer tiles)
-    return min(range(1, most + 1), key=lambda P: streamed_us(math.ceil(visible / 32), items, 128 * D, B * H, P))
+    def waves(w):
+        return (4, 1, False) if D > 128 else (8, 1, False) if w <= 256 else (4, 2, False)
+
+    return min(range(1, most + 1), key=lambda P: streamed_us(math.ceil(visible / 32), items, 128 * D, B * H, P, *waves(items * P)))
 
 
 def attention(a: Heads, q, rows, block_tables, ctx_lens, cu_q=None, tiles=None, P: int = 1, workspace=None, gate: Cols | None = None,

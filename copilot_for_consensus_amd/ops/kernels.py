@@ -194,16 +194,28 @@ def rope_kv_write(qkv, positions, slots, cos_sin, k_cache, v_cache, Hq, Hkv, D, 
     return q_out
 
 
-def streamed_us(tiles: int, items: int, tile_bytes: int, rows: int, P: int) -> float:
-    """What a decode step's attention and merge take in us, less its start: ``items`` workgroups by ``P`` slices of ``tiles`` tiles
-    of 32 keys (``tile_bytes`` of keys and values each) that come through LDS (csrc/kernels/lds_ring.h), ``rows`` query rows.  The
-    chip's 6.5 TB/s, or the busiest of 256 CUs, 3.4 us for its eight waves' tiles of 16 KB, whichever is longer; eight waves of one
-    workgroup, or four of each of two.  Its best P takes 0.8 % more than the best of 1400 measured (2 to 128 sequences, 32 query and
-    8 key heads of 128 columns, 100 to 5500 keys, 1 to 24 slices)."""
-    w = items * P
-    cu = math.ceil(tiles / P / 8) if w <= 256 else math.ceil(w / 256) * math.ceil(tiles / P / 4) / 2
-    merge = 3.4 + 0.06 * rows * P / 32 if P > 1 else 0.0
-    return merge + ((items * tiles * tile_bytes / 6.5e6) ** 4 + (cu * tile_bytes / 16384 * 3.4) ** 4) ** 0.25
+def paged_waves(wgs: int, blocks: int, P: int) -> tuple[int, int, bool]:
+    """Of a launch of the paged decode attention over P slices of ``blocks`` blocks: waves of a workgroup, workgroups a CU has at once,
+    and whether keys and values come straight to registers (attention.hip ``paged_waves``)."""
+    if wgs <= 32 or (wgs <= 256 and blocks <= 8) or (P > 1 and math.ceil(blocks / P) <= 4):
+        return 4, 2, True
+    return (4, 1, False) if wgs <= 64 else (8, 1, False) if wgs <= 256 else (4 if blocks > 2 else 1, 2, False)
+
+
+def streamed_us(tiles: int, items: int, tile_bytes: int, rows: int, P: int, waves: int, held: int, straight: bool) -> float:
+    """What a decode step's attention and merge take in us: ``items`` workgroups by ``P`` slices of ``tiles`` tiles of 32 keys
+    (``tile_bytes`` of keys and values together), ``rows`` query rows, by the kernel's ``waves`` a workgroup, workgroups ``held`` by a
+    CU, and tiles that come ``straight`` to registers or by a ring.  The chip's 7.1 TB/s, or the rounds of the busiest of 256 CUs, 0.65
+    and for each tile of a wave 0.36 (straight 0.23) and what the CU's waves have under way at 55 GB/ms, whichever is longer.  Its best P takes 0.4 % more
+    than the best of 3500 measured paged launches (5 to 128 sequences, 1 to 8 key heads for 8 to 64 query heads of 128 columns, 30 to
+    5500 keys, 1 to 32 slices), and 2 % more than that of 9556 grouped ones (heads of 32 to 256, 1 to 100 sequences)."""
+    w, steps = items * P, math.ceil(tiles / P / waves)
+    rounds = w / (256 * held)
+    rounds = rounds if rounds > 3 else math.ceil(rounds)
+    under = min(held, math.ceil(w / 256)) * min(waves, math.ceil(tiles / P)) * tile_bytes / 55e3
+    merge = 2.8 + 0.02 * rows * P * tile_bytes / 2 ** 19 if P > 1 else 0.0
+    return (3.5 + merge + ((items * tiles * tile_bytes / 7.1e6) ** 4
+                           + (rounds * (0.65 + steps * ((0.23 if straight else 0.36) + under))) ** 4) ** 0.25)
 
 
 def decode_partitions(max_ctx: int, part_blocks: int) -> int:

@@ -609,25 +609,14 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
   }
 
   // lane (col, g) holds O^T[d = 16 dt + 4 g + i][col]
-  if constexpr (NWV == 1) {
+  if constexpr (NWV == 1) {        // one slice
     if (col >= G) return;
     const size_t row = (size_t)b * Hq + h * G + col;
-    const float inv = P == 1 ? (l > 0.f ? v_scale / l : 0.f) : v_scale;
+    const float inv = l > 0.f ? v_scale / l : 0.f;
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      const int d = 16 * dt + 4 * g;
-      if (P == 1) {
+    for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) out[row * D + d + i] = f2bf(o[dt][i] * inv);         // out is aligned to its elements only
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) part_o[(row * P + p) * D + d + i] = o[dt][i] * inv;
-      }
-    }
-    if (P > 1 && g == 0) {
-      part_ml[(row * P + p) * 2] = m;
-      part_ml[(row * P + p) * 2 + 1] = l;
-    }
+      for (int i = 0; i < 4; ++i) out[row * D + 16 * dt + 4 * g + i] = f2bf(o[dt][i] * inv);         // out is aligned to its elements only
     return;
   }
   __syncthreads();                                 // every wave's tiles are used up
@@ -1703,6 +1692,22 @@ __global__ void __launch_bounds__(256, D == 32 ? (ENC_R == 4 ? 4 : 6) : 2) encod
 }  // namespace
 
 // q: [B, Hq, 128] bf16; caches per layer as documented above; out: [B, Hq, 128] bf16.
+// Waves of a workgroup of the paged decode attention of `seen` blocks of a table in P slices, less than zero: those of
+// paged_decode_kernel, keys and values straight to registers.  By the ring 128 KB are under way in a CU, in the eight waves of one
+// workgroup (four with rings of twice the depth: 24 of 1500 28.1 us against 25.7, 16 of 700 14.5 against 13.8) or the four of each of two (two
+// waves with twice the depth: 40 of 1500 52.7 against 49.1, 48 of 300 15.4 against 14.3); two blocks in one wave, which has nothing to merge
+// (128 of 60 11.4 -> 9.1).  Up to 64 workgroups in four waves all the same: those of the fused step, whose small batches get the same bits
+// either way.
+// us of 8 key heads, one slice, straight -> ring: 8 of 2617 keys 50.3 -> 31.4, 24 59.9 -> 42.6, 32 66.2 -> 57.5, 48 97 -> 88, 72 158 -> 131, 90
+// 170 -> 157, 128 219 -> 212, from 0.8 of it 198 -> 191; 24 of 700 19.1 -> 14.9; but 12 of 64 4.5 -> 5.1, 192 of 2617 315 -> 330 (more sequences than
+// are ordered have 2 GB of cache and more to read from, and what waits in registers is deeper).  With four blocks or fewer to a slice, one a
+// wave, a ring has nothing to have under way, and so for very few workgroups of any length: 1 of 400 in 12 slices 7.1 -> 7.7, 5 of 1500 in 24
+// 14.5 -> 16.1, 24 of 400 in 12 20.8 -> 25.0, 3 of 2617 in one 38.0 -> 39.7.
+constexpr int paged_waves(int64_t wgs, int seen, int P, int max_blocks) {
+  if (wgs <= 32 || (wgs <= 256 && seen <= 8) || (P > 1 && (seen + P - 1) / P <= 4)) return -4;
+  return wgs <= 64 ? 4 : wgs <= 256 ? 8 : max_blocks > 2 ? 4 : 1;
+}
+
 // part_o / part_ml: fp32 workspaces of B*Hq*P*128 and B*Hq*P*2 floats (unused when P == 1).
 template <bool F8>
 static int launch_paged_decode(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_tables,
@@ -1731,28 +1736,21 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
   // read once, 5.9 through the caches, B=8: 3.8, 4.2; runs through LDS are read once
   static const int nt_env = [] { const char* e = getenv("CFC_DECODE_NT"); return e ? atoi(e) : -1; }();
   const bool nt = nt_env >= 0 ? nt_env != 0 : B >= 32;
-  // Through LDS in whole runs, unless the table holds 256 keys at most and the workgroups are few, or more sequences than are
-  // ordered wait: those have 2 GB of cache and more to read from, and what waits in registers is deeper.
-  // us of 8 key heads, one partition, fragments from memory -> this: 8 of 2617 keys 50.3 -> 31.4, 24 59.9 -> 42.6, 32 66.2 -> 57.5, 48
-  // 97 -> 88, 72 158 -> 131, 90 170 -> 157, 128 219 -> 212, from 0.8 of it 198 -> 191; 24 of 700 19.1 -> 14.9, 8 of 300 9.1 -> 7.7; 12 of
-  // 64 4.5 -> 5.1, 192 of 2617 315 -> 330.
   if constexpr (!F8) {
-    if (!rope && part_blocks <= 0 && (wgs > 256 || max_blocks > 8) && B <= DEC_ORDER_ROWS) {
+    const int seen = window > 0 ? min(max_blocks, (window + 30) / KV_BS + 1) : max_blocks;
+    const int nw = rope || part_blocks > 0 || B > DEC_ORDER_ROWS ? -4 : paged_waves(wgs, seen, P, max_blocks);
+    if (nw > 0) {
 #define PDS_GO(NWV, T)                                                                                                      \
   paged_stream_kernel<GG, NWV, T><<<grid, 64 * NWV, 0, stream>>>((const uint16_t*)q, (const uint16_t*)k_cache,               \
       (const uint16_t*)v_cache, block_tables, ctx_lens, sl2, Hkv, max_blocks, P, window, v_scale, part_o, part_ml,           \
       (uint16_t*)out, shared_blocks, nt_env == 0 ? INT_MAX : 0, ordered)
-      // 128 KB under way in a CU, in the eight waves of one workgroup (four with rings of twice the depth: 24 of 1500 28.1 against
-      // 25.7, 16 of 700 14.5 against 13.8) or the four of each of two (two waves with twice the depth: 40 of 1500 52.7 against 49.1,
-      // 48 of 300 15.4 against 14.3); two blocks in one wave, which has nothing to merge (128 of 60 11.4 -> 9.1 us).  Up to
-      // 64 workgroups in four waves all the same: those of the fused step, whose small batches get the same bits either way
 #define PDS_CASE(G_)                        \
   case G_: {                                \
     constexpr int GG = G_;                  \
-    if (wgs <= 64) PDS_GO(4, 4);            \
-    else if (wgs <= 256) PDS_GO(8, 2);      \
-    else if (max_blocks > 2) PDS_GO(4, 2);  \
-    else PDS_GO(1, 4);                      \
+    if (nw == 8) PDS_GO(8, 2);              \
+    else if (nw == 1) PDS_GO(1, 4);         \
+    else if (wgs <= 64) PDS_GO(4, 4);       \
+    else PDS_GO(4, 2);                      \
   } break;
       switch (G) {
         PDS_CASE(1) PDS_CASE(2) PDS_CASE(4) PDS_CASE(8) PDS_CASE(16)
@@ -1782,6 +1780,11 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
 #undef DEC_ARGS
   if (P > 1) decode_combine_kernel<<<(Hq * B + 3) / 4, 256, 0, stream>>>(part_o, part_ml, P, Hq * B, (uint16_t*)out);
   return CFC_CHECK_LAUNCH();
+}
+
+// what a launch takes (see paged_waves)
+CFC_API int cfc_paged_waves(int64_t wgs, int seen, int P, int max_blocks) {
+  return wgs < 1 || P < 1 ? 0 : paged_waves(wgs, seen, P, max_blocks);
 }
 
 // q: [B, Hq, 128] bf16; caches per layer as documented above; out: [B, Hq, 128] bf16.

@@ -4,7 +4,10 @@ import math
 import pytest
 import torch
 
+from copilot_for_consensus_amd.models.decoder import kv_partitions
 from copilot_for_consensus_amd.ops import gqa as A
+from copilot_for_consensus_amd.ops import kernels as K
+from copilot_for_consensus_amd.ops._native import kernels, kernels_available
 
 
 @pytest.mark.parametrize("visible", (255, 512, 1536, 1537, 2048, 6000, 100_000))
@@ -31,3 +34,25 @@ def test_latent_plans_follow_the_measured_best(B, heads, RS, keys, plan):
     slice 11.0; 14.6 and in sixteen 16.0."""
     from copilot_for_consensus_amd.ops import latent as L
     assert L.decode_plan(B, heads, RS, keys) == plan
+
+
+@pytest.mark.parametrize("B,heads,kv,keys,least", [(5, 32, 8, 400, 3), (8, 32, 8, 400, 3), (8, 64, 8, 700, 3), (5, 32, 2, 700, 5), (24, 32, 2, 700, 2), (5, 8, 1, 1500, 8)])
+def test_few_items_are_sliced(B, heads, kv, keys, least):
+    """us in one slice (as many as the merge was thought to allow) and in these: 5 x 400 10.4 and 8.1, 8 x 400 10.6 and 8.8, 8 x 700 of 64
+    heads 14.9 and 12.0, two key heads 11.2 and 9.2, 15.8 and 12.4, one 10.2 and 8.3."""
+    assert kv_partitions(B, heads, kv, math.ceil(keys / 32)) >= least
+
+
+@pytest.mark.parametrize("B,keys", [(24, 700), (24, 1500), (24, 2617), (32, 2617), (128, 2617)])
+def test_a_full_round_is_not(B, keys):
+    assert kv_partitions(B, 32, 8, math.ceil(keys / 32)) == 1
+
+
+@pytest.mark.skipif(not kernels_available(), reason="the built library is missing")
+def test_paged_plan_knows_the_launch():
+    lib = kernels()
+    for wgs in (1, 32, 33, 64, 65, 256, 257, 4000):
+        for blocks in (1, 2, 3, 8, 9, 40, 41, 300):
+            for P in (1, 2, 3, 10, 64):
+                waves, _, straight = K.paged_waves(wgs, blocks, P)
+                assert lib.cfc_paged_waves(wgs, blocks, P, blocks) == (-waves if straight else waves)
