@@ -397,7 +397,7 @@ class PemolornModel:
     def decode_partitions(self, B: int, max_blocks: int, full: bool = True, fp8: bool = False) -> int:
         """Key slices per sequence of a B-row decode step over block tables ``max_blocks`` wide."""
         ctx = max_blocks * KV_BLOCK
-        return max(A.decode_slices(B, a.H, a.G, a.D, a.mask.visible(ctx), self.w.dtype) for a in (lw["heads"] for lw in self.w.layers))
+        return max(A.decode_slices(B, a.H, a.G, a.D, a.mask.visible(ctx), self.w.dtype, a.mask.pool > 0) for a in (lw["heads"] for lw in self.w.layers))
 
     def decode_workspace(self, B: int, P: int) -> int:
         return max(B * lw["heads"].H * P * (lw["heads"].D + 2) for lw in self.w.layers) if P > 1 else 1

@@ -396,7 +396,7 @@ class TadolixModel:
     def decode_partitions(self, B: int, max_blocks: int, full: bool = True, fp8: bool = False) -> int:
         """Key slices per sequence of a B-row decode step over block tables ``max_blocks`` wide."""
         ctx = max_blocks * KV_BLOCK
-        return max([1] + [A.decode_slices(B, a.H, a.G, a.D, a.mask.visible(ctx), self.w.dtype) for a in self._heads()])
+        return max([1] + [A.decode_slices(B, a.H, a.G, a.D, a.mask.visible(ctx), self.w.dtype, a.mask.pool > 0) for a in self._heads()])
 
     def decode_workspace(self, B: int, P: int) -> int:
         return max([1] + [B * a.H * P * (a.D + 2) for a in self._heads()]) if P > 1 else 1

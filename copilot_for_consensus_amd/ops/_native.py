@@ -63,6 +63,7 @@ _KERNEL_SIGS = {
     "cfc_latent_norm": [I, P, I, I, I, I, P, P, F, P, P, I, P, I, P],
     "cfc_latent_rope": [I, P, I, c_int64, c_int64, I, I, P, F, P, P, I, I, P, I, c_int64, c_int64, I, I, P, I, I, P, P, I,
                         c_int64, c_int64, I, P, P, I, F, P, P],
+    "cfc_gqa_decode_waves": [I, I, c_int64, I, I],
     "cfc_paged_waves": [c_int64, I, I, I],
     "cfc_head_linear_slabs": [P, I, c_int64, c_int64, P, I, I, I, I, I, I, P, c_int64, c_int64, P],
     "cfc_head_linear": [I, P, c_int64, c_int64, P, I, I, I, I, I, I, P, c_int64, c_int64, P, c_int64, P],

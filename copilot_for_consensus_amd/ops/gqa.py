@@ -257,26 +257,50 @@ def prompt_tiles(cu, ctx, H: int, G: int, rows: int) -> np.ndarray:
     return np.stack([np.concatenate(seq)[order], np.concatenate(m0)[order]]).astype(np.int32)
 
 
+def straight_tiles(D: int, pooled: bool, wgs: int) -> float:
+    """Tiles of a slice up to which keys and values come straight to registers (gqa.hip ``straight_tiles``)."""
+    if pooled:
+        return math.inf if wgs <= (math.inf if D <= 32 else 512 if D <= 64 else 256 if D <= 96 else 64 if D <= 128 else 256 if D <= 192 else 0) else 0
+    if D <= 32:
+        return math.inf
+    if D <= 64:
+        return 8 if wgs <= 64 else 4 if wgs <= 512 else 0
+    if D <= 96:
+        return 8 if wgs <= 64 else 2 if wgs <= 256 else 0
+    if D <= 128:
+        return 2 if wgs <= 64 else 1 if wgs <= 256 else 0
+    return math.inf if D <= 192 and wgs <= 64 else 0
+
+
+def decode_waves(D: int, pooled: bool, wgs: int, tiles: int, blocks: int) -> tuple[int, int, bool]:
+    """Of a decode step of slices of ``tiles`` tiles over tables of ``blocks``: waves of a workgroup, workgroups a CU has at once, and
+    whether keys and values come straight to registers (gqa.hip ``decode_waves``)."""
+    if tiles <= straight_tiles(D, pooled, wgs):
+        return 4, 2 if D <= 128 else 1, True
+    if D > 128:
+        return (2, 2, False) if 256 < wgs <= 512 else (4, 1, False)
+    if blocks <= 2 and wgs > 512:
+        return 1, 2, False
+    return (8, 2 if D <= 64 else 1, False) if blocks > 4 and wgs <= (512 if D <= 64 else 256) else (4, 2, False)
+
+
 @functools.lru_cache(maxsize=4096)
-def decode_slices(B: int, H: int, G: int, D: int, visible: int, dtype) -> int:
-    """Key slices per row of a decode step, at least eight 32-key tiles each.  MFMA kernel: from 384 items on one slice where few
+def decode_slices(B: int, H: int, G: int, D: int, visible: int, dtype, pooled: bool = False) -> int:
+    """Key slices per row of a decode step, at least eight 32-key tiles each.  MFMA kernels: from 384 items on one slice where few
     keys are seen, else 1024 in all: what more gain grows with the longest row, whose keys are one workgroup's work, and the rows'
     differences.  Fewer: at most 768 in all, and as many as :func:`streamed_us` finds fastest.  us of 8 key heads with 768 and with
-    this many: 24 of 512 keys 16.0 -> 12.5, 24 of 2000 41.3 -> 35.3, 32 of 1024 31.2 -> 25.1, 8 of 4000 31.4 -> 27.3, 12 of 1024 16.0 ->
-    15.3.  One row: as many as there are.  Others: about four workgroups per CU."""
+    this many: 24 of 512 keys 14.8 -> 11.2, 24 of 2048 38.1 -> 32.0, 12 of 1024 14.5 -> 14.0.  One row, and heads of 32 (straight to registers): as many as there are.  Others: about four workgroups per CU."""
     if dtype != torch.bfloat16 or D not in MFMA_DIMS:
         return max(1, min(math.ceil(1024 / (B * math.ceil(H / ANY_ROWS))), visible // 256, MAX_PARTITIONS))
     items = B * G * math.ceil(H / G / 16)
     if items >= 384 and visible <= 1536:
         return 1
     most = max(1, min(math.ceil((768 if items < 384 else 1024) / items), visible // 256, MAX_PARTITIONS))
-    if items >= 384 or B == 1:
+    if items >= 384 or B == 1 or D <= 32:
         return most
     most = max(1, min(math.ceil(768 / items), math.ceil(visible / 256), MAX_PARTITIONS))      # (the last slice may have fewer tiles)
-    def waves(w):
-        return (4, 1, False) if D > 128 else (8, 1, False) if w <= 256 else (4, 2, False)
-
-    return min(range(1, most + 1), key=lambda P: streamed_us(math.ceil(visible / 32), items, 128 * D, B * H, P, *waves(items * P)))
+    tiles = math.ceil(visible / 32)
+    return min(range(1, most + 1), key=lambda P: streamed_us(tiles, items, 128 * D, B * H, P, *decode_waves(D, pooled, items * P, math.ceil(tiles / P), tiles)))
 
 
 def attention(a: Heads, q, rows, block_tables, ctx_lens, cu_q=None, tiles=None, P: int = 1, workspace=None, gate: Cols | None = None,

@@ -13,6 +13,7 @@
 //                  tiles of their own, which come to LDS in whole runs; values are read back transposed
 //                  (ds_read_b64_tr_b16); the score product's result is the output product's operand as it lies.  No
 //                  barrier until the waves merge
+//   * gqa_straight the same for slices of few tiles: keys to registers, and values by way of them to a wave's LDS tile
 //   * gqa_prompt   portions of prompts: 32 rows of the flattened (token, head of the group) rows per wave, 64-key tiles
 //                  of both ranges double-buffered in LDS
 //   * gqa_any      any head size and the 32-bit path: a wave per (token, head) row
@@ -135,14 +136,57 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 
 // ------------------------------------------------------------------------------------------ decoded tokens
+// the waves' outputs (wave i's [16][LD] fp32 at smem + i STEP, its rows' maxima and sums in ml) to the slice's or the result's rows
+template <int D, int NWV, int STEP, int LD>
+__device__ __forceinline__ void merge_waves(const char* smem, const float (&ml)[NWV][16][2], const GqaArgs& a, int s, int hk, int r0, int nr,
+                                            uint16_t* __restrict__ out) {
+  const int R = a.R;
+  const size_t qrow = (size_t)s * a.H + hk * R + r0;
+  for (int e = threadIdx.x; e < nr * (D / 4); e += 64 * NWV) {
+    const int r = e / (D / 4), c = 4 * (e % (D / 4));
+    float M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int i = 0; i < NWV; ++i) M = fmaxf(M, ml[i][r][0]);
+    const float ref = M == -INFINITY ? 0.f : M;
+    f32x4_t y{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NWV; ++i) {
+      const float f = exp2f(ml[i][r][0] - ref);
+      L += f * ml[i][r][1];
+      y += f * *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(smem + i * STEP) + r * LD + c);
+    }
+    const size_t grow = qrow + r;
+    if (a.P > 1) {
+      *reinterpret_cast<f32x4_t*>(a.part_o + (grow * a.P + blockIdx.y) * D + c) = y;
+      if (c == 0) {
+        a.part_ml[(grow * a.P + blockIdx.y) * 2] = M;
+        a.part_ml[(grow * a.P + blockIdx.y) * 2 + 1] = L;
+      }
+      continue;
+    }
+    const float inv = sink_inv(a, hk * R + r0 + r, M, L);
+    const int oc = (hk * R + r0 + r) * a.DV + c;
+    uint16_t* dst = out + s * a.og.ld + oc;
+    if (a.og.vec) {
+      if (c < a.DV) {
+        const f32x4_t f = inv * out_gate4<uint16_t>(a.og, s, oc);
+        *reinterpret_cast<uint2*>(dst) = make_uint2(cvt_pk_bf16_f32(y[0] * f[0], y[1] * f[1]), cvt_pk_bf16_f32(y[2] * f[2], y[3] * f[3]));
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (c + i < a.DV) dst[i] = f2bf(y[i] * inv * out_gate<uint16_t>(a.og, s, oc + i));
+    }
+  }
+}
+
 // grid (B * G * ceil(R / 16), P).  A workgroup of NWV waves, wave w on its slice's tiles w, w + NWV, ..; keys and values come
 // through a ring of T tiles of the wave's own (lds_ring.h), chunks swizzled through the pieces' source addresses.  A tile that is
 // one cache block's is one run; those of pooled pages of fewer entries and the last of the far range, past whose keys nothing
 // is read, come by rows.  What bounds it is memory: loads straight to registers (keys 64 bytes of 16 rows each) kept one tile of
 // each wave under way, 3.6 to 5.4 TB/s; us of heads of 128, 8 key heads, 0.7 to 1 times the keys, with the slices of either: 12
 // of 4000 39.8 -> 36, 32 of 1024 31.7 -> 23, 48 of 1024 39.7 -> 34.3, 105 of 852 65.9 -> 57.3, 128 of 2600 212 -> 191; heads of 256, 64
-// of 1024 39.6 -> 29; of 64, 64 of 3000 69.7 -> 62.9.  Of 30 keys, one tile, 4.9 -> 5.1, and heads of 32 to 96 of up to 100 keys
-// 0.2 to 0.4 more than before.
+// of 1024 39.6 -> 29; of 64, 64 of 3000 69.7 -> 62.9.  Slices of few tiles are gqa_straight_kernel's.
 template <int D, bool SHAPED, int NWV, int T>
 __global__ void __launch_bounds__(64 * NWV, D <= 64 || (D <= 128 && NWV < 8 && T == 2) ? 2 : 1) gqa_decode_kernel(const uint16_t* __restrict__ q,
                                                                                        const uint16_t* __restrict__ kc,
@@ -338,42 +382,185 @@ __global__ void __launch_bounds__(64 * NWV, D <= 64 || (D <= 128 && NWV < 8 && T
     ml[w][lane][1] = l;
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < nr * (D / 4); e += 64 * NWV) {
-    const int r = e / (D / 4), c = 4 * (e % (D / 4));
-    float M = -INFINITY, L = 0.f;
+  merge_waves<D, NWV, RING, D + 4>(smem, ml, a, s, hk, r0, nr, out);
+}
+
+// The same for slices of few tiles: a wave's next tile comes straight to its registers under the present one, keys into the score
+// product's operand.  With a tile or two a wave there is nothing for a ring to have under way, and a trip through LDS
+// more: us of 8 key heads, one slice, this / the ring: heads of 64, 12 sequences of 60 keys 4.4 / 4.8, of 32, 24 of 200 5.1 / 5.5, pooled
+// means of heads of 128, 1 of 1024 keys 7.9 / 8.8; straight_tiles() has the rest.
+template <int D, bool SHAPED>
+__global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) gqa_straight_kernel(const uint16_t* __restrict__ q,
+                                                                          const uint16_t* __restrict__ kc,
+                                                                          const uint16_t* __restrict__ vc,
+                                                                          const uint16_t* __restrict__ pk,
+                                                                          const uint16_t* __restrict__ pv, GqaArgs a,
+                                                                          uint16_t* __restrict__ out) {
+  constexpr int KS = D / 32, NV = D / 16, CH = D / 8, DT = D / 16;
+  __shared__ __attribute__((aligned(16))) char smem[4 * 64 * D];     // a wave's 32 x D values; then its 16 x D outputs
+  __shared__ float ml[4][16][2];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, kq = lane >> 4;
+  const int R = a.R, RG = a.RG;
+  int item = blockIdx.x;
+  const int rg = item % RG;
+  item /= RG;
+  const int hk = item % a.G, s = item / a.G, pos = a.ctx_lens[s] - 1;
+  const int32_t* bt = a.block_tables + (size_t)s * a.max_blocks;
+  const KeyTiles kt = key_tiles<32>(a, pos, pos);
+  const int t0 = share_of(kt.nt, blockIdx.y, a.P), t1 = share_of(kt.nt, blockIdx.y + 1, a.P);
+  const int r0 = 16 * rg, nr = min(16, R - r0);
+  const size_t qrow = (size_t)s * a.H + hk * R + r0;
+
+  u32x4_t qf[KS];
+  char* vbuf = smem + w * 64 * D;
+  const float* bias = SHAPED && a.bias ? a.bias + (size_t)(hk * R + r0 + min(col, nr - 1)) * a.nb : nullptr;
+  const float far_bias = bias ? bias[a.nb - 1] : 0.f;
+  u32x4_t kf[2][KS], vf[NV];
+  const int first = a.size ? window_first(a, pos) : 0;
+  // This lane's key (lane & 31) in a tile (past the slice: its last), the cache block that it is in, and its row.  The block goes
+  // from one step to the next, and not the row: that would be waited for as soon as it is asked for, and with it all that was
+  // asked for before it, the next tile (one slice of 2800 keys, heads of 128: 38 us with rows, 30).  Heads of more than 160
+  // columns have no registers left for it (of 256: 62 with rows, 80).
+  constexpr bool ROWS = D > 160;
+  auto key_of = [&](int t) {
+    t = min(t, t1 - 1);
+    return t < kt.nat ? min(32 * t + (lane & 31), kt.na - 1) : kt.lo + 32 * (t - kt.nat) + (lane & 31);
+  };
+  auto pooled_at = [&](int t) { return a.pool && min(t, t1 - 1) < kt.nat; };
+  auto row_in = [&](int t, int block) { return key_row(a, pooled_at(t), block, hk, key_of(t)); };
+  auto find = [&](int t) {
+    const int block = bt[key_page(a, pooled_at(t), key_of(t))];
+    return ROWS ? row_in(t, block) : block;
+  };
+  auto load = [&](int t, int found) {
+    const bool pooled = pooled_at(t);
+    const int row = ROWS ? found : row_in(t, found);
+    const uint16_t *kb = pooled ? pk : kc, *vb = pooled ? pv : vc;
 #pragma unroll
-    for (int i = 0; i < NWV; ++i) M = fmaxf(M, ml[i][r][0]);
-    const float ref = M == -INFINITY ? 0.f : M;
-    f32x4_t y{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < 2; ++g) {
+      const uint16_t* p = kb + (size_t)__shfl(row, 16 * g + col, 64) * D + 8 * kq;
 #pragma unroll
-    for (int i = 0; i < NWV; ++i) {
-      const float f = exp2f(ml[i][r][0] - ref);
-      L += f * ml[i][r][1];
-      y += f * *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(smem + i * RING) + r * (D + 4) + c);
+      for (int k = 0; k < KS; ++k) kf[g][k] = *reinterpret_cast<const u32x4_t*>(p + 32 * k);
     }
-    const size_t grow = qrow + r;
-    if (a.P > 1) {
-      *reinterpret_cast<f32x4_t*>(a.part_o + (grow * a.P + blockIdx.y) * D + c) = y;
-      if (c == 0) {
-        a.part_ml[(grow * a.P + blockIdx.y) * 2] = M;
-        a.part_ml[(grow * a.P + blockIdx.y) * 2 + 1] = L;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int e = lane + 64 * i;
+      vf[i] = *reinterpret_cast<const u32x4_t*>(vb + (size_t)__shfl(row, e / CH, 64) * D + 8 * (e % CH));
+    }
+  };
+
+  f32x4_t o[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) o[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  int t = t0 + w;
+  if (t < t1) {
+    int found = find(t);
+    load(t, found);
+#pragma unroll
+    for (int k = 0; k < KS; ++k)             // behind the first tile, which waits for indexes
+      qf[k] = *reinterpret_cast<const u32x4_t*>(q + (qrow + min(col, nr - 1)) * D + 32 * k + 8 * kq);
+    found = find(t + 4);
+    auto step = [&](auto more) {
+      wave_lds_fence();                      // the last tile's values have been read
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int e = lane + 64 * i, key = e / CH, c = e % CH;
+        *reinterpret_cast<u32x4_t*>(vbuf + key * (2 * D) + ((c ^ vswz<D>(key)) << 4)) = vf[i];
       }
-      continue;
-    }
-    const float inv = sink_inv(a, hk * R + r0 + r, M, L);
-    const int oc = (hk * R + r0 + r) * a.DV + c;
-    uint16_t* dst = out + s * a.og.ld + oc;
-    if (a.og.vec) {
-      if (c < a.DV) {
-        const f32x4_t f = inv * out_gate4<uint16_t>(a.og, s, oc);
-        *reinterpret_cast<uint2*>(dst) = make_uint2(cvt_pk_bf16_f32(y[0] * f[0], y[1] * f[1]), cvt_pk_bf16_f32(y[2] * f[2], y[3] * f[3]));
-      }
-    } else {
+      f32x4_t sc[2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (c + i < a.DV) dst[i] = f2bf(y[i] * inv * out_gate<uint16_t>(a.og, s, oc + i));
-    }
+      for (int g = 0; g < 2; ++g) {
+        sc[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < KS; ++k) sc[g] = mfma16(kf[g][k], qf[k], sc[g]);
+      }
+      if constexpr (decltype(more)::value) {
+        load(t + 4, found);
+        found = find(t + 8);
+      }
+      const bool far = t < kt.nat;
+      // (key <= last ..: what sees() says of the tile's keys, without its branches at each of them)
+      const int k0 = far ? 32 * t : kt.lo + 32 * (t - kt.nat), last = far ? kt.na - 1 : pos, lo = far ? 0 : first;
+      if constexpr (SHAPED) {
+        float bt8[2][4];
+        if (bias && pos - k0 - 31 < a.nb - 1) {
+#pragma unroll
+          for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bt8[g][i] = bias[min(max(pos - k0 - (16 * g + 4 * kq + i), 0), a.nb - 1)];
+        } else {
+#pragma unroll
+          for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bt8[g][i] = far_bias;
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sc[g][i] = a.capped ? cap_score<uint16_t>(a, sc[g][i], bt8[g][i]) : sc[g][i] + bt8[g][i];
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = k0 + 16 * g + 4 * kq + i;
+          const bool see = ROWS ? (far ? key < kt.na : sees(a, pos, key)) : (key <= last) & ((key >= lo) | (key < a.keep));
+          if (!see) sc[g][i] = -INFINITY;
+          mx = fmaxf(mx, sc[g][i]);
+        }
+      mx = xor32_max(xor16_max(mx));
+      const float mn = fmaxf(m, mx), ref = mn == -INFINITY ? 0.f : mn, alpha = __builtin_amdgcn_exp2f(m - ref);
+      m = mn;
+      l *= alpha;
+      if (!__all(alpha == 1.f)) {
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[d] *= alpha;
+      }
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sc[g][i] = __builtin_amdgcn_exp2f(sc[g][i] - ref);
+          l += sc[g][i];
+        }
+      // operand slots 8 kq + j: keys 4 kq + j of the first 16, then of the second
+      u32x4_t pf;
+      pf[0] = cvt_pk_bf16_f32(sc[0][0], sc[0][1]);
+      pf[1] = cvt_pk_bf16_f32(sc[0][2], sc[0][3]);
+      pf[2] = cvt_pk_bf16_f32(sc[1][0], sc[1][1]);
+      pf[3] = cvt_pk_bf16_f32(sc[1][2], sc[1][3]);
+      wave_lds_fence();
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        u32x4_t vt;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int key = 16 * u + 4 * kq + (col >> 2), c = 2 * d + ((col & 3) >> 1);
+          const uint2 v = tr_read(vbuf + key * (2 * D) + ((c ^ vswz<D>(key)) << 4) + 8 * (col & 1));
+          vt[2 * u] = v.x;
+          vt[2 * u + 1] = v.y;
+        }
+        o[d] = mfma16(vt, pf, o[d]);
+      }
+    };
+    // The last step asks for nothing: a tile that no one uses was one in three or four of a short slice's loads.  In a step of its
+    // own: behind a condition in the loop the loads stay where they are (2800 keys in one slice 38 -> 50 us)
+    for (; t + 4 < t1; t += 4) step(std::true_type{});
+    step(std::false_type{});
   }
+  l = xor32_sum(xor16_sum(l));
+  wave_lds_fence();
+  float* ob = reinterpret_cast<float*>(vbuf);            // [16][D]
+#pragma unroll
+  for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(ob + col * D + 16 * d + 4 * kq) = o[d];
+  if (lane < 16) {
+    ml[w][lane][0] = m;
+    ml[w][lane][1] = l;
+  }
+  __syncthreads();
+  merge_waves<D, 4, 64 * D, D>(smem, ml, a, s, hk, r0, nr, out);
 }
 
 // ------------------------------------------------------------------------------------------ prompt portions
@@ -731,26 +918,57 @@ int prompt_go(int grid, hipStream_t s, const void* q, const void* kc, const void
   return CFC_CHECK_LAUNCH();
 }
 
+// Tiles of a slice up to which gqa_straight_kernel is the faster one, by the launch's workgroups, from 9556 measured (heads of 32 to 256, 1 to
+// 100 sequences of 30 to 4000 keys, 1 to 32 slices of any key head count): time by the ring over time straight, by the geometric mean of a range's,
+//   heads of 32   1.04 to 1.14 up to 512 workgroups and 16 tiles, 0.93 to 1.03 beyond
+//   of 64         up to 64 workgroups 1.01 to 1.06 to 8 tiles, 0.90 to 0.98 beyond; to 512 workgroups 1.02 to 1.10 to 4, 0.86 to 0.96 beyond
+//   of 96         the same to 64 workgroups; to 256 1.04 to 1.08 to 2 tiles, 0.90 to 1.00 beyond
+//   of 128        to 64 workgroups 1.01 to 1.04 to 2 tiles, 0.87 to 0.98 beyond; to 256 1.04 of one, 0.88 to 1.00 beyond
+//   of 160        to 64 workgroups 1.00 to 1.14, of 300 to 512 0.66 to 0.88;  of 256  0.59 to 0.95
+// Pooled means come by rows either way, which is dearer by the ring: of heads of 32 to 160 1.03 to 1.27 where the ring would gain little.
+constexpr int straight_tiles(int D, bool pooled, int64_t wgs) {
+  constexpr int ALL = 1 << 30;
+  if (pooled) return wgs <= (D <= 32 ? ALL : D <= 64 ? 512 : D <= 96 ? 256 : D <= 128 ? 64 : D <= 192 ? 256 : 0) ? ALL : 0;
+  if (D <= 32) return ALL;
+  if (D <= 64) return wgs <= 64 ? 8 : wgs <= 512 ? 4 : 0;
+  if (D <= 96) return wgs <= 64 ? 8 : wgs <= 256 ? 2 : 0;
+  if (D <= 128) return wgs <= 64 ? 2 : wgs <= 256 ? 1 : 0;
+  return D <= 192 && wgs <= 64 ? ALL : 0;
+}
+
+// Waves of a workgroup of a decode step, `tiles` to a slice of a table of max_blocks, less than zero: gqa_straight_kernel's.
+// By the ring 64 to 128 KB under way in a CU, as in attention.hip: eight waves of one workgroup, or of each of two where the rings are small
+// enough (heads of 128, four waves with rings of twice the depth -> eight: 5 of 700 15.4 -> 11.7 us, 24 of 1500 30.9 -> 27.6), four of
+// two (two of twice the depth: 48 of 1024 38.4 -> 34.3); one for two blocks (128 of 60 12.4 -> 11.4); heads of more than 128
+// columns four of one, two of each of two (heads of 160, 300 to 512 workgroups: 22.5 -> 19.4; more in fours: 158 -> 142)
+constexpr int decode_waves(int D, bool pooled, int64_t wgs, int tiles, int max_blocks) {
+  if (tiles <= straight_tiles(D, pooled, wgs)) return -4;
+  if (D > 128) return wgs > 256 && wgs <= 512 ? 2 : 4;
+  if (max_blocks <= 2 && wgs > 512) return 1;
+  return max_blocks > 4 && wgs <= (D <= 64 ? 512 : 256) ? 8 : 4;
+}
+
 template <int D, bool SHAPED>
 int decode_go(dim3 grid, hipStream_t s, const void* q, const void* kc, const void* vc, const void* pk, const void* pv, const GqaArgs& a,
               void* out) {
-#define GDK(NWV, T)                                                                                                                 \
-  gqa_decode_kernel<D, SHAPED, NWV, T><<<grid, 64 * NWV, 0, s>>>((const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc,        \
-                                                                 (const uint16_t*)pk, (const uint16_t*)pv, a, (uint16_t*)out)
-  // 64 to 128 KB under way in a CU, as in attention.hip: eight waves of one workgroup, or of each of two where the rings are small
-  // enough (heads of 128, four waves with rings of twice the depth -> eight: 5 of 700 15.4 -> 11.7 us, 24 of 1500 30.9 -> 27.6), four of
-  // two (two of twice the depth: 48 of 1024 38.4 -> 34.3); one for two blocks (128 of 60 12.4 -> 11.4); heads of more than 128
-  // columns four of one, two of each of two (heads of 160, 300 to 512 workgroups: 22.5 -> 19.4; more in fours: 158 -> 142)
-  const int64_t wgs = (int64_t)grid.x * grid.y;
-  if constexpr (D > 128) {
-    if (wgs > 256 && wgs <= 512) GDK(2, 2);
+#define GD_ARGS (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, (const uint16_t*)pk, (const uint16_t*)pv, a, (uint16_t*)out
+#define GDK(NWV, T) gqa_decode_kernel<D, SHAPED, NWV, T><<<grid, 64 * NWV, 0, s>>>(GD_ARGS)
+  // the most tiles that a row of the table can have: those of its window, and what it keeps or pools
+  const int near = a.size ? min(a.max_blocks, (a.size + 30) / 32 + 1) : a.max_blocks;
+  const int far = !a.size ? 0 : a.pool ? max(0, 32 * a.max_blocks - a.size) / a.pool / 32 + 1 : (a.keep + 31) / 32;
+  const int tiles = min(a.max_blocks + (a.pool ? 1 : 0), near + far);
+  const int nw = decode_waves(D, a.pool > 0, (int64_t)grid.x * grid.y, (tiles + grid.y - 1) / grid.y, a.max_blocks);
+  if (nw < 0) gqa_straight_kernel<D, SHAPED><<<grid, 256, 0, s>>>(GD_ARGS);
+  else if constexpr (D > 128) {
+    if (nw == 2) GDK(2, 2);
     else GDK(4, 2);
-  } else {
-    if (a.max_blocks <= 2 && wgs > 512) GDK(1, 4);
-    else if (a.max_blocks > 4 && wgs <= (D <= 64 ? 512 : 256)) GDK(8, 2);
+  } else if constexpr (D > 32) {
+    if (nw == 1) GDK(1, 4);
+    else if (nw == 8) GDK(8, 2);
     else GDK(4, 2);
   }
 #undef GDK
+#undef GD_ARGS
   return CFC_CHECK_LAUNCH();
 }
 
@@ -761,6 +979,11 @@ constexpr int prompt_waves(int D) { return D == 64 || D == 128 ? 8 : 4; }
 // rows of one key head's prompt tile for cached heads of D columns (0: the general kernel's, 4 rows over all heads)
 CFC_API int cfc_gqa_prompt_rows(int D) {
   return D == 32 || D == 64 || D == 96 || D == 128 || D == 160 || D == 192 || D == 256 ? 32 * prompt_waves(D) : 0;
+}
+
+// what decode_go takes (see decode_waves)
+CFC_API int cfc_gqa_decode_waves(int D, int pooled, int64_t wgs, int tiles, int max_blocks) {
+  return decode_waves(D, pooled != 0, wgs, tiles, max_blocks);
 }
 
 // q [T][H][D] scaled by log2(e); caches [blocks][G][32][D], pooled [blocks][G][1 << le][D]; out [T][H][DV].

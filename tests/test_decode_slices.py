@@ -56,3 +56,21 @@ def test_paged_plan_knows_the_launch():
             for P in (1, 2, 3, 10, 64):
                 waves, _, straight = K.paged_waves(wgs, blocks, P)
                 assert lib.cfc_paged_waves(wgs, blocks, P, blocks) == (-waves if straight else waves)
+
+
+@pytest.mark.parametrize("H,G,D,B,keys,P", [(16, 1, 32, 24, 2048, 8), (32, 8, 32, 8, 2048, 8), (32, 8, 32, 5, 1024, 4)])
+def test_few_items_of_narrow_heads_are_sliced(H, G, D, B, keys, P):
+    """us in one slice and in these: heads of 32 with one key head 13.4 and 8.4, with eight 13.3 and 10.1, 8.6 and 7.8."""
+    assert A.decode_slices(B, H, G, D, keys, torch.bfloat16) == P
+
+
+@pytest.mark.skipif(not kernels_available(), reason="the built library is missing")
+def test_grouped_plan_knows_the_launch():
+    lib = kernels()
+    for D in (32, 64, 96, 128, 160, 192, 256):
+        for wgs in (1, 64, 65, 256, 257, 512, 513, 5000):
+            for tiles in (1, 2, 3, 4, 5, 8, 9, 33, 200):
+                for pooled in (False, True):
+                    for blocks in (2, 3, 4, 5, 200):
+                        waves, _, straight = A.decode_waves(D, pooled, wgs, tiles, blocks)
+                        assert lib.cfc_gqa_decode_waves(D, int(pooled), wgs, tiles, blocks) == (-waves if straight else waves)

@@ -68,6 +68,28 @@ def test_many_heads_a_key_head(heads, kv, ctx, P):
         _close(got[s], *_paged_want(q[s], kc, vc, bt[s, :-(-n // 32)], n))
 
 
+# keys straight to registers and by the ring, one and several to a slice
+@pytest.mark.parametrize("D", [32, 64, 96, 128, 160, 192, 256])
+@pytest.mark.parametrize("B,P", [(3, 1), (3, 7), (40, 1), (40, 2), (70, 1)])
+def test_grouped(D, B, P):
+    from copilot_for_consensus_amd.ops import gqa
+    from copilot_for_consensus_amd.runtime.kv_cache import PagedHeads
+    ctx = [700 - 37 * (i % 18) for i in range(B)]
+    g = torch.Generator(device=DEV).manual_seed(D + B)
+    n = -(-max(ctx) // 32)
+    bt = torch.randperm(B * n, device=DEV, generator=g).int().view(B, n).contiguous()
+    rows = PagedHeads(B * n, 8, D, 0, 0, DEV, torch.bfloat16)
+    for t in (rows.k, rows.v):
+        t.copy_(torch.randn(t.shape, device=DEV, generator=g))
+    a = gqa.Heads(24, 8, D, D, D ** -0.5, gqa.Mask(0), 1e-6, None, None, False, None)
+    q = (torch.randn(B, 24, D, device=DEV, generator=g) * a.q_scale).bfloat16()
+    out = gqa.attention(a, q, rows, bt, torch.tensor(ctx, dtype=torch.int32, device=DEV), P=P)
+    for s in {0, 1, B // 2, B - 1}:
+        k, v = (t[bt[s].long()].transpose(0, 1).reshape(8, -1, D)[:, :ctx[s]].double() for t in (rows.k, rows.v))
+        p = torch.softmax((q[s].double().view(8, 3, 1, D) * k[:, None]).sum(-1) / gqa.LOG2E, -1)
+        _close(out[s].view(8, 3, D), torch.matmul(p, v), torch.matmul(p, v.abs()).max())
+
+
 @pytest.mark.parametrize("D", [32, 64])
 @pytest.mark.parametrize("lens", [[40], [200, 31, 7]])
 def test_encoder_scores_at_the_end_of_the_range(D, lens):
