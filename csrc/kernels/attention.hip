@@ -1738,7 +1738,8 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
   const bool nt = nt_env >= 0 ? nt_env != 0 : B >= 32;
   if constexpr (!F8) {
     const int seen = window > 0 ? min(max_blocks, (window + 30) / KV_BS + 1) : max_blocks;
-    const int nw = rope || part_blocks > 0 || B > DEC_ORDER_ROWS ? -4 : paged_waves(wgs, seen, P, max_blocks);
+    const bool aligned = (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;       // LDS-DMA's sources
+    const int nw = rope || part_blocks > 0 || B > DEC_ORDER_ROWS || !aligned ? -4 : paged_waves(wgs, seen, P, max_blocks);
     if (nw > 0) {
 #define PDS_GO(NWV, T)                                                                                                      \
   paged_stream_kernel<GG, NWV, T><<<grid, 64 * NWV, 0, stream>>>((const uint16_t*)q, (const uint16_t*)k_cache,               \

@@ -957,7 +957,8 @@ int decode_go(dim3 grid, hipStream_t s, const void* q, const void* kc, const voi
   const int near = a.size ? min(a.max_blocks, (a.size + 30) / 32 + 1) : a.max_blocks;
   const int far = !a.size ? 0 : a.pool ? max(0, 32 * a.max_blocks - a.size) / a.pool / 32 + 1 : (a.keep + 31) / 32;
   const int tiles = min(a.max_blocks + (a.pool ? 1 : 0), near + far);
-  const int nw = decode_waves(D, a.pool > 0, (int64_t)grid.x * grid.y, (tiles + grid.y - 1) / grid.y, a.max_blocks);
+  const bool aligned = (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)pk | (uintptr_t)pv) & 15) == 0;       // LDS-DMA's sources
+  const int nw = aligned ? decode_waves(D, a.pool > 0, (int64_t)grid.x * grid.y, (tiles + grid.y - 1) / grid.y, a.max_blocks) : -4;
   if (nw < 0) gqa_straight_kernel<D, SHAPED><<<grid, 256, 0, s>>>(GD_ARGS);
   else if constexpr (D > 128) {
     if (nw == 2) GDK(2, 2);

@@ -150,13 +150,21 @@ __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restric
         }
       }
     };
-    uint4 a[2][KC];                  // the next 16 rows in flight under these (144 -> 131 us)
-    rows.load(a[0], lo);
-    for (int r0 = lo; r0 < hi; r0 += 32) {
-      if (r0 + 16 < hi) rows.load(a[1], r0 + 16);
-      take(a[0], r0);
-      if (r0 + 32 < hi) rows.load(a[0], r0 + 32);
-      if (r0 + 16 < hi) take(a[1], r0 + 16);
+    if constexpr (KC <= 16) {          // the next 16 rows in flight under these (144 -> 131 us); wider rows fill the registers alone
+      uint4 a[2][KC];
+      rows.load(a[0], lo);
+      for (int r0 = lo; r0 < hi; r0 += 32) {
+        if (r0 + 16 < hi) rows.load(a[1], r0 + 16);
+        take(a[0], r0);
+        if (r0 + 32 < hi) rows.load(a[0], r0 + 32);
+        if (r0 + 16 < hi) take(a[1], r0 + 16);
+      }
+    } else {
+      uint4 a[KC];
+      for (int r0 = lo; r0 < hi; r0 += 16) {
+        rows.load(a, r0);
+        take(a, r0);
+      }
     }
     if constexpr (MAXIMA) {
       if (qv && lo + 16 * g < hi) out[col * ld + 4 * blk + g] = key2f(best);
@@ -915,6 +923,8 @@ constexpr int KNN_ROUND = 512;
 // values; rows of 128, a quarter of a unit each, do not (200 MB 44 -> 65, 400 97 -> 127).
 constexpr long KNN_STREAM_BYTES = 288l << 20;
 constexpr int KNN_CUS = 256;
+// LDS-DMA's sources are whole sixteens of bytes; rows that lie otherwise come to registers
+bool knn_aligned(const void* X) { return ((uintptr_t)X & 15) == 0; }
 
 #define KNN_ARGS(OUT, B) (const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, qnorm2, alive, OUT, (size_t)ld, B
 
@@ -929,12 +939,11 @@ CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, c
   const long bytes = (long)N * dim * 2;
 #define KS(KC)                                                                                                             \
   if constexpr (KC > 4)                                                                                                    \
-    if (KC > 16 || bytes > KNN_STREAM_BYTES) {                                                                             \
+    if (knn_aligned(X) && (KC > 16 || bytes > KNN_STREAM_BYTES)) {                                                         \
       knn_stream_kernel<KC, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B);                     \
       break;                                                                                                               \
     }                                                                                                                      \
-  if constexpr (KC <= 16)                                                                                                  \
-    knn_scan_kernel<KC, false><<<bytes <= KNN_ROUND_BYTES ? min(all, KNN_ROUND) : all, 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B); \
+  knn_scan_kernel<KC, false><<<KC <= 16 && bytes <= KNN_ROUND_BYTES ? min(all, KNN_ROUND) : all, 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B); \
   break
   KNN_DIMS(KS)
 #undef KS
@@ -946,9 +955,13 @@ CFC_API int cfc_knn_maxima(const void* X, const void* Q, int N, int nq, int dim,
                            const uint8_t* alive, float* out, long ld, hipStream_t stream) {
   if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || ld < (N - 1) / 16 + 1) return -1;
   const int nb = (N - 1) / 64 + 1, all = (nb + 3) / 4;
-#define KS(KC)                                                                                                  \
-  if constexpr (KC > 4) knn_stream_kernel<KC, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64); \
-  else knn_scan_kernel<KC, true><<<all, 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);                       \
+#define KS(KC)                                                                                                              \
+  if constexpr (KC > 4)                                                                                                     \
+    if (knn_aligned(X)) {                                                                                                   \
+      knn_stream_kernel<KC, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);                   \
+      break;                                                                                                                \
+    }                                                                                                                       \
+  knn_scan_kernel<KC, true><<<all, 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);                                       \
   break
   KNN_DIMS(KS)
 #undef KS

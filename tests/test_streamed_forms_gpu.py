@@ -1,9 +1,17 @@
-"""What comes by LDS-DMA, in forms beside the usual, sixteen query heads a key head among them; encoder scores at the end of the range.  Against float64."""
+"""What comes by LDS-DMA (index rows, decode attention's keys and values) in forms beside the usual: sources that are no whole
+sixteens of bytes, masks at any byte, sixteen query heads a key head; and encoder scores at the end of the range.  Against float64."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+
+
+def _shifted(t):
+    """The same values two bytes further on."""
+    out = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    assert out.data_ptr() % 16 == 2
+    return out.copy_(t)
 
 
 def _close(got, want, scale):
@@ -13,11 +21,15 @@ def _close(got, want, scale):
 
 @pytest.mark.parametrize("dim,N", [(768, 5000), (768, 177), (1024, 333), (384, 393_300)])
 @pytest.mark.parametrize("lo", [0, 1, 2, 3, 35])
-@pytest.mark.parametrize("form", ["l2", "mask", "both"])
+@pytest.mark.parametrize("form", ["l2", "mask", "both", "rows"])
 def test_search(dim, N, lo, form):
     from copilot_for_consensus_amd.ops import kernels as K
     g = torch.Generator(device=DEV).manual_seed(N + lo)
     X, Q = (torch.randn(n, dim, device=DEV, generator=g).bfloat16() for n in (N, 3))
+    if form == "rows":
+        if N > 5000:
+            pytest.skip("rows from memory to registers: the smaller ones show it")
+        X = _shifted(X)
     xn, qn = (t.float().pow(2).sum(1) if form in ("l2", "both") else None for t in (X, Q))
     alive = torch.rand(N, device=DEV, generator=g) > 0.3 if form in ("mask", "both") else None
     v, i = K.knn_topk(X, Q, 40, xn, qn, alive=alive, row_lo=lo, N=N - 1)
@@ -68,10 +80,22 @@ def test_many_heads_a_key_head(heads, kv, ctx, P):
         _close(got[s], *_paged_want(q[s], kc, vc, bt[s, :-(-n // 32)], n))
 
 
-# keys straight to registers and by the ring, one and several to a slice
+@pytest.mark.parametrize("P", [1, 2])
+def test_paged_queries_at_any_element(P):
+    from copilot_for_consensus_amd.ops import kernels as K
+    ctx = [700, 1, 333, 640, 90, 512, 700]
+    bt, kc, vc, q, lens = _paged(32, 8, ctx, 0, torch.Generator(device=DEV).manual_seed(P))
+    want = K.paged_decode_attention(q, kc, vc, bt, lens, 128 ** -0.5, part_blocks=-P)
+    got = K.paged_decode_attention(_shifted(q), kc, vc, bt, lens, 128 ** -0.5, part_blocks=-P)
+    # the same weights to bf16 from maxima of other waves' blocks
+    assert bool(((got.double() - want.double()).abs() <= 2.0 ** -8 * want.double().abs() + 2.0 ** -8).all())
+
+
+# keys straight to registers and by the ring, one and several to a slice, pooled means and a window
 @pytest.mark.parametrize("D", [32, 64, 96, 128, 160, 192, 256])
 @pytest.mark.parametrize("B,P", [(3, 1), (3, 7), (40, 1), (40, 2), (70, 1)])
-def test_grouped(D, B, P):
+@pytest.mark.parametrize("shift", [False, True])
+def test_grouped(D, B, P, shift):
     from copilot_for_consensus_amd.ops import gqa
     from copilot_for_consensus_amd.runtime.kv_cache import PagedHeads
     ctx = [700 - 37 * (i % 18) for i in range(B)]
@@ -83,7 +107,7 @@ def test_grouped(D, B, P):
         t.copy_(torch.randn(t.shape, device=DEV, generator=g))
     a = gqa.Heads(24, 8, D, D, D ** -0.5, gqa.Mask(0), 1e-6, None, None, False, None)
     q = (torch.randn(B, 24, D, device=DEV, generator=g) * a.q_scale).bfloat16()
-    out = gqa.attention(a, q, rows, bt, torch.tensor(ctx, dtype=torch.int32, device=DEV), P=P)
+    out = gqa.attention(a, _shifted(q) if shift else q, rows, bt, torch.tensor(ctx, dtype=torch.int32, device=DEV), P=P)
     for s in {0, 1, B // 2, B - 1}:
         k, v = (t[bt[s].long()].transpose(0, 1).reshape(8, -1, D)[:, :ctx[s]].double() for t in (rows.k, rows.v))
         p = torch.softmax((q[s].double().view(8, 3, 1, D) * k[:, None]).sum(-1) / gqa.LOG2E, -1)
