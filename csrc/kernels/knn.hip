@@ -192,14 +192,15 @@ struct KnnUnit {
   static_assert(KC % KU == 0 && KU % 4 == 0 && 4 * R * KU <= 160, "");
 };
 
-template <int KC, bool MAXIMA>
+// WORDS: there are norms or a mask
+template <int KC, bool MAXIMA, bool WORDS>
 __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
                                                             int nq, const float* __restrict__ xnorm2,
                                                             const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
                                                             float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
                                                             int B) {
   constexpr int KU = KnnUnit<KC>::KU, R = KnnUnit<KC>::R, NU = KnnUnit<KC>::NU, UB = KU * 1024;
-  __shared__ __attribute__((aligned(16))) char kn_smem[4 * R * (UB + 256)];      // rings, then those of norms and masks
+  __shared__ __attribute__((aligned(16))) char kn_smem[4 * R * (UB + (WORDS ? 256 : 0))];      // rings, then those of norms and masks
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), stride = gridDim.x * 4;
   const bool qv = col < nq;
@@ -210,7 +211,6 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
   if (blk >= nb) return;
   const char* ring = kn_smem + w * (R * UB);
   const uint32_t lds0 = lds_at(ring);
-  const bool extra = xnorm2 || alive;
   const char* words = kn_smem + 4 * R * UB + w * (R * 256);
   const uint32_t words0 = lds_at(words);
   uint32_t voff[KU];
@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
   int iblk = blk, ir0 = blk * B, iu = 0, fill = 0, wfill = 0;
   auto issue = [&]() {
     if (iblk >= nb) return;
-    if (extra && iu == 0) {
+    if (WORDS && iu == 0) {
       ring_word_at(rows.word(ir0), words0 + wfill * 256);
       wfill = wfill + 1 == R ? 0 : wfill + 1;
     }
@@ -262,7 +262,7 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
         // place the next one takes
         constexpr int LATER = KU * (R - 2);
         if (iblk >= nb) ring_wait<0>();
-        else if (NU == 1 && extra) ring_wait<LATER + R - 2>();       // (more units a row: a word of the next rows, too, now and then)
+        else if (NU == 1 && WORDS) ring_wait<LATER + R - 2>();       // (more units a row: a word of the next rows, too, now and then)
         else ring_wait<LATER>();
         issue();
         const char* img = ring + slot * UB + col * (KU * 64);
@@ -274,7 +274,7 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
         }
         slot = slot + 1 == R ? 0 : slot + 1;
       }
-      if (extra) {
+      if constexpr (WORDS) {
         v = rows.finish(v, r0, words + wslot * 256);
         wslot = wslot + 1 == R ? 0 : wslot + 1;
       }
@@ -940,7 +940,8 @@ CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, c
 #define KS(KC)                                                                                                             \
   if constexpr (KC > 4)                                                                                                    \
     if (knn_aligned(X) && (KC > 16 || bytes > KNN_STREAM_BYTES)) {                                                         \
-      knn_stream_kernel<KC, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B);                     \
+      if (xnorm2 || alive) knn_stream_kernel<KC, false, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B); \
+      else knn_stream_kernel<KC, false, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B);         \
       break;                                                                                                               \
     }                                                                                                                      \
   knn_scan_kernel<KC, false><<<KC <= 16 && bytes <= KNN_ROUND_BYTES ? min(all, KNN_ROUND) : all, 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B); \
@@ -958,7 +959,8 @@ CFC_API int cfc_knn_maxima(const void* X, const void* Q, int N, int nq, int dim,
 #define KS(KC)                                                                                                              \
   if constexpr (KC > 4)                                                                                                     \
     if (knn_aligned(X)) {                                                                                                   \
-      knn_stream_kernel<KC, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);                   \
+      if (xnorm2 || alive) knn_stream_kernel<KC, true, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64); \
+      else knn_stream_kernel<KC, true, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);       \
       break;                                                                                                                \
     }                                                                                                                       \
   knn_scan_kernel<KC, true><<<all, 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);                                       \

@@ -23,4 +23,4 @@ def test_index_rows_norms_and_masks_come_by_the_stream(tmp_path):
                 at = body.index("global_load_lds_dword")
                 assert not re.search(r"\sglobal_load_(?!lds)", body[at:]), name
                 assert not re.search(r"\sscratch_(load|store)", body), name
-    assert found == 10
+    assert found == 20

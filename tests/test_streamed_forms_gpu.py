@@ -27,8 +27,6 @@ def test_search(dim, N, lo, form):
     g = torch.Generator(device=DEV).manual_seed(N + lo)
     X, Q = (torch.randn(n, dim, device=DEV, generator=g).bfloat16() for n in (N, 3))
     if form == "rows":
-        if N > 5000:
-            pytest.skip("rows from memory to registers: the smaller ones show it")
         X = _shifted(X)
     xn, qn = (t.float().pow(2).sum(1) if form in ("l2", "both") else None for t in (X, Q))
     alive = torch.rand(N, device=DEV, generator=g) > 0.3 if form in ("mask", "both") else None
