@@ -279,12 +279,13 @@ double prompt_best(int M, int N, int K, int kind, int* plan) {
   if (all < best) best = all, plan[1] = bm, plan[2] = split;
   const int rounds = (int)((int64_t)tm * tn / MG_CUS), head = rounds ? (int)((int64_t)MG_CUS * rounds / tn) * 256 : 0;
   if (head > 0 && head < M && K >= 128) {
-    // behind another launch its own start is hidden, and W waits in the 256 MB cache for a row tile or two (tails of 1 to 128 rows of
-    // 28672 x 4096 40 to 49 us, alone 58; of 679 of 4096 x 2048 19, alone 24)
+    // behind another launch its own start is hidden, and W waits in the 256 MB cache for a row tile or two if what the head read and
+    // wrote fits there as well, nearly (1 to 128 rows of 28672 x 4096 behind 512 40 to 49 us, alone 58; 80 of 16384 x 4096 behind 1024
+    // 28, alone 42, behind 7168 46)
     double rest = mgemm_best(M - head, N, K, kind, kind == MG_ACT, false, bm, split) - 3.0;
-    if (M - head <= 256 && weights <= 1 << 27) rest *= 0.8;
+    if (M - head <= 256 && 2 * (weights + (int64_t)head * (N + K)) <= 280ll << 20) rest *= 0.8;
     const double both = ppp_us(head, N, K, kind != MG_ACT) + rest;
-    if (both < best) best = both, plan[0] = head, plan[1] = bm, plan[2] = split;
+    if (both < 0.99 * best) best = both, plan[0] = head, plan[1] = bm, plan[2] = split;       // two launches for less than that: as often a loss
   }
   return best;
 }
