@@ -6,7 +6,8 @@
 // of peak.  What the measurements on this chip said (scripts/bench_dgemm.py --ablate):
 //   * with the MFMAs removed an LDS-ring kernel was exactly as fast -- the limit is how the W bytes
 //     are fetched, not the math;
-//   * an LDS-DMA W ring (4-6 stages in flight per CU) stayed at ~4.1-4.5 TB/s however deep.
+//   * an LDS-DMA W ring of the workgroup's (4-6 stages in flight per CU) stayed at ~4.1-4.5 TB/s however deep.  (Rings of
+//     a wave's own, read once and without barriers, bring keys and index rows at up to 6.8, lds_ring.h: not tried for W.)
 // So here W never touches LDS:
 //
 //   * workgroup = BN/16 compute waves + 2 X-loader waves, tile = ALL M rows (BM = 16/32/64/96/128/256) x BN
