@@ -286,10 +286,12 @@ def decode_waves(D: int, pooled: bool, wgs: int, tiles: int, blocks: int) -> tup
 
 @functools.lru_cache(maxsize=4096)
 def decode_slices(B: int, H: int, G: int, D: int, visible: int, dtype, pooled: bool = False) -> int:
-    """Key slices per row of a decode step, at least eight 32-key tiles each.  MFMA kernels: from 384 items on one slice where few
-    keys are seen, else 1024 in all: what more gain grows with the longest row, whose keys are one workgroup's work, and the rows'
-    differences.  Fewer: at most 768 in all, and as many as :func:`streamed_us` finds fastest.  us of 8 key heads with 768 and with
-    this many: 24 of 512 keys 14.8 -> 11.2, 24 of 2048 38.1 -> 32.0, 12 of 1024 14.5 -> 14.0.  One row, and heads of 32 (straight to registers): as many as there are.  Others: about four workgroups per CU."""
+    """Key slices per row of a decode step, of eight 32-key tiles and more (the last may have fewer).  MFMA kernels: from 384 items on one
+    slice where few keys are seen, else 1024 in all: what more gain grows with the longest row, whose keys are one workgroup's work, and
+    the rows' differences (1.0 % more than the best of one to three slices on average of 224 measured, heads of 128).  Fewer: at most 768
+    in all, and as many as :func:`streamed_us` finds fastest; us of 8 key heads with 768 and with this many: 24 of 512 keys 14.8 -> 11.2,
+    24 of 2048 38.1 -> 32.0, 12 of 1024 14.5 -> 14.0.  One row, and heads of 32 (straight to registers): as many as there are.  Others:
+    about four workgroups per CU."""
     if dtype != torch.bfloat16 or D not in MFMA_DIMS:
         return max(1, min(math.ceil(1024 / (B * math.ceil(H / ANY_ROWS))), visible // 256, MAX_PARTITIONS))
     items = B * G * math.ceil(H / G / 16)
@@ -298,7 +300,7 @@ def decode_slices(B: int, H: int, G: int, D: int, visible: int, dtype, pooled: b
     most = max(1, min(math.ceil((768 if items < 384 else 1024) / items), visible // 256, MAX_PARTITIONS))
     if items >= 384 or B == 1 or D <= 32:
         return most
-    most = max(1, min(math.ceil(768 / items), math.ceil(visible / 256), MAX_PARTITIONS))      # (the last slice may have fewer tiles)
+    most = max(1, min(math.ceil(768 / items), math.ceil(visible / 256), MAX_PARTITIONS))
     tiles = math.ceil(visible / 32)
     return min(range(1, most + 1), key=lambda P: streamed_us(tiles, items, 128 * D, B * H, P, *decode_waves(D, pooled, items * P, math.ceil(tiles / P), tiles)))
 
