@@ -1691,7 +1691,6 @@ __global__ void __launch_bounds__(256, D == 32 ? (ENC_R == 4 ? 4 : 6) : 2) encod
 
 }  // namespace
 
-// q: [B, Hq, 128] bf16; caches per layer as documented above; out: [B, Hq, 128] bf16.
 // Waves of a workgroup of the paged decode attention of `seen` blocks of a table in P slices, less than zero: those of
 // paged_decode_kernel, keys and values straight to registers.  By the ring 128 KB are under way in a CU, in the eight waves of one
 // workgroup (four with rings of twice the depth: 24 of 1500 28.1 us against 25.7, 16 of 700 14.5 against 13.8) or the four of each of two (two
@@ -1708,6 +1707,7 @@ constexpr int paged_waves(int64_t wgs, int seen, int P, int max_blocks) {
   return wgs <= 64 ? 4 : wgs <= 256 ? 8 : max_blocks > 2 ? 4 : 1;
 }
 
+// q: [B, Hq, 128] bf16; caches per layer as documented above; out: [B, Hq, 128] bf16.
 // part_o / part_ml: fp32 workspaces of B*Hq*P*128 and B*Hq*P*2 floats (unused when P == 1).
 template <bool F8>
 static int launch_paged_decode(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_tables,

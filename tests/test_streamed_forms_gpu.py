@@ -3,6 +3,8 @@ sixteens of bytes, masks at any byte, sixteen query heads a key head; and encode
 import pytest
 import torch
 
+import test_gqa_stream_gpu as stream
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
@@ -89,7 +91,7 @@ def test_paged_queries_at_any_element(P):
     assert bool(((got.double() - want.double()).abs() <= 2.0 ** -8 * want.double().abs() + 2.0 ** -8).all())
 
 
-# keys straight to registers and by the ring, one and several to a slice, pooled means and a window
+# keys straight to registers and by the ring, one and several to a slice
 @pytest.mark.parametrize("D", [32, 64, 96, 128, 160, 192, 256])
 @pytest.mark.parametrize("B,P", [(3, 1), (3, 7), (40, 1), (40, 2), (70, 1)])
 @pytest.mark.parametrize("shift", [False, True])
@@ -110,6 +112,14 @@ def test_grouped(D, B, P, shift):
         k, v = (t[bt[s].long()].transpose(0, 1).reshape(8, -1, D)[:, :ctx[s]].double() for t in (rows.k, rows.v))
         p = torch.softmax((q[s].double().view(8, 3, 1, D) * k[:, None]).sum(-1) / gqa.LOG2E, -1)
         _close(out[s].view(8, 3, D), torch.matmul(p, v), torch.matmul(p, v.abs()).max())
+
+
+# the same with windows, kept tokens, pooled means and biases: queries at any element send every form straight to registers
+@pytest.mark.parametrize("case", stream.CASES)
+def test_grouped_forms_straight(case, monkeypatch):
+    attention = stream.A.attention
+    monkeypatch.setattr(stream.A, "attention", lambda a, q, *rest, **kw: attention(a, _shifted(q), *rest, **kw))
+    stream.test_decoded_tokens_by_the_stream(case)
 
 
 @pytest.mark.parametrize("D", [32, 64])
