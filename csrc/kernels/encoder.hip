@@ -80,6 +80,19 @@ __device__ __forceinline__ void en_gelu(Gelu& g, float& v) {
   }
 }
 
+// of a whole accumulator, part by part: one value's chain of operations is the others' waits
+template <int N>
+__device__ __forceinline__ void en_gelus(float __attribute__((ext_vector_type(N))) & a) {
+  Gelu ge[N];
+  float v[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) v[e] = a[e], en_gelu<0>(ge[e], v[e]);
+#pragma unroll
+  for (int e = 0; e < N; ++e) en_gelu<1>(ge[e], v[e]);
+#pragma unroll
+  for (int e = 0; e < N; ++e) en_gelu<2>(ge[e], v[e]), a[e] = v[e];
+}
+
 // Sixteen columns of a row block between its two layouts, its own inverse.  Accumulators: a lane holds columns
 // 4 hi + 0..3 and 8 + 4 hi + 0..3 (hi = lane >> 5); operands: columns 8 hi + 0..7.
 __device__ __forceinline__ u32x4_t trade(u32x4_t v) {
@@ -613,10 +626,12 @@ __global__ void __launch_bounds__(256, 1)
 
 // ================================================================ few rows
 // A query or a few texts would leave most CUs idle above, and one CU brings in no more than some 30 bytes a
-// nanosecond: a layer's 3.5 MB of weights have to be spread over many.  All four products run in tiles of 64 rows and
+// nanosecond: a layer's 3.5 MB of weights have to be spread over many.  All four products run in tiles of 16 or 32 rows and
 // 64 or 16 columns; what a LayerNorm follows leaves unnormed, and every tile of the next product norms its rows itself
-// (a launch less, and rows that few are in every L2).  A query of 12 tokens takes 27 us a layer, attention
-// included, where tiles of 256 and 128 rows took 75.
+// (a launch less, and rows that few are in every L2).  A launch of so little is one wait for memory after another, so a
+// workgroup asks for all that it reads at once: rows in batches took a wait each, and 64 of them to a tile the norms of all of
+// them in each of 24 tiles (us of a launch, 73 rows: up product 12.2 -> 4.6, down 11.4 -> 5.1, query, key and value 11.1 -> 4.6;
+// six layers of MiniLM, 73 / 150 / 300 rows: 192 / 199 / 206 -> 130 / 134 / 167).
 
 // What the next product reads: x, or LN(proj + bias + res) rounded to bf16, which the first column's tiles also
 // store to x for the next residual.
@@ -625,137 +640,300 @@ struct EncNorm {
   float eps;
 };
 
-// y = x W^T + b (GELU: x Phi(x) of it) for a 384-wide x and a W of N rows.  A wave owns 16 columns: its fragments of W
-// go straight to registers, all in flight before the tile's rows are staged.
-template <bool GELU, bool LN>
-__global__ void __launch_bounds__(256) enc_tile_kernel(uint16_t* x, EncNorm ln, const uint16_t* __restrict__ W,
+__device__ __forceinline__ float row16_sum(float v) {
+  v += row_ror<8>(v);
+  v += row_ror<4>(v);
+  v += row_ror<2>(v);
+  return v + row_ror<1>(v);
+}
+
+// p: LN(v + bias + q) of a row in bf16, sixteen lanes a row, three chunks each
+__device__ __forceinline__ void en_norm16(float (&v)[24], uint4 (&p)[3], const uint4 (&q)[3], const uint4 (&bias)[3],
+                                          const uint4 (&gamma)[3], const uint4 (&beta)[3], float eps) {
+  float s = 0.f, d2 = 0.f;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    float t[8], b[8];
+    unpack8(q[j], t);
+    unpack8(bias[j], b);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[8 * j + i] = v[8 * j + i] + b[i] + t[i];
+      s += v[8 * j + i];
+    }
+  }
+  const float mean = row16_sum(s) * (1.f / EN_H);
+#pragma unroll
+  for (int i = 0; i < 24; ++i) {
+    v[i] -= mean;
+    d2 = fmaf(v[i], v[i], d2);
+  }
+  const float rstd = rsqrtf(row16_sum(d2) * (1.f / EN_H) + eps);
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    float ga[8], be[8];
+    unpack8(gamma[j], ga);
+    unpack8(beta[j], be);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[8 * j + i] = fmaf(v[8 * j + i] * rstd, ga[i], be[i]);
+    p[j] = pack8(v + 8 * j);
+  }
+}
+
+// y = x W^T + b (GELU: x Phi(x) of it) for a 384-wide x and a W of N rows, in tiles of 16 RG rows and 16 WAVES columns.  A wave
+// owns 16 columns: its fragments of W go straight to registers, all in flight with all of the tile's rows.
+template <bool GELU, bool LN, int RG, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) enc_tile_kernel(uint16_t* x, EncNorm ln, const uint16_t* __restrict__ W,
                                                        const uint16_t* __restrict__ bias, uint16_t* __restrict__ out, int M, int N) {
   constexpr int CH = EN_H / 8, KS = EN_H / 32;    // 16-byte chunks of a row, k steps
-  __shared__ __attribute__((aligned(16))) char smem[64 * EN_H * 2];
+  constexpr int B = 4 * RG / WAVES;               // rows of a lane group: four rows a wave at a time, 16 lanes each
+  static_assert(4 * RG % WAVES == 0 && CH == 48);
+  __shared__ __attribute__((aligned(16))) char smem[16 * RG * EN_H * 2];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 64 + 16 * w, m0 = blockIdx.y * 64, rows = min(64, M - m0);
-  uint4 wf[KS];
+  const int n0 = (blockIdx.x * WAVES + w) * 16, m0 = blockIdx.y * 16 * RG, rows = min(16 * RG, M - m0);
+  uint4 wf[KS], p[B][3], q[B][3];
+  // row 4 (w + WAVES b) + g, its chunks r16 + 16 j
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const size_t at = (size_t)(m0 + min(4 * (w + WAVES * b) + g, rows - 1)) * EN_H + 8 * r16;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      p[b][j] = *reinterpret_cast<const uint4*>((LN ? ln.proj : x) + at + 128 * j);
+      if constexpr (LN) q[b][j] = *reinterpret_cast<const uint4*>(ln.res + at + 128 * j);
+    }
+  }
   const uint16_t* wr = W + (size_t)(n0 + r16) * EN_H + 8 * g;
+  uint4 vb[3], vg[3], ve[3];
+  if constexpr (LN) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      vb[j] = *reinterpret_cast<const uint4*>(ln.bias + 8 * r16 + 128 * j);
+      vg[j] = *reinterpret_cast<const uint4*>(ln.gamma + 8 * r16 + 128 * j);
+      ve[j] = *reinterpret_cast<const uint4*>(ln.beta + 8 * r16 + 128 * j);
+    }
+  }
 #pragma unroll
   for (int k = 0; k < KS; ++k) wf[k] = *reinterpret_cast<const uint4*>(wr + 32 * k);
   const uint2 bb = *reinterpret_cast<const uint2*>(bias + n0 + 4 * g);
+  __builtin_amdgcn_sched_barrier(0);
   // chunk c of row r at slot c ^ (r & 7): 16-row fragment reads without bank conflicts
-  if constexpr (LN) {
-    // a wave per row, chunk `lane` of it in lanes 0 .. 47; four rows' loads at a time
-    const bool on = lane < CH;
-    const int c = on ? lane : 0;
-    float pb[8], ga[8], be[8];
-    unpack8(*reinterpret_cast<const uint4*>(ln.bias + 8 * c), pb);
-    unpack8(*reinterpret_cast<const uint4*>(ln.gamma + 8 * c), ga);
-    unpack8(*reinterpret_cast<const uint4*>(ln.beta + 8 * c), be);
-    for (int r0 = w; r0 < rows; r0 += 16) {
-      uint4 p[4], q[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const size_t at = (size_t)(m0 + min(r0 + 4 * u, rows - 1)) * EN_H + 8 * c;
-        p[u] = *reinterpret_cast<const uint4*>(ln.proj + at);
-        q[u] = *reinterpret_cast<const uint4*>(ln.res + at);
-      }
+  for (int b = 0; b < B; ++b) {
+    const int r = 4 * (w + WAVES * b) + g;
+    if constexpr (LN) {
+      float v[24];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int r = r0 + 4 * u;
-        float v[8], t[8], s = 0.f, d2 = 0.f;
-        unpack8(p[u], v);
-        unpack8(q[u], t);
+      for (int j = 0; j < 3; ++j) unpack8(p[b][j], v + 8 * j);
+      en_norm16(v, p[b], q[b], vb, vg, ve, ln.eps);
+      if (blockIdx.x == 0 && r < rows)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          v[j] = on ? v[j] + pb[j] + t[j] : 0.f;
-          s += v[j];
-        }
-        const float mean = wave_sum(s) * (1.f / EN_H);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) d2 += on ? (v[j] - mean) * (v[j] - mean) : 0.f;
-        const float rstd = rsqrtf(wave_sum(d2) * (1.f / EN_H) + ln.eps);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (v[j] - mean) * rstd * ga[j] + be[j];
-        if (on && r < rows) {
-          const uint4 y = pack8(v);
-          *reinterpret_cast<uint4*>(smem + r * (EN_H * 2) + ((c ^ (r & 7)) << 4)) = y;
-          if (blockIdx.x == 0) *reinterpret_cast<uint4*>(x + (size_t)(m0 + r) * EN_H + 8 * c) = y;
-        }
-      }
+        for (int j = 0; j < 3; ++j) *reinterpret_cast<uint4*>(x + (size_t)(m0 + r) * EN_H + 8 * r16 + 128 * j) = p[b][j];
     }
-  } else {
-    for (int id = threadIdx.x; id < rows * CH; id += 256) {
-      const int r = id / CH, c = id - r * CH;
-      *reinterpret_cast<uint4*>(smem + r * (EN_H * 2) + ((c ^ (r & 7)) << 4)) =
-          *reinterpret_cast<const uint4*>(x + (size_t)(m0 + r) * EN_H + 8 * c);
-    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) *reinterpret_cast<uint4*>(smem + r * (EN_H * 2) + (((r16 + 16 * j) ^ (r & 7)) << 4)) = p[b][j];
   }
   __syncthreads();
   const float b[4] = {__uint_as_float(bb.x << 16), __uint_as_float(bb.x & 0xffff0000u), __uint_as_float(bb.y << 16),
                       __uint_as_float(bb.y & 0xffff0000u)};
+  f32x4_t acc[RG];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (16 * i >= rows) break;                    // rows past `rows` of the last group: stale LDS, not stored
-    f32x4_t acc = {b[0], b[1], b[2], b[3]};
+  for (int i = 0; i < RG; ++i) acc[i] = f32x4_t{b[0], b[1], b[2], b[3]};
 #pragma unroll
-    for (int k = 0; k < KS; ++k) {
+  for (int k = 0; k < KS; ++k)
+#pragma unroll
+    for (int i = 0; i < RG; ++i) {                // rows past `rows` repeat the last one and are not stored
       const uint4 xv = *reinterpret_cast<const uint4*>(smem + (16 * i + r16) * (EN_H * 2) + (((4 * k + g) ^ (r16 & 7)) << 4));
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[k]), __builtin_bit_cast(bf16x8_t, xv), acc, 0, 0, 0);
+      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[k]), __builtin_bit_cast(bf16x8_t, xv), acc[i], 0, 0, 0);
     }
-    if constexpr (GELU) {
-      Gelu ge;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float v = acc[e];
-        en_gelu<0>(ge, v);
-        en_gelu<1>(ge, v);
-        en_gelu<2>(ge, v);
-        acc[e] = v;
-      }
+  for (int i = 0; i < RG; ++i) {
+    if constexpr (GELU) {
+      en_gelus(acc[i]);
     }
     if (16 * i + r16 < rows)
-      *reinterpret_cast<uint2*>(out + (size_t)(m0 + 16 * i + r16) * N + n0 + 4 * g) = make_uint2(pack2bf(acc[0], acc[1]), pack2bf(acc[2], acc[3]));
+      *reinterpret_cast<uint2*>(out + (size_t)(m0 + 16 * i + r16) * N + n0 + 4 * g) = make_uint2(pack2bf(acc[i][0], acc[i][1]), pack2bf(acc[i][2], acc[i][3]));
   }
 }
 
-// y = x W^T for a K-wide x and a W of 384 rows, rounded to bf16: 64 rows x 16 columns a workgroup, a quarter of K per wave
-// with W's and the rows' fragments straight from memory, the quarters summed through LDS.
-template <int K>
+// y = x W^T for a K-wide x and a W of 384 rows, rounded to bf16: 16 RG rows x 16 columns a workgroup, a quarter of K per wave
+// with W's and the rows' fragments straight from memory, all in flight at once, the quarters summed through LDS.
+template <int K, int RG>
 __global__ void __launch_bounds__(256) enc_ksplit_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ W,
                                                          uint16_t* __restrict__ out, int M) {
   constexpr int KS = K / 128;                     // k steps of a wave
-  __shared__ float part[3][4][64][4];
+  __shared__ float part[4][RG][64][4];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 64, rows = min(64, M - m0);
+  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16 * RG, rows = min(16 * RG, M - m0);
   const int k0 = w * (K / 4) + 8 * g;
-  uint4 wf[KS];
-  const uint16_t* wr = W + (size_t)(n0 + r16) * K + k0;
+  uint4 wf[KS], xv[RG][KS];
 #pragma unroll
-  for (int k = 0; k < KS; ++k) wf[k] = *reinterpret_cast<const uint4*>(wr + 32 * k);
-  f32x4_t acc[4];
+  for (int i = 0; i < RG; ++i)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    if (16 * i >= rows) break;
-    const uint16_t* xr = x + (size_t)(m0 + min(16 * i + r16, rows - 1)) * K + k0;
-    uint4 xv[KS];
+    for (int k = 0; k < KS; ++k) xv[i][k] = *reinterpret_cast<const uint4*>(x + (size_t)(m0 + min(16 * i + r16, rows - 1)) * K + k0 + 32 * k);
 #pragma unroll
-    for (int k = 0; k < KS; ++k) xv[k] = *reinterpret_cast<const uint4*>(xr + 32 * k);
+  for (int k = 0; k < KS; ++k) wf[k] = *reinterpret_cast<const uint4*>(W + (size_t)(n0 + r16) * K + k0 + 32 * k);
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4_t acc[RG];
 #pragma unroll
-    for (int k = 0; k < KS; ++k)
-      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[k]), __builtin_bit_cast(bf16x8_t, xv[k]), acc[i], 0, 0, 0);
-  }
-  // wave q takes the sums of row group q
+  for (int i = 0; i < RG; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    if (i != w && 16 * i < rows) *reinterpret_cast<f32x4_t*>(part[w - (w > i)][i][lane]) = acc[i];
+  for (int k = 0; k < KS; ++k)
+#pragma unroll
+    for (int i = 0; i < RG; ++i)
+      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[k]), __builtin_bit_cast(bf16x8_t, xv[i][k]), acc[i], 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < RG; ++i) *reinterpret_cast<f32x4_t*>(part[w][i][lane]) = acc[i];
   __syncthreads();
-  if (16 * w >= rows) return;
-  f32x4_t s = acc[0];
+  // wave q takes the sums of row group q
+  if (w >= RG) return;
+  f32x4_t s = *reinterpret_cast<const f32x4_t*>(part[0][w][lane]);
 #pragma unroll
-  for (int i = 1; i < 4; ++i)
-    if (w == i) s = acc[i];
-#pragma unroll
-  for (int q = 0; q < 3; ++q) s += *reinterpret_cast<const f32x4_t*>(part[q][w][lane]);
+  for (int q = 1; q < 4; ++q) s += *reinterpret_cast<const f32x4_t*>(part[q][w][lane]);
   if (16 * w + r16 < rows)
     *reinterpret_cast<uint2*>(out + (size_t)(m0 + 16 * w + r16) * EN_H + n0 + 4 * g) = make_uint2(pack2bf(s[0], s[1]), pack2bf(s[2], s[3]));
+}
+
+// x = LN(proj + bias + res) of 32-bit projections, sixteen lanes a row (a wave a row took 5.5 and 8.7 us of 4823 and 12184 rows of
+// 16-bit ones where this takes 4.4 and 7.4).
+__global__ void __launch_bounds__(256) enc_norm_kernel(uint16_t* __restrict__ x, const float* __restrict__ proj, EncNorm ln, int M) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
+  const int r = xcd_remap(blockIdx.x, gridDim.x) * 16 + 4 * w + g;      // the XCD that has them from the product
+  const size_t at = (size_t)min(r, M - 1) * EN_H + 8 * r16;
+  float4 f[3][2];
+  uint4 p[3], q[3], vb[3], vg[3], ve[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    f[j][0] = *reinterpret_cast<const float4*>(proj + at + 128 * j);
+    f[j][1] = *reinterpret_cast<const float4*>(proj + at + 128 * j + 4);
+    q[j] = *reinterpret_cast<const uint4*>(ln.res + at + 128 * j);
+    vb[j] = *reinterpret_cast<const uint4*>(ln.bias + 8 * r16 + 128 * j);
+    vg[j] = *reinterpret_cast<const uint4*>(ln.gamma + 8 * r16 + 128 * j);
+    ve[j] = *reinterpret_cast<const uint4*>(ln.beta + 8 * r16 + 128 * j);
+  }
+  float v[24];
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      v[8 * j + 4 * i] = f[j][i].x; v[8 * j + 4 * i + 1] = f[j][i].y;
+      v[8 * j + 4 * i + 2] = f[j][i].z; v[8 * j + 4 * i + 3] = f[j][i].w;
+    }
+  en_norm16(v, p, q, vb, vg, ve, ln.eps);
+  if (r < M)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) *reinterpret_cast<uint4*>(x + at + 128 * j) = p[j];
+}
+
+// ================================================================ between few and many rows
+// From some 300 rows on a tile's norms, made again for each column of tiles, cost more than a launch of their own, and fragments
+// straight from memory bring each row into a CU once per 16 columns (2201 rows: up product 26.9 us, down 30); up to 16 k rows
+// the kernels of 128 rows a workgroup leave CUs without one and the 256-row tiles of the general products leave most.
+// y = x W^T (32-bit: LayerNorm reads it as the matrix cores left it), or x W^T + b, or GELU of that (bf16), in tiles of BM rows
+// and BN columns, both through a ring of NS LDS-DMA stages 64 deep; a wave takes 32 TM rows and 32 TN columns.  K is 6 or 24
+// stages, so a tile is mostly start and end: two or three workgroups a CU cover one another's.  An XCD takes neighbouring rows in
+// every launch of a layer, which then are in its L2 (six layers of 4823 / 12184 rows 386 / 748 -> 342 / 676 us).
+// Six layers of MiniLM before and now: 481 rows 216 -> 187 us, 1218 323 -> 208, 2201 502 -> 239, 4823 721 -> 342, 8000 745 -> 481,
+// 12184 815 -> 669, 16000 838 -> 767.  What bounds it: launches of 3 to 5 us up to 1000 rows; then the LDS, which every MFMA
+// takes 1 to 1.5 KB from, and the GELU (8000 rows: up 19.9 us = 470 TFLOP/s, down 16.0).
+enum { EG_RAW = 0, EG_BIAS = 1, EG_GELU = 2 };
+template <int K, int BM, int BN, int TM, int TN, int NS, int EPI>
+__global__ void __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * 64)
+    enc_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ W, const uint16_t* __restrict__ bias,
+                    void* __restrict__ out, int M, int N) {
+  constexpr int WM = BM / 32 / TM, NW = WM * (BN / 32 / TN), S = K / 64, PIECES = (BM + BN) / 8, PW = PIECES / NW, STAGE = (BM + BN) * 128;
+  static_assert(PIECES % NW == 0 && S >= NS);
+  extern __shared__ __attribute__((aligned(16))) char eg_smem[];
+  const int lane = threadIdx.x & 63, hi = lane >> 5, r32 = lane & 31;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // an XCD takes neighbouring rows, all columns of them
+  const int cols = N / BN, tile = xcd_remap(blockIdx.x, gridDim.x);
+  const int m0 = tile / cols * BM, n0 = tile % cols * BN;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(en_lds_t*)eg_smem);
+  // piece p: rows 8 p .. 8 p + 7 of the tile's BM rows of x, then of its BN rows of W; chunk c of row r at c ^ (r >> 1 & 7)
+  uint32_t voff[PW];
+#pragma unroll
+  for (int i = 0; i < PW; ++i) {
+    const int p = PW * w + i, r = 8 * p + (lane >> 3);
+    const int row = p < BM / 8 ? min(m0 + r, M - 1) : n0 + r - BM;
+    voff[i] = (uint32_t)row * (K * 2) + (((lane & 7) ^ (r >> 1 & 7)) << 4);
+  }
+  auto issue = [&](int st, int slot) {
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      const int p = PW * w + i;
+      en_glds16(voff[i], reinterpret_cast<const char*>(p < BM / 8 ? x : W) + st * 128, lds0 + slot * STAGE + p * 1024);
+    }
+  };
+#pragma unroll
+  for (int st = 0; st < NS - 1; ++st) issue(st, st);
+  const int wm = w % WM, wn = w / WM;
+  f32x16_t acc[TM][TN];
+#pragma unroll
+  for (int b = 0; b < TN; ++b) {
+    f32x16_t a;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint2 v = make_uint2(0, 0);
+      if constexpr (EPI != EG_RAW) v = *reinterpret_cast<const uint2*>(bias + n0 + 32 * (wn * TN + b) + 8 * i + 4 * hi);
+      a[4 * i] = __uint_as_float(v.x << 16); a[4 * i + 1] = __uint_as_float(v.x & 0xffff0000u);
+      a[4 * i + 2] = __uint_as_float(v.y << 16); a[4 * i + 3] = __uint_as_float(v.y & 0xffff0000u);
+    }
+#pragma unroll
+    for (int t = 0; t < TM; ++t) acc[t][b] = a;
+  }
+  uint32_t go[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) go[s] = r32 * 128 + (((2 * s + hi) ^ (r32 >> 1 & 7)) << 4);
+  typedef const __attribute__((address_space(3))) bf16x8_t* lds_frag_t;
+#pragma unroll
+  for (int st = 0; st < S; ++st) {
+    constexpr int AHEAD = NS - 2;
+    // stage st is there in every wave, and stage st - 1 read (the bias was asked for later than the first stages: counted safe)
+    const int left = S - 1 - st < AHEAD ? S - 1 - st : AHEAD;
+    if (left == 0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else if (left == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(PW) : "memory");
+    else if (left == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(2 * PW) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(3 * PW) : "memory");
+    if (st + NS - 1 < S) issue(st + NS - 1, (st + NS - 1) % NS);
+    const uint32_t base = lds0 + (st % NS) * STAGE;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      bf16x8_t fx[TM], fw[TN];
+#pragma unroll
+      for (int t = 0; t < TM; ++t) fx[t] = *reinterpret_cast<lds_frag_t>(base + (wm * TM + t) * 4096 + go[s]);
+#pragma unroll
+      for (int b = 0; b < TN; ++b) fw[b] = *reinterpret_cast<lds_frag_t>(base + BM * 128 + (wn * TN + b) * 4096 + go[s]);
+#pragma unroll
+      for (int t = 0; t < TM; ++t)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[t][b] = mfma32(fw[b], fx[t], acc[t][b]);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < TM; ++t) {
+    const int row = m0 + 32 * (wm * TM + t) + r32;
+#pragma unroll
+    for (int b = 0; b < TN; ++b) {
+      f32x16_t a = acc[t][b];
+      if constexpr (EPI == EG_GELU) {
+        en_gelus(a);
+      }
+      const int n = n0 + 32 * (wn * TN + b);
+      if constexpr (EPI == EG_RAW) {
+        if (row < M)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float4*>((float*)out + (size_t)row * N + n + 8 * i + 4 * hi) = make_float4(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]);
+      } else {
+        const bf16x8_t y0 = frag_of(a, 0), y1 = frag_of(a, 1);
+        if (row < M) {
+          uint16_t* o = (uint16_t*)out + (size_t)row * N + n + 8 * hi;
+          *reinterpret_cast<bf16x8_t*>(o) = y0;
+          *reinterpret_cast<bf16x8_t*>(o + 16) = y1;
+        }
+      }
+    }
+  }
 }
 
 // ================================================================ a query or a few short texts
@@ -1272,14 +1450,14 @@ CFC_API int cfc_encoder_attention(const void* qkv, const int32_t* cu_seqlens, co
                                   int n_tiles, int tile_rows, int H, int head_dim, int max_seqlen, float scale, void* out,
                                   hipStream_t stream);
 
-// A few texts of 64 rows in all: enc_tiny_kernel.  Few rows: up to 2560, where a forward of MiniLM takes 627 us here and 733 in
-// pgemm.hip's tiles (2048 rows: 520 and 732, 3072: 735 and 738).  Many: from 10753, where the tiles need another round of the
-// chip (10752 rows: 866 us here and 817 in tiles, 11008: 867 and 929, 16384: 931 and 1124).  Between them neither is
-// faster than the tiles.
-constexpr int EN_FEW_ROWS = 2560, EN_MANY_ROWS = 10753;
+// A few texts of 64 rows in all: enc_tiny_kernel.  Few: up to 2560 rows.  Many: from 10753, where the general tiles need another
+// round of the chip.  All of these, and with cfc_enc_forward those between, take small tiles up to 320 rows, LDS tiles up to
+// 16383 and the layer's one kernel above (six layers of MiniLM in LDS tiles and in it: 14000 rows 712 and 826 us, 16000 767
+// and 838, 18000 845 and 848).
+constexpr int EN_FEW_ROWS = 2560, EN_MANY_ROWS = 10753, EN_FUSED_ROWS = 16384;
 
-// Which rows this file's kernels take: 1 few, 2 many, 0 neither.
-CFC_API int cfc_enc_rows(int T) { return T <= EN_FEW_ROWS ? 1 : T >= EN_MANY_ROWS ? 2 : 0; }
+// How many rows T are: 1 few, 3 between, 4 many, 2 as many as the layer's one kernel takes, which alone needs no y and h.
+CFC_API int cfc_enc_rows(int T) { return T <= EN_FEW_ROWS ? 1 : T < EN_MANY_ROWS ? 3 : T < EN_FUSED_ROWS ? 4 : 2; }
 
 // Values of workspace (bf16) that the one launch for T rows of a model takes on a stream; 0: it does not take them, or so few
 // CUs are the stream's that its workgroups would be long in coming.
@@ -1292,10 +1470,58 @@ CFC_API int cfc_enc_tiny(int T, int layers, int heads, hipStream_t stream) {
   return cus >= 4 * (EN_HEADS + EN_BLOCKS + EN_INNER) ? layers * T * (3 * EN_H + EN_F) + 8 : 0;
 }
 
+namespace {
+constexpr int EN_CUS = 256;
+
+template <bool GELU, bool LN>
+void en_tile(int groups, uint16_t* x, const EncNorm& ln, const uint16_t* W, const uint16_t* bias, uint16_t* out, int T, int N, hipStream_t stream) {
+  const dim3 grid(N / 64, (T + 16 * groups - 1) / (16 * groups));
+  if (groups == 1) enc_tile_kernel<GELU, LN, 1, 4><<<grid, 256, 0, stream>>>(x, ln, W, bias, out, T, N);
+  else enc_tile_kernel<GELU, LN, 2, 4><<<grid, 256, 0, stream>>>(x, ln, W, bias, out, T, N);
+}
+
+template <int K>
+void en_ksplit(int groups, const uint16_t* x, const uint16_t* W, uint16_t* out, int T, hipStream_t stream) {
+  const dim3 grid(EN_H / 16, (T + 16 * groups - 1) / (16 * groups));
+  if (groups == 1) enc_ksplit_kernel<K, 1><<<grid, 256, 0, stream>>>(x, W, out, T);
+  else enc_ksplit_kernel<K, 2><<<grid, 256, 0, stream>>>(x, W, out, T);
+}
+
+template <int K, int BM, int BN, int TM, int TN, int NS, int EPI>
+void en_gemm(const uint16_t* x, const uint16_t* W, const uint16_t* bias, void* out, int T, int N, hipStream_t stream) {
+  constexpr int LDS = NS * (BM + BN) * 128;
+  if constexpr (LDS > 64 * 1024) {
+    static const hipError_t raised =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&enc_gemm_kernel<K, BM, BN, TM, TN, NS, EPI>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    (void)raised;
+  }
+  enc_gemm_kernel<K, BM, BN, TM, TN, NS, EPI><<<N / BN * ((T + BM - 1) / BM), 64 * (BM / 32 / TM) * (BN / 32 / TN), LDS, stream>>>(x, W, bias, out, T, N);
+}
+
+// The tiles of the products of 384-wide rows with 1152 or 1536 columns, and of those that leave 384 columns: the largest whose
+// workgroups, of which as many fit a CU as the LDS has rings for, are about one round of the chip.  Us of six layers with 64 x 64
+// / 64 x 128 / 128 x 128 tiles of the wide products: 1000 rows 197 / 212 / 228, 1800 249 / 245 / 252, 3600 320 / 303 / 310,
+// 4823 366 / 353 / 340, 9500 593 / 550 / 532, 16000 903 / 810 / 776; of the down product: 2560 247 / 263 / 278, 3000 286 / 278 /
+// 292, 6500 451 / 452 / 434, 9500 568 / 551 / 540, 11000 659 / 657 / 668.
+template <int EPI>
+void en_wide(const uint16_t* x, const uint16_t* W, const uint16_t* bias, uint16_t* out, int T, int N, hipStream_t stream) {
+  if (T <= 1280) en_gemm<EN_H, 64, 64, 1, 1, 4, EPI>(x, W, bias, out, T, N, stream);
+  else if (T <= 4096) en_gemm<EN_H, 64, 128, 1, 2, 2, EPI>(x, W, bias, out, T, N, stream);
+  else en_gemm<EN_H, 128, 128, 2, 2, 2, EPI>(x, W, bias, out, T, N, stream);
+}
+
+template <int K>
+void en_raw(const uint16_t* x, const uint16_t* W, void* y, int T, hipStream_t stream) {
+  if (T <= 2688) en_gemm<K, 64, 64, 1, 1, 4, EG_RAW>(x, W, nullptr, y, T, EN_H, stream);
+  else if (K == EN_F && T > 5440 && T <= 10880) en_gemm<EN_F, 128, 128, 1, 2, 3, EG_RAW>(x, W, nullptr, y, T, EN_H, stream);
+  else en_gemm<K, 64, 128, 1, 2, 3, EG_RAW>(x, W, nullptr, y, T, EN_H, stream);
+}
+}  // namespace
+
 // Token states of a packed batch: embeddings, then every layer, one call for all launches.  W: host array of twelve
 // device pointers per layer (qkv, qkv_b, o, o_b, ln1_g, ln1_b, up, up_b, down, down_b, ln2_g, ln2_b).  x [T][384] the
-// states; att [T][384], qkv [T][1152], and for few rows y [T][384] and h [T][1536]: workspace.  All bf16 and 16-byte
-// aligned.  With att null, h is the workspace of cfc_enc_tiny and no other is read; a wait in that launch is given up after
+// states; att [T][384], qkv [T][1152], and unless cfc_enc_rows is 2 y [T][384] of 32 bits and h [T][1536]: workspace.  All else
+// bf16, all 16-byte aligned.  With att null, h is the workspace of cfc_enc_tiny and no other is read; a wait in that launch is given up after
 // `polls` loads (below 0: EN_POLLS).
 CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* word, const void* pos_emb, const void* type_emb,
                             const void* emb_g, const void* emb_b, const int32_t* cu, const int32_t* tile_seq, const int32_t* tile_q0,
@@ -1322,38 +1548,47 @@ CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* 
 #undef TINY
     return CFC_CHECK_LAUNCH();
   }
-  if (T < 1 || layers < 1 || heads < 1 || EN_H % heads || kind == 0 || (kind == 1 && (h == nullptr || y == nullptr))) return -1;
+  if (T < 1 || layers < 1 || heads < 1 || EN_H % heads || (kind != 2 && (h == nullptr || y == nullptr))) return -1;
   int rc = cfc_layernorm(x, word, nullptr, nullptr, emb_g, emb_b, ids, pos, pos_emb, type_emb, T, EN_H, eps, 2, stream);
   uint16_t *xp = (uint16_t*)x, *yp = (uint16_t*)y, *ap = (uint16_t*)att, *qp = (uint16_t*)qkv, *hp = (uint16_t*)h;
-  const int blocks = (T + EN_ROWS - 1) / EN_ROWS, tiles = (T + 63) / 64;
+  const int blocks = (T + EN_ROWS - 1) / EN_ROWS;
   const uint16_t* const* P = (const uint16_t* const*)W;
+  // Small tiles of 16 or 32 rows while a round of the chip takes those of the widest product's 24 columns (160 / 161 rows: 134 /
+  // 161 us; of 16 rows still: 161), else tiles by way of the LDS (300 rows 167 in small tiles and 187; 350 rows 186 and 187)
+  const int small = (T + 15) / 16 * 24 <= EN_CUS ? 1 : (T + 31) / 32 * 24 <= EN_CUS ? 2 : 0;
+  auto attend = [&]() { return cfc_encoder_attention(qkv, cu, tile_seq, tile_q0, n_tiles, tile_rows, heads, EN_H / heads, max_seqlen, scale, att, stream); };
   for (int l = 0; l < layers && rc == 0; ++l) {
     const uint16_t* const* p = P + 12 * l;
-    const dim3 gq(3 * EN_H / 64, tiles), gu(EN_F / 64, tiles), gk(EN_H / 16, tiles);
-    // few rows: a sublayer's last product waits in y for the next tiles' norm, which puts the layer's states in x, those
-    // between its sublayers in att (the attention's output is used up by then)
-    if (kind == 2)
-      if (T > 256 * EN_ROWS)          // more than a workgroup of 128 rows a CU
+    if (kind == 2) {
+      if (T > EN_CUS * EN_ROWS)       // more than a workgroup of 128 rows a CU
         enc_proj_wide_kernel<<<(T + EW_ROWS - 1) / EW_ROWS, 256, 0, stream>>>(xp, p[0], p[1], qp, T);
       else
         enc_proj_kernel<<<blocks, 256, 0, stream>>>(xp, p[0], p[1], qp, T, 3 * EN_T);
-    else if (l == 0)
-      enc_tile_kernel<false, false><<<gq, 256, 0, stream>>>(xp, EncNorm{}, p[0], p[1], qp, T, 3 * EN_H);
-    else
-      enc_tile_kernel<false, true><<<gq, 256, 0, stream>>>(xp, EncNorm{yp, p[-3], ap, p[-2], p[-1], eps}, p[0], p[1], qp, T, 3 * EN_H);
-    rc = cfc_encoder_attention(qkv, cu, tile_seq, tile_q0, n_tiles, tile_rows, heads, EN_H / heads, max_seqlen, scale, att, stream);
-    if (rc) break;
-    if (kind == 2) {
+      if ((rc = attend())) break;
       const EncLayer L = {p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], p[10], p[11]};
       enc_layer_kernel<<<blocks, 512, EN_LDS, stream>>>(ap, xp, L, xp, T, eps);
+    } else if (small) {
+      // a sublayer's last product waits in y for the next tiles' norm, which puts the layer's states in x, those between its
+      // sublayers in att (the attention's output is used up by then)
+      const EncNorm first = l ? EncNorm{yp, p[-3], ap, p[-2], p[-1], eps} : EncNorm{}, second = {yp, p[3], xp, p[4], p[5], eps};
+      if (l == 0) en_tile<false, false>(small, xp, first, p[0], p[1], qp, T, 3 * EN_H, stream);
+      else en_tile<false, true>(small, xp, first, p[0], p[1], qp, T, 3 * EN_H, stream);
+      if ((rc = attend())) break;
+      en_ksplit<EN_H>(small, ap, p[2], yp, T, stream);
+      en_tile<true, true>(small, ap, second, p[6], p[7], hp, T, EN_F, stream);
+      en_ksplit<EN_F>(small, hp, p[8], yp, T, stream);
     } else {
-      enc_ksplit_kernel<EN_H><<<gk, 256, 0, stream>>>(ap, p[2], yp, T);
-      enc_tile_kernel<true, true><<<gu, 256, 0, stream>>>(ap, EncNorm{yp, p[3], xp, p[4], p[5], eps}, p[6], p[7], hp, T, EN_F);
-      enc_ksplit_kernel<EN_F><<<gk, 256, 0, stream>>>(hp, p[8], yp, T);
+      en_wide<EG_BIAS>(xp, p[0], p[1], qp, T, 3 * EN_H, stream);
+      if ((rc = attend())) break;
+      en_raw<EN_H>(ap, p[2], y, T, stream);
+      enc_norm_kernel<<<(T + 15) / 16, 256, 0, stream>>>(ap, (const float*)y, EncNorm{nullptr, p[3], xp, p[4], p[5], eps}, T);
+      en_wide<EG_GELU>(ap, p[6], p[7], hp, T, EN_F, stream);
+      en_raw<EN_F>(hp, p[8], y, T, stream);
+      enc_norm_kernel<<<(T + 15) / 16, 256, 0, stream>>>(xp, (const float*)y, EncNorm{nullptr, p[9], ap, p[10], p[11], eps}, T);
     }
   }
   if (rc) return rc;
-  if (kind == 1) {
+  if (kind != 2 && small) {
     const uint16_t* const* p = P + 12 * layers;
     return cfc_layernorm(x, y, p[-3], att, p[-2], p[-1], nullptr, nullptr, nullptr, nullptr, T, EN_H, eps, 1, stream);
   }

@@ -55,6 +55,27 @@ def test_rows_against_float64(lens):
     assert rel < 2.0 ** -9 * (3 * 10) ** 0.5, float(rel)
 
 
+@pytest.mark.parametrize("T", [159, 160, 161, 319, 320, 321, 1279, 1280, 1281, 2687, 2688, 2689, 4095, 4096, 4097, 5440, 5441, 10752, 10753,
+                               10880, 10881, 12161, 16383])
+def test_rows_at_the_edges_of_the_tiles_rules(T):
+    """Where the next larger tiles take over, with last tiles of one row, of all but one and of all."""
+    import dataclasses
+    from copilot_for_consensus_amd.models.encoder import get_encoder_config
+    from copilot_for_consensus_amd.ops import kernels as K
+    m = _model(dataclasses.replace(get_encoder_config("minilm-l6"), layers=2), seed=T)
+    lens = [250] * (T // 250) + [T % 250]
+    g = torch.Generator(device=DEV).manual_seed(T)
+    ids = torch.randint(0, m.cfg.vocab_size, (T,), device=DEV, dtype=torch.int32, generator=g)
+    pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).to(DEV)
+    cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).to(torch.int32)
+    tiles = tuple(torch.tensor(t, dtype=torch.int32, device=DEV) for t in K.prefill_tiles(cu.tolist(), K.ENCODER_TILE_ROWS))
+    assert K.encoder_weights(T, m.p, m.layers, m.cfg.heads, 250, between=True) is not None
+    got = m.forward_packed(ids, pos, cu.to(DEV), 250, tiles=tiles).double()
+    want = _states(m, ids.long(), lens)
+    rel = ((got - want).norm(dim=1) / want.norm(dim=1)).max()
+    assert rel < 2.0 ** -9 * (2 * 10) ** 0.5, float(rel)        # roundings as above
+
+
 def test_what_the_kernels_are_not_built_for():
     """Other shapes, types and alignments keep the general path."""
     from copilot_for_consensus_amd.models.encoder import EncoderModel
