@@ -48,9 +48,10 @@ typedef __attribute__((address_space(3))) void dg_lds_t;
 typedef unsigned int dg_u32x4 __attribute__((ext_vector_type(4)));
 
 // X-loader waves per workgroup: fill the workgroup up to 8 waves (2 per SIMD, 256 VGPRs each), at
-// least one
+// least one; two beside seven, though their ring of W is shorter for it (28672 x 4096 of 5 / 32 / 64 / 128 rows, us: 36.4 / 36.7 /
+// 38.6 / 50.8 by one, 35.8 / 36.4 / 38.2 / 50.5 by two)
 template <int BN>
-constexpr int dg_loaders() { return BN / 16 >= 7 ? 1 : 8 - BN / 16 > 2 ? 2 : 8 - BN / 16; }
+constexpr int dg_loaders() { return BN / 16 >= 8 ? 1 : 2; }
 // DG_PART_WT: the split-K slabs stored write-through (sc1): they reach memory while the kernel
 // runs instead of as dirty L2 lines the kernel boundary must write back before the consumer (the
 // residual + RMSNorm reduce, rope_kv) may start -- MI355X_MICROARCH "boundary": +B / 6 TB/s behind
@@ -62,7 +63,7 @@ struct DgGlu { float limit = 0.f, alpha = 1.f, beta = 0.f, cubic = 0.f; };
 
 // MX (ablation 64): two X-loader waves and an 8-slot X ring whatever BN -- one loader wave's
 // vmcnt window (63 pieces = 3 stages at BM = 128) may cap the X stream of the wide-BN shapes.
-template <int BM, int BN, bool MX = false>
+template <int BM, int BN, bool MX = false, bool EXPERTS = false>
 struct DgShape {
   static constexpr int NW = BN / 16;                  // compute waves
   static constexpr int LOADERS = MX ? 2 : dg_loaders<BN>();
@@ -72,9 +73,12 @@ struct DgShape {
   static constexpr int D = BM == 256 ? 4 : (WAVES > 8 ? 6 : 8);
   static constexpr int XSTAGE = BM * 128;             // X bytes per 64-deep stage
   static constexpr int XP = BM / 8 / LOADERS;         // 1-KB DMA pieces per loader wave per stage
-  // X ring slots (64-128 KB); a loader keeps NSX - 2 stages in flight at its wait, and vmcnt
-  // counts at most 63 of its pieces
-  static constexpr int NSX_BASE = MX ? 8 : (BM == 256 ? 4 : (BM == 128 ? 6 : 8));    // BM 16, 32: a ring of 16 is no faster
+  // X ring slots; a loader keeps NSX - 2 stages in flight at its wait, and vmcnt counts at most 63 of its pieces.  X on its
+  // way takes the place of W on its way: from 64 rows on four slots are faster than more (us of a 7B layer's four products,
+  // 48 / 64 / 96 / 128 rows: 6 or 8 slots 81.9 / 83.4 / 91.0 / 104.6, 5 80.1 / 82.1 / 90.2 / 103.7, 4 79.7 / 81.4 / 89.5 / 103.5, 3 of 128 rows 106;
+  // of 16 rows 8 slots 75.0, 4 75.5); not of experts' matrices, whose workgroups are several rounds (110 rows of pemolorn, a pass of
+  // two steps: 4 slots 1968, more 1949)
+  static constexpr int NSX_BASE = MX ? 8 : BM == 256 ? 4 : BM < 64 ? 8 : !EXPERTS ? 4 : BM == 128 ? 6 : 8;    // BM 16, 32: a ring of 16 is no faster
   static constexpr int NSX = (NSX_BASE - 2 <= 63 / XP ? NSX_BASE : 2 + 63 / XP);
 };
 
@@ -169,7 +173,7 @@ template <int BM, int EPI, int GRP>
 constexpr bool dg_twice() { return BM <= 64 && GRP == 1 && EPI == DG_BF16; }
 
 template <int BM, int BN, int EPI, bool NTW, int ABL = 0, bool PACKED = true, int GRP = 0>
-__global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES), (dg_twice<BM, EPI, GRP>() ? 5 : 1))
+__global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0, GRP == 1>::WAVES), (dg_twice<BM, EPI, GRP>() ? 5 : 1))
     dgemm_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, int M, int N, int K, int ntiles,
                  int split, float* __restrict__ part, uint16_t* __restrict__ out, int ldo, DgGlu gp, DgGroup grp) {
   if constexpr (GRP == 1) {
@@ -177,7 +181,7 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
     if (e < 0) return;
     W += (size_t)e * N * K;
   }
-  using S = DgShape<BM, BN, (ABL & 64) != 0>;
+  using S = DgShape<BM, BN, (ABL & 64) != 0, GRP == 1>;
   constexpr int NW = S::NW;
   constexpr int D = dg_twice<BM, EPI, GRP>() ? 4 : S::D;
   __shared__ __attribute__((aligned(16))) char smem[S::NSX * S::XSTAGE];
@@ -312,7 +316,7 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
   // read past the slice (the tail computes only real stages).
   constexpr bool TAIL_RELOAD = (ABL & 256) != 0;    // probe: the former tail, which reads again
   int st = 0;
-  for (; st + D <= nst; st += D) {
+  auto round = [&]() {
 #pragma unroll
     for (int u = 0; u < D; ++u) {
       if constexpr (!NOBAR) dg_barrier();   // X stage st+u is in LDS
@@ -320,7 +324,9 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0>::WAVES)
       if constexpr (PACKED && !TAIL_RELOAD) load_stage_past(st + u + D, ring[u]);
       else load_stage(phys(min(st + u + D, nst - 1)), ring[u]);
     }
-  }
+    st += D;
+  };
+  while (st + D <= nst) round();
 #pragma unroll
   for (int u = 0; u < D; ++u) {
     if (st + u < nst) {
@@ -703,7 +709,7 @@ template <int BM, int BN>
 void dgemm_group_go(int glu, const void* x, const void* w, int M, int N, int K, void* out, int ldo, const DgGlu& gp,
                     const DgGroup& g, hipStream_t stream) {
   const dim3 grid(N / BN, M / BM);
-  constexpr int threads = 64 * DgShape<BM, BN>::WAVES;
+  constexpr int threads = 64 * DgShape<BM, BN, false, true>::WAVES;
   if (glu)
     dgemm_kernel<BM, BN, DG_GLU, DG_NT, 0, true, 1><<<grid, threads, 0, stream>>>(
         (const uint16_t*)x, (const uint16_t*)w, M, N, K, N / BN, 1, nullptr, (uint16_t*)out, ldo, gp, g);
