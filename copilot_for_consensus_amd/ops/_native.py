@@ -101,6 +101,8 @@ _KERNEL_SIGS = {
     "cfc_prefill_attention_expanded": [P, P, P, P, c_int64, P, P, P, P, I, I, F, P, c_int64, P],
     "cfc_enc_rows": [I],
     "cfc_knn_queries": [P, P, P, I, I, I, P],
+    "cfc_knn_search": [P, P, I, I, I, I, P, P, I, L, P, L, P, P, P],
+    "cfc_knn_search_bytes": [I, I, I],
     "cfc_enc_tiny": [I, I, I, P],
     "cfc_put_ints": [P, P, I, P],
     "cfc_enc_forward": [P] * 10 + [I, I, I, I, P, I, F, F, I] + [P] * 5 + [I, P],
@@ -184,7 +186,7 @@ _RUNTIME_SIGS = {
 
 _RESTYPES = {
     "cfc_bpe_create": c_void_p, "cfc_wp_create": c_void_p, "cfc_blockpool_create": c_void_p,
-    "cfc_mbox_split": c_int64, "cfc_prompt_us": c_double,
+    "cfc_mbox_split": c_int64, "cfc_prompt_us": c_double, "cfc_knn_search_bytes": c_int64,
 }
 
 

@@ -1671,6 +1671,28 @@ def knn_topk(X, Q, k: int, xnorm2=None, qnorm2=None, alive=None, row_lo: int = 0
     return _select(sc, 16 * kb, min(k, n), ids, bmax)
 
 
+def knn_search(X, q, k: int, unit: bool, xnorm2=None, alive=None, row_lo: int = 0, N: int | None = None):
+    """:func:`knn_topk` of fp32 queries ``q`` [nq, dim] on the GPU, of unit length if ``unit``: up to KNN_SCORES rows by one call."""
+    N = X.shape[0] if N is None else N
+    nq, dim, n = q.shape[0], X.shape[1], N - row_lo
+    if not 1 <= k <= 256 or not 1 <= nq <= 16 or not 0 <= row_lo < N <= X.shape[0] or n > KNN_SCORES or _topk_parts(n) > 1:
+        Q, qnorm2 = knn_queries(q, unit)
+        return knn_topk(X, Q, k, xnorm2, qnorm2, alive, row_lo, N)
+    _req(q, torch.float32, "knn_search")
+    if q.shape != (nq, dim):
+        raise ValueError(f"knn_search: queries {tuple(q.shape)} for rows of {dim}")
+    lib, dev, k = kernels(), X.device, min(k, n)
+    room = lib.cfc_knn_search_bytes(n, nq, dim)
+    ws = torch.empty(room, dtype=torch.uint8, device=dev)
+    v = torch.empty(nq, k, dtype=torch.float32, device=dev)
+    i = torch.empty(nq, k, dtype=torch.int64, device=dev)
+    check(lib.cfc_knn_search(X.data_ptr() + row_lo * dim * 2, q.data_ptr(), int(unit), n, nq, dim,
+                             None if xnorm2 is None else xnorm2.data_ptr() + row_lo * 4,
+                             None if alive is None else alive.data_ptr() + row_lo * alive.element_size(), k, row_lo, ws.data_ptr(), room,
+                             v.data_ptr(), i.data_ptr(), _stream(X)), "cfc_knn_search")
+    return v, i
+
+
 def ivf_topk(X, Q, probe: torch.Tensor, list_off: torch.Tensor, maxc: int, k: int, xnorm2=None, qnorm2=None,
              alive=None):
     """IVF scan of the probed lists, one launch for every (query, probe, chunk): candidates

@@ -351,19 +351,19 @@ class HipFlatIndex(VectorStore):
         """Device-side exact search: (scores [nq, k], row indices [nq, k]) for queries Q."""
         from ..ops import kernels as K
         lo, hi = rows if rows is not None else (0, self._n)
-        # floats that lie beside the index need no launch of their own to be rounded
+        # floats that lie beside the index are searched by one call
         beside = (isinstance(Q, torch.Tensor) and Q.is_cuda and Q.device == self._X.device and Q.dtype == torch.float32
                   and Q.dim() == 2 and Q.shape[1] == self.dim and Q.shape[0] > 0 and self.dim % 8 == 0 and Q.is_contiguous()
                   and Q.data_ptr() % 16 == 0 and hi > lo and Q.shape[0] <= 16 and k <= 256)
-        if not beside:
-            Q = _as_matrix(Q, self.dim, device=self.device, dtype=torch.bfloat16)
+        if beside:
+            return K.knn_search(self._X, Q, k, self.metric == "cosine", self._norm2 if self.metric == "l2" else None,
+                                self._alive if self._dead else None, lo, hi)
+        Q = _as_matrix(Q, self.dim, device=self.device, dtype=torch.bfloat16)
         nq = Q.shape[0]
         if hi <= lo:
             return (torch.empty(nq, 0, device=self.device), torch.empty(nq, 0, dtype=torch.long, device=self.device))
         X = self._X[lo:hi]
-        if beside:
-            Qn, qn2 = K.knn_queries(Q, self.metric == "cosine")
-        elif self.metric == "cosine":
+        if self.metric == "cosine":
             Qn = K.l2_normalize(Q.contiguous())
             qn2 = None
         else:

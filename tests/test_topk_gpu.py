@@ -266,3 +266,22 @@ def test_knn_scores_by_the_stream(dim, nq, N, metric):
     v, i = K.knn_topk(X, Q, min(50, N), xn, qn, alive=alive & fine)
     rv, ri = got.masked_fill(~(alive & fine)[None], float("-inf")).sort(dim=1, descending=True, stable=True)
     assert torch.equal(v, rv[:, :min(50, N)]) and torch.equal(i, ri[:, :min(50, N)])
+
+
+@pytest.mark.parametrize("lo,n", [(0, 1), (3, 15), (0, 16), (5, 17), (0, 262144), (1, 262145), (0, 1 << 20), (0, (1 << 20) + 1)])
+@pytest.mark.parametrize("nq,k,unit,dead", [(1, 5, True, False), (3, 256, False, False), (16, 20, True, True), (7, 1, False, True)])
+def test_a_search_by_one_call(lo, n, nq, k, unit, dead):
+    """The same values and rows as from queries, scores and selection one after the other, bit for bit."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(n + nq)
+    X = torch.randn(lo + n + 2, 128, device="cuda", generator=g).bfloat16()
+    q = torch.randn(nq, 128, device="cuda", generator=g)
+    norms = None if unit else X.float().pow(2).sum(1)
+    alive = torch.rand(len(X), device="cuda", generator=g) < 0.9 if dead else None
+    Q, n2 = K.knn_queries(q, unit)
+    want = K.knn_topk(X, Q, k, norms, n2, alive, lo, lo + n)
+    got = K.knn_search(X, q, k, unit, norms, alive, lo, lo + n)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    for bad in (dict(k=0), dict(k=257), dict(row_lo=-1), dict(N=len(X) + 1)):
+        with pytest.raises(ValueError):
+            K.knn_search(X, q, **{"k": k, "unit": unit, "row_lo": lo, "N": lo + n, **bad})
