@@ -224,6 +224,14 @@ def test_projections_to_cache_rows(device, dtype, case):
 
 
 @pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("case", [(2, 1, 64, 64, True, 0, 0, 17, 0), (3, 1, 96, 64, False, 2, 32, 18, 2), (33, 33, 128, 128, True, 0, 64, 7, 0)])
+def test_rows_of_a_mean_together(device, dtype, case):
+    """One row, two rows more than are asked for at once; rows of several vectors a thread, which ask for four."""
+    test_projections_to_cache_rows(device, dtype, case)
+
+
+@pytest.mark.parametrize("device", DEVICES)
 def test_queries_alone_leave_the_cache(device):
     a = heads_of(4, 2, 32, 32, True, 0, 0, A.Mask(9, keep=2), device=device, shared=True)
     rows = PagedHeads(2, 2, a.D, 0, 0, device, torch.float32)
