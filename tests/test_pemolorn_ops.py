@@ -142,6 +142,19 @@ def test_recurrence_in_portions_and_decoded(device, dtype, W):
     assert last.shape == (W,)
 
 
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("size", [16, 32])
+def test_recurrence_in_chunks_of_larger_passes(device, size, monkeypatch):
+    """The chunks of passes of more rows than the portions here have; chunk and pass edges of every size."""
+    monkeypatch.setattr(R, "chunk_rows", lambda rows: size)
+    for W in (33, 260):
+        test_recurrence_in_portions_and_decoded(device, torch.float32, W)
+    for rows, want in ((1, 8), (512, 8), (513, 16), (2048, 16), (2049, 32)):
+        monkeypatch.undo()
+        ch, cu = R.chunk_plan([0, rows])
+        assert ch[0].tolist() == [0, min(want, rows)] and ch[:, 1].sum() == rows and cu.tolist() == [0, -(-rows // want)]
+
+
 # ------------------------------------------------------------------ projections to queries and cache rows
 def heads_of(H, G, dim, vdim, per_head, conv, rot, mask, seed=0, device="cpu", shared=False, sink=True):
     nq, nk, nv = H * dim, G * dim, G * vdim
