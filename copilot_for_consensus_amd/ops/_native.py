@@ -73,7 +73,8 @@ _KERNEL_SIGS = {
     "cfc_final_norm": [I, P, P, I, P, F, I, P, P],
     "cfc_wkv_chunk_floats": [I],
     "cfc_wkv_tanh": [I, P, I, c_int64, c_int64, I, I, I, P, P],
-    "cfc_wkv_chunked": [I] + [P, c_int64] * 4 + [P, I, P, P, P, P, F, I, I, I, I, P, P, P, P, P, P, P, P, c_int64, P],
+    "cfc_wkv_chunked": [I] + [P, c_int64] * 4 + [P, I, P, P, P, P, F, I, I, I, I, P, P, P, P, P, P, P, I, P, P, c_int64, P],
+    "cfc_wkv_run_floats": [I],
     "cfc_wkv_step": [I, P, P, P, P, I, c_int64, c_int64, P, I, c_int64, c_int64, I, I, P, P, P, P, F, I, I, I, P, P, P, P, P,
                      c_int64, P],
     "cfc_moe_route": [P, I, c_int64, c_int64, P, I, I, I, I, I, F, I, I, P, P, P],

@@ -54,6 +54,15 @@ def chunk_plan(cu) -> tuple[np.ndarray, np.ndarray]:
     return np.asarray(chunks, np.int32), np.asarray(at, np.int32)
 
 
+def scan_runs(H: int, sequences: int, chunks: int) -> int:
+    """Runs that each portion's chunks are scanned in, beside each other.  A scan is a chain, 1.6 us a chunk in a workgroup a head and
+    sequence; what the runs do to a state (0.4 us a chunk) is known without the states before them.  us of a pass of zisapel (64
+    heads), portions in 1, 2, 4, 8 and 16 runs: one of 150 rows 1386, 1383, 1374, 1381, 1392, of 1400 3967, 3897, 3794, 3771, 3804, of 2800
+    6360, 6215, 6049, 6027, 6065; two of 1240 5800, 5752, 5723, 5748, 5804; but three of 390 3500, 3515, 3519, 3539, four of 1240 9815,
+    9865, 9874, 9949: from 192 workgroups on the CUs have enough to do."""
+    return max(1, min(512 // (H * sequences), chunks // sequences // 3)) if H * sequences <= 128 else 1
+
+
 def _ref(p: Wkv, r, k, v, g, w1, slots, cu, ctx, state, out):
     T = out.shape[0]
 
@@ -103,8 +112,10 @@ def prefill(p: Wkv, r: Cols, k: Cols, v: Cols, g: Cols, w1: Cols, slots, cu_q, c
     check(lib.cfc_wkv_tanh(_act(out.dtype), *w1.args(out.dtype), T, p.R, RP, th.data_ptr(), _stream(out)), "cfc_wkv_tanh")
     n = chunks.shape[0]
     rec = torch.empty(n * p.H * lib.cfc_wkv_chunk_floats(p.D), dtype=torch.float32, device=out.device)
+    nz = scan_runs(p.H, slots.numel(), n)
+    runs = torch.empty(nz * slots.numel() * p.H * lib.cfc_wkv_run_floats(p.D), dtype=torch.float32, device=out.device) if nz > 1 else None
     ops = [x for c in a for x in (c[0], c[2])]
     check(lib.cfc_wkv_chunked(_act(out.dtype), *ops, th.data_ptr(), RP, *p.tail(), n, slots.numel(), chunk_cu.data_ptr(),
-                              chunks.data_ptr(), slots.data_ptr(), cu_q.data_ptr(), ctx_lens.data_ptr(), rec.data_ptr(),
+                              chunks.data_ptr(), slots.data_ptr(), cu_q.data_ptr(), ctx_lens.data_ptr(), rec.data_ptr(), _p(runs), nz,
                               state.data_ptr(), out.data_ptr(), out.stride(0), _stream(out)), "cfc_wkv_chunked")
     return out

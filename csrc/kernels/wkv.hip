@@ -13,6 +13,8 @@
 //                coefficients, written in the fragment order of the scan's fp32 MFMAs
 //   * wkv_scan   one workgroup per (sequence, head), a wave per 16 value channels: the state stays in the
 //                accumulators over all chunks and is the B operand of the next one as it lies
+//   * wkv_ahead  where sequences and heads leave CUs idle a portion's chunks are cut into runs that wkv_scan takes beside
+//                each other: what each run but the last does to a state, which is all that the next ones need of it
 //   * wkv_step   token by token: decoded tokens (one pass over the state: read, output, update), and prompt
 //                portions of head sizes the chunked kernels are not built for
 #include "common.h"
@@ -295,10 +297,101 @@ __device__ __forceinline__ float row16_sum(float x) {
   return x;
 }
 
+// Runs of chunks: of nc, run z of nz is nc z / nz .. nc (z + 1) / nz.  S <- diag(d) S + U for a run of chunks as for one, so a run
+// starts from the states before it without their tokens.  Per (sequence, head), in `runs`: nz pieces of a state in the order
+// of its accumulators [wave][ND][64 lanes][4], behind each the decays d [16 ND].  Piece 0: the state that the portion starts from;
+// piece 1: the state behind run 0; piece z > 1: U and d of run z - 1.
+template <int ND>
+struct RunRec { static constexpr int S = ND * ND * 256, SIZE = S + 16 * ND; };
+
+
+// grid (H, sequences, nz - 1).  A wave needs no other: k, decays and v come straight to its registers
+template <typename ACT, int ND>
+__global__ void __launch_bounds__(64 * ND, 2) wkv_ahead_kernel(const float* __restrict__ rec, Cols v, ScanSeq sq, int H, int D, int nz,
+                                                              const float* __restrict__ state, float* __restrict__ runs) {
+  using Rec = ChunkRec<ND>;
+  using RAW = typename RawOf<ACT>::type;
+  constexpr int AHEAD_FLIGHT = ND > 4 ? 2 : 3;    // chunks on their way
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, q = lane >> 4;
+  const int h = blockIdx.x, s = blockIdx.y, z = blockIdx.z;
+  const int all = sq.chunk_cu[s + 1] - sq.chunk_cu[s], first = (int)((int64_t)all * z / nz), nc = (int)((int64_t)all * (z + 1) / nz) - first;
+  if (all <= 0) return;
+  const int c0 = sq.chunk_cu[s] + first, row0 = sq.cu_q[s], len = sq.cu_q[s + 1] - row0;
+  const bool fresh = sq.ctx_lens[s] == len;
+  const int vc = 16 * w + col;
+  const bool live = vc < D;
+  const int hv = h * D + min(vc, D - 1);
+  f32x4_t S[ND], L[ND];
+  f32x4_t* o = reinterpret_cast<f32x4_t*>(runs + ((size_t)s * H + h) * nz * RunRec<ND>::SIZE);
+  constexpr int PIECE = RunRec<ND>::SIZE / 4;
+#pragma unroll
+  for (int T = 0; T < ND; ++T) S[T] = f32x4_t{0.f, 0.f, 0.f, 0.f}, L[T] = f32x4_t{1.f, 1.f, 1.f, 1.f};
+  if (z == 0) {
+    const float* st = state + (((size_t)sq.slots[s] * H + h) * D) * D + min(vc, D - 1);
+#pragma unroll
+    for (int T = 0; T < ND; ++T) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int kc = 16 * T + 4 * q + i;
+        S[T][i] = !fresh && live && kc < D ? st[(size_t)min(kc, D - 1) * D] : 0.f;
+      }
+      o[(w * ND + T) * 64 + lane] = S[T];
+    }
+  }
+  if (nc > 0) {
+    constexpr int EB = sizeof(ACT);
+    const __amdgpu_buffer_rsrc_t vb = rows_of(reinterpret_cast<const ACT*>(v.p) + row0 * v.ld, len * v.ld * EB);
+    int vo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) vo[i] = ((4 * q + i) * (int)v.ld + hv) * EB;
+    f32x4_t kk[AHEAD_FLIGHT][ND], dd[AHEAD_FLIGHT][ND];
+    RAW rv[AHEAD_FLIGHT][4];
+    auto load = [&](int c, int u) {          // chunk c (past the last: re-read, not used)
+      c = __builtin_amdgcn_readfirstlane(min(c, nc - 1));
+      const f32x4_t* p = reinterpret_cast<const f32x4_t*>(rec + ((size_t)(c0 + c) * H + h) * Rec::SIZE);
+#pragma unroll
+      for (int T = 0; T < ND; ++T) {
+        kk[u][T] = p[Rec::K / 4 + T * 64 + lane];
+        dd[u][T] = p[Rec::DEC / 4 + 4 * T + q];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) rv[u][i] = ld_raw<ACT>(vb, vo[i], (first + c) * CT * (int)v.ld * EB);
+    };
+#pragma unroll
+    for (int u = 0; u < AHEAD_FLIGHT; ++u) load(u, u);
+    for (int c = 0; c < nc; c += AHEAD_FLIGHT)
+#pragma unroll
+      for (int u = 0; u < AHEAD_FLIGHT; ++u) {
+        if (c + u < nc) {
+          float vv[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) vv[i] = raw2f<ACT>(rv[u][i]);
+#pragma unroll
+          for (int T = 0; T < ND; ++T)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) S[T][i] *= dd[u][T][i], L[T][i] *= dd[u][T][i];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int T = 0; T < ND; ++T) S[T] = mfma4(kk[u][T][i], vv[i], S[T]);
+        }
+        load(c + AHEAD_FLIGHT + u, u);
+      }
+  }
+  o += (size_t)(z + 1) * PIECE;
+#pragma unroll
+  for (int T = 0; T < ND; ++T) {
+    o[(w * ND + T) * 64 + lane] = S[T];
+    if (w == 0 && col == 0) o[RunRec<ND>::S / 4 + 4 * T + q] = L[T];
+  }
+}
+
+// runs null: a portion's chunks in one run (grid (H, sequences)); else grid (H, sequences, runs)
 template <typename ACT, int ND>
 __global__ void __launch_bounds__(64 * ND, 2) wkv_scan_kernel(const float* __restrict__ rec, Cols v, Cols g, ScanSeq sq, int H,
                                                              int D, const float* __restrict__ norm, float eps,
-                                                             float* __restrict__ state, ACT* __restrict__ out, int64_t ldo) {
+                                                             float* __restrict__ state, const float* __restrict__ runs,
+                                                             ACT* __restrict__ out, int64_t ldo) {
   using Rec = ChunkRec<ND>;
   using RAW = typename RawOf<ACT>::type;
   constexpr int NV4 = Rec::SIZE / 4, NT = 64 * ND, NLD = (NV4 + NT - 1) / NT;
@@ -306,10 +399,11 @@ __global__ void __launch_bounds__(64 * ND, 2) wkv_scan_kernel(const float* __res
   __shared__ __attribute__((aligned(16))) float red[2][ND][16];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, q = lane >> 4;
   const int h = blockIdx.x, s = blockIdx.y;
-  const int c0 = sq.chunk_cu[s], nc = sq.chunk_cu[s + 1] - c0;
-  if (nc <= 0) return;
-  const int row0 = sq.cu_q[s], len = sq.cu_q[s + 1] - row0;
-  const bool fresh = sq.ctx_lens[s] == len;
+  const int all = sq.chunk_cu[s + 1] - sq.chunk_cu[s], z = blockIdx.z, nz = gridDim.z, first = (int)((int64_t)all * z / nz);
+  const int c0 = sq.chunk_cu[s] + first, nc = (int)((int64_t)all * (z + 1) / nz) - first;
+  if (nc <= 0) return;                            // of fewer chunks than runs; the last run has one
+  const int rows = sq.cu_q[s + 1] - sq.cu_q[s], row0 = sq.cu_q[s] + CT * first, len = min(rows - CT * first, CT * nc);
+  const bool fresh = sq.ctx_lens[s] == rows;
   const int vc = 16 * w + col;                    // value channel of this lane
   const bool live = vc < D;
   const int hv = h * D + min(vc, D - 1);
@@ -320,8 +414,21 @@ __global__ void __launch_bounds__(64 * ND, 2) wkv_scan_kernel(const float* __res
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int kc = 16 * T + 4 * q + i;
-      S[T][i] = !fresh && live && kc < D ? st[(size_t)min(kc, D - 1) * D] : 0.f;
+      S[T][i] = !runs && !fresh && live && kc < D ? st[(size_t)min(kc, D - 1) * D] : 0.f;
     }
+  if (runs) {
+    const f32x4_t* p = reinterpret_cast<const f32x4_t*>(runs + ((size_t)s * H + h) * nz * RunRec<ND>::SIZE);
+    constexpr int PIECE = RunRec<ND>::SIZE / 4;
+#pragma unroll
+    for (int T = 0; T < ND; ++T) S[T] = p[min(z, 1) * PIECE + (w * ND + T) * 64 + lane];
+    for (int j = 2; j <= z; ++j)
+#pragma unroll
+      for (int T = 0; T < ND; ++T) {
+        const f32x4_t d = p[j * PIECE + RunRec<ND>::S / 4 + 4 * T + q], a = p[j * PIECE + (w * ND + T) * 64 + lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[T][i] = d[i] * S[T][i] + a[i];
+      }
+  }
   const float nw = norm[hv], rD = 1.f / (float)D;
   typedef float f4_t __attribute__((ext_vector_type(4)));      // arrays of these stay in registers
   f4_t rr[SCAN_AHEAD][NLD];
@@ -443,7 +550,7 @@ __global__ void __launch_bounds__(64 * ND, 2) wkv_scan_kernel(const float* __res
     if (c + u < nc) chunk(c + u, u);
   barrier();
   finish(nc - 1, (nc - 1) & 1);
-  if (live) {
+  if (live && z + 1 == nz) {
 #pragma unroll
     for (int T = 0; T < ND; ++T)
 #pragma unroll
@@ -602,12 +709,17 @@ __global__ void __launch_bounds__(WS_T, ONE ? 6 : 4) wkv_step_kernel(Cols r, Col
 template <typename ACT, int ND>
 int chunked_go(hipStream_t s, const Cols& r, const Cols& k, const Cols& v, const Cols& g, const uint16_t* th, int RP,
                const uint16_t* w2, const float* w0, const float* u, const float* norm, float eps, int H, int D, int n_chunks,
-               int n_seq, const ScanSeq& sq, float* rec, float* state, void* out, int64_t ldo) {
+               int n_seq, const ScanSeq& sq, float* rec, float* runs, int nz, float* state, void* out, int64_t ldo) {
   constexpr int WV = ND <= 4 ? 4 : 2;
   constexpr int lds = WV * 49 * (16 * ND + 4) * 4;
   wkv_prep_kernel<ACT, ND, WV><<<dim3(n_chunks, (H + WV - 1) / WV), 64 * WV, lds, s>>>(r, k, th, RP, w2, w0, u, sq.chunks, H, D, rec);
   if (const int e = (int)hipGetLastError()) return e;
-  wkv_scan_kernel<ACT, ND><<<dim3(H, n_seq), 64 * ND, 0, s>>>(rec, v, g, sq, H, D, norm, eps, state, (ACT*)out, ldo);
+  if (nz > 1) {
+    wkv_ahead_kernel<ACT, ND><<<dim3(H, n_seq, nz - 1), 64 * ND, 0, s>>>(rec, v, sq, H, D, nz, state, runs);
+    if (const int e = (int)hipGetLastError()) return e;
+  }
+  wkv_scan_kernel<ACT, ND><<<dim3(H, n_seq, nz), 64 * ND, 0, s>>>(rec, v, g, sq, H, D, norm, eps, state, nz > 1 ? runs : nullptr,
+                                                                 (ACT*)out, ldo);
   return CFC_CHECK_LAUNCH();
 }
 
@@ -620,6 +732,13 @@ CFC_API int cfc_wkv_chunk_floats(int D) {
   if (D < 1 || D > WKV_MAX_CHUNKED) return 0;
   const int nd = D <= 64 ? (D + 15) / 16 : D <= 96 ? 6 : 8;
   return 2 * nd * 256 + 256 + 16 * nd;
+}
+
+// floats of scratch per (run, sequence, head) where portions are scanned in several runs
+CFC_API int cfc_wkv_run_floats(int D) {
+  if (D < 1 || D > WKV_MAX_CHUNKED) return 0;
+  const int nd = D <= 64 ? (D + 15) / 16 : D <= 96 ? 6 : 8;
+  return nd * nd * 256 + 16 * nd;
 }
 
 // out [T][3][RP] bf16 parts of tanh(w1) (split 0: w1 are activations)
@@ -635,13 +754,16 @@ CFC_API int cfc_wkv_tanh(int f32, const void* w1, int split, int64_t ld, int64_t
 }
 
 // r, k, v, g: activations with row strides; th from cfc_wkv_tanh; chunks [n][2] = {first row, rows <= 16} in
-// sequence order, chunk_cu [sequences + 1]; rec: cfc_wkv_chunk_floats(D) floats per (chunk, head)
+// sequence order, chunk_cu [sequences + 1]; rec: cfc_wkv_chunk_floats(D) floats per (chunk, head); nz > 1: portions are scanned
+// in so many runs beside each other, through runs, cfc_wkv_run_floats(D) floats per (run, sequence, head)
 CFC_API int cfc_wkv_chunked(int f32, const void* r, int64_t ldr, const void* k, int64_t ldk, const void* v, int64_t ldv,
                             const void* g, int64_t ldg, const void* th, int RP, const void* w2, const float* w0,
                             const float* u, const float* norm, float eps, int H, int D, int n_chunks, int n_seq,
                             const int32_t* chunk_cu, const int32_t* chunks, const int32_t* slots, const int32_t* cu_q,
-                            const int32_t* ctx_lens, float* rec, float* state, void* out, int64_t ldo, hipStream_t stream) {
+                            const int32_t* ctx_lens, float* rec, float* runs, int nz, float* state, void* out, int64_t ldo,
+                            hipStream_t stream) {
   if (n_seq <= 0 || n_chunks <= 0) return 0;
+  if (nz < 1 || nz > 65536 || (nz > 1 && !runs)) return -1;
   if (H < 1 || D < 1 || D > WKV_MAX_CHUNKED || RP < 32 || RP % 32 || n_seq > 65535) return -1;
   // 32-bit offsets within a portion
   const int64_t ldm = ldo > ldv ? (ldo > ldg ? ldo : ldg) : (ldv > ldg ? ldv : ldg);
@@ -650,7 +772,7 @@ CFC_API int cfc_wkv_chunked(int f32, const void* r, int64_t ldr, const void* k, 
   const ScanSeq sq{chunk_cu, chunks, slots, cu_q, ctx_lens};
 #define WC(ACT, ND)                                                                                                      \
   return chunked_go<ACT, ND>(stream, cr, ck, cv, cg, (const uint16_t*)th, RP, (const uint16_t*)w2, w0, u, norm, eps, H, \
-                             D, n_chunks, n_seq, sq, rec, state, out, ldo)
+                             D, n_chunks, n_seq, sq, rec, runs, nz, state, out, ldo)
 #define WN(ACT)                                      \
   switch (D <= 64 ? (D + 15) / 16 : D <= 96 ? 6 : 8) { \
     case 1: WC(ACT, 1);                              \

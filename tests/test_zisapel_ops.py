@@ -205,6 +205,26 @@ def test_recurrence_of_a_packed_batch(device):
         close(out[at:at + n], wkv_want(p, cases[i][1], cases[i][2], H, D, eps)[o:], 2e-5)
         at += n
 
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("runs", [2, 3, 7, 16])
+def test_recurrence_in_runs_of_chunks(device, runs, monkeypatch):
+    """A portion's chunks in several runs beside each other, down to fewer chunks than runs: the same outputs and states, portions
+    that continue among them, and decays from next to one to immediate."""
+    monkeypatch.setattr(R, "scan_runs", lambda *a: runs)
+    test_recurrence_of_a_packed_batch(device)
+    for dtype, H, D, rank in ((torch.float32, 3, 24, 1), (torch.bfloat16, 2, 64, 24), (torch.float32, 2, 96, 16), (torch.bfloat16, 1, 128, 64)):
+        test_recurrence_in_portions_and_decoded(device, dtype, H, D, rank)
+    for w0, spread in ((-9.0, 0.1), (3.0, 0.5), (0.0, 6.0)):
+        test_recurrence_from_no_decay_to_immediate(device, w0, spread)
+
+
+def test_runs_of_a_scan():
+    """Never more workgroups than run side by side, nor runs of under three chunks; one where heads and sequences fill the chip."""
+    for H, n, chunks in ((64, 1, 1), (64, 1, 10), (64, 1, 1000), (64, 2, 90), (64, 3, 500), (1, 1, 4096), (128, 1, 50), (200, 1, 50), (1, 7, 6)):
+        k = R.scan_runs(H, n, chunks)
+        assert k == 1 or (k * H * n <= 512 and 3 * k * n <= chunks)
+        assert k >= 1 and (H * n <= 128 or k == 1)
+
 
 # ------------------------------------------------------------------ latent attention
 SCALING = {"factor": 4.0, "original": 64, "fast": 8.0, "slow": 1.0}
