@@ -44,7 +44,6 @@ from .projection import JointProjection, Projection
 POSITION_BASE = 10000.0                              # of the embedding's sinusoids
 RATE = -8.0                                          # of the linear recurrence's log decay
 GELU = dict(limit=math.inf, alpha=2.0 * math.sqrt(2.0 / math.pi), beta=0.0, cubic=0.044715)     # tanh form, as a gated sigmoid
-CONV_ROWS = 32                                       # prompt rows per tile of the convolutions
 DEFAULT_SEQUENCES = 256
 
 
@@ -409,7 +408,7 @@ class TadolixModel:
         the device."""
         n = np.diff(np.asarray(cu))
         portions = [(int(a), int(k), int(c - k), s) for s, (a, k, c) in enumerate(zip(cu, n, ctx))]
-        rows = max([CONV_ROWS, self.cfg.taps - 1] + [lw["lru"].taps - 1 for lw in self.w.layers if "lru" in lw])
+        rows = max([S.conv_rows(int(cu[-1] - cu[0])), self.cfg.taps - 1] + [lw["lru"].taps - 1 for lw in self.w.layers if "lru" in lw])
         plan = {"states": np.asarray(states, np.int32), "row_states": np.repeat(np.asarray(states, np.int32), n),
                 "lead": np.concatenate([np.arange(k, dtype=np.int32) for k in n]), "conv_tiles": S.conv_tiles(portions, rows)}
         for lw in self.w.layers:

@@ -323,7 +323,7 @@ class VofosunModel:
     def plan_prefill(self, cu, ctx, slots) -> dict:
         """Host-side launch plan of a packed pass over portions cu / ctx: int32 arrays for the device."""
         por = [(cu[s], cu[s + 1] - cu[s], ctx[s] - (cu[s + 1] - cu[s]), s) for s in range(len(ctx))]
-        plan = {"conv_tiles": S.conv_tiles(por)}
+        plan = {"conv_tiles": S.conv_tiles(por, taps=self.cfg.taps, most=S.conv_rows(cu[-1] - cu[0]))}
         for i, lw in enumerate(self.w.layers):
             key = f"attn_{lw['H']}_{self._rows(i)}"
             if key not in plan:

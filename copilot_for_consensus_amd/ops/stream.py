@@ -161,15 +161,31 @@ def depth_conv_decode(x, hist, up: Update | None, norm_w, eps: float, convs, pos
            outs[1] if two else None, convs[0], convs[1] if two else None, positions, tail, hist)
 
 
-def conv_tiles(portions, rows: int | None = None) -> np.ndarray:
+def conv_rows(rows: int) -> int:
+    """Rows of a convolution's tile in a pass of so many.  A thread walks its channels down a tile, 11 to 14 us for 32 rows however
+    few the tiles are; every tile reads taps - 1 rows again.  us of a pass in tiles of 32, 16 and 8 rows: tadolix of 54 rows 650,
+    625, 617, of 291 1038, 1016, 1012, of 1166 2453, 2444, 2449, vofosun of 291 1030, 1018, 1012, of 1166 2400, 2395, 2394, of 2800
+    4385, 4390, 4397, of 9800 12890, 12915, 13014."""
+    return 8 if rows <= 1024 else KV_BLOCK
+
+
+def conv_tiles(portions, rows: int | None = None, taps: int | None = None, most: int = KV_BLOCK) -> np.ndarray:
     """[2, n, 4] int32 tiles of :func:`input_conv`: each portion (first row, rows, first position,
     sequence) cut at the cache blocks' borders, or (tails in slots) after every ``rows`` of its rows, at least
-    taps - 1; then per tile the portion's rows before it and in all."""
+    taps - 1; then per tile the portion's rows before it and in all, and whether it leaves no tail.  ``taps``: a block's rows
+    are cut again after every ``most``, at least taps - 1 (its first tile must not read tail rows that its last one writes, which
+    leaves the tail and so has taps - 1 rows or all)."""
     tiles, lead = [], []
+    few = max(most, taps - 1) if taps else KV_BLOCK
     for row0, n, pos0, seq in portions:
         r = 0
         while r < n:
             m = min(n - r, rows or KV_BLOCK - (pos0 + r) % KV_BLOCK)
+            cut = few if r or pos0 % KV_BLOCK == 0 else m
+            while taps and m - cut >= taps - 1 and m > cut:
+                tiles.append((row0 + r, cut, pos0 + r, seq))
+                lead.append((r, n, 1, 0))
+                r, m = r + cut, m - cut
             tiles.append((row0 + r, m, pos0 + r, seq))
             lead.append((r, n, 0, 0))
             r += m

@@ -302,11 +302,12 @@ __global__ void __launch_bounds__(256) depth_pre_kernel(const float* __restrict_
   for (int l = 0; l < CNT; ++l) stv<V>(pre + (size_t)l * plane + c, acc[l]);
 }
 
-// Packed prompt portions.  A tile is the rows of one portion inside ONE cache block: {first row, rows,
+// Packed prompt portions.  A tile is rows of one portion inside ONE cache block: {first row, rows,
 // first position, sequence}; a thread walks its V channels down the tile.  Rows before the portion come
 // from the tail: of this tile's own block they are read here before the tile's last rows replace them
-// (same thread, same channels), and an earlier block's are not written in this launch unless another
-// sequence owns it, which the engine rules out by sharing blocks only after they are computed.
+// (same thread, same channels: such a tile has all of the portion's rows in the block), and an earlier block's are
+// not written in this launch unless another sequence owns it, which the engine rules out by sharing blocks only after
+// they are computed.  A block's last tile leaves its tail, the others are marked.
 // TAPS 0: any number of taps, the inputs recomputed per tap instead of kept in a register window.
 constexpr int IC_AHEAD = 4;
 template <typename ACT, int V, int TAPS>
@@ -323,7 +324,7 @@ __global__ void __launch_bounds__(256) input_conv_kernel(const float* __restrict
   const Vec<V> g = ldv<V>(norm_w + c);
   // rows of this portion that precede the tile: tile_lead rows are in x, the rest in the tail
   const int lead = tiles[4 * (gridDim.x + blockIdx.x)];
-  const bool paged = ta.max_blocks != 0;
+  const bool paged = ta.max_blocks != 0, keeps = paged && !tiles[4 * (gridDim.x + blockIdx.x) + 2];
   auto input = [&](int r) -> Vec<V> {        // convolution input of row row0 + r (r may be negative)
     Vec<V> h;
     if (pos0 + r < 0) {
@@ -342,7 +343,7 @@ __global__ void __launch_bounds__(256) input_conv_kernel(const float* __restrict
   auto put = [&](int r, const Vec<V>& h, const Vec<V>& y1, const Vec<V>& y2) {
     stv<V>(h1 + (size_t)(row0 + r) * ld_1 + c, y1);
     if (w2) stv<V>(h2 + (size_t)(row0 + r) * ld_2 + c, y2);
-    if (paged && r >= n - (taps - 1)) stv<V>(tail_row(ta, seq, pos0 + r, W) + c, h);
+    if (keeps && r >= n - (taps - 1)) stv<V>(tail_row(ta, seq, pos0 + r, W) + c, h);
   };
   if constexpr (TAPS > 0) {
     float k1[TAPS][V], k2[TAPS][V];

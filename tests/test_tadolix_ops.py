@@ -137,6 +137,15 @@ def test_input_convolution_in_portions_and_decoded(device, dtype, taps, W):
         assert torch.equal(tail[[0, 2, 4]], before[[0, 2, 4]])
 
 
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("taps,W", [(4, 260), (7, 96), (35, 64)])
+def test_input_convolution_in_short_tiles(device, taps, W, monkeypatch):
+    """In tiles of eight rows, or as many as a tail has."""
+    cut = S.conv_tiles
+    monkeypatch.setattr(S, "conv_tiles", lambda portions, rows: cut(portions, max(8, taps - 1)))
+    test_input_convolution_in_portions_and_decoded(device, torch.bfloat16, taps, W)
+
+
 def test_tiles_of_a_convolution_with_slots():
     """Cut from the portion's start on, so that only its first tile reads what lies before it."""
     t = S.conv_tiles([(0, 70, 31, 0), (70, 1, 5, 1)], 32)

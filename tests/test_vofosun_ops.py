@@ -141,6 +141,24 @@ def test_input_convolution_over_portions_and_decode(device, W, taps, two):
 
 
 @pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("W,taps,most", [(104, 4, 8), (65, 3, 2), (64, 2, 1), (40, 1, 8), (36, 7, 8), (24, 40, 8), (1100, 5, 16)])
+def test_input_convolution_in_short_tiles(device, W, taps, most, monkeypatch):
+    """A cache block's rows in several tiles, of which the last alone leaves the block's tail."""
+    cut = S.conv_tiles
+    monkeypatch.setattr(S, "conv_tiles", lambda portions: cut(portions, taps=taps, most=most))
+    test_input_convolution_over_portions_and_decode(device, W, taps, True)
+
+
+def test_short_tiles_of_a_convolution():
+    """What starts within a block stays whole there (its first tile would read what its last writes); a rest of fewer rows than a
+    tail stays with the tile before it."""
+    t = S.conv_tiles([(0, 45, 30, 0), (45, 18, 64, 1), (63, 2, 0, 2)], taps=4, most=8)
+    assert t[0].tolist() == [[0, 2, 30, 0], [2, 8, 32, 0], [10, 8, 40, 0], [18, 8, 48, 0], [26, 8, 56, 0], [34, 8, 64, 0],
+                             [42, 3, 72, 0], [45, 8, 64, 1], [53, 10, 72, 1], [63, 2, 0, 2]]
+    assert t[1, :, :3].tolist() == [[0, 45, 0], [2, 45, 1], [10, 45, 1], [18, 45, 1], [26, 45, 0], [34, 45, 1], [42, 45, 0], [0, 18, 1], [8, 18, 0], [0, 2, 0]]
+
+
+@pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("limit", [0.7, 1.0, 3.0])
 @pytest.mark.parametrize("F,interleaved,split", [(48, True, 1), (33, False, 1), (40, True, 5)])
