@@ -719,6 +719,12 @@ class DecoderModel:
             torch.distributed.all_reduce(x, group=self.tp_group)
         return x
 
+    def _begin(self, ids):
+        """(normed input of layer 0, residual stream) of tokens."""
+        if self.fp8:
+            return self._layer_pre(0, K.embedding(self.w.embed, ids), None)
+        return K.embed_rmsnorm(self.w.embed, ids, self.w.layers[0]["attn_norm"], self.cfg.rms_eps)
+
     def _layer_pre(self, i, x, residual):
         """Returns normed input of layer i and the residual stream."""
         lw = self.w.layers[i]
@@ -749,10 +755,9 @@ class DecoderModel:
         cfg, w = self.cfg, self.w
         if plan is not None:
             tiles, v_runs = (plan["tile_seq"], plan["tile_q0"]), plan["v_runs"]
-        x = K.embedding(w.embed, ids)
-        residual = None
+        x = None
         x32 = None                     # TP fp32: this rank's fp32 partial of the previous layer's down
-        normed = None                  # the layer's normed input, made with the sum of the previous one's slabs
+        normed, residual = self._begin(ids)      # the layer's normed input, made with the sum of the previous one's slabs
         eps = cfg.rms_eps
         for i in range(cfg.layers):
             lw = w.layers[i]
@@ -787,8 +792,7 @@ class DecoderModel:
                 x32, residual = x32.index_select(0, last_idx), residual.index_select(0, last_idx)
             return self._tp_norm(x32.contiguous(), residual, w.final_norm)
         if last_idx is not None:
-            x = x.index_select(0, last_idx)
-            residual = residual.index_select(0, last_idx)
+            return K.rmsnorm_rows(x, residual, last_idx, w.final_norm, cfg.rms_eps)
         return K.rmsnorm(x, w.final_norm, cfg.rms_eps, residual=residual)
 
     def supports_prefill_overlap(self) -> bool:
@@ -868,20 +872,20 @@ class DecoderModel:
         the caches instead of nontemporal."""
         self._shared_blocks = shared_blocks
         cfg, w = self.cfg, self.w
-        x = K.embedding(w.embed, ids)
         B = ids.shape[0]
-        if (self.fused_decode and x.is_cuda and (B <= DGEMM_MAX_ROWS or self.w.packed_only)
+        if (self.fused_decode and ids.is_cuda and (B <= DGEMM_MAX_ROWS or self.w.packed_only)
                 and not (B <= K.GEMV_MAX_M and (self.decode_gemv and not self._small_dgemm(B) or self.decode_qgemv))):
-            return self._forward_decode_fused(x, positions, slots, ctx_lens, block_tables, kv, attn_workspace,
+            return self._forward_decode_fused(ids, positions, slots, ctx_lens, block_tables, kv, attn_workspace,
                                               part_blocks)
-        if self.decode_gemm in ("splitk", "dgemm") and x.is_cuda and self.w.tp_size == 1:
-            return self._forward_decode_splitk(x, positions, slots, ctx_lens, block_tables, kv, attn_workspace,
+        if self.decode_gemm in ("splitk", "dgemm") and ids.is_cuda and self.w.tp_size == 1:
+            return self._forward_decode_splitk(ids, positions, slots, ctx_lens, block_tables, kv, attn_workspace,
                                                part_blocks)
-        residual = None
         x32 = None
         for i in range(cfg.layers):
             lw = w.layers[i]
-            if x32 is not None:
+            if i == 0:
+                h, residual = self._begin(ids)
+            elif x32 is not None:
                 h = self._tp_norm(x32, residual, lw["attn_norm"])
             else:
                 h, residual = self._layer_pre(i, x, residual)
@@ -933,17 +937,16 @@ class DecoderModel:
                                         part_blocks=part_blocks, workspace=attn_workspace, window=self.window,
                                         k_scale=kv.k_scale, v_scale=kv.v_scale, shared_blocks=sb)
 
-    def _forward_decode_fused(self, x, positions, slots, ctx_lens, block_tables, kv, attn_workspace, part_blocks):
+    def _forward_decode_fused(self, ids, positions, slots, ctx_lens, block_tables, kv, attn_workspace, part_blocks):
         """Decode layer on the hand-written decode GEMM (dgemm.hip), elementwise work in epilogues:
         qkv -> RoPE/KV write -> attention -> [o + residual + mlp RMSNorm] -> [gate_up + SwiGLU] ->
         [down + residual + next layer's RMSNorm].  Same rounding points as the library path.
         With TP the row-parallel o/down outputs are all-reduced (one-shot IPC all-reduce inside the
         decode graph when available) before the residual + RMSNorm."""
         cfg, w = self.cfg, self.w
-        B = x.shape[0]
+        B = ids.shape[0]
         eps = cfg.rms_eps
-        residual = x.clone()
-        h = K.rmsnorm(x, w.layers[0]["attn_norm"], eps)
+        h, residual = K.embed_rmsnorm(w.embed, ids, w.layers[0]["attn_norm"], eps)
         tp = w.tp_size > 1
         for i in range(cfg.layers):
             lw = w.layers[i]
@@ -978,13 +981,12 @@ class DecoderModel:
         bn, split = K.dgemm_config(B, w.shape[0], Kd, bn=getattr(w, "bn", None))
         return self._tp_norm(K.dgemm(x, w, "part", split, bn=bn), residual, norm_w)
 
-    def _forward_decode_splitk(self, x, positions, slots, ctx_lens, block_tables, kv, attn_workspace, part_blocks):
+    def _forward_decode_splitk(self, ids, positions, slots, ctx_lens, block_tables, kv, attn_workspace, part_blocks):
         """Library GEMMs; o and down as batched split-K with residual + next RMSNorm in the reduce."""
         cfg, w = self.cfg, self.w
-        B = x.shape[0]
+        B = ids.shape[0]
         eps = cfg.rms_eps
-        residual = x.clone()
-        h = K.rmsnorm(x, w.layers[0]["attn_norm"], eps)
+        h, residual = K.embed_rmsnorm(w.embed, ids, w.layers[0]["attn_norm"], eps)
         s_o = K.lib_split_for(w.heads * cfg.head_dim, cfg.hidden)
         s_d = K.lib_split_for(w.ffn, cfg.hidden)
         if self.decode_qgemv and B <= K.GEMV_MAX_M:

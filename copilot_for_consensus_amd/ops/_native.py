@@ -27,6 +27,8 @@ L = c_int64
 # name -> argtypes (every kernel launcher returns int: 0 = ok, <0 = bad arguments, >0 = hipError)
 _KERNEL_SIGS = {
     "cfc_rmsnorm": [P, P, P, P, I, I, F, I, P],
+    "cfc_embed_rmsnorm": [P, P, P, P, P, I, I, F, P],
+    "cfc_rmsnorm_rows": [P, P, P, P, P, I, I, F, P],
     "cfc_layernorm": [P, P, P, P, P, P, P, P, P, P, I, I, F, I, P],
     "cfc_paged_decode_attention": [P, P, P, P, P, I, I, I, I, I, I, I, F, I, P, P, P, P, P],
     "cfc_prefill_attention": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, P, P],

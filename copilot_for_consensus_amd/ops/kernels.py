@@ -67,6 +67,36 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, residual: torch.Tensor
     return out
 
 
+def embed_rmsnorm(table: torch.Tensor, ids: torch.Tensor, w: torch.Tensor, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """(RMSNorm(x) * w, x) of the rows x = table[ids], in one launch."""
+    if not table.is_cuda:
+        x = embedding(table, ids)
+        return rmsnorm(x, w, eps), x
+    _req(table, torch.bfloat16, "table")
+    _req(ids, torch.int32, "ids")
+    T, dim = ids.numel(), table.shape[1]
+    x = torch.empty(T, dim, dtype=table.dtype, device=table.device)
+    out = torch.empty_like(x)
+    check(kernels().cfc_embed_rmsnorm(out.data_ptr(), x.data_ptr(), table.data_ptr(), ids.data_ptr(), w.data_ptr(), T, dim, float(eps),
+                                      _stream(table)), "cfc_embed_rmsnorm")
+    return out, x
+
+
+def rmsnorm_rows(x: torch.Tensor, residual: torch.Tensor, rows: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    """RMSNorm of the rows ``rows`` of x + residual, neither of which is changed, * w."""
+    if not x.is_cuda:
+        return rmsnorm(x.index_select(0, rows), w, eps, residual=residual.index_select(0, rows))
+    _req(x, torch.bfloat16, "x")
+    _req(residual, torch.bfloat16, "residual")
+    if x.shape != residual.shape or x.dim() != 2:
+        raise ValueError(f"rmsnorm_rows: x {tuple(x.shape)}, residual {tuple(residual.shape)}")
+    rows = rows.to(torch.int32).contiguous()
+    out = torch.empty(rows.numel(), x.shape[1], dtype=x.dtype, device=x.device)
+    check(kernels().cfc_rmsnorm_rows(out.data_ptr(), residual.data_ptr(), x.data_ptr(), rows.data_ptr(), w.data_ptr(), rows.numel(),
+                                     x.shape[1], float(eps), _stream(x)), "cfc_rmsnorm_rows")
+    return out
+
+
 def layernorm(x, gamma, beta, eps, bias=None, residual=None, out=None):
     """LN(x [+ bias + residual]) (post-LN BERT sub-layer epilogue)."""
     if not x.is_cuda:

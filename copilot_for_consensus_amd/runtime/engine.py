@@ -277,7 +277,7 @@ class LLMEngine:
         d_ids, d_pos, d_slots, d_cu, d_ctx, d_last, d_extra, d_bt = views[:8]
         plan.update((k, v.view(plan[k].shape)) for k, v in zip(arrays, views[8:]))
         kw = dict(ids=d_ids, positions=d_pos, slots=d_slots, cu_q=d_cu, ctx_lens=d_ctx,
-                  block_tables=d_bt.view(len(tables), maxb), plan=plan, last_idx=d_last.long() if last_rows else None)
+                  block_tables=d_bt.view(len(tables), maxb), plan=plan, last_idx=d_last if last_rows else None)
         return kw, d_extra
 
     # ------------------------------------------------------------------ single steps

@@ -13,16 +13,21 @@ namespace {
 // F8: out is e4m3fn of the bf16-rounded normalised row divided by a per-row scale
 // (scale[row] = amax / 448) -- the W8A8 projection's activation quantisation fused into the norm
 // that produces it, so the row makes no extra HBM round trip through a bf16 tensor.
-template <int VPT, bool F8>
+// RN_EMBED: x is a table of embeddings whose rows ids[] begin the stream: they are stored as the residual, too.  An embedding, a
+// copy and a norm of their own cost a decode step two launches more, 2.8 us each, and a prompt a pass over its rows more (15760 rows of
+// 4096: 171 us, so 78).  RN_ROWS: rows ids[] of x and of the residual, neither of which is written: the last tokens of prompts.
+enum { RN_ALL = 0, RN_EMBED = 1, RN_ROWS = 2 };
+template <int VPT, bool F8, int SRC = RN_ALL>
 __global__ void __launch_bounds__(1024) rmsnorm_kernel(void* __restrict__ out, float* __restrict__ scale,
                                                       uint16_t* __restrict__ residual,
                                                       const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                      int dim, float eps, int add_residual) {
+                                                      int dim, float eps, int add_residual, const int32_t* __restrict__ ids) {
   __shared__ float red[16];
   const int row = blockIdx.x;
   const int nvec = dim >> 3;
-  const uint4* xr = reinterpret_cast<const uint4*>(x + (size_t)row * dim);
-  uint4* rr = reinterpret_cast<uint4*>(residual + (size_t)row * dim);
+  const int from = SRC == RN_ALL ? row : ids[row];
+  const uint4* xr = reinterpret_cast<const uint4*>(x + (size_t)from * dim);
+  uint4* rr = reinterpret_cast<uint4*>(residual + (size_t)(SRC == RN_ROWS ? from : row) * dim);
   float v[VPT][8];
   float ss = 0.f;
   const uint4* wr = reinterpret_cast<const uint4*>(w);
@@ -32,15 +37,21 @@ __global__ void __launch_bounds__(1024) rmsnorm_kernel(void* __restrict__ out, f
     const int c = threadIdx.x + i * blockDim.x;
     if (c < nvec) {
       if constexpr (VPT == 1) gain = wr[c];
-      unpack8(xr[c], v[i]);
-      if (add_residual) {
+      if constexpr (SRC == RN_EMBED) {
+        const uint4 e = xr[c];
+        rr[c] = e;
+        unpack8(e, v[i]);
+      } else {
+        unpack8(xr[c], v[i]);
+      }
+      if (SRC != RN_EMBED && add_residual) {
         float r[8];
         unpack8(rr[c], r);
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[i][j] += r[j];
         // residual <- x + residual (rounded to bf16 exactly like the stored stream)
         uint4 p = pack8(v[i]);
-        rr[c] = p;
+        if constexpr (SRC == RN_ALL) rr[c] = p;
         unpack8(p, v[i]);
       }
 #pragma unroll
@@ -164,21 +175,22 @@ __global__ void __launch_bounds__(1024) layernorm_kernel(uint16_t* __restrict__ 
 // a row is a single load round trip instead of VPT dependent ones (10 us -> ~3 us per call).
 inline int pick_block(int nvec) { return nvec >= 1024 ? 1024 : ((nvec + 63) / 64) * 64; }
 
-template <bool F8>
+template <bool F8, int SRC = RN_ALL>
 int launch_rmsnorm(void* out, float* scale, void* residual, const void* x, const void* w, int rows, int dim, float eps,
-                   int add_residual, hipStream_t stream) {
+                   int add_residual, hipStream_t stream, const int32_t* ids = nullptr) {
   const int nvec = dim / 8, block = pick_block(nvec);
   const int vpt = (nvec + block - 1) / block;
-  auto r = (uint16_t*)residual;
-  auto xi = (const uint16_t*)x; auto wi = (const uint16_t*)w;
+#define RN(V)                                                                                                               \
+  rmsnorm_kernel<V, F8, SRC><<<rows, block, 0, stream>>>(out, scale, (uint16_t*)residual, (const uint16_t*)x, (const uint16_t*)w, dim, \
+                                                         eps, add_residual, ids)
   switch (vpt) {
-    case 1: rmsnorm_kernel<1, F8><<<rows, block, 0, stream>>>(out, scale, r, xi, wi, dim, eps, add_residual); break;
-    case 2: rmsnorm_kernel<2, F8><<<rows, block, 0, stream>>>(out, scale, r, xi, wi, dim, eps, add_residual); break;
-    case 3: case 4: rmsnorm_kernel<4, F8><<<rows, block, 0, stream>>>(out, scale, r, xi, wi, dim, eps, add_residual); break;
-    case 5: case 6: case 7: case 8:
-      rmsnorm_kernel<8, F8><<<rows, block, 0, stream>>>(out, scale, r, xi, wi, dim, eps, add_residual); break;
+    case 1: RN(1); break;
+    case 2: RN(2); break;
+    case 3: case 4: RN(4); break;
+    case 5: case 6: case 7: case 8: RN(8); break;
     default: return -2;
   }
+#undef RN
   return CFC_CHECK_LAUNCH();
 }
 
@@ -190,6 +202,20 @@ CFC_API int cfc_rmsnorm(void* out, void* residual, const void* x, const void* w,
                         int add_residual, hipStream_t stream) {
   if (dim % 8 != 0 || rows <= 0) return -1;
   return launch_rmsnorm<false>(out, nullptr, residual, x, w, rows, dim, eps, add_residual, stream);
+}
+
+// residual [rows, dim] = rows ids[] of a table, out = RMSNorm of them * w
+CFC_API int cfc_embed_rmsnorm(void* out, void* residual, const void* table, const int32_t* ids, const void* w, int rows, int dim,
+                              float eps, hipStream_t stream) {
+  if (dim % 8 != 0 || rows <= 0 || !ids || !residual) return -1;
+  return launch_rmsnorm<false, RN_EMBED>(out, nullptr, residual, table, w, rows, dim, eps, 0, stream, ids);
+}
+
+// out [rows, dim] = RMSNorm of (x + residual)'s rows ids[] * w; x and residual stay as they are
+CFC_API int cfc_rmsnorm_rows(void* out, const void* residual, const void* x, const int32_t* ids, const void* w, int rows, int dim,
+                             float eps, hipStream_t stream) {
+  if (dim % 8 != 0 || rows <= 0 || !ids || !residual) return -1;
+  return launch_rmsnorm<false, RN_ROWS>(out, nullptr, (void*)residual, x, w, rows, dim, eps, 1, stream, ids);
 }
 
 // FP8 output: out [rows, dim] e4m3fn, scale [rows] f32 with RMSNorm(...) ~= out * scale.
