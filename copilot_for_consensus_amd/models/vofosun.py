@@ -358,10 +358,11 @@ class VofosunModel:
         if plan is None:
             plan = self.plan_prefill(cu_q.tolist(), ctx_lens.tolist(), None)
             plan = {k: torch.as_tensor(v, device=ids.device) if isinstance(v, np.ndarray) else v for k, v in plan.items()}
-        hist, x = self._embed(ids)
+        bufs = {}
+        hist, x = self._embed(ids, bufs)
         T = ids.numel()
         rstd = torch.empty(T, dtype=torch.float32, device=ids.device)
-        cur, up, bufs = hist[0], None, {}
+        cur, up = hist[0], None
         for i, lw in enumerate(self.w.layers):
             S.depth_stats(cur, hist, up, self.cfg.norm_eps, x, rstd)
             cur = x
@@ -382,8 +383,9 @@ class VofosunModel:
         slices per sequence (the engine's form); ``shared_blocks`` is not used (latents are read once per
         token for all heads, through the caches)."""
         P = max(1, -part_blocks)
-        hist, x = self._embed(ids)
-        cur, up, bufs = hist[0], None, {}
+        bufs = {}
+        hist, x = self._embed(ids, bufs)
+        cur, up = hist[0], None
         for i, lw in enumerate(self.w.layers):
             hs = self._inputs(ids.numel(), lw, ids.device, bufs)
             S.depth_conv_decode(cur, hist, up, lw["norm"], self.cfg.norm_eps, lw["convs"], positions,
@@ -394,25 +396,25 @@ class VofosunModel:
             up = self._average(i, self._layer(i, hs, slots, ctx_lens, block_tables, kv, attn), hist, bufs)
         return S.depth_norm(cur, hist, up, self.w.final_norm, self.cfg.norm_eps, self.w.dtype)
 
-    def _embed(self, ids):
-        T = ids.numel()
-        hist = torch.empty(self.cfg.layers + 1, T, self.cfg.hidden, dtype=torch.float32, device=ids.device)
-        S.embed_f32(self.w.embed, ids, hist[0])
+    def _embed(self, ids, bufs):
+        """The stream's history with its first rows, and a buffer like one of them; the sublayers' inputs that have constant
+        columns, with these."""
+        T, W, dev = ids.numel(), self.cfg.hidden, ids.device
+        hist = torch.empty(self.cfg.layers + 1, T, W, dtype=torch.float32, device=dev)
+        ones = None
+        if any(len(lw["convs"]) > 1 and lw["fused_glu"] for lw in self.w.layers):
+            hs = bufs[True, True] = [torch.empty(T, W + n, dtype=self.w.dtype, device=dev) for n in (0, BIAS_COLS)]
+            ones = hs[1][:, W:]
+        S.embed_f32(self.w.embed, ids, hist[0], ones=ones)
         return hist, torch.empty_like(hist[0])
 
     def _inputs(self, T, lw, device, bufs):
-        """Activation buffers of the sublayers' inputs (the feed-forward's with its constant bias columns),
+        """Activation buffers of the sublayers' inputs (the feed-forward's with its constant bias columns, of :meth:`_embed`),
         one set per forward pass, kept in ``bufs``."""
-        W, two = self.cfg.hidden, len(lw["convs"]) > 1
-        wide = two and lw["fused_glu"]
+        two = len(lw["convs"]) > 1
+        wide = two and bool(lw["fused_glu"])
         if (two, wide) not in bufs:
-            hs = [torch.empty(T, W, dtype=self.w.dtype, device=device)]
-            if two:
-                hs.append(torch.empty(T, W + (BIAS_COLS if wide else 0), dtype=self.w.dtype, device=device))
-            if wide:
-                hs[1][:, W:].zero_()
-                hs[1][:, W].fill_(1.0)
-            bufs[two, wide] = hs
+            bufs[two, wide] = [torch.empty(T, self.cfg.hidden, dtype=self.w.dtype, device=device) for _ in range(1 + two)]
         return bufs[two, wide]
 
     def _average(self, i, part, hist, bufs) -> S.Update:

@@ -28,10 +28,16 @@ def sinusoid_turns(width: int, base: float, device) -> torch.Tensor:
     return torch.tensor(base ** (-2.0 * i / width) / (2.0 * np.pi), dtype=torch.float64, device=device)
 
 
-def embed_f32(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: float = 1.0, positions=None, turns=None) -> torch.Tensor:
+def embed_f32(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: float = 1.0, positions=None, turns=None,
+              ones: torch.Tensor | None = None) -> torch.Tensor:
     """Token rows times ``scale`` as fp32 into ``out`` [T, W]; with ``positions`` plus their sinusoids (``turns`` of
-    :func:`sinusoid_turns`)."""
+    :func:`sinusoid_turns`).  ``ones`` [T, n], row-strided, in the table's type: the first column ones, the others zeros."""
+    if ones is not None and (ones.dtype != table.dtype or ones.shape[0] != ids.numel() or ones.stride(1) != 1):
+        raise ValueError(f"embed_f32: ones {tuple(ones.shape)} {ones.dtype} beside {ids.numel()} rows of {table.dtype}")
     if not table.is_cuda:
+        if ones is not None:
+            ones.zero_()
+            ones[:, 0] = 1.0
         out.copy_(table[ids.long()])
         if scale != 1.0:
             out.mul_(scale)
@@ -44,7 +50,8 @@ def embed_f32(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: 
         _req(positions, torch.int32, "positions")
         _req(turns, torch.float64, "turns")
     check(kernels().cfc_embed_f32(out.data_ptr(), table.data_ptr(), ids.data_ptr(), ids.numel(), table.shape[1],
-                                  table.shape[0], _act(table.dtype), float(scale), _p(positions), _p(turns), _stream(table)),
+                                  table.shape[0], _act(table.dtype), float(scale), _p(positions), _p(turns), _p(ones),
+                                  ones.stride(0) if ones is not None else 0, ones.shape[1] if ones is not None else 0, _stream(table)),
           "cfc_embed_f32")
     return out
 

@@ -35,8 +35,14 @@ __device__ __forceinline__ void st1(float* p, float v) { *p = v; }
 template <typename TAB, int V>
 __global__ void __launch_bounds__(1024) embed_f32_kernel(float* __restrict__ out, const TAB* __restrict__ table,
                                                         const int32_t* __restrict__ ids, int W, int vocab, float scale,
-                                                        const int32_t* __restrict__ positions, const double* __restrict__ turns) {
+                                                        const int32_t* __restrict__ positions, const double* __restrict__ turns,
+                                                        TAB* __restrict__ ones, int64_t ldo, int n_ones) {
   const int t = blockIdx.x;
+  // constant columns beside the rows of a product's input: launches of their own cost 2.8 us each
+  for (int c = threadIdx.x; c < n_ones; c += blockDim.x) {
+    const Vec<1> v{{c ? 0.f : 1.f}};
+    stv<1>(ones + t * ldo + c, v);
+  }
   const int id = min(max(ids[t], 0), vocab - 1);
   const double pos = positions ? positions[t] : 0;
   const TAB* row = table + (size_t)id * W;
@@ -524,13 +530,14 @@ int conv_launch(dim3 grid, hipStream_t s, const float* x, const float* rstd, con
 
 // table: bf16 (f32 = 0) or fp32 rows; ids outside [0, vocab) are clamped
 // positions (null: none): entries 2i and 2i + 1 get the sine and the cosine of positions * turns[i] turns
+// ones: n_ones columns of rows of stride ldo, in the table's type, the first of them one and the others zero
 CFC_API int cfc_embed_f32(float* out, const void* table, const int32_t* ids, int T, int W, int vocab, int f32, float scale,
-                          const int32_t* positions, const double* turns, hipStream_t stream) {
+                          const int32_t* positions, const double* turns, void* ones, int64_t ldo, int n_ones, hipStream_t stream) {
   if (T <= 0) return 0;
-  if (W <= 0 || vocab <= 0 || (positions && !turns)) return -1;
+  if (W <= 0 || vocab <= 0 || (positions && !turns) || n_ones < 0 || (n_ones && !ones)) return -1;
   const bool v4 = W % 4 == 0 && (((uintptr_t)out | (uintptr_t)table) & 15) == 0;
   const int vecs = v4 ? W / 4 : W, threads = vecs <= 256 ? 256 : vecs <= 512 ? 512 : 1024;
-#define EM(TAB, V) embed_f32_kernel<TAB, V><<<T, threads, 0, stream>>>(out, (const TAB*)table, ids, W, vocab, scale, positions, turns)
+#define EM(TAB, V) embed_f32_kernel<TAB, V><<<T, threads, 0, stream>>>(out, (const TAB*)table, ids, W, vocab, scale, positions, turns, (TAB*)ones, ldo, n_ones)
   if (f32) { if (v4) EM(float, 4); else EM(float, 1); }
   else if (v4) EM(uint16_t, 4);
   else EM(uint16_t, 1);

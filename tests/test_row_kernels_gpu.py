@@ -43,6 +43,21 @@ def test_embedded_rows(W, dtype, place):
     assert torch.equal(again, out)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("W,T,n,gap", [(5, 3, 1, 0), (4096, 300, 64, 0), (1020, 2, 1500, 3)])
+def test_constant_columns_beside_embedded_rows(W, T, n, gap, dtype):
+    from copilot_for_consensus_amd.ops import stream
+    table = torch.randn(9, W, device=DEV).to(dtype)
+    ids = torch.arange(T, dtype=torch.int32, device=DEV) % 9
+    rows = torch.full((T, W + n + gap), 5.0, dtype=dtype, device=DEV)
+    out = stream.embed_f32(table, ids, torch.empty(T, W, device=DEV), ones=rows[:, W:W + n])
+    out = torch.empty(T, W, device=DEV) if out is None else out
+    assert bool((rows[:, W] == 1).all()) and not rows[:, W + 1:W + n].any()
+    assert bool((rows[:, :W] == 5).all()) and bool((rows[:, W + n:] == 5).all())
+    with pytest.raises(ValueError):
+        stream.embed_f32(table, ids, out, ones=rows[:-1, W:])
+
+
 @pytest.mark.parametrize("dim,T", [(8, 1), (512, 7), (4096, 300), (4104, 5), (8200, 3), (24576, 2), (65536, 2)])
 def test_norms_of_gathered_rows(dim, T):
     """The norm that begins a stream and that of its last rows: the bits of gathering, copying and norming one after the other."""
