@@ -53,6 +53,16 @@ struct KnnRows {
       qf[c] = as_bf16x8(qv ? *reinterpret_cast<const uint4*>(qr + 32 * c + 8 * g) : make_uint4(0, 0, 0, 0));
     qn = (qnorm2 && qv) ? qnorm2[col] : 0.f;
   }
+  // from what KnnFloats::put left in LDS
+  __device__ __forceinline__ void queries(const char* lds, const float* n2, int nq, int row_bytes) {
+    const int col = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    const bool qv = col < nq;
+    const char* qr = lds + (qv ? col : 0) * row_bytes;
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+      qf[c] = as_bf16x8(qv ? *reinterpret_cast<const uint4*>(qr + 64 * c + 16 * g) : make_uint4(0, 0, 0, 0));
+    qn = qv ? n2[col] : 0.f;
+  }
   __device__ __forceinline__ void load(uint4* a, int r0) const {
     const int col = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
     const uint16_t* xr = X + (size_t)min(r0 + col, N - 1) * (KC * 32);
@@ -112,21 +122,90 @@ struct KnnRows {
   }
 };
 
+// Queries of floats to LDS, as l2_normalize_kernel takes them to memory, a wave a query, to the bit: the workgroups of a round each do
+// so beside their first rows' way from memory, and a search has a launch less (us: 1 query of 20 k rows of 384 17.0 -> 14.3, of 27 k of
+// 768 19.4 -> 16.3, 4 queries of 27 k of 384 17.8 -> 15.6, 1 of 1M 136 -> 133.7, 16 163 -> 159.6).  Asked for before the rows are, by four
+// waves; FROWS queries at most, for which there is room beside the rings.
+template <int KC>
+struct KnnFloats {
+  static constexpr int FROWS = KC <= 16 ? 16 : 8, ROW = KC * 64 + 16, NV = (KC * 4 + 63) / 64, BYTES = FROWS * ROW;
+  uint4 v[FROWS / 4][NV][2];
+  __device__ __forceinline__ void ask(const float* q, int nq) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < FROWS / 4; ++i)
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        const uint4* src = reinterpret_cast<const uint4*>(q + (size_t)min(w + 4 * i, nq - 1) * (KC * 32)) + 2 * min(lane + 64 * j, KC * 4 - 1);
+        v[i][j][0] = src[0];
+        v[i][j][1] = src[1];
+      }
+  }
+  __device__ __forceinline__ void put(char* lds, float* n2, int nq, bool unit) const {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < FROWS / 4; ++i) {
+      if (w + 4 * i >= nq) break;
+      uint4 b[NV];
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        const uint4 x = v[i][j][0], y = v[i][j][1];
+        b[j] = make_uint4(pack2bf(__uint_as_float(x.x), __uint_as_float(x.y)), pack2bf(__uint_as_float(x.z), __uint_as_float(x.w)),
+                          pack2bf(__uint_as_float(y.x), __uint_as_float(y.y)), pack2bf(__uint_as_float(y.z), __uint_as_float(y.w)));
+        float f[8];
+        unpack8(b[j], f);
+        if (lane + 64 * j < KC * 4)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
+      }
+      ss = wave_sum(ss);
+      if (lane == 0) n2[w + 4 * i] = ss;
+      const float inv = ss > 0.f ? rsqrtf(ss) : 0.f;
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        float f[8];
+        unpack8(b[j], f);
+        if (unit) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] *= inv;
+        }
+        if (lane + 64 * j < KC * 4) *reinterpret_cast<uint4*>(lds + (w + 4 * i) * ROW + 16 * (lane + 64 * j)) = pack8(f);
+      }
+    }
+  }
+};
+
 // One wave scores a block of B rows (16, 32 or 64) against all queries.  Every lane holds four rows' scores of one query;
 // they are stored as they lie and their largest key goes to bmax [nq][nb].  Nothing is selected here, so the pass is a plain
 // stream over X: 1M x 384 bf16 with one query in 131 us (5.9 TB/s) where scoring 2048-row chunks into LDS and selecting in
 // them took 172 us (4.5 TB/s; 489 workgroups, two on most CUs and one on the rest, the selecting wave alone at each one's end).
 // MAXIMA: only the best score of every 16 rows is stored, to out [nq][ld] (B = 64).  A wave takes every gridDim-th block.
-template <int KC, bool MAXIMA>
-__global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
+// FQ: the queries are floats, taken to unit length if `unit` (KC <= 16).
+template <int KC, bool MAXIMA, bool FQ = false>
+__global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restrict__ X, const void* __restrict__ Q, int N,
                                                        int nq, const float* __restrict__ xnorm2,
                                                        const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
                                                        float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
-                                                       int B) {
+                                                       int B, bool unit) {
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const bool qv = col < nq;
   KnnRows<KC> rows{X, N, xnorm2, alive};
-  rows.queries(Q, qnorm2, nq);
+  uint4 a[KC <= 16 ? 2 : 1][KC];
+  if constexpr (FQ) {
+    static_assert(KC <= 16, "");
+    __shared__ __attribute__((aligned(16))) char qs[KnnFloats<KC>::BYTES];
+    __shared__ float n2[KnnFloats<KC>::FROWS];
+    KnnFloats<KC> f;
+    f.ask((const float*)Q, nq);
+    rows.load(a[0], min((int)(blockIdx.x * 4 + (threadIdx.x >> 6)), nb - 1) * B);
+    f.put(qs, n2, nq, unit);
+    __syncthreads();
+    rows.queries(qs, n2, nq, KnnFloats<KC>::ROW);
+  } else {
+    rows.queries((const uint16_t*)Q, qnorm2, nq);
+  }
+  bool first = FQ;
   const bool vec = (ld & 3) == 0 && ((uintptr_t)out & 15) == 0;
   for (int blk = blockIdx.x * 4 + (threadIdx.x >> 6); blk < nb; blk += gridDim.x * 4) {
     const int lo = blk * B, hi = min(N, lo + B);
@@ -151,8 +230,8 @@ __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restric
       }
     };
     if constexpr (KC <= 16) {          // the next 16 rows in flight under these (144 -> 131 us); wider rows fill the registers alone
-      uint4 a[2][KC];
-      rows.load(a[0], lo);
+      if (!first) rows.load(a[0], lo);
+      first = false;
       for (int r0 = lo; r0 < hi; r0 += 32) {
         if (r0 + 16 < hi) rows.load(a[1], r0 + 16);
         take(a[0], r0);
@@ -160,10 +239,9 @@ __global__ void __launch_bounds__(256) knn_scan_kernel(const uint16_t* __restric
         if (r0 + 16 < hi) take(a[1], r0 + 16);
       }
     } else {
-      uint4 a[KC];
       for (int r0 = lo; r0 < hi; r0 += 16) {
-        rows.load(a, r0);
-        take(a, r0);
+        rows.load(a[0], r0);
+        take(a[0], r0);
       }
     }
     if constexpr (MAXIMA) {
@@ -192,23 +270,25 @@ struct KnnUnit {
   static_assert(KC % KU == 0 && KU % 4 == 0 && 4 * R * KU <= 160, "");
 };
 
-// WORDS: there are norms or a mask
-template <int KC, bool MAXIMA, bool WORDS>
-__global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
+// WORDS: there are norms or a mask.  FQ: the queries are floats, as above
+template <int KC, bool MAXIMA, bool WORDS, bool FQ = false>
+__global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __restrict__ X, const void* __restrict__ Q, int N,
                                                             int nq, const float* __restrict__ xnorm2,
                                                             const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
                                                             float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
-                                                            int B) {
+                                                            int B, bool unit) {
   constexpr int KU = KnnUnit<KC>::KU, R = KnnUnit<KC>::R, NU = KnnUnit<KC>::NU, UB = KU * 1024;
   __shared__ __attribute__((aligned(16))) char kn_smem[4 * R * (UB + (WORDS ? 256 : 0))];      // rings, then those of norms and masks
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), stride = gridDim.x * 4;
   const bool qv = col < nq;
   KnnRows<KC> rows{X, N, xnorm2, alive};
-  rows.queries(Q, qnorm2, nq);
+  KnnFloats<KC> f;
+  if constexpr (FQ) f.ask((const float*)Q, nq);
+  else rows.queries((const uint16_t*)Q, qnorm2, nq);
   const bool vec = (ld & 3) == 0 && ((uintptr_t)out & 15) == 0;
   int blk = blockIdx.x * 4 + w;
-  if (blk >= nb) return;
+  if (!FQ && blk >= nb) return;
   const char* ring = kn_smem + w * (R * UB);
   const uint32_t lds0 = lds_at(ring);
   const char* words = kn_smem + 4 * R * UB + w * (R * 256);
@@ -250,6 +330,13 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
   };
 #pragma unroll
   for (int i = 0; i < R - 1; ++i) issue();
+  if constexpr (FQ) {
+    __shared__ __attribute__((aligned(16))) char qs[KnnFloats<KC>::BYTES];
+    __shared__ float n2[KnnFloats<KC>::FROWS];
+    f.put(qs, n2, nq, unit);
+    __syncthreads();
+    rows.queries(qs, n2, nq, KnnFloats<KC>::ROW);
+  }
   int slot = 0, wslot = 0;
   for (; blk < nb; blk += stride) {
     const int lo = blk * B, hi = min(N, lo + B);
@@ -926,29 +1013,47 @@ constexpr int KNN_CUS = 256;
 // LDS-DMA's sources are whole sixteens of bytes; rows that lie otherwise come to registers
 bool knn_aligned(const void* X) { return ((uintptr_t)X & 15) == 0; }
 
-#define KNN_ARGS(OUT, B) (const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, qnorm2, alive, OUT, (size_t)ld, B
+#define KNN_ARGS(OUT, B) (const uint16_t*)X, Q, N, nq, xnorm2, qnorm2, alive, OUT, (size_t)ld, B
 
-// Scores of rows [0, N) of X for nq queries into out [nq][ld], and the largest key of every cfc_topk_block(N) rows into
-// bmax [nq][blocks] (null: not wanted), which has room for `room` of them.
-CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
-                         const uint8_t* alive, float* out, long ld, uint32_t* bmax, long room, hipStream_t stream) {
+// floats: where Q holds floats the scan takes them itself, if its workgroups are no more than a round (each takes the queries to LDS) and
+// these fit beside the rings; where it does not, *floats is cleared and nothing launched
+static int knn_scan_go(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
+                       const uint8_t* alive, float* out, long ld, uint32_t* bmax, long room, hipStream_t stream, bool* floats, bool unit) {
   if (nq < 1 || nq > 16 || dim % 32 != 0 || N <= 0 || ld < N) return -1;
   const int B = cfc_topk_block(N), nb = (N - 1) / B + 1;
   if (bmax && (long)nq * nb > room) return -1;
   const int all = (nb + 3) / 4;
   const long bytes = (long)N * dim * 2;
-#define KS(KC)                                                                                                             \
-  if constexpr (KC > 4)                                                                                                    \
-    if (knn_aligned(X) && (KC > 16 || bytes > KNN_STREAM_BYTES)) {                                                         \
-      if (xnorm2 || alive) knn_stream_kernel<KC, false, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B); \
-      else knn_stream_kernel<KC, false, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B);         \
-      break;                                                                                                               \
-    }                                                                                                                      \
-  knn_scan_kernel<KC, false><<<KC <= 16 && bytes <= KNN_ROUND_BYTES ? min(all, KNN_ROUND) : all, 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B); \
-  break
+#define ST(KC, W, F) knn_stream_kernel<KC, false, W, F><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B, unit)
+#define SC(KC, F) knn_scan_kernel<KC, false, F><<<grid, 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B, unit)
+#define KS(KC)                                                                                         \
+  {                                                                                                    \
+    if constexpr (KC > 4)                                                                              \
+      if (knn_aligned(X) && (KC > 16 || bytes > KNN_STREAM_BYTES)) {                                   \
+        if (floats && nq > KnnFloats<KC>::FROWS) { *floats = false; return 0; }                        \
+        if (xnorm2 || alive) { if (floats) ST(KC, true, true); else ST(KC, true, false); }             \
+        else { if (floats) ST(KC, false, true); else ST(KC, false, false); }                           \
+        break;                                                                                         \
+      }                                                                                                \
+    const int grid = KC <= 16 && bytes <= KNN_ROUND_BYTES ? min(all, KNN_ROUND) : all;                 \
+    if constexpr (KC <= 16)                                                                            \
+      if (floats && grid <= KNN_ROUND) { SC(KC, true); break; }                                        \
+    if (floats) { *floats = false; return 0; }                                                         \
+    SC(KC, false);                                                                                     \
+    break;                                                                                             \
+  }
   KNN_DIMS(KS)
 #undef KS
+#undef SC
+#undef ST
   return CFC_CHECK_LAUNCH();
+}
+
+// Scores of rows [0, N) of X for nq queries into out [nq][ld], and the largest key of every cfc_topk_block(N) rows into
+// bmax [nq][blocks] (null: not wanted), which has room for `room` of them.
+CFC_API int cfc_knn_scan(const void* X, const void* Q, int N, int nq, int dim, const float* xnorm2, const float* qnorm2,
+                         const uint8_t* alive, float* out, long ld, uint32_t* bmax, long room, hipStream_t stream) {
+  return knn_scan_go(X, Q, N, nq, dim, xnorm2, qnorm2, alive, out, ld, bmax, room, stream, nullptr, false);
 }
 
 // The best score of every 16 rows of [0, N) of X for nq queries, into out [nq][ld].
@@ -959,11 +1064,11 @@ CFC_API int cfc_knn_maxima(const void* X, const void* Q, int N, int nq, int dim,
 #define KS(KC)                                                                                                              \
   if constexpr (KC > 4)                                                                                                     \
     if (knn_aligned(X)) {                                                                                                   \
-      if (xnorm2 || alive) knn_stream_kernel<KC, true, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64); \
-      else knn_stream_kernel<KC, true, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);       \
+      if (xnorm2 || alive) knn_stream_kernel<KC, true, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64, false); \
+      else knn_stream_kernel<KC, true, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64, false);       \
       break;                                                                                                                \
     }                                                                                                                       \
-  knn_scan_kernel<KC, true><<<all, 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);                                       \
+  knn_scan_kernel<KC, true><<<all, 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64, false);                                       \
   break
   KNN_DIMS(KS)
 #undef KS
@@ -1026,7 +1131,7 @@ static KnnRoom knn_room(int N, int nq, int dim) {
 CFC_API int64_t cfc_knn_search_bytes(int N, int nq, int dim) { return N < 1 || nq < 1 || dim < 1 ? -1 : knn_room(N, nq, dim).bytes; }
 
 // A flat search of floats q [nq][dim] (16-byte aligned) from end to end by one call, whose host takes as long as the GPU does for an
-// index of up to some 100 k rows (20 k rows, 1 query: three calls 27.1 us, this 16.8): queries, scores, the k best of N rows
+// index of up to some 100 k rows (20 k rows, 1 query: three calls 27.1 us, this 14.3): queries, scores, the k best of N rows
 // that cfc_topk_select takes in one segment.  As cfc_knn_queries, cfc_knn_scan and cfc_topk_select; ws 16-byte aligned.
 CFC_API int cfc_knn_search(const void* X, const float* q, int unit, int N, int nq, int dim, const float* xnorm2, const uint8_t* alive,
                            int k, long row0, void* ws, int64_t room, float* out_v, int64_t* out_i, hipStream_t stream) {
@@ -1035,6 +1140,10 @@ CFC_API int cfc_knn_search(const void* X, const float* q, int unit, int N, int n
   if (room < r.bytes) return -1;
   char* const p = (char*)ws;
   float *const n2 = (float*)(p + r.n2), *const scores = (float*)(p + r.scores);
+  bool floats = true;
+  if (const int e = knn_scan_go(X, q, N, nq, dim, xnorm2, nullptr, alive, scores, r.ld, (uint32_t*)ws, nq * r.nb, stream, &floats, unit))
+    return e;
+  if (floats) return cfc_topk_select(scores, nullptr, nq, N, r.ld, k, (uint32_t*)ws, nq * r.nb, 0, row0, out_v, out_i, stream);
   if (const int e = cfc_knn_queries(p + r.q, q, n2, unit, nq, dim, stream)) return e;
   if (const int e = cfc_knn_scan(X, p + r.q, N, nq, dim, xnorm2, n2, alive, scores, r.ld, (uint32_t*)ws, nq * r.nb, stream)) return e;
   return cfc_topk_select(scores, nullptr, nq, N, r.ld, k, (uint32_t*)ws, nq * r.nb, 0, row0, out_v, out_i, stream);

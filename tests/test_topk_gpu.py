@@ -285,3 +285,23 @@ def test_a_search_by_one_call(lo, n, nq, k, unit, dead):
     for bad in (dict(k=0), dict(k=257), dict(row_lo=-1), dict(N=len(X) + 1)):
         with pytest.raises(ValueError):
             K.knn_search(X, q, **{"k": k, "unit": unit, "row_lo": lo, "N": lo + n, **bad})
+
+
+@pytest.mark.parametrize("dim,n", [(128, 17), (256, 40_001), (256, 600_000), (384, 20_000), (384, 250_000), (384, 400_001), (512, 300_000), (768, 5_003),
+                                   (1024, 1_000)])
+@pytest.mark.parametrize("nq,unit,dead", [(1, True, False), (4, False, False), (5, True, True), (8, False, True), (9, True, False), (16, False, True)])
+def test_float_queries_in_the_scan(dim, n, nq, unit, dead):
+    """Queries that the scan's workgroups take to LDS themselves, by fragments and by rings, and those that are too many or whose
+    workgroups are: the bits of a launch for the queries.  A query of zeros and one that is not finite among them."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(n + nq)
+    X = torch.randn(n, dim, device="cuda", generator=g).bfloat16()
+    q = torch.randn(nq, dim, device="cuda", generator=g) * 3.0
+    if nq > 4:
+        q[1], q[4, dim - 1] = 0.0, float("inf")
+    norms = None if unit else X.float().pow(2).sum(1)
+    alive = torch.rand(n, device="cuda", generator=g) < 0.9 if dead else None
+    Q, n2 = K.knn_queries(q, unit)
+    k = min(150, n)
+    want, got = K.knn_topk(X, Q, k, norms, n2, alive, 0, n), K.knn_search(X, q, k, unit, norms, alive, 0, n)
+    assert torch.equal(got[0].view(torch.int32), want[0].view(torch.int32)) and torch.equal(got[1], want[1])
