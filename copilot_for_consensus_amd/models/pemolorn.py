@@ -453,10 +453,12 @@ class PemolornModel:
         decode, hs = io.plan is None, h[None]
         c = lw["in"].joint(hs) if decode else lw["in"].prompt(hs)
         b = N.Branch(lw["norm1b"], self.cfg.norm_eps)
-        s = None
+        s = step = None
         if "gru" in lw:
             s = self._recur(i, c[1], io)
-        o = self._attend(i, c[0], io)
+            if decode:
+                step, s = s, s.out
+        o = self._attend(i, c[0], io, step)
         if s is None:
             b.y = self._sum(lw["o"].slabs(o))
         else:
@@ -464,11 +466,11 @@ class PemolornModel:
             b.y2 = self._sum(lw["o2"].slabs(s))
         return b
 
-    def _attend(self, i, cols: Cols, io: _Pass) -> torch.Tensor:
-        """Attention of layer i: its heads' outputs [T, H vdim]."""
+    def _attend(self, i, cols: Cols, io: _Pass, step=None) -> torch.Tensor:
+        """Attention of layer i: its heads' outputs [T, H vdim]; beside its decoded rows a recurrence's ``step``."""
         a, rows, tail = self.w.layers[i]["heads"], io.kv.heads[i], io.kv.tail[i]
         if io.plan is None:
-            q = A.qkv_rows(a, cols, rows, io.positions, io.slots, io.states, io.block_tables, tail)
+            q = A.qkv_rows(a, cols, rows, io.positions, io.slots, io.states, io.block_tables, tail, beside=step)
             return A.attention(a, q, rows, io.block_tables, io.ctx_lens, P=io.P, workspace=io.workspace)
         p = io.plan
         q = A.qkv_rows(a, cols, rows, io.positions, io.slots, p["row_states"], io.block_tables, tail, p["lead"])
@@ -477,14 +479,14 @@ class PemolornModel:
             A.pool_rows(a, rows, p[f"ended_{a.mask.pool}"], io.block_tables)
         return A.attention(a, q, rows, io.block_tables, io.ctx_lens, io.cu_q, p[self._tiles(a)])
 
-    def _recur(self, i, cols: Cols, io: _Pass) -> torch.Tensor:
-        """Recurrence of layer i: its gated states [T, width]."""
+    def _recur(self, i, cols: Cols, io: _Pass):
+        """Recurrence of layer i: its gated states [T, width]; of decoded rows the step that leaves them."""
         g, state = self.w.layers[i]["gru"], io.kv.recur[i]
         n = g.width
         zxg = [Cols(cols.t, cols.c0 + k * n, n) for k in range(3)]
         out = torch.empty(cols.rows, n, dtype=self.w.dtype, device=cols.t.device)
         if io.plan is None:
-            return R.step(g, *zxg, io.states, io.ctx_lens, state, out)
+            return R.Step(g, *zxg, io.states, io.ctx_lens, state, out)
         return R.prefill(g, *zxg, io.states, io.cu_q, io.ctx_lens, io.plan["chunks"], io.plan["chunk_cu"], state, out)
 
     def _sum(self, slabs) -> torch.Tensor:

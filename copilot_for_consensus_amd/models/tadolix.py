@@ -468,27 +468,28 @@ class TadolixModel:
             return self._sum(lw["o"].slabs(self._lru(lw["lru"], run, c[0], io)))
         a, n = lw["heads"], lw["gru"].width
         both = torch.empty(h.shape[0], a.H * a.vdim + n, dtype=self.w.dtype, device=h.device)
-        self._recur(lw["gru"], run, c[1], io, m.right_scale, both[:, a.H * a.vdim:])
-        self._attend(a, run, c[0], c[2], io, m.left_scale, both[:, :a.H * a.vdim])
+        step = self._recur(lw["gru"], run, c[1], io, m.right_scale, both[:, a.H * a.vdim:])
+        self._attend(a, run, c[0], c[2], io, m.left_scale, both[:, :a.H * a.vdim], step)
         return self._sum(lw["o"].slabs(both))
 
-    def _attend(self, a: A.Heads, run, cols: Cols, gate: Cols, io: _Pass, factor, out) -> None:
+    def _attend(self, a: A.Heads, run, cols: Cols, gate: Cols, io: _Pass, factor, out, step=None) -> None:
+        """``step``: a recurrence's, beside decoded rows."""
         rows = io.kv.heads[run]
         if io.plan is None:
-            q = A.qkv_rows(a, cols, rows, io.positions, io.slots, io.states, io.block_tables)
+            q = A.qkv_rows(a, cols, rows, io.positions, io.slots, io.states, io.block_tables, beside=step)
             A.attention(a, q, rows, io.block_tables, io.ctx_lens, P=io.P, workspace=io.workspace, gate=gate, factor=factor, out=out)
             return
         p = io.plan
         q = A.qkv_rows(a, cols, rows, io.positions, io.slots, p["row_states"], io.block_tables, None, p["lead"])
         A.attention(a, q, rows, io.block_tables, io.ctx_lens, io.cu_q, p[self._tiles(a)], gate=gate, factor=factor, out=out)
 
-    def _recur(self, g: R.Gru, run, cols: Cols, io: _Pass, factor, out) -> None:
+    def _recur(self, g: R.Gru, run, cols: Cols, io: _Pass, factor, out) -> R.Step | None:
+        """The recurrence into ``out``; of decoded rows the step that does."""
         state = io.kv.recur[run]
         zxg = [Cols(cols.t, cols.c0 + k * g.width, g.width) for k in range(3)]
         if io.plan is None:
-            R.step(g, *zxg, io.states, io.ctx_lens, state, out, factor)
-        else:
-            R.prefill(g, *zxg, io.states, io.cu_q, io.ctx_lens, io.plan["chunks"], io.plan["chunk_cu"], state, out, factor)
+            return R.Step(g, *zxg, io.states, io.ctx_lens, state, out, factor)
+        R.prefill(g, *zxg, io.states, io.cu_q, io.ctx_lens, io.plan["chunks"], io.plan["chunk_cu"], state, out, factor)
 
     def _lru(self, r: L.RgLru, run, cols: Cols, io: _Pass) -> torch.Tensor:
         y, x = (Cols(cols.t, cols.c0 + k * r.width, r.width) for k in range(2))

@@ -148,25 +148,34 @@ def rope_freq(dims: int, base: float, device) -> torch.Tensor | None:
     return torch.tensor(f, dtype=torch.float32, device=device)
 
 
-def qkv_rows(a: Heads, cols: Cols, rows, positions, slots, states, block_tables, tail=None, lead=None) -> torch.Tensor:
+def qkv_rows(a: Heads, cols: Cols, rows, positions, slots, states, block_tables, tail=None, lead=None, beside=None) -> torch.Tensor:
     """Projections [q | k | v] of packed rows to queries [T, H, D] (scaled by ``q_scale``) and rows of the cache ``rows``
     (runtime.kv_cache.PagedHeads) at ``slots``.  ``lead``: rows of the same portion before each row (prompts: afterwards
     :func:`conv_tail` and :func:`pool_rows`); None: one token per sequence, whose state in ``tail`` [states, taps - 1, C]
-    and pooled entries are written here."""
+    and pooled entries are written here.  ``beside`` (ops.gru.Step, of the same sequences): run in the same launch."""
     T, dt = cols.rows, rows.k.dtype
     if cols.n != a.columns or rows.k.shape[1] != a.G or rows.k.shape[3] != a.D:
         raise ValueError(f"qkv_rows: {cols.n} columns of {a.columns}, cache {tuple(rows.k.shape)}")
+    if beside is not None and (lead is not None or beside.slots is not states or beside.out.shape[0] != T or beside.out.dtype != dt):
+        raise ValueError("qkv_rows: a step beside it is one of the same decoded rows")
     if not rows.k.is_cuda:
+        if beside is not None:
+            beside.run()
         return _qkv_ref(a, cols, rows, positions, slots, states, block_tables, tail, lead, dt)
     for name, t in (("positions", positions), ("slots", slots)):
         _req(t, torch.int32, name)
     q = (torch.empty if a.D == a.dim else torch.zeros)(T, a.H, a.D, dtype=dt, device=rows.k.device)
     rot = 2 * a.freq.numel() if a.freq is not None else 0
-    check(kernels().cfc_qkv_rows(_act(dt), *cols.args(dt), T, a.H, a.G, a.dim, a.vdim, a.D, 1 if a.shared else 3, _p(a.q_norm),
-                                 _p(a.k_norm), int(a.per_head), float(a.eps), _p(a.freq), rot, float(a.q_scale), _p(a.conv),
-                                 a.taps, _p(tail), _p(lead), _p(states), positions.data_ptr(), slots.data_ptr(), q.data_ptr(),
-                                 rows.k.data_ptr(), rows.v.data_ptr(), _p(rows.pk), _p(rows.pv), a.mask.pool, rows.log2_entries,
-                                 block_tables.data_ptr(), block_tables.shape[1], _stream(q)), "cfc_qkv_rows")
+    args = [_act(dt), *cols.args(dt), T, a.H, a.G, a.dim, a.vdim, a.D, 1 if a.shared else 3, _p(a.q_norm),
+            _p(a.k_norm), int(a.per_head), float(a.eps), _p(a.freq), rot, float(a.q_scale), _p(a.conv),
+            a.taps, _p(tail), _p(lead), _p(states), positions.data_ptr(), slots.data_ptr(), q.data_ptr(),
+            rows.k.data_ptr(), rows.v.data_ptr(), _p(rows.pk), _p(rows.pv), a.mask.pool, rows.log2_entries,
+            block_tables.data_ptr(), block_tables.shape[1]]
+    if beside is not None:
+        _req(states, torch.int32, "states")
+        check(kernels().cfc_qkv_rows_gru(*args, *beside.args(), _stream(q)), "cfc_qkv_rows_gru")
+    else:
+        check(kernels().cfc_qkv_rows(*args, _stream(q)), "cfc_qkv_rows")
     return q
 
 

@@ -75,6 +75,30 @@ def step(p: Gru, z: Cols, u: Cols, g: Cols, slots, ctx_lens, state, out, factor:
     return out
 
 
+@dataclasses.dataclass
+class Step:
+    """:func:`step`'s arguments, for a launch that does something else beside it (ops.gqa.qkv_rows)."""
+    p: Gru
+    z: Cols
+    u: Cols
+    g: Cols
+    slots: torch.Tensor
+    ctx_lens: torch.Tensor
+    state: torch.Tensor
+    out: torch.Tensor
+    factor: float = 1.0
+
+    def run(self) -> torch.Tensor:
+        return step(self.p, self.z, self.u, self.g, self.slots, self.ctx_lens, self.state, self.out, self.factor)
+
+    def args(self) -> list:
+        """What the native step takes from the products' columns on, without the slots and the number of rows."""
+        _req(self.ctx_lens, torch.int32, "ctx_lens")
+        ops = [x for c in _fits(self.p, (self.z, self.u, self.g), self.out, self.state) for x in c]
+        return ops + [self.p.bz.data_ptr(), self.p.bx.data_ptr(), self.ctx_lens.data_ptr(), self.p.width, self.state.data_ptr(),
+                      self.out.data_ptr(), self.out.stride(0), float(self.factor)]
+
+
 def prefill(p: Gru, z: Cols, u: Cols, g: Cols, slots, cu_q, ctx_lens, chunks, chunk_cu, state, out, factor: float = 1.0) -> torch.Tensor:
     """Packed portions, ``z``, ``u``, ``g`` activations (``chunks``, ``chunk_cu`` of :func:`chunk_plan` on the device)."""
     if not out.is_cuda:

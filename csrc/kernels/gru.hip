@@ -7,23 +7,9 @@
 //                 it adds to a state of zero
 //   * carry       per sequence through its chunks: the state ahead of each, and the one the portion leaves (recur.h)
 //   * gru_apply   the chunks again from their states: outputs
-#include "recur.h"
+#include "gru_step.h"
 
 namespace {
-
-struct GruCols { const void* p; int split; int64_t ld, plane; };      // split 0: activations, else fp32 slabs
-
-// decay 1 - z and contribution z c of one token.  With t = exp(pre_z): 1 - z = 1 / (1 + t) and z = t / (1 + t), neither
-// the other's difference from 1, so that small ones keep their digits; sigmoid(min(u, 0)) is 1/2 where u >= 0
-template <typename ACT>
-__device__ __forceinline__ void gru_gates(float pz, float u, float& a, float& b) {
-  const float t = exp_of<ACT>(fminf(pz, 60.f)), v = exp_of<ACT>(fminf(u, 0.f));
-  a = over1<ACT>(t);
-  b = t * a * (fmaxf(u, 0.f) + v * over1<ACT>(v));
-}
-
-template <typename ACT>
-__device__ __forceinline__ float silu(float g) { return g * over1<ACT>(exp_of<ACT>(fminf(-g, 60.f))); }
 
 // V activations as loaded
 template <typename ACT, int V> struct Raw;
@@ -47,32 +33,8 @@ template <typename ACT> struct Raw<ACT, 1> {
 };
 
 template <typename ACT, int V>
-__global__ void __launch_bounds__(64) gru_step_kernel(GruCols z, GruCols u, GruCols g, const float* __restrict__ bz,
-                                                     const float* __restrict__ bx, const int32_t* __restrict__ slots,
-                                                     const int32_t* __restrict__ ctx_lens, int W, float* __restrict__ state,
-                                                     ACT* __restrict__ out, int64_t ldo, float oscale) {
-  const int b = blockIdx.x, c = (blockIdx.y * 64 + threadIdx.x) * V;
-  if (c >= W) return;
-  // all at once; the state last, as it waits for its index (32 rows of 4096: 6.3 -> 4.9 us)
-  ColsIn<ACT, V> zi, ui, gi;
-  zi.ask(z.p, z.split, z.plane, b * z.ld + c);
-  ui.ask(u.p, u.split, u.plane, b * u.ld + c);
-  gi.ask(g.p, g.split, g.plane, b * g.ld + c);
-  const Vec<V> vz = ldv<V>(bz + c), vx = ldv<V>(bx + c);
-  float* sp = state + (size_t)slots[b] * W + c;
-  Vec<V> S = ctx_lens[b] > 1 ? ldv<V>(sp) : zerov<V>();
-  const Vec<V> zv = zi.get(z.p, z.split, z.plane, b * z.ld + c), uv = ui.get(u.p, u.split, u.plane, b * u.ld + c);
-  const Vec<V> gv = gi.get(g.p, g.split, g.plane, b * g.ld + c);
-  Vec<V> o;
-#pragma unroll
-  for (int e = 0; e < V; ++e) {
-    float a, k;
-    gru_gates<ACT>(zv.v[e] + vz.v[e], uv.v[e] + vx.v[e], a, k);
-    S.v[e] = a * S.v[e] + k;
-    o.v[e] = S.v[e] * silu<ACT>(gv.v[e]) * oscale;
-  }
-  stv<V>(sp, S);
-  stv<V>(out + b * ldo + c, o);
+__global__ void __launch_bounds__(64) gru_step_kernel(GruStep s) {
+  gru_step_row<ACT, V>(s, blockIdx.x, (blockIdx.y * 64 + threadIdx.x) * V);
 }
 
 constexpr int GRU_FLIGHT = 8;        // rows requested ahead of their use
@@ -160,14 +122,6 @@ __global__ void __launch_bounds__(64) gru_apply_kernel(GruRows z, GruRows u, Gru
     }
 }
 
-// vectors of four where every operand's rows allow them
-bool gru_vec(const GruCols* a, int n, int W, int f32, const void* out, int64_t ldo) {
-  bool v = W % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out & (f32 ? 15 : 7)) == 0;
-  for (int i = 0; i < n; ++i)
-    v = v && a[i].ld % 4 == 0 && a[i].plane % 4 == 0 && ((uintptr_t)a[i].p & (a[i].split == 0 && !f32 ? 7 : 15)) == 0;
-  return v;
-}
-
 }  // namespace
 
 // z, u, g: columns of products (pointer, split (0: activations, else fp32 slabs), row stride, slab stride); out rows of stride
@@ -179,8 +133,8 @@ CFC_API int cfc_gru_step(int f32, const void* z, int z_split, int64_t z_ld, int6
   if (B <= 0) return 0;
   if (W < 1 || !slots || !ctx_lens || !state || ldo < W) return -1;
   const GruCols a[3] = {{z, z_split, z_ld, z_plane}, {u, u_split, u_ld, u_plane}, {g, g_split, g_ld, g_plane}};
-#define GS(ACT, V) \
-  gru_step_kernel<ACT, V><<<dim3(B, (W + 64 * V - 1) / (64 * V)), 64, 0, stream>>>(a[0], a[1], a[2], bz, bx, slots, ctx_lens, W, state, (ACT*)out, ldo, oscale)
+  const GruStep s{a[0], a[1], a[2], bz, bx, slots, ctx_lens, W, state, out, ldo, oscale};
+#define GS(ACT, V) gru_step_kernel<ACT, V><<<dim3(B, (W + 64 * V - 1) / (64 * V)), 64, 0, stream>>>(s)
   const bool v4 = gru_vec(a, 3, W, f32, out, ldo);
   if (f32) { if (v4) GS(float, 4); else GS(float, 1); }
   else if (v4) GS(uint16_t, 4);

@@ -12,7 +12,7 @@
 // Convolution state: [slots][taps - 1][channels] fp32, position p at row p % (taps - 1).  Pooled block b lies at entry
 // b % E of page b / E (E a power of two, at least 32 / pool: the page of a block's mean exists when its tokens do).
 // D: columns of a cached head, dim (or vdim) rounded up; the pad stays zero.
-#include "rows.h"
+#include "gru_step.h"
 
 namespace {
 
@@ -44,9 +44,16 @@ __device__ __forceinline__ float round_act(float v, const float*) { return v; }
 constexpr int ROT_MAX = 1024;
 constexpr int MAX_BACK = 3;          // convolution rows before the own that a thread holds in registers
 
-// grid (rows, parts).  Dynamic LDS: per-vector sums, and for V = 1 the row
-template <typename ACT, int V, int NV, int BT>
-__global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a) {
+// grid (rows, parts).  Dynamic LDS: per-vector sums, and for V = 1 the row.
+// GRU: workgroups past the parts step the recurrence beside the attention, whose inputs the same product leaves: a launch less in each of
+// a decode step's layers that have both (us of two steps: pemolorn 32 x 1024 1477 -> 1467, tadolix 5 x 700 900 -> 890)
+template <typename ACT, int V, int NV, int BT, bool GRU = false>
+__global__ void __launch_bounds__(BT) qkv_rows_kernel(QkvArgs a, GruStep step) {
+  if constexpr (GRU)
+    if ((int)blockIdx.y >= a.parts) {
+      if (blockIdx.z == 0) gru_step_row<ACT, V>(step, blockIdx.x, ((blockIdx.y - a.parts) * BT + threadIdx.x) * V);
+      return;
+    }
   __shared__ float red[16];
   __shared__ float2 cs[ROT_MAX / 2];
   extern __shared__ float dyn[];
@@ -464,8 +471,11 @@ int qkv_prompt_go(hipStream_t s, int T, int threads, const QkvArgs& a) {
   return CFC_CHECK_LAUNCH();
 }
 
+constexpr int QKV_APART = -1000;       // the step needs a launch of its own; nothing was launched
+
+// step: of as many rows, in the same launch
 template <typename ACT, int V>
-int qkv_go(hipStream_t s, int T, const QkvArgs& a) {
+int qkv_go(hipStream_t s, int T, const QkvArgs& a, const GruStep* step = nullptr) {
   // few rows with norms per head: runs of heads beside each other, so their loads do not follow one another
   const int most = max(a.H, a.parts > 1 ? a.G : 0);
   const int z = a.per_head && T * a.parts < 512 ? max(1, min(min(most, 8), 512 / (T * a.parts))) : 1;
@@ -474,13 +484,22 @@ int qkv_go(hipStream_t s, int T, const QkvArgs& a) {
   const int vecs = (C + V - 1) / V;
   const size_t lds = (size_t)(vecs + max(a.H, a.G)) * 4;
   if (lds > 49152) return -4;
-#define GO(NV, BT) qkv_rows_kernel<ACT, V, NV, BT><<<dim3(T, a.parts, z), BT, lds, s>>>(a)
-  if (vecs <= 64) GO(1, 64);
-  else if (vecs <= 256) GO(1, 256);
-  else if (vecs <= 512) GO(1, 512);
-  else if (vecs <= 1024) GO(1, 1024);
-  else if (vecs <= 4096) GO(4, 1024);
-  else if (vecs <= 16384) GO(16, 1024);
+#define GO(NV, BT)                                                                                                                        \
+  {                                                                                                                                       \
+    if constexpr (NV == 1 && V == 4) {                                                                                                    \
+      if (step) qkv_rows_kernel<ACT, V, NV, BT, true><<<dim3(T, a.parts + (step->W + V * BT - 1) / (V * BT), z), BT, lds, s>>>(a, *step); \
+      else qkv_rows_kernel<ACT, V, NV, BT><<<dim3(T, a.parts, z), BT, lds, s>>>(a, GruStep{});                                            \
+    } else {                                                                                                                              \
+      if (step) return QKV_APART;                                                                                                         \
+      qkv_rows_kernel<ACT, V, NV, BT><<<dim3(T, a.parts, z), BT, lds, s>>>(a, GruStep{});                                                 \
+    }                                                                                                                                     \
+  }
+  if (vecs <= 64) GO(1, 64)
+  else if (vecs <= 256) GO(1, 256)
+  else if (vecs <= 512) GO(1, 512)
+  else if (vecs <= 1024) GO(1, 1024)
+  else if (vecs <= 4096) GO(4, 1024)
+  else if (vecs <= 16384) GO(16, 1024)
   else return -4;
 #undef GO
   return CFC_CHECK_LAUNCH();
@@ -532,11 +551,11 @@ __global__ void __launch_bounds__(256) pool_rows_kernel(const int32_t* __restric
 }  // namespace
 
 // lead null: decoded rows (conv state and pooled blocks are written here).  parts 1: queries only (kc .. pv unused)
-CFC_API int cfc_qkv_rows(int f32, const void* p, int split, int64_t ld, int64_t plane, int T, int H, int G, int dim, int vdim, int D,
+static int qkv_rows_go(int f32, const void* p, int split, int64_t ld, int64_t plane, int T, int H, int G, int dim, int vdim, int D,
                          int parts, const float* qn, const float* kn, int per_head, float eps, const float* freq, int rot,
                          float qscale, const float* conv, int taps, float* tail, const int32_t* lead, const int32_t* slots,
                          const int32_t* positions, const int32_t* cslots, void* q, void* kc, void* vc, void* pk, void* pv, int pool,
-                         int le, const int32_t* bt, int max_blocks, hipStream_t stream) {
+                         int le, const int32_t* bt, int max_blocks, hipStream_t stream, const GruStep* step) {
   if (T <= 0) return 0;
   if (H < 1 || G < 1 || dim < 1 || vdim < 1 || D < dim || D < vdim || rot < 0 || rot % 2 || rot > dim || rot > ROT_MAX ||
       (parts != 1 && parts != 3))
@@ -549,8 +568,45 @@ CFC_API int cfc_qkv_rows(int f32, const void* p, int split, int64_t ld, int64_t 
                   ((uintptr_t)p & (split == 0 && !f32 ? 7 : 15)) == 0;
   if (const int th = f32 ? prompt_threads<float, 4>(a) : prompt_threads<uint16_t, 8>(a))
     return f32 ? qkv_prompt_go<float, 4>(stream, T, th, a) : qkv_prompt_go<uint16_t, 8>(stream, T, th, a);
-  if (f32) return v4 ? qkv_go<float, 4>(stream, T, a) : qkv_go<float, 1>(stream, T, a);
-  return v4 ? qkv_go<uint16_t, 4>(stream, T, a) : qkv_go<uint16_t, 1>(stream, T, a);
+  if (step && !v4) return QKV_APART;
+  if (f32) return v4 ? qkv_go<float, 4>(stream, T, a, step) : qkv_go<float, 1>(stream, T, a);
+  return v4 ? qkv_go<uint16_t, 4>(stream, T, a, step) : qkv_go<uint16_t, 1>(stream, T, a);
+}
+
+CFC_API int cfc_qkv_rows(int f32, const void* p, int split, int64_t ld, int64_t plane, int T, int H, int G, int dim, int vdim, int D,
+                         int parts, const float* qn, const float* kn, int per_head, float eps, const float* freq, int rot,
+                         float qscale, const float* conv, int taps, float* tail, const int32_t* lead, const int32_t* slots,
+                         const int32_t* positions, const int32_t* cslots, void* q, void* kc, void* vc, void* pk, void* pv, int pool,
+                         int le, const int32_t* bt, int max_blocks, hipStream_t stream) {
+  return qkv_rows_go(f32, p, split, ld, plane, T, H, G, dim, vdim, D, parts, qn, kn, per_head, eps, freq, rot, qscale, conv, taps, tail, lead, slots, positions, cslots, q, kc, vc, pk, pv, pool, le, bt, max_blocks, stream, nullptr);
+}
+
+CFC_API int cfc_gru_step(int f32, const void* z, int z_split, int64_t z_ld, int64_t z_plane, const void* u, int u_split,
+                         int64_t u_ld, int64_t u_plane, const void* g, int g_split, int64_t g_ld, int64_t g_plane, const float* bz,
+                         const float* bx, const int32_t* slots, const int32_t* ctx_lens, int B, int W, float* state, void* out,
+                         int64_t ldo, float oscale, hipStream_t stream);
+
+// cfc_qkv_rows of decoded rows and cfc_gru_step of as many, in one launch where both go by vectors of four
+CFC_API int cfc_qkv_rows_gru(int f32, const void* p, int split, int64_t ld, int64_t plane, int T, int H, int G, int dim, int vdim, int D,
+                         int parts, const float* qn, const float* kn, int per_head, float eps, const float* freq, int rot,
+                         float qscale, const float* conv, int taps, float* tail, const int32_t* lead, const int32_t* slots,
+                         const int32_t* positions, const int32_t* cslots, void* q, void* kc, void* vc, void* pk, void* pv, int pool,
+                         int le, const int32_t* bt, int max_blocks,
+                              const void* gz, int gz_split, int64_t gz_ld, int64_t gz_plane, const void* gu, int gu_split, int64_t gu_ld,
+                              int64_t gu_plane, const void* gg, int gg_split, int64_t gg_ld, int64_t gg_plane, const float* bz, const float* bx,
+                              const int32_t* ctx_lens, int W, float* state, void* out, int64_t ldo, float oscale, hipStream_t stream) {
+  if (T <= 0) return 0;
+  if (lead || W < 1 || !slots || !ctx_lens || !state || ldo < W) return -1;
+  const GruCols g[3] = {{gz, gz_split, gz_ld, gz_plane}, {gu, gu_split, gu_ld, gu_plane}, {gg, gg_split, gg_ld, gg_plane}};
+  const GruStep step{g[0], g[1], g[2], bz, bx, slots, ctx_lens, W, state, out, ldo, oscale};
+  if (gru_vec(g, 3, W, f32, out, ldo)) {
+    const int rc = qkv_rows_go(f32, p, split, ld, plane, T, H, G, dim, vdim, D, parts, qn, kn, per_head, eps, freq, rot, qscale, conv, taps, tail, lead, slots, positions, cslots, q, kc, vc, pk, pv, pool, le, bt, max_blocks, stream, &step);
+    if (rc != QKV_APART) return rc;
+  }
+  if (const int rc = cfc_gru_step(f32, gz, gz_split, gz_ld, gz_plane, gu, gu_split, gu_ld, gu_plane, gg, gg_split, gg_ld, gg_plane, bz, bx, slots,
+                                  ctx_lens, T, W, state, out, ldo, oscale, stream))
+    return rc;
+  return qkv_rows_go(f32, p, split, ld, plane, T, H, G, dim, vdim, D, parts, qn, kn, per_head, eps, freq, rot, qscale, conv, taps, tail, lead, slots, positions, cslots, q, kc, vc, pk, pv, pool, le, bt, max_blocks, stream, nullptr);
 }
 
 CFC_API int cfc_conv_tail(int f32, const void* p, int split, int64_t ld, int64_t plane, int C, const int32_t* cu_q,

@@ -245,6 +245,37 @@ def test_rows_of_a_mean_together(device, dtype, case):
 
 
 @pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("case,W,split", [((8, 2, 64, 64, True, 0, 16), 260, 3), ((32, 8, 128, 128, False, 4, 64), 4096, 4), ((2, 1, 64, 64, False, 4, 8), 1100, 0),
+                                          ((3, 1, 18, 14, False, 3, 6), 64, 2), ((8, 2, 64, 64, True, 0, 16), 65, 1), ((33, 33, 128, 128, True, 0, 0), 96, 2)])
+def test_recurrence_beside_the_rows_of_attention(device, dtype, case, W, split):
+    """A decoded step of both in one launch, and where shapes ask for two: the bits of one after the other."""
+    H, G, dim, vdim, per_head, taps, rot = case
+    a, n = heads_of(H, G, dim, vdim, per_head, taps, rot, A.Mask(20, pool=4), device=device), 5
+    C, at = a.columns, -(-a.columns // 4) * 4
+    x = rnd(n, at + 3 * W, seed=3).to(dtype)
+    t = slabs(x.float(), split).to(device) if split else x.to(device)
+    p = R.Gru((rnd(W, seed=4) - 1.0).to(device), rnd(W, seed=5).to(device))
+    pos, slots = i32([3, 0, 8, 31, 7], device), i32([37, 64, 104, 159, 7], device)
+    states, bt = i32([2, 0, 3, 1, 4], device), i32([[1], [2], [3], [4], [0]], device)
+    got = []
+    for apart in (True, False):
+        rows = PagedHeads(6, G, a.D, 4, A.pool_entries(4), device, dtype)
+        tail = rnd(6, taps - 1, C, seed=12).to(device) if taps > 1 else None
+        state, out = rnd(6, W, seed=6).to(device), torch.zeros(n, W + 4, dtype=dtype, device=device)
+        step = R.Step(p, *(Cols(t, at + k * W, W) for k in range(3)), states, pos + 1, state, out[:, :W], 0.5)
+        if apart:
+            step.run()
+        q = A.qkv_rows(a, Cols(t, 0, C), rows, pos, slots, states, bt, tail, beside=None if apart else step)
+        got.append([q, rows.k, rows.v, rows.pk, rows.pv, state, out] + ([tail] if taps > 1 else []))
+    assert all(torch.equal(x, y) for x, y in zip(*got)) and not got[0][6][:, W:].any() and got[0][6][:, :W].any()
+    with pytest.raises(ValueError):
+        A.qkv_rows(a, Cols(t, 0, C), rows, pos, slots, states, bt, tail, lead=pos, beside=step)
+    with pytest.raises(ValueError):
+        A.qkv_rows(a, Cols(t, 0, C), rows, pos, slots, states.clone(), bt, tail, beside=step)
+
+
+@pytest.mark.parametrize("device", DEVICES)
 def test_queries_alone_leave_the_cache(device):
     a = heads_of(4, 2, 32, 32, True, 0, 0, A.Mask(9, keep=2), device=device, shared=True)
     rows = PagedHeads(2, 2, a.D, 0, 0, device, torch.float32)
