@@ -920,7 +920,8 @@ class DecoderModel:
         cfg, w = self.cfg, self.w
         sb = getattr(self, "_shared_blocks", None)
         B = qkv.shape[-2]
-        fused = self.rope_fused == "1" or (self.rope_fused == "" and B <= K.GEMV_MAX_M)
+        fused = self.rope_fused == "1" or (self.rope_fused == "" and K.rope_inside(
+            B, w.kv_heads, block_tables.shape[1], part_blocks, kv.k[i].dtype == torch.bfloat16))
         if fused and qkv.is_cuda:
             return K.paged_decode_rope_attention(qkv, positions, slots, w.cos_sin, kv.k[i], kv.v[i], block_tables,
                                                  ctx_lens, self.scale, w.heads, w.kv_heads, cfg.head_dim,

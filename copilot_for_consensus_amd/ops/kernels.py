@@ -301,6 +301,15 @@ def paged_decode_attention(q, k_cache, v_cache, block_tables, ctx_lens, scale, o
     return out
 
 
+def rope_inside(B: int, Hkv: int, max_blocks: int, part_blocks: int, bf16: bool) -> bool:
+    """Whether a decode step's rotation and cache write are best inside its attention (:func:`paged_decode_rope_attention`): of few sequences, and
+    of more where the bf16 kernels that stream keys and values take them, but for contexts of more than 2048 keys
+    in two workgroups a CU (both measured in attention.hip)."""
+    if B <= GEMV_MAX_M:
+        return True
+    return bf16 and B <= 128 and part_blocks < 0 and (B * Hkv * -part_blocks <= 256 or max_blocks <= 64)
+
+
 def paged_decode_rope_attention(qkv, positions, slots, cos_sin, k_cache, v_cache, block_tables, ctx_lens, scale,
                                 Hq, Hkv, D, part_blocks=-1, workspace=None, window=0, k_scale=1.0, v_scale=1.0,
                                 out=None, shared_blocks=None):

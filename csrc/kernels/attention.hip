@@ -34,6 +34,7 @@ namespace {
 constexpr int KV_BS = 32;          // tokens per KV-cache block
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr int DEC_ORDER_ROWS = 128;   // sequences that longest_first orders at most
+constexpr int DEC_FUSED_ROWS = 4;     // sequences whose step with its rotation inside takes loads to registers, whatever their lengths
 constexpr int DEC_ORDER_FROM = 1024;  // the longest context from which it does
 
 __device__ __forceinline__ bf16x8_t as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8_t, v); }
@@ -464,17 +465,23 @@ __global__ void __launch_bounds__(256, F8 ? 2 : 1) paged_decode_kernel(
 // Chunk c of K's row r lies at c ^ (r & 15) (through the pieces' source addresses), so that sixteen rows' reads touch all
 // banks; V's slot groups lie as in the cache.
 // A workgroup of NWV waves has one (partition of a) sequence and kv head, wave w its blocks w, w + NWV, ...
-// bf16 cache, queries roped.
+// bf16 cache, queries roped.  ROPE: they are not, and neither are the new keys in the cache, as in paged_decode_kernel (DecRope): what it
+// takes of the projection comes ahead of the first waves' tiles, the new key and value replace in LDS what came for them.  us of two decode
+// steps of four layers, 32 query and 8 key heads, contexts from 0.8 of the longest, a launch of its own -> this: 5 of 700 851 -> 845, 8 of
+// 1500 898 -> 880, 16 of 1000 937 -> 922, 24 of 1500 1018 -> 1001, 32 of 1024 1018 -> 995, of 2600 1256 -> 1230, 64 of 300 1078 -> 1051, 72 of
+// 700 1261 -> 1252, 100 of 1200 1686 -> 1671, 128 of 40 1205 -> 1191.  The start is a chain of loads, 4 us, that a CU with two long workgroups does not
+// win back: 39 of 4152 1716 -> 1736, 128 of 2617 2648 -> 2653 (Python's ops.kernels.rope_inside knows).
 // ------------------------------------------------------------------------------------------
-template <int G, int NWV, int T>
+template <int G, int NWV, int T, bool ROPE = false>
 __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ ctx_lens, float scale_log2, int Hkv, int max_blocks,
     int P, int window, float v_scale, float* __restrict__ part_o, float* __restrict__ part_ml, uint16_t* __restrict__ out,
-    const int32_t* __restrict__ shared_blocks, int cached, int ordered) {
-  constexpr int D = 128, TILE = KV_BS * D * 2, QB = (G + 3) / 4 * 1024, RING = T * TILE;
+    const int32_t* __restrict__ shared_blocks, int cached, int ordered, DecRope rp) {
+  constexpr int D = 128, TILE = KV_BS * D * 2, QB = ROPE ? 0 : (G + 3) / 4 * 1024, RING = T * TILE;
   constexpr bool ORD = NWV == 4 && T == 2;
-  __shared__ __attribute__((aligned(16))) char smem[NWV * (RING + QB)];
+  __shared__ __attribute__((aligned(16))) char smem[NWV * (RING + QB) + (ROPE ? (G + 2) * D * 2 : 0)];
+  uint16_t(*sm_q)[D] = reinterpret_cast<uint16_t(*)[D]>(smem + NWV * (RING + QB)), (*sm_kv)[D] = sm_q + G;      // ROPE: queries, the new key and value
   static_assert(sizeof(smem) <= (T == 2 && NWV == 4 ? 80 : 160) * 1024 && sizeof(smem) >= ORDER_LDS, "four waves: two workgroups a CU");
   const int p = blockIdx.x, h = blockIdx.y;
   int b = blockIdx.z, ctx;
@@ -524,12 +531,41 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
   for (int i = 0; i < 8; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
   bf16x8_t qf[4];
+  const int slot = ROPE ? rp.slots[b] : -1;
+  const bool owner = ROPE && slot >= 0 && blk0 <= nblk - 1 && nblk - 1 < blk1;   // holds the new key's block
+  const int last = owner ? bt[nblk - 1] : 0;
+  if constexpr (ROPE) {
+    // by the first waves ahead of their tiles: behind these it would wait for all that the chip asks for at first
+    constexpr int NV = D / 16;    // 8-vectors per half-head
+    const size_t stride = (size_t)(Hq + 2 * Hkv) * D;
+    const size_t row0 = (size_t)b * stride, slab = (size_t)gridDim.z * stride;
+    const float* cs = rp.cos_sin + (size_t)rp.positions[b] * (D / 2) * 2;
+    for (int t = threadIdx.x; t < (G + 1) * NV + D / 8; t += 64 * NWV) {
+      const int hh = t / NV, c = t - hh * NV;      // hh < G: query head h G + hh; hh == G: key head h
+      if (hh < G || (hh == G && owner)) {
+        uint4 pa, pb;
+        rope_rot8(rp.qkv, rp.part, rp.split, slab, row0 + (size_t)(hh < G ? h * G + hh : Hq + h) * D, D / 2, c, cs, pa, pb);
+        uint16_t* to = hh < G ? sm_q[hh] : sm_kv[0];
+        *reinterpret_cast<uint4*>(to + c * 8) = pa;
+        *reinterpret_cast<uint4*>(to + D / 2 + c * 8) = pb;
+        if (hh == G) kv_write_k<false>(const_cast<uint16_t*>(kc), slot, h, Hkv, D, c, pa, pb, 1.f);
+      } else if (hh > G && owner) {
+        const int cv = t - (G + 1) * NV;
+        float vv[8];
+        qkv_load8(rp.qkv, rp.part, rp.split, slab, row0 + (size_t)(Hq + Hkv + h) * D + cv * 8, vv);
+        *reinterpret_cast<uint4*>(&sm_kv[1][cv * 8]) = pack8(vv);
+      }
+    }
+  }
+  int ahead = 0;                                   // the block of the tiles T on
   if (n > 0) {
-    // the queries' rows first: they are there when the first keys are (past the G heads: the last one's, not used)
-    const char* qs = reinterpret_cast<const char*>(q + ((size_t)b * Hq + h * G) * D);
+    if constexpr (!ROPE) {
+      // the queries' rows first: they are there when the first keys are (past the G heads: the last one's, not used)
+      const char* qs = reinterpret_cast<const char*>(q + ((size_t)b * Hq + h * G) * D);
 #pragma unroll
-    for (int e = 0; e < QB / 1024; ++e)
-      ring_piece<false>((uint32_t)min(4 * e + (lane >> 4), G - 1) * 256u + (lane & 15) * 16u, qs, lds0 + RING + e * 1024);
+      for (int e = 0; e < QB / 1024; ++e)
+        ring_piece<false>((uint32_t)min(4 * e + (lane >> 4), G - 1) * 256u + (lane & 15) * 16u, qs, lds0 + RING + e * 1024);
+    }
 #pragma unroll
     for (int j = 0; j < T; j += 2)
       if (j < 2 * n) {
@@ -537,18 +573,28 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
         issue(j, block);
         issue(j + 1, block);
       }
-    int ahead = id(T / 2);                         // the block of the tiles T on
+    ahead = id(T / 2);
+  }
+  if constexpr (ROPE) lds_barrier();
+  {
     for (int i = 0; i < n; ++i) {
       const int bi = first + i * NWV, next = id(i + 1 + T / 2);
       ring_landed<T, 8>(2 * i, 2 * n);
       if (i == 0) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
-          qf[c] = col < G ? as_bf16x8(*reinterpret_cast<const uint4*>(mine + RING + min(col, G - 1) * 256 + c * 64 + g * 16))
+          qf[c] = col < G ? as_bf16x8(*reinterpret_cast<const uint4*>(ROPE ? reinterpret_cast<const char*>(sm_q[min(col, G - 1)]) + c * 64 + g * 16
+                                                                          : mine + RING + min(col, G - 1) * 256 + c * 64 + g * 16))
                           : as_bf16x8(make_uint4(0, 0, 0, 0));
       }
       uint4 kf[2][4];
-      const char* ki = mine + (2 * i & (T - 1)) * TILE;
+      char* ki = mine + (2 * i & (T - 1)) * TILE;
+      const bool fresh = ROPE && owner && bi == nblk - 1;         // the new key's row replaces what came for it
+      if (fresh) {
+        if (lane < 16)
+          *reinterpret_cast<uint4*>(ki + (slot % KV_BS) * 256 + ((lane ^ (slot & 15)) << 4)) = *reinterpret_cast<const uint4*>(&sm_kv[0][8 * lane]);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // by other lanes than read it
+      }
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
@@ -593,6 +639,18 @@ __global__ void __launch_bounds__(64 * NWV, T == 2 ? 2 : 1) paged_stream_kernel(
       m = mn;
       const bf16x8_t pf = pack_p(s[0], s[1]);
       ring_landed<T, 8>(2 * i + 1, 2 * n);
+      if (fresh) {
+        // and its values', whose slot group goes back to the cache, 16 whole lines
+        const int ps = kv_v_slot(slot % KV_BS);
+        char* vg = mine + ((2 * i + 1) & (T - 1)) * TILE + (ps >> 3) * 2048;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) *reinterpret_cast<uint16_t*>(vg + (2 * lane + e) * 16 + (ps & 7) * 2) = sm_kv[1][2 * lane + e];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // in another type, and by other lanes, than read
+        char* to = reinterpret_cast<char*>(const_cast<uint16_t*>(vc)) + ((size_t)last * Hkv + h) * TILE + (ps >> 3) * 2048;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          *reinterpret_cast<uint4*>(to + e * 1024 + lane * 16) = *reinterpret_cast<const uint4*>(vg + e * 1024 + lane * 16);
+      }
       uint4 vf[8];
       const char* vi = mine + ((2 * i + 1) & (T - 1)) * TILE + g * 2048 + col * 16;
 #pragma unroll
@@ -1739,19 +1797,25 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
   if constexpr (!F8) {
     const int seen = window > 0 ? min(max_blocks, (window + 30) / KV_BS + 1) : max_blocks;
     const bool aligned = (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;       // LDS-DMA's sources
-    const int nw = rope || part_blocks > 0 || B > DEC_ORDER_ROWS || !aligned ? -4 : paged_waves(wgs, seen, P, max_blocks);
+    const bool few = rope && (B <= DEC_FUSED_ROWS || rope->probe);
+    const int nw = few || part_blocks > 0 || B > DEC_ORDER_ROWS || !aligned ? -4 : paged_waves(wgs, seen, P, max_blocks);
     if (nw > 0) {
-#define PDS_GO(NWV, T)                                                                                                      \
-  paged_stream_kernel<GG, NWV, T><<<grid, 64 * NWV, 0, stream>>>((const uint16_t*)q, (const uint16_t*)k_cache,               \
+#define PDS_R(NWV, T, R)                                                                                                    \
+  paged_stream_kernel<GG, NWV, T, R><<<grid, 64 * NWV, 0, stream>>>((const uint16_t*)q, (const uint16_t*)k_cache,            \
       (const uint16_t*)v_cache, block_tables, ctx_lens, sl2, Hkv, max_blocks, P, window, v_scale, part_o, part_ml,           \
-      (uint16_t*)out, shared_blocks, nt_env == 0 ? INT_MAX : 0, ordered)
+      (uint16_t*)out, shared_blocks, nt_env == 0 ? INT_MAX : 0, ordered, rp)
+#define PDS_GO(NWV, T)                     \
+  {                                        \
+    if (rope) PDS_R(NWV, T, true);         \
+    else PDS_R(NWV, T, false);             \
+  }
 #define PDS_CASE(G_)                        \
   case G_: {                                \
     constexpr int GG = G_;                  \
-    if (nw == 8) PDS_GO(8, 2);              \
-    else if (nw == 1) PDS_GO(1, 4);         \
-    else if (wgs <= 64) PDS_GO(4, 4);       \
-    else PDS_GO(4, 2);                      \
+    if (nw == 8) PDS_GO(8, 2)               \
+    else if (nw == 1) PDS_GO(1, 4)          \
+    else if (wgs <= 64) PDS_GO(4, 4)        \
+    else PDS_GO(4, 2)                       \
   } break;
       switch (G) {
         PDS_CASE(1) PDS_CASE(2) PDS_CASE(4) PDS_CASE(8) PDS_CASE(16)
@@ -1759,6 +1823,7 @@ static int launch_paged_decode(const void* q, const void* k_cache, const void* v
       }
 #undef PDS_CASE
 #undef PDS_GO
+#undef PDS_R
       if (P > 1) decode_combine_kernel<<<(Hq * B + 3) / 4, 256, 0, stream>>>(part_o, part_ml, P, Hq * B, (uint16_t*)out);
       return CFC_CHECK_LAUNCH();
     }

@@ -49,3 +49,13 @@ def test_engines_partitions_are_no_slower_for_short_contexts(heads, kv_heads, dt
                 assert full == (kv_partitions(B, heads, kv_heads, blocks) if (heads, kv_heads) == (32, 8) else P)
     monkeypatch.setenv("CFC_DECODE_WGS", "2048")
     assert -LLMEngine._part_blocks(engine, 128, 88) == m.decode_partitions(128, 88) == math.ceil(2048 / (128 * kv_heads))
+
+
+def test_where_a_decode_step_turns_its_queries():
+    """Inside its attention: few sequences always, more where the streaming kernels take them and win back the longer start."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    inside = K.rope_inside
+    assert all(inside(b, 8, n, p, t) for b in (1, 4) for n in (2, 500) for p in (-3, 16) for t in (True, False))
+    assert inside(5, 8, 500, -6, True) and inside(32, 8, 90, -1, True) and inside(128, 8, 64, -1, True)
+    assert not inside(33, 8, 65, -1, True) and not inside(128, 8, 88, -2, True)      # long contexts, two workgroups a CU
+    assert not inside(5, 8, 40, -6, False) and not inside(5, 8, 40, 16, True) and not inside(129, 8, 4, -1, True)

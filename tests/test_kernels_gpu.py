@@ -775,6 +775,38 @@ def test_paged_decode_rope_attention_fused_matches_two_kernels(G, part_blocks, s
     _close(o2, ref, 3e-2 if kv == "fp8" else 2e-2)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,P,longest,window", [
+    (5, 32, 8, 1, 700, 0), (5, 32, 8, 4, 1500, 0), (8, 32, 8, 1, 1200, 0), (9, 8, 8, 3, 2100, 90), (24, 32, 8, 1, 600, 0), (12, 64, 4, 2, 1100, 0),
+    (40, 32, 8, 2, 900, 0), (72, 32, 8, 1, 2500, 0), (100, 16, 8, 1, 64, 0), (128, 32, 8, 1, 1300, 200), (128, 16, 1, 1, 40, 0), (70, 128, 8, 1, 400, 0),
+    (129, 32, 8, 1, 300, 0)])
+@pytest.mark.parametrize("src", ["bf16", "slabs4"])
+def test_paged_decode_rope_attention_by_the_ring(B, Hq, Hkv, P, longest, window, src):
+    """The rotation inside the kernels that stream keys and values: each one's waves and tiles, contexts in order and not, new keys in
+    every place of a block and in blocks of their own, an idle row.  The bits of two launches, output and cache."""
+    D, N = 128, (Hq + 2 * Hkv) * 128
+    g = torch.Generator().manual_seed(B + P)
+    ctx = [1 + int(x) for x in torch.randint(0, longest, (B,), generator=g)]
+    ctx[0], ctx[1], ctx[2], ctx[3] = longest, 1, min(33, longest), min(32, longest)
+    kc, vc, bt = _fill_cache(ctx, Hkv, D)
+    pos = torch.tensor([n - 1 for n in ctx], dtype=torch.int32)
+    slots = torch.tensor([int(bt[b, (n - 1) // 32]) * 32 + (n - 1) % 32 for b, n in enumerate(ctx)], dtype=torch.int32)
+    slots[4] = -1
+    args = (pos.to(DEV), slots.to(DEV), R.rope_cos_sin(4096, D, 1e6, device=DEV))
+    qkv = torch.randn(B, N, device=DEV).bfloat16() if src == "bf16" else torch.randn(4, B, N, device=DEV)
+    bt_d, cl = bt.to(DEV), torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    k1, v1, k2, v2 = kc.to(DEV), vc.to(DEV), kc.to(DEV), vc.to(DEV)
+    q = (K.rope_kv_write if src == "bf16" else K.rope_kv_write_part)(qkv, *args, k1, v1, Hq, Hkv, D)
+    o1 = K.paged_decode_attention(q, k1, v1, bt_d, cl, D ** -0.5, part_blocks=-P, window=window)
+    for _ in range(2):                     # a step that is run again replaces what it wrote
+        o2 = K.paged_decode_rope_attention(qkv, *args, k2, v2, bt_d, cl, D ** -0.5, Hq, Hkv, D, part_blocks=-P, window=window)
+        assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(o1, o2)
+    qb = (qkv.float().sum(0).bfloat16() if src != "bf16" else qkv).cpu()
+    kr, vr, some = kc.clone(), vc.clone(), [0, 1, 2, 3, B - 1]
+    qr = R.rope_kv_write(qb, pos, slots, args[2].cpu(), kr, vr, Hq, Hkv, D)
+    want = R.paged_decode_attention(qr[some], kr, vr, bt[some], cl.cpu()[some], D ** -0.5, window=window)
+    _close(o2[some], want, 2e-2)
+
+
 def test_paged_decode_rope_attention_rejects_bad_shapes():
     Hq, Hkv, D = 8, 2, 128
     kc, vc, bt = _fill_cache([40, 70], Hkv, D)
