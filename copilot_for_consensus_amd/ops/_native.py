@@ -39,9 +39,10 @@ _KERNEL_SIGS = {
     "cfc_rope_kv_write": [P, P, P, P, P, P, P, I, I, I, I, I, P],
     "cfc_set_kv_vstore_mode": [I],
     "cfc_set_decode_rope_probe": [I],
-    "cfc_rope_kv_write_runs": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, F, P],
+    "cfc_v_cache_write_runs": [P, P, I, P, I, I, I, P],
     "cfc_decode_advance_cb": [P, P, I, P, P, P, P, P, P, P, I, P, P, I, I] + [P] * 6 + [I] * 4 + [P] * 4,
     "cfc_rope_kv_write_fp8": [P, P, P, P, P, P, P, I, I, I, I, I, F, F, P],
+    "cfc_v_cache_write_runs_fp8": [P, P, I, P, I, I, I, F, P],
     "cfc_paged_decode_attention_fp8": [P, P, P, P, P, I, I, I, I, I, I, I, F, I, F, F, P, P, P, P, P],
     "cfc_paged_decode_rope_attention": [P, P, I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, F, F, P, P, P, P,
                                         P],

@@ -206,23 +206,18 @@ def rope_kv_write(qkv, positions, slots, cos_sin, k_cache, v_cache, Hq, Hkv, D, 
     if runs is not None:
         _req(runs, torch.int32, "runs")
     q_out = torch.empty(T, Hq, D, dtype=qkv.dtype, device=qkv.device) if q_out is None else q_out
+    write_v = 0 if runs is not None else 1
     _apply_vstore()
-    if runs is not None:
-        f8 = _fp8(k_cache)
-        check(kernels().cfc_rope_kv_write_runs(qkv.data_ptr(), positions.data_ptr(), slots.data_ptr(), cos_sin.data_ptr(), q_out.data_ptr(),
-                                               k_cache.data_ptr(), v_cache.data_ptr(), runs.data_ptr(), runs.shape[0], T, Hq, Hkv, D, int(f8),
-                                               1.0 / k_scale if f8 else 1.0, 1.0 / v_scale if f8 else 1.0, _stream(qkv)),
-              "cfc_rope_kv_write_runs")
-    elif _fp8(k_cache):
+    if _fp8(k_cache):
         check(kernels().cfc_rope_kv_write_fp8(qkv.data_ptr(), positions.data_ptr(), slots.data_ptr(),
                                               cos_sin.data_ptr(), q_out.data_ptr(), k_cache.data_ptr(),
-                                              v_cache.data_ptr(), T, Hq, Hkv, D, 1, 1.0 / k_scale,
+                                              v_cache.data_ptr(), T, Hq, Hkv, D, write_v, 1.0 / k_scale,
                                               1.0 / v_scale, _stream(qkv)), "cfc_rope_kv_write_fp8")
-    else:
-        check(kernels().cfc_rope_kv_write(qkv.data_ptr(), positions.data_ptr(), slots.data_ptr(), cos_sin.data_ptr(),
-                                          q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), T, Hq, Hkv, D,
-                                          1, _stream(qkv)), "cfc_rope_kv_write")
-    return q_out
+        if runs is not None:
+            check(kernels().cfc_v_cache_write_runs_fp8(qkv.data_ptr(), runs.data_ptr(), runs.shape[0],
+                                                       v_cache.data_ptr(), Hq, Hkv, D, 1.0 / v_scale, _stream(qkv)),
+                  "cfc_v_cache_write_runs_fp8")
+        return q_out
     check(kernels().cfc_rope_kv_write(qkv.data_ptr(), positions.data_ptr(), slots.data_ptr(), cos_sin.data_ptr(),
                                       q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), T, Hq, Hkv, D,
                                       write_v, _stream(qkv)), "cfc_rope_kv_write")

@@ -317,9 +317,8 @@ __device__ __forceinline__ void rope_rot8(const uint16_t* qkv, const float* part
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const float cv = csv[2 * j], sv = csv[2 * j + 1];
-    // which product is rounded is not left to the kernel that this is inlined in: all of them write the same bits
-    ra[j] = __builtin_fmaf(a[j], cv, -(b[j] * sv));
-    rb[j] = __builtin_fmaf(b[j], cv, a[j] * sv);
+    ra[j] = a[j] * cv - b[j] * sv;
+    rb[j] = b[j] * cv + a[j] * sv;
   }
   pa = pack8(ra);
   pb = pack8(rb);

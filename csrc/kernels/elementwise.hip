@@ -18,19 +18,25 @@ __device__ __forceinline__ int v_slot(int key_in_block) { return kv_v_slot(key_i
 // qkv: [T, (Hq + 2*Hkv) * D] (q heads | k heads | v heads), positions [T], slots [T] (-1 = skip
 // cache write), cos_sin [max_pos][D/2][2] fp32 (cos, sin interleaved); the per-item math lives in
 // common.h (rope_rot8 / kv_write_k / kv_write_v), shared with the fused decode attention.
-// 8-element item `it` of token `tok`: (Hq + Hkv) * D/16 rotation items, then n_v V items (none: V goes by runs of whole blocks).  F8: the
-// caches hold e4m3 of value * inv_k / inv_v (the attention kernels scale back).
-template <bool F8, int VM>
-__device__ __forceinline__ void rope_kv_item(const uint16_t* __restrict__ qkv, const int32_t* __restrict__ positions,
-                                             const int32_t* __restrict__ slots, const float* __restrict__ cos_sin,
-                                             uint16_t* __restrict__ q_out, void* __restrict__ k_cache, void* __restrict__ v_cache, int tok,
-                                             int it, int T, int Hq, int Hkv, int D, int n_v, float inv_k, float inv_v,
-                                             const float* __restrict__ part, int split) {
+template <bool F8, int VM = 0>
+__global__ void __launch_bounds__(64) rope_kv_kernel(const uint16_t* __restrict__ qkv, const int32_t* __restrict__ positions,
+                                                     const int32_t* __restrict__ slots, const float* __restrict__ cos_sin,
+                                                     uint16_t* __restrict__ q_out, void* __restrict__ k_cache,
+                                                     void* __restrict__ v_cache, int Hq, int Hkv, int D,
+                                                     int write_v, float inv_k, float inv_v,
+                                                     const float* __restrict__ part = nullptr, int split = 0) {
+  // grid = (T, ceil(items / 64)): one 8-element item per thread -- (Hq + Hkv) * D/16 rotation
+  // items then Hkv * D/8 V items -- so a decode batch of 128 tokens is ~900 blocks, not 128.
+  // write_v = 0: V goes through v_cache_runs_kernel instead (prefill: whole blocks, 16-B stores).
+  // F8: the caches hold e4m3 of value * inv_k / inv_v (the attention kernels scale back).
+  const int tok = blockIdx.x;
   const int half = D / 2, nv = half / 8;  // 8-element vectors per half-head
   const int n_rot = (Hq + Hkv) * nv;
+  const int n_v = write_v ? Hkv * (D / 8) : 0;
+  const int it = blockIdx.y * 64 + threadIdx.x;
   if (it >= n_rot + n_v) return;
   const int stride = (Hq + 2 * Hkv) * D;
-  const size_t row0 = (size_t)tok * stride, slab = (size_t)T * stride;
+  const size_t row0 = (size_t)tok * stride, slab = (size_t)gridDim.x * stride;
   const int slot = slots[tok];
   if (it < n_rot) {
     const int head = it / nv, c = it - head * nv;  // head < Hq: query, else key (head - Hq)
@@ -53,18 +59,6 @@ __device__ __forceinline__ void rope_kv_item(const uint16_t* __restrict__ qkv, c
   }
 }
 
-// grid = (T, ceil(items / 64)): a decode batch of 128 tokens is ~900 blocks, not 128
-template <bool F8, int VM = 0>
-__global__ void __launch_bounds__(64) rope_kv_kernel(const uint16_t* __restrict__ qkv, const int32_t* __restrict__ positions,
-                                                     const int32_t* __restrict__ slots, const float* __restrict__ cos_sin,
-                                                     uint16_t* __restrict__ q_out, void* __restrict__ k_cache,
-                                                     void* __restrict__ v_cache, int Hq, int Hkv, int D,
-                                                     int write_v, float inv_k, float inv_v,
-                                                     const float* __restrict__ part = nullptr, int split = 0) {
-  rope_kv_item<F8, VM>(qkv, positions, slots, cos_sin, q_out, k_cache, v_cache, blockIdx.x, blockIdx.y * 64 + threadIdx.x, gridDim.x, Hq,
-                       Hkv, D, write_v ? Hkv * (D / 8) : 0, inv_k, inv_v, part, split);
-}
-
 // Prefill V-cache writer.  One workgroup per (run, kv-head); a run = consecutive tokens that land
 // in ONE cache block at consecutive offsets (runs[r] = {first token, count, block, first offset},
 // built on the host from the slots).  The run's V rows are staged in LDS and written out as the
@@ -72,24 +66,13 @@ __global__ void __launch_bounds__(64) rope_kv_kernel(const uint16_t* __restrict_
 // 8-slot chunks, a partial run (chunk edges, prefix-cache continuations) per element so the
 // block's other slots are left untouched.  Replaces the 2-byte scattered stores of the per-token
 // path (1.85 TB/s effective for rope_kv at a prefill chunk, profiles/elementwise_bw_probe_r01.log).
-// The same launch turns queries and keys, a wave 64 items of a token, in the workgroups past the runs': neither waits for the other, and a
-// launch of its own cost 2.8 us a layer and its host (us of a pass of four: 30 rows 474 -> 461, 291 881 -> 870, 420 991 -> 983, 15.8 k 20.83 ms -> 20.72).
 template <bool F8>
-__global__ void __launch_bounds__(256) rope_kv_runs_kernel(const uint16_t* __restrict__ qkv, const int32_t* __restrict__ positions,
-                                                           const int32_t* __restrict__ slots, const float* __restrict__ cos_sin,
-                                                           uint16_t* __restrict__ q_out, void* __restrict__ k_cache,
-                                                           void* __restrict__ v_cache, const int32_t* __restrict__ runs, int R, int T,
-                                                           int Hq, int Hkv, int D, float inv_k, float inv_v) {
-  if ((int)blockIdx.x >= R * Hkv) {
-    const int per = ((Hq + Hkv) * (D / 16) + 63) / 64;       // waves of a token
-    const int wave = __builtin_amdgcn_readfirstlane(((int)blockIdx.x - R * Hkv) * 4 + (threadIdx.x >> 6)), tok = wave / per;
-    if (tok < T)
-      rope_kv_item<F8, 0>(qkv, positions, slots, cos_sin, q_out, k_cache, v_cache, tok, (wave - tok * per) * 64 + (threadIdx.x & 63), T, Hq,
-                          Hkv, D, 0, inv_k, inv_v, nullptr, 0);
-    return;
-  }
+__global__ void __launch_bounds__(256) v_cache_runs_kernel(const uint16_t* __restrict__ qkv,
+                                                           const int32_t* __restrict__ runs,
+                                                           void* __restrict__ v_cache, int Hq, int Hkv, int D,
+                                                           float inv_v) {
   __shared__ __attribute__((aligned(16))) uint16_t sv[KV_BS][256 + 8];
-  const int kh = blockIdx.x / R, r = blockIdx.x - kh * R, tid = threadIdx.x;
+  const int r = blockIdx.x, kh = blockIdx.y, tid = threadIdx.x;
   const int t0 = runs[4 * r], n = runs[4 * r + 1], blk = runs[4 * r + 2], off0 = runs[4 * r + 3];
   const int nc = D / 8;
   const size_t stride = (size_t)(Hq + 2 * Hkv) * D;
@@ -680,21 +663,22 @@ CFC_API int cfc_rope_kv_write_fp8(const void* qkv, const int32_t* positions, con
   return CFC_CHECK_LAUNCH();
 }
 
-// cfc_rope_kv_write without V (fp8 != 0: as cfc_rope_kv_write_fp8) and V by runs, in one launch.
 // runs: [R][4] int32 {first token, count (1..32), cache block, first offset (count + offset <= 32)}
-CFC_API int cfc_rope_kv_write_runs(const void* qkv, const int32_t* positions, const int32_t* slots, const float* cos_sin, void* q_out,
-                                   void* k_cache, void* v_cache, const int32_t* runs, int R, int T, int Hq, int Hkv, int head_dim, int fp8,
-                                   float inv_k, float inv_v, hipStream_t stream) {
-  if (head_dim % 16 != 0 || head_dim > 256 || T < 0 || R < 0) return -1;
-  const int64_t waves = (int64_t)T * (((Hq + Hkv) * (head_dim / 16) + 63) / 64), blocks = (int64_t)R * Hkv + (waves + 3) / 4;
-  if (blocks == 0) return 0;
-  if (blocks > 0x7fffffff || waves > 0x7ffffff0) return -1;
-#define RR(F8)                                                                                                                   \
-  rope_kv_runs_kernel<F8><<<(unsigned)blocks, 256, 0, stream>>>((const uint16_t*)qkv, positions, slots, cos_sin, (uint16_t*)q_out, \
-                                                                k_cache, v_cache, runs, R, T, Hq, Hkv, head_dim, inv_k, inv_v)
-  if (fp8) RR(true);
-  else RR(false);
-#undef RR
+CFC_API int cfc_v_cache_write_runs(const void* qkv, const int32_t* runs, int R, void* v_cache, int Hq, int Hkv,
+                                   int head_dim, hipStream_t stream) {
+  if (head_dim % 8 != 0 || head_dim > 256 || R < 0) return -1;
+  if (R == 0) return 0;
+  v_cache_runs_kernel<false><<<dim3(R, Hkv), 256, 0, stream>>>((const uint16_t*)qkv, runs, v_cache, Hq, Hkv,
+                                                               head_dim, 1.f);
+  return CFC_CHECK_LAUNCH();
+}
+
+CFC_API int cfc_v_cache_write_runs_fp8(const void* qkv, const int32_t* runs, int R, void* v_cache, int Hq, int Hkv,
+                                       int head_dim, float inv_v, hipStream_t stream) {
+  if (head_dim % 8 != 0 || head_dim > 256 || R < 0) return -1;
+  if (R == 0) return 0;
+  v_cache_runs_kernel<true><<<dim3(R, Hkv), 256, 0, stream>>>((const uint16_t*)qkv, runs, v_cache, Hq, Hkv, head_dim,
+                                                              inv_v);
   return CFC_CHECK_LAUNCH();
 }
 

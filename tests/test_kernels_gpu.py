@@ -76,24 +76,6 @@ def test_rope_kv_write():
     _close(vc, vc2, 1e-6, 0)
 
 
-@pytest.mark.parametrize("Hq,Hkv,D", [(1, 1, 16), (3, 1, 64), (8, 2, 128), (32, 8, 128), (6, 3, 256), (28, 4, 48)])
-@pytest.mark.parametrize("slots", [[0], [37], list(range(64, 96)), list(range(5, 32)) + list(range(160, 192)) + [200, 100, 101], [7, -1]])
-def test_rope_kv_write_of_runs_in_one_launch(Hq, Hkv, D, slots):
-    """Queries, keys and whole-block values side by side: the bytes of the path that writes a token's values one by one."""
-    T = len(slots)
-    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, device=DEV).bfloat16()
-    pos, sl = (torch.tensor(x, dtype=torch.int32, device=DEV) for x in (list(range(3, 3 + T)), slots))
-    cs = R.rope_cos_sin(256, D, 1e4, device=DEV)
-    kc, vc = (torch.randn(7, Hkv, *d, device=DEV).bfloat16() for d in ((32, D), (D, 32)))
-    k2, v2 = kc.clone(), vc.clone()
-    runs = torch.from_numpy(K.v_runs([s for s in slots if s >= 0])).to(DEV)      # the idle row is the last
-    q = K.rope_kv_write(qkv, pos, sl, cs, kc, vc, Hq, Hkv, D)
-    assert torch.equal(q, K.rope_kv_write(qkv, pos, sl, cs, k2, v2, Hq, Hkv, D, runs=runs))
-    assert torch.equal(kc, k2) and torch.equal(vc, v2)
-    k2.zero_(), v2.zero_()
-    assert torch.equal(q, K.rope_kv_write(qkv, pos, sl, cs, k2, v2, Hq, Hkv, D, runs=runs[:0])) and not v2.any()
-
-
 def test_rope_kv_write_prefill_runs():
     """The prefill V path (whole-block runs, 16-B stores; partial runs per element) writes exactly
     what the per-token path writes and leaves the other slots of partially written blocks alone."""
