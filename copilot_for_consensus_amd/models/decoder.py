@@ -483,11 +483,9 @@ class DecoderModel:
                             and not self.fp8)
         self.fused_decode = mode == "dgemm"
         # decode RoPE + KV write inside the attention kernel's prologue: CFC_DECODE_ROPE_FUSED "1"
-        # always, "0" never, unset: for B <= 4.  Measured in the headline (profiles/r04_ab_*.log) the
-        # fused BATCHED step decodes slower (6.30 vs 6.09 s per batch): every attention workgroup
-        # waits ~5 us for its q slabs, the RoPE and the K/V store before its first KV load, twice
-        # per CU, which costs more than the 10.6-us rope_kv launch it removes.  At B = 1 the launch
-        # is the larger cost: 296.5 -> 299.9 tok/s Mistral-7B (profiles/r04_latprof_*).
+        # always, "0" never, unset: where K.rope_inside finds that it pays.  Every attention workgroup
+        # starts 4 us later for it, which two long ones a CU do not win back; elsewhere the launch
+        # is the larger cost (B = 1: 296.5 -> 299.9 tok/s Mistral-7B, profiles/r04_latprof_*).
         self.rope_fused = os.environ.get("CFC_DECODE_ROPE_FUSED", "")
         # B <= 4 over packed weights: residual + RMSNorm folded into the next GEMV (K.gemv_norm).
         # Opt-in: bit-identical, two launches fewer per layer, but slower -- the prologue's slab reads
@@ -914,8 +912,8 @@ class DecoderModel:
 
     def _rope_attention(self, i, qkv, positions, slots, ctx_lens, block_tables, kv, attn_workspace, part_blocks):
         """RoPE + K/V cache write + paged decode attention of layer ``i`` from the qkv projection output
-        (bf16 [B, N], or fp32 split-K slabs [split, B, N]).  Default: ONE kernel (the attention's
-        prologue does the RoPE / KV write, ``CFC_DECODE_ROPE_FUSED=1``); else rope_kv then attention.
+        (bf16 [B, N], or fp32 split-K slabs [split, B, N]).  ONE kernel (the attention's prologue does
+        the RoPE / KV write) where that pays or with ``CFC_DECODE_ROPE_FUSED=1``; else rope_kv then attention.
         Both write the same cache bytes and return the same output."""
         cfg, w = self.cfg, self.w
         sb = getattr(self, "_shared_blocks", None)
