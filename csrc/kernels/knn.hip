@@ -271,12 +271,11 @@ struct KnnUnit {
 };
 
 // WORDS: there are norms or a mask.  FQ: the queries are floats, as above
-template <int KC, bool MAXIMA, bool WORDS, bool FQ = false>
-__global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __restrict__ X, const void* __restrict__ Q, int N,
-                                                            int nq, const float* __restrict__ xnorm2,
-                                                            const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
-                                                            float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
-                                                            int B, bool unit) {
+template <int KC, bool MAXIMA, bool WORDS, bool FQ>
+__device__ __forceinline__ void knn_stream(const uint16_t* __restrict__ X, const void* __restrict__ Q, int N, int nq,
+                                           const float* __restrict__ xnorm2, const float* __restrict__ qnorm2,
+                                           const uint8_t* __restrict__ alive, float* __restrict__ out, size_t ld,
+                                           uint32_t* __restrict__ bmax, int nb, int B, bool unit) {
   constexpr int KU = KnnUnit<KC>::KU, R = KnnUnit<KC>::R, NU = KnnUnit<KC>::NU, UB = KU * 1024;
   __shared__ __attribute__((aligned(16))) char kn_smem[4 * R * (UB + (WORDS ? 256 : 0))];      // rings, then those of norms and masks
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
@@ -389,6 +388,23 @@ __global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __re
       bmax[(size_t)col * nb + blk] = best;
     }
   }
+}
+
+template <int KC, bool MAXIMA, bool WORDS>
+__global__ void __launch_bounds__(256, 1) knn_stream_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Q, int N,
+                                                            int nq, const float* __restrict__ xnorm2,
+                                                            const float* __restrict__ qnorm2, const uint8_t* __restrict__ alive,
+                                                            float* __restrict__ out, size_t ld, uint32_t* __restrict__ bmax, int nb,
+                                                            int B) {
+  knn_stream<KC, MAXIMA, WORDS, false>(X, Q, N, nq, xnorm2, qnorm2, alive, out, ld, bmax, nb, B, false);
+}
+
+template <int KC, bool WORDS>
+__global__ void __launch_bounds__(256, 1) knn_stream_floats_kernel(const uint16_t* __restrict__ X, const float* __restrict__ Q, int N,
+                                                                   int nq, const float* __restrict__ xnorm2,
+                                                                   const uint8_t* __restrict__ alive, float* __restrict__ out,
+                                                                   size_t ld, uint32_t* __restrict__ bmax, int nb, int B, bool unit) {
+  knn_stream<KC, false, WORDS, true>(X, Q, N, nq, xnorm2, nullptr, alive, out, ld, bmax, nb, B, unit);
 }
 
 // The scores of `kb` blocks of 16 rows per query (blocks [nq][kb], in any order) into out [nq][16 kb] and their rows into
@@ -1013,7 +1029,7 @@ constexpr int KNN_CUS = 256;
 // LDS-DMA's sources are whole sixteens of bytes; rows that lie otherwise come to registers
 bool knn_aligned(const void* X) { return ((uintptr_t)X & 15) == 0; }
 
-#define KNN_ARGS(OUT, B) (const uint16_t*)X, Q, N, nq, xnorm2, qnorm2, alive, OUT, (size_t)ld, B
+#define KNN_ARGS(OUT, B) (const uint16_t*)X, (const uint16_t*)Q, N, nq, xnorm2, qnorm2, alive, OUT, (size_t)ld, B
 
 // floats: where Q holds floats the scan takes them itself, if its workgroups are no more than a round (each takes the queries to LDS) and
 // these fit beside the rings; where it does not, *floats is cleared and nothing launched
@@ -1024,15 +1040,18 @@ static int knn_scan_go(const void* X, const void* Q, int N, int nq, int dim, con
   if (bmax && (long)nq * nb > room) return -1;
   const int all = (nb + 3) / 4;
   const long bytes = (long)N * dim * 2;
-#define ST(KC, W, F) knn_stream_kernel<KC, false, W, F><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B, unit)
+#define ST(KC, W)                                                                                                                      \
+  if (floats) knn_stream_floats_kernel<KC, W><<<min(all, KNN_CUS), 256, 0, stream>>>((const uint16_t*)X, (const float*)Q, N, nq, xnorm2, \
+                                                                                     alive, out, (size_t)ld, bmax, nb, B, unit);        \
+  else knn_stream_kernel<KC, false, W><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B)
 #define SC(KC, F) knn_scan_kernel<KC, false, F><<<grid, 256, 0, stream>>>(KNN_ARGS(out, bmax), nb, B, unit)
 #define KS(KC)                                                                                         \
   {                                                                                                    \
     if constexpr (KC > 4)                                                                              \
       if (knn_aligned(X) && (KC > 16 || bytes > KNN_STREAM_BYTES)) {                                   \
         if (floats && nq > KnnFloats<KC>::FROWS) { *floats = false; return 0; }                        \
-        if (xnorm2 || alive) { if (floats) ST(KC, true, true); else ST(KC, true, false); }             \
-        else { if (floats) ST(KC, false, true); else ST(KC, false, false); }                           \
+        if (xnorm2 || alive) { ST(KC, true); }                                                         \
+        else { ST(KC, false); }                                                                        \
         break;                                                                                         \
       }                                                                                                \
     const int grid = KC <= 16 && bytes <= KNN_ROUND_BYTES ? min(all, KNN_ROUND) : all;                 \
@@ -1064,8 +1083,8 @@ CFC_API int cfc_knn_maxima(const void* X, const void* Q, int N, int nq, int dim,
 #define KS(KC)                                                                                                              \
   if constexpr (KC > 4)                                                                                                     \
     if (knn_aligned(X)) {                                                                                                   \
-      if (xnorm2 || alive) knn_stream_kernel<KC, true, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64, false); \
-      else knn_stream_kernel<KC, true, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64, false);       \
+      if (xnorm2 || alive) knn_stream_kernel<KC, true, true><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64); \
+      else knn_stream_kernel<KC, true, false><<<min(all, KNN_CUS), 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64);       \
       break;                                                                                                                \
     }                                                                                                                       \
   knn_scan_kernel<KC, true><<<all, 256, 0, stream>>>(KNN_ARGS(out, nullptr), nb, 64, false);                                       \
