@@ -15,15 +15,7 @@ from .cols import Cols
 from .kernels import _req, _stream
 from .stream import _act
 
-
-
-def chunk_rows(rows: int) -> int:
-    """Tokens per chunk of the prompt kernels in a pass of so many rows.  A chunk is a chain, 13 and 16 us for 64 tokens of the two
-    passes over it; a short one has its two sums to write, read and carry for fewer tokens.  us of a pass in chunks of 64, 32, 16
-    and 8: tadolix of 54 rows 692, 653, 635, 628, of 291 1083, 1043, 1030, 1022, of 1166 2490, 2448, 2447, 2451, of 2800 4712, 4687, 4677,
-    4747, of 9300 14160, 14139, 14148, 14198; pemolorn of 291 1182, 1147, 1131, 1125, of 1166 2253, 2215, 2208, 2207, of 2800 4141, 4139,
-    4152, 4180, of 5300 6613, 6581, 6603, 6641."""
-    return 8 if rows <= 512 else 16 if rows <= 2048 else 32
+CHUNK = 64               # tokens per chunk of the prompt kernels
 
 
 @dataclasses.dataclass
@@ -37,10 +29,9 @@ class Gru:
         return self.bz.numel()
 
 
-def chunk_plan(cu, size: int | None = None) -> tuple[np.ndarray, np.ndarray]:
-    """(chunks [n, 2]: first row and rows, first chunk per portion [portions + 1]) of packed portions, in chunks of ``size``
-    (None: :func:`chunk_rows`)."""
-    chunks, at, size = [], [0], size or chunk_rows(int(cu[-1]) - int(cu[0]))
+def chunk_plan(cu, size: int = CHUNK) -> tuple[np.ndarray, np.ndarray]:
+    """(chunks [n, 2]: first row and rows, first chunk per portion [portions + 1]) of packed portions."""
+    chunks, at = [], [0]
     for a, b in zip(cu, cu[1:]):
         chunks += [(r, min(size, b - r)) for r in range(a, b, size)]
         at.append(len(chunks))

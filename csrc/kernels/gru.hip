@@ -3,7 +3,7 @@
 // element by element, and the layer's output S_t silu(pre_g).  States are fp32, one row per sequence slot; a sequence's
 // first token starts from zero whatever the slot holds.
 //   * gru_step    one token per sequence, straight from a joint product's slabs
-//   * gru_chunk   prompt portions, chunks of 8 to 32 tokens in parallel: each chunk's decay (the product of 1 - z) and what
+//   * gru_chunk   prompt portions, chunks of 64 tokens in parallel: each chunk's decay (the product of 1 - z) and what
 //                 it adds to a state of zero
 //   * carry       per sequence through its chunks: the state ahead of each, and the one the portion leaves (recur.h)
 //   * gru_apply   the chunks again from their states: outputs

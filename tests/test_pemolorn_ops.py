@@ -143,16 +143,30 @@ def test_recurrence_in_portions_and_decoded(device, dtype, W):
 
 
 @pytest.mark.parametrize("device", DEVICES)
-@pytest.mark.parametrize("size", [16, 32])
-def test_recurrence_in_chunks_of_larger_passes(device, size, monkeypatch):
-    """The chunks of passes of more rows than the portions here have; chunk and pass edges of every size."""
-    monkeypatch.setattr(R, "chunk_rows", lambda rows: size)
-    for W in (33, 260):
-        test_recurrence_in_portions_and_decoded(device, torch.float32, W)
-    for rows, want in ((1, 8), (512, 8), (513, 16), (2048, 16), (2049, 32)):
-        monkeypatch.undo()
-        ch, cu = R.chunk_plan([0, rows])
-        assert ch[0].tolist() == [0, min(want, rows)] and ch[:, 1].sum() == rows and cu.tolist() == [0, -(-rows // want)]
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_recurrence_of_a_portion_whatever_else_is_in_its_pass(device, dtype):
+    """A portion's chunks, so the order of its sums: the bits of its outputs and state alone are those beside others."""
+    lens, W = [130, 203, 300, 1500], 260
+    cu = np.cumsum([0] + lens).tolist()
+    for a, b in zip(cu, cu[1:]):
+        rows = R.chunk_plan([0, b - a])[0][:, 1]
+        assert (rows[:-1] == 64).all() and rows.sum() == b - a
+    zug = torch.cat([rnd(cu[-1], W, seed=s, scale=2.0) for s in (1, 2, 3)], 1).to(device, dtype)
+    p = R.Gru((rnd(W, seed=4) - 2.0).to(device), rnd(W, seed=5).to(device))
+
+    def run(parts):
+        rows = torch.cat([zug[cu[s]:cu[s + 1]] for s in parts])
+        at = np.cumsum([0] + [lens[s] for s in parts]).tolist()
+        ch, ccu = R.chunk_plan(at)
+        state = torch.zeros(len(lens), W, device=device)
+        out = R.prefill(p, *(Cols(rows, k * W, W) for k in range(3)), i32(parts, device), i32(at, device), i32([lens[s] for s in parts], device),
+                        i32(ch, device), i32(ccu, device), state, torch.empty(at[-1], W, dtype=dtype, device=device))
+        return state, out.split([lens[s] for s in parts])
+
+    state, outs = run([3, 1, 0, 2])
+    for s, out in zip([3, 1, 0, 2], outs):
+        alone, (own,) = run([s])
+        assert torch.equal(alone[s], state[s]) and torch.equal(own, out)
 
 
 # ------------------------------------------------------------------ projections to queries and cache rows
