@@ -28,10 +28,13 @@ KV_BLOCK = ref.KV_BLOCK
 
 
 def _stream(t: torch.Tensor) -> int:
-    """The current stream of t's GPU.  (Its handle alone: torch.cuda.current_stream makes an object of it first, which took a
-    tenth of the host's time of a short prompt, some 60 launches: four layers of vofosun, 75 rows, 744 -> 627 us, of mistral,
-    24 rows, 601 -> 483, a search of 30 000 rows 33 -> 27.)"""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    """The current stream of t's GPU; a tensor that is on none must not reach a kernel.  (The stream's handle alone:
+    torch.cuda.current_stream makes an object of it first, which took a tenth of the host's time of a short prompt, some 60
+    launches: four layers of vofosun, 75 rows, 744 -> 627 us, of mistral, 24 rows, 601 -> 483, a search of 30 000 rows 33 -> 27.)"""
+    device = t.get_device()
+    if device < 0:                     # which would mean the current GPU
+        raise ValueError(f"expected a tensor on a GPU, not one on {t.device}")
+    return torch._C._cuda_getCurrentRawStream(device)
 
 
 def _p(t):

@@ -1,0 +1,42 @@
+"""Tensors in host memory never reach a kernel: what has no path for them refuses them before anything is launched."""
+import pytest
+import torch
+
+from copilot_for_consensus_amd.ops import kernels as K
+
+
+class _Launched(Exception):
+    pass
+
+
+@pytest.fixture
+def no_launch(monkeypatch):
+    """Any call of the native library is one too many."""
+    class Lib:
+        def __getattr__(self, name):
+            def call(*a):
+                raise _Launched(name)
+            return call
+    monkeypatch.setattr(K, "kernels", Lib)
+    # what a process with a GPU gives for a device of -1: the current device's stream
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 0)
+
+
+def test_the_stream_of_a_host_tensor(no_launch):
+    with pytest.raises(ValueError, match="cpu"):
+        K._stream(torch.empty(1))
+
+
+def _quantized():
+    return K.QWeight(8, 4, 32, torch.zeros(64, dtype=torch.uint8), (0,))
+
+
+@pytest.mark.parametrize("call", [
+    lambda: K.qgemv(torch.zeros(1, 32, dtype=torch.bfloat16), _quantized()),
+    lambda: K.knn_queries(torch.zeros(2, 64), True),
+    lambda: K.ivf_topk(torch.zeros(8, 64, dtype=torch.bfloat16), torch.zeros(1, 64, dtype=torch.bfloat16), torch.zeros(1, 1, dtype=torch.int32),
+                       torch.tensor([0, 8]), 1, 4),
+], ids=["qgemv", "knn_queries", "ivf_topk"])
+def test_what_has_no_host_path(no_launch, call):
+    with pytest.raises(ValueError, match="cpu"):
+        call()
