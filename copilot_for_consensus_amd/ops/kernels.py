@@ -1714,7 +1714,8 @@ def knn_topk(X, Q, k: int, xnorm2=None, qnorm2=None, alive=None, row_lo: int = 0
 
 
 def knn_search(X, q, k: int, unit: bool, xnorm2=None, alive=None, row_lo: int = 0, N: int | None = None):
-    """:func:`knn_topk` of fp32 queries ``q`` [nq, dim] on the GPU, of unit length if ``unit``: up to KNN_SCORES rows by one call."""
+    """:func:`knn_topk` of fp32 queries ``q`` [nq, dim], 16-byte aligned on X's GPU, of unit length if ``unit``: up to KNN_SCORES rows
+    by one call."""
     N = X.shape[0] if N is None else N
     nq, dim, n = q.shape[0], X.shape[1], N - row_lo
     if not 1 <= k <= 256 or not 1 <= nq <= 16 or not 0 <= row_lo < N <= X.shape[0] or n > KNN_SCORES or _topk_parts(n) > 1:
@@ -1723,6 +1724,8 @@ def knn_search(X, q, k: int, unit: bool, xnorm2=None, alive=None, row_lo: int = 
     _req(q, torch.float32, "knn_search")
     if q.shape != (nq, dim):
         raise ValueError(f"knn_search: queries {tuple(q.shape)} for rows of {dim}")
+    if q.device != X.device or q.data_ptr() % 16:
+        raise ValueError(f"knn_search: queries on {q.device} at {q.data_ptr():#x}, to lie at 16 bytes on {X.device}")
     lib, dev, k = kernels(), X.device, min(k, n)
     room = lib.cfc_knn_search_bytes(n, nq, dim)
     ws = torch.empty(room, dtype=torch.uint8, device=dev)

@@ -40,3 +40,33 @@ def _quantized():
 def test_what_has_no_host_path(no_launch, call):
     with pytest.raises(ValueError, match="cpu"):
         call()
+
+
+class _Rows(torch.Tensor):
+    """Rows of an index that say to be on a GPU."""
+    @property
+    def device(self):
+        return torch.device("cuda", 0)
+
+    def get_device(self):
+        return 0
+
+
+def test_queries_of_a_search_lie_beside_the_index(no_launch, monkeypatch):
+    monkeypatch.setattr(K, "_topk_parts", lambda n: 1)
+    X = torch.zeros(8, 64, dtype=torch.bfloat16).as_subclass(_Rows)
+    for q in (torch.zeros(1, 64), torch.zeros(1, 64, device="meta")):
+        with pytest.raises(ValueError, match="queries on"):
+            K.knn_search(X, q, 4, True)
+    with pytest.raises(_Launched):                   # what lies there goes on to the kernels
+        K.knn_search(X, torch.zeros(1, 64).as_subclass(_Rows), 4, True)
+
+
+@pytest.mark.gpu
+def test_queries_of_a_search_on_the_gpu():
+    X, q = torch.zeros(8, 64, dtype=torch.bfloat16, device="cuda"), torch.zeros(66, device="cuda")
+    with pytest.raises(ValueError, match="queries on"):
+        K.knn_search(X, q[:64].view(1, 64).cpu(), 4, True)
+    with pytest.raises(ValueError, match="16 bytes"):
+        K.knn_search(X, q[1:65].view(1, 64), 4, True)
+    assert K.knn_search(X, q[:64].view(1, 64), 4, True)[1].tolist() == [[0, 1, 2, 3]]
