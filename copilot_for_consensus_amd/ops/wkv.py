@@ -60,7 +60,7 @@ def scan_runs(H: int, sequences: int, chunks: int) -> int:
     heads), portions in 1, 2, 4, 8 and 16 runs: one of 150 rows 1386, 1383, 1374, 1381, 1392, of 1400 3967, 3897, 3794, 3771, 3804, of 2800
     6360, 6215, 6049, 6027, 6065; two of 1240 5800, 5752, 5723, 5748, 5804; but three of 390 3500, 3515, 3519, 3539, four of 1240 9815,
     9865, 9874, 9949: from 192 workgroups on the CUs have enough to do."""
-    return max(1, min(512 // (H * sequences), chunks // sequences // 3)) if H * sequences <= 128 else 1
+    return max(1, min(512 // (H * sequences), chunks // sequences // 3)) if 0 < H * sequences <= 128 else 1
 
 
 def _ref(p: Wkv, r, k, v, g, w1, slots, cu, ctx, state, out):

@@ -224,6 +224,19 @@ def test_runs_of_a_scan():
         k = R.scan_runs(H, n, chunks)
         assert k == 1 or (k * H * n <= 512 and 3 * k * n <= chunks)
         assert k >= 1 and (H * n <= 128 or k == 1)
+    assert R.scan_runs(64, 0, 0) == 1 == R.scan_runs(64, 1, 0)               # of nothing, one that returns
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_recurrence_of_no_sequences(device):
+    H, D, rank = 2, 64, 24
+    p = {k: v.to(device) for k, v in wkv_case(H, D, rank, 1, seed=5)[0].items()}
+    mix = R.Wkv(H, D, rank, p["w2"], p["w0"], p["u"], p["norm"], 1e-4)
+    none, state, empty = i32([], device), torch.ones(3, H, D, D, device=device), torch.empty(0, H * D, device=device)
+    ch, ccu = R.chunk_plan([0])
+    out = R.prefill(mix, *(Cols(empty) for _ in "rkvg"), Cols(torch.empty(1, 0, rank, device=device)), none, i32([0], device), none,
+                    i32(ch, device), i32(ccu, device), state, torch.empty_like(empty))
+    assert out.shape == (0, H * D) and bool((state == 1).all())
 
 
 # ------------------------------------------------------------------ latent attention
