@@ -28,7 +28,7 @@ L = c_int64
 _KERNEL_SIGS = {
     "cfc_rmsnorm": [P, P, P, P, I, I, F, I, P],
     "cfc_embed_rmsnorm": [P, P, P, P, P, I, I, F, P],
-    "cfc_rmsnorm_rows": [P, P, P, P, P, I, I, F, P],
+    "cfc_rmsnorm_rows": [P, P, P, P, P, I, I, I, F, P],
     "cfc_layernorm": [P, P, P, P, P, P, P, P, P, P, I, I, F, I, P],
     "cfc_paged_decode_attention": [P, P, P, P, P, I, I, I, I, I, I, I, F, I, P, P, P, P, P],
     "cfc_prefill_attention": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, P, P],

@@ -86,17 +86,20 @@ def embed_rmsnorm(table: torch.Tensor, ids: torch.Tensor, w: torch.Tensor, eps: 
 
 
 def rmsnorm_rows(x: torch.Tensor, residual: torch.Tensor, rows: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
-    """RMSNorm of the rows ``rows`` of x + residual, neither of which is changed, * w."""
+    """RMSNorm of the rows ``rows`` of x + residual, neither of which is changed, * w.  (On the GPU a row that there is not is NaN.)"""
     if not x.is_cuda:
         return rmsnorm(x.index_select(0, rows), w, eps, residual=residual.index_select(0, rows))
     _req(x, torch.bfloat16, "x")
     _req(residual, torch.bfloat16, "residual")
     if x.shape != residual.shape or x.dim() != 2:
         raise ValueError(f"rmsnorm_rows: x {tuple(x.shape)}, residual {tuple(residual.shape)}")
-    rows = rows.to(torch.int32).contiguous()
+    if rows.device != x.device or rows.dtype not in (torch.int32, torch.int64) or rows.dim() > 1:
+        raise ValueError(f"rmsnorm_rows: rows {tuple(rows.shape)} {rows.dtype} on {rows.device} of x on {x.device}")
+    n = x.shape[0]
+    rows = (rows if rows.dtype == torch.int32 else rows.clamp(-1, n).to(torch.int32)).contiguous()
     out = torch.empty(rows.numel(), x.shape[1], dtype=x.dtype, device=x.device)
     check(kernels().cfc_rmsnorm_rows(out.data_ptr(), residual.data_ptr(), x.data_ptr(), rows.data_ptr(), w.data_ptr(), rows.numel(),
-                                     x.shape[1], float(eps), _stream(x)), "cfc_rmsnorm_rows")
+                                     n, x.shape[1], float(eps), _stream(x)), "cfc_rmsnorm_rows")
     return out
 
 

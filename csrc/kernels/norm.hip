@@ -15,17 +15,20 @@ namespace {
 // that produces it, so the row makes no extra HBM round trip through a bf16 tensor.
 // RN_EMBED: x is a table of embeddings whose rows ids[] begin the stream: they are stored as the residual, too.  An embedding, a
 // copy and a norm of their own cost a decode step two launches more, 2.8 us each, and a prompt a pass over its rows more (15760 rows of
-// 4096: 171 us, so 78).  RN_ROWS: rows ids[] of x and of the residual, neither of which is written: the last tokens of prompts.
+// 4096: 171 us, so 78).  RN_ROWS: rows ids[] of x and of the residual, `sources` rows each, neither of which is written: the last tokens of
+// prompts; what is asked for and not there is NaN.
 enum { RN_ALL = 0, RN_EMBED = 1, RN_ROWS = 2 };
 template <int VPT, bool F8, int SRC = RN_ALL>
 __global__ void __launch_bounds__(1024) rmsnorm_kernel(void* __restrict__ out, float* __restrict__ scale,
                                                       uint16_t* __restrict__ residual,
                                                       const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                      int dim, float eps, int add_residual, const int32_t* __restrict__ ids) {
+                                                      int dim, float eps, int add_residual, const int32_t* __restrict__ ids, int sources) {
   __shared__ float red[16];
   const int row = blockIdx.x;
   const int nvec = dim >> 3;
-  const int from = SRC == RN_ALL ? row : ids[row];
+  const int at = SRC == RN_ALL ? row : ids[row];
+  const bool there = SRC != RN_ROWS || (unsigned)at < (unsigned)sources;
+  const int from = there ? at : 0;
   const uint4* xr = reinterpret_cast<const uint4*>(x + (size_t)from * dim);
   uint4* rr = reinterpret_cast<uint4*>(residual + (size_t)(SRC == RN_ROWS ? from : row) * dim);
   float v[VPT][8];
@@ -59,7 +62,7 @@ __global__ void __launch_bounds__(1024) rmsnorm_kernel(void* __restrict__ out, f
     }
   }
   ss = block_sum(ss, red);
-  const float inv = rsqrtf(ss / (float)dim + eps);
+  const float inv = there ? rsqrtf(ss / (float)dim + eps) : NAN;
   if constexpr (!F8) {
     uint4* orow = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + (size_t)row * dim);
 #pragma unroll
@@ -177,12 +180,12 @@ inline int pick_block(int nvec) { return nvec >= 1024 ? 1024 : ((nvec + 63) / 64
 
 template <bool F8, int SRC = RN_ALL>
 int launch_rmsnorm(void* out, float* scale, void* residual, const void* x, const void* w, int rows, int dim, float eps,
-                   int add_residual, hipStream_t stream, const int32_t* ids = nullptr) {
+                   int add_residual, hipStream_t stream, const int32_t* ids = nullptr, int sources = 0) {
   const int nvec = dim / 8, block = pick_block(nvec);
   const int vpt = (nvec + block - 1) / block;
 #define RN(V)                                                                                                               \
   rmsnorm_kernel<V, F8, SRC><<<rows, block, 0, stream>>>(out, scale, (uint16_t*)residual, (const uint16_t*)x, (const uint16_t*)w, dim, \
-                                                         eps, add_residual, ids)
+                                                         eps, add_residual, ids, sources)
   switch (vpt) {
     case 1: RN(1); break;
     case 2: RN(2); break;
@@ -211,11 +214,11 @@ CFC_API int cfc_embed_rmsnorm(void* out, void* residual, const void* table, cons
   return launch_rmsnorm<false, RN_EMBED>(out, nullptr, residual, table, w, rows, dim, eps, 0, stream, ids);
 }
 
-// out [rows, dim] = RMSNorm of (x + residual)'s rows ids[] * w; x and residual stay as they are
-CFC_API int cfc_rmsnorm_rows(void* out, const void* residual, const void* x, const int32_t* ids, const void* w, int rows, int dim,
-                             float eps, hipStream_t stream) {
-  if (dim % 8 != 0 || rows <= 0 || !ids || !residual) return -1;
-  return launch_rmsnorm<false, RN_ROWS>(out, nullptr, (void*)residual, x, w, rows, dim, eps, 1, stream, ids);
+// out [rows, dim] = RMSNorm of (x + residual)'s rows ids[] * w, NaN for what is none of [0, sources); x and residual stay as they are
+CFC_API int cfc_rmsnorm_rows(void* out, const void* residual, const void* x, const int32_t* ids, const void* w, int rows, int sources,
+                             int dim, float eps, hipStream_t stream) {
+  if (dim % 8 != 0 || rows <= 0 || sources <= 0 || !ids || !residual) return -1;
+  return launch_rmsnorm<false, RN_ROWS>(out, nullptr, (void*)residual, x, w, rows, dim, eps, 1, stream, ids, sources);
 }
 
 // FP8 output: out [rows, dim] e4m3fn, scale [rows] f32 with RMSNorm(...) ~= out * scale.

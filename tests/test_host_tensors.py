@@ -62,11 +62,19 @@ def test_queries_of_a_search_lie_beside_the_index(no_launch, monkeypatch):
         K.knn_search(X, torch.zeros(1, 64).as_subclass(_Rows), 4, True)
 
 
+def test_rows_of_a_norm_lie_beside_what_they_are_of(no_launch):
+    class OnGpu(_Rows):
+        is_cuda = True
+    x = torch.zeros(4, 8, dtype=torch.bfloat16).as_subclass(OnGpu)
+    with pytest.raises(ValueError, match="rows"):
+        K.rmsnorm_rows(x, x, torch.zeros(1, dtype=torch.int32), x[0], 1e-5)
+
+
 @pytest.mark.gpu
 def test_queries_of_a_search_on_the_gpu():
-    X, q = torch.zeros(8, 64, dtype=torch.bfloat16, device="cuda"), torch.zeros(66, device="cuda")
+    X, q = torch.zeros(8, 128, dtype=torch.bfloat16, device="cuda"), torch.zeros(130, device="cuda")
     with pytest.raises(ValueError, match="queries on"):
-        K.knn_search(X, q[:64].view(1, 64).cpu(), 4, True)
+        K.knn_search(X, q[:128].view(1, 128).cpu(), 4, True)
     with pytest.raises(ValueError, match="16 bytes"):
-        K.knn_search(X, q[1:65].view(1, 64), 4, True)
-    assert K.knn_search(X, q[:64].view(1, 64), 4, True)[1].tolist() == [[0, 1, 2, 3]]
+        K.knn_search(X, q[1:129].view(1, 128), 4, True)
+    assert K.knn_search(X, q[:128].view(1, 128), 4, True)[1].tolist() == [[0, 1, 2, 3]]

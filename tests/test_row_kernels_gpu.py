@@ -79,6 +79,21 @@ def test_norms_of_gathered_rows(dim, T):
         K.rmsnorm_rows(x, res, ids[:0], w, 1e-5)
 
 
+@pytest.mark.parametrize("dim", [8, 4096, 8200])
+def test_norms_of_rows_that_are_not_there(dim):
+    """Nothing is read past the rows; a place beside the rows, or an index of no whole numbers, is refused."""
+    from copilot_for_consensus_amd.ops import kernels as K
+    x, res = (torch.randn(5, dim, device=DEV).to(torch.bfloat16) for _ in range(2))
+    w = torch.ones(dim, device=DEV, dtype=torch.bfloat16)
+    good = K.rmsnorm(x[4:].clone(), w, 1e-5, residual=res[4:].clone())
+    for dtype, rows in ((torch.int32, [5, 4, -1, 2 ** 31 - 1, -2 ** 31]), (torch.int64, [5, 4, -1, 2 ** 32, -2 ** 40])):
+        got = K.rmsnorm_rows(x, res, torch.tensor(rows, dtype=dtype, device=DEV), w, 1e-5)
+        assert torch.equal(got[1:2], good) and bool(got[[0, 2, 3, 4]].isnan().all())
+    for rows in (torch.tensor([0]), torch.tensor([0.0], device=DEV), torch.tensor([True], device=DEV), torch.tensor([[0]], device=DEV)):
+        with pytest.raises(ValueError):
+            K.rmsnorm_rows(x, res, rows, w, 1e-5)
+
+
 @pytest.mark.parametrize("E,top", [(1, 1), (8, 8), (63, 2), (64, 6), (65, 8), (200, 5), (1024, 8)])
 @pytest.mark.parametrize("kind", ["normal", "ties", "equal", "few"])
 def test_experts_chosen_among_equals(E, top, kind):
