@@ -919,7 +919,8 @@ class DecoderModel:
         sb = getattr(self, "_shared_blocks", None)
         B = qkv.shape[-2]
         fused = self.rope_fused == "1" or (self.rope_fused == "" and K.rope_inside(
-            B, w.kv_heads, block_tables.shape[1], part_blocks, kv.k[i].dtype == torch.bfloat16))
+            B, w.kv_heads, block_tables.shape[1], part_blocks,
+            kv.k[i].dtype == torch.bfloat16 and (kv.k[i].data_ptr() | kv.v[i].data_ptr()) % 16 == 0, self.window))
         if fused and qkv.is_cuda:
             return K.paged_decode_rope_attention(qkv, positions, slots, w.cos_sin, kv.k[i], kv.v[i], block_tables,
                                                  ctx_lens, self.scale, w.heads, w.kv_heads, cfg.head_dim,

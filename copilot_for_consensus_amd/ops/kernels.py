@@ -307,13 +307,21 @@ def paged_decode_attention(q, k_cache, v_cache, block_tables, ctx_lens, scale, o
     return out
 
 
-def rope_inside(B: int, Hkv: int, max_blocks: int, part_blocks: int, bf16: bool) -> bool:
-    """Whether a decode step's rotation and cache write are best inside its attention (:func:`paged_decode_rope_attention`): of few sequences, and
-    of more where the bf16 kernels that stream keys and values take them, but for contexts of more than 2048 keys
-    in two workgroups a CU (both measured in attention.hip)."""
+def rope_inside(B: int, Hkv: int, max_blocks: int, part_blocks: int, bf16: bool, window: int = 0) -> bool:
+    """Whether a decode step's rotation and cache write are best inside its attention (:func:`paged_decode_rope_attention`), of a cache in
+    ``bf16`` at whole sixteens of bytes.  Of up to four sequences always.  Of more in balanced slices: where the kernels that stream keys
+    and values take them, but for contexts of more than 2048 keys in two workgroups a CU (measured in attention.hip); where those
+    decline (:func:`paged_waves`), of up to two workgroups a CU: us a layer by a launch of its own and inside, 32 query and 8
+    key heads, 5 of 130 9.7 and 8.5, 5 of 700 in 6 slices 13.1 and 12.3, 24 of 250 14.2 and 12.3, 32 of 250 15.5 and 12.4, 16 of 500 in 4 17.1
+    and 16.3, 4 and 1 key heads, 5 of 400 in 5 11.3 and 9.9, 16 of 20 7.0 and 6.2; but 33 of 250 in 2 19.4 and
+    21.1, 24 of 350 in 3 19.2 and 20.3, 64 of 500 in 4 38.6 and 45.9, 128 of 250 in 2 41.8 and 47.6."""
     if B <= GEMV_MAX_M:
         return True
-    return bf16 and B <= 128 and part_blocks < 0 and (B * Hkv * -part_blocks <= 256 or max_blocks <= 64)
+    P, wgs = -part_blocks, B * Hkv * -part_blocks
+    if not bf16 or B > 128 or P <= 0 or (wgs > 256 and max_blocks > 64):
+        return False
+    seen = min(max_blocks, (window + 30) // KV_BLOCK + 1) if window else max_blocks
+    return wgs <= 512 or not paged_waves(wgs, seen, P)[2]
 
 
 def paged_decode_rope_attention(qkv, positions, slots, cos_sin, k_cache, v_cache, block_tables, ctx_lens, scale,

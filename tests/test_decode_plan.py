@@ -59,3 +59,20 @@ def test_where_a_decode_step_turns_its_queries():
     assert inside(5, 8, 500, -6, True) and inside(32, 8, 90, -1, True) and inside(128, 8, 64, -1, True)
     assert not inside(33, 8, 65, -1, True) and not inside(128, 8, 88, -2, True)      # long contexts, two workgroups a CU
     assert not inside(5, 8, 40, -6, False) and not inside(5, 8, 40, 16, True) and not inside(129, 8, 4, -1, True)
+
+
+def test_where_a_decode_step_turns_its_queries_without_the_ring():
+    """Kernels that take keys and values to registers: inside for up to two workgroups a CU, and so whatever the engine plans; not in
+    slices of a few blocks that are more, by their number or by a window."""
+    from copilot_for_consensus_amd.models.decoder import kv_partitions
+    from copilot_for_consensus_amd.ops import kernels as K
+    inside = K.rope_inside
+    for B in range(5, 129):
+        for Hq, Hkv in ((32, 8), (16, 4), (8, 2), (4, 1), (64, 8)):
+            for blocks in (1, 2, 3, 8, 9, 16, 22, 47, 64):
+                P = kv_partitions(B, Hq, Hkv, blocks)
+                assert inside(B, Hkv, blocks, -P, True) == (B * Hkv * P <= 512 or not K.paged_waves(B * Hkv * P, blocks, P)[2]), (B, Hkv, blocks, P)
+    for B, blocks, P, window in ((64, 16, 4, 0), (128, 8, 2, 0), (128, 64, 2, 200), (33, 8, 2, 0)):
+        assert K.paged_waves(B * 8 * P, min(blocks, (window + 30) // 32 + 1) if window else blocks, P)[2]
+        assert not inside(B, 8, blocks, -P, True, window)
+    assert inside(32, 8, 8, -2, True) and inside(128, 8, 64, -2, True) and inside(128, 8, 64, -2, True, 2048)
