@@ -125,7 +125,8 @@ struct KnnRows {
 // Queries of floats to LDS, as l2_normalize_kernel takes them to memory, a wave a query, to the bit: the workgroups of a round each do
 // so beside their first rows' way from memory, and a search has a launch less (us: 1 query of 20 k rows of 384 17.0 -> 14.3, of 27 k of
 // 768 19.4 -> 16.3, 4 queries of 27 k of 384 17.8 -> 15.6, 1 of 1M 136 -> 133.7, 16 163 -> 159.6).  Asked for before the rows are, by four
-// waves; FROWS queries at most, for which there is room beside the rings.
+// waves; their wait is one for the first rows, too, as that ahead of the first use of queries in bf16 is (taken to LDS before a row is asked
+// for: 1.000 of the time, 20 k to 1M rows).  FROWS queries at most, for which there is room beside the rings.
 template <int KC>
 struct KnnFloats {
   static constexpr int FROWS = KC <= 16 ? 16 : 8, ROW = KC * 64 + 16, NV = (KC * 4 + 63) / 64, BYTES = FROWS * ROW;
