@@ -158,7 +158,7 @@ class EncoderModel:
         c = self.cfg
         if (ids.is_cuda and tiles is not None and os.environ.get("CFC_ENCODER_GEMM", "auto") == "auto"
                 and os.environ.get("CFC_ENCODER_LN_FUSED", "1") != "0"):
-            w = K.encoder_weights(ids.numel(), self.p, self.layers, c.heads, max_seqlen, between=True)
+            w = K.encoder_weights(ids.numel(), self.p, self.layers, c.heads, max_seqlen)
             if w is not None:
                 return K.encoder_forward(ids, positions, w, len(self.layers), cu_seqlens, tiles, c.heads, max_seqlen, self.scale, c.ln_eps)
         x = K.embed_layernorm(ids, positions, self.p["word"], self.p["pos"], self.p["type"], self.p["emb_g"],

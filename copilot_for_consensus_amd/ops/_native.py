@@ -104,7 +104,7 @@ _KERNEL_SIGS = {
     "cfc_prefill_attention_expanded2": [P, c_int64, c_int64, P, P, P, P, P, c_int64, P, P, P, P, I, I, F, I, P, P, c_int64, P,
                                         c_int64, P],
     "cfc_prefill_attention_expanded": [P, P, P, P, c_int64, P, P, P, P, I, I, F, P, c_int64, P],
-    "cfc_enc_rows": [I],
+    "cfc_enc_fused": [I],
     "cfc_knn_queries": [P, P, P, I, I, I, P],
     "cfc_knn_search": [P, P, I, I, I, I, P, P, I, L, P, L, P, P, P],
     "cfc_knn_search_bytes": [I, I, I],

@@ -480,12 +480,11 @@ def put_ints(host: torch.Tensor, device) -> torch.Tensor:
     return out
 
 
-def encoder_weights(T: int, p: dict, layers: list[dict], heads: int, max_seqlen: int, between: bool = False) -> list[int] | None:
+def encoder_weights(T: int, p: dict, layers: list[dict], heads: int, max_seqlen: int) -> list[int] | None:
     """Addresses of what :func:`encoder_forward` reads, embeddings first; None where encoder.hip is not built for T rows
-    (few or many; with ``between`` also those between) of this model: hidden 384, inner 1536, contiguous bf16 tensors on one GPU."""
+    (any number) of this model: hidden 384, inner 1536, contiguous bf16 tensors on one GPU."""
     H, word = ENCODER_HIDDEN, p["word"]
-    if not word.is_cuda or T < 1 or not (between or kernels().cfc_enc_rows(T) != 3) or not layers or not 1 <= max_seqlen <= 512 \
-            or heads not in (H // 32, H // 64):
+    if not word.is_cuda or T < 1 or not layers or not 1 <= max_seqlen <= 512 or heads not in (H // 32, H // 64):
         return None
     emb = [p[k] for k in ("word", "pos", "type", "emb_g", "emb_b")]
     ts = emb + [t for lw in layers for t in _ENCODER_TENSORS(lw)]
@@ -517,7 +516,7 @@ def encoder_forward(ids, positions, weights: list[int], layers: int, cu_seqlens,
         h = torch.empty(tiny, dtype=torch.bfloat16, device=dev)
     else:
         att, qkv = rows(H), rows(3 * H)
-        y, h = (rows(2 * H), rows(ENCODER_FFN)) if lib.cfc_enc_rows(T) != 2 else (None, None)     # y: 32 bits
+        y, h = (rows(2 * H), rows(ENCODER_FFN)) if not lib.cfc_enc_fused(T) else (None, None)     # y: 32 bits
     W = (ctypes.c_void_p * (len(weights) - 5))(*weights[5:])
     check(lib.cfc_enc_forward(ids.data_ptr(), positions.data_ptr(), *weights[:5],
                               cu_seqlens.data_ptr(), tiles[0].data_ptr(), tiles[1].data_ptr(), tiles[0].numel(), ENCODER_TILE_ROWS,

@@ -680,23 +680,23 @@ __device__ __forceinline__ void en_norm16(float (&v)[24], uint4 (&p)[3], const u
   }
 }
 
-// y = x W^T + b (GELU: x Phi(x) of it) for a 384-wide x and a W of N rows, in tiles of 16 RG rows and 16 WAVES columns.  A wave
+// y = x W^T + b (GELU: x Phi(x) of it) for a 384-wide x and a W of N rows, in tiles of 16 RG rows and 64 columns.  A wave
 // owns 16 columns: its fragments of W go straight to registers, all in flight with all of the tile's rows.
-template <bool GELU, bool LN, int RG, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES) enc_tile_kernel(uint16_t* x, EncNorm ln, const uint16_t* __restrict__ W,
+template <bool GELU, bool LN, int RG>
+__global__ void __launch_bounds__(256) enc_tile_kernel(uint16_t* x, EncNorm ln, const uint16_t* __restrict__ W,
                                                        const uint16_t* __restrict__ bias, uint16_t* __restrict__ out, int M, int N) {
   constexpr int CH = EN_H / 8, KS = EN_H / 32;    // 16-byte chunks of a row, k steps
-  constexpr int B = 4 * RG / WAVES;               // rows of a lane group: four rows a wave at a time, 16 lanes each
-  static_assert(4 * RG % WAVES == 0 && CH == 48);
+  constexpr int B = RG;                           // rows of a lane group: four rows a wave at a time, 16 lanes each
+  static_assert(CH == 48);
   __shared__ __attribute__((aligned(16))) char smem[16 * RG * EN_H * 2];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
-  const int n0 = (blockIdx.x * WAVES + w) * 16, m0 = blockIdx.y * 16 * RG, rows = min(16 * RG, M - m0);
+  const int n0 = (blockIdx.x * 4 + w) * 16, m0 = blockIdx.y * 16 * RG, rows = min(16 * RG, M - m0);
   uint4 wf[KS], q[B][3];
   u32x4_t p[B][3];      // as uint4 rows that no norm follows went through scratch: 6.7 us of 73 rows, 6.2 of 300, so 4.3 and 4.9
-  // row 4 (w + WAVES b) + g, its chunks r16 + 16 j
+  // row 4 (w + 4 b) + g, its chunks r16 + 16 j
 #pragma unroll
   for (int b = 0; b < B; ++b) {
-    const size_t at = (size_t)(m0 + min(4 * (w + WAVES * b) + g, rows - 1)) * EN_H + 8 * r16;
+    const size_t at = (size_t)(m0 + min(4 * (w + 4 * b) + g, rows - 1)) * EN_H + 8 * r16;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       p[b][j] = *reinterpret_cast<const u32x4_t*>((LN ? ln.proj : x) + at + 128 * j);
@@ -720,7 +720,7 @@ __global__ void __launch_bounds__(64 * WAVES) enc_tile_kernel(uint16_t* x, EncNo
   // chunk c of row r at slot c ^ (r & 7): 16-row fragment reads without bank conflicts
 #pragma unroll
   for (int b = 0; b < B; ++b) {
-    const int r = 4 * (w + WAVES * b) + g;
+    const int r = 4 * (w + 4 * b) + g;
     if constexpr (LN) {
       float v[24];
 #pragma unroll
@@ -941,8 +941,8 @@ __global__ void __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * 64)
 }
 
 // ================================================================ a query or a few short texts
-// Up to 64 tokens, all layers in one launch: five launches a layer, each waiting for the one before, took 27 us of which
-// the work itself is 3.  60 workgroups of three kinds: one per head takes the layer's q, k, v and attention of its head,
+// Up to 64 tokens, all layers in one launch: five launches a layer, each waiting for the one before, take 17 to 20 us (small tiles; 27
+// when this kernel was written) of which the work itself is 3.  60 workgroups of three kinds: one per head takes the layer's q, k, v and attention of its head,
 // 24 take 16 columns each of the output projection and of the down product, 24 take 64 columns of the up product.
 // Those that need normed rows norm all of them and keep them in registers, so nothing but products passes between
 // workgroups: attention, o, hidden rows and down, four hand-overs a layer.  Each goes through a place of its own per layer
@@ -951,7 +951,9 @@ __global__ void __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * 64)
 // Weights come a layer ahead of their use, straight to the registers they are used from; a CU brings in some 25 B/ns, so
 // they are spread (a quarter of the workgroups took 94 us where these take 80), and are asked for only when nothing is
 // waited for, as loads return in order (104 -> 94 us).
-// 12 tokens through MiniLM's six layers 136 -> 80 us, 32 tokens 188 -> 119, 64 tokens 295 -> 178.  A layer's 12 us are
+// MiniLM's six layers in small tiles and in this, us of a captured forward: 1 token 100 and 69, 12 108 and 81, 16 113 and 84, 24 114 and 113,
+// 32 115 and 119, 33 118 and 162, 64 122 and 179 (136, 188 and 295 of 12, 32 and 64 in the tiles of its day): from some 30 rows on
+// small tiles are the faster ones now, though their sums come in another order.  A layer's 12 us are
 // its four hand-overs of 2 to 2.5 us (a store and a poll of about 1 us each), two norms and the products between.
 //
 // The workgroups wait for one another, so all have to be resident, and nothing can promise that: launches of other streams
@@ -1454,14 +1456,13 @@ CFC_API int cfc_encoder_attention(const void* qkv, const int32_t* cu_seqlens, co
                                   int n_tiles, int tile_rows, int H, int head_dim, int max_seqlen, float scale, void* out,
                                   hipStream_t stream);
 
-// A few texts of 64 rows in all: enc_tiny_kernel.  Few: up to 2560 rows.  Many: from 10753, where the general tiles need another
-// round of the chip.  All of these, and with cfc_enc_forward those between, take small tiles up to 320 rows, LDS tiles up to
-// 16383 and the layer's one kernel above (six layers of MiniLM in LDS tiles and in it: 14000 rows 712 and 826 us, 16000 767
-// and 838, 18000 845 and 848).
-constexpr int EN_FEW_ROWS = 2560, EN_MANY_ROWS = 10753, EN_FUSED_ROWS = 16384;
+// A few texts of 64 rows in all: enc_tiny_kernel.  More take small tiles up to 320 rows, LDS tiles up to 16383 and the layer's one
+// kernel above from there on (six layers of MiniLM in LDS tiles and in it: 14000 rows 712 and 826 us, 16000 767 and 838, 18000 845
+// and 848).
+constexpr int EN_FUSED_ROWS = 16384;
 
-// How many rows T are: 1 few, 3 between, 4 many, 2 as many as the layer's one kernel takes, which alone needs no y and h.
-CFC_API int cfc_enc_rows(int T) { return T <= EN_FEW_ROWS ? 1 : T < EN_MANY_ROWS ? 3 : T < EN_FUSED_ROWS ? 4 : 2; }
+// Whether T rows are as many as the layer's one kernel takes, which needs no y and h.
+CFC_API int cfc_enc_fused(int T) { return T >= EN_FUSED_ROWS; }
 
 // Values of workspace (bf16) that the one launch for T rows of a model takes on a stream; 0: it does not take them, or so few
 // CUs are the stream's that its workgroups would be long in coming.
@@ -1480,8 +1481,8 @@ constexpr int EN_CUS = 256;
 template <bool GELU, bool LN>
 void en_tile(int groups, uint16_t* x, const EncNorm& ln, const uint16_t* W, const uint16_t* bias, uint16_t* out, int T, int N, hipStream_t stream) {
   const dim3 grid(N / 64, (T + 16 * groups - 1) / (16 * groups));
-  if (groups == 1) enc_tile_kernel<GELU, LN, 1, 4><<<grid, 256, 0, stream>>>(x, ln, W, bias, out, T, N);
-  else enc_tile_kernel<GELU, LN, 2, 4><<<grid, 256, 0, stream>>>(x, ln, W, bias, out, T, N);
+  if (groups == 1) enc_tile_kernel<GELU, LN, 1><<<grid, 256, 0, stream>>>(x, ln, W, bias, out, T, N);
+  else enc_tile_kernel<GELU, LN, 2><<<grid, 256, 0, stream>>>(x, ln, W, bias, out, T, N);
 }
 
 template <int K>
@@ -1494,11 +1495,6 @@ void en_ksplit(int groups, const uint16_t* x, const uint16_t* W, uint16_t* out, 
 template <int K, int BM, int BN, int TM, int TN, int NS, int EPI>
 void en_gemm(const uint16_t* x, const uint16_t* W, const uint16_t* bias, void* out, int T, int N, hipStream_t stream) {
   constexpr int LDS = NS * (BM + BN) * 128;
-  if constexpr (LDS > 64 * 1024) {
-    static const hipError_t raised =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&enc_gemm_kernel<K, BM, BN, TM, TN, NS, EPI>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-    (void)raised;
-  }
   enc_gemm_kernel<K, BM, BN, TM, TN, NS, EPI><<<N / BN * ((T + BM - 1) / BM), 64 * (BM / 32 / TM) * (BN / 32 / TN), LDS, stream>>>(x, W, bias, out, T, N);
 }
 
@@ -1524,14 +1520,14 @@ void en_raw(const uint16_t* x, const uint16_t* W, void* y, int T, hipStream_t st
 
 // Token states of a packed batch: embeddings, then every layer, one call for all launches.  W: host array of twelve
 // device pointers per layer (qkv, qkv_b, o, o_b, ln1_g, ln1_b, up, up_b, down, down_b, ln2_g, ln2_b).  x [T][384] the
-// states; att [T][384], qkv [T][1152], and unless cfc_enc_rows is 2 y [T][384] of 32 bits and h [T][1536]: workspace.  All else
+// states; att [T][384], qkv [T][1152], and unless cfc_enc_fused y [T][384] of 32 bits and h [T][1536]: workspace.  All else
 // bf16, all 16-byte aligned.  With att null, h is the workspace of cfc_enc_tiny and no other is read; a wait in that launch is given up after
 // `polls` loads (below 0: EN_POLLS).
 CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* word, const void* pos_emb, const void* type_emb,
                             const void* emb_g, const void* emb_b, const int32_t* cu, const int32_t* tile_seq, const int32_t* tile_q0,
                             int n_tiles, int tile_rows, int max_seqlen, int layers, const void* const* W, int heads, float scale,
                             float eps, int T, void* x, void* y, void* att, void* qkv, void* h, int polls, hipStream_t stream) {
-  const int kind = cfc_enc_rows(T);
+  const bool fused = cfc_enc_fused(T);
   if (att == nullptr) {
     const int n = cfc_enc_tiny(T, layers, heads, stream);
     if (n == 0 || h == nullptr || tile_rows < EN_TINY_ROWS || n_tiles < 0) return -1;
@@ -1552,7 +1548,7 @@ CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* 
 #undef TINY
     return CFC_CHECK_LAUNCH();
   }
-  if (T < 1 || layers < 1 || heads < 1 || EN_H % heads || (kind != 2 && (h == nullptr || y == nullptr))) return -1;
+  if (T < 1 || layers < 1 || heads < 1 || EN_H % heads || (!fused && (h == nullptr || y == nullptr))) return -1;
   int rc = cfc_layernorm(x, word, nullptr, nullptr, emb_g, emb_b, ids, pos, pos_emb, type_emb, T, EN_H, eps, 2, stream);
   uint16_t *xp = (uint16_t*)x, *yp = (uint16_t*)y, *ap = (uint16_t*)att, *qp = (uint16_t*)qkv, *hp = (uint16_t*)h;
   const int blocks = (T + EN_ROWS - 1) / EN_ROWS;
@@ -1563,7 +1559,7 @@ CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* 
   auto attend = [&]() { return cfc_encoder_attention(qkv, cu, tile_seq, tile_q0, n_tiles, tile_rows, heads, EN_H / heads, max_seqlen, scale, att, stream); };
   for (int l = 0; l < layers && rc == 0; ++l) {
     const uint16_t* const* p = P + 12 * l;
-    if (kind == 2) {
+    if (fused) {
       if (T > EN_CUS * EN_ROWS)       // more than a workgroup of 128 rows a CU
         enc_proj_wide_kernel<<<(T + EW_ROWS - 1) / EW_ROWS, 256, 0, stream>>>(xp, p[0], p[1], qp, T);
       else
@@ -1592,7 +1588,7 @@ CFC_API int cfc_enc_forward(const int32_t* ids, const int32_t* pos, const void* 
     }
   }
   if (rc) return rc;
-  if (kind != 2 && small) {
+  if (!fused && small) {
     const uint16_t* const* p = P + 12 * layers;
     return cfc_layernorm(x, y, p[-3], att, p[-2], p[-1], nullptr, nullptr, nullptr, nullptr, T, EN_H, eps, 1, stream);
   }
