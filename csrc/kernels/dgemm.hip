@@ -316,6 +316,7 @@ __global__ void __launch_bounds__((64 * DgShape<BM, BN, (ABL & 64) != 0, GRP == 
   // read past the slice (the tail computes only real stages).
   constexpr bool TAIL_RELOAD = (ABL & 256) != 0;    // probe: the former tail, which reads again
   int st = 0;
+  // (in a plain loop hipcc makes 2 % more code of it: decode steps of four layers, 16 rows 837 -> 843 us, 64 986 -> 1000)
   auto round = [&]() {
 #pragma unroll
     for (int u = 0; u < D; ++u) {
