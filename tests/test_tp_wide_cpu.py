@@ -87,7 +87,7 @@ def _tp_rank(rank, world, port, prefixes, q):
         eng = _engine(m, w.kv_heads)
         toks = eng.generate(PROMPTS, N_NEW, ignore_eos=True).tokens
         logits = _prefix_logits(eng, m, prefixes)
-        q.put((rank, True, (w.kv_heads, w.heads, toks, logits)))
+        q.put((rank, True, (w.kv_heads, w.heads, toks, logits.numpy())))     # the bytes: a tensor is fetched from a rank that may have ended
     except Exception:  # noqa: BLE001
         q.put((rank, False, traceback.format_exc()))
     finally:
@@ -111,7 +111,7 @@ def test_tp_wide_matches_tp1_70b_head_layout(tp):
             if not q.empty():
                 r, ok, payload = q.get()
                 assert ok, f"rank {r}:\n{payload}"
-                res[r] = payload
+                res[r] = (*payload[:3], torch.from_numpy(payload[3]))
             else:
                 time.sleep(0.05)
         assert len(res) == tp, f"ranks answered: {sorted(res)}"
